@@ -36,3 +36,21 @@ def test_host_side_argument_checks_without_gpu():
   assert moe.m_max_for(4096, 8, 128) == 65536                                     # (ceil(T*k/256) + E) * 256, moe_routing.py:89-90
   b = moe.to_bf16_bits(np.array([1.0, 1.00390625, -2.5, 1.01171875], np.float32))     # 1 + 2^-8 ties to even (1.0); 1 + 3*2^-8 rounds up
   np.testing.assert_array_equal(moe.from_bf16_bits(b), np.array([1.0, 1.0, -2.5, 1.015625], np.float32))
+
+@pytest.mark.gpu
+def test_freed_blocks_are_kept_and_given_back(gpu):
+  """tga_free keeps a block for later requests of its size class, never hands it out while kernels may still use it, and tga_trim gives everything back: results computed into
+  blocks that were freed and allocated again many times over are right, and the library still allocates afterwards."""
+  import numpy as np
+  n = 3 << 20
+  src = [gpu.Buffer.from_numpy(np.full(n, i, np.uint8)) for i in range(4)]
+  streams = [gpu.Stream() for _ in range(2)]
+  for r in range(40):                                                              # more rounds than dirty blocks are collected before they are settled
+    outs = [gpu.Buffer((n,), np.uint8) for _ in range(4)]
+    for i, o in enumerate(outs): gpu.check(gpu.lib().tga_copy_kernel(o.ptr, src[(i + r) % 4].ptr, n, streams[i % 2].handle))
+    if r % 7 == 0:
+      gpu.synchronize()
+      for i, o in enumerate(outs): assert (o.numpy() == (i + r) % 4).all()
+  gpu.check(gpu.lib().tga_trim())
+  b = gpu.Buffer((n,), np.uint8); gpu.check(gpu.lib().tga_copy_kernel(b.ptr, src[3].ptr, n, None)); gpu.synchronize()
+  assert (b.numpy() == 3).all()

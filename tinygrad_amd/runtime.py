@@ -26,7 +26,7 @@ c_void_pp = ctypes.POINTER(ctypes.c_void_p)
 def _declare(lib):
   vp, i, i64, sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_size_t
   sig = {
-    "tga_init": [i], "tga_device_name": [ctypes.c_char_p, sz], "tga_malloc": [c_void_pp, sz], "tga_free": [vp],
+    "tga_init": [i], "tga_device_name": [ctypes.c_char_p, sz], "tga_malloc": [c_void_pp, sz], "tga_free": [vp], "tga_trim": [],
     "tga_memcpy_h2d": [vp, vp, sz], "tga_memcpy_d2h": [vp, vp, sz], "tga_memcpy_d2d": [vp, vp, sz, vp], "tga_memset": [vp, i, sz, vp],
     "tga_sync": [], "tga_stream_create": [c_void_pp], "tga_stream_destroy": [vp], "tga_stream_sync": [vp],
     "tga_event_create": [c_void_pp], "tga_event_destroy": [vp], "tga_event_record": [vp, vp], "tga_event_sync": [vp],
