@@ -223,3 +223,40 @@ def test_grouped_gemm_with_counts_skips_padding(gpu):
     np.testing.assert_array_equal(c2[lo + n:pad16], c1[lo + n:pad16])
     assert (c2[pad16:hi] == 0).all(), f"padding rows of expert {e}"
   assert (c2[off[-1]:] == 0xABAB).all()
+
+@pytest.mark.parametrize("rows,K", [(1, 32), (3, 96), (5, 160), (257, 128), (33, 1056), (2048, 4096)])
+def test_quantize_rows_of_any_length(gpu, rows, K):
+  """Four lanes per block: single blocks, rows that end inside a wave, several trips per thread; float32 and bf16 rows, with and without the packed scales, bit for bit."""
+  from tinygrad_amd import moe
+  rng = np.random.default_rng(rows + K)
+  x = (rng.standard_normal((rows, K)) * np.exp2(rng.integers(-20, 12, size=(rows, 1)))).astype(np.float32)
+  bits = moe.to_bf16_bits(x)
+  for src, ref in ((x, x), (bits, moe.from_bf16_bits(bits))):
+    q, e8, packed = moe.quantize_mxfp8(gpu.Buffer.from_numpy(src))
+    rq, re8 = omx.quantize_mxfp8(ref)
+    np.testing.assert_array_equal(e8.numpy(), re8); np.testing.assert_array_equal(q.numpy(), rq)
+    assert (packed is None) == (K % 128 != 0)
+    if packed is not None: np.testing.assert_array_equal(packed.numpy(), re8.reshape(rows, K // 128, 4).view(np.uint32)[..., 0].T)
+
+@pytest.mark.parametrize("M,N", [(32, 64), (96, 128), (128, 64), (160, 192), (512, 256)])
+def test_transpose_quantize_of_ragged_row_counts(gpu, M, N):
+  """Row counts that end inside a 128-row tile (no packed scales there) against quantize_mxfp8 of the transposed matrix, bit for bit."""
+  from tinygrad_amd import moe
+  bits = moe.to_bf16_bits(np.random.default_rng(M + N).standard_normal((M, N)).astype(np.float32) * 3)
+  q, e8, packed = moe.transpose_quantize_mxfp8(gpu.Buffer.from_numpy(bits))
+  rq, re8 = omx.quantize_mxfp8(np.ascontiguousarray(moe.from_bf16_bits(bits).T))
+  np.testing.assert_array_equal(q.numpy(), rq); np.testing.assert_array_equal(e8.numpy(), re8)
+  if packed is not None: np.testing.assert_array_equal(packed.numpy(), re8.reshape(N, M // 128, 4).view(np.uint32)[..., 0].T)
+
+def test_swiglu_beyond_one_trip_and_off_alignment(gpu):
+  """More outputs than one pass of the grid holds, a length that is no multiple of four, and operands that start off a 16-byte boundary: the same values as small aligned calls."""
+  from tinygrad_amd import moe
+  rng = np.random.default_rng(5)
+  unit = moe.to_bf16_bits((rng.standard_normal((1, 2 * 4099)) * 4).astype(np.float32))
+  ref = omx.swiglu_interleaved(moe.from_bf16_bits(unit))[0]
+  rows = (1 << 24) // 4099 + 300                                       # > 2^24 outputs, rows of an odd length
+  y = moe.swiglu(gpu.Buffer.from_numpy(np.tile(unit, (rows, 1)))).numpy()
+  np.testing.assert_allclose(moe.from_bf16_bits(y[0]), ref, rtol=2 ** -7, atol=1e-30)
+  assert (y == y[0]).all()
+  off = gpu.Buffer.from_numpy(np.concatenate([np.zeros(1, np.uint16), unit[0]])).view(2, (1, 2 * 4099), np.uint16)
+  np.testing.assert_array_equal(moe.swiglu(off).numpy()[0], y[0])

@@ -2,124 +2,112 @@
 // (route / dispatch / combine) and the grouped GEMM on CDNA4 scaled MFMA.
 // Reference: extra/gemm/cdna_asm_gemm.py:149-173 (quantize_mxfp8, mx_pack), extra/gemm/moe_routing.py:89-131 (route, dispatch,
 // combine), extra/gemm/moe_gemm.py:112-134 (grouped_mx_gemm; its HIP kernel source is absent from the reference tree).
-#include "common.h"
+#include "mxfp8.h"
 #include "host.h"
 #include <string.h>
 
-typedef int v8i32 __attribute__((ext_vector_type(8)));
-typedef float v4f32 __attribute__((ext_vector_type(4)));
-
 #define MX_BLOCK_ROW 256
 
-__device__ __forceinline__ float bf16_to_f(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
-__device__ __forceinline__ uint16_t f_to_bf16(float f) {   // round to nearest even (tinygrad/dtype.py:224-226)
-  uint32_t u = __builtin_bit_cast(uint32_t, f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
-  return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1)) >> 16);
-}
-// float -> E4M3 (fn) bits, RNE, finite saturation (tinygrad/dtype.py:237-260); |x| is already clamped to 448 by the caller
-__device__ __forceinline__ uint32_t f_to_e4m3(float x) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, x), sign = (u >> 24) & 0x80;
-  const float a = fabsf(x);
-  if (!(a == a)) return sign | 0x7f;
-  if (a >= 464.0f) return sign | 0x7e;
-  if (a < 0.0009765625f) return sign;                       // <= 2^-10 (half the smallest subnormal) rounds to zero (ties to even)
-  int e; (void)frexpf(a, &e); e -= 1;                       // a = m * 2^e, 1 <= m < 2
-  if (e < -6) e = -6;
-  const float q = rintf(ldexpf(a, 3 - e));                  // mantissa grid: 8..16 (normal) or 0..8 (subnormal)
-  float v = ldexpf(q, e - 3);
-  if (v > 448.0f) v = 448.0f;
-  int e2; const float m2 = frexpf(v, &e2); e2 -= 1;
-  if (v < 0.015625f) return sign | (uint32_t)(v * 512.0f);  // subnormal: v / 2^-9
-  return sign | ((uint32_t)(e2 + 7) << 3) | (uint32_t)((m2 * 2.0f - 1.0f) * 8.0f);
-}
-
 // ------------------------------------------------------------------------------------------------ quantize_mxfp8
-// One thread per 32-element block: amax, e8 = clamp(floor(log2(max(amax, 1e-38))) + 127, 0, 254), q = e4m3(clamp(x * 2^(127-e8), +-448)).
-// Also writes the packed scales of mx_pack: packed[k/128][row] = 4 consecutive e8 bytes (little-endian).
-// One 32-element block: e8 = clamp(floor(log2(max(amax, 1e-38))) + 127, 0, 254); out = 32 E4M3 bytes of clamp(v * 2^(127 - e8), +-448).
-__device__ __forceinline__ int mx_quant32(const float* v, uint32_t* out) {
-  float amax = 0.f;
-#pragma unroll
-  for (int i = 0; i < 32; i++) amax = fmaxf(amax, fabsf(v[i]));
-  int ex; (void)frexpf(amax, &ex);                         // floor(log2(a)) = ex - 1
-  // below the smallest normal float the reference's max(amax, 1e-38) floor gives floor(log2) = -127 -> e8 = 0
-  int e = amax < 1.17549435e-38f ? 0 : ex - 1 + 127; e = e < 0 ? 0 : (e > 254 ? 254 : e);
-  const float qs = __builtin_bit_cast(float, (uint32_t)(254 - e) << 23);   // 2^(127 - e), exact for e in 0..253; e = 254 -> 2^-127 below
-  const float scale = (e == 254) ? __builtin_bit_cast(float, 0x00400000u) : qs;
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    uint32_t w = 0;
-#pragma unroll
-    for (int j = 0; j < 4; j++) { float s = v[4 * i + j] * scale; s = fminf(fmaxf(s, -448.0f), 448.0f); w |= f_to_e4m3(s) << (8 * j); }
-    out[i] = w;
-  }
-  return e;
-}
+// A block of 32 values: e8 = clamp(floor(log2(max(amax, 1e-38))) + 127, 0, 254), q = e4m3(clamp(x * 2^(127 - e8), +-448)).  Four neighbouring lanes hold a block, eight
+// values each: every load and store of a wave covers one contiguous span (a thread per block read 16 bytes of every 64, and converted in ~30 operations per value
+// what v_cvt_pk_fp8_f32 converts two at a time: 16384 x 4096 bf16 rows 59 us; now 46 us for the whole call, 4.5 TB/s where a large copy moves 5.0), the block maximum takes two quad permutations.
+// Also writes the packed scales of mx_pack: packed[k / 128][row] = 4 consecutive e8 bytes (little-endian), one dword per sixteen lanes.
 // MODE 0: x float32; 1: x bf16; 2: fused SwiGLU producer, value = w1 * sigmoid(w1) * w3 in float32 from two bf16 tensors x (= x_w1)
 // and x2 (= x_w3), sigmoid as 1 / (1 + exp2(-w1 * log2(e)))  (extra/llama_kernels/fused_silu_mul_quantize_mxfp8/__init__.py:33-36)
+__device__ __forceinline__ void bf16x8(const u32x4 w, float* o) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) { o[2 * i] = bf16_lo(w[i]); o[2 * i + 1] = bf16_hi(w[i]); }
+}
 template <int MODE>
-__global__ __launch_bounds__(256) void quantize_mxfp8_kernel(const void* __restrict__ x, const void* __restrict__ x2, long long rows, int K, uint8_t* __restrict__ q,
+__global__ __launch_bounds__(256) void quantize_mxfp8_kernel(const void* __restrict__ x, const void* __restrict__ x2, const long long rows, const int K, uint8_t* __restrict__ q,
                                                              uint8_t* __restrict__ e8, uint8_t* __restrict__ packed) {
-  const long long nb = rows * (K / 32);
-  for (long long b = (long long)blockIdx.x * 256 + threadIdx.x; b < nb; b += (long long)gridDim.x * 256) {
-    const long long row = b / (K / 32); const int kb = (int)(b % (K / 32));
-    float v[32];
-    auto load_bf16 = [&](const void* src, float* o) {
-      const u32x4* p = (const u32x4*)((const uint16_t*)src + row * K + kb * 32);
+  const long long n8 = rows * (K / 8), stride = (long long)gridDim.x * 256;             // pieces of eight values
+  constexpr int U = MODE == 1 ? 4 : 2;                                                   // pieces per thread and trip: their loads go out together
+  for (long long p0 = (long long)blockIdx.x * 256 + threadIdx.x; p0 < n8; p0 += U * stride) {
+    u32x4 a[U], b[U];
 #pragma unroll
-      for (int i = 0; i < 4; i++) { const u32x4 w = p[i];
-        o[8*i] = bf16_to_f(w.x & 0xFFFF); o[8*i+1] = bf16_to_f(w.x >> 16); o[8*i+2] = bf16_to_f(w.y & 0xFFFF); o[8*i+3] = bf16_to_f(w.y >> 16);
-        o[8*i+4] = bf16_to_f(w.z & 0xFFFF); o[8*i+5] = bf16_to_f(w.z >> 16); o[8*i+6] = bf16_to_f(w.w & 0xFFFF); o[8*i+7] = bf16_to_f(w.w >> 16); }
-    };
-    if constexpr (MODE == 1) load_bf16(x, v);
-    else if constexpr (MODE == 2) {
-      float u[32];
-      load_bf16(x, v); load_bf16(x2, u);
-#pragma unroll
-      for (int i = 0; i < 32; i++) { const float sig = 1.0f / (1.0f + exp2f(v[i] * -1.4426950408889634f)); v[i] = v[i] * sig * u[i]; }
-    } else {
-      const f32x4* p = (const f32x4*)((const float*)x + row * K + kb * 32);
-#pragma unroll
-      for (int i = 0; i < 8; i++) { const f32x4 w = p[i]; v[4*i] = w.x; v[4*i+1] = w.y; v[4*i+2] = w.z; v[4*i+3] = w.w; }
+    for (int u = 0; u < U; u++) {
+      const long long p = p0 + u * stride < n8 ? p0 + u * stride : p0;
+      if constexpr (MODE == 0) { a[u] = ((const u32x4*)x)[2 * p]; b[u] = ((const u32x4*)x)[2 * p + 1]; }
+      else { a[u] = ((const u32x4*)x)[p]; if constexpr (MODE == 2) b[u] = ((const u32x4*)x2)[p]; }
     }
-    uint32_t out[8];
-    const int e = mx_quant32(v, out);
-    u32x4* qo = (u32x4*)(q + row * K + kb * 32);
-    qo[0] = u32x4{out[0], out[1], out[2], out[3]}; qo[1] = u32x4{out[4], out[5], out[6], out[7]};
-    e8[row * (K / 32) + kb] = (uint8_t)e;
-    if (packed) packed[((long long)(kb >> 2) * rows + row) * 4 + (kb & 3)] = (uint8_t)e;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const long long p = p0 + u * stride;
+      if (p >= n8) break;                                                                // (whole quads leave together: n8 is a multiple of 4)
+      float v[8];
+      if constexpr (MODE == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) { const uint32_t lo = a[u][i], hi = b[u][i]; v[i] = __builtin_bit_cast(float, lo); v[4 + i] = __builtin_bit_cast(float, hi); }   // (through scalars: a bit cast of a vector element reads element 0)
+      } else bf16x8(a[u], v);
+      if constexpr (MODE == 2) {
+        float w[8];
+        bf16x8(b[u], w);
+#pragma unroll
+        for (int i = 0; i < 8; i++) { const float sig = 1.0f / (1.0f + exp2f(v[i] * -1.4426950408889634f)); v[i] = v[i] * sig * w[i]; }
+      }
+      float amax = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v[i]));
+      const int e = mx_e8(quad_max(amax));
+      const float s = mx_scale(e);
+      ((u32x2*)q)[p] = u32x2{e4m3x4(v[0] * s, v[1] * s, v[2] * s, v[3] * s), e4m3x4(v[4] * s, v[5] * s, v[6] * s, v[7] * s)};
+      const int lane = threadIdx.x & 63;
+      if ((lane & 3) == 0) e8[p >> 2] = (uint8_t)e;
+      if (packed) {                                                                      // (K % 128 == 0: the sixteen lanes of a dword sit in one row)
+        const uint32_t w = (uint32_t)(__shfl(e, lane & 48) | (__shfl(e, (lane & 48) + 4) << 8) | (__shfl(e, (lane & 48) + 8) << 16) | (__shfl(e, (lane & 48) + 12) << 24));
+        if ((lane & 15) == 0) { const long long kb = p >> 4, row = kb / (K >> 7); ((uint32_t*)packed)[(kb - row * (K >> 7)) * rows + row] = w; }
+      }
+    }
   }
 }
 
 // transpose_quantize_mxfp8 (extra/llama_kernels/transpose_quantize_mxfp8/__init__.py:24-37) == quantize_mxfp8(g.T) without the transposed
-// tensor: g (M, N) bf16 -> q (N, M), e8 (N, M / 32), packed (M / 128, N).  One workgroup takes 128 rows x 64 columns of g through LDS
-// (row-wise 16-byte loads, column-wise reads), thread (column c, 32-row run r) quantizes one block, and the four runs of a column fill one
-// 128-byte line of q.
+// tensor: g (M, N) bf16 -> q (N, M), e8 (N, M / 32), packed (M / 128, N).  One workgroup takes 128 rows x 64 columns of g through LDS (row-wise 16-byte loads).  A thread
+// reads two neighbouring columns at once (one dword per row), sixteen rows of them; a block is the sixteen rows of two threads eight lanes apart in the row
+// run index, and the eight runs of a column fill one 128-byte line of q.
 __global__ __launch_bounds__(256) void transpose_quantize_mxfp8_kernel(const uint16_t* __restrict__ g, int M, int N, uint8_t* __restrict__ q,
                                                                        uint8_t* __restrict__ e8, uint8_t* __restrict__ packed) {
-  __shared__ uint16_t tile[128][64 + 8];                    // 144-byte rows: 16-byte aligned, column reads of a wave hit 32 different banks
+  __shared__ uint32_t tile[128][33];                        // 132-byte rows: the column reads of eight 16-row runs fall on different banks
   const int n0 = blockIdx.x * 64, m0 = blockIdx.y * 128, t = threadIdx.x;
 #pragma unroll
   for (int p = 0; p < 4; p++) {
-    const int r = p * 32 + (t >> 3), c8 = (t & 7) * 8;
+    const int r = p * 32 + (t >> 3), c4 = (t & 7) * 4;
     u32x4 w = {0, 0, 0, 0};
-    if (m0 + r < M) w = *(const u32x4*)(g + (size_t)(m0 + r) * N + n0 + c8);
-    *(u32x4*)&tile[r][c8] = w;
+    if (m0 + r < M) w = *(const u32x4*)(g + (size_t)(m0 + r) * N + n0 + 2 * c4);
+#pragma unroll
+    for (int i = 0; i < 4; i++) tile[r][c4 + i] = w[i];
   }
   __syncthreads();
-  const int c = t & 63, run = t >> 6;
-  if (m0 + run * 32 >= M) return;
-  float v[32];
+  const int run = t & 7, c = t >> 3;                        // rows 16 run .. 16 run + 15 of columns 2 c, 2 c + 1: eight lanes write one 128-byte line
+  uint32_t w[16];
 #pragma unroll
-  for (int i = 0; i < 32; i++) v[i] = bf16_to_f(tile[run * 32 + i][c]);
-  uint32_t out[8];
-  const int e = mx_quant32(v, out);
-  const int kb = (m0 >> 5) + run;
-  u32x4* qo = (u32x4*)(q + (size_t)(n0 + c) * M + m0 + run * 32);
-  qo[0] = u32x4{out[0], out[1], out[2], out[3]}; qo[1] = u32x4{out[4], out[5], out[6], out[7]};
-  e8[(size_t)(n0 + c) * (M / 32) + kb] = (uint8_t)e;
-  if (packed) packed[((size_t)(kb >> 2) * N + n0 + c) * 4 + (kb & 3)] = (uint8_t)e;
+  for (int i = 0; i < 16; i++) w[i] = tile[run * 16 + i][c];
+  const bool live = m0 + run * 16 < M;                      // (M is a multiple of 32: both runs of a block are live or neither)
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    float v[16], amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) { v[i] = h ? bf16_hi(w[i]) : bf16_lo(w[i]); amax = fmaxf(amax, fabsf(v[i])); }
+    amax = fmaxf(amax, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, amax), 0xB1, 0xF, 0xF, true)));   // the other run of the block: lane ^ 1
+    const int e = mx_e8(amax);
+    const float s = mx_scale(e);
+    const size_t n = (size_t)(n0 + 2 * c + h);
+    u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = e4m3x4(v[4 * i] * s, v[4 * i + 1] * s, v[4 * i + 2] * s, v[4 * i + 3] * s);
+    const int kb = (m0 >> 5) + (run >> 1);
+    if (live) {
+      *(u32x4*)(q + n * M + m0 + run * 16) = o;
+      if (!(run & 1)) e8[n * (M / 32) + kb] = (uint8_t)e;
+    }
+    if (packed) {                                           // (M % 128 == 0: every run is live)
+      const int lane = t & 63, b = lane & 56;
+      const uint32_t pw = (uint32_t)(__shfl(e, b) | (__shfl(e, b + 2) << 8) | (__shfl(e, b + 4) << 16) | (__shfl(e, b + 6) << 24));
+      if (run == 0) ((uint32_t*)packed)[(size_t)(kb >> 2) * N + n] = pw;
+    }
+  }
 }
 
 // ------------------------------------------------------------------------------------------------ route
@@ -243,11 +231,6 @@ struct GemmArgs {
 #define GG_TILE 256
 #define GG_THREADS 512
 #define GG_STAGE_BYTES (2 * GG_TILE * 128 + 2 * GG_TILE * 4)   // operand tiles + one scale dword per row
-__device__ __forceinline__ int gg_slot_off(int R, int c) {       // byte offset inside a 256-row operand region of (row R, 16-byte chunk c)
-  const int sub = R >> 4, r = R & 15, p = c >> 2, g = c & 3;
-  return sub * 2048 + p * 1024 + ((16 * g + (r ^ (g + 4 * p))) << 4);
-}
-
 // Which tile workgroup b computes.  Consecutive workgroups go to different XCDs (the dispatcher deals them round-robin), so XCD x = b % 8
 // gets a contiguous run of the routed tiles: the N tiles of one row block (which share the activation tile) and the row blocks of one
 // expert (which share the weight tile) meet in one L2.  The routed tiles (rows below expert_off[E]) are shared evenly; the workgroups an
@@ -272,11 +255,6 @@ __device__ __forceinline__ int gg_tile_of_workgroup(int b, int nwg, int nact, bo
 //     store instruction writes eight whole 128-byte row segments.
 #define GG_OFF_MAX 4096                                           // expert offsets 0 .. E kept in LDS when E < GG_OFF_MAX
 #define GG_EPI_PITCH 144                                          // bytes per 64-column bf16 row in the epilogue slab (128 + 16: conflict-free 8-byte writes)
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {          // round to nearest even (tinygrad/dtype.py:224-226); one v_cvt_pk_bf16_f32
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
-}
 struct GGCur { const uint8_t* A; const uint8_t* B; const uint8_t* sc; int row0, tn, valid; };   // valid: rows of the tile that are not padding   // scalar (wave-uniform) state of one tile
 
 __device__ __forceinline__ void grouped_mxfp8_gemm_tile(const GemmArgs& g, uint8_t* smem, int* s_off) {
@@ -479,17 +457,26 @@ extern "C" __global__ __launch_bounds__(GG_THREADS) void tga_grouped_mxfp8_gemm_
 }
 
 // clamped, interleaved SwiGLU between the two grouped GEMMs (examples/mlperf/models/gpt_oss.py:94-98): bf16 in/out
-__global__ __launch_bounds__(256) void swiglu_interleaved_kernel(const uint16_t* __restrict__ h, long long rows, int two_inter, float limit, float alpha, uint16_t* __restrict__ y) {
-  const int inter = two_inter / 2;
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < rows * inter; i += (long long)gridDim.x * 256) {
-    const long long r = i / inter; const int c = (int)(i % inter);
-    float glu = bf16_to_f(h[r * two_inter + 2 * c]), lin = bf16_to_f(h[r * two_inter + 2 * c + 1]);
-    glu = fminf(glu, limit); lin = fminf(fmaxf(lin, -limit), limit);
-    // bf16 elementwise chain like the reference's bf16 tensors: each op rounds to bf16
-    const float sg = bf16_to_f(f_to_bf16(1.0f / (1.0f + expf(-bf16_to_f(f_to_bf16(alpha * glu))))));
-    const float a = bf16_to_f(f_to_bf16(glu * sg)), b = bf16_to_f(f_to_bf16(lin + 1.0f));
-    y[r * inter + c] = f_to_bf16(a * b);
+// Rows follow each other without a gap on both sides, so output i takes inputs 2 i and 2 i + 1 whatever the row length.  Four outputs per thread (a scalar loop over single
+// outputs came out of the compiler wrong for more than 2^24 of them, where its threads take a second trip, and moved 2 bytes per lane).
+__device__ __forceinline__ float swiglu1(float glu, float lin, float limit, float alpha) {
+  glu = fminf(glu, limit); lin = fminf(fmaxf(lin, -limit), limit);
+  // bf16 elementwise chain like the reference's bf16 tensors: each op rounds to bf16
+  const float sg = bf16_to_f(f_to_bf16(1.0f / (1.0f + expf(-bf16_to_f(f_to_bf16(alpha * glu))))));
+  const float a = bf16_to_f(f_to_bf16(glu * sg)), b = bf16_to_f(f_to_bf16(lin + 1.0f));
+  return a * b;
+}
+__global__ __launch_bounds__(256) void swiglu_interleaved_kernel(const uint16_t* __restrict__ h, const long long n, const long long n4, const float limit, const float alpha, uint16_t* __restrict__ y) {
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n4; i += (long long)gridDim.x * 256) {
+    const u32x4 v = ((const u32x4*)h)[i];
+    float o[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) { const uint32_t w = v[j]; o[j] = swiglu1(bf16_lo(w), bf16_hi(w), limit, alpha); }
+    ((u32x2*)y)[i] = u32x2{(uint32_t)f_to_bf16(o[0]) | ((uint32_t)f_to_bf16(o[1]) << 16), (uint32_t)f_to_bf16(o[2]) | ((uint32_t)f_to_bf16(o[3]) << 16)};
   }
+#pragma clang loop vectorize(disable) interleave(disable)
+  for (long long i = n4 * 4 + (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)      // the last n % 4, or all where a pointer is not aligned
+    y[i] = f_to_bf16(swiglu1(bf16_to_f(h[2 * i]), bf16_to_f(h[2 * i + 1]), limit, alpha));
 }
 
 // h[r, :] += bias[e(r), :] for the rows of every expert (examples/mlperf/models/gpt_oss.py:219-224: `+ (onehot @ bias.float()).cast(bf16)`
@@ -507,6 +494,12 @@ __global__ __launch_bounds__(256) void add_expert_bias_kernel(uint16_t* __restri
   }
 }
 
+// workgroups for n8 pieces of eight values, u per thread and trip: one trip each up to 8192 workgroups
+static int quantize_grid(long long n8, int u) {
+  const long long full = (n8 + 255) / 256, want = (full + u - 1) / u;
+  return (int)(want < 512 ? (full < 512 ? full : 512) : want < 8192 ? want : 8192);
+}
+
 extern "C" {
 
 int tga_quantize_mxfp8(const void* x, int x_is_bf16, int64_t rows, int64_t K, void* q, void* e8, void* packed, void* stream) {
@@ -514,8 +507,7 @@ int tga_quantize_mxfp8(const void* x, int x_is_bf16, int64_t rows, int64_t K, vo
   TGA_REQUIRE(rows >= 0 && K > 0 && K % 32 == 0, "tga_quantize_mxfp8: K=%lld must be a positive multiple of 32", (long long)K);
   TGA_REQUIRE(!packed || K % 128 == 0, "tga_quantize_mxfp8: packed scales need K %% 128 == 0");
   if (rows == 0) return 0;
-  const long long nb = rows * (K / 32);
-  const int grid = (int)((nb + 255) / 256 < 65536 ? (nb + 255) / 256 : 65536);
+  const int grid = quantize_grid(rows * (K / 8), x_is_bf16 ? 4 : 2);
   if (x_is_bf16) quantize_mxfp8_kernel<1><<<grid, 256, 0, (hipStream_t)stream>>>(x, nullptr, rows, (int)K, (uint8_t*)q, (uint8_t*)e8, (uint8_t*)packed);
   else quantize_mxfp8_kernel<0><<<grid, 256, 0, (hipStream_t)stream>>>(x, nullptr, rows, (int)K, (uint8_t*)q, (uint8_t*)e8, (uint8_t*)packed);
   TGA_LAUNCH_CHECK();
@@ -527,8 +519,7 @@ int tga_silu_mul_quantize_mxfp8(const void* x_w1_bf16, const void* x_w3_bf16, in
   TGA_REQUIRE(rows >= 0 && K > 0 && K % 32 == 0, "tga_silu_mul_quantize_mxfp8: K=%lld must be a positive multiple of 32", (long long)K);
   TGA_REQUIRE(!packed || K % 128 == 0, "tga_silu_mul_quantize_mxfp8: packed scales need K %% 128 == 0");
   if (rows == 0) return 0;
-  const long long nb = rows * (K / 32);
-  const int grid = (int)((nb + 255) / 256 < 65536 ? (nb + 255) / 256 : 65536);
+  const int grid = quantize_grid(rows * (K / 8), 2);
   quantize_mxfp8_kernel<2><<<grid, 256, 0, (hipStream_t)stream>>>(x_w1_bf16, x_w3_bf16, rows, (int)K, (uint8_t*)q, (uint8_t*)e8, (uint8_t*)packed);
   TGA_LAUNCH_CHECK();
   return 0;
@@ -669,9 +660,8 @@ int tga_add_expert_bias(void* h_bf16, const float* bias, const int32_t* expert_o
 int tga_swiglu_interleaved(const void* h_bf16, int64_t rows, int two_inter, float limit, float alpha, void* y_bf16, void* stream) {
   TGA_REQUIRE(h_bf16 && y_bf16 && two_inter > 0 && two_inter % 2 == 0, "tga_swiglu_interleaved: bad argument");
   if (rows == 0) return 0;
-  const long long n = rows * (two_inter / 2);
-  const int grid = (int)((n + 255) / 256 < 65536 ? (n + 255) / 256 : 65536);
-  swiglu_interleaved_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const uint16_t*)h_bf16, rows, two_inter, limit, alpha, (uint16_t*)y_bf16);
+  const long long n = rows * (two_inter / 2), n4 = ((uintptr_t)h_bf16 & 15) || ((uintptr_t)y_bf16 & 7) ? 0 : n / 4, wg = ((n4 ? n4 : n) + 255) / 256;
+  swiglu_interleaved_kernel<<<(int)(wg < 1 ? 1 : wg < 16384 ? wg : 16384), 256, 0, (hipStream_t)stream>>>((const uint16_t*)h_bf16, n, n4, limit, alpha, (uint16_t*)y_bf16);
   TGA_LAUNCH_CHECK();
   return 0;
 }
