@@ -364,6 +364,12 @@ int tga_grouped_mxfp8_gemm_routed(void* C, const void* A, const void* B, const v
  * (e.g. the second GEMM of a feed-forward whose first GEMM added an expert bias to them) these rows differ from it - combine never reads them. */
 int tga_grouped_mxfp8_gemm_counts(void* C, const void* A, const void* B, const void* x_e8, const void* w_e8, const int32_t* expert_off, const int32_t* counts,
                                   int64_t M, int64_t N, int64_t K, int n_experts, void* stream);
+/* The grouped MoE feed-forward of examples/mlperf/models/gpt_oss.py:213-226 as one call (moe_ffn.hip): x (T, D) bf16 normed activations, logits (T, E) float32, weights
+ * (E, 2 I, D) / (E, D, I) E4M3 with (.., K / 32) E8M0 scales, float32 biases -> out (T, D) bf16.  Values as route -> dispatch -> quantize -> grouped GEMM + bias -> swiglu ->
+ * quantize -> grouped GEMM + bias -> combine.  _plan: bytes of the caller's workspace, 0 when the sizes are outside the range (D, I multiples of 256, E <= 512, k <= 64). */
+int tga_moe_feed_forward_plan(int64_t T, int64_t D, int64_t I, int n_experts, int k, int64_t* nbytes);
+int tga_moe_feed_forward(const void* x_bf16, const float* logits, int64_t T, int64_t D, int64_t I, int n_experts, int k, const void* w_gate_up, const void* e8_gate_up,
+                         const float* b_gate_up, const void* w_down, const void* e8_down, const float* b_down, float limit, void* workspace, void* out_bf16, void* stream);
 /* Device symbol for a pre-compiled PROGRAM bound through Tensor.custom_kernel (tinygrad/tensor.py:390-396, extra/gemm/moe_gemm.py:36-48):
  *   extern "C" __global__ void tga_grouped_mxfp8_gemm_kernel(bf16* C, const fp8* A, const fp8* B, const uint32_t* x_si, const uint32_t* w_si,
  *                                                            const uint8_t* x_e8, const uint8_t* w_e8, const int32_t* expert_off,

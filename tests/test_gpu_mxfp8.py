@@ -260,3 +260,20 @@ def test_swiglu_beyond_one_trip_and_off_alignment(gpu):
   assert (y == y[0]).all()
   off = gpu.Buffer.from_numpy(np.concatenate([np.zeros(1, np.uint16), unit[0]])).view(2, (1, 2 * 4099), np.uint16)
   np.testing.assert_array_equal(moe.swiglu(off).numpy()[0], y[0])
+
+@pytest.mark.parametrize("T,D,I,E,k", [(1, 256, 256, 8, 1), (1, 512, 256, 128, 8), (33, 256, 512, 3, 3), (64, 512, 256, 16, 4), (65, 256, 256, 65, 2), (129, 256, 256, 200, 5), (300, 512, 256, 4, 2), (700, 256, 256, 2, 1)])
+def test_moe_feed_forward_at_tile_edges(gpu, T, D, I, E, k):
+  """The fused feed-forward at one token, one and two routing workgroups, more experts than a wave has lanes, experts of no rows, of fewer rows than a tile and of several tiles (both
+  tile heights), against the reference's per-expert loop restated in the oracle.  Bar as in the composition test above: the two branches round to bf16 at different points."""
+  from tinygrad_amd import moe
+  rng = np.random.default_rng(T + E)
+  inp = moe.to_bf16_bits(rng.standard_normal((T, D)).astype(np.float32))
+  logits = rng.standard_normal((T, E)).astype(np.float32) + np.linspace(0, 3, E, dtype=np.float32)
+  wgu, wdn = (rng.standard_normal((E, 2 * I, D)) * D ** -0.5).astype(np.float32), (rng.standard_normal((E, D, I)) * I ** -0.5).astype(np.float32)
+  bgu, bdn = (rng.standard_normal((E, 2 * I)) * 0.1).astype(np.float32), (rng.standard_normal((E, D)) * 0.1).astype(np.float32)
+  (gq, ge), (dq, de) = omx.quantize_mxfp8(wgu), omx.quantize_mxfp8(wdn)
+  B = gpu.Buffer.from_numpy
+  ref = omx.moe_feed_forward_loop(moe.from_bf16_bits(inp), logits, k, gq, ge, bgu, dq, de, bdn)
+  got = moe.from_bf16_bits(moe.moe_feed_forward(B(inp), B(logits), k, (B(gq), B(ge)), B(bgu), (B(dq), B(de)), B(bdn)).numpy())
+  assert np.isfinite(got).all() and np.abs(got - ref).mean() / np.abs(ref).mean() < 1e-2
+  np.testing.assert_allclose(got, ref, rtol=0.05, atol=0.02 * np.abs(ref).max())

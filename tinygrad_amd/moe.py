@@ -2,6 +2,7 @@
 extra/gemm/cdna_asm_gemm.py): route / dispatch / combine, quantize_mxfp8, grouped_mx_gemm.  bf16 and E4M3 tensors are device
 Buffers of uint16 / uint8 (numpy has neither type); shapes follow the reference."""
 from __future__ import annotations
+import ctypes
 from dataclasses import dataclass
 import numpy as np
 from tinygrad_amd import runtime as rt
@@ -145,6 +146,14 @@ def moe_feed_forward(inp: Buffer, logits: Buffer, experts_per_tok: int, w_gate_u
   T, D = inp.shape
   E, N2, _ = w_gate_up[0].shape
   assert D % 256 == 0 and N2 % 256 == 0 and (N2 // 2) % 256 == 0, f"dim {D}, 2*inter {N2} and inter {N2 // 2} must be multiples of 256"
+  need = ctypes.c_int64(0)
+  rt.check(rt.lib().tga_moe_feed_forward_plan(T, D, N2 // 2, E, experts_per_tok, ctypes.byref(need)))
+  ptrs = [b.ptr for b in (inp, *w_gate_up, b_gate_up, *w_down, b_down)]
+  if need.value and all(p % 16 == 0 for p in ptrs):             # one native call: five launches over compact rows, no padding rows (whatever routed_only says: combine reads none)
+    ws, out = Buffer((need.value,), np.uint8), Buffer((T, D), np.uint16)
+    rt.check(rt.lib().tga_moe_feed_forward(inp.ptr, logits.ptr, T, D, N2 // 2, E, experts_per_tok, w_gate_up[0].ptr, w_gate_up[1].ptr, b_gate_up.ptr, w_down[0].ptr, w_down[1].ptr,
+                                           b_down.ptr, swiglu_limit, ws.ptr, out.ptr, stream))
+    return out                                                  # (ws: a freed block is handed out again only after the device has been synchronised)
   r = route(logits, experts_per_tok, E, stream)
   xg = dispatch(inp, r, stream)
   cnt = r.counts if routed_only else None                     # padding rows are never gathered by combine: their 16-row groups are not multiplied

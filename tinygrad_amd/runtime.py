@@ -52,6 +52,8 @@ def _declare(lib):
     "tga_quantize_mxfp8": [vp, i, i64, i64, vp, vp, vp, vp],
     "tga_silu_mul_quantize_mxfp8": [vp, vp, i64, i64, vp, vp, vp, vp],
     "tga_transpose_quantize_mxfp8": [vp, i64, i64, vp, vp, vp, vp],
+    "tga_moe_feed_forward_plan": [i64, i64, i64, i, i, ctypes.POINTER(i64)],
+    "tga_moe_feed_forward": [vp, vp, i64, i64, i64, i, i, vp, vp, vp, vp, vp, vp, ctypes.c_float, vp, vp, vp],
     "tga_moe_route": [vp, i, i, i, vp, vp, vp, vp, vp, vp, vp],
     "tga_moe_route_static": [vp, i, i, i, vp, vp, vp, vp, vp, vp],
     "tga_moe_dispatch": [vp, vp, vp, vp, i, i, i, i64, i, vp, vp],
