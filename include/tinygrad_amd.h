@@ -398,6 +398,17 @@ int tga_mfma_peak(int n_workgroups, int loops, float* scratch, void* stream);
  * constant `amp`; TGA_MXFP4 ignores amp: uniform E2M1 codes with E8M0 bytes uniform in [119, 123] (block scales 2^-8 .. 2^-4). */
 int tga_synth_weights(int ggml_type, void* out, int64_t n_elements, uint32_t seed, float amp, void* stream);
 
+/* ---- many activation rows (qgemm_rows.hip): y = x . W^T for fp16 rows of any number, plain / + residual / silu(gate) * up, up to three matrices that share the rows; the
+ * workspace (may be NULL) takes the partial tiles of a split K.  K a multiple of 128 (superblock types: 256). ---- */
+int tga_qlinear_many(int ggml_type, int nseg, const void* const* w, void* const* y, const int64_t* n, const void* x_f16, int y_dtype, int64_t M, int64_t K, int epilogue,
+                     const float* resid, void* workspace, int64_t workspace_bytes, void* stream);
+int tga_rows_format_ok(int ggml_type, int64_t K, int* ok);
+/* A prefill step of any number of rows (prefill.hip; model.py:464, 476-481): positions pos0 .. pos0 + P - 1 of nseq sequences through all blocks, keys and values appended to
+ * the caches.  model / blocks: tables of int64 (pointers as integers) in the order of the PM_ / PB_ enumerations there; tokens: (nseq, P) ids on the device.
+ * _plan: bytes of the caller's workspace for that many rows (nseq * P). */
+int tga_prefill_plan(const int64_t* model, int64_t rows, int64_t* nbytes);
+int tga_prefill_step(const int64_t* model, const int64_t* blocks, const int32_t* tokens, int64_t nseq, int64_t P, int64_t pos0, void* workspace, void* state, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,112 @@
+"""Prefill steps of many rows on the GPU: tga_qlinear_many for every format at tile edges against a float64 product over the dequantized (fp16-rounded) weights, and whole steps - one
+sequence and several, dense and MoE, one step and a prompt cut into several - against the same models prefilled position by position."""
+import ctypes
+import numpy as np, pytest
+from oracle import ggml as og, linear as ol, llm as ollm
+from tinygrad_amd import synth
+
+pytestmark = pytest.mark.gpu
+FORMATS = ["Q4_0", "Q8_0", "F16", "MXFP4", "Q4_K", "Q5_K", "Q6_K", "IQ4_XS", "Q4_1", "Q5_0", "Q5_1"]
+
+def _weight(rng, rt, t, n, k):
+  if t == rt.F16:
+    w = (rng.standard_normal((n, k)) * k ** -0.5).astype(np.float16)
+    return w.view(np.uint8).reshape(-1), w.astype(np.float32)
+  raw = synth.random_blocks(rng, t, n, k, sigma=0.0002 if t == rt.IQ4_XS else 0.003)
+  return raw, og.ggml_data_to_tensor(raw, n * k, t).reshape(n, k).astype(np.float16).astype(np.float32)      # (the kernel multiplies fp16-rounded weights, model.py:376)
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_many_rows_linear_at_tile_edges(gpu, fmt):
+  """Rows 1 / 31 / 33 / 64 / 65 / 129 and outputs 16 / 127 / 129 / 300 around the tile heights, K of one and several steps; plain fp32 and fp16 results, + residual in place,
+  silu(gate) * up, three matrices in one launch, with and without a workspace (split K).  Bar: float32 accumulation of exact products of fp16 values, K <= 768: each sum carries
+  at most K 2^-24 relative to its absolute sum, 5e-5 of the largest result; fp16 results one more rounding, 2^-11.  Where a weight is a product and a difference of scales (K-quants,
+  IQ4_XS, Q4_1, Q5_1) the kernel forms it with fused multiply-adds and the oracle with separate roundings: some weights then round to the neighbouring fp16 value, 2^-10 relative each,
+  which bounds a sum by 2^-10 of its absolute sum; the linears' common bar of 1e-3 of the largest result holds them."""
+  from tinygrad_amd import runtime as rt
+  t = getattr(rt, fmt)
+  rng = np.random.default_rng(t)
+  ws = rt.Buffer((8 << 20,), np.uint8)
+  def call(layers, x, outs, ydt, epi=0, resid=None, work=True):
+    n = len(layers); VP = ctypes.c_void_p * n
+    rt.check(rt.lib().tga_qlinear_many(t, n, VP(*[l[0].ptr for l in layers]), VP(*[(outs[i].ptr if i < len(outs) else None) for i in range(n)]), (ctypes.c_int64 * n)(*[l[1] for l in layers]),
+                                       x.ptr, ydt, x.shape[0], x.shape[1], epi, resid.ptr if resid is not None else None, ws.ptr if work else None, ws.nbytes if work else 0, None))
+  bar = 1e-3 if fmt in ("Q4_K", "Q5_K", "IQ4_XS", "Q4_1", "Q5_1") else 5e-5
+  def close(got, ref, f16=False): assert ol.rel_err(got.astype(np.float32), ref) <= bar + (2.0 ** -11 if f16 else 0)
+  for m, n, k in ((1, 16, 256), (31, 127, 768), (33, 300, 256), (64, 129, 512), (65, 16, 768), (129, 300, 512)):
+    raw, w = _weight(rng, rt, t, n, k); raw2, w2 = _weight(rng, rt, t, n, k)
+    wb, wb2 = rt.Buffer.from_numpy(raw), rt.Buffer.from_numpy(raw2)
+    x = synth.activations(rng, m, k, np.float16); xb = rt.Buffer.from_numpy(x)
+    ref, ref2 = ol.linear_f64(x.astype(np.float32), w), ol.linear_f64(x.astype(np.float32), w2)
+    for work in (True, False):
+      y = rt.Buffer((m, n), np.float32); call([(wb, n)], xb, [y], rt.F32, work=work); close(y.numpy(), ref)
+      h = rt.Buffer((m, n), np.float16); call([(wb, n)], xb, [h], rt.F16, work=work); close(h.numpy(), ref, True)
+      r = rng.standard_normal((m, n)).astype(np.float32); y = rt.Buffer.from_numpy(r); call([(wb, n)], xb, [y], rt.F32, 1, y, work=work); close(y.numpy(), ref + r)
+    y = rt.Buffer((m, n), np.float32); call([(wb, n), (wb2, n)], xb, [y], rt.F32, 2)
+    sw = ref / (1 + np.exp(-ref)) * ref2
+    assert ol.rel_err(y.numpy(), sw) <= 4 * bar                                    # (two such sums and the exponential of one of them multiplied)
+  ns, k, m = (128, 64, 80), 512, 70
+  parts = [_weight(rng, rt, t, n, k) for n in ns]
+  x = synth.activations(rng, m, k, np.float16); xb = rt.Buffer.from_numpy(x)
+  bufs = [rt.Buffer.from_numpy(p[0]) for p in parts]
+  for work in (True, False):
+    outs = [rt.Buffer((m, n), np.float32) for n in ns]
+    call(list(zip(bufs, ns)), xb, outs, rt.F32, work=work)
+    for o, p in zip(outs, parts): close(o.numpy(), ol.linear_f64(x.astype(np.float32), p[1]))
+  assert rt.lib().tga_qlinear_many(t, 1, (ctypes.c_void_p * 1)(bufs[0].ptr), (ctypes.c_void_p * 1)(outs[0].ptr), (ctypes.c_int64 * 1)(128), xb.ptr, rt.F32, m, 96, 0, None, None, 0, None) != 0
+
+DENSE = dict(num_blocks=2, dim=512, hidden_dim=768, n_heads=8, n_kv_heads=2, norm_eps=1e-5, vocab_size=512, head_dim=64, rope_theta=500000.0)
+DENSE128 = dict(num_blocks=2, dim=768, hidden_dim=512, n_heads=6, n_kv_heads=6, norm_eps=1e-5, vocab_size=512, head_dim=128, rope_theta=10000.0)
+MOE = dict(num_blocks=2, dim=256, hidden_dim=256, n_heads=4, n_kv_heads=4, norm_eps=1e-5, vocab_size=512, head_dim=64, rope_theta=10000.0, qk_norm=256, num_experts=8, num_experts_per_tok=2)
+
+def _model(cfg, seed, ctx=320, batch=0, **kw):
+  from tinygrad_amd.llm import BatchedTransformer, Transformer, TransformerConfig, synth_state, synth_state_moe
+  c = TransformerConfig(max_context=ctx, **cfg)
+  sd = synth_state_moe(c, seed=seed) if c.num_experts else synth_state(c, seed=seed, **kw)
+  return BatchedTransformer(c, sd, batch, max_new=8) if batch else Transformer(c, sd, max_new=8)
+
+@pytest.mark.parametrize("cfg,kw", [(DENSE, {}), (DENSE, {"q4_k_m": True}), (DENSE128, {"linear_type": 8}), (DENSE128, {"linear_type": 1})], ids=["gqa4-hd64-q4_0", "gqa4-hd64-q4_k_m", "mha-hd128-q8_0", "mha-hd128-f16"])
+@pytest.mark.parametrize("n,rows", [(18, 2048), (65, 2048), (130, 2048), (300, 2048), (300, 100)])
+def test_prefill_of_many_rows_vs_position_by_position(gpu, monkeypatch, cfg, kw, n, rows):
+  """Prompts around the row tiles of the attention (16 / 64) and of the linears, in one step and cut into steps of a hundred rows that attend to the cache of the ones before: caches within fp16
+  rounding of the model prefilled token by token (2e-3, the bar of the chunked prefill), nothing written beyond the prompt, logits of the next step within 2e-3 (both sides
+  are within 1e-3 of the reference's numerics)."""
+  from tinygrad_amd import llm
+  monkeypatch.setattr(llm, "MANY_ROWS", rows)
+  a, b = _model(cfg, 5, **kw), _model(cfg, 5, **kw)
+  b.prefill_chunk = 1
+  prompt = [int(t) for t in np.random.default_rng(n).integers(0, cfg["vocab_size"], size=n)]
+  for m in (a, b): m.prefill(prompt)
+  assert (a._chunker or a._tail_chunkers[16]).x is None and a.prefill_steps == n - 1     # (no plain step was run)
+  for ba, bb in zip(a.blk, b.blk):
+    for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)):
+      ca, cb = ca.numpy().astype(np.float32), cb.numpy().astype(np.float32)
+      assert ol.rel_err(ca[:, :n - 1], cb[:, :n - 1]) <= 2e-3 and not ca[:, n - 1:].any()
+  for m in (a, b): m.decode_step()
+  assert ol.rel_err(a.logits(), b.logits()) <= 2e-3
+  longer = prompt[:n - 4] + [7] * 20                                               # a follow-up that keeps the cached prefix
+  for m in (a, b): m.prefill(longer); m.decode_step(); m.check_state()
+  assert ol.rel_err(a.logits(), b.logits()) <= 2e-3
+
+@pytest.mark.parametrize("cfg,B,n", [(DENSE, 3, 7), (DENSE, 5, 70), (DENSE128, 2, 33), (MOE, 4, 20), (MOE, 1, 40)], ids=["dense-3x7", "dense-5x70", "hd128-2x33", "moe-4x20", "moe-1x40"])
+@pytest.mark.parametrize("rows", [2048, 24])
+def test_batched_prefill_of_many_rows_vs_step_by_step(gpu, monkeypatch, cfg, B, n, rows):
+  """The prompts of several sequences as steps of (sequences x positions) rows against the lockstep steps: every cache within 2e-3 except rows behind a router near-tie (MoE), whose share is
+  bounded, and the logits of the first decoded token."""
+  from tinygrad_amd import llm
+  prompts = np.random.default_rng(B + n).integers(0, cfg["vocab_size"], size=(B, n)).tolist()
+  a, b = _model(cfg, 9, 128, B), _model(cfg, 9, 128, B)
+  monkeypatch.setattr(llm, "MANY_ROWS", rows)
+  a.prefill(prompts)
+  assert a._rows_ws is not None
+  monkeypatch.setattr(llm, "MANY_ROWS_MIN", 1 << 30)
+  b.prefill(prompts)
+  assert b._rows_ws is None
+  for ba, bb in zip(a.blk, b.blk):
+    for nm in ("cache_k", "cache_v"):
+      ca, cb = ba[nm].numpy().astype(np.float32), bb[nm].numpy().astype(np.float32)
+      off = np.abs(ca - cb).max(axis=(1, 3)) / np.abs(cb).max()                    # per (sequence, position)
+      assert not ca[:, :, n - 1:].any() and (off > 2e-3).mean() <= (0.05 if "num_experts" in cfg else 0)
+  for m in (a, b): m.decode_step(); m.check_state()
+  la, lb = a.logits(), b.logits()
+  bad = np.abs(la - lb).max(axis=1) / np.abs(lb).max()
+  assert (bad > 2e-3).sum() <= ((B + 3) // 4 if "num_experts" in cfg else 0), bad

@@ -1,0 +1,366 @@
+// A prefill step of any number of rows: the positions pos0 .. pos0 + P - 1 of one or more sequences go through all blocks together (the reference's chunked prefill,
+// tinygrad/llm/model.py:464, 476-481, with the prompt as one chunk), every linear as ONE pass over its weights (qgemm_rows.h).  Per block: norm -> q / k / v -> rotation +
+// append -> attention -> attn_output (+ residual) -> norm -> gate / up + SwiGLU -> down (+ residual): nine launches, or for a MoE block norm -> router logits -> gating ->
+// grouping -> selected experts' gate / up + SwiGLU -> down -> weighted sum (+ residual), model.py:110-135.  The launches are issued by one native call.
+// MI355X, prompt to first logits: 8B-arch Q4_0 of 1024 tokens 42.6 ms (steps of 128 rows, qgemm64.hip) -> 23.8; OLMoE-arch of 512 tokens 64.0 (steps of 16 rows, an expert GEMV per
+// token and slot) -> 5.9; four 8B-arch Q4_K_M sequences of 128 tokens 334 (one lockstep step per position) -> 17.0.
+#include "qgemm_rows.h"
+#include "decode.h"
+#include "moe_gate.h"
+#include <string.h>
+
+int tga_rows_fmt(int ggml_type, int64_t K);                                              // qgemm_rows.hip
+int64_t tga_rows_row_bytes(int fmt, int64_t K);
+int tga_rows_dispatch(int fmt, const RowsArgs& a, int tt, unsigned grid, hipStream_t s);
+
+// ------------------------------------------------------------------------------------------------ rotation + append
+// One workgroup per row.  q is rotated (after its norm) and leaves as TWO fp16 values per element, the rounded value and what the rounding left over, so that the matrix-core
+// scores see the float32 query; k is rotated into the cache, v copied.  The rotation is apply_rope's (model.py:29-33) written as one rounded product and one fused multiply-add,
+// like every kernel that rotates, so a cache row has the same bits whichever path appended it.  norm: 0 none, 1 RMSNorm over the whole q / k rows (model.py:169), 2 per head (:180).
+struct RopeArgs {
+  const float* q; const float* k; const float* v; const float* qn; const float* kn; const float* rope;
+  uint16_t* qh; uint16_t* ql; uint16_t* ck; uint16_t* cv; int* zero;      // zero: n_zero counters cleared for the launches behind this one
+  int H, KV, hd, max_ctx, P, pos0, norm, n_zero; float eps;
+};
+__global__ __launch_bounds__(256) void rows_rope_kernel(const RopeArgs a) {
+  __shared__ float red[8];
+  const int r = blockIdx.x, z = r / a.P, pos = a.pos0 + r % a.P, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = a.hd >> 1;
+  const int nq = a.H * a.hd, nk = a.KV * a.hd;
+  if (r == 0) for (int i = tid; i < a.n_zero; i += 256) a.zero[i] = 0;
+  const float* q = a.q + (size_t)r * nq; const float* k = a.k + (size_t)r * nk; const float* v = a.v + (size_t)r * nk;
+  float qs = 1.f, ks = 1.f;
+  if (a.norm == 1) {
+    float s0 = 0.f, s1 = 0.f;
+    for (int i = tid; i < (nq >> 2); i += 256) { const f32x4 x = ((const f32x4*)q)[i]; s0 += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w; }
+    for (int i = tid; i < (nk >> 2); i += 256) { const f32x4 x = ((const f32x4*)k)[i]; s1 += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w; }
+    s0 = wave_sum(s0); s1 = wave_sum(s1);
+    if (lane == 0) { red[wave] = s0; red[4 + wave] = s1; }
+    __syncthreads();
+    qs = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)nq + a.eps);
+    ks = 1.0f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)nk + a.eps);
+  }
+  const float* rr = a.rope + (size_t)pos * a.hd;
+  const size_t crow = ((size_t)z * a.KV * a.max_ctx + pos) * a.hd, cstep = (size_t)a.max_ctx * a.hd;
+  const bool live = lane < half;                                          // (half is 32 or 64)
+  const int i = live ? lane : half - 1;
+  const float c = rr[i], s = rr[half + i];
+  for (int h = wave; h < a.H + a.KV; h += 4) {
+    const bool isq = h < a.H;
+    const int hh = isq ? h : h - a.H;
+    const float* src = isq ? q + hh * a.hd : k + hh * a.hd;
+    float x1 = src[i], x2 = src[half + i];
+    if (a.norm) {
+      float sc = isq ? qs : ks;
+      if (a.norm == 2) sc = 1.0f / sqrtf(wave_sum(live ? x1 * x1 + x2 * x2 : 0.f) / (float)a.hd + a.eps);
+      const float* w = isq ? a.qn : a.kn;
+      const int wo = a.norm == 2 ? 0 : hh * a.hd;
+      x1 = (x1 * sc) * w[wo + i]; x2 = (x2 * sc) * w[wo + half + i];
+    }
+    const float lo = __builtin_fmaf(x1, c, -(x2 * s)), hi = __builtin_fmaf(x2, c, x1 * s);
+    if (!live) continue;
+    if (isq) {
+      const size_t o = (size_t)r * nq + hh * a.hd + i;
+      const _Float16 l16 = (_Float16)lo, h16 = (_Float16)hi;
+      a.qh[o] = __builtin_bit_cast(uint16_t, l16); a.qh[o + half] = __builtin_bit_cast(uint16_t, h16);
+      a.ql[o] = (uint16_t)f2h_bits(lo - (float)l16); a.ql[o + half] = (uint16_t)f2h_bits(hi - (float)h16);
+    } else {
+      uint16_t* d = a.ck + crow + hh * cstep;
+      d[i] = (uint16_t)f2h_bits(lo); d[half + i] = (uint16_t)f2h_bits(hi);
+    }
+  }
+  for (int e = tid; e < nk; e += 256) { const int hh = e / a.hd; a.cv[crow + hh * cstep + (e - hh * a.hd)] = (uint16_t)f2h_bits(v[e]); }
+}
+
+// ------------------------------------------------------------------------------------------------ attention
+// Causal attention of the rows over the cache (their own keys included): workgroup = 64 rows of one query head, wave = 16 of them, tiles of 64 keys with a running maximum.
+// S^T = K Q^T: keys as A operand from LDS (rows of head_dim values, 16-byte pieces XORed with the key), the rotated queries as two fp16 B operands held in registers.
+// O^T = V^T P^T: the probabilities as a rounded value and its remainder, so that they count in float32 like the decode kernels' (each product once more on matrix cores
+// that are far from busy here); the eight keys a lane holds after the first product are taken as they are, and V is written to LDS transposed with its keys in that order, two keys
+// per dword, pieces XORed with the dimension.  The next tile is fetched while this one is multiplied.  flattened workgroup = (kv head, sequence) innermost: with eight
+// kv heads all readers of a head's rows run on one XCD and share its L2; the longest row tiles come first.
+struct RowsAttnArgs { const uint16_t* qh; const uint16_t* ql; const uint16_t* ck; const uint16_t* cv; uint16_t* out; int H, KV, max_ctx, P, pos0, nseq, qtiles; float scale; };
+
+template <int HD>
+__global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
+  constexpr int NJ = HD / 32, NH = HD / 16, PC = HD / 8, IK = HD / 32, IV = HD / 64;     // 16-byte pieces per row; loads per thread and tile
+  __shared__ __attribute__((aligned(16))) uint8_t kl[64 * HD * 2];
+  __shared__ __attribute__((aligned(16))) uint8_t vl[HD * 128];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, c = lane & 15;
+  const int group = a.H / a.KV, kz = a.KV * a.nseq;
+  int b = blockIdx.x;
+  const int kvz = b % kz; b /= kz;
+  const int hh = b % group, qt = a.qtiles - 1 - b / group;
+  const int kvh = kvz % a.KV, z = kvz / a.KV, head = kvh * group + hh;
+  const int row_first = qt * 64, nq = a.H * HD;
+  const int wrow = row_first + wave * 16;                                 // first row of this wave
+  const int row = min(wrow + c, a.P - 1), pos = a.pos0 + row;
+  const uint16_t* ck = a.ck + ((size_t)z * a.KV + kvh) * a.max_ctx * HD; const uint16_t* cv = a.cv + ((size_t)z * a.KV + kvh) * a.max_ctx * HD;
+  u32x4 qb[NJ], qr[NJ];
+  const size_t qo = ((size_t)z * a.P + row) * nq + head * HD + 8 * g;
+#pragma unroll
+  for (int j = 0; j < NJ; j++) { qb[j] = *(const u32x4*)(a.qh + qo + 32 * j); qr[j] = *(const u32x4*)(a.ql + qo + 32 * j); }
+  const int last_wg = a.pos0 + min(row_first + 63, a.P - 1), ntiles = last_wg / 64 + 1;      // keys 0 .. last_wg are visible to some row of the workgroup
+  const int last_wave = a.pos0 + min(wrow + 15, a.P - 1), first_wave = a.pos0 + min(wrow, a.P - 1);
+  u32x4 kq[IK], vq[IV][2];
+  const int vchunk = tid % PC, vpair = tid / PC;                          // V: dimensions 8 vchunk .. + 7 of keys 2 pair, 2 pair + 1
+  auto fetch = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < IK; i++) {
+      const int it = tid + 256 * i, key = min(64 * t + it / PC, a.max_ctx - 1);               // (rows beyond the cache are masked: they lie beyond every position)
+      kq[i] = *(const u32x4*)(ck + (size_t)key * HD + (it % PC) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < IV; i++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) { const int key = min(64 * t + 2 * (vpair + i * (256 / PC)) + h, a.max_ctx - 1); vq[i][h] = *(const u32x4*)(cv + (size_t)key * HD + vchunk * 8); }
+  };
+  auto put = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < IK; i++) { const int it = tid + 256 * i, key = it / PC; *(u32x4*)(kl + key * HD * 2 + (((it % PC) ^ (key & 7)) << 4)) = kq[i]; }
+#pragma unroll
+    for (int i = 0; i < IV; i++) {
+      const int j = 2 * (vpair + i * (256 / PC)), slot = (j & 32) + 8 * ((j & 15) >> 2) + 4 * ((j >> 4) & 1) + (j & 3);
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const uint32_t lo = vq[i][0][e >> 1], hi = vq[i][1][e >> 1];
+        const int d = vchunk * 8 + e;
+        *(uint32_t*)(vl + d * 128 + (((slot >> 3) ^ ((d ^ (d >> 3)) & 7)) << 4) + (slot & 7) * 2) = (e & 1) ? pack_odd(lo, hi) : pack_even(lo, hi);
+      }
+    }
+  };
+  v4f32 O[NH];
+#pragma unroll
+  for (int h = 0; h < NH; h++) O[h] = v4f32{0.f, 0.f, 0.f, 0.f};
+  float M = -INFINITY, L = 0.f;
+  fetch(0);
+  for (int t = 0; t < ntiles; t++) {
+    put();
+    if (t + 1 < ntiles) fetch(t + 1);
+    __syncthreads();
+    if (64 * t <= last_wave) {
+      v4f32 sc[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        sc[k] = v4f32{0.f, 0.f, 0.f, 0.f};
+        const int key = 16 * k + c;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+          const v8f16 ka = *(const v8f16*)(kl + key * HD * 2 + (((4 * j + g) ^ (key & 7)) << 4));
+          sc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, __builtin_bit_cast(v8f16, qr[j]), sc[k], 0, 0, 0);
+          sc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, __builtin_bit_cast(v8f16, qb[j]), sc[k], 0, 0, 0);
+        }
+      }
+      float m = -INFINITY;
+      const bool mask = 64 * t + 63 > first_wave;
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float s = sc[k][i] * a.scale;                                    // (log2(e) folded into the scale)
+          if (mask) s = 64 * t + 16 * k + 4 * g + i <= pos ? s : -INFINITY;
+          sc[k][i] = s; m = fmaxf(m, s);
+        }
+      m = fmaxf(m, __shfl_xor(m, 16)); m = fmaxf(m, __shfl_xor(m, 32));
+      const float mn = fmaxf(M, m);                                        // (finite: key 0 is visible to every row)
+      const float alpha = __builtin_amdgcn_exp2f(M - mn);
+      float l = 0.f;
+      u32x4 ph[2], pl[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+          const int k = 2 * u + (w >> 1), i = 2 * (w & 1);
+          const float p0 = __builtin_amdgcn_exp2f(sc[k][i] - mn), p1 = __builtin_amdgcn_exp2f(sc[k][i + 1] - mn);
+          l += p0 + p1;
+          const _Float16 h0 = (_Float16)p0, h1 = (_Float16)p1;
+          ph[u][w] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
+          pl[u][w] = f2h_bits(p0 - (float)h0) | (f2h_bits(p1 - (float)h1) << 16);
+        }
+      l += __shfl_xor(l, 16); l += __shfl_xor(l, 32);
+      L = L * alpha + l; M = mn;
+#pragma unroll
+      for (int h = 0; h < NH; h++) {
+        v4f32 o = O[h] * alpha;
+        const int d = 16 * h + c;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const v8f16 va = *(const v8f16*)(vl + d * 128 + (((4 * u + g) ^ ((d ^ (d >> 3)) & 7)) << 4));
+          o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, __builtin_bit_cast(v8f16, pl[u]), o, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, __builtin_bit_cast(v8f16, ph[u]), o, 0, 0, 0);
+        }
+        O[h] = o;
+      }
+    }
+    __syncthreads();
+  }
+  if (wrow + c < a.P) {
+    const float inv = 1.0f / L;
+    uint16_t* o = a.out + ((size_t)z * a.P + wrow + c) * nq + head * HD + 4 * g;
+#pragma unroll
+    for (int h = 0; h < NH; h++) *(u32x2*)(o + 16 * h) = u32x2{f2h_bits(O[h][0] * inv) | (f2h_bits(O[h][1] * inv) << 16), f2h_bits(O[h][2] * inv) | (f2h_bits(O[h][3] * inv) << 16)};
+  }
+}
+
+// ------------------------------------------------------------------------------------------------ grouping of the routed rows by expert
+#define PF_MAX_E 512
+// One wave per token: selection and weights (gate_topk_wave), and this assignment's place among the rows of its expert.  The order of places is that of arrival: a row's
+// values do not depend on its place, and the weighted sum of a token runs over its slots in order.
+__global__ __launch_bounds__(256) void rows_gate_kernel(const float* __restrict__ logits, int R, int E, int k, int gating, int norm_topk, float scale, int* __restrict__ sel,
+                                                        float* __restrict__ probs, int* __restrict__ counts, int* __restrict__ place) {
+  __shared__ float sc[4][PF_MAX_E]; __shared__ float tmp[4][192];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, t = blockIdx.x * 4 + wave;
+  if (t >= R) return;
+  gate_topk_wave(logits + (size_t)t * E, E, k, gating, norm_topk, scale, sel + (size_t)t * k, probs + (size_t)t * k, sc[wave], tmp[wave], lane);
+  if (lane < k) { const int e = ((const int*)tmp[wave])[lane]; place[(size_t)t * k + lane] = atomicAdd(&counts[e], 1); }
+}
+// Offsets of the experts' rows, the list of tiles of tt rows, and every row's token and assignment; each workgroup scans the counts for itself, the first writes the lists
+__global__ __launch_bounds__(512) void rows_group_kernel(const int* __restrict__ counts, const int* __restrict__ sel, const int* __restrict__ place, int R, int E, int k, int tt,
+                                                         int* __restrict__ off, int2* __restrict__ tiles, int* __restrict__ n_tiles, int* __restrict__ row_tok, int* __restrict__ row_dst) {
+  __shared__ int s_off[PF_MAX_E + 1], s_t[8], s_o[8];
+  const int e = threadIdx.x, lane = e & 63, wave = e >> 6;
+  const int c = e < E ? counts[e] : 0, nt = (c + tt - 1) / tt;
+  int io = c, it = nt;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) { const int uo = __shfl_up(io, o), ut = __shfl_up(it, o); if (lane >= o) { io += uo; it += ut; } }
+  if (lane == 63) { s_o[wave] = io; s_t[wave] = it; }
+  __syncthreads();
+  for (int w = 0; w < wave; w++) { io += s_o[w]; it += s_t[w]; }
+  if (e < E) s_off[e] = io - c;
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    if (e < E) {
+      off[e] = io - c;
+      for (int i = 0; i < nt; i++) tiles[it - nt + i] = int2{e, i * tt};
+      if (e == E - 1) { off[E] = io; *n_tiles = it; }
+    }
+  }
+  const int n = R * k;
+  for (int j = blockIdx.x * 512 + threadIdx.x; j < n; j += gridDim.x * 512) {
+    const int row = s_off[sel[j]] + place[j];
+    row_tok[row] = j / k; row_dst[row] = j;
+  }
+}
+
+// ------------------------------------------------------------------------------------------------ the step
+// Indices of the int64 tables a caller passes (pointers as integers)
+enum { PM_NBLOCKS, PM_DIM, PM_HEADS, PM_KV, PM_HD, PM_MAXCTX, PM_EMB, PM_EMB_TYPE, PM_ROPE, PM_EXPERTS, PM_TOPK, PM_GATING, PM_NORM_TOPK, PM_QKNORM, PM_HIDDEN, PM_DENSE_HIDDEN, PM_EPS_BITS, PM_SCALE_BITS, PM_COUNT };
+enum { PB_ATTN_NORM, PB_FFN_NORM, PB_QN, PB_KN, PB_CK, PB_CV, PB_MOE, PB_WQ, PB_WK, PB_WV, PB_WO, PB_GATE, PB_UP, PB_DOWN, PB_ROUTER, PB_TQ, PB_TK, PB_TV, PB_TO, PB_TGATE, PB_TDOWN, PB_COUNT };
+
+static float bits_f(int64_t b) { uint32_t u = (uint32_t)b; float f; memcpy(&f, &u, 4); return f; }
+
+#define PF_PART ((size_t)64 << 20)            // partial tiles of a split K
+
+struct PfWs { size_t x, xn, q, k, v, qh, ql, attn, act, part, logits, sel, probs, place, counts, off, tiles, ntiles, row_tok, row_dst, act_e, y_e, total; };
+static PfWs pf_layout(const int64_t* m, int64_t R) {
+  PfWs w = {}; size_t o = 0;
+  auto take = [&](size_t n) { const size_t at = o; o += (n + 255) & ~(size_t)255; return at; };
+  const int64_t dim = m[PM_DIM], nq = m[PM_HEADS] * m[PM_HD], nk = m[PM_KV] * m[PM_HD], E = m[PM_EXPERTS], k = m[PM_TOPK];
+  const int64_t h = E ? m[PM_DENSE_HIDDEN] : m[PM_HIDDEN];
+  w.x = take(R * dim * 4); w.xn = take(R * dim * 2); w.q = take(R * nq * 4); w.k = take(R * nk * 4); w.v = take(R * nk * 4); w.qh = take(R * nq * 2); w.ql = take(R * nq * 2);
+  w.attn = take(R * nq * 2); w.act = take(R * (h > 0 ? h : 1) * 2);
+  w.part = take(PF_PART);
+  if (E) {
+    w.logits = take(R * E * 4); w.sel = take(R * k * 4); w.probs = take(R * k * 4); w.place = take(R * k * 4); w.counts = take(E * 4); w.off = take((E + 1) * 4);
+    w.tiles = take((R * k / 32 + E + 1) * 8); w.ntiles = take(4); w.row_tok = take(R * k * 4); w.row_dst = take(R * k * 4);
+    w.act_e = take(R * k * m[PM_HIDDEN] * 2); w.y_e = take(R * k * dim * 4);
+  }
+  w.total = o;
+  return w;
+}
+
+// one expert-grouped product over the tiles rows_group_kernel listed; up != nullptr: silu(gate) * up
+static int pf_experts(int type, const void* wgt, const void* up, int64_t N, int64_t K, const uint16_t* x, void* y, int y_f32, int tt, int64_t max_tiles, const int2* tiles, const int* n_tiles,
+                      const int* off, const int* row_tok, const int* row_dst, hipStream_t s) {
+  RowsArgs a = {};
+  const int fmt = tga_rows_fmt(type, K);
+  a.w[0] = (const uint8_t*)wgt; a.w[1] = (const uint8_t*)up; a.y[0] = y; a.n[0] = N; a.n[1] = N; a.ntot = N; a.row_bytes = tga_rows_row_bytes(fmt, K); a.estride = a.row_bytes * N;
+  a.x = x; a.nseg = 1; a.epi = up ? ROWS_SWIGLU : ROWS_PLAIN; a.y_f32 = y_f32; a.K = (int)K; a.ks = 1;
+  const int per = up ? ROWS_WT / 2 : ROWS_WT;
+  a.row_tiles = (int)((N + per - 1) / per);
+  a.tiles = tiles; a.n_tiles = n_tiles; a.off = off; a.row_tok = row_tok; a.row_dst = row_dst;
+  return tga_rows_dispatch(fmt, a, tt, (unsigned)((max_tiles * a.row_tiles + 7) / 8 * 8), s);
+}
+
+extern "C" {
+
+int tga_prefill_plan(const int64_t* model, int64_t rows, int64_t* nbytes) {
+  TGA_REQUIRE(model && nbytes && rows >= 1, "tga_prefill_plan: null pointer or no rows");
+  *nbytes = (int64_t)pf_layout(model, rows).total;
+  return 0;
+}
+
+int tga_rows_format_ok(int ggml_type, int64_t K, int* ok) { TGA_REQUIRE(ok, "tga_rows_format_ok: null pointer"); *ok = tga_rows_fmt(ggml_type, K) >= 0; return 0; }
+
+int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tokens, int64_t nseq, int64_t P, int64_t pos0, void* workspace, void* state, void* stream) {
+  TGA_REQUIRE(m && blocks && tokens && workspace && state && nseq >= 1 && P >= 1 && pos0 >= 0 && pos0 + P <= m[PM_MAXCTX], "tga_prefill_step: null pointer or rows beyond the cache");
+  const int64_t R = nseq * P, dim = m[PM_DIM], H = m[PM_HEADS], KV = m[PM_KV], hd = m[PM_HD], nq = H * hd, nk = KV * hd, E = m[PM_EXPERTS], k = m[PM_TOPK];
+  TGA_REQUIRE((hd == 64 || hd == 128) && KV > 0 && H % KV == 0 && E <= PF_MAX_E && k <= 64 && R < (1 << 20), "tga_prefill_step: geometry outside the range");
+  const PfWs w = pf_layout(m, R);
+  uint8_t* ws = (uint8_t*)workspace;
+  float* x = (float*)(ws + w.x); uint16_t* xn = (uint16_t*)(ws + w.xn); float* q = (float*)(ws + w.q); float* kk = (float*)(ws + w.k); float* v = (float*)(ws + w.v);
+  uint16_t* attn = (uint16_t*)(ws + w.attn); uint16_t* act = (uint16_t*)(ws + w.act);
+  hipStream_t s = (hipStream_t)stream;
+  const float eps = bits_f(m[PM_EPS_BITS]);
+  int rc;
+#define PF_DO(call) do { if ((rc = (call))) return rc; } while (0)
+  auto linear = [&](int type, int nseg, const void* const* wt, void* const* y, const int64_t* n, const void* in, int ydt, int64_t K, int epi, const float* resid) {
+    return tga_qlinear_many(type, nseg, wt, y, n, in, ydt, R, K, epi, resid, ws + w.part, (int64_t)PF_PART, stream);
+  };
+  PF_DO(tga_embed_rows((const void*)m[PM_EMB], (int)m[PM_EMB_TYPE], (int)dim, tokens, (int)R, state, x, stream));
+  for (int64_t bi = 0; bi < m[PM_NBLOCKS]; bi++) {
+    const int64_t* b = blocks + bi * PB_COUNT;
+    const bool pending = bi > 0 && blocks[(bi - 1) * PB_COUNT + PB_MOE];  // the block before left its weighted expert sum to this norm
+    if (pending) PF_DO(tga_moe_combine_rmsnorm_rows((float*)(ws + w.y_e), (float*)(ws + w.probs), x, (const float*)b[PB_ATTN_NORM], (int)R, (int)k, (int)dim, eps, xn, nullptr, stream));
+    else PF_DO(tga_rmsnorm_rows(x, (const float*)b[PB_ATTN_NORM], (int)R, (int)dim, eps, xn, nullptr, 0, stream));
+    const void* wt[3] = {(const void*)b[PB_WQ], (const void*)b[PB_WK], (const void*)b[PB_WV]};
+    void* y[3] = {q, kk, v}; const int64_t n[3] = {nq, nk, nk};
+    for (int i = 0; i < 3;) {                                             // one launch per run of equal block types
+      int j = i + 1;
+      while (j < 3 && b[PB_TQ + j] == b[PB_TQ + i]) j++;
+      PF_DO(linear((int)b[PB_TQ + i], j - i, wt + i, y + i, n + i, xn, TGA_F32, dim, 0, nullptr));
+      i = j;
+    }
+    RopeArgs ra;
+    ra.q = q; ra.k = kk; ra.v = v; ra.qn = (const float*)b[PB_QN]; ra.kn = (const float*)b[PB_KN]; ra.rope = (const float*)m[PM_ROPE];
+    ra.qh = (uint16_t*)(ws + w.qh); ra.ql = (uint16_t*)(ws + w.ql); ra.ck = (uint16_t*)b[PB_CK]; ra.cv = (uint16_t*)b[PB_CV];
+    ra.zero = b[PB_MOE] ? (int*)(ws + w.counts) : nullptr; ra.n_zero = b[PB_MOE] ? (int)E : 0;
+    ra.H = (int)H; ra.KV = (int)KV; ra.hd = (int)hd; ra.max_ctx = (int)m[PM_MAXCTX]; ra.P = (int)P; ra.pos0 = (int)pos0; ra.eps = eps;
+    ra.norm = !b[PB_QN] ? 0 : m[PM_QKNORM] == hd ? 2 : 1;
+    rows_rope_kernel<<<(unsigned)R, 256, 0, s>>>(ra);
+    TGA_LAUNCH_CHECK();
+    RowsAttnArgs aa;
+    aa.qh = ra.qh; aa.ql = ra.ql; aa.ck = ra.ck; aa.cv = ra.cv; aa.out = attn; aa.H = (int)H; aa.KV = (int)KV; aa.max_ctx = ra.max_ctx; aa.P = (int)P; aa.pos0 = (int)pos0; aa.nseq = (int)nseq;
+    aa.qtiles = (int)((P + 63) / 64); aa.scale = 1.4426950408889634f / sqrtf((float)hd);
+    const unsigned ag = (unsigned)(aa.qtiles * H * nseq);
+    if (hd == 64) rows_attn_kernel<64><<<ag, 256, 0, s>>>(aa); else rows_attn_kernel<128><<<ag, 256, 0, s>>>(aa);
+    TGA_LAUNCH_CHECK();
+    { const void* wo[1] = {(const void*)b[PB_WO]}; void* yo[1] = {x}; const int64_t no[1] = {dim}; PF_DO(linear((int)b[PB_TO], 1, wo, yo, no, attn, TGA_F32, nq, 1, x)); }
+    PF_DO(tga_rmsnorm_rows(x, (const float*)b[PB_FFN_NORM], (int)R, (int)dim, eps, xn, nullptr, 0, stream));
+    if (!b[PB_MOE]) {
+      const int64_t h = E ? m[PM_DENSE_HIDDEN] : m[PM_HIDDEN];
+      const void* wg[2] = {(const void*)b[PB_GATE], (const void*)b[PB_UP]}; void* yg[2] = {act, nullptr}; const int64_t ng[2] = {h, h};
+      PF_DO(linear((int)b[PB_TGATE], 2, wg, yg, ng, xn, TGA_F16, dim, 2, nullptr));
+      const void* wd[1] = {(const void*)b[PB_DOWN]}; void* yd[1] = {x}; const int64_t nd[1] = {dim};
+      PF_DO(linear((int)b[PB_TDOWN], 1, wd, yd, nd, act, TGA_F32, h, 1, x));
+      continue;
+    }
+    float* logits = (float*)(ws + w.logits); int* counts = (int*)(ws + w.counts); int* sel = (int*)(ws + w.sel); int* place = (int*)(ws + w.place);
+    { const void* wr[1] = {(const void*)b[PB_ROUTER]}; void* yr[1] = {logits}; const int64_t nr[1] = {E}; PF_DO(linear(TGA_F16, 1, wr, yr, nr, xn, TGA_F32, dim, 0, nullptr)); }
+    rows_gate_kernel<<<(unsigned)((R + 3) / 4), 256, 0, s>>>(logits, (int)R, (int)E, (int)k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), sel, (float*)(ws + w.probs), counts, place);
+    TGA_LAUNCH_CHECK();
+    const int64_t avg = R * k / E;
+    const int tt = avg <= 32 ? 32 : avg <= 96 ? 64 : 128;
+    const int64_t max_tiles = R * k / tt + (R * k < E ? R * k : E);
+    int2* tiles = (int2*)(ws + w.tiles); int* nt = (int*)(ws + w.ntiles); int* off = (int*)(ws + w.off); int* row_tok = (int*)(ws + w.row_tok); int* row_dst = (int*)(ws + w.row_dst);
+    const int64_t gb = (R * k + 511) / 512;
+    rows_group_kernel<<<(unsigned)(gb < 64 ? gb : 64), 512, 0, s>>>(counts, sel, place, (int)R, (int)E, (int)k, tt, off, tiles, nt, row_tok, row_dst);
+    TGA_LAUNCH_CHECK();
+    const int64_t hid = m[PM_HIDDEN];
+    PF_DO(pf_experts((int)b[PB_TGATE], (const void*)b[PB_GATE], (const void*)b[PB_UP], hid, dim, xn, ws + w.act_e, 0, tt, max_tiles, tiles, nt, off, row_tok, nullptr, s));
+    PF_DO(pf_experts((int)b[PB_TDOWN], (const void*)b[PB_DOWN], nullptr, dim, hid, (const uint16_t*)(ws + w.act_e), ws + w.y_e, 1, tt, max_tiles, tiles, nt, off, nullptr, row_dst, s));
+  }
+#undef PF_DO
+  return 0;
+}
+
+}  // extern "C"

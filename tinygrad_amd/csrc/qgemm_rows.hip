@@ -1,0 +1,118 @@
+// Entry points of the many-rows linears (kernel: qgemm_rows.h).
+#include "qgemm_rows.h"
+
+#define X(F) int tga_rows_launch_##F(const RowsArgs& a, int tt, unsigned grid, hipStream_t s);
+ROWS_FORMATS(X)
+#undef X
+
+// format id of a block type with rows of K values, -1: not taken (K a multiple of 128 and of the superblock; the pair formats read 4-byte aligned rows)
+int tga_rows_fmt(int ggml_type, int64_t K) {
+  const bool k256 = K % 256 == 0;
+  if (K < 128 || K % 128) return -1;
+  switch (ggml_type) {
+    case GGML_Q4_0: return F_Q4_0P;
+    case GGML_Q8_0: return F_Q8_0P;
+    case GGML_F16: case GGML_MXFP4: case GGML_Q4_1: case GGML_Q5_0: case GGML_Q5_1: return ggml_type;
+    case GGML_Q4_K: case GGML_Q5_K: case GGML_Q6_K: case GGML_IQ4_XS: return k256 ? ggml_type : -1;
+  }
+  return -1;
+}
+int64_t tga_rows_row_bytes(int fmt, int64_t K) {
+  switch (fmt) {
+    case F_Q4_0P: return K / 32 * 18;
+    case F_Q8_0P: return K / 32 * 34;
+    case GGML_F16: return K * 2;
+    case GGML_MXFP4: return K / 32 * 17;
+    case GGML_Q4_1: return K / 32 * 20;
+    case GGML_Q5_0: return K / 32 * 22;
+    case GGML_Q5_1: return K / 32 * 24;
+    case GGML_Q4_K: return K / 256 * 144;
+    case GGML_Q5_K: return K / 256 * 176;
+    case GGML_Q6_K: return K / 256 * 210;
+    case GGML_IQ4_XS: return K / 256 * 136;
+  }
+  return 0;
+}
+int tga_rows_dispatch(int fmt, const RowsArgs& a, int tt, unsigned grid, hipStream_t s) {
+  switch (fmt) {
+#define X(F) case F: return tga_rows_launch_##F(a, tt, grid, s);
+    ROWS_FORMATS(X)
+#undef X
+  }
+  return tga_set_error("tga_qlinear_many: no kernel for format %d", fmt);
+}
+
+// y = [residual +] the partial sums of a split K in its order; 4 neighbouring weight rows per thread
+__global__ __launch_bounds__(256) void rows_reduce_kernel(const RowsArgs a) {
+  const long long q4 = a.ntot / 4, total = (long long)a.M * q4, plane = (long long)a.M * a.ntot;
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
+    const long long t = i / q4; long long row = (i - t * q4) * 4;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    const float* p = a.part + t * a.ntot + row;
+    for (int k = 0; k < a.ks; k++) { const f32x4 v = *(const f32x4*)(p + k * plane); o.x += v.x; o.y += v.y; o.z += v.z; o.w += v.w; }
+    int sg = 0;
+    if (a.nseg > 1 && row >= a.n[0]) { row -= a.n[0]; sg = 1; if (a.nseg > 2 && row >= a.n[1]) { row -= a.n[1]; sg = 2; } }
+    void* yb = sg == 0 ? a.y[0] : sg == 1 ? a.y[1] : a.y[2];
+    const long long at = t * (sg == 0 ? a.n[0] : sg == 1 ? a.n[1] : a.n[2]) + row;
+    if (a.epi == ROWS_RESID) { const f32x4 r = *(const f32x4*)(a.resid + at); o.x += r.x; o.y += r.y; o.z += r.z; o.w += r.w; }
+    if (a.y_f32) *(f32x4*)((float*)yb + at) = o;
+    else *(u32x2*)((uint16_t*)yb + at) = u32x2{f2h_bits(o.x) | (f2h_bits(o.y) << 16), f2h_bits(o.z) | (f2h_bits(o.w) << 16)};
+  }
+}
+
+// Tile height and K split for M rows of one set of matrices: rows of at most 32 / 64 take the lower tiles; K is split while the tiles leave CUs with fewer than two workgroups
+static void rows_plan(long long row_tiles, int M, int K, bool may_split, size_t part_bytes, long long ntot, int* tt, int* ks) {
+  *tt = M <= 32 ? 32 : M <= 64 ? 64 : 128;
+  const long long wgs = row_tiles * ((M + *tt - 1) / *tt);
+  int k = 1;
+  if (may_split) {
+    k = (int)(512 / (wgs > 0 ? wgs : 1));
+    const int kmax = K / ROWS_KS / 4;
+    if (k > kmax) k = kmax;
+    while (k > 1 && (size_t)k * M * ntot * 4 > part_bytes) k--;
+    if (k < 1) k = 1;
+  }
+  *ks = k;
+}
+
+extern "C" {
+
+int tga_qlinear_many(int ggml_type, int nseg, const void* const* w, void* const* y, const int64_t* n, const void* x_f16, int y_dtype, int64_t M, int64_t K, int epilogue,
+                     const float* resid, void* workspace, int64_t workspace_bytes, void* stream) {
+  TGA_REQUIRE(w && y && n && x_f16 && nseg >= 1 && nseg <= 3, "tga_qlinear_many: null pointer or %d matrices", nseg);
+  TGA_REQUIRE(epilogue >= 0 && epilogue <= 2 && (epilogue != 2 || nseg == 2) && (epilogue != 1 || (nseg == 1 && resid)), "tga_qlinear_many: epilogue %d with %d matrices", epilogue, nseg);
+  TGA_REQUIRE(y_dtype == TGA_F32 || y_dtype == TGA_F16, "tga_qlinear_many: y_dtype must be TGA_F16 or TGA_F32");
+  const int fmt = tga_rows_fmt(ggml_type, K);
+  TGA_REQUIRE(fmt >= 0 && M >= 1 && M * K < (1ll << 32) && M < (1 << 24), "tga_qlinear_many: type %d with K=%lld, M=%lld is outside the range", ggml_type, (long long)K, (long long)M);
+  RowsArgs a = {};
+  const int segs = epilogue == 2 ? 1 : nseg;
+  for (int i = 0; i < nseg; i++) {
+    TGA_REQUIRE(w[i] && n[i] > 0 && (i >= segs || y[i]), "tga_qlinear_many: null pointer in matrix %d", i);
+    TGA_REQUIRE(((uintptr_t)w[i] & (ggml_type == GGML_F16 ? 15 : ggml_type == GGML_MXFP4 ? 0 : 3)) == 0, "tga_qlinear_many: weights must be 4-byte aligned (fp16: 16-byte)");
+    TGA_REQUIRE(i + 1 >= segs || n[i] % 16 == 0, "tga_qlinear_many: matrices that share a launch need a multiple of 16 rows");
+    a.w[i] = (const uint8_t*)w[i]; a.n[i] = n[i];
+    if (i < segs) { a.y[i] = y[i]; a.ntot += n[i]; TGA_REQUIRE(((uintptr_t)y[i] & 15) == 0, "tga_qlinear_many: results must be 16-byte aligned"); }
+  }
+  TGA_REQUIRE(epilogue != 2 || n[0] == n[1], "tga_qlinear_many: gate and up differ in rows");
+  TGA_REQUIRE((((uintptr_t)x_f16 | (uintptr_t)resid | (uintptr_t)workspace) & 15) == 0, "tga_qlinear_many: activations must be 16-byte aligned");
+  a.row_bytes = tga_rows_row_bytes(fmt, K); a.x = (const uint16_t*)x_f16; a.resid = resid; a.part = (float*)workspace; a.nseg = segs; a.epi = epilogue; a.y_f32 = y_dtype == TGA_F32;
+  a.M = (int)M; a.K = (int)K;
+  a.row_tiles = (int)((a.ntot + (epilogue == 2 ? ROWS_WT / 2 : ROWS_WT) - 1) / (epilogue == 2 ? ROWS_WT / 2 : ROWS_WT));
+  bool split = epilogue != 2 && workspace && a.ntot % 4 == 0;
+  for (int i = 0; i < segs; i++) split = split && n[i] % 4 == 0;
+  int tt;
+  rows_plan(a.row_tiles, (int)M, (int)K, split, (size_t)workspace_bytes, a.ntot, &tt, &a.ks);
+  a.tok_tiles = (int)((M + tt - 1) / tt);
+  if (a.ks > 1) a.epi = ROWS_PART;
+  const unsigned grid = (unsigned)(((long long)a.row_tiles * a.tok_tiles + 7) / 8 * 8);
+  if (const int rc = tga_rows_dispatch(fmt, a, tt, grid, (hipStream_t)stream)) return rc;
+  if (a.ks > 1) {
+    a.epi = epilogue;
+    const long long total = M * (a.ntot / 4), wg = (total + 255) / 256;
+    rows_reduce_kernel<<<(unsigned)(wg < 4096 ? wg : 4096), 256, 0, (hipStream_t)stream>>>(a);
+    TGA_LAUNCH_CHECK();
+  }
+  return 0;
+}
+
+}  // extern "C"

@@ -53,6 +53,9 @@ LLAMA3_8B = dict(num_blocks=32, dim=4096, hidden_dim=14336, n_heads=32, n_kv_hea
 OLMOE = dict(num_blocks=16, dim=2048, hidden_dim=1024, n_heads=16, n_kv_heads=16, norm_eps=1e-5, vocab_size=50304, head_dim=128,
              rope_theta=10000.0, qk_norm=2048, num_experts=64, num_experts_per_tok=8, norm_topk_prob=False, expert_gating_func=1)
 
+MANY_ROWS = 2048                   # rows of a prefill step at most (its buffers grow with the rows: 0.5 GB for the 8B architecture)
+MANY_ROWS_MIN = 17                 # fewer rows are one step of the small-batch kernels
+
 def precompute_freqs_cis(dim: int, end: int, theta: float) -> np.ndarray:
   """tinygrad/llm/model.py:16-19 in float32: cat(cos(pos * f), sin(pos * f)), f = 1 / theta^(2i/dim)."""
   freqs = (np.float32(1.0) / (np.float32(theta) ** (np.arange(0, dim, 2, dtype=np.float32)[:dim // 2] / np.float32(dim)))).astype(np.float32)
@@ -374,7 +377,7 @@ class Transformer:
     self._cached_tokens, self._last_input, self.prefill_steps = [], None, 0   # tokens whose K / V rows the cache holds (KV-prefix reuse, model.py:455-462)
     self.replay = "cmdlist"                                          # how a captured step is replayed: "cmdlist" (plain launches in capture order) or "graph" (hipGraphLaunch)
     self._state_dict, self._chunker, self._tail_chunkers = state_dict, None, {}   # (references to the weight buffers: the chunked prefill builds its linears over the same bytes)
-    self.prefill_chunk = 128                                         # prompt positions per prefill step, 2..128 (the reference's chunks hold 32, model.py:464; MoE models: at most 16); 1: token by token
+    self.prefill_chunk = 128                                         # prompt positions per prefill step, 2..128 (128: as many as the prompt has where the model allows, see prefill) (the reference's chunks hold 32, model.py:464; MoE models: at most 16); 1: token by token
 
   def check_state(self):
     """Raises when a kernel of the last steps refused its input (state.error: bit 0 = a token id outside the vocabulary reached the embedding
@@ -514,6 +517,13 @@ class Transformer:
     self.prefill_steps = len(tokens) - 1 - start                        # (positions the last call actually computed)
     self._cached_tokens = self._cached_tokens[:start]                   # the rows from here on are about to be overwritten: if a step below raises, they are not claimed
     B = self.prefill_chunk if on_block is None else 1
+    # From MANY_ROWS_MIN positions on, and with the chunk size left at its largest, the positions are steps of many rows: one pass over the weights for (nearly) any prompt
+    n_rows = len(tokens) - 1 - start
+    if B == 128 and n_rows >= MANY_ROWS_MIN:
+      if n_rows >= B and self._chunker is None: self._chunker = BatchedTransformer(self.config, self._state_dict, B, max_new=1, chunk_of=self)
+      if self._chunker is None and 16 not in self._tail_chunkers: self._tail_chunkers[16] = BatchedTransformer(self.config, self._state_dict, 16, max_new=1, chunk_of=self)
+      chunker = self._chunker or self._tail_chunkers[16]
+      if chunker._rows_tables is not None: start += chunker.prefill_rows(tokens, start, n_rows)
     if B > 16 and self.config.num_experts: B = 16                       # (MoE blocks keep steps of sixteen positions: longer ones are not measured there)
     # Whole chunks as small-batch steps (model.py:476-481) of the largest size that the prompt holds (the chosen one, else 64, 32, 16, 8 or 4 positions).  Dense models: what
     # they leave is ONE more chunk that ends at the last position and computes some positions again - every row of a step depends on the cache and on its own token
@@ -624,23 +634,9 @@ class BatchedTransformer:
         b["cache_k"] = Buffer((B, c.n_kv_heads, c.max_context, c.head_dim), f16).zero_()
         b["cache_v"] = Buffer((B, c.n_kv_heads, c.max_context, c.head_dim), f16).zero_()
       self.blk.append(b)
-    k = max(1, c.num_experts_per_tok)
     self.state = Buffer((16,), np.int32).zero_()
     self.tokens = Buffer((B,), np.int32).zero_()
-    self.x, self.xn = Buffer((B, c.dim), f32), Buffer((B, c.dim), f16)
-    self.q, self.k, self.v = Buffer((B, nq), f32), Buffer((B, nkv), f32), Buffer((B, nkv), f32)
-    self.attn = Buffer((B, nq), f16)
-    self.attn_part = Buffer((B * c.n_heads * ((c.max_context + 63) // 64) * (c.head_dim + 2),), f32).zero_()
-    self.act = Buffer((B, max(1, c.hidden_dim, c.dense_hidden_dim)), f16)
-    if any(not b["moe"] and b["ffn_gate"].ggml_type != b["ffn_up"].ggml_type for b in self.blk):      # (gate and up rows of such a block, before silu(gate) * up)
-      self.gate32, self.up32 = Buffer((B, max(c.hidden_dim, c.dense_hidden_dim)), f32), Buffer((B, max(c.hidden_dim, c.dense_hidden_dim)), f32)
-    if c.shared_expert_dim:
-      self.act_sh, self.y_sh = Buffer((B, c.shared_expert_dim), f16), Buffer((B, c.dim), f32)
-      self.p_sh, self.sh_logit, self.sh_sel = Buffer.from_numpy(np.ones(B, dtype=f32)), Buffer((B, 1), f32), Buffer((B,), np.int32)   # weight 1 unless the shared expert is gated
-    if c.num_experts:
-      self.router_logits, self.sel, self.probs = Buffer((B, c.num_experts), f32), Buffer((B * k,), np.int32), Buffer((B * k,), f32)
-      self.job_table, self.job_flags = Buffer((c.num_experts, 16), np.int32).zero_(), Buffer((1,), np.int32).zero_()
-      self.act_e, self.y_e = Buffer((B * k, c.hidden_dim), f16), Buffer((B * k, c.dim), f32)
+    if c.num_experts: self.job_flags = Buffer((1,), np.int32).zero_()
     self.logits_buf = Buffer((B, c.vocab_size), f32) if chunk_of is None else None
     self.rope = Buffer.from_numpy(rope_table(c.head_dim, c.rope_dim or c.head_dim, c.max_context, c.rope_theta)) if chunk_of is None else chunk_of.s.rope
     self.prompts = Buffer((B if chunk_of is None else 1, c.max_context), np.int32).zero_()
@@ -660,8 +656,84 @@ class BatchedTransformer:
                and all(b[nm].out_features % 16 == 0 for nm in ("attn_q", "attn_k", "attn_v")) for b in self.blk)
       if ok and c.dim % 256 == 0 and c.hidden_dim % 256 == 0 and nq % 256 == 0:
         self.rows64 = 2 if B <= 32 else 4 if B <= 64 else 8             # column groups of sixteen rows in the layout
-        R = 16 * self.rows64
-        self.xn_st, self.attn_st, self.act_st = Buffer((R, c.dim), f16).zero_(), Buffer((R, nq), f16).zero_(), Buffer((R, c.hidden_dim), f16).zero_()
+    self._rows_tables, self._rows_ws, self._rows_tok = self._many_rows_tables(), None, None
+    self.x = None
+    if not self.chunked: self._alloc_step()
+
+  def _alloc_step(self):
+    """The row buffers of a plain step (a prefill that runs as steps of many rows needs none of them)."""
+    c, B = self.config, self.batch
+    f32, f16 = np.float32, np.float16
+    nq, nkv = c.n_heads * c.head_dim, c.n_kv_heads * c.head_dim
+    k = max(1, c.num_experts_per_tok)
+    self.x, self.xn = Buffer((B, c.dim), f32), Buffer((B, c.dim), f16)
+    self.q, self.k, self.v = Buffer((B, nq), f32), Buffer((B, nkv), f32), Buffer((B, nkv), f32)
+    self.attn = Buffer((B, nq), f16)
+    self.attn_part = Buffer((B * c.n_heads * ((c.max_context + 63) // 64) * (c.head_dim + 2),), f32).zero_()
+    self.act = Buffer((B, max(1, c.hidden_dim, c.dense_hidden_dim)), f16)
+    if any(not b["moe"] and b["ffn_gate"].ggml_type != b["ffn_up"].ggml_type for b in self.blk):      # (gate and up rows of such a block, before silu(gate) * up)
+      self.gate32, self.up32 = Buffer((B, max(c.hidden_dim, c.dense_hidden_dim)), f32), Buffer((B, max(c.hidden_dim, c.dense_hidden_dim)), f32)
+    if c.shared_expert_dim:
+      self.act_sh, self.y_sh = Buffer((B, c.shared_expert_dim), f16), Buffer((B, c.dim), f32)
+      self.p_sh, self.sh_logit, self.sh_sel = Buffer.from_numpy(np.ones(B, dtype=f32)), Buffer((B, 1), f32), Buffer((B,), np.int32)   # weight 1 unless the shared expert is gated
+    if c.num_experts:
+      self.router_logits, self.sel, self.probs = Buffer((B, c.num_experts), f32), Buffer((B * k,), np.int32), Buffer((B * k,), f32)
+      self.job_table = Buffer((c.num_experts, 16), np.int32).zero_()
+      self.act_e, self.y_e = Buffer((B * k, c.hidden_dim), f16), Buffer((B * k, c.dim), f32)
+    if self.rows64:
+      R = 16 * self.rows64
+      self.xn_st, self.attn_st, self.act_st = Buffer((R, c.dim), f16).zero_(), Buffer((R, nq), f16).zero_(), Buffer((R, c.hidden_dim), f16).zero_()
+
+  def _many_rows_tables(self):
+    """The tables of tga_prefill_step (csrc/prefill.hip: PM_ / PB_ enumerations), or None for a model outside its range: q / k / v biases, head sizes other than 64 and 128, a
+    shared expert, an expert selection bias, ffn_gate / ffn_up of different block types, a router that is not fp16, or block types and row lengths its linears do not take."""
+    c = self.config
+    def fits(l):
+      ok = ctypes.c_int(0); rt.check(rt.lib().tga_rows_format_ok(l.ggml_type, l.in_features, ctypes.byref(ok)))
+      return bool(ok.value) and l.blocks.ptr % (16 if l.ggml_type == rt.F16 else 1 if l.ggml_type == rt.MXFP4 else 4) == 0
+    if c.head_dim not in (64, 128) or c.shared_expert_dim or c.num_experts > 512 or c.num_experts_per_tok > 64 or os.environ.get("TGA_ROWS64", "1") != "1": return None
+    rows = []
+    for b in self.blk:
+      ffn = [b["gate_exps"], b["up_exps"], b["down_exps"]] if b["moe"] else [b["ffn_gate"], b["ffn_up"], b["ffn_down"]]
+      lins = [b["attn_q"], b["attn_k"], b["attn_v"], b["attn_output"], *ffn] + ([b["router"]] if b["moe"] else [])
+      if "bias" in b or not all(fits(l) for l in lins) or ffn[0].ggml_type != ffn[1].ggml_type: return None
+      if b["moe"] and (b["sel_bias"] is not None or b["router"].ggml_type != rt.F16): return None
+      rows.append([b["attn_norm"].ptr, b["ffn_norm"].ptr, b["q_norm"].ptr if c.qk_norm else 0, b["k_norm"].ptr if c.qk_norm else 0, b["cache_k"].ptr, b["cache_v"].ptr, int(b["moe"]),
+                   *[l.blocks.ptr for l in lins[:7]], b["router"].blocks.ptr if b["moe"] else 0, *[l.ggml_type for l in lins[:4]], ffn[0].ggml_type, ffn[2].ggml_type])
+    bits = lambda f: int(np.float32(f).view(np.uint32))
+    model = [c.num_blocks, c.dim, c.n_heads, c.n_kv_heads, c.head_dim, c.max_context, self.token_embd.ptr, self.embd_type, self.rope.ptr, c.num_experts, c.num_experts_per_tok, c.expert_gating_func,
+             int(c.norm_topk_prob), c.qk_norm, c.hidden_dim, c.dense_hidden_dim, bits(c.norm_eps), bits(c.routed_scaling_factor)]
+    return (ctypes.c_int64 * len(model))(*model), (ctypes.c_int64 * (len(rows) * len(rows[0])))(*sum(rows, []))
+
+  def _prefill_many_rows(self, ids: np.ndarray, pos0: int):
+    """Positions pos0 .. pos0 + n - 1 of every sequence of ids (sequences, n) in steps of at most MANY_ROWS rows, each one native call."""
+    nseq, n = ids.shape
+    per = max(1, MANY_ROWS // nseq)
+    steps = [(i, min(per, n - i)) for i in range(0, n, per)]
+    need = ctypes.c_int64(0)
+    rt.check(rt.lib().tga_prefill_plan(self._rows_tables[0], nseq * steps[0][1], ctypes.byref(need)))
+    if self._rows_ws is None or self._rows_ws.nbytes < need.value: self._rows_ws = Buffer((need.value,), np.uint8)
+    if self._rows_tok is None or self._rows_tok.nbytes < ids.nbytes: self._rows_tok = Buffer((ids.nbytes,), np.uint8)
+    flat = np.concatenate([ids[:, i:i + m].reshape(-1) for i, m in steps]).astype(np.int32)
+    self._rows_tok.view(0, flat.shape, np.int32).copyin(flat)
+    at = 0
+    for i, m in steps:
+      rt.check(rt.lib().tga_prefill_step(*self._rows_tables, self._rows_tok.ptr + 4 * at, nseq, m, pos0 + i, self._rows_ws.ptr, self.state.ptr, self.stream.handle))
+      at += nseq * m
+
+  def prefill_rows(self, tokens: list[int], start: int, n: int) -> int:
+    """Chunked prefill for `chunk_of` in steps of many rows: the positions start .. start + n - 1 of the prompt into its KV caches.  Returns the number of positions done."""
+    c = self.config
+    if not self.chunked or self._rows_tables is None: raise RuntimeError("prefill_rows needs a model built with chunk_of and linears in the range of tga_prefill_step")
+    if not (0 <= start and n >= 1 and start + n <= len(tokens) < c.max_context): raise ValueError(f"positions {start}+{n} outside the prompt of {len(tokens)} tokens")
+    if min(tokens) < 0 or max(tokens) >= c.vocab_size: raise ValueError(f"token id outside the vocabulary of {c.vocab_size}")
+    st = np.zeros(16, np.int32); st[0], st[3], st[5] = start, len(tokens), c.vocab_size
+    self.state.copyin(st)
+    self._owner_stream.synchronize()
+    self._prefill_many_rows(np.array(tokens[start:start + n], np.int32)[None, :], start)
+    self.stream.synchronize()
+    self.check_state()
+    return n
 
   def _linear(self, layers, x, outs, **kw): qlinear_multi(layers, x, outs, stream=self.stream.handle, **kw)
 
@@ -806,6 +878,7 @@ class BatchedTransformer:
     if n_chunks <= 0: return 0
     if not (0 <= start and start + n_chunks * B <= len(tokens) < c.max_context): raise ValueError(f"chunks {start}+{n_chunks}x{B} outside the prompt of {len(tokens)} tokens")
     if min(tokens) < 0 or max(tokens) >= c.vocab_size: raise ValueError(f"token id outside the vocabulary of {c.vocab_size}")
+    if self.x is None: self._alloc_step()
     pr = np.zeros((1, c.max_context), np.int32); pr[0, :len(tokens)] = tokens
     self.prompts.copyin(pr)
     self.tokens.copyin(np.ascontiguousarray(pr[0, start:start + B]))
@@ -827,10 +900,14 @@ class BatchedTransformer:
     if min(map(min, prompts)) < 0 or max(map(max, prompts)) >= c.vocab_size: raise ValueError(f"token id outside the vocabulary of {c.vocab_size}")
     pr = np.zeros((B, c.max_context), np.int32); pr[:, :n] = np.array(prompts, np.int32)
     self.prompts.copyin(pr)
-    self.tokens.copyin(np.ascontiguousarray(pr[:, 0]))
-    st = np.zeros(16, np.int32); st[3], st[5] = n, c.vocab_size
+    # all but the last position of every prompt: as steps of many rows (sequences x positions) where the model is in their range and there are rows enough, else step by step
+    many = self._rows_tables is not None and on_block is None and B * (n - 1) >= MANY_ROWS_MIN and n > 2 and self.expert_path == "jobs"     # (a chosen expert path runs every step)
+    done = n - 1 if many else 0
+    self.tokens.copyin(np.ascontiguousarray(pr[:, done]))
+    st = np.zeros(16, np.int32); st[0], st[3], st[5] = done, n, c.vocab_size
     self.state.copyin(st)
-    for _ in range(n - 1):
+    if many: self._prefill_many_rows(pr[:, :n - 1], 0)
+    for _ in range(n - 1 - done):
       if use_graph and on_block is None: self._graph(False).launch()
       else: self._step(False, on_block)
     self._steps_done = n - 1

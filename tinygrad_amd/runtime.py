@@ -44,6 +44,9 @@ def _declare(lib):
     "tga_qlinear_experts": [i, vp, vp, i64, vp, i, i, vp, i, vp, i, i64, i64, vp],
     "tga_qlinear_experts_routed": [i, vp, vp, i64, vp, i, i, i, ctypes.c_float, vp, vp, vp, vp, i, i64, i64, vp],
     "tga_qlinear_experts_routed_rows": [i, vp, vp, i64, vp, i, i, i, i, ctypes.c_float, vp, vp, vp, vp, i, i64, i64, vp],
+    "tga_qlinear_many": [i, i, c_void_pp, c_void_pp, ctypes.POINTER(i64), vp, i, i64, i64, i, vp, vp, i64, vp],
+    "tga_rows_format_ok": [i, i64, ctypes.POINTER(i)], "tga_prefill_plan": [ctypes.POINTER(i64), i64, ctypes.POINTER(i64)],
+    "tga_prefill_step": [ctypes.POINTER(i64), ctypes.POINTER(i64), vp, i64, i64, i64, vp, vp, vp],
     "tga_moe_gate": [vp, i, i, i, i, i, ctypes.c_float, vp, vp, vp],
     "tga_moe_gate_biased": [vp, vp, i, i, i, i, i, ctypes.c_float, vp, vp, vp],
     "tga_moe_combine": [vp, vp, vp, i, i, i, vp, vp],
@@ -192,7 +195,7 @@ def _capture_begin(stream: Stream) -> bool:
   objects (hipFree is not allowed while a capture is open: it invalidates the capture).  Returns whether the collector has to be switched on again."""
   import gc
   was = gc.isenabled()
-  gc.collect(); gc.disable()
+  gc.disable()                                              # (no collection first: a full one takes 10 ms and more in a process with many objects, at every first step)
   try: check(lib().tga_graph_begin(stream.handle))
   except Exception:
     if was: gc.enable()
