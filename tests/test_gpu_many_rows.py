@@ -54,6 +54,28 @@ def test_many_rows_linear_at_tile_edges(gpu, fmt):
     for o, p in zip(outs, parts): close(o.numpy(), ol.linear_f64(x.astype(np.float32), p[1]))
   assert rt.lib().tga_qlinear_many(t, 1, (ctypes.c_void_p * 1)(bufs[0].ptr), (ctypes.c_void_p * 1)(outs[0].ptr), (ctypes.c_int64 * 1)(128), xb.ptr, rt.F32, m, 96, 0, None, None, 0, None) != 0
 
+@pytest.mark.parametrize("m,n,k,epi", [(1283, (7500,), 3072, 0), (1281, (7501,), 3328, 0), (1408, (7440,), 3072, 1), (1345, (4096, 1616, 1808), 3072, 0), (1283, (3830,), 3072, 2), (1283, (2560,), 12544, 1)],
+                         ids=["ragged", "odd", "resid", "three", "swiglu", "split"])
+def test_wide_tiles_of_q4_0(gpu, m, n, k, epi):
+  """The 256 x 128 tiles (twelve steps of 256 per workgroup and 320 workgroups or more): last tiles of 1, 3, 65 and 128 rows and of 12, 76, 96 and 118 outputs, thirteen steps, matrices that meet
+  inside a tile, results that are no multiple of four, K split into parts of twelve and thirteen steps.  Weights are the same fp16 values as in the smaller tiles; float32 sums of K products in another order than the
+  reference's (sgemm): each within K 2^-24 of its absolute sum at the very worst and about sqrt(K) 2^-24 in practice, 5e-5 of the largest result."""
+  from tinygrad_amd import runtime as rt
+  rng = np.random.default_rng(m)
+  ws = rt.Buffer((64 << 20,), np.uint8)
+  ns = n * 2 if epi == 2 else n
+  parts = [_weight(rng, rt, rt.Q4_0, i, k) for i in ns]
+  bufs = [rt.Buffer.from_numpy(p[0]) for p in parts]
+  x = synth.activations(rng, m, k, np.float16); xb = rt.Buffer.from_numpy(x)
+  refs = [x.astype(np.float32) @ p[1].T for p in parts]
+  r = rng.standard_normal((m, n[0])).astype(np.float32)
+  outs = [rt.Buffer.from_numpy(r) if epi == 1 else rt.Buffer((m, i), np.float32) for i in n]
+  VP = ctypes.c_void_p * len(ns)
+  rt.check(rt.lib().tga_qlinear_many(rt.Q4_0, len(ns), VP(*[b.ptr for b in bufs]), VP(*[(outs[i].ptr if i < len(outs) else None) for i in range(len(ns))]), (ctypes.c_int64 * len(ns))(*ns),
+                                     xb.ptr, rt.F32, m, k, epi, outs[0].ptr if epi == 1 else None, ws.ptr, ws.nbytes, None))
+  if epi == 2: refs = [refs[0] / (1 + np.exp(-refs[0])) * refs[1]]
+  for o, ref in zip(outs, refs): assert ol.rel_err(o.numpy(), ref + r if epi == 1 else ref) <= (2e-4 if epi == 2 else 5e-5)
+
 DENSE = dict(num_blocks=2, dim=512, hidden_dim=768, n_heads=8, n_kv_heads=2, norm_eps=1e-5, vocab_size=512, head_dim=64, rope_theta=500000.0)
 DENSE128 = dict(num_blocks=2, dim=768, hidden_dim=512, n_heads=6, n_kv_heads=6, norm_eps=1e-5, vocab_size=512, head_dim=128, rope_theta=10000.0)
 MOE = dict(num_blocks=2, dim=256, hidden_dim=256, n_heads=4, n_kv_heads=4, norm_eps=1e-5, vocab_size=512, head_dim=64, rope_theta=10000.0, qk_norm=256, num_experts=8, num_experts_per_tok=2)

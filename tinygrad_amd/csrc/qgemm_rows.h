@@ -261,9 +261,156 @@ __global__ __launch_bounds__(256, 2) void qgemm_rows_kernel(const RowsArgs a) {
   rows_store<IS, JS, 0, JS, SW, MOE>(a, acc, lds + wave * ((XU + WU) / 2), rt * (ROWS_WT / 16) + ww * IS, wt * JS, lane, cnt, MOE ? erow : t0);
 }
 
+// ------------------------------------------------------------------------------------------------ 256 weight rows x 128 activation rows
+// Long runs of Q4_0 (the rule: rows_wide, qgemm_rows.hip).  In the kernel above both operands of every product go through LDS: 64 x 64 results per wave read 16 KB for 16 KB of written
+// tile and step, and LDS is busy longer than the matrix cores.  Here a wave owns 64 weight rows for itself and decodes them straight into its A operands: lane (r16, g) of sub-tile i
+// holds the weights of row 16 i + r16 at K position group g of the products, half a unit of 64 at a time, so no weight passes through LDS and none is decoded twice.
+// Only the activations are shared: two halves of 128 rows x 128 values, filled by requests that write LDS themselves, one barrier per half step (128 products of a wave); they are read
+// as 16-byte pieces in the order in which the weights fall out of their blocks (elem).  Twice the results per byte read from LDS, half of its writes.
+// 254 registers at two waves per SIMD are what bounds the formats: Q8_0 and Q4_K, whose half units take twice the registers, were built the same way and were no faster than above.
+// 1023 rows x 4096 -> 2 x 14336 (gate / up) 301 -> 268 us, x 14336 -> 4096 (down) 158 -> 145 us, 2047 rows 603 -> 505 us and 304 -> 271 us.
+#define WIDE_WT 256
+#define WIDE_TT 128
+#define ROWS_WIDE 256             // the tile height that asks a launcher for this kernel
+
+// Natural pairs (b0, b1), (b2, b3) of the four bytes of w, one byte per halfword
+__device__ __forceinline__ uint32_t bytes01(uint32_t w) { return __builtin_amdgcn_perm(0u, w, 0x0c010c00u); }
+__device__ __forceinline__ uint32_t bytes23(uint32_t w) { return __builtin_amdgcn_perm(0u, w, 0x0c030c02u); }
+
+// A buffer descriptor on a wave-uniform address: a request is descriptor + 32-bit lane offset + scalar offset, so that the loop keeps one register per sub-tile where 64-bit lane addresses
+// would take two per load.  Nothing relies on its range check: rows are clamped.
+typedef __amdgpu_buffer_rsrc_t wide_rsrc;
+__device__ __forceinline__ wide_rsrc wide_desc(const void* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, -1, 0x00027000); }
+struct WideRow { wide_rsrc r; uint32_t off; };          // sixteen weight rows and the lane's offset in them
+__device__ __forceinline__ u32x4 bld16(const WideRow& w, uint32_t at) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w.r, w.off, at, 0)); }
+__device__ __forceinline__ uint32_t bld4(const WideRow& w, uint32_t at) { return __builtin_amdgcn_raw_buffer_load_b32(w.r, w.off, at, 0); }
+
+// Half a unit per lane: 32 weights of a row at K positions elem(g, h, v) .. + 7 of the 256 of a step, v = 0 .. 3.  prep: behind the arrival;
+// pair(v, t): weights 4 t .. 4 t + 3 of eight, as fp16 rounded like Fmt::to_f16.
+template <int T> struct WideFmt { static constexpr bool ok = false; };
+template <> struct WideFmt<F_Q4_0P> {                   // block 2 (4 s + g) + h
+  static constexpr bool ok = true;
+  static constexpr uint32_t K0 = 0x64006400u, K1 = 0x54005400u;
+  struct Raw { u32x4 q; uint32_t d; };
+  static __device__ __forceinline__ int elem(int g, int h, int v) { return 64 * g + 32 * h + 8 * v; }
+  static __device__ __forceinline__ uint32_t lane_off(int g) { return 36 * g; }
+  static __device__ __forceinline__ void load(Raw& r, const WideRow& w, int s, int h) { r.q = bld16(w, 144 * s + (h ? 20 : 0)); r.d = bld4(w, 144 * s + 16); }
+  static __device__ __forceinline__ void prep(Raw& r, int h) {
+    if (h) { r.d >>= 16; return; }
+    const uint32_t d = r.q.x & 0xFFFFu;
+    r.q = u32x4{__builtin_amdgcn_alignbit(r.q.y, r.q.x, 16), __builtin_amdgcn_alignbit(r.q.z, r.q.y, 16), __builtin_amdgcn_alignbit(r.q.w, r.q.z, 16), __builtin_amdgcn_alignbit(r.d, r.q.w, 16)};
+    r.d = d;
+  }
+  static __device__ __forceinline__ u32x2 pair(const Raw& r, const uint32_t* kc, int v, int t) {
+    const half2_t d = h2_splat_bits(r.d & 0xFFFFu);
+    uint32_t w = r.q[2 * (v & 1) + t];
+    if (v >= 2) w = vgpr_const(w);                      // (the byte pairs are formed again: kept from v - 2 on they would take sixteen registers)
+    const uint32_t a = bytes01(w), b = bytes23(w);
+    if (v < 2) return u32x2{h2_unbias_scale(and_or(a, 0x000F000Fu, kc[0]), 1032.f, d), h2_unbias_scale(and_or(b, 0x000F000Fu, kc[0]), 1032.f, d)};
+    return u32x2{h2_unbias_scale(and_or(a, 0x00F000F0u, kc[1]), 72.f, d), h2_unbias_scale(and_or(b, 0x00F000F0u, kc[1]), 72.f, d)};
+  }
+};
+
+template <int T, bool SW>
+__global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const RowsArgs a) {
+  using WF = WideFmt<T>;
+  constexpr int HB = WIDE_TT * 256;                                                     // bytes of one half: 128 rows x 128 values
+  // (two variables, so that the compiler knows a read of one half from the requests that fill the other and places no wait between them)
+  __shared__ __attribute__((aligned(16))) uint8_t half0[HB];
+  __shared__ __attribute__((aligned(16))) uint8_t half1[HB];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+  const int nwg = a.row_tiles * a.tok_tiles, per = (nwg + 7) >> 3, b = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  if (((int)blockIdx.x >> 3) >= per || b >= nwg) return;
+  const int rt = b / a.tok_tiles, t0 = (b - rt * a.tok_tiles) * WIDE_TT, cnt = min(a.M - t0, WIDE_TT);
+  const int nsteps = a.K / 256, s0 = (int)((long long)blockIdx.y * nsteps / a.ks), s1 = (int)((long long)(blockIdx.y + 1) * nsteps / a.ks);
+  // This lane's rows.  A sub-tile of sixteen lies in one matrix (its descriptor is wave-uniform); rows beyond the last repeat it, their results are dropped
+  wide_rsrc wr[4]; int wlast[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int last = (int)a.ntot - 1;
+    int row0 = SW ? rt * (WIDE_WT / 2) + wave * 32 + (i >> 1) * 16 : rt * WIDE_WT + wave * 64 + i * 16;
+    row0 = min(row0, last & ~15);
+    wlast[i] = last - row0;
+    const uint8_t* wb = a.w[0];
+    if constexpr (SW) { if (i & 1) wb = a.w[1]; }                                       // (sub-tiles alternate gate / up, so partner values meet in one lane)
+    else if (a.nseg > 1 && row0 >= a.n[0]) { row0 -= (int)a.n[0]; wb = a.w[1]; if (a.nseg > 2 && row0 >= a.n[1]) { row0 -= (int)a.n[1]; wb = a.w[2]; } }
+    wr[i] = wide_desc(wb + (size_t)row0 * a.row_bytes);
+  }
+  // Activations: thread = slot tid & 15 of rows (tid >> 4) + 16 j; slot = piece ^ row, piece 4 v + g = K positions elem(g, h, v) .. + 7
+  const int xr = tid >> 4, piece = (tid & 15) ^ xr, pg = piece & 3, pv = piece >> 2;
+  const wide_rsrc xd = wide_desc(a.x + (size_t)t0 * a.K);
+  const uint32_t xe = (uint32_t)WF::elem(pg, 0, pv) * 2, row_bytes = (uint32_t)a.row_bytes, K2 = (uint32_t)a.K * 2;
+  const int xh = WF::elem(0, 1, 0);                                                     // (the second half lies a constant behind the first)
+  // (lane offsets are formed at each request: eleven registers that the loop has no room for)
+  auto xrequest = [&](uint8_t* buf, int s, int h, int j) __attribute__((always_inline)) {     // piece of lane l of wave w, row group j: LDS byte 4096 j + 1024 w + 16 l
+    int row = xr; asm volatile("" : "+v"(row));
+    const uint32_t off = __umul24((uint32_t)min(row + 16 * j, cnt - 1), K2) + xe;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xd, (__attribute__((address_space(3))) void*)(buf + j * 4096 + wave * 1024), 16, off, 512 * s + 2 * h * xh, 0, 0);
+  };
+  auto wrow = [&](int i) __attribute__((always_inline)) {
+    int row = r16; asm volatile("" : "+v"(row));
+    return WideRow{wr[i], __umul24((uint32_t)min(row, wlast[i]), row_bytes) + WF::lane_off(g)};
+  };
+  uint32_t kc[2] = {vgpr_const(WF::K0), vgpr_const(WF::K1)};
+  v4f32 acc[4][8];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 8; j++) acc[i][j] = v4f32{0.f, 0.f, 0.f, 0.f};
+  typename WF::Raw raw[4], nxt[4];
+#pragma unroll
+  for (int j = 0; j < 8; j++) xrequest(half0, s0, 0, j);
+#pragma unroll
+  for (int i = 0; i < 4; i++) WF::load(nxt[i], wrow(i), s0, 0);
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  for (int s = s0; s < s1; s++) {
+    const int sn = min(s + 1, s1 - 1);                                                  // (behind the last step the requests repeat it; nothing reads what they bring)
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      uint8_t* const here = h ? half1 : half0; uint8_t* const there = h ? half0 : half1;
+      const int st = h ? sn : s;                                                        // step of the next half
+      u32x4 w[2][4]; v8f16 x[3];
+      auto xread = [&](int n) __attribute__((always_inline)) { return *(const v8f16*)(here + r16 * 256 + (((4 * (n >> 3) + g) ^ r16) << 4) + (n & 7) * 4096); };
+      x[0] = xread(0); x[1] = xread(1);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        raw[i] = nxt[i];
+        WF::prep(raw[i], h);
+        const u32x2 p = WF::pair(raw[i], kc, 0, 0), q = WF::pair(raw[i], kc, 0, 1);
+        w[0][i] = u32x4{p.x, p.y, q.x, q.y};
+      }
+      // 32 groups of four products, in this order: with each, the activations of two groups further are read, four weights of the next eight of a sub-tile are decoded, and one
+      // request of the next half is made
+#pragma unroll
+      for (int n = 0; n < 32; n++) {
+        const int v = n >> 3, j = n & 7;
+        if (n + 2 < 32) x[(n + 2) % 3] = xread(n + 2);
+        if (v == 0) xrequest(there, st, h ^ 1, j);
+        if (v == 1 && j < 4) WF::load(nxt[j], wrow(j), st, h ^ 1);
+        if (v < 3) {
+          const u32x2 p = WF::pair(raw[j >> 1], kc, v + 1, j & 1);
+          u32x4& d = w[(v + 1) & 1][j >> 1];
+          if (j & 1) { d.z = p.x; d.w = p.y; } else { d.x = p.x; d.y = p.y; }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8f16, w[v & 1][i]), x[n % 3], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");          // what this half has requested is there; every wave has read its own
+    }
+  }
+  // (a wave's results in two halves of 64 rows, 16 KB each: its quarter of LDS; every wave is behind the last barrier)
+  rows_store<4, 8, 0, 4, SW, false>(a, acc, (wave < 2 ? half0 : half1) + (wave & 1) * (HB / 2), rt * (WIDE_WT / 16) + wave * 4, 0, lane, cnt, t0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  rows_store<4, 8, 4, 4, SW, false>(a, acc, (wave < 2 ? half0 : half1) + (wave & 1) * (HB / 2), rt * (WIDE_WT / 16) + wave * 4, 4, lane, cnt, t0);
+}
+
 template <int T, bool MOE> int rows_launch_tt(const RowsArgs& a, int tt, unsigned grid, hipStream_t s) {
   const dim3 g(grid, a.ks);
   const bool sw = a.epi == ROWS_SWIGLU;
+  if constexpr (!MOE && WideFmt<T>::ok) {
+    if (tt == ROWS_WIDE) { if (sw) qgemm_wide_kernel<T, true><<<g, 256, 0, s>>>(a); else qgemm_wide_kernel<T, false><<<g, 256, 0, s>>>(a); TGA_LAUNCH_CHECK(); return 0; }
+  }
   if (tt == 128) { if (sw) qgemm_rows_kernel<T, 128, true, MOE><<<g, 256, 0, s>>>(a); else qgemm_rows_kernel<T, 128, false, MOE><<<g, 256, 0, s>>>(a); }
   else if (tt == 64) { if (sw) qgemm_rows_kernel<T, 64, true, MOE><<<g, 256, 0, s>>>(a); else qgemm_rows_kernel<T, 64, false, MOE><<<g, 256, 0, s>>>(a); }
   else { if (sw) qgemm_rows_kernel<T, 32, true, MOE><<<g, 256, 0, s>>>(a); else qgemm_rows_kernel<T, 32, false, MOE><<<g, 256, 0, s>>>(a); }

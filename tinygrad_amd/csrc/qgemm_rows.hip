@@ -60,19 +60,31 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(const RowsArgs a) {
   }
 }
 
-// Tile height and K split for M rows of one set of matrices: rows of at most 32 / 64 take the lower tiles; K is split while the tiles leave CUs with fewer than two workgroups
-static void rows_plan(long long row_tiles, int M, int K, bool may_split, size_t part_bytes, long long ntot, int* tt, int* ks) {
-  *tt = M <= 32 ? 32 : M <= 64 ? 64 : 128;
-  const long long wgs = row_tiles * ((M + *tt - 1) / *tt);
-  int k = 1;
-  if (may_split) {
-    k = (int)(512 / (wgs > 0 ? wgs : 1));
-    const int kmax = K / ROWS_KS / 4;
-    if (k > kmax) k = kmax;
-    while (k > 1 && (size_t)k * M * ntot * 4 > part_bytes) k--;
-    if (k < 1) k = 1;
-  }
-  *ks = k;
+// How a set of matrices is cut: tiles (tt: ROWS_WIDE or the activation rows of a tile of ROWS_WT weight rows) and the split of K, which is cut while the tiles leave CUs with fewer than
+// two workgroups and a part keeps at least `least` values of it.
+static int rows_split(const RowsArgs& a, bool may_split, size_t part_bytes, int least) {
+  if (!may_split) return 1;
+  int k = (int)(512 / ((long long)a.row_tiles * a.tok_tiles));
+  if (k > a.K / least) k = a.K / least;
+  while (k > 1 && (size_t)k * a.M * a.ntot * 4 > part_bytes) k--;
+  return k < 1 ? 1 : k;
+}
+// The 256 x 128 tiles: a workgroup's start and end cost about 4 us more than the smaller tile's, so it takes them where a workgroup has twelve steps of 256 or more and at least 320 of
+// them are running (4096 -> 6144 of 1023 rows, eight steps each: 87 us, the smaller tiles 83; 2047 rows, sixteen steps: 141 and 144; 4096 -> 2 x 14336 of 300 rows, 336 workgroups: 140 and 146,
+// of 128 rows, 112 workgroups: 79 and 62).
+static bool rows_wide(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t part_bytes) {
+  if (fmt != F_Q4_0P || a.M <= 64 || a.K % 256 || a.K > (1 << 20) || a.ntot >= (1ll << 30)) return false;
+  const int wt = swiglu ? WIDE_WT / 2 : WIDE_WT;
+  a.row_tiles = (int)((a.ntot + wt - 1) / wt); a.tok_tiles = (a.M + WIDE_TT - 1) / WIDE_TT;
+  a.ks = rows_split(a, may_split, part_bytes, 512);
+  return a.K / 256 / a.ks >= 12 && (long long)a.row_tiles * a.tok_tiles * a.ks >= 320;
+}
+static int rows_plan(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t part_bytes) {
+  if (rows_wide(a, fmt, swiglu, may_split, part_bytes)) return ROWS_WIDE;
+  const int tt = a.M <= 32 ? 32 : a.M <= 64 ? 64 : 128, wt = swiglu ? ROWS_WT / 2 : ROWS_WT;
+  a.row_tiles = (int)((a.ntot + wt - 1) / wt); a.tok_tiles = (a.M + tt - 1) / tt;
+  a.ks = rows_split(a, may_split, part_bytes, 4 * ROWS_KS);
+  return tt;
 }
 
 extern "C" {
@@ -97,12 +109,9 @@ int tga_qlinear_many(int ggml_type, int nseg, const void* const* w, void* const*
   TGA_REQUIRE((((uintptr_t)x_f16 | (uintptr_t)resid | (uintptr_t)workspace) & 15) == 0, "tga_qlinear_many: activations must be 16-byte aligned");
   a.row_bytes = tga_rows_row_bytes(fmt, K); a.x = (const uint16_t*)x_f16; a.resid = resid; a.part = (float*)workspace; a.nseg = segs; a.epi = epilogue; a.y_f32 = y_dtype == TGA_F32;
   a.M = (int)M; a.K = (int)K;
-  a.row_tiles = (int)((a.ntot + (epilogue == 2 ? ROWS_WT / 2 : ROWS_WT) - 1) / (epilogue == 2 ? ROWS_WT / 2 : ROWS_WT));
   bool split = epilogue != 2 && workspace && a.ntot % 4 == 0;
   for (int i = 0; i < segs; i++) split = split && n[i] % 4 == 0;
-  int tt;
-  rows_plan(a.row_tiles, (int)M, (int)K, split, (size_t)workspace_bytes, a.ntot, &tt, &a.ks);
-  a.tok_tiles = (int)((M + tt - 1) / tt);
+  const int tt = rows_plan(a, fmt, epilogue == 2, split, (size_t)workspace_bytes);
   if (a.ks > 1) a.epi = ROWS_PART;
   const unsigned grid = (unsigned)(((long long)a.row_tiles * a.tok_tiles + 7) / 8 * 8);
   if (const int rc = tga_rows_dispatch(fmt, a, tt, grid, (hipStream_t)stream)) return rc;
