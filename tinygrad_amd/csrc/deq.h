@@ -1,4 +1,5 @@
 // Bit-exact block decode of ggml_data_to_tensor (tinygrad/llm/gguf.py:23-119): 4 consecutive elements of one block at a time.
+// The four codes lie in four neighbouring bytes (or fewer) at any address: one dword request, not four of a byte.
 // Float contraction is off inside every get4: each product must round exactly like the reference's separate multiplies.
 #pragma once
 #include "common.h"
@@ -12,9 +13,9 @@ template <> struct Deq<GGML_Q4_0> {
   static __device__ __forceinline__ void get4(const uint8_t* b, int e0, float* o) {
 #pragma clang fp contract(off)
     const float d = h2f_bits(ld2(b));
-    const int sh = (e0 >= 16) ? 4 : 0; const uint8_t* q = b + 2 + (e0 & 15);
+    const uint32_t q = ld4(b + 2 + (e0 & 15)) >> ((e0 >= 16) ? 4 : 0);
 #pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = (float)((int)((q[i] >> sh) & 0xF) - 8) * d;
+    for (int i = 0; i < 4; i++) o[i] = (float)((int)((q >> (8 * i)) & 0xF) - 8) * d;
   }
 };
 // Q4_1 (20 B: d, m, qs[16]), tinygrad/llm/gguf.py:47-49: q * d + m
@@ -23,9 +24,9 @@ template <> struct Deq<GGML_Q4_1> {
   static __device__ __forceinline__ void get4(const uint8_t* b, int e0, float* o) {
 #pragma clang fp contract(off)
     const float d = h2f_bits(ld2(b)), m = h2f_bits(ld2(b + 2));
-    const int sh = (e0 >= 16) ? 4 : 0; const uint8_t* q = b + 4 + (e0 & 15);
+    const uint32_t q = ld4(b + 4 + (e0 & 15)) >> ((e0 >= 16) ? 4 : 0);
 #pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = (float)((q[i] >> sh) & 0xF) * d + m;
+    for (int i = 0; i < 4; i++) o[i] = (float)((q >> (8 * i)) & 0xF) * d + m;
   }
 };
 // Q5_0 (22 B: d, qh[4], qs[16]) and Q5_1 (24 B: d, m, qh[4], qs[16]), tinygrad/llm/gguf.py:50-55: q = nibble + 16 * bit e of the
@@ -36,10 +37,9 @@ template <bool ONE> struct DeqQ5 {
 #pragma clang fp contract(off)
     const float d = h2f_bits(ld2(b)), off = ONE ? h2f_bits(ld2(b + 2)) : -16.0f * d;
     const uint8_t* p = b + (ONE ? 4 : 2);
-    const uint32_t qh = (uint32_t)ld2(p) | ((uint32_t)ld2(p + 2) << 16);
-    const int sh = (e0 >= 16) ? 4 : 0; const uint8_t* q = p + 4 + (e0 & 15);
+    const uint32_t qh = ld4(p), q = ld4(p + 4 + (e0 & 15)) >> ((e0 >= 16) ? 4 : 0);
 #pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = (float)(((q[i] >> sh) & 0xF) | (((qh >> (e0 + i)) & 1u) << 4)) * d + off;
+    for (int i = 0; i < 4; i++) o[i] = (float)(((q >> (8 * i)) & 0xF) | (((qh >> (e0 + i)) & 1u) << 4)) * d + off;
   }
 };
 template <> struct Deq<GGML_Q5_0> : DeqQ5<false> {};
@@ -49,8 +49,9 @@ template <> struct Deq<GGML_Q8_0> {
   static __device__ __forceinline__ void get4(const uint8_t* b, int e0, float* o) {
 #pragma clang fp contract(off)
     const float d = h2f_bits(ld2(b));
+    const uint32_t q = ld4(b + 2 + e0);
 #pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = d * (float)(int8_t)b[2 + e0 + i];
+    for (int i = 0; i < 4; i++) o[i] = d * (float)(int8_t)(q >> (8 * i));
   }
 };
 template <> struct Deq<GGML_Q6_K> {
@@ -59,13 +60,11 @@ template <> struct Deq<GGML_Q6_K> {
 #pragma clang fp contract(off)
     const float d = h2f_bits(ld2(b + 208));
     const int half = e0 >> 7, r = e0 & 127, j = r >> 5, l = r & 31;      // element = 128*half + 32*j + l
-    const uint8_t* ql = b + 64 * half + ((j & 1) ? 32 : 0) + l;
-    const uint8_t* qh = b + 128 + 32 * half + l;
+    const uint32_t ql = ld4(b + 64 * half + ((j & 1) ? 32 : 0) + l) >> ((j & 2) ? 4 : 0), qh = ld4(b + 128 + 32 * half + l) >> (2 * j);
     const float sc = (float)(int8_t)b[192 + (e0 >> 4)];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int lo = (j & 2) ? (ql[i] >> 4) : (ql[i] & 0xF);
-      const int q = (int)(int8_t)(lo | (((qh[i] >> (2 * j)) & 3) << 4)) - 32;
+      const int q = (int)(((ql >> (8 * i)) & 0xF) | (((qh >> (8 * i)) & 3) << 4)) - 32;
       o[i] = (d * (float)q) * sc;                                        // reference association: (d * q) * scale
     }
   }
@@ -77,20 +76,15 @@ template <bool FIVE> struct DeqK45 {
   static constexpr int NEL = 256, NBY = FIVE ? 176 : 144;
   static __device__ __forceinline__ void get4(const uint8_t* b, int e0, float* o) {
 #pragma clang fp contract(off)
-    const float d = h2f_bits(ld2(b)), dmin = h2f_bits(ld2(b + 2));
-    const int sb = e0 >> 5, l = e0 & 31;
-    const uint8_t* s = b + 4;
-    int sc, mn;
-    if (sb < 4) { sc = s[sb] & 63; mn = s[sb + 4] & 63; }
-    else { sc = (s[sb + 4] & 0xF) | ((s[sb - 4] >> 6) << 4); mn = (s[sb + 4] >> 4) | ((s[sb] >> 6) << 4); }
+    const u32x4 h = ld16(b);                                             // d, dmin and all twelve scale bytes
+    const float d = h2f_bits(h.x & 0xFFFFu), dmin = h2f_bits(h.x >> 16);
+    const int sb = e0 >> 5, l = e0 & 31, sh = 8 * (sb & 3);
+    const uint32_t y = h.y >> sh, z = h.z >> sh, w = h.w >> sh;
+    const uint32_t sc = sb < 4 ? y & 63 : (w & 0xF) | (((y >> 6) & 3) << 4), mn = sb < 4 ? z & 63 : ((w >> 4) & 0xF) | (((z >> 6) & 3) << 4);
     const float d1 = d * (float)sc, m1 = dmin * (float)mn;
-    const uint8_t* q = b + (FIVE ? 48 : 16) + 32 * (sb >> 1) + l;
+    const uint32_t q = ld4(b + (FIVE ? 48 : 16) + 32 * (sb >> 1) + l) >> (4 * (sb & 1)), q5 = FIVE ? ld4(b + 16 + l) >> sb : 0;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      int v = (sb & 1) ? (q[i] >> 4) : (q[i] & 0xF);
-      if (FIVE) v += ((b[16 + l + i] >> sb) & 1) << 4;
-      o[i] = d1 * (float)v - m1;
-    }
+    for (int i = 0; i < 4; i++) o[i] = d1 * (float)(((q >> (8 * i)) & 0xF) | (((q5 >> (8 * i)) & 1) << 4)) - m1;
   }
 };
 template <> struct Deq<GGML_Q4_K> : DeqK45<false> {};
@@ -112,9 +106,9 @@ template <> struct Deq<GGML_IQ4_XS> {
     const int ib = e0 >> 5, l = e0 & 31;
     const int ls = (int)(((b[4 + (ib >> 1)] >> (4 * (ib & 1))) & 0xF) | (((sh >> (2 * ib)) & 3) << 4));
     const float dl = d * (float)(ls - 32);
-    const int hi = (l >= 16) ? 4 : 0; const uint8_t* q = b + 8 + 16 * ib + (l & 15);
+    const uint32_t q = ld4(b + 8 + 16 * ib + (l & 15)) >> ((l >= 16) ? 4 : 0);
 #pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = dl * iq4nl_value((q[i] >> hi) & 0xF);
+    for (int i = 0; i < 4; i++) o[i] = dl * iq4nl_value((q >> (8 * i)) & 0xF);
   }
 };
 // The codebook types (tinygrad/llm/gguf.py:73-95).  A codebook entry is kept as its digits over the codebook's alphabet (iq_grids.h); sign bit k
@@ -129,7 +123,7 @@ template <> struct Deq<GGML_IQ3_XXS> {
     const float d = h2f_bits(ld2(b));
     const int ib = e0 >> 5, l = (e0 >> 3) & 3;
     const uint8_t* w = b + 66 + 4 * ib;
-    const uint32_t aux = (uint32_t)ld2(w) | ((uint32_t)ld2(w + 2) << 16);
+    const uint32_t aux = ld4(w);
     const float db = d * ((float)(aux >> 28) + 0.5f) * 0.5f;
     const uint32_t s7 = (aux >> (7 * l)) & 127u, signs = (s7 | ((__builtin_popcount(s7) & 1u) << 7)) >> (e0 & 4);
     const uint32_t code = IQ3XXS_CODE[b[2 + (e0 >> 2)]];
@@ -191,10 +185,10 @@ template <> struct Deq<GGML_MXFP4> {
 #pragma clang fp contract(off)
     const uint32_t e = b[0];
     const float d = __builtin_bit_cast(float, e < 2 ? (0x00200000u << e) : ((e - 1) << 23));   // 2^(e-128)
-    const int sh = (e0 >= 16) ? 4 : 0; const uint8_t* q = b + 1 + (e0 & 15);
+    const uint32_t q = ld4(b + 1 + (e0 & 15)) >> ((e0 >= 16) ? 4 : 0);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const uint32_t c = (q[i] >> sh) & 0xF, mag = c & 7;
+      const uint32_t c = (q >> (8 * i)) & 0xF, mag = c & 7;
       // doubled E2M1 table {0,1,2,3,4,6,8,12}; bit 3 is the sign (code 8 is -0.0 in the reference's float LUT)
       const float v = (float)(mag < 4 ? mag : (mag < 6 ? 2 * mag - 4 : 4 * mag - 16));
       o[i] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) | ((c & 8) << 28)) * d;
