@@ -28,6 +28,13 @@ __global__ __launch_bounds__(256) void rows_rope_kernel(const RopeArgs a) {
   const int nq = a.H * a.hd, nk = a.KV * a.hd;
   if (r == 0) for (int i = tid; i < a.n_zero; i += 256) a.zero[i] = 0;
   const float* q = a.q + (size_t)r * nq; const float* k = a.k + (size_t)r * nk; const float* v = a.v + (size_t)r * nk;
+  const size_t crow = ((size_t)z * a.KV * a.max_ctx + pos) * a.hd, cstep = (size_t)a.max_ctx * a.hd;
+#pragma unroll 2
+  for (int e = 4 * tid; e < nk; e += 1024) {
+    const int hh = e / a.hd;
+    const f32x4 x = *(const f32x4*)(v + e);
+    *(u32x2*)(a.cv + crow + hh * cstep + (e - hh * a.hd)) = u32x2{f2h_bits(x.x) | (f2h_bits(x.y) << 16), f2h_bits(x.z) | (f2h_bits(x.w) << 16)};
+  }
   float qs = 1.f, ks = 1.f;
   if (a.norm == 1) {
     float s0 = 0.f, s1 = 0.f;
@@ -40,35 +47,47 @@ __global__ __launch_bounds__(256) void rows_rope_kernel(const RopeArgs a) {
     ks = 1.0f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)nk + a.eps);
   }
   const float* rr = a.rope + (size_t)pos * a.hd;
-  const size_t crow = ((size_t)z * a.KV * a.max_ctx + pos) * a.hd, cstep = (size_t)a.max_ctx * a.hd;
   const bool live = lane < half;                                          // (half is 32 or 64)
   const int i = live ? lane : half - 1;
   const float c = rr[i], s = rr[half + i];
-  for (int h = wave; h < a.H + a.KV; h += 4) {
-    const bool isq = h < a.H;
-    const int hh = isq ? h : h - a.H;
-    const float* src = isq ? q + hh * a.hd : k + hh * a.hd;
-    float x1 = src[i], x2 = src[half + i];
-    if (a.norm) {
-      float sc = isq ? qs : ks;
-      if (a.norm == 2) sc = 1.0f / sqrtf(wave_sum(live ? x1 * x1 + x2 * x2 : 0.f) / (float)a.hd + a.eps);
-      const float* w = isq ? a.qn : a.kn;
-      const int wo = a.norm == 2 ? 0 : hh * a.hd;
-      x1 = (x1 * sc) * w[wo + i]; x2 = (x2 * sc) * w[wo + half + i];
+  // (a wave's heads in groups of RU, whose values are requested together: a head at a time, the ten heads of a wave are ten trips to memory)
+  constexpr int RU = 5;
+  const int nh = a.H + a.KV;
+  for (int h0 = wave; h0 < nh; h0 += 4 * RU) {
+    float xa[RU], xb[RU];
+#pragma unroll
+    for (int u = 0; u < RU; u++) {
+      const int h = min(h0 + 4 * u, nh - 1);
+      const float* src = h < a.H ? q + h * a.hd : k + (h - a.H) * a.hd;
+      xa[u] = src[i]; xb[u] = src[half + i];
     }
-    const float lo = __builtin_fmaf(x1, c, -(x2 * s)), hi = __builtin_fmaf(x2, c, x1 * s);
-    if (!live) continue;
-    if (isq) {
-      const size_t o = (size_t)r * nq + hh * a.hd + i;
-      const _Float16 l16 = (_Float16)lo, h16 = (_Float16)hi;
-      a.qh[o] = __builtin_bit_cast(uint16_t, l16); a.qh[o + half] = __builtin_bit_cast(uint16_t, h16);
-      a.ql[o] = (uint16_t)f2h_bits(lo - (float)l16); a.ql[o + half] = (uint16_t)f2h_bits(hi - (float)h16);
-    } else {
-      uint16_t* d = a.ck + crow + hh * cstep;
-      d[i] = (uint16_t)f2h_bits(lo); d[half + i] = (uint16_t)f2h_bits(hi);
+#pragma unroll
+    for (int u = 0; u < RU; u++) {
+      const int h = h0 + 4 * u;
+      if (h >= nh) break;
+      const bool isq = h < a.H;
+      const int hh = isq ? h : h - a.H;
+      float x1 = xa[u], x2 = xb[u];
+      if (a.norm) {
+        float sc = isq ? qs : ks;
+        if (a.norm == 2) sc = 1.0f / sqrtf(wave_sum(live ? x1 * x1 + x2 * x2 : 0.f) / (float)a.hd + a.eps);
+        const float* w = isq ? a.qn : a.kn;
+        const int wo = a.norm == 2 ? 0 : hh * a.hd;
+        x1 = (x1 * sc) * w[wo + i]; x2 = (x2 * sc) * w[wo + half + i];
+      }
+      const float lo = __builtin_fmaf(x1, c, -(x2 * s)), hi = __builtin_fmaf(x2, c, x1 * s);
+      if (!live) continue;
+      if (isq) {
+        const size_t o = (size_t)r * nq + hh * a.hd + i;
+        const _Float16 l16 = (_Float16)lo, h16 = (_Float16)hi;
+        a.qh[o] = __builtin_bit_cast(uint16_t, l16); a.qh[o + half] = __builtin_bit_cast(uint16_t, h16);
+        a.ql[o] = (uint16_t)f2h_bits(lo - (float)l16); a.ql[o + half] = (uint16_t)f2h_bits(hi - (float)h16);
+      } else {
+        uint16_t* d = a.ck + crow + hh * cstep;
+        d[i] = (uint16_t)f2h_bits(lo); d[half + i] = (uint16_t)f2h_bits(hi);
+      }
     }
   }
-  for (int e = tid; e < nk; e += 256) { const int hh = e / a.hd; a.cv[crow + hh * cstep + (e - hh * a.hd)] = (uint16_t)f2h_bits(v[e]); }
 }
 
 // ------------------------------------------------------------------------------------------------ attention
