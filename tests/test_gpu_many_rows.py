@@ -109,6 +109,20 @@ def test_prefill_of_many_rows_vs_position_by_position(gpu, monkeypatch, cfg, kw,
   for m in (a, b): m.prefill(longer); m.decode_step(); m.check_state()
   assert ol.rel_err(a.logits(), b.logits()) <= 2e-3
 
+@pytest.mark.parametrize("dim", [2048, 2304, 4352, 8192, 8448])
+def test_prefill_rows_of_every_norm_width(gpu, dim):
+  """The norm behind a linear keeps its row in one, two or four vectors per thread (up to 2048, 4096, 8192 values) and is a launch of its own beyond: the same bars as above."""
+  cfg = dict(num_blocks=2, dim=dim, hidden_dim=512, n_heads=4, n_kv_heads=2, norm_eps=1e-5, vocab_size=256, head_dim=64, rope_theta=10000.0)
+  a, b = _model(cfg, 7, 64), _model(cfg, 7, 64)
+  b.prefill_chunk = 1
+  prompt = np.random.default_rng(dim).integers(0, 256, size=40).tolist()
+  for m in (a, b): m.prefill(prompt)
+  assert (a._chunker or a._tail_chunkers[16]).x is None
+  for ba, bb in zip(a.blk, b.blk):
+    for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): assert ol.rel_err(ca.numpy().astype(np.float32), cb.numpy().astype(np.float32)) <= 2e-3
+  for m in (a, b): m.decode_step()
+  assert ol.rel_err(a.logits(), b.logits()) <= 2e-3
+
 @pytest.mark.parametrize("cfg,B,n", [(DENSE, 3, 7), (DENSE, 5, 70), (DENSE128, 2, 33), (MOE, 4, 20), (MOE, 1, 40)], ids=["dense-3x7", "dense-5x70", "hd128-2x33", "moe-4x20", "moe-1x40"])
 @pytest.mark.parametrize("rows", [2048, 24])
 def test_batched_prefill_of_many_rows_vs_step_by_step(gpu, monkeypatch, cfg, B, n, rows):

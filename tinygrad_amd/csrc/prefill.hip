@@ -1,9 +1,9 @@
 // A prefill step of any number of rows: the positions pos0 .. pos0 + P - 1 of one or more sequences go through all blocks together (the reference's chunked prefill,
-// tinygrad/llm/model.py:464, 476-481, with the prompt as one chunk), every linear as ONE pass over its weights (qgemm_rows.h).  Per block: norm -> q / k / v -> rotation +
-// append -> attention -> attn_output (+ residual) -> norm -> gate / up + SwiGLU -> down (+ residual): nine launches, or for a MoE block norm -> router logits -> gating ->
+// tinygrad/llm/model.py:464, 476-481, with the prompt as one chunk), every linear as ONE pass over its weights (qgemm_rows.h).  Per block: q / k / v -> rotation +
+// append -> attention -> attn_output (+ residual, norm) -> gate / up + SwiGLU -> down (+ residual, the next block's norm): eight launches and the sums of a split q / k / v, or for a MoE block norm -> router logits -> gating ->
 // grouping -> selected experts' gate / up + SwiGLU -> down -> weighted sum (+ residual), model.py:110-135.  The launches are issued by one native call.
-// MI355X, prompt to first logits: 8B-arch Q4_0 of 1024 tokens 42.6 ms (steps of 128 rows, qgemm64.hip) -> 23.8; OLMoE-arch of 512 tokens 64.0 (steps of 16 rows, an expert GEMV per
-// token and slot) -> 5.9; four 8B-arch Q4_K_M sequences of 128 tokens 334 (one lockstep step per position) -> 17.0.
+// MI355X, prompt to first logits: 8B-arch Q4_0 of 1024 tokens 42.4 ms (steps of 128 rows, qgemm64.hip) -> 21.4; OLMoE-arch of 512 tokens 64.0 (steps of 16 rows, an expert GEMV per
+// token and slot) -> 5.5; four 8B-arch Q4_K_M sequences of 128 tokens 333 (one lockstep step per position) -> 15.6.
 #include "qgemm_rows.h"
 #include "decode.h"
 #include "moe_gate.h"
@@ -12,6 +12,9 @@
 int tga_rows_fmt(int ggml_type, int64_t K);                                              // qgemm_rows.hip
 int64_t tga_rows_row_bytes(int fmt, int64_t K);
 int tga_rows_dispatch(int fmt, const RowsArgs& a, int tt, unsigned grid, hipStream_t s);
+int tga_rows_linear(int ggml_type, int nseg, const void* const* w, void* const* y, const int64_t* n, const void* x_f16, int y_dtype, int64_t M, int64_t K, int epilogue, const float* resid,
+                    void* workspace, int64_t workspace_bytes, const float* norm_w, float norm_eps, void* xn, void* stream);
+int tga_rows_norm(float* x, const float* w, int M, int n, float eps, void* xn, void* stream);
 
 // ------------------------------------------------------------------------------------------------ rotation + append
 // One workgroup per row.  q is rotated (after its norm) and leaves as TWO fp16 values per element, the rounded value and what the rounding left over, so that the matrix-core
@@ -325,12 +328,17 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
   auto linear = [&](int type, int nseg, const void* const* wt, void* const* y, const int64_t* n, const void* in, int ydt, int64_t K, int epi, const float* resid) {
     return tga_qlinear_many(type, nseg, wt, y, n, in, ydt, R, K, epi, resid, ws + w.part, (int64_t)PF_PART, stream);
   };
+  // x += in . W^T, and xn = the norm that follows (norm nullptr: nothing follows)
+  auto linear_norm = [&](int type, int64_t wp, const void* in, int64_t K, const float* norm) {
+    const void* wt[1] = {(const void*)wp}; void* y[1] = {x}; const int64_t n[1] = {dim};
+    return tga_rows_linear(type, 1, wt, y, n, in, TGA_F32, R, K, 1, x, ws + w.part, (int64_t)PF_PART, norm, eps, xn, stream);
+  };
   PF_DO(tga_embed_rows((const void*)m[PM_EMB], (int)m[PM_EMB_TYPE], (int)dim, tokens, (int)R, state, x, stream));
   for (int64_t bi = 0; bi < m[PM_NBLOCKS]; bi++) {
     const int64_t* b = blocks + bi * PB_COUNT;
     const bool pending = bi > 0 && blocks[(bi - 1) * PB_COUNT + PB_MOE];  // the block before left its weighted expert sum to this norm
     if (pending) PF_DO(tga_moe_combine_rmsnorm_rows((float*)(ws + w.y_e), (float*)(ws + w.probs), x, (const float*)b[PB_ATTN_NORM], (int)R, (int)k, (int)dim, eps, xn, nullptr, stream));
-    else PF_DO(tga_rmsnorm_rows(x, (const float*)b[PB_ATTN_NORM], (int)R, (int)dim, eps, xn, nullptr, 0, stream));
+    else if (bi == 0) PF_DO(tga_rows_norm(x, (const float*)b[PB_ATTN_NORM], (int)R, (int)dim, eps, xn, stream));      // (later ones come behind the block before)
     const void* wt[3] = {(const void*)b[PB_WQ], (const void*)b[PB_WK], (const void*)b[PB_WV]};
     void* y[3] = {q, kk, v}; const int64_t n[3] = {nq, nk, nk};
     for (int i = 0; i < 3;) {                                             // one launch per run of equal block types
@@ -353,14 +361,12 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
     const unsigned ag = (unsigned)(aa.qtiles * H * nseq);
     if (hd == 64) rows_attn_kernel<64><<<ag, 256, 0, s>>>(aa); else rows_attn_kernel<128><<<ag, 256, 0, s>>>(aa);
     TGA_LAUNCH_CHECK();
-    { const void* wo[1] = {(const void*)b[PB_WO]}; void* yo[1] = {x}; const int64_t no[1] = {dim}; PF_DO(linear((int)b[PB_TO], 1, wo, yo, no, attn, TGA_F32, nq, 1, x)); }
-    PF_DO(tga_rmsnorm_rows(x, (const float*)b[PB_FFN_NORM], (int)R, (int)dim, eps, xn, nullptr, 0, stream));
+    PF_DO(linear_norm((int)b[PB_TO], b[PB_WO], attn, nq, (const float*)b[PB_FFN_NORM]));
     if (!b[PB_MOE]) {
       const int64_t h = E ? m[PM_DENSE_HIDDEN] : m[PM_HIDDEN];
       const void* wg[2] = {(const void*)b[PB_GATE], (const void*)b[PB_UP]}; void* yg[2] = {act, nullptr}; const int64_t ng[2] = {h, h};
       PF_DO(linear((int)b[PB_TGATE], 2, wg, yg, ng, xn, TGA_F16, dim, 2, nullptr));
-      const void* wd[1] = {(const void*)b[PB_DOWN]}; void* yd[1] = {x}; const int64_t nd[1] = {dim};
-      PF_DO(linear((int)b[PB_TDOWN], 1, wd, yd, nd, act, TGA_F32, h, 1, x));
+      PF_DO(linear_norm((int)b[PB_TDOWN], b[PB_DOWN], act, h, bi + 1 < m[PM_NBLOCKS] ? (const float*)blocks[(bi + 1) * PB_COUNT + PB_ATTN_NORM] : nullptr));
       continue;
     }
     float* logits = (float*)(ws + w.logits); int* counts = (int*)(ws + w.counts); int* sel = (int*)(ws + w.sel); int* place = (int*)(ws + w.place);
