@@ -60,15 +60,18 @@ template <> struct RowsFmt<GGML_MXFP4> {                // two blocks of 32
   static constexpr int NKC = F::NKC;
   static __device__ __forceinline__ Raw load(const uint8_t* row, int u) { Raw r; r.b[0] = F::load(row, 2 * u); r.b[1] = F::load(row, 2 * u + 1); return r; }
   static __device__ __forceinline__ int elem(int u, int v) { return 64 * u + 8 * v; }
+  // A byte of a block holds weights e and e + 16: two neighbours are put into one byte first (shifts and a bit-field insert for two pairs), so that the conversions give natural pairs and
+  // nothing is packed behind them; the kernel's loop is bound by its VALU work here (150 -> 118 operations for 32 products of a wave at 64 rows)
   static __device__ __forceinline__ void nat(const Raw& r, const uint32_t*, u32x4* out) {
+    const uint32_t M = vgpr_const(0x000F000Fu);         // (a register: of a constant mask the compiler makes two operations instead of v_bfi)
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-      uint32_t wv[F::NWV];
-      F::to_f16(r.b[h], wv);                            // dword q: (element q, element q + 16)
+      const float sc = __builtin_bit_cast(float, r.b[h].e ? (r.b[h].e << 23) : 0x00400000u);
 #pragma unroll
-      for (int k = 0; k < 8; k++) {
-        out[4 * h + (k >> 2)][k & 3] = pack_even(wv[2 * k], wv[2 * k + 1]);
-        out[4 * h + 2 + (k >> 2)][k & 3] = pack_odd(wv[2 * k], wv[2 * k + 1]);
+      for (int t = 0; t < 4; t++) {
+        const uint32_t w = r.b[h].q[t], s4 = w >> 4, s8 = w >> 8, lo = (M & w) | (~M & s4), hi = (M & s4) | (~M & s8);
+        out[4 * h + (t >> 1)][2 * (t & 1)] = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 0)); out[4 * h + (t >> 1)][2 * (t & 1) + 1] = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 2));
+        out[4 * h + 2 + (t >> 1)][2 * (t & 1)] = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 0)); out[4 * h + 2 + (t >> 1)][2 * (t & 1) + 1] = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 2));
       }
     }
   }
