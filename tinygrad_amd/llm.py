@@ -55,6 +55,7 @@ OLMOE = dict(num_blocks=16, dim=2048, hidden_dim=1024, n_heads=16, n_kv_heads=16
 
 MANY_ROWS = 2048                   # rows of a prefill step at most (its buffers grow with the rows: 0.5 GB for the 8B architecture)
 MANY_ROWS_MIN = 17                 # fewer rows are one step of the small-batch kernels
+MANY_ROWS_POSITIONS = 4            # sequences in lockstep: fewer positions than that are so many steps, on the bits of the steps behind them
 
 def precompute_freqs_cis(dim: int, end: int, theta: float) -> np.ndarray:
   """tinygrad/llm/model.py:16-19 in float32: cat(cos(pos * f), sin(pos * f)), f = 1 / theta^(2i/dim)."""
@@ -901,7 +902,7 @@ class BatchedTransformer:
     pr = np.zeros((B, c.max_context), np.int32); pr[:, :n] = np.array(prompts, np.int32)
     self.prompts.copyin(pr)
     # all but the last position of every prompt: as steps of many rows (sequences x positions) where the model is in their range and there are rows enough, else step by step
-    many = self._rows_tables is not None and on_block is None and B * (n - 1) >= MANY_ROWS_MIN and n > 2 and self.expert_path == "jobs"     # (a chosen expert path runs every step)
+    many = self._rows_tables is not None and on_block is None and B * (n - 1) >= MANY_ROWS_MIN and n - 1 >= MANY_ROWS_POSITIONS and self.expert_path == "jobs"     # (a chosen expert path runs every step)
     done = n - 1 if many else 0
     self.tokens.copyin(np.ascontiguousarray(pr[:, done]))
     st = np.zeros(16, np.int32); st[0], st[3], st[5] = done, n, c.vocab_size
