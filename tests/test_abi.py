@@ -54,3 +54,20 @@ def test_freed_blocks_are_kept_and_given_back(gpu):
   gpu.check(gpu.lib().tga_trim())
   b = gpu.Buffer((n,), np.uint8); gpu.check(gpu.lib().tga_copy_kernel(b.ptr, src[3].ptr, n, None)); gpu.synchronize()
   assert (b.numpy() == 3).all()
+
+@pytest.mark.gpu
+def test_a_capture_gets_no_block(gpu):
+  """A block that tga_free keeps is never handed to a thread whose own capture is open: the recorded launches would use it after the call that took it gave it back."""
+  import numpy as np
+  n = 5 << 20
+  stream, src, dst = gpu.Stream(), gpu.Buffer((4096,), np.uint8).zero_(), gpu.Buffer((4096,), np.uint8)
+  bufs = [gpu.Buffer((n,), np.uint8) for _ in range(9)]
+  kept = {b.ptr for b in bufs}
+  bufs.clear()
+  gpu.Buffer((n,), np.uint8)                                                       # (settles the class: its blocks may be handed out from here on)
+  with pytest.raises(RuntimeError, match="captures"):
+    with gpu.Graph(stream):
+      gpu.check(gpu.lib().tga_copy_kernel(dst.ptr, src.ptr, 4096, stream.handle))
+      gpu.Buffer((n,), np.uint8)
+  gpu.check(gpu.lib().tga_copy_kernel(dst.ptr, src.ptr, 4096, stream.handle)); stream.synchronize()
+  assert gpu.Buffer((n,), np.uint8).ptr in kept                                    # the capture is over: kept blocks are handed out again

@@ -24,6 +24,7 @@ int tga_set_error(const char* fmt, ...) {
 //  * at most POOL_BYTES per device are kept; beyond, blocks go back to the driver, all of them do before a request is refused for want of memory, and on tga_trim().
 //  * size classes are eighths of a power of two (at most 12.5 % of a block is idle).  One mutex; nothing here runs while a stream is being captured except taking a clean
 //    block or putting one aside (a synchronisation or a hipFree would invalidate the capture).
+//  * a thread with a capture of its own open gets no block: the replays would go on using one that its call gave back when it returned (and hipMalloc itself refuses then).
 #define POOL_BLOCK_MAX ((size_t)1 << 30)
 #define POOL_BYTES ((size_t)4 << 30)
 #define POOL_DIRTY_BYTES ((size_t)1 << 30)
@@ -57,7 +58,9 @@ static int pool_release(Pool& p) {                                              
 }
 static int pool_trim() { for (auto& p : g_pools) if (const int rc = pool_release(p.second)) return rc; return 0; }
 
+static thread_local int t_captures = 0;                                              // those of this thread (captures are thread-local: they end where they began)
 static int pool_malloc(void** ptr, size_t n) {
+  TGA_REQUIRE(!t_captures, "tga_malloc: not while this thread captures a stream");
   if (n > POOL_BLOCK_MAX) {
     hipError_t e = hipMalloc(ptr, n);
     if (e != hipErrorOutOfMemory) { TGA_HIP(e); return 0; }
@@ -85,7 +88,7 @@ static int pool_malloc(void** ptr, size_t n) {
   g_pool_blocks[*ptr] = {cls, dev};
   return 0;
 }
-static void capture_closed() { std::lock_guard<std::mutex> lock(g_pool_mutex); if (g_captures > 0) g_captures--; }
+static void capture_closed() { if (t_captures > 0) t_captures--; std::lock_guard<std::mutex> lock(g_pool_mutex); if (g_captures > 0) g_captures--; }
 static int pool_free(void* ptr) {
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   auto it = g_pool_blocks.find(ptr);
@@ -243,7 +246,7 @@ int tga_graph_begin(void* stream) {
   TGA_REQUIRE(stream, "tga_graph_begin: capture needs a non-null stream");
   TGA_HIP(hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeThreadLocal));
   std::lock_guard<std::mutex> lock(g_pool_mutex);
-  g_captures++;
+  g_captures++; t_captures++;
   return 0;
 }
 int tga_graph_end(void* stream, void** graph_exec) {
