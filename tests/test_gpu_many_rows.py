@@ -146,3 +146,14 @@ def test_batched_prefill_of_many_rows_vs_step_by_step(gpu, monkeypatch, cfg, B, 
   la, lb = a.logits(), b.logits()
   bad = np.abs(la - lb).max(axis=1) / np.abs(lb).max()
   assert (bad > 2e-3).sum() <= ((B + 3) // 4 if "num_experts" in cfg else 0), bad
+
+@pytest.mark.parametrize("n", [18, 65, 130])
+def test_rows_beyond_the_prompt_do_not_count(gpu, n):
+  """What an earlier prompt left in the cache beyond this one's positions is never multiplied, finite or not: the caches have the bits of a fresh model's."""
+  prompt = np.random.default_rng(n).integers(0, DENSE["vocab_size"], size=n).tolist()
+  a, b = _model(DENSE, 11), _model(DENSE, 11)
+  for blk in a.blk:
+    for cache in (blk.cache_k, blk.cache_v): cache.copyin(np.full(cache.shape, np.nan, np.float16))
+  for m in (a, b): m.prefill(prompt)
+  for ba, bb in zip(a.blk, b.blk):
+    for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): np.testing.assert_array_equal(ca.numpy()[:, :n - 1], cb.numpy()[:, :n - 1])

@@ -128,13 +128,13 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
   auto fetch = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < IK; i++) {
-      const int it = tid + 256 * i, key = min(64 * t + it / PC, a.max_ctx - 1);               // (rows beyond the cache are masked: they lie beyond every position)
+      const int it = tid + 256 * i, key = min(64 * t + it / PC, last_wg);                     // (rows that no position here sees are masked, but 0 times what an earlier prompt left there would be NaN if that is not finite)
       kq[i] = *(const u32x4*)(ck + (size_t)key * HD + (it % PC) * 8);
     }
 #pragma unroll
     for (int i = 0; i < IV; i++)
 #pragma unroll
-      for (int h = 0; h < 2; h++) { const int key = min(64 * t + 2 * (vpair + i * (256 / PC)) + h, a.max_ctx - 1); vq[i][h] = *(const u32x4*)(cv + (size_t)key * HD + vchunk * 8); }
+      for (int h = 0; h < 2; h++) { const int key = min(64 * t + 2 * (vpair + i * (256 / PC)) + h, last_wg); vq[i][h] = *(const u32x4*)(cv + (size_t)key * HD + vchunk * 8); }
   };
   auto put = [&]() __attribute__((always_inline)) {
 #pragma unroll
