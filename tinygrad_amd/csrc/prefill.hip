@@ -2,8 +2,8 @@
 // tinygrad/llm/model.py:464, 476-481, with the prompt as one chunk), every linear as ONE pass over its weights (qgemm_rows.h).  Per block: q / k / v -> rotation +
 // append -> attention -> attn_output (+ residual, norm) -> gate / up + SwiGLU -> down (+ residual, the next block's norm): eight launches and the sums of a split q / k / v, or for a MoE block norm -> router logits -> gating ->
 // grouping -> selected experts' gate / up + SwiGLU -> down -> weighted sum (+ residual), model.py:110-135.  The launches are issued by one native call.
-// MI355X, prompt to first logits: 8B-arch Q4_0 of 1024 tokens 42.4 ms (steps of 128 rows, qgemm64.hip) -> 21.4; OLMoE-arch of 512 tokens 64.0 (steps of 16 rows, an expert GEMV per
-// token and slot) -> 5.5; four 8B-arch Q4_K_M sequences of 128 tokens 333 (one lockstep step per position) -> 15.6.
+// MI355X, prompt to first logits: 8B-arch Q4_0 of 1024 tokens 42.4 ms (steps of 128 rows, qgemm64.hip) -> 21.2; OLMoE-arch of 512 tokens 64.0 (steps of 16 rows, an expert GEMV per
+// token and slot) -> 5.0; four 8B-arch Q4_K_M sequences of 128 tokens 333 (one lockstep step per position) -> 15.5.
 #include "qgemm_rows.h"
 #include "decode.h"
 #include "moe_gate.h"
