@@ -132,9 +132,9 @@ def test_batched_prefill_of_many_rows_vs_step_by_step(gpu, monkeypatch, cfg, B, 
   prompts = np.random.default_rng(B + n).integers(0, cfg["vocab_size"], size=(B, n)).tolist()
   a, b = _model(cfg, 9, 128, B), _model(cfg, 9, 128, B)
   monkeypatch.setattr(llm, "MANY_ROWS", rows)
+  a.many_rows, b.many_rows = True, False
   a.prefill(prompts)
   assert a._rows_ws is not None
-  monkeypatch.setattr(llm, "MANY_ROWS_MIN", 1 << 30)
   b.prefill(prompts)
   assert b._rows_ws is None
   for ba, bb in zip(a.blk, b.blk):
@@ -157,3 +157,17 @@ def test_rows_beyond_the_prompt_do_not_count(gpu, n):
   for m in (a, b): m.prefill(prompt)
   for ba, bb in zip(a.blk, b.blk):
     for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): np.testing.assert_array_equal(ca.numpy()[:, :n - 1], cb.numpy()[:, :n - 1])
+
+def test_moe_prompts_keep_their_steps_unless_asked(gpu):
+  """A MoE model's prefill computes the bits of steps of sixteen rows (and of lockstep steps): another order of sums turns expert choices at near-ties, so steps of many rows are the user's
+  choice there (many_rows), not the default."""
+  prompt = np.random.default_rng(3).integers(0, MOE["vocab_size"], size=90).tolist()
+  a, b, rows = _model(MOE, 13), _model(MOE, 13), _model(MOE, 13)
+  b.prefill_chunk, rows.many_rows = 16, True
+  for m in (a, b, rows): m.prefill(prompt)
+  for ba, bb in zip(a.blk, b.blk):
+    for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): np.testing.assert_array_equal(ca.numpy(), cb.numpy())
+  assert a._chunker.batch == 16 and a._chunker._rows_ws is None and rows._tail_chunkers[16]._rows_ws is not None
+  batch = _model(MOE, 13, 128, 4)
+  batch.prefill([prompt] * 4)
+  assert batch._rows_ws is None

@@ -378,6 +378,10 @@ class Transformer:
     self._cached_tokens, self._last_input, self.prefill_steps = [], None, 0   # tokens whose K / V rows the cache holds (KV-prefix reuse, model.py:455-462)
     self.replay = "cmdlist"                                          # how a captured step is replayed: "cmdlist" (plain launches in capture order) or "graph" (hipGraphLaunch)
     self._state_dict, self._chunker, self._tail_chunkers = state_dict, None, {}   # (references to the weight buffers: the chunked prefill builds its linears over the same bytes)
+    # Prompts of MANY_ROWS_MIN positions and more as steps of many rows (prefill, below).  Not for MoE models unless asked for: their sums then run in another order than in steps of sixteen
+    # rows, which is no less exact, but turns expert choices at near-ties - of the last token in four of fifty OLMoE-architecture prompts of 512 tokens, whose logits move by 2e-2 .. 5e-2 (1e-3
+    # in the others, as between steps of sixteen rows and of one).  Those 512 tokens take 64 ms in steps of sixteen rows, 5.0 ms in one of many
+    self.many_rows = not config.num_experts
     self.prefill_chunk = 128                                         # prompt positions per prefill step, 2..128 (128: as many as the prompt has where the model allows, see prefill) (the reference's chunks hold 32, model.py:464; MoE models: at most 16); 1: token by token
 
   def check_state(self):
@@ -520,7 +524,7 @@ class Transformer:
     B = self.prefill_chunk if on_block is None else 1
     # From MANY_ROWS_MIN positions on, and with the chunk size left at its largest, the positions are steps of many rows: one pass over the weights for (nearly) any prompt
     n_rows = len(tokens) - 1 - start
-    if B == 128 and n_rows >= MANY_ROWS_MIN:
+    if self.many_rows and B == 128 and n_rows >= MANY_ROWS_MIN:
       if n_rows >= B and self._chunker is None: self._chunker = BatchedTransformer(self.config, self._state_dict, B, max_new=1, chunk_of=self)
       if self._chunker is None and 16 not in self._tail_chunkers: self._tail_chunkers[16] = BatchedTransformer(self.config, self._state_dict, 16, max_new=1, chunk_of=self)
       chunker = self._chunker or self._tail_chunkers[16]
@@ -658,6 +662,7 @@ class BatchedTransformer:
       if ok and c.dim % 256 == 0 and c.hidden_dim % 256 == 0 and nq % 256 == 0:
         self.rows64 = 2 if B <= 32 else 4 if B <= 64 else 8             # column groups of sixteen rows in the layout
     self._rows_tables, self._rows_ws, self._rows_tok = self._many_rows_tables(), None, None
+    self.many_rows = not c.num_experts                                  # lockstep prompts as steps of many rows (see Transformer.many_rows)
     self.x = None
     if not self.chunked: self._alloc_step()
 
@@ -902,7 +907,7 @@ class BatchedTransformer:
     pr = np.zeros((B, c.max_context), np.int32); pr[:, :n] = np.array(prompts, np.int32)
     self.prompts.copyin(pr)
     # all but the last position of every prompt: as steps of many rows (sequences x positions) where the model is in their range and there are rows enough, else step by step
-    many = self._rows_tables is not None and on_block is None and B * (n - 1) >= MANY_ROWS_MIN and n - 1 >= MANY_ROWS_POSITIONS and self.expert_path == "jobs"     # (a chosen expert path runs every step)
+    many = self.many_rows and self._rows_tables is not None and on_block is None and B * (n - 1) >= MANY_ROWS_MIN and n - 1 >= MANY_ROWS_POSITIONS and self.expert_path == "jobs"     # (a chosen expert path runs every step)
     done = n - 1 if many else 0
     self.tokens.copyin(np.ascontiguousarray(pr[:, done]))
     st = np.zeros(16, np.int32); st[0], st[3], st[5] = done, n, c.vocab_size
