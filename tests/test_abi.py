@@ -37,6 +37,35 @@ def test_host_side_argument_checks_without_gpu():
   b = moe.to_bf16_bits(np.array([1.0, 1.00390625, -2.5, 1.01171875], np.float32))     # 1 + 2^-8 ties to even (1.0); 1 + 3*2^-8 rounds up
   np.testing.assert_array_equal(moe.from_bf16_bits(b), np.array([1.0, 1.0, -2.5, 1.015625], np.float32))
 
+def test_moe_feed_forward_refuses_operands_of_other_sizes(monkeypatch):
+  """Every operand of the fused feed-forward is looked at before the native call, which reads what the sizes ask for: logits of another width or fewer rows, weights of another K or
+  number of experts, and scales, biases or activations that are too small are AssertionErrors; a down projection to another width takes the single steps, which return that width."""
+  import numpy as np
+  from tinygrad_amd import moe, runtime as rt
+  class Lib:
+    def tga_moe_feed_forward_plan(self, T, D, I, E, k, need): need._obj.value = 256; return 0
+    def tga_malloc(self, p, n): p._obj.value = 1 << 20; return 0
+    def tga_moe_feed_forward(self, *a): calls.append("fused"); return 0
+    def tga_moe_route(self, *a): calls.append("single"); return 1
+  calls, lib = [], Lib()
+  monkeypatch.setattr(rt, "lib", lambda: lib)
+  monkeypatch.setattr(rt.Buffer, "__del__", lambda self: None)
+  T, D, I, E, k = 40, 512, 256, 8, 2
+  def buf(shape, dtype): return rt.Buffer(shape, dtype, ptr=4096)
+  good = dict(inp=((T, D), np.uint16), logits=((T, E), np.float32), gq=((E, 2 * I, D), np.uint8), ge=((E, 2 * I, D // 32), np.uint8), gb=((E, 2 * I), np.float32),
+              dq=((E, D, I), np.uint8), de=((E, D, I // 32), np.uint8), db=((E, D), np.float32))
+  def call(**other):
+    b = {n: buf(*v) for n, v in {**good, **other}.items()}
+    return moe.moe_feed_forward(b["inp"], b["logits"], k, (b["gq"], b["ge"]), b["gb"], (b["dq"], b["de"]), b["db"])
+  assert call().shape == (T, D) and calls == ["fused"]
+  for other in (dict(logits=((T, E // 2), np.float32)), dict(logits=((T - 1, E), np.float32)), dict(logits=((T, E), np.float16)), dict(inp=((T, D), np.uint8)),
+                dict(gq=((E, 2 * I, D // 2), np.uint8)), dict(dq=((E, D, I // 2), np.uint8)), dict(dq=((E // 2, D, I), np.uint8)), dict(dq=((E, D, 2 * I), np.uint8)),
+                dict(ge=((E, 2 * I, D // 64), np.uint8)), dict(de=((E // 2, D, I // 32), np.uint8)), dict(gb=((E, I), np.float32)), dict(db=((E // 2, D), np.float32))):
+    with pytest.raises(AssertionError): call(**other)
+  assert calls == ["fused"]
+  with pytest.raises(RuntimeError): call(dq=((E, 256, I), np.uint8))               # (the library above refuses the single steps' first call)
+  assert calls == ["fused", "single"]
+
 @pytest.mark.gpu
 def test_freed_blocks_are_kept_and_given_back(gpu):
   """tga_free keeps a block for later requests of its size class, never hands it out while kernels may still use it, and tga_trim gives everything back: results computed into

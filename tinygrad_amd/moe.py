@@ -144,12 +144,18 @@ def moe_feed_forward(inp: Buffer, logits: Buffer, experts_per_tok: int, w_gate_u
   b_down (E, D) float32 -> (T, D) bf16 bits.  D, 2I and I must be multiples of 256 (the reference pads to that, gpt_oss.py:85-92; the
   padding is not built here).  routed_only: the two GEMMs skip the tiles beyond the routed rows, which combine never reads."""
   T, D = inp.shape
-  E, N2, _ = w_gate_up[0].shape
+  E, N2, K = w_gate_up[0].shape
   assert D % 256 == 0 and N2 % 256 == 0 and (N2 // 2) % 256 == 0, f"dim {D}, 2*inter {N2} and inter {N2 // 2} must be multiples of 256"
+  E2, N, I = w_down[0].shape
+  assert logits.shape == (T, E), f"logits {logits.shape} for {T} tokens and {E} experts"
+  assert (K, E2, I) == (D, E, N2 // 2), f"shape mismatch {(T, D)} {w_gate_up[0].shape} {w_down[0].shape}"
+  for name, b, nb in (("inp", inp, T * D * 2), ("logits", logits, T * E * 4), ("w_gate_up", w_gate_up[0], E * N2 * D), ("w_gate_up scales", w_gate_up[1], E * N2 * D // 32),
+                      ("b_gate_up", b_gate_up, E * N2 * 4), ("w_down", w_down[0], E * N * I), ("w_down scales", w_down[1], E * N * I // 32), ("b_down", b_down, E * N * 4)):
+    assert b.nbytes >= nb, f"{name}: {b.nbytes} bytes where the sizes ask for {nb}"
   need = ctypes.c_int64(0)
   rt.check(rt.lib().tga_moe_feed_forward_plan(T, D, N2 // 2, E, experts_per_tok, ctypes.byref(need)))
   ptrs = [b.ptr for b in (inp, *w_gate_up, b_gate_up, *w_down, b_down)]
-  if need.value and all(p % 16 == 0 for p in ptrs):             # one native call: five launches over compact rows, no padding rows (whatever routed_only says: combine reads none)
+  if need.value and N == D and all(p % 16 == 0 for p in ptrs):  # one native call: five launches over compact rows, no padding rows (whatever routed_only says: combine reads none)
     ws, out = Buffer((need.value,), np.uint8), Buffer((T, D), np.uint16)
     rt.check(rt.lib().tga_moe_feed_forward(inp.ptr, logits.ptr, T, D, N2 // 2, E, experts_per_tok, w_gate_up[0].ptr, w_gate_up[1].ptr, b_gate_up.ptr, w_down[0].ptr, w_down[1].ptr,
                                            b_down.ptr, swiglu_limit, ws.ptr, out.ptr, stream))
