@@ -1,0 +1,71 @@
+// The rules of csrc/pool.h against a runtime of this file's own: a device that is busy until something waits for it, calls that a capture refuses, a limit on memory, frees that fail.
+#include <stdarg.h>
+#include <stdint.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+#include <map>
+#include <set>
+#include <string>
+#include <unordered_map>
+#include <vector>
+
+typedef int hipError_t;
+enum { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorStreamCaptureUnsupported = 900 };
+static std::string g_msg;
+static int tga_set_error(const char* fmt, ...) { char b[256]; va_list ap; va_start(ap, fmt); vsnprintf(b, sizeof(b), fmt, ap); va_end(ap); g_msg = b; return 1; }
+#define TGA_HIP(expr) do { hipError_t _e = (expr); if (_e != hipSuccess) return tga_set_error("HIP Error %d [%s]", (int)_e, #expr); } while (0)
+#define TGA_REQUIRE(cond, ...) do { if (!(cond)) return tga_set_error(__VA_ARGS__); } while (0)
+
+static std::set<void*> g_live; static uintptr_t g_next = 1 << 20; static size_t g_limit = ~(size_t)0, g_used = 0;
+static std::unordered_map<void*, size_t> g_size;
+static int g_waits = 0, g_mallocs = 0, g_fail_free_after = -1;
+static bool g_capturing = false, g_capture_broken = false;                // a capture of the calling thread that something else opened
+static hipError_t refused() { if (g_capturing) { g_capture_broken = true; return hipErrorStreamCaptureUnsupported; } return hipSuccess; }
+static hipError_t hipMalloc(void** p, size_t n) {
+  if (hipError_t e = refused()) return e;
+  if (g_used + n > g_limit) return hipErrorOutOfMemory;
+  *p = (void*)g_next; g_next += n + 4096; g_live.insert(*p); g_size[*p] = n; g_used += n; g_mallocs++;
+  return hipSuccess;
+}
+static hipError_t hipFree(void* p) {
+  if (hipError_t e = refused()) return e;
+  if (!p) return hipSuccess;
+  if (!g_live.count(p)) return hipErrorInvalidValue;
+  if (g_fail_free_after == 0) return hipErrorInvalidValue;
+  if (g_fail_free_after > 0) g_fail_free_after--;
+  g_live.erase(p); g_used -= g_size[p]; g_waits++;                          // (waits for the device)
+  return hipSuccess;
+}
+[[maybe_unused]] static hipError_t hipDeviceSynchronize() { if (hipError_t e = refused()) return e; g_waits++; return hipSuccess; }
+static hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+[[maybe_unused]] static hipError_t hipGetLastError() { return hipSuccess; }
+
+#include "../../tinygrad_amd/csrc/pool.h"
+
+#define CHECK(c) do { if (!(c)) { printf("%s:%d: %s (last error: %s)\n", __FILE__, __LINE__, #c, g_msg.c_str()); exit(1); } } while (0)
+
+static void freed_twice() {
+  void* a; CHECK(!pool_malloc(&a, 1 << 20));
+  CHECK(!pool_free(a)); CHECK(pool_free(a) != 0);
+  std::set<void*> got;
+  for (int i = 0; i < 40; i++) {                                           // every block handed out once, however often the class is settled
+    void* b[4]; for (auto& q : b) { CHECK(!pool_malloc(&q, 1 << 20)); CHECK(got.insert(q).second); }
+    for (auto& q : b) { CHECK(!pool_free(q)); CHECK(pool_free(q) != 0); got.erase(q); }
+  }
+}
+static void waits_before_handing_out() {
+  for (int i = 0; i < 30; i++) {
+    void* a; CHECK(!pool_malloc(&a, 3 << 20)); const int w = g_waits; CHECK(!pool_free(a));
+    std::vector<void*> got;
+    for (int j = 0; j < 12; j++) { void* b; CHECK(!pool_malloc(&b, 3 << 20)); if (b == a) CHECK(g_waits > w); got.push_back(b); }
+    for (void* b : got) CHECK(!pool_free(b));
+  }
+}
+
+int main(int argc, char** argv) {
+  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}};
+  CHECK(argc == 2 && tests.count(argv[1]));
+  tests.at(argv[1])();
+  puts("ok");
+}

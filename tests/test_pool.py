@@ -1,0 +1,17 @@
+"""The rules of the allocation pool (csrc/pool.h) on the host: tests/c/pool_test.cpp compiles it against a runtime of its own and runs one case per process."""
+import pathlib, subprocess
+import pytest
+
+ROOT = pathlib.Path(__file__).resolve().parent
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+  exe = tmp_path_factory.mktemp("pool") / "pool_test"
+  r = subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-pthread", str(ROOT / "c" / "pool_test.cpp"), "-o", str(exe)], capture_output=True, text=True)
+  assert r.returncode == 0, r.stderr
+  return exe
+
+@pytest.mark.parametrize("case", ["freed_twice", "waits_before_handing_out"])
+def test_pool(program, case):
+  r = subprocess.run([str(program), case], capture_output=True, text=True, timeout=60)
+  assert r.returncode == 0, r.stdout + r.stderr

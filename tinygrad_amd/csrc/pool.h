@@ -1,0 +1,94 @@
+// Device allocations behind tga_malloc / tga_free (included by runtime.hip, and on the host by the test of its rules, which brings functions of its own under the names of the runtime's).
+#pragma once
+#include <map>
+#include <mutex>
+#include <unordered_map>
+#include <vector>
+
+// ---- Device allocations.  hipFree waits for the device and unmaps, hipMalloc maps again: an entry point that allocates its result (ggml_data_to_tensor, quantize_mxfp8,
+// moe_feed_forward) spent 1.6 ms (three results of 70 MB in all) to 3.3 ms (one of 117 MB) per call on them where its kernels take 40 .. 60 us, back to back; with
+// freed blocks kept, 0.07 ms for the latter.  So a freed block of at most POOL_BLOCK_MAX bytes is kept for the next request of its size class:
+//  * freed blocks are first `dirty`: kernels on any stream may still be using them, exactly as before a hipFree.  They become `clean`, i.e. may be handed out again,
+//    after a hipDeviceSynchronize, which is what hipFree itself did - but one for many blocks: when a request finds no clean block of its class while POOL_DIRTY_COUNT
+//    blocks of the class or POOL_DIRTY_BYTES in all are dirty.  No stream has to be named, no caller synchronises more than it did.
+//  * at most POOL_BYTES per device are kept; beyond, blocks go back to the driver, all of them do before a request is refused for want of memory, and on tga_trim().
+//  * size classes are eighths of a power of two (at most 12.5 % of a block is idle).  One mutex; nothing here runs while a stream is being captured except taking a clean
+//    block or putting one aside (a synchronisation or a hipFree would invalidate the capture).
+//  * a thread with a capture of its own open gets no block: the replays would go on using one that its call gave back when it returned (and hipMalloc itself refuses then).
+#define POOL_BLOCK_MAX ((size_t)1 << 30)
+#define POOL_BYTES ((size_t)4 << 30)
+#define POOL_DIRTY_BYTES ((size_t)1 << 30)
+#define POOL_DIRTY_COUNT 8
+
+struct PoolClass { std::vector<void*> clean, dirty; };
+struct Pool { std::map<size_t, PoolClass> classes; size_t kept = 0, dirty = 0; };
+static std::mutex g_pool_mutex;
+static std::unordered_map<int, Pool> g_pools;                                        // by device
+struct PoolBlock { size_t cls; int dev; bool out; };                                  // size class, device, handed out (or kept)
+static std::unordered_map<void*, PoolBlock> g_pool_blocks;                           // every block that belongs to a size class
+static int g_captures = 0;                                                           // captures open (tga_graph_begin .. tga_graph_end / tga_cmdlist_end)
+
+static size_t pool_class(size_t n) {
+  if (n <= 4096) return (n + 511) & ~(size_t)511;
+  int b = 0; for (size_t t = n - 1; t >>= 1;) b++;                                   // 2^b < n <= 2^(b + 1)
+  const size_t step = (size_t)1 << (b - 2);
+  return (n + step - 1) & ~(step - 1);
+}
+static int pool_settle(Pool& p) {                                                     // every dirty block becomes clean
+  TGA_HIP(hipDeviceSynchronize());
+  for (auto& c : p.classes) { c.second.clean.insert(c.second.clean.end(), c.second.dirty.begin(), c.second.dirty.end()); c.second.dirty.clear(); }
+  p.dirty = 0;
+  return 0;
+}
+static int pool_release(Pool& p) {                                                    // everything kept goes back to the driver (hipFree waits for the block's users)
+  for (auto& c : p.classes) {
+    for (auto* v : {&c.second.clean, &c.second.dirty}) { for (void* q : *v) { g_pool_blocks.erase(q); TGA_HIP(hipFree(q)); } v->clear(); }
+  }
+  p.classes.clear(); p.kept = p.dirty = 0;
+  return 0;
+}
+static int pool_trim() { for (auto& p : g_pools) if (const int rc = pool_release(p.second)) return rc; return 0; }
+
+static thread_local int t_captures = 0;                                              // those of this thread (captures are thread-local: they end where they began)
+static int pool_malloc(void** ptr, size_t n) {
+  TGA_REQUIRE(!t_captures, "tga_malloc: not while this thread captures a stream");
+  if (n > POOL_BLOCK_MAX) {
+    hipError_t e = hipMalloc(ptr, n);
+    if (e != hipErrorOutOfMemory) { TGA_HIP(e); return 0; }
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> lock(g_pool_mutex);
+    if (const int rc = g_captures ? 0 : pool_trim()) return rc;
+    TGA_HIP(hipMalloc(ptr, n));
+    return 0;
+  }
+  int dev = 0;
+  TGA_HIP(hipGetDevice(&dev));
+  const size_t cls = pool_class(n);
+  std::lock_guard<std::mutex> lock(g_pool_mutex);
+  Pool& p = g_pools[dev];
+  PoolClass& c = p.classes[cls];
+  if (c.clean.empty() && !c.dirty.empty() && !g_captures && (c.dirty.size() >= POOL_DIRTY_COUNT || p.dirty >= POOL_DIRTY_BYTES)) { if (const int rc = pool_settle(p)) return rc; }
+  if (!c.clean.empty()) { *ptr = c.clean.back(); c.clean.pop_back(); p.kept -= cls; g_pool_blocks[*ptr].out = true; return 0; }
+  hipError_t e = hipMalloc(ptr, cls);
+  if (e == hipErrorOutOfMemory && !g_captures) {
+    (void)hipGetLastError();
+    if (const int rc = pool_trim()) return rc;
+    e = hipMalloc(ptr, cls);
+  }
+  TGA_HIP(e);
+  g_pool_blocks[*ptr] = {cls, dev, true};
+  return 0;
+}
+static void capture_closed() { if (t_captures > 0) t_captures--; std::lock_guard<std::mutex> lock(g_pool_mutex); if (g_captures > 0) g_captures--; }
+static int pool_free(void* ptr) {
+  std::lock_guard<std::mutex> lock(g_pool_mutex);
+  auto it = g_pool_blocks.find(ptr);
+  if (it == g_pool_blocks.end()) { TGA_HIP(hipFree(ptr)); return 0; }
+  TGA_REQUIRE(it->second.out, "tga_free: the block has been freed before");               // (as hipFree refuses it: kept twice, it would be handed out twice)
+  const size_t cls = it->second.cls;
+  Pool& p = g_pools[it->second.dev];
+  if (p.kept + cls > POOL_BYTES && !g_captures) { g_pool_blocks.erase(it); TGA_HIP(hipFree(ptr)); return 0; }
+  p.classes[cls].dirty.push_back(ptr);
+  p.kept += cls; p.dirty += cls; it->second.out = false;
+  return 0;
+}
