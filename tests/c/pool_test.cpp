@@ -63,8 +63,21 @@ static void waits_before_handing_out() {
   }
 }
 
+static void keep(size_t n, int count) {                                    // so many kept blocks of a class, free to be handed out
+  std::vector<void*> b(count + 8); for (auto& q : b) CHECK(!pool_malloc(&q, n)); for (auto& q : b) CHECK(!pool_free(q));
+  void* q; CHECK(!pool_malloc(&q, n)); CHECK(!pool_free(q));
+}
+static void capture_opened_elsewhere() {
+  keep(5 << 20, 8);
+  g_capturing = true;
+  void* a = nullptr; CHECK(pool_malloc(&a, 5 << 20) != 0 && !a); CHECK(g_msg.find("900") != std::string::npos);
+  CHECK(pool_malloc(&a, (size_t)2 << 30) != 0 && !a);
+  g_capturing = false;
+  CHECK(!pool_malloc(&a, 5 << 20)); CHECK(!pool_free(a));
+}
+
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}};
+  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}};
   CHECK(argc == 2 && tests.count(argv[1]));
   tests.at(argv[1])();
   puts("ok");

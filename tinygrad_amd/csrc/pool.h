@@ -14,7 +14,8 @@
 //  * at most POOL_BYTES per device are kept; beyond, blocks go back to the driver, all of them do before a request is refused for want of memory, and on tga_trim().
 //  * size classes are eighths of a power of two (at most 12.5 % of a block is idle).  One mutex; nothing here runs while a stream is being captured except taking a clean
 //    block or putting one aside (a synchronisation or a hipFree would invalidate the capture).
-//  * a thread with a capture of its own open gets no block: the replays would go on using one that its call gave back when it returned (and hipMalloc itself refuses then).
+//  * a thread with a capture of its own open gets no block: the replays would go on using one that its call gave back when it returned (and hipMalloc itself refuses then).  Captures that
+//    the library did not open are the runtime's to know: an hipFree of nothing is refused during exactly those that hipMalloc is refused during (measured for the three capture modes).
 #define POOL_BLOCK_MAX ((size_t)1 << 30)
 #define POOL_BYTES ((size_t)4 << 30)
 #define POOL_DIRTY_BYTES ((size_t)1 << 30)
@@ -52,6 +53,7 @@ static int pool_trim() { for (auto& p : g_pools) if (const int rc = pool_release
 static thread_local int t_captures = 0;                                              // those of this thread (captures are thread-local: they end where they began)
 static int pool_malloc(void** ptr, size_t n) {
   TGA_REQUIRE(!t_captures, "tga_malloc: not while this thread captures a stream");
+  TGA_HIP(hipFree(nullptr));                                                          // (0.2 us) a capture that something else opened: refused (error 900) where hipMalloc is, else nothing
   if (n > POOL_BLOCK_MAX) {
     hipError_t e = hipMalloc(ptr, n);
     if (e != hipErrorOutOfMemory) { TGA_HIP(e); return 0; }
