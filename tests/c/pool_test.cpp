@@ -21,6 +21,7 @@ static std::set<void*> g_live; static uintptr_t g_next = 1 << 20; static size_t 
 static std::unordered_map<void*, size_t> g_size;
 static int g_waits = 0, g_mallocs = 0, g_fail_free_after = -1;
 static bool g_capturing = false, g_capture_broken = false;                // a capture of the calling thread that something else opened
+static bool g_other_capture = false;                                       // ... and one of another thread: only a device synchronisation is refused then
 static hipError_t refused() { if (g_capturing) { g_capture_broken = true; return hipErrorStreamCaptureUnsupported; } return hipSuccess; }
 static hipError_t hipMalloc(void** p, size_t n) {
   if (hipError_t e = refused()) return e;
@@ -37,7 +38,7 @@ static hipError_t hipFree(void* p) {
   g_live.erase(p); g_used -= g_size[p]; g_waits++;                          // (waits for the device)
   return hipSuccess;
 }
-[[maybe_unused]] static hipError_t hipDeviceSynchronize() { if (hipError_t e = refused()) return e; g_waits++; return hipSuccess; }
+[[maybe_unused]] static hipError_t hipDeviceSynchronize() { if (hipError_t e = refused()) return e; if (g_other_capture) { g_capture_broken = true; return hipErrorStreamCaptureUnsupported; } g_waits++; return hipSuccess; }
 static hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 [[maybe_unused]] static hipError_t hipGetLastError() { return hipSuccess; }
 
@@ -75,9 +76,18 @@ static void capture_opened_elsewhere() {
   g_capturing = false;
   CHECK(!pool_malloc(&a, 5 << 20)); CHECK(!pool_free(a));
 }
+static void capture_of_another_thread() {
+  g_other_capture = true;
+  std::set<void*> seen; int again = 0;
+  for (int i = 0; i < 40; i++) {
+    void* b[4]; for (auto& q : b) { CHECK(!pool_malloc(&q, 6 << 20)); again += !seen.insert(q).second; }
+    for (auto& q : b) CHECK(!pool_free(q));
+  }
+  CHECK(again && !g_capture_broken);
+}
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}};
+  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}};
   CHECK(argc == 2 && tests.count(argv[1]));
   tests.at(argv[1])();
   puts("ok");

@@ -9,11 +9,12 @@
 // moe_feed_forward) spent 1.6 ms (three results of 70 MB in all) to 3.3 ms (one of 117 MB) per call on them where its kernels take 40 .. 60 us, back to back; with
 // freed blocks kept, 0.07 ms for the latter.  So a freed block of at most POOL_BLOCK_MAX bytes is kept for the next request of its size class:
 //  * freed blocks are first `dirty`: kernels on any stream may still be using them, exactly as before a hipFree.  They become `clean`, i.e. may be handed out again,
-//    after a hipDeviceSynchronize, which is what hipFree itself did - but one for many blocks: when a request finds no clean block of its class while POOL_DIRTY_COUNT
-//    blocks of the class or POOL_DIRTY_BYTES in all are dirty.  No stream has to be named, no caller synchronises more than it did.
+//    after the wait for the device that an hipFree performs - but one for many blocks: when a request finds no clean block of its class while POOL_DIRTY_COUNT
+//    blocks of the class or POOL_DIRTY_BYTES in all are dirty.  No stream has to be named, no caller synchronises more than it did.  The wait is that of an hipFree of a few bytes allocated
+//    for it (1.4 us where the device is idle): an hipDeviceSynchronize is refused during a capture of any thread and ends that capture, an hipFree only during one of its own (measured).
 //  * at most POOL_BYTES per device are kept; beyond, blocks go back to the driver, all of them do before a request is refused for want of memory, and on tga_trim().
-//  * size classes are eighths of a power of two (at most 12.5 % of a block is idle).  One mutex; nothing here runs while a stream is being captured except taking a clean
-//    block or putting one aside (a synchronisation or a hipFree would invalidate the capture).
+//  * size classes are eighths of a power of two (at most 12.5 % of a block is idle).  One mutex.  While its thread captures a stream, tga_free puts a block aside without a call to the runtime (an hipFree would
+//    invalidate the capture).
 //  * a thread with a capture of its own open gets no block: the replays would go on using one that its call gave back when it returned (and hipMalloc itself refuses then).  Captures that
 //    the library did not open are the runtime's to know: an hipFree of nothing is refused during exactly those that hipMalloc is refused during (measured for the three capture modes).
 #define POOL_BLOCK_MAX ((size_t)1 << 30)
@@ -27,7 +28,6 @@ static std::mutex g_pool_mutex;
 static std::unordered_map<int, Pool> g_pools;                                        // by device
 struct PoolBlock { size_t cls; int dev; bool out; };                                  // size class, device, handed out (or kept)
 static std::unordered_map<void*, PoolBlock> g_pool_blocks;                           // every block that belongs to a size class
-static int g_captures = 0;                                                           // captures open (tga_graph_begin .. tga_graph_end / tga_cmdlist_end)
 
 static size_t pool_class(size_t n) {
   if (n <= 4096) return (n + 511) & ~(size_t)511;
@@ -35,8 +35,10 @@ static size_t pool_class(size_t n) {
   const size_t step = (size_t)1 << (b - 2);
   return (n + step - 1) & ~(step - 1);
 }
-static int pool_settle(Pool& p) {                                                     // every dirty block becomes clean
-  TGA_HIP(hipDeviceSynchronize());
+static int pool_settle(Pool& p) {                                                     // every dirty block becomes clean (not where there is no memory left: the caller trims then)
+  void* few = nullptr;
+  if (hipMalloc(&few, 512) != hipSuccess) { (void)hipGetLastError(); return 0; }
+  TGA_HIP(hipFree(few));
   for (auto& c : p.classes) { c.second.clean.insert(c.second.clean.end(), c.second.dirty.begin(), c.second.dirty.end()); c.second.dirty.clear(); }
   p.dirty = 0;
   return 0;
@@ -50,7 +52,7 @@ static int pool_release(Pool& p) {                                              
 }
 static int pool_trim() { for (auto& p : g_pools) if (const int rc = pool_release(p.second)) return rc; return 0; }
 
-static thread_local int t_captures = 0;                                              // those of this thread (captures are thread-local: they end where they began)
+static thread_local int t_captures = 0;                                              // captures of this thread (tga_graph_begin .. tga_graph_end / tga_cmdlist_end: they end where they began)
 static int pool_malloc(void** ptr, size_t n) {
   TGA_REQUIRE(!t_captures, "tga_malloc: not while this thread captures a stream");
   TGA_HIP(hipFree(nullptr));                                                          // (0.2 us) a capture that something else opened: refused (error 900) where hipMalloc is, else nothing
@@ -59,7 +61,7 @@ static int pool_malloc(void** ptr, size_t n) {
     if (e != hipErrorOutOfMemory) { TGA_HIP(e); return 0; }
     (void)hipGetLastError();
     std::lock_guard<std::mutex> lock(g_pool_mutex);
-    if (const int rc = g_captures ? 0 : pool_trim()) return rc;
+    if (const int rc = pool_trim()) return rc;
     TGA_HIP(hipMalloc(ptr, n));
     return 0;
   }
@@ -69,10 +71,10 @@ static int pool_malloc(void** ptr, size_t n) {
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   Pool& p = g_pools[dev];
   PoolClass& c = p.classes[cls];
-  if (c.clean.empty() && !c.dirty.empty() && !g_captures && (c.dirty.size() >= POOL_DIRTY_COUNT || p.dirty >= POOL_DIRTY_BYTES)) { if (const int rc = pool_settle(p)) return rc; }
+  if (c.clean.empty() && !c.dirty.empty() && (c.dirty.size() >= POOL_DIRTY_COUNT || p.dirty >= POOL_DIRTY_BYTES)) { if (const int rc = pool_settle(p)) return rc; }
   if (!c.clean.empty()) { *ptr = c.clean.back(); c.clean.pop_back(); p.kept -= cls; g_pool_blocks[*ptr].out = true; return 0; }
   hipError_t e = hipMalloc(ptr, cls);
-  if (e == hipErrorOutOfMemory && !g_captures) {
+  if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     if (const int rc = pool_trim()) return rc;
     e = hipMalloc(ptr, cls);
@@ -81,7 +83,6 @@ static int pool_malloc(void** ptr, size_t n) {
   g_pool_blocks[*ptr] = {cls, dev, true};
   return 0;
 }
-static void capture_closed() { if (t_captures > 0) t_captures--; std::lock_guard<std::mutex> lock(g_pool_mutex); if (g_captures > 0) g_captures--; }
 static int pool_free(void* ptr) {
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   auto it = g_pool_blocks.find(ptr);
@@ -89,7 +90,7 @@ static int pool_free(void* ptr) {
   TGA_REQUIRE(it->second.out, "tga_free: the block has been freed before");               // (as hipFree refuses it: kept twice, it would be handed out twice)
   const size_t cls = it->second.cls;
   Pool& p = g_pools[it->second.dev];
-  if (p.kept + cls > POOL_BYTES && !g_captures) { g_pool_blocks.erase(it); TGA_HIP(hipFree(ptr)); return 0; }
+  if (p.kept + cls > POOL_BYTES && !t_captures) { g_pool_blocks.erase(it); TGA_HIP(hipFree(ptr)); return 0; }
   p.classes[cls].dirty.push_back(ptr);
   p.kept += cls; p.dirty += cls; it->second.out = false;
   return 0;

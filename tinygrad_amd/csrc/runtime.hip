@@ -107,7 +107,7 @@ struct TgaCmdList { hipGraph_t graph; std::vector<hipKernelNodeParams> kernels; 
 int tga_cmdlist_end(void* stream, void** cmdlist) {
   TGA_REQUIRE(stream && cmdlist, "tga_cmdlist_end: null pointer");
   hipGraph_t g = nullptr;
-  capture_closed();
+  if (t_captures > 0) t_captures--;
   TGA_HIP(hipStreamEndCapture((hipStream_t)stream, &g));
   size_t n = 0;
   hipError_t e = hipGraphGetNodes(g, nullptr, &n);
@@ -157,13 +157,12 @@ int tga_cmdlist_destroy(void* cmdlist) {
 int tga_graph_begin(void* stream) {
   TGA_REQUIRE(stream, "tga_graph_begin: capture needs a non-null stream");
   TGA_HIP(hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeThreadLocal));
-  std::lock_guard<std::mutex> lock(g_pool_mutex);
-  g_captures++; t_captures++;
+  t_captures++;
   return 0;
 }
 int tga_graph_end(void* stream, void** graph_exec) {
   hipGraph_t g = nullptr;
-  capture_closed();
+  if (t_captures > 0) t_captures--;
   TGA_HIP(hipStreamEndCapture((hipStream_t)stream, &g));
   hipGraphExec_t ge = nullptr;
   hipError_t e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
