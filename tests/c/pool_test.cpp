@@ -85,9 +85,19 @@ static void capture_of_another_thread() {
   }
   CHECK(again && !g_capture_broken);
 }
+static void a_free_that_fails() {
+  keep(5 << 20, 12); keep(1 << 16, 12);
+  g_fail_free_after = 7;
+  { std::lock_guard<std::mutex> lock(g_pool_mutex); CHECK(pool_trim() != 0); }
+  g_fail_free_after = -1;
+  size_t kept = 0, dirty = 0;
+  for (auto& c : g_pools[0].classes) { kept += c.first * (c.second.clean.size() + c.second.dirty.size()); dirty += c.first * c.second.dirty.size(); }
+  CHECK(kept && kept == g_pools[0].kept && dirty == g_pools[0].dirty);
+  for (int i = 0; i < 60; i++) { void* q; CHECK(!pool_malloc(&q, i & 1 ? 5 << 20 : 1 << 16)); CHECK(g_live.count(q)); }
+}
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}};
+  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}};
   CHECK(argc == 2 && tests.count(argv[1]));
   tests.at(argv[1])();
   puts("ok");

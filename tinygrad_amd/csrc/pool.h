@@ -45,9 +45,16 @@ static int pool_settle(Pool& p) {                                               
 }
 static int pool_release(Pool& p) {                                                    // everything kept goes back to the driver (hipFree waits for the block's users)
   for (auto& c : p.classes) {
-    for (auto* v : {&c.second.clean, &c.second.dirty}) { for (void* q : *v) { g_pool_blocks.erase(q); TGA_HIP(hipFree(q)); } v->clear(); }
+    for (auto* v : {&c.second.clean, &c.second.dirty}) {
+      while (!v->empty()) {                                                           // (out of the lists first: where an hipFree fails, no block that is gone may stay in them)
+        void* q = v->back();
+        v->pop_back(); g_pool_blocks.erase(q); p.kept -= c.first;
+        if (v == &c.second.dirty) p.dirty -= c.first;
+        TGA_HIP(hipFree(q));
+      }
+    }
   }
-  p.classes.clear(); p.kept = p.dirty = 0;
+  p.classes.clear();
   return 0;
 }
 static int pool_trim() { for (auto& p : g_pools) if (const int rc = pool_release(p.second)) return rc; return 0; }
