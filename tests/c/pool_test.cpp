@@ -88,16 +88,28 @@ static void capture_of_another_thread() {
 static void a_free_that_fails() {
   keep(5 << 20, 12); keep(1 << 16, 12);
   g_fail_free_after = 7;
-  { std::lock_guard<std::mutex> lock(g_pool_mutex); CHECK(pool_trim() != 0); }
+  CHECK(pool_give_back() != 0);
   g_fail_free_after = -1;
   size_t kept = 0, dirty = 0;
   for (auto& c : g_pools[0].classes) { kept += c.first * (c.second.clean.size() + c.second.dirty.size()); dirty += c.first * c.second.dirty.size(); }
   CHECK(kept && kept == g_pools[0].kept && dirty == g_pools[0].dirty);
   for (int i = 0; i < 60; i++) { void* q; CHECK(!pool_malloc(&q, i & 1 ? 5 << 20 : 1 << 16)); CHECK(g_live.count(q)); }
 }
+static void capture_of_its_own() {                                          // (no call of the library may reach the runtime then)
+  void *a, *b; CHECK(!pool_malloc(&a, (size_t)3 << 30)); CHECK(!pool_malloc(&b, 1 << 20));
+  std::vector<void*> many(12); for (auto& q : many) CHECK(!pool_malloc(&q, (size_t)1 << 29));
+  t_captures = 1; g_capturing = true;
+  void* c = nullptr; CHECK(pool_malloc(&c, 1 << 20) != 0 && !c);
+  CHECK(!pool_free(a)); CHECK(!pool_free(b)); for (auto& q : many) CHECK(!pool_free(q));      // (6 GiB: more than are kept)
+  CHECK(pool_give_back() != 0);
+  CHECK(!g_capture_broken && g_live.count(a));
+  t_captures = 0; g_capturing = false;
+  CHECK(!pool_malloc(&c, 1 << 20)); CHECK(!g_live.count(a)); CHECK(!pool_free(c));
+  CHECK(!pool_give_back()); CHECK(g_live.empty() && !g_pools[0].kept && !g_pools[0].dirty);
+}
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}};
+  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}, {"capture_of_its_own", capture_of_its_own}};
   CHECK(argc == 2 && tests.count(argv[1]));
   tests.at(argv[1])();
   puts("ok");

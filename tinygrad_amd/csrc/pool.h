@@ -13,8 +13,8 @@
 //    blocks of the class or POOL_DIRTY_BYTES in all are dirty.  No stream has to be named, no caller synchronises more than it did.  The wait is that of an hipFree of a few bytes allocated
 //    for it (1.4 us where the device is idle): an hipDeviceSynchronize is refused during a capture of any thread and ends that capture, an hipFree only during one of its own (measured).
 //  * at most POOL_BYTES per device are kept; beyond, blocks go back to the driver, all of them do before a request is refused for want of memory, and on tga_trim().
-//  * size classes are eighths of a power of two (at most 12.5 % of a block is idle).  One mutex.  While its thread captures a stream, tga_free puts a block aside without a call to the runtime (an hipFree would
-//    invalidate the capture).
+//  * size classes are eighths of a power of two (at most 12.5 % of a block is idle).  One mutex.  While its thread captures a stream, tga_free puts any block aside without a call to the runtime (an hipFree would
+//    invalidate the capture); one of more than POOL_BLOCK_MAX bytes is freed with the next call of that thread outside a capture.  tga_trim is refused then.
 //  * a thread with a capture of its own open gets no block: the replays would go on using one that its call gave back when it returned (and hipMalloc itself refuses then).  Captures that
 //    the library did not open are the runtime's to know: an hipFree of nothing is refused during exactly those that hipMalloc is refused during (measured for the three capture modes).
 #define POOL_BLOCK_MAX ((size_t)1 << 30)
@@ -60,8 +60,11 @@ static int pool_release(Pool& p) {                                              
 static int pool_trim() { for (auto& p : g_pools) if (const int rc = pool_release(p.second)) return rc; return 0; }
 
 static thread_local int t_captures = 0;                                              // captures of this thread (tga_graph_begin .. tga_graph_end / tga_cmdlist_end: they end where they began)
+static thread_local std::vector<void*> t_large;                                      // blocks of no size class freed during one
+static int pool_free_large() { while (!t_large.empty()) { void* q = t_large.back(); t_large.pop_back(); TGA_HIP(hipFree(q)); } return 0; }
 static int pool_malloc(void** ptr, size_t n) {
   TGA_REQUIRE(!t_captures, "tga_malloc: not while this thread captures a stream");
+  if (const int rc = pool_free_large()) return rc;
   TGA_HIP(hipFree(nullptr));                                                          // (0.2 us) a capture that something else opened: refused (error 900) where hipMalloc is, else nothing
   if (n > POOL_BLOCK_MAX) {
     hipError_t e = hipMalloc(ptr, n);
@@ -91,9 +94,14 @@ static int pool_malloc(void** ptr, size_t n) {
   return 0;
 }
 static int pool_free(void* ptr) {
+  if (!t_captures) { if (const int rc = pool_free_large()) return rc; }
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   auto it = g_pool_blocks.find(ptr);
-  if (it == g_pool_blocks.end()) { TGA_HIP(hipFree(ptr)); return 0; }
+  if (it == g_pool_blocks.end()) {
+    if (t_captures) { t_large.push_back(ptr); return 0; }
+    TGA_HIP(hipFree(ptr));
+    return 0;
+  }
   TGA_REQUIRE(it->second.out, "tga_free: the block has been freed before");               // (as hipFree refuses it: kept twice, it would be handed out twice)
   const size_t cls = it->second.cls;
   Pool& p = g_pools[it->second.dev];
@@ -101,4 +109,10 @@ static int pool_free(void* ptr) {
   p.classes[cls].dirty.push_back(ptr);
   p.kept += cls; p.dirty += cls; it->second.out = false;
   return 0;
+}
+static int pool_give_back() {
+  TGA_REQUIRE(!t_captures, "tga_trim: not while this thread captures a stream");
+  if (const int rc = pool_free_large()) return rc;
+  std::lock_guard<std::mutex> lock(g_pool_mutex);
+  return pool_trim();
 }

@@ -43,7 +43,7 @@ int tga_malloc(void** ptr, size_t nbytes) {
   return pool_malloc(ptr, nbytes ? nbytes : 1);
 }
 int tga_free(void* ptr) { return ptr ? pool_free(ptr) : 0; }
-int tga_trim(void) { std::lock_guard<std::mutex> lock(g_pool_mutex); return pool_trim(); }
+int tga_trim(void) { return pool_give_back(); }
 int tga_memcpy_h2d(void* dst, const void* src, size_t n) { TGA_HIP(hipMemcpy(dst, src, n, hipMemcpyHostToDevice)); return 0; }
 int tga_memcpy_d2h(void* dst, const void* src, size_t n) { TGA_HIP(hipMemcpy(dst, src, n, hipMemcpyDeviceToHost)); return 0; }
 int tga_memcpy_d2d(void* dst, const void* src, size_t n, void* stream) {
