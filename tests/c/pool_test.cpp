@@ -107,9 +107,17 @@ static void capture_of_its_own() {                                          // (
   CHECK(!pool_malloc(&c, 1 << 20)); CHECK(!g_live.count(a)); CHECK(!pool_free(c));
   CHECK(!pool_give_back()); CHECK(g_live.empty() && !g_pools[0].kept && !g_pools[0].dirty);
 }
+static void classes_hold_little_more() {
+  for (size_t n = 4097; n <= POOL_BLOCK_MAX; n += 1 + n / 97)
+    for (size_t m : {n, n - n % 4096, n - n % 4096 + 1}) {
+      if (m < 4097) continue;
+      const size_t c = pool_class(m); CHECK(c >= m && (c - m) * 9 <= c && c % 512 == 0 && pool_class(c) == c);
+    }
+  for (int b = 12; b < 30; b++) { const size_t m = ((size_t)1 << b) + 1, c = pool_class(m); CHECK((c - m) * 9 <= c); }
+}
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}, {"capture_of_its_own", capture_of_its_own}};
+  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}, {"capture_of_its_own", capture_of_its_own}, {"classes_hold_little_more", classes_hold_little_more}};
   CHECK(argc == 2 && tests.count(argv[1]));
   tests.at(argv[1])();
   puts("ok");

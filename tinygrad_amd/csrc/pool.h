@@ -13,7 +13,7 @@
 //    blocks of the class or POOL_DIRTY_BYTES in all are dirty.  No stream has to be named, no caller synchronises more than it did.  The wait is that of an hipFree of a few bytes allocated
 //    for it (1.4 us where the device is idle): an hipDeviceSynchronize is refused during a capture of any thread and ends that capture, an hipFree only during one of its own (measured).
 //  * at most POOL_BYTES per device are kept; beyond, blocks go back to the driver, all of them do before a request is refused for want of memory, and on tga_trim().
-//  * size classes are eighths of a power of two (at most 12.5 % of a block is idle).  One mutex.  While its thread captures a stream, tga_free puts any block aside without a call to the runtime (an hipFree would
+//  * size classes are eighths of a power of two (at most 11.1 % of a block is idle).  One mutex.  While its thread captures a stream, tga_free puts any block aside without a call to the runtime (an hipFree would
 //    invalidate the capture); one of more than POOL_BLOCK_MAX bytes is freed with the next call of that thread outside a capture.  tga_trim is refused then.
 //  * a thread with a capture of its own open gets no block: the replays would go on using one that its call gave back when it returned (and hipMalloc itself refuses then).  Captures that
 //    the library did not open are the runtime's to know: an hipFree of nothing is refused during exactly those that hipMalloc is refused during (measured for the three capture modes).
@@ -32,7 +32,7 @@ static std::unordered_map<void*, PoolBlock> g_pool_blocks;                      
 static size_t pool_class(size_t n) {
   if (n <= 4096) return (n + 511) & ~(size_t)511;
   int b = 0; for (size_t t = n - 1; t >>= 1;) b++;                                   // 2^b < n <= 2^(b + 1)
-  const size_t step = (size_t)1 << (b - 2);
+  const size_t step = (size_t)1 << (b - 3);
   return (n + step - 1) & ~(step - 1);
 }
 static int pool_settle(Pool& p) {                                                     // every dirty block becomes clean (not where there is no memory left: the caller trims then)
