@@ -1,5 +1,6 @@
 // Device allocations behind tga_malloc / tga_free (included by runtime.hip, and on the host by the test of its rules, which brings functions of its own under the names of the runtime's).
 #pragma once
+#include <exception>
 #include <map>
 #include <mutex>
 #include <unordered_map>
@@ -62,7 +63,7 @@ static int pool_trim() { for (auto& p : g_pools) if (const int rc = pool_release
 static thread_local int t_captures = 0;                                              // captures of this thread (tga_graph_begin .. tga_graph_end / tga_cmdlist_end: they end where they began)
 static thread_local std::vector<void*> t_large;                                      // blocks of no size class freed during one
 static int pool_free_large() { while (!t_large.empty()) { void* q = t_large.back(); t_large.pop_back(); TGA_HIP(hipFree(q)); } return 0; }
-static int pool_malloc(void** ptr, size_t n) {
+static int pool_malloc_(void** ptr, size_t n) {
   TGA_REQUIRE(!t_captures, "tga_malloc: not while this thread captures a stream");
   if (const int rc = pool_free_large()) return rc;
   TGA_HIP(hipFree(nullptr));                                                          // (0.2 us) a capture that something else opened: refused (error 900) where hipMalloc is, else nothing
@@ -90,10 +91,10 @@ static int pool_malloc(void** ptr, size_t n) {
     e = hipMalloc(ptr, cls);
   }
   TGA_HIP(e);
-  g_pool_blocks[*ptr] = {cls, dev, true};
+  try { g_pool_blocks[*ptr] = {cls, dev, true}; } catch (...) { (void)hipFree(*ptr); *ptr = nullptr; throw; }
   return 0;
 }
-static int pool_free(void* ptr) {
+static int pool_free_(void* ptr) {
   if (!t_captures) { if (const int rc = pool_free_large()) return rc; }
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   auto it = g_pool_blocks.find(ptr);
@@ -110,9 +111,16 @@ static int pool_free(void* ptr) {
   p.kept += cls; p.dirty += cls; it->second.out = false;
   return 0;
 }
-static int pool_give_back() {
+static int pool_give_back_() {
   TGA_REQUIRE(!t_captures, "tga_trim: not while this thread captures a stream");
   if (const int rc = pool_free_large()) return rc;
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   return pool_trim();
 }
+// (the lists may throw where the host has no memory left: an error at the C entries)
+template <typename F> static int pool_guarded(const char* who, F f) {
+  try { return f(); } catch (const std::exception& e) { return tga_set_error("%s: %s", who, e.what()); }
+}
+static int pool_malloc(void** ptr, size_t n) { return pool_guarded("tga_malloc", [&] { return pool_malloc_(ptr, n); }); }
+static int pool_free(void* ptr) { return pool_guarded("tga_free", [&] { return pool_free_(ptr); }); }
+static int pool_give_back() { return pool_guarded("tga_trim", [] { return pool_give_back_(); }); }
