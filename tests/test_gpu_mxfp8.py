@@ -277,3 +277,33 @@ def test_moe_feed_forward_at_tile_edges(gpu, T, D, I, E, k):
   got = moe.from_bf16_bits(moe.moe_feed_forward(B(inp), B(logits), k, (B(gq), B(ge)), B(bgu), (B(dq), B(de)), B(bdn)).numpy())
   assert np.isfinite(got).all() and np.abs(got - ref).mean() / np.abs(ref).mean() < 1e-2
   np.testing.assert_allclose(got, ref, rtol=0.05, atol=0.02 * np.abs(ref).max())
+
+def _single_steps(moe, inp, logits, k, gate_up, b_gate_up, down, b_down):
+  r = moe.route(logits, k, logits.shape[1])
+  xg = moe.dispatch(inp, r)
+  h = moe.add_expert_bias(moe.grouped_mx_gemm(xg, gate_up, r.off, routed_only=True, counts=r.counts), b_gate_up, r.off)
+  y = moe.swiglu(h)
+  z = moe.add_expert_bias(moe.grouped_mx_gemm(y, down, r.off, routed_only=True, counts=r.counts), b_down, r.off)
+  return moe.combine(z, r, inp.shape[0], k).numpy()
+
+@pytest.mark.parametrize("case", ["random", "masked", "fewer than k", "tiny"])
+def test_moe_feed_forward_has_the_bits_of_the_single_steps(gpu, case):
+  """Random rows; logits masked with -inf so that exactly k, or fewer than k, experts are left (the surplus picks weigh nothing); gate values whose sigmoid is a subnormal number."""
+  from tinygrad_amd import moe
+  T, D, I, E, k = 70, 512, 256, 16, 3
+  rng = np.random.default_rng(len(case))
+  B = gpu.Buffer.from_numpy
+  inp, logits = moe.to_bf16_bits(rng.standard_normal((T, D)).astype(np.float32)), rng.standard_normal((T, E)).astype(np.float32)
+  wgu, wdn = (rng.standard_normal((E, 2 * I, D)) * D ** -0.5).astype(np.float32), (rng.standard_normal((E, D, I)) * I ** -0.5).astype(np.float32)
+  bgu, bdn = (rng.standard_normal((E, 2 * I)) * 0.1).astype(np.float32), (rng.standard_normal((E, D)) * 0.1).astype(np.float32)
+  if case in ("masked", "fewer than k"):
+    keep = np.argsort(rng.random((T, E)), axis=1)[:, :k if case == "masked" else k - 1]
+    mask = np.full((T, E), -np.inf, np.float32); np.put_along_axis(mask, keep, 0, axis=1)
+    logits += mask
+  if case == "tiny":                                                   # gate = bias: 1.702 times it rounds to -87.5, -88 and -88.5, whose logistic function lies below the normal numbers
+    wgu[:] = 0; bdn[:] = 0
+    bgu[:, 0::2], bgu[:, 1::2] = np.array([-51.5, -51.75, -52.0], np.float32)[np.arange(E) % 3][:, None], 6.0
+  args = (B(inp), B(logits), k, tuple(map(B, omx.quantize_mxfp8(wgu))), B(bgu), tuple(map(B, omx.quantize_mxfp8(wdn))), B(bdn))
+  got, ref = moe.moe_feed_forward(*args).numpy(), _single_steps(moe, *args)
+  assert case != "tiny" or (ref & 0x7FFF).any()
+  np.testing.assert_array_equal(got, ref)

@@ -314,7 +314,7 @@ __global__ __launch_bounds__(256 * WM) void ffn_gemm_kernel(const FfnArgs a) {
             const float gl0 = fminf(bf16_lo(g01), a.limit), gl1 = fminf(bf16_lo(g23), a.limit);
             const float li0 = fminf(fmaxf(bf16_hi(g01), -a.limit), a.limit), li1 = fminf(fmaxf(bf16_hi(g23), -a.limit), a.limit);
             const uint32_t ag = pack_bf16x2(1.702f * gl0, 1.702f * gl1);
-            const uint32_t sg = pack_bf16x2(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * bf16_lo(ag))), __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * bf16_hi(ag))));
+            const uint32_t sg = pack_bf16x2(mx_sigmoid_bf16(bf16_lo(ag)), mx_sigmoid_bf16(bf16_hi(ag)));
             const uint32_t p = pack_bf16x2(gl0 * bf16_lo(sg), gl1 * bf16_hi(sg)), q = pack_bf16x2(li0 + 1.0f, li1 + 1.0f);
             const uint32_t o = pack_bf16x2(bf16_lo(p) * bf16_lo(q), bf16_hi(p) * bf16_hi(q));
             y[2 * j] = bf16_lo(o); y[2 * j + 1] = bf16_hi(o);
