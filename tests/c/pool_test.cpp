@@ -66,13 +66,13 @@ static void waits_before_handing_out() {
   for (int i = 0; i < 30; i++) {
     void* a; CHECK(!pool_malloc(&a, 3 << 20)); const int w = g_waits; CHECK(!pool_free(a));
     std::vector<void*> got;
-    for (int j = 0; j < 12; j++) { void* b; CHECK(!pool_malloc(&b, 3 << 20)); if (b == a) CHECK(g_waits > w); got.push_back(b); }
+    for (int j = 0; j < 40; j++) { void* b; CHECK(!pool_malloc(&b, 3 << 20)); if (b == a) CHECK(g_waits > w); got.push_back(b); }
     for (void* b : got) CHECK(!pool_free(b));
   }
 }
 
 static void keep(size_t n, int count) {                                    // so many kept blocks of a class, free to be handed out
-  std::vector<void*> b(count + 8); for (auto& q : b) CHECK(!pool_malloc(&q, n)); for (auto& q : b) CHECK(!pool_free(q));
+  std::vector<void*> b(count + POOL_DIRTY_COUNT_MAX); for (auto& q : b) CHECK(!pool_malloc(&q, n)); for (auto& q : b) CHECK(!pool_free(q));
   void* q; CHECK(!pool_malloc(&q, n)); CHECK(!pool_free(q));
 }
 static void capture_opened_elsewhere() {
@@ -130,9 +130,22 @@ static void no_host_memory() {
   CHECK(rc && !a && rf && g_live.size() == 1);
   CHECK(!pool_free(b)); CHECK(!pool_malloc(&a, 7 << 20));                  // (the block that could not be listed is still the caller's)
 }
+static void full_of_other_blocks() {
+  for (size_t n : {(size_t)200 << 20, (size_t)300 << 20}) {                // 6 GiB of two classes, all freed: 4 GiB are kept
+    std::vector<void*> b(12); for (auto& q : b) CHECK(!pool_malloc(&q, n)); for (auto& q : b) CHECK(!pool_free(q));
+  }
+  CHECK(g_pools[0].kept <= POOL_BYTES && g_pools[0].kept > POOL_BYTES - 2 * ((size_t)320 << 20));
+  int mallocs = 0;
+  for (int i = 0; i < 400; i++) {
+    if (i == 200) mallocs = g_mallocs;
+    void *a, *b; CHECK(!pool_malloc(&a, 2 << 20)); CHECK(!pool_malloc(&b, 128 << 10)); CHECK(!pool_free(a)); CHECK(!pool_free(b));
+  }
+  CHECK(g_mallocs - mallocs <= 2 * 200 / POOL_DIRTY_COUNT);                 // (the few bytes of each wait)
+  CHECK(g_pools[0].kept <= POOL_BYTES);
+}
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}, {"capture_of_its_own", capture_of_its_own}, {"classes_hold_little_more", classes_hold_little_more}, {"no_host_memory", no_host_memory}};
+  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}, {"capture_of_its_own", capture_of_its_own}, {"classes_hold_little_more", classes_hold_little_more}, {"no_host_memory", no_host_memory}, {"full_of_other_blocks", full_of_other_blocks}};
   CHECK(argc == 2 && tests.count(argv[1]));
   tests.at(argv[1])();
   puts("ok");
