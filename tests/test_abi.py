@@ -66,6 +66,25 @@ def test_moe_feed_forward_refuses_operands_of_other_sizes(monkeypatch):
   with pytest.raises(RuntimeError): call(dq=((E, 256, I), np.uint8))               # (the library above refuses the single steps' first call)
   assert calls == ["fused", "single"]
 
+def test_prefill_step_refuses_what_its_kernels_cannot_address():
+  """Rows whose activations lie beyond 2^32 values, expert counts and gating kinds that do not exist and expert formats without a kernel are errors before anything is launched (pointers here lead nowhere)."""
+  from tinygrad_amd import runtime as rt
+  L = rt.load_library()
+  NAMES = "NBLOCKS DIM HEADS KV HD MAXCTX EMB EMB_TYPE ROPE EXPERTS TOPK GATING NORM_TOPK QKNORM HIDDEN DENSE_HIDDEN EPS_BITS SCALE_BITS".split()
+  good = dict(NBLOCKS=1, DIM=2048, HEADS=16, KV=16, HD=128, MAXCTX=1 << 20, EMB=4096, EMB_TYPE=2, ROPE=4096, EXPERTS=64, TOPK=8, GATING=1, NORM_TOPK=0, QKNORM=0, HIDDEN=1024, DENSE_HIDDEN=0, EPS_BITS=0, SCALE_BITS=0)
+  def call(rows, words, types=(39, 39), **other):
+    m = (ctypes.c_int64 * len(NAMES))(*[{**good, **other}[n] for n in NAMES])
+    b = (ctypes.c_int64 * 21)(*([4096] * 6 + [1] + [4096] * 8 + [1, 1, 1, 1, *types]))
+    assert L.tga_prefill_step(m, b, 4096, 1, rows, 0, 4096, 4096, None) != 0
+    assert words in L.tga_last_error().decode(), L.tga_last_error()
+  call((1 << 20) - 1, "more than a step takes")                                    # 2^20 rows x 8 experts x 1024 values
+  call((1 << 19) + 8, "more than a step takes")
+  call((1 << 19) + 8, "more than a step takes", EXPERTS=0, HIDDEN=8192)
+  call(1 << 19, "more than a step takes", DIM=8192, HIDDEN=256)
+  call(32, "of 64 experts", TOPK=0); call(32, "of 4 experts", EXPERTS=4)
+  call(32, "ExpertGating 0", GATING=0); call(32, "ExpertGating 5", GATING=5)
+  call(32, "experts of block 0", types=(39, 22)); call(32, "experts of block 0", types=(12, 39), DIM=2048 + 128)
+
 @pytest.mark.gpu
 def test_freed_blocks_are_kept_and_given_back(gpu):
   """tga_free keeps a block for later requests of its size class, never hands it out while kernels may still use it, and tga_trim gives everything back: results computed into

@@ -317,6 +317,15 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
   TGA_REQUIRE(m && blocks && tokens && workspace && state && nseq >= 1 && P >= 1 && pos0 >= 0 && pos0 + P <= m[PM_MAXCTX], "tga_prefill_step: null pointer or rows beyond the cache");
   const int64_t R = nseq * P, dim = m[PM_DIM], H = m[PM_HEADS], KV = m[PM_KV], hd = m[PM_HD], nq = H * hd, nk = KV * hd, E = m[PM_EXPERTS], k = m[PM_TOPK];
   TGA_REQUIRE((hd == 64 || hd == 128) && KV > 0 && H % KV == 0 && E <= PF_MAX_E && k <= 64 && R < (1 << 20), "tga_prefill_step: geometry outside the range");
+  // (the kernels form the place of an activation row, row * values, in 32 bits)
+  const int64_t hidden = m[PM_HIDDEN];
+  TGA_REQUIRE(R * dim < (1ll << 32) && R * nq < (1ll << 32) && R * (E ? m[PM_DENSE_HIDDEN] : hidden) < (1ll << 32), "tga_prefill_step: %lld rows of that model are more than a step takes", (long long)R);
+  TGA_REQUIRE(!E || (k >= 1 && k <= E && hidden >= 1 && R * k * hidden < (1ll << 32)), "tga_prefill_step: %lld rows of %lld of %lld experts are more than a step takes", (long long)R, (long long)k, (long long)E);
+  TGA_REQUIRE(!E || (m[PM_GATING] >= 1 && m[PM_GATING] <= 4), "tga_prefill_step: unknown ExpertGating %lld", (long long)m[PM_GATING]);
+  for (int64_t bi = 0; bi < m[PM_NBLOCKS]; bi++) {
+    const int64_t* b = blocks + bi * PB_COUNT;
+    TGA_REQUIRE(!b[PB_MOE] || (E && tga_rows_fmt((int)b[PB_TGATE], dim) >= 0 && tga_rows_fmt((int)b[PB_TDOWN], hidden) >= 0), "tga_prefill_step: the experts of block %lld are outside the range", (long long)bi);
+  }
   const PfWs w = pf_layout(m, R);
   uint8_t* ws = (uint8_t*)workspace;
   float* x = (float*)(ws + w.x); uint16_t* xn = (uint16_t*)(ws + w.xn); float* q = (float*)(ws + w.q); float* kk = (float*)(ws + w.k); float* v = (float*)(ws + w.v);
