@@ -158,6 +158,21 @@ def test_rows_beyond_the_prompt_do_not_count(gpu, n):
   for ba, bb in zip(a.blk, b.blk):
     for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): np.testing.assert_array_equal(ca.numpy()[:, :n - 1], cb.numpy()[:, :n - 1])
 
+@pytest.mark.parametrize("cfg", [DENSE, DENSE128], ids=["hd64", "hd128"])
+def test_cache_rows_have_the_bits_of_the_other_appends(gpu, cfg):
+  """A rotated key is the float32 result of one rounded product and one fused multiply-add, then rounded to fp16 (model.py:29-33 as every kernel that appends writes it): the bits of the cache rows,
+  from the keys in the step's workspace.  (The exact sum in float64 carries the float32 rounding's ties right: products of two 24-bit numbers and a third one.)"""
+  n, dim, nq, nk, hd = 300, cfg["dim"], cfg["n_heads"] * cfg["head_dim"], cfg["n_kv_heads"] * cfg["head_dim"], cfg["head_dim"]
+  a = _model(dict(cfg, num_blocks=1), 17)
+  a.prefill(np.random.default_rng(n).integers(0, cfg["vocab_size"], size=n + 1).tolist())
+  up = lambda b: (b + 255) // 256 * 256                                            # (x, xn, q, k: pf_layout)
+  k = a._chunker._rows_ws.view(up(n * dim * 4) + up(n * dim * 2) + up(n * nq * 4), (n, nk // hd, hd), np.float32).numpy()
+  rope = a.s.rope.numpy().reshape(-1, hd)[:n, None, :]
+  x1, x2, c, s = k[..., :hd // 2], k[..., hd // 2:], rope[..., :hd // 2], rope[..., hd // 2:]
+  f = np.float64
+  ref = np.concatenate([(f(x1) * f(c) - f(x2 * s)).astype(np.float32), (f(x2) * f(c) + f(x1 * s)).astype(np.float32)], -1).astype(np.float16)
+  np.testing.assert_array_equal(a.blk[0].cache_k.numpy()[:, :n].view(np.uint16), ref.transpose(1, 0, 2).view(np.uint16))
+
 def test_moe_prompts_keep_their_steps_unless_asked(gpu):
   """A MoE model's prefill computes the bits of steps of sixteen rows (and of lockstep steps): another order of sums turns expert choices at near-ties, so steps of many rows are the user's
   choice there (many_rows), not the default."""

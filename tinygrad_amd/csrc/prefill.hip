@@ -78,7 +78,8 @@ __global__ __launch_bounds__(256) void rows_rope_kernel(const RopeArgs a) {
         const int wo = a.norm == 2 ? 0 : hh * a.hd;
         x1 = (x1 * sc) * w[wo + i]; x2 = (x2 * sc) * w[wo + half + i];
       }
-      const float lo = __builtin_fmaf(x1, c, -(x2 * s)), hi = __builtin_fmaf(x2, c, x1 * s);
+      float lo = __builtin_fmaf(x1, c, -(x2 * s)), hi = __builtin_fmaf(x2, c, x1 * s);
+      asm volatile("" : "+v"(lo), "+v"(hi));                            // (float32 values: folded with the conversion into v_fma_mixlo_f16 they round once, and some cache rows had other bits)
       if (!live) continue;
       if (isq) {
         const size_t o = (size_t)r * nq + hh * a.hd + i;
