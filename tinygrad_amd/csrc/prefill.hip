@@ -17,8 +17,8 @@ int tga_rows_linear(int ggml_type, int nseg, const void* const* w, void* const* 
 int tga_rows_norm(float* x, const float* w, int M, int n, float eps, void* xn, void* stream);
 
 // ------------------------------------------------------------------------------------------------ rotation + append
-// One workgroup per row.  q is rotated (after its norm) and leaves as TWO fp16 values per element, the rounded value and what the rounding left over, so that the matrix-core
-// scores see the float32 query; k is rotated into the cache, v copied.  The rotation is apply_rope's (model.py:29-33) written as one rounded product and one fused multiply-add,
+// One workgroup per row.  q is rotated (after its norm) and leaves as TWO fp16 values per element, the rounded value and what the rounding left over, for matrix-core
+// scores of the float32 query (rows_attn_kernel); k is rotated into the cache, v copied.  The rotation is apply_rope's (model.py:29-33) written as one rounded product and one fused multiply-add,
 // like every kernel that rotates, so a cache row has the same bits whichever path appended it.  norm: 0 none, 1 RMSNorm over the whole q / k rows (model.py:169), 2 per head (:180).
 struct RopeArgs {
   const float* q; const float* k; const float* v; const float* qn; const float* kn; const float* rope;
@@ -97,10 +97,13 @@ __global__ __launch_bounds__(256) void rows_rope_kernel(const RopeArgs a) {
 // ------------------------------------------------------------------------------------------------ attention
 // Causal attention of the rows over the cache (their own keys included): workgroup = 64 rows of one query head, wave = 16 of them, tiles of 64 keys with a running maximum.
 // S^T = K Q^T: keys as A operand from LDS (rows of head_dim values, 16-byte pieces XORed with the key), the rotated queries as two fp16 B operands held in registers.
-// O^T = V^T P^T: the probabilities as a rounded value and its remainder, so that they count in float32 like the decode kernels' (each product once more on matrix cores
-// that are far from busy here); the eight keys a lane holds after the first product are taken as they are, and V is written to LDS transposed with its keys in that order, two keys
+// O^T = V^T P^T: the probabilities likewise as a rounded value and its remainder (each product once more on matrix cores that are far from busy here); the eight keys a lane holds after the first product are taken as they are, and V is written to LDS transposed with its keys in that order, two keys
 // per dword, pieces XORed with the dimension.  The next tile is fetched while this one is multiplied.  flattened workgroup = (kv head, sequence) innermost: with eight
 // kv heads all readers of a head's rows run on one XCD and share its L2; the longest row tiles come first.
+// Two fp16 values hold 22 bits and more of a query or probability, and sums are formed in few additions at their full size (remainders first, two chains per score, a tile's products from
+// zero).  Share of fp16 results that are not the rounded float64 attention, 64 and 1024 positions, heads of 64 and 128, scores of standard deviation 0.03 .. 5: 1.8e-4 .. 2.2e-3; the float32
+// kernel of eight rows and fewer: 2.4e-4 .. 2.4e-3.  (Queries beyond 65504 have no such pair, as keys beyond have no cache row.)
+#define PSCALE 32768.0f             // of probabilities on their way to two fp16 values (the remainder of 0.2 is a subnormal number already: the absolute step 2^-24)
 struct RowsAttnArgs { const uint16_t* qh; const uint16_t* ql; const uint16_t* ck; const uint16_t* cv; uint16_t* out; int H, KV, max_ctx, P, pos0, nseq, qtiles; float scale; };
 
 template <int HD>
@@ -166,12 +169,19 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
       for (int k = 0; k < 4; k++) {
         sc[k] = v4f32{0.f, 0.f, 0.f, 0.f};
         const int key = 16 * k + c;
+        v8f16 ka[NJ];
 #pragma unroll
-        for (int j = 0; j < NJ; j++) {
-          const v8f16 ka = *(const v8f16*)(kl + key * HD * 2 + (((4 * j + g) ^ (key & 7)) << 4));
-          sc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, __builtin_bit_cast(v8f16, qr[j]), sc[k], 0, 0, 0);
-          sc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, __builtin_bit_cast(v8f16, qb[j]), sc[k], 0, 0, 0);
+        for (int j = 0; j < NJ; j++) ka[j] = *(const v8f16*)(kl + key * HD * 2 + (((4 * j + g) ^ (key & 7)) << 4));
+        // (the remainders' products first, then two chains: fewer additions at the size of the whole sum)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) sc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[j], __builtin_bit_cast(v8f16, qr[j]), sc[k], 0, 0, 0);
+        v4f32 s2 = v4f32{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NJ / 2; j++) {
+          sc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[j], __builtin_bit_cast(v8f16, qb[j]), sc[k], 0, 0, 0);
+          s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[NJ / 2 + j], __builtin_bit_cast(v8f16, qb[NJ / 2 + j]), s2, 0, 0, 0);
         }
+        sc[k] += s2;
       }
       float m = -INFINITY;
       const bool mask = 64 * t + 63 > first_wave;
@@ -179,12 +189,12 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
       for (int k = 0; k < 4; k++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          float s = sc[k][i] * a.scale;                                    // (log2(e) folded into the scale)
+          float s = sc[k][i];
           if (mask) s = 64 * t + 16 * k + 4 * g + i <= pos ? s : -INFINITY;
           sc[k][i] = s; m = fmaxf(m, s);
         }
       m = fmaxf(m, __shfl_xor(m, 16)); m = fmaxf(m, __shfl_xor(m, 32));
-      const float mn = fmaxf(M, m);                                        // (finite: key 0 is visible to every row)
+      const float mn = fmaxf(M, m * a.scale);                              // (finite: key 0 is visible to every row; log2(e) folded into the scale)
       const float alpha = __builtin_amdgcn_exp2f(M - mn);
       float l = 0.f;
       u32x4 ph[2], pl[2];
@@ -193,31 +203,34 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
 #pragma unroll
         for (int w = 0; w < 4; w++) {
           const int k = 2 * u + (w >> 1), i = 2 * (w & 1);
-          const float p0 = __builtin_amdgcn_exp2f(sc[k][i] - mn), p1 = __builtin_amdgcn_exp2f(sc[k][i + 1] - mn);
+          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[k][i], a.scale, -mn)), p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[k][i + 1], a.scale, -mn));
           l += p0 + p1;
-          const _Float16 h0 = (_Float16)p0, h1 = (_Float16)p1;
+          const float q0 = p0 * PSCALE, q1 = p1 * PSCALE;
+          const _Float16 h0 = (_Float16)q0, h1 = (_Float16)q1;
           ph[u][w] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-          pl[u][w] = f2h_bits(p0 - (float)h0) | (f2h_bits(p1 - (float)h1) << 16);
+          pl[u][w] = f2h_bits(q0 - (float)h0) | (f2h_bits(q1 - (float)h1) << 16);
         }
       l += __shfl_xor(l, 16); l += __shfl_xor(l, 32);
       L = L * alpha + l; M = mn;
 #pragma unroll
       for (int h = 0; h < NH; h++) {
-        v4f32 o = O[h] * alpha;
+        // (the tile's products sum from zero, remainders first: one addition at the size of the whole sum)
+        v8f16 va[2]; v4f32 o = v4f32{0.f, 0.f, 0.f, 0.f};
         const int d = 16 * h + c;
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-          const v8f16 va = *(const v8f16*)(vl + d * 128 + (((4 * u + g) ^ ((d ^ (d >> 3)) & 7)) << 4));
-          o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, __builtin_bit_cast(v8f16, pl[u]), o, 0, 0, 0);
-          o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, __builtin_bit_cast(v8f16, ph[u]), o, 0, 0, 0);
-        }
-        O[h] = o;
+        for (int u = 0; u < 2; u++) va[u] = *(const v8f16*)(vl + d * 128 + (((4 * u + g) ^ ((d ^ (d >> 3)) & 7)) << 4));
+#pragma unroll
+        for (int u = 0; u < 2; u++) o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[u], __builtin_bit_cast(v8f16, pl[u]), o, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 2; u++) o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[u], __builtin_bit_cast(v8f16, ph[u]), o, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) O[h][i] = __builtin_fmaf(O[h][i], alpha, o[i]);
       }
     }
     __syncthreads();
   }
   if (wrow + c < a.P) {
-    const float inv = 1.0f / L;
+    const float inv = (1.0f / PSCALE) / L;
     uint16_t* o = a.out + ((size_t)z * a.P + wrow + c) * nq + head * HD + 4 * g;
 #pragma unroll
     for (int h = 0; h < NH; h++) *(u32x2*)(o + 16 * h) = u32x2{f2h_bits(O[h][0] * inv) | (f2h_bits(O[h][1] * inv) << 16), f2h_bits(O[h][2] * inv) | (f2h_bits(O[h][3] * inv) << 16)};
@@ -367,7 +380,7 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
     TGA_LAUNCH_CHECK();
     RowsAttnArgs aa;
     aa.qh = ra.qh; aa.ql = ra.ql; aa.ck = ra.ck; aa.cv = ra.cv; aa.out = attn; aa.H = (int)H; aa.KV = (int)KV; aa.max_ctx = ra.max_ctx; aa.P = (int)P; aa.pos0 = (int)pos0; aa.nseq = (int)nseq;
-    aa.qtiles = (int)((P + 63) / 64); aa.scale = 1.4426950408889634f / sqrtf((float)hd);
+    aa.qtiles = (int)((P + 63) / 64); aa.scale = (float)(1.4426950408889634 / sqrt((double)hd));
     const unsigned ag = (unsigned)(aa.qtiles * H * nseq);
     if (hd == 64) rows_attn_kernel<64><<<ag, 256, 0, s>>>(aa); else rows_attn_kernel<128><<<ag, 256, 0, s>>>(aa);
     TGA_LAUNCH_CHECK();
