@@ -115,7 +115,7 @@ def test_chunked_prefill_vs_token_by_token_and_oracle(gpu, n_prompt, chunk):
   greedy tokens are the oracle's.  Prompt lengths that leave 0..7 positions behind the whole chunks (computed by one more chunk that ends at the last position) and cross the 64-position splits."""
   model, host = _build(gpu, SMALL, 192, seed=21)
   single, _ = _build(gpu, SMALL, 192, seed=21)
-  model.prefill_chunk, single.prefill_chunk = chunk, 1
+  model.prefill_chunk, single.prefill_chunk, model.many_rows = chunk, 1, False           # (steps of `chunk` positions: prompts in one step are tests/test_gpu_many_rows.py)
   rng = np.random.default_rng(21 + n_prompt)
   prompt = [int(t) for t in rng.integers(0, SMALL["vocab_size"], size=n_prompt)]
   model.prefill(prompt); single.prefill(prompt)
@@ -148,9 +148,9 @@ def test_prefill_steps_with_rows_in_the_multiplying_layout_equal_the_plain_steps
       c = TransformerConfig(max_context=192, **cfg)
       model = Transformer(c, synth_state(c, seed=33, q4_k_m=True), max_new=64)
     else: model, _ = _build(gpu, cfg, 192, seed=33, linear_type=getattr(rt, ltype))
-    model.prefill_chunk = chunk
+    model.prefill_chunk, model.many_rows = chunk, False
     model.prefill(prompt)
-    assert bool(model._chunker.rows64) == (flag == "1")
+    assert bool(model._chunker.rows64) == (flag == "1") and model._chunker.x is not None and model._chunker._rows_ws is None      # (the steps ran, not one of many rows)
     caches.append([(b.cache_k.numpy().astype(np.float32), b.cache_v.numpy().astype(np.float32)) for b in model.blk])
     toks.append(list(model.generate(prompt, 8)))
   for (k1, v1), (k0, v0) in zip(*caches):

@@ -697,7 +697,7 @@ class BatchedTransformer:
     def fits(l):
       ok = ctypes.c_int(0); rt.check(rt.lib().tga_rows_format_ok(l.ggml_type, l.in_features, ctypes.byref(ok)))
       return bool(ok.value) and l.blocks.ptr % (16 if l.ggml_type == rt.F16 else 1 if l.ggml_type == rt.MXFP4 else 4) == 0
-    if c.head_dim not in (64, 128) or c.shared_expert_dim or c.num_experts > 512 or c.num_experts_per_tok > 64 or os.environ.get("TGA_ROWS64", "1") != "1": return None
+    if c.head_dim not in (64, 128) or c.shared_expert_dim or c.num_experts > 512 or c.num_experts_per_tok > 64: return None
     rows = []
     for b in self.blk:
       ffn = [b["gate_exps"], b["up_exps"], b["down_exps"]] if b["moe"] else [b["ffn_gate"], b["ffn_up"], b["ffn_down"]]
