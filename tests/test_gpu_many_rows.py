@@ -1,6 +1,6 @@
 """Prefill steps of many rows on the GPU: tga_qlinear_many for every format at tile edges against a float64 product over the dequantized (fp16-rounded) weights, and whole steps - one
 sequence and several, dense and MoE, one step and a prompt cut into several - against the same models prefilled position by position."""
-import ctypes
+import ctypes, dataclasses
 import numpy as np, pytest
 from oracle import ggml as og, linear as ol, llm as ollm
 from tinygrad_amd import synth
@@ -230,3 +230,99 @@ def test_moe_prompts_keep_their_steps_unless_asked(gpu):
   batch = _model(MOE, 13, 128, 4)
   batch.prefill([prompt] * 4)
   assert batch._rows_ws is None
+
+# ---- expert products: models whose embeddings decide the routing (no near-ties: the rows path and the steps agree at every position)
+def _blocks_of_unit_gain(rng, rt, t, n, k):
+  """(n, k) random blocks whose weights are about k ** -0.5."""
+  if t == rt.F16: return (rng.standard_normal((n, k)) * k ** -0.5).astype(np.float16).view(np.uint8).reshape(-1)
+  if t == rt.MXFP4: return synth.random_blocks(rng, t, n, k, mx_exp=(120, 124))
+  seed, sigma = rng.integers(1 << 30), 0.003
+  std = og.ggml_data_to_tensor(synth.random_blocks(np.random.default_rng(seed), t, n, k, sigma), n * k, t).std()
+  return synth.random_blocks(np.random.default_rng(seed), t, n, k, sigma * k ** -0.5 / float(std))
+
+def _routed(rt, seed=23, expert_type=None, gate=0.2, **over):
+  """(config, state) of a MoE model in which token t goes to expert t % E first and to another one, given by t // E, second; experts add about as much to a row as its embedding has."""
+  from tinygrad_amd.llm import TransformerConfig, synth_state_moe
+  c = TransformerConfig(max_context=1152, **dict(MOE, **over))
+  sd = synth_state_moe(c, seed=seed)
+  rng, E, D, H = np.random.default_rng(seed), c.num_experts, c.dim, c.hidden_dim
+  u = np.linalg.qr(rng.standard_normal((D, E)))[0].T * D ** 0.5                       # E directions, orthogonal, unit root mean square
+  t = np.arange(c.vocab_size)
+  first, second = t % E, (t % E + 1 + t // E % (E - 1)) % E
+  put = lambda name, a, dt=np.float16: sd[name][0].view(0, a.shape, dt).copyin(a.astype(dt))
+  put("token_embd.weight", 0.3 * (0.2 * rng.standard_normal((c.vocab_size, D)) + 0.8 * u[first] + 0.5 * u[second]))
+  for i in range(c.num_blocks):
+    p = f"blk.{i}."
+    put(p + "attn_output.weight", 0.1 * rng.standard_normal((D, c.n_heads * c.head_dim)) * (c.n_heads * c.head_dim) ** -0.5)
+    if i < c.leading_dense_blocks: continue
+    put(p + "ffn_gate_inp.weight", gate * u * 10 / D)
+    for nm, n, k in (("ffn_gate_exps", H, D), ("ffn_up_exps", H, D), ("ffn_down_exps", D, H)):
+      if expert_type is None: continue
+      sd[p + nm + ".weight"] = (rt.Buffer.from_numpy(np.concatenate([_blocks_of_unit_gain(rng, rt, expert_type, n, k) for _ in range(E)])), expert_type, (E, n, k))
+  return c, sd
+
+def _rows_and_steps_agree(rt, c, sd, prompt):
+  """The prompt as steps of many rows and as the steps a MoE model takes by default: caches and logits within the bars of the dense models.  Returns the model of many rows."""
+  from tinygrad_amd.llm import Transformer
+  a, b = Transformer(c, sd, max_new=8), Transformer(c, sd, max_new=8)
+  a.many_rows, b.many_rows = True, False
+  for m in (a, b): m.prefill(prompt)
+  chunker = a._chunker or a._tail_chunkers[16]
+  assert chunker.x is None and chunker._rows_ws is not None
+  for ba, bb in zip(a.blk, b.blk):
+    for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)):
+      ca, cb = ca.numpy().astype(np.float32), cb.numpy().astype(np.float32)
+      assert np.isfinite(ca).all() and ol.rel_err(ca, cb) <= 2e-3
+  for m in (a, b): m.decode_step(); m.check_state()
+  assert ol.rel_err(a.logits(), b.logits()) <= 2e-3
+  return a
+
+@pytest.mark.parametrize("counts", [(0, 1, 31, 32, 33, 65, 63, 31), (0, 1, 63, 64, 65, 129, 33, 32), (0, 1, 127, 128, 129, 257, 64, 100), (0, 0, 0, 700, 0, 0, 70, 10)], ids=["32", "64", "128", "skewed"])
+def test_expert_tiles_of_every_height(gpu, counts):
+  """Expert counts of no row, one, and one less and more than the tiles of 32, 64 and 128 rows that the average count asks for."""
+  c, sd = _routed(gpu, num_experts_per_tok=1)
+  E = c.num_experts
+  rng = np.random.default_rng(sum(counts))
+  cls = rng.permutation(np.repeat(np.arange(E), counts))
+  prompt = [int(e + E * rng.integers(0, c.vocab_size // E)) for e in cls]
+  _rows_and_steps_agree(gpu, c, sd, prompt + [3])                                   # (what block 0's experts add is in the keys and values of block 1)
+  from tinygrad_amd.llm import Transformer
+  a = Transformer(dataclasses.replace(c, num_blocks=1), sd, max_new=8)
+  a.many_rows = True
+  a.prefill(prompt + [3])
+  n, up = len(prompt), lambda b: (b + 255) // 256 * 256
+  r = _regions(a, MOE, n)
+  at = sum(up(b.nbytes) for b in r.values()) + up(2 * n) + (64 << 20) + up(4 * n * E) + 3 * up(4 * n)        # (activations, partial sums, logits; selection, weights, places)
+  assert (a._chunker or a._tail_chunkers[16])._rows_ws.view(at, (E,), np.int32).numpy().tolist() == list(counts)
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_experts_of_every_format(gpu, fmt):
+  """Expert matrices of every format the rows linears take, at tiles of 32 and of 64 rows."""
+  c, sd = _routed(gpu, expert_type=getattr(gpu, fmt))
+  rng = np.random.default_rng(1)
+  for n in (70, 200): _rows_and_steps_agree(gpu, c, sd, rng.integers(0, c.vocab_size, size=n).tolist())
+
+@pytest.mark.parametrize("over", [dict(expert_gating_func=2), dict(expert_gating_func=3), dict(expert_gating_func=4), dict(norm_topk_prob=True), dict(expert_gating_func=2, norm_topk_prob=True, routed_scaling_factor=2.5),
+                                  dict(leading_dense_blocks=1, dense_hidden_dim=512, num_blocks=3), dict(head_dim=128, n_heads=2, n_kv_heads=2)],
+                         ids=["sigmoid", "softmax of the picked", "sqrt softplus", "normed", "sigmoid, normed, scaled", "dense block first", "heads of 128"])
+def test_routed_rows_of_other_kinds(gpu, over):
+  c, sd = _routed(gpu, **over)
+  _rows_and_steps_agree(gpu, c, sd, np.random.default_rng(2).integers(0, c.vocab_size, size=150).tolist())
+
+@pytest.mark.parametrize("cfg", [DENSE, DENSE128], ids=["hd64", "hd128"])
+def test_prefill_rows_with_norms_per_head(gpu, cfg):
+  """q / k norms over each head (their weights differ from value to value) against the model prefilled token by token."""
+  from tinygrad_amd.llm import Transformer, TransformerConfig, synth_state
+  c = TransformerConfig(max_context=256, qk_norm=cfg["head_dim"], **cfg)
+  sd, rng = synth_state(c, seed=29), np.random.default_rng(29)
+  for i in range(c.num_blocks):
+    for nm in ("q", "k"): sd[f"blk.{i}.attn_{nm}_norm.weight"] = (gpu.Buffer.from_numpy(rng.uniform(0.5, 2, c.head_dim).astype(np.float32)), gpu.F32, (1, c.head_dim))
+  prompt = rng.integers(0, c.vocab_size, size=140).tolist()
+  a, b = Transformer(c, sd, max_new=8), Transformer(c, sd, max_new=8)
+  b.prefill_chunk = 1
+  for m in (a, b): m.prefill(prompt)
+  assert a._chunker._rows_ws is not None
+  for ba, bb in zip(a.blk, b.blk):
+    for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): assert ol.rel_err(ca.numpy().astype(np.float32), cb.numpy().astype(np.float32)) <= 2e-3
+  for m in (a, b): m.decode_step(); m.check_state()
+  assert ol.rel_err(a.logits(), b.logits()) <= 2e-3
