@@ -129,3 +129,46 @@ def _moe_run(gpu, B):
 def test_config4_olmoe_mxfp4_32_tokens(gpu): _moe_run(gpu, 1)
 
 def test_config4_olmoe_mxfp4_32_tokens_eight_sequences(gpu): _moe_run(gpu, 8)
+
+def _prompt_errors(gpu, c, sd, oracle, prompt, many):
+  """Prefill and one decode step: per position the relative error (2-norm) of the last block's keys and values against the oracle's cache, and the logits' (largest)."""
+  from tinygrad_amd.llm import Transformer
+  m = Transformer(c, sd, max_new=8)
+  m.many_rows = many
+  m.prefill(prompt)
+  assert ((m._chunker or m._tail_chunkers[16])._rows_ws is not None) == many
+  n, i = len(prompt) - 1, c.num_blocks - 1
+  err = []
+  for got, ref in ((m.blk[i].cache_k, oracle.ck[i]), (m.blk[i].cache_v, oracle.cv[i])):
+    g, r = got.numpy()[:, :n].astype(np.float64), ref[:, :n].astype(np.float64)
+    err.append(np.sqrt(((g - r) ** 2).sum((0, 2)) / (r ** 2).sum((0, 2))))
+  m.decode_step(); m.check_state()
+  return np.maximum(*err), m.logits().reshape(-1).copy()
+
+@pytest.mark.parametrize("name,n", [("dense", 400), ("moe", 800)])
+def test_prompt_in_steps_of_many_rows(gpu, name, n):
+  """Two blocks of each architecture at its real widths, a prompt of several hundred tokens in one step of many rows (800 tokens of the MoE model: 100 rows per expert, tiles of 128), against the oracle.  The
+  second block's keys and values hold all that the first block computed; a position counts where the oracle's own expert choices are no near-ties (TIE: either choice is correct there).  Bars: the
+  rows are no further from the oracle than the steps of sixteen (MoE) or 128 (dense) rows by more than a tenth, on the mean over the positions, and within 1e-3 at each
+  (fp16 rounding of the cache row, 2.8e-4 of it in the 2-norm, and of the activations before it; see above for the MoE weights); logits as above where the last position is no near-tie either."""
+  from tinygrad_amd.llm import TransformerConfig, synth_state, synth_state_moe, LLAMA3_8B, OLMOE
+  cfg = dict(LLAMA3_8B if name == "dense" else OLMOE, num_blocks=2)
+  c = TransformerConfig(max_context=896, **cfg)
+  sd = (synth_state if name == "dense" else synth_state_moe)(c, seed=1003 + n)
+  gpu.synchronize()
+  prompt = np.random.default_rng(n).integers(0, c.vocab_size, size=n).tolist()
+  oracle, gaps = PackedModel(cfg, _host(sd), c.max_context, threads=min(16, cref.max_threads())), []
+  t0 = time.perf_counter()
+  for pos, t in enumerate(prompt):
+    oracle.min_route_gap = np.inf
+    lg = oracle.forward(t, pos)
+    gaps.append(oracle.min_route_gap)
+    if pos % 100 == 99: _say(f"{name}, {pos + 1} of {n} positions, {time.perf_counter() - t0:.0f} s")
+  clear = np.array(gaps) > (TIE if name == "moe" else 0)
+  rows, lr = _prompt_errors(gpu, c, sd, oracle, prompt, True)
+  steps, ls = _prompt_errors(gpu, c, sd, oracle, prompt, False)
+  ok = clear[:-1]
+  print(f"{name}, {n} tokens: {int(ok.sum())} of {n - 1} positions without a near-tie; keys and values against the oracle, mean / largest: rows {rows[ok].mean():.2e} / {rows[ok].max():.2e}, "
+        f"steps {steps[ok].mean():.2e} / {steps[ok].max():.2e}; logits {ol.rel_err(lr, lg):.2e} / {ol.rel_err(ls, lg):.2e}")
+  assert ok.mean() >= 0.5 and rows[ok].mean() <= 1.1 * steps[ok].mean() and rows[ok].max() <= 1e-3
+  if clear[-1]: assert ol.rel_err(lr, lg) <= (TOL_MOE if name == "moe" else TOL)
