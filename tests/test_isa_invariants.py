@@ -127,3 +127,56 @@ def test_wave_private_loop_keeps_its_ring_in_flight(kernels):
     assert not bad, (name, bad)
     checked += 1
   assert checked >= 4
+
+def _wide_loop(L):
+  """Instructions of a wide-tile kernel's loop over K, [(text, written by hand)]: the backward branch whose span holds sixteen requests into LDS."""
+  ins, by_hand, at = [], False, {}
+  for l in L:
+    t = l.strip()
+    m = re.match(r"(\.LBB\d+_\d+):", t)
+    if m: at[m.group(1)] = len(ins)
+    elif t.startswith(";;#ASMSTART"): by_hand = True
+    elif t.startswith(";;#ASMEND"): by_hand = False
+    elif t and not t.startswith((";", ".")):
+      ins.append((t.split(";")[0].strip(), by_hand))
+      m = re.match(r"s_cbranch\w+ (\.LBB\d+_\d+)$", ins[-1][0])
+      if m and m.group(1) in at and sum(" lds" in x for x, _ in ins[at[m.group(1)]:]) == 16: return ins[at[m.group(1)]:]
+  raise AssertionError("no loop with sixteen requests into LDS")
+
+def _wide_findings(ins):
+  """What would break or empty the loop's pipeline: spills, a wait of the compiler's that a request of this half has to land for, a half without its eight requests into LDS and its hand-written
+  wait for all of them in front of the barrier."""
+  bad, issued, into_lds, halves, waited = [], 0, 0, [], False
+  for t, by_hand in ins:
+    if t.startswith("scratch_"): bad.append(t)
+    elif t.startswith("buffer_load"): issued += 1; into_lds += " lds" in t; waited = False
+    elif t.startswith("s_waitcnt") and "vmcnt" in t:
+      n = int(re.search(r"vmcnt\((\d+)\)", t).group(1))
+      if by_hand: waited = n == 0 and "lgkmcnt(0)" in t; issued = 0 if n == 0 else issued
+      elif issued > n: bad.append(f"{t} behind {issued} requests")
+    elif t == "s_barrier":
+      if not (by_hand and waited): bad.append("a barrier without its wait")
+      halves.append(into_lds); into_lds = 0
+  if halves != [8, 8] or into_lds: bad.append(f"requests into LDS per half: {halves}, {into_lds} behind the last barrier")
+  return bad
+
+def test_wide_tiles_keep_their_requests_in_flight():
+  """qgemm_wide_kernel (csrc/qgemm_rows.h) fills one half of its LDS by requests that write it themselves while it reads the other, and waits for them by hand in front of each of its two barriers."""
+  try: hipcc = tb._hipcc()
+  except RuntimeError: pytest.skip("hipcc not found")
+  with tempfile.TemporaryDirectory() as d:
+    out = pathlib.Path(d) / "rows.s"
+    r = subprocess.run([hipcc, *tb.HIPCC_FLAGS, "--cuda-device-only", "-S", str(tb.CSRC / "qgemm_rows_a.hip"), "-o", str(out)], capture_output=True, text=True)
+    if r.returncode != 0: pytest.fail(f"hipcc -S failed:\n{r.stderr[-2000:]}")
+    text = out.read_text()
+  names = re.findall(r"^(_Z17qgemm_wide_kernelI\w+):", text, re.M)
+  assert len(names) == 2, names
+  for name in names:
+    ins = _wide_loop(text[text.index("\n" + name + ":"):text.index(".set " + name + ".uses_flat_scratch")].split("\n"))
+    assert sum(t.startswith("v_mfma") for t, _ in ins) == 256, name
+    assert not (bad := _wide_findings(ins)), (name, bad[:5])
+  good = ins
+  at = next(i for i, (t, _) in enumerate(good) if t == "s_barrier")
+  assert _wide_findings(good[:at - 1] + good[at:])                                  # (the wait gone)
+  assert _wide_findings(good[:at - 1] + [("s_waitcnt vmcnt(3)", False)] + good[at - 1:])
+  assert _wide_findings(good[:9] + [("scratch_load_dword v1, off, off", False)] + good[9:])
