@@ -123,7 +123,7 @@ def test_prefill_rows_of_every_norm_width(gpu, dim):
   for m in (a, b): m.decode_step()
   assert ol.rel_err(a.logits(), b.logits()) <= 2e-3
 
-@pytest.mark.parametrize("cfg,B,n", [(DENSE, 3, 7), (DENSE, 5, 70), (DENSE128, 2, 33), (MOE, 4, 20), (MOE, 1, 40)], ids=["dense-3x7", "dense-5x70", "hd128-2x33", "moe-4x20", "moe-1x40"])
+@pytest.mark.parametrize("cfg,B,n", [(DENSE, 3, 7), (DENSE, 9, 3), (DENSE, 5, 70), (DENSE128, 2, 33), (MOE, 4, 20), (MOE, 1, 40)], ids=["dense-3x7", "dense-9x3", "dense-5x70", "hd128-2x33", "moe-4x20", "moe-1x40"])
 @pytest.mark.parametrize("rows", [2048, 24])
 def test_batched_prefill_of_many_rows_vs_step_by_step(gpu, monkeypatch, cfg, B, n, rows):
   """The prompts of several sequences as steps of (sequences x positions) rows against the lockstep steps: every cache within 2e-3 except rows behind a router near-tie (MoE), whose share is

@@ -53,9 +53,10 @@ LLAMA3_8B = dict(num_blocks=32, dim=4096, hidden_dim=14336, n_heads=32, n_kv_hea
 OLMOE = dict(num_blocks=16, dim=2048, hidden_dim=1024, n_heads=16, n_kv_heads=16, norm_eps=1e-5, vocab_size=50304, head_dim=128,
              rope_theta=10000.0, qk_norm=2048, num_experts=64, num_experts_per_tok=8, norm_topk_prob=False, expert_gating_func=1)
 
-MANY_ROWS = 2048                   # rows of a prefill step at most (its buffers grow with the rows: 0.5 GB for the 8B architecture)
-MANY_ROWS_MIN = 17                 # fewer rows are one step of the small-batch kernels
-MANY_ROWS_POSITIONS = 4            # sequences in lockstep: fewer positions than that are so many steps, on the bits of the steps behind them
+MANY_ROWS = 2048                   # rows of a prefill step at most (its buffers grow with the rows: 277 MB for the 8B architecture)
+# Fewer rows are one step of the small-batch kernels.  Lockstep prompts, one step of many rows against so many lockstep steps (eight blocks of the 8B architecture, Q8_0 / Q4_0 / Q4_K_M): 16 sequences of two
+# positions 1079 against 1534 / 988 against 1336 / 1132 against 1619 us, 8 of three 1059 against 2038 / 956 against 1795 / 1129 against 2234, 4 of five 1018 against 3073 / 944 against 2655 / 1097 against 3349
+MANY_ROWS_MIN = 17
 
 def precompute_freqs_cis(dim: int, end: int, theta: float) -> np.ndarray:
   """tinygrad/llm/model.py:16-19 in float32: cat(cos(pos * f), sin(pos * f)), f = 1 / theta^(2i/dim)."""
@@ -907,7 +908,7 @@ class BatchedTransformer:
     pr = np.zeros((B, c.max_context), np.int32); pr[:, :n] = np.array(prompts, np.int32)
     self.prompts.copyin(pr)
     # all but the last position of every prompt: as steps of many rows (sequences x positions) where the model is in their range and there are rows enough, else step by step
-    many = self.many_rows and self._rows_tables is not None and on_block is None and B * (n - 1) >= MANY_ROWS_MIN and n - 1 >= MANY_ROWS_POSITIONS and self.expert_path == "jobs"     # (a chosen expert path runs every step)
+    many = self.many_rows and self._rows_tables is not None and on_block is None and B * (n - 1) >= MANY_ROWS_MIN and self.expert_path == "jobs"     # (a chosen expert path runs every step)
     done = n - 1 if many else 0
     self.tokens.copyin(np.ascontiguousarray(pr[:, done]))
     st = np.zeros(16, np.int32); st[0], st[3], st[5] = done, n, c.vocab_size
