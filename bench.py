@@ -214,7 +214,7 @@ def main():
     sys.exit(2)
 
   from tinygrad_amd import runtime as rt
-  from tinygrad_amd.llm import Transformer, TransformerConfig, synth_state, LLAMA3_8B
+  from tinygrad_amd.llm import Transformer, TransformerConfig, synth_state, LLAMA3_8B, MANY_ROWS
   rt.init(0)
   cfg = dict(LLAMA3_8B); cfg["num_blocks"] = args.layers
   max_new = args.steps + args.warmup + 16                    # + the parity step and the eager steps of the per-kernel timing below
@@ -331,8 +331,10 @@ def main():
                                "(profiles/decode_llama3_8b_q4_0_kernel_stats.md), neither re-measured by this run",
                      "share_of_block_time": round(dom["avg_us"] / per_block, 3),
                      "per_op_kernels": {k: v for k, v in kern.items() if k != "gate_up"}}
-  out["prefill"] = {"positions": args.prefill - 1, "ms": round(prefill_s * 1e3, 2), "positions_per_s": round((args.prefill - 1) / prefill_s, 1), "positions_per_step": int(model.prefill_chunk),
-                    "what": "the prompt prefilled once more before the timed decode steps (recorded steps replayed; one pass over the weights per step of positions_per_step rows), host wall clock; not part of `value`"}
+  many = (model._chunker or next(iter(model._tail_chunkers.values()), None)) if model.many_rows else None             # (steps of many rows where the model is in their range, else of prefill_chunk)
+  per_step = min(args.prefill - 1, MANY_ROWS) if many is not None and many._rows_ws is not None else int(model.prefill_chunk)
+  out["prefill"] = {"positions": args.prefill - 1, "ms": round(prefill_s * 1e3, 2), "positions_per_s": round((args.prefill - 1) / prefill_s, 1), "positions_per_step": per_step,
+                    "what": "the prompt prefilled once more before the timed decode steps (one pass over the weights per step of positions_per_step rows), host wall clock; not part of `value`"}
   if parity is not None: out["parity"] = parity
   if not args.no_cpu:
     from oracle import cref

@@ -39,8 +39,8 @@ extern "C" {
 const char* tga_last_error(void);
 int tga_init(int device);                                  /* hipSetDevice + kernel attribute set-up; ops_hip.py:14-20.  Also allocates, once per device, the 160 MB workspace of the 17 .. 128 row linears */
 int tga_device_name(char* buf, size_t len);
-int tga_malloc(void** ptr, size_t nbytes);                 /* ops_hip.py:60-62; served from freed blocks of the same size class where one is kept; refused while the thread captures */
-int tga_free(void* ptr);                                   /* ops_hip.py:63; keeps the block for later requests (at most 4 GiB per device, blocks of at most 1 GiB): it is handed out again only after the device has been synchronised */
+int tga_malloc(void** ptr, size_t nbytes);                 /* ops_hip.py:60-62; served from freed blocks of the same size class where one is kept; refused while the thread captures a stream, whoever opened the capture (as hipMalloc is) */
+int tga_free(void* ptr);                                   /* ops_hip.py:63; keeps the block for later requests (at most 4 GiB per device, blocks of at most 1 GiB): it is handed out again only after a wait for the device; a block freed before is an error */
 int tga_trim(void);                                        /* gives every kept block back to the driver; refused while the thread captures */
 int tga_memcpy_h2d(void* dst, const void* src, size_t n);  /* ops_hip.py:64-66, synchronous */
 int tga_memcpy_d2h(void* dst, const void* src, size_t n);  /* ops_hip.py:67-69, synchronous */

@@ -8,7 +8,7 @@
 // add_expert_bias -> swiglu -> quantize_mxfp8 -> grouped_mx_gemm -> add_expert_bias -> combine: every rounding to bf16 and to E4M3 sits where it sits there.  What
 // is gone are the passes between them (T = 4096, k = 8, E = 128, D = 2048, I = 768: dispatch, two quantisations, two bias adds, SwiGLU over 65536 padded rows) and the
 // padding of every expert's rows to 256, and the host work of eleven entry points.  MI355X, back to back: T = 2000, k = 8, E = 64, D = 2048, I = 512 2480 (single passes:
-// 810) -> 182 us; T = 32, k = 8, E = 64, I = 768 840 (single) -> 79 us; the benchmark's T = 4096, E = 128, I = 768 1340 (single) -> 406 us.
+// 810) -> 186 us; T = 32, k = 8, E = 64, I = 768 840 (single) -> 81 us; the benchmark's T = 4096, E = 128, I = 768 1340 (single) -> 406 us.
 #include "mxfp8.h"
 #include "host.h"
 
@@ -438,6 +438,10 @@ int tga_moe_feed_forward(const void* x_bf16, const float* logits, int64_t T, int
   else moe_prep_kernel<FFN_MAX_E / 64><<<pg, 1024, 0, s>>>(a);
   TGA_LAUNCH_CHECK();
   static const int n_cu = [] { int dev = 0, n = 0; return (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) ? n : 256; }();
+  // Tiles of 32 or 256 rows by the rows per expert, us of the call (32 / 256): 64 experts, D 2048, I 512, even popularity: 16 rows 61.5 / 65.8, 24 71.3 / 67.1, 40 71.7 / 70.1, 48 90.0 / 72.3, 128 125 / 93,
+  // 200 181 / 114; popularity by 1 / rank^1.1: 16 67.5 / 74.6, 48 73.2 / 110, 64 91.7 / 132, 128 126 / 150, 200 185 / 167.  128 experts, I 768: even 32 189 / 182, 48 221 / 192, 128 349 / 231; skewed 32
+  // 191 / 219, 48 229 / 235, 64 238 / 242, 96 304 / 271.  16 experts, D 1536, I 768: 48 45.0 / 50.7, 128 53.2 / 64.9, 200 71.6 / 77.5 even, 46.0 / 68.0, 52.5 / 75.7, 72.1 / 78.5 skewed.  At 48 the even
+  // popularity gains; where it is skewed, or the experts are few, 32 rows stay better up to 128 and more, but the host does not know the counts.
   const bool small = T * k < 48ll * n_experts;
   if (small) {
     ffn_gemm_kernel<32, 1, true><<<2 * n_cu, 256, 0, s>>>(a); TGA_LAUNCH_CHECK();

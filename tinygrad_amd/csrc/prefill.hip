@@ -2,8 +2,8 @@
 // tinygrad/llm/model.py:464, 476-481, with the prompt as one chunk), every linear as ONE pass over its weights (qgemm_rows.h).  Per block: q / k / v -> rotation +
 // append -> attention -> attn_output (+ residual, norm) -> gate / up + SwiGLU -> down (+ residual, the next block's norm): eight launches and the sums of a split q / k / v, or for a MoE block norm -> router logits -> gating ->
 // grouping -> selected experts' gate / up + SwiGLU -> down -> weighted sum (+ residual), model.py:110-135.  The launches are issued by one native call.
-// MI355X, prompt to first logits: 8B-arch Q4_0 of 1024 tokens 42.4 ms (steps of 128 rows, qgemm64.hip) -> 21.2; OLMoE-arch of 512 tokens 64.0 (steps of 16 rows, an expert GEMV per
-// token and slot) -> 5.0; four 8B-arch Q4_K_M sequences of 128 tokens 333 (one lockstep step per position) -> 15.5.
+// MI355X, prompt to first logits: 8B-arch Q4_0 of 1024 tokens 42.4 ms (steps of 128 rows, qgemm64.hip) -> 21.2; OLMoE-arch of 512 tokens, where its user asks for it, 64.0 (steps of 16 rows, an
+// expert GEMV per token and slot) -> 5.0; four 8B-arch Q4_K_M sequences of 128 tokens 333 (one lockstep step per position) -> 15.5.
 #include "qgemm_rows.h"
 #include "decode.h"
 #include "moe_gate.h"
@@ -396,6 +396,10 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
     { const void* wr[1] = {(const void*)b[PB_ROUTER]}; void* yr[1] = {logits}; const int64_t nr[1] = {E}; PF_DO(linear(TGA_F16, 1, wr, yr, nr, xn, TGA_F32, dim, 0, nullptr)); }
     rows_gate_kernel<<<(unsigned)((R + 3) / 4), 256, 0, s>>>(logits, (int)R, (int)E, (int)k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), sel, (float*)(ws + w.probs), counts, place);
     TGA_LAUNCH_CHECK();
+    // Rows of an expert's tile, us a block with 32 / 64 / 128 (D 2048, H 1024, 64 experts, top 8 | H 1024, 16, top 8 | H 1536, 32, top 8): 24 rows per expert 189 / 185 / 226 | 107 / 112 / 125 | 159 / 152 / 186,
+    // 32: 213 / 196 / 236 | 119 / 114 / 127 | 174 / 157 / 191, 80: 319 / 307 / 285 | 142 / 140 / 140 | 245 / 236 / 218, 104: 373 / 338 / 344 | 162 / 146 / 147 | 279 / 243 / 231, 160: 496 / 447 / 474 | 194 / 174 / 183 |
+    // 350 / 314 / 332, 255: 712 / 632 / 630 | 243 / 222 / 232 | 484 / 426 / 427, 510: - | 377 / 338 / 337 | 860 / 738 / 712, 1000: - | 660 / 578 / 561; D 1024, H 512, 8 experts, top 4: 128 rows
+    // 8 .. 14 % slower from 104 to 160, alike from 255 on.  At either line the sides are about a tenth apart, one way or the other.
     const int64_t avg = R * k / E;
     const int tt = avg <= 32 ? 32 : avg <= 96 ? 64 : 128;
     const int64_t max_tiles = R * k / tt + (R * k < E ? R * k : E);

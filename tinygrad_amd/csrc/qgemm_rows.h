@@ -318,7 +318,8 @@ __global__ __launch_bounds__(256, 2) void qgemm_rows_kernel(const RowsArgs a) {
 // holds the weights of row 16 i + r16 at K position group g of the products, half a unit of 64 at a time, so no weight passes through LDS and none is decoded twice.
 // Only the activations are shared: two halves of 128 rows x 128 values, filled by requests that write LDS themselves, one barrier per half step (128 products of a wave); they are read
 // as 16-byte pieces in the order in which the weights fall out of their blocks (elem).  Twice the results per byte read from LDS, half of its writes.
-// 254 registers at two waves per SIMD are what bounds the formats: Q8_0 and Q4_K, whose half units take twice the registers, were built the same way and were no faster than above.
+// 254 registers at two waves per SIMD are what bounds the formats: Q8_0 and Q4_K, whose half units take twice the registers, were built the same way and were no faster than above (the loop
+// of Q4_K spilled; the plain Q4_0 variant keeps five registers in scratch from before its loop to behind it, none inside).
 // 1023 rows x 4096 -> 2 x 14336 (gate / up) 301 -> 268 us, x 14336 -> 4096 (down) 158 -> 145 us, 2047 rows 603 -> 505 us and 304 -> 271 us.
 #define WIDE_WT 256
 #define WIDE_TT 128

@@ -141,7 +141,8 @@ static int rows_plan(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t p
   // A product of few 128 x 128 x 128 steps takes tiles of fewer rows: more workgroups, each done sooner.  us with 128 / 64 / 32 rows a tile: 16 steps (Q4_0 512 -> 512, 100 rows) 11.4 / 7.9 / 7.0,
   // 224 (Q8_0 3584 -> 1024, 100) 15.9 / 12.6 / 11.4, 512 (fp16 2048 -> 2048, 200) 17.3 / 14.5 / 14.6, 1536 (Q4_0 4096 -> 6144, 100) 25.9 / 23.9 / 27.3, 1792 (Q8_0 3584 -> 1024, 1000) 27.6 / 23.9 / 27.0,
   // 3072 (Q4_0 4096 -> 6144, 200) 31.0 / 33.7 / 40.4, 3584 (Q4_K 14336 -> 4096, 100) 36.2 / 38.9 / 54.1; fp16, which decodes nothing: 3072 (2048 -> 6144, 511) 34.7 / 30.7 / 30.2, 6144 (1000) 46.4 / 40.8 / 54.7;
-  // Q6_K, whose decode is the longest: 1024 (4096 -> 1024, 508) 18.2 / 19.2.
+  // Q6_K, whose decode is the longest, 64 / 128 rows a tile: 768 steps 21.4 / 20.8 and 21.9 / 21.5, 1024 (five products, K 2048 .. 8192) 23.9 / 23.8, 22.1 / 22.1, 24.5 / 23.7, 24.2 / 22.9, 21.4 / 21.0,
+  // 1152 (3072 -> 3072, 200) 25.2 / 28.0, 1536 30.9 / 28.3, 28.4 / 28.0, 26.9 / 28.3, 2048 31.6 / 30.0, 31.3 / 28.9, 4096 50.7 / 41.5: alike up to 1536 steps, 128 rows from there on.
   const long long steps = (long long)a.row_tiles * ((a.M + 127) / 128) * (a.K / ROWS_KS);
   const int tt = a.M <= 32 || steps < 512 ? 32 : a.M <= 64 || steps <= (fmt == GGML_F16 ? 6144 : fmt == GGML_Q6_K ? 1023 : 2048) ? 64 : 128;
   a.tok_tiles = (a.M + tt - 1) / tt;

@@ -159,7 +159,7 @@ def moe_feed_forward(inp: Buffer, logits: Buffer, experts_per_tok: int, w_gate_u
     ws, out = Buffer((need.value,), np.uint8), Buffer((T, D), np.uint16)
     rt.check(rt.lib().tga_moe_feed_forward(inp.ptr, logits.ptr, T, D, N2 // 2, E, experts_per_tok, w_gate_up[0].ptr, w_gate_up[1].ptr, b_gate_up.ptr, w_down[0].ptr, w_down[1].ptr,
                                            b_down.ptr, swiglu_limit, ws.ptr, out.ptr, stream))
-    return out                                                  # (ws: a freed block is handed out again only after the device has been synchronised)
+    return out                                                  # (ws: a freed block is handed out again only after a wait for the device)
   r = route(logits, experts_per_tok, E, stream)
   xg = dispatch(inp, r, stream)
   cnt = r.counts if routed_only else None                     # padding rows are never gathered by combine: their 16-row groups are not multiplied
