@@ -326,3 +326,21 @@ def test_prefill_rows_with_norms_per_head(gpu, cfg):
     for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): assert ol.rel_err(ca.numpy().astype(np.float32), cb.numpy().astype(np.float32)) <= 2e-3
   for m in (a, b): m.decode_step(); m.check_state()
   assert ol.rel_err(a.logits(), b.logits()) <= 2e-3
+
+def test_prompts_without_memory_for_their_rows_take_the_smaller_steps(gpu, monkeypatch):
+  """No memory for the buffers of a step of many rows (277 MB at the 8B architecture's widths): the prompt is prefilled in the steps that need a few MB, for one sequence and for several."""
+  from tinygrad_amd import llm
+  prompt = np.random.default_rng(4).integers(0, DENSE["vocab_size"], size=150).tolist()
+  a, b, several, several_b = _model(DENSE, 31), _model(DENSE, 31), _model(DENSE, 31, 160, 4), _model(DENSE, 31, 160, 4)
+  b.many_rows = several_b.many_rows = False
+  b.prefill(prompt); several_b.prefill([prompt[:40]] * 4)
+  buffer = llm.Buffer
+  def none_left(shape, dtype=np.uint8, **kw):
+    if int(np.prod(shape)) * np.dtype(dtype).itemsize >= 60 << 20: raise RuntimeError("HIP Error 2, out of memory  [hipMalloc(ptr, cls) at pool.h:1]")
+    return buffer(shape, dtype, **kw)
+  none_left.from_numpy = buffer.from_numpy
+  monkeypatch.setattr(llm, "Buffer", none_left)
+  a.prefill(prompt); several.prefill([prompt[:40]] * 4)
+  assert a._chunker._rows_ws is None and a._chunker.x is not None and several._rows_ws is None
+  for ba, bb in zip(a.blk, b.blk): np.testing.assert_array_equal(ba.cache_k.numpy(), bb.cache_k.numpy())
+  for ba, bb in zip(several.blk, several_b.blk): np.testing.assert_array_equal(ba["cache_k"].numpy(), bb["cache_k"].numpy())

@@ -712,15 +712,23 @@ class BatchedTransformer:
              int(c.norm_topk_prob), c.qk_norm, c.hidden_dim, c.dense_hidden_dim, bits(c.norm_eps), bits(c.routed_scaling_factor)]
     return (ctypes.c_int64 * len(model))(*model), (ctypes.c_int64 * (len(rows) * len(rows[0])))(*sum(rows, []))
 
+  def _rows_reserve(self, nseq: int, n: int) -> bool:
+    """The buffers of steps of many rows for n positions of nseq sequences; False where the device has no memory left for them (smaller steps need a few MB)."""
+    need = ctypes.c_int64(0)
+    rt.check(rt.lib().tga_prefill_plan(self._rows_tables[0], nseq * min(n, max(1, MANY_ROWS // nseq)), ctypes.byref(need)))
+    try:
+      if self._rows_ws is None or self._rows_ws.nbytes < need.value: self._rows_ws = Buffer((need.value,), np.uint8)
+      if self._rows_tok is None or self._rows_tok.nbytes < 4 * nseq * n: self._rows_tok = Buffer((4 * nseq * n,), np.uint8)
+    except RuntimeError as e:
+      if "HIP Error 2," not in str(e): raise
+      return False
+    return True
+
   def _prefill_many_rows(self, ids: np.ndarray, pos0: int):
-    """Positions pos0 .. pos0 + n - 1 of every sequence of ids (sequences, n) in steps of at most MANY_ROWS rows, each one native call."""
+    """Positions pos0 .. pos0 + n - 1 of every sequence of ids (sequences, n) in steps of at most MANY_ROWS rows, each one native call (behind _rows_reserve)."""
     nseq, n = ids.shape
     per = max(1, MANY_ROWS // nseq)
     steps = [(i, min(per, n - i)) for i in range(0, n, per)]
-    need = ctypes.c_int64(0)
-    rt.check(rt.lib().tga_prefill_plan(self._rows_tables[0], nseq * steps[0][1], ctypes.byref(need)))
-    if self._rows_ws is None or self._rows_ws.nbytes < need.value: self._rows_ws = Buffer((need.value,), np.uint8)
-    if self._rows_tok is None or self._rows_tok.nbytes < ids.nbytes: self._rows_tok = Buffer((ids.nbytes,), np.uint8)
     flat = np.concatenate([ids[:, i:i + m].reshape(-1) for i, m in steps]).astype(np.int32)
     self._rows_tok.view(0, flat.shape, np.int32).copyin(flat)
     at = 0
@@ -729,11 +737,13 @@ class BatchedTransformer:
       at += nseq * m
 
   def prefill_rows(self, tokens: list[int], start: int, n: int) -> int:
-    """Chunked prefill for `chunk_of` in steps of many rows: the positions start .. start + n - 1 of the prompt into its KV caches.  Returns the number of positions done."""
+    """Chunked prefill for `chunk_of` in steps of many rows: the positions start .. start + n - 1 of the prompt into its KV caches.  Returns the number of positions done
+    (none where there is no memory for the step's buffers)."""
     c = self.config
     if not self.chunked or self._rows_tables is None: raise RuntimeError("prefill_rows needs a model built with chunk_of and linears in the range of tga_prefill_step")
     if not (0 <= start and n >= 1 and start + n <= len(tokens) < c.max_context): raise ValueError(f"positions {start}+{n} outside the prompt of {len(tokens)} tokens")
     if min(tokens) < 0 or max(tokens) >= c.vocab_size: raise ValueError(f"token id outside the vocabulary of {c.vocab_size}")
+    if not self._rows_reserve(1, n): return 0
     st = np.zeros(16, np.int32); st[0], st[3], st[5] = start, len(tokens), c.vocab_size
     self.state.copyin(st)
     self._owner_stream.synchronize()
@@ -909,6 +919,7 @@ class BatchedTransformer:
     self.prompts.copyin(pr)
     # all but the last position of every prompt: as steps of many rows (sequences x positions) where the model is in their range and there are rows enough, else step by step
     many = self.many_rows and self._rows_tables is not None and on_block is None and B * (n - 1) >= MANY_ROWS_MIN and self.expert_path == "jobs"     # (a chosen expert path runs every step)
+    many = many and self._rows_reserve(B, n - 1)
     done = n - 1 if many else 0
     self.tokens.copyin(np.ascontiguousarray(pr[:, done]))
     st = np.zeros(16, np.int32); st[0], st[3], st[5] = done, n, c.vocab_size
