@@ -149,9 +149,9 @@ def moe_feed_forward(inp: Buffer, logits: Buffer, experts_per_tok: int, w_gate_u
   E2, N, I = w_down[0].shape
   assert logits.shape == (T, E), f"logits {logits.shape} for {T} tokens and {E} experts"
   assert (K, E2, I) == (D, E, N2 // 2), f"shape mismatch {(T, D)} {w_gate_up[0].shape} {w_down[0].shape}"
-  for name, b, nb in (("inp", inp, T * D * 2), ("logits", logits, T * E * 4), ("w_gate_up", w_gate_up[0], E * N2 * D), ("w_gate_up scales", w_gate_up[1], E * N2 * D // 32),
-                      ("b_gate_up", b_gate_up, E * N2 * 4), ("w_down", w_down[0], E * N * I), ("w_down scales", w_down[1], E * N * I // 32), ("b_down", b_down, E * N * 4)):
-    assert b.nbytes >= nb, f"{name}: {b.nbytes} bytes where the sizes ask for {nb}"
+  sizes = (T * D * 2, T * E * 4, E * N2 * D, E * N2 * D // 32, E * N2 * 4, E * N * I, E * N * I // 32, E * N * 4)
+  held = (inp.nbytes, logits.nbytes, w_gate_up[0].nbytes, w_gate_up[1].nbytes, b_gate_up.nbytes, w_down[0].nbytes, w_down[1].nbytes, b_down.nbytes)
+  assert all(map(int.__le__, sizes, held)), f"operands of {held} bytes where the sizes ask for {sizes}"
   need = ctypes.c_int64(0)
   rt.check(rt.lib().tga_moe_feed_forward_plan(T, D, N2 // 2, E, experts_per_tok, ctypes.byref(need)))
   ptrs = [b.ptr for b in (inp, *w_gate_up, b_gate_up, *w_down, b_down)]
