@@ -135,12 +135,14 @@ static void full_of_other_blocks() {
     std::vector<void*> b(12); for (auto& q : b) CHECK(!pool_malloc(&q, n)); for (auto& q : b) CHECK(!pool_free(q));
   }
   CHECK(g_pools[0].kept <= POOL_BYTES && g_pools[0].kept > POOL_BYTES - 2 * ((size_t)320 << 20));
-  int mallocs = 0;
-  for (int i = 0; i < 400; i++) {
-    if (i == 200) mallocs = g_mallocs;
-    void *a, *b; CHECK(!pool_malloc(&a, 2 << 20)); CHECK(!pool_malloc(&b, 128 << 10)); CHECK(!pool_free(a)); CHECK(!pool_free(b));
+  for (size_t n : {(size_t)2 << 20, (size_t)90 << 20}) {                   // small blocks, then some that keep more bytes than any other class in the end
+    int mallocs = 0;
+    for (int i = 0; i < 400; i++) {
+      if (i == 200) mallocs = g_mallocs;
+      void *a, *b; CHECK(!pool_malloc(&a, n)); CHECK(!pool_malloc(&b, n / 16)); CHECK(!pool_free(a)); CHECK(!pool_free(b));
+    }
+    CHECK(g_mallocs - mallocs <= 2 * 200 / POOL_DIRTY_COUNT);               // (the few bytes of each wait)
   }
-  CHECK(g_mallocs - mallocs <= 2 * 200 / POOL_DIRTY_COUNT);                 // (the few bytes of each wait)
   CHECK(g_pools[0].kept <= POOL_BYTES);
 }
 

@@ -13,8 +13,8 @@
 //    after the wait for the device that an hipFree performs - but one for many blocks: when a request finds no clean block of its class while POOL_DIRTY_COUNT
 //    blocks of the class (more at each further wait) or POOL_DIRTY_BYTES in all are dirty.  No stream has to be named, no caller synchronises more than it did.  The wait is that of an hipFree of a few bytes allocated
 //    for it (1.4 us where the device is idle): an hipDeviceSynchronize is refused during a capture of any thread and ends that capture, an hipFree only during one of its own (measured).
-//  * at most POOL_BYTES per device are kept; beyond, blocks of the class that keeps the most bytes go back to the driver (of what large results of an earlier phase left behind, say,
-//    not the block at hand: 20 us a call of moe_feed_forward at 32 tokens), all of them do before a request is refused for want of memory, and on tga_trim().
+//  * at most POOL_BYTES per device are kept; beyond, blocks of the class used least recently go back to the driver (what an earlier phase left behind, not the block at hand nor
+//    one of the classes in use: 20 and 180 us a call of moe_feed_forward at 32 and 2000 tokens), all of them do before a request is refused for want of memory, and on tga_trim().
 //  * size classes are eighths of a power of two (at most 11.1 % of a block is idle).  One mutex.  While its thread captures a stream, tga_free puts any block aside without a call to the runtime (an hipFree would
 //    invalidate the capture); one of more than POOL_BLOCK_MAX bytes is freed with the next call of that thread outside a capture.  tga_trim is refused then.
 //  * a thread with a capture of its own open gets no block: the replays would go on using one that its call gave back when it returned (and hipMalloc itself refuses then).  Captures that
@@ -23,10 +23,10 @@
 #define POOL_BYTES ((size_t)4 << 30)
 #define POOL_DIRTY_BYTES ((size_t)2 << 30)
 #define POOL_DIRTY_COUNT 8                   // of a class at its first wait, twice as many at further ones
-#define POOL_DIRTY_COUNT_MAX 16              // (31 us behind running kernels, where a device synchronisation costs 13)
+#define POOL_DIRTY_COUNT_MAX 32              // (31 us behind running kernels, where a device synchronisation costs 13)
 
-struct PoolClass { std::vector<void*> clean, dirty; size_t due = POOL_DIRTY_COUNT; };
-struct Pool { std::map<size_t, PoolClass> classes; size_t kept = 0, dirty = 0; };
+struct PoolClass { std::vector<void*> clean, dirty; size_t due = POOL_DIRTY_COUNT, used = 0; };   // due: dirty blocks at the next wait; used: when one was last taken or put aside
+struct Pool { std::map<size_t, PoolClass> classes; size_t kept = 0, dirty = 0, clock = 0; };
 static std::mutex g_pool_mutex;
 static std::unordered_map<int, Pool> g_pools;                                        // by device
 struct PoolBlock { size_t cls; int dev; bool out; };                                  // size class, device, handed out (or kept)
@@ -60,14 +60,14 @@ static int pool_release(Pool& p) {                                              
   p.classes.clear();
   return 0;
 }
-static int pool_make_room(Pool& p, size_t n) {                                        // blocks of the class that keeps the most bytes go back until n more may be kept
+static int pool_make_room(Pool& p, size_t n) {                                        // blocks of the class that was used least recently go back until n more may be kept
   while (p.kept && p.kept + n > POOL_BYTES) {
-    std::pair<const size_t, PoolClass>* most = nullptr;
-    for (auto& c : p.classes) if (!most || c.first * (c.second.clean.size() + c.second.dirty.size()) > most->first * (most->second.clean.size() + most->second.dirty.size())) most = &c;
-    std::vector<void*>& v = most->second.clean.empty() ? most->second.dirty : most->second.clean;
+    std::pair<const size_t, PoolClass>* idle = nullptr;
+    for (auto& c : p.classes) if (c.second.clean.size() + c.second.dirty.size() && (!idle || c.second.used < idle->second.used)) idle = &c;
+    std::vector<void*>& v = idle->second.clean.empty() ? idle->second.dirty : idle->second.clean;
     void* q = v.back();
-    if (&v == &most->second.dirty) p.dirty -= most->first;
-    v.pop_back(); g_pool_blocks.erase(q); p.kept -= most->first;
+    if (&v == &idle->second.dirty) p.dirty -= idle->first;
+    v.pop_back(); g_pool_blocks.erase(q); p.kept -= idle->first;
     TGA_HIP(hipFree(q));
   }
   return 0;
@@ -96,6 +96,7 @@ static int pool_malloc_(void** ptr, size_t n) {
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   Pool& p = g_pools[dev];
   PoolClass& c = p.classes[cls];
+  c.used = ++p.clock;
   if (c.clean.empty() && !c.dirty.empty() && (c.dirty.size() >= c.due || p.dirty >= POOL_DIRTY_BYTES)) {
     if (const int rc = pool_settle(p)) return rc;
     if (c.due < POOL_DIRTY_COUNT_MAX) c.due *= 2;
@@ -124,7 +125,9 @@ static int pool_free_(void* ptr) {
   const size_t cls = it->second.cls;
   Pool& p = g_pools[it->second.dev];
   if (!t_captures && p.kept + cls > POOL_BYTES) { if (const int rc = pool_make_room(p, cls)) return rc; }
-  p.classes[cls].dirty.push_back(ptr);
+  PoolClass& c = p.classes[cls];
+  c.dirty.push_back(ptr);
+  c.used = ++p.clock;
   p.kept += cls; p.dirty += cls; it->second.out = false;
   return 0;
 }
