@@ -41,7 +41,7 @@ int tga_init(int device);                                  /* hipSetDevice + ker
 int tga_device_name(char* buf, size_t len);
 int tga_malloc(void** ptr, size_t nbytes);                 /* ops_hip.py:60-62; served from freed blocks of the same size class where one is kept; refused while the thread captures a stream, whoever opened the capture (as hipMalloc is) */
 int tga_free(void* ptr);                                   /* ops_hip.py:63; keeps the block for later requests (at most 4 GiB per device, blocks of at most 1 GiB): it is handed out again only after a wait for the device; a block freed before is an error */
-int tga_trim(void);                                        /* gives every kept block back to the driver; refused while the thread captures */
+int tga_trim(void);                                        /* gives every kept block back to the runtime; refused while the thread captures */
 int tga_memcpy_h2d(void* dst, const void* src, size_t n);  /* ops_hip.py:64-66, synchronous */
 int tga_memcpy_d2h(void* dst, const void* src, size_t n);  /* ops_hip.py:67-69, synchronous */
 int tga_memcpy_d2d(void* dst, const void* src, size_t n, void* stream);

@@ -13,7 +13,7 @@
 //    after the wait for the device that an hipFree performs - but one for many blocks: when a request finds no clean block of its class while POOL_DIRTY_COUNT
 //    blocks of the class (more at each further wait) or POOL_DIRTY_BYTES in all are dirty.  No stream has to be named, no caller synchronises more than it did.  The wait is that of an hipFree of a few bytes allocated
 //    for it (1.4 us where the device is idle): an hipDeviceSynchronize is refused during a capture of any thread and ends that capture, an hipFree only during one of its own (measured).
-//  * at most POOL_BYTES per device are kept; beyond, blocks of the class used least recently go back to the driver (what an earlier phase left behind, not the block at hand nor
+//  * at most POOL_BYTES per device are kept; beyond, blocks of the class used least recently go back to the runtime (what an earlier phase left behind, not the block at hand nor
 //    one of the classes in use: 20 and 180 us a call of moe_feed_forward at 32 and 2000 tokens), all of them do before a request is refused for want of memory, and on tga_trim().
 //  * size classes are eighths of a power of two (at most 11.1 % of a block is idle).  One mutex.  While its thread captures a stream, tga_free puts any block aside without a call to the runtime (an hipFree would
 //    invalidate the capture); one of more than POOL_BLOCK_MAX bytes is freed with the next call of that thread outside a capture.  tga_trim is refused then.
@@ -46,7 +46,7 @@ static int pool_settle(Pool& p) {                                               
   p.dirty = 0;
   return 0;
 }
-static int pool_release(Pool& p) {                                                    // everything kept goes back to the driver (hipFree waits for the block's users)
+static int pool_release(Pool& p) {                                                    // everything kept goes back to the runtime (hipFree waits for the block's users)
   for (auto& c : p.classes) {
     for (auto* v : {&c.second.clean, &c.second.dirty}) {
       while (!v->empty()) {                                                           // (out of the lists first: where an hipFree fails, no block that is gone may stay in them)
