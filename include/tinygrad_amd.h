@@ -408,6 +408,10 @@ int tga_rows_format_ok(int ggml_type, int64_t K, int* ok);
  * _plan: bytes of the caller's workspace for that many rows (nseq * P). */
 int tga_prefill_plan(const int64_t* model, int64_t rows, int64_t* nbytes);
 int tga_prefill_step(const int64_t* model, const int64_t* blocks, const int32_t* tokens, int64_t nseq, int64_t P, int64_t pos0, void* workspace, void* state, void* stream);
+/* The same for one sequence of an MoE model with every sum in the order of steps of sixteen rows - the last `tail` rows: of eight and four - whose bits its keys and values have (prefill16.hip, which
+ * says which models it takes).  _plan: *ok, and bytes of the caller's workspace for `rows` rows that end in front of position `end`. */
+int tga_prefill16_plan(const int64_t* model, const int64_t* blocks, int64_t rows, int64_t end, int* ok, int64_t* nbytes);
+int tga_prefill16_step(const int64_t* model, const int64_t* blocks, const int32_t* tokens, int64_t P, int64_t tail, int64_t pos0, void* workspace, void* state, void* stream);
 
 #ifdef __cplusplus
 }

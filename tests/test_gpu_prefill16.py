@@ -1,0 +1,41 @@
+"""Prompts of MoE models in steps of many rows whose sums run in the order of the steps of sixteen, eight and four rows (csrc/prefill16.hip): caches and logits have those steps' bits."""
+import numpy as np, pytest
+
+pytestmark = pytest.mark.gpu
+BASE = dict(norm_eps=1e-5, vocab_size=512, rope_theta=10000.0)
+# the rows of the dense linears dealt to eight waves (2048, 1024) and to four (1536: two rounds; 512: waves without a step), experts of 64, 48, 32, 24 and 8 units, heads of 64 and 128, query groups
+CONFIGS = {
+  "2048x1024": dict(num_blocks=3, dim=2048, hidden_dim=1024, n_heads=16, n_kv_heads=16, head_dim=128, qk_norm=2048, num_experts=64, num_experts_per_tok=8, **BASE),
+  "1536x768": dict(num_blocks=2, dim=1536, hidden_dim=768, n_heads=12, n_kv_heads=12, head_dim=128, qk_norm=1536, num_experts=16, num_experts_per_tok=4, norm_topk_prob=True, **BASE),
+  "1024x1536": dict(num_blocks=2, dim=1024, hidden_dim=1536, n_heads=16, n_kv_heads=4, head_dim=64, qk_norm=1024, num_experts=32, num_experts_per_tok=2, expert_gating_func=2, **BASE),
+  "512x256": dict(num_blocks=3, dim=512, hidden_dim=256, n_heads=8, n_kv_heads=8, head_dim=64, qk_norm=512, num_experts=8, num_experts_per_tok=1, **BASE),
+}
+
+def _models(cfg, seed, ctx):
+  from tinygrad_amd.llm import Transformer, TransformerConfig, synth_state_moe
+  c = TransformerConfig(max_context=ctx, **cfg)
+  sd = synth_state_moe(c, seed=seed)
+  return Transformer(c, sd, max_new=8), Transformer(c, sd, max_new=8)
+
+@pytest.mark.parametrize("name", list(CONFIGS))
+@pytest.mark.parametrize("n,rows", [(17, 1024), (30, 1024), (78, 32), (134, 1024), (333, 128)])
+def test_bits_of_the_steps_of_sixteen_rows(gpu, monkeypatch, name, n, rows):
+  """Positions 16, 28 (16 + 8 + 4), 76, 132 and 332 in one step and in several: every key and value of every block, the logits behind them, and a follow-up prompt that keeps a prefix."""
+  from tinygrad_amd import llm
+  cfg = CONFIGS[name]
+  a, b = _models(cfg, 11 + n, 384)
+  prompt = np.random.default_rng(n).integers(0, cfg["vocab_size"], size=n).tolist()
+  for p in (prompt, prompt[:n // 2] + [7] * 40):
+    monkeypatch.setattr(llm, "ROWS16", rows); monkeypatch.setattr(llm, "ROWS16_MIN", 1)
+    a.prefill(p)
+    assert a._chunker._rows_ws is not None and a._chunker.x is None        # (no step of sixteen was run)
+    monkeypatch.setattr(llm, "ROWS16_MIN", 1 << 30)
+    b.prefill(p)
+    assert b._chunker is None or b._chunker._rows_ws is None
+    for i, (ba, bb) in enumerate(zip(a.blk, b.blk)):
+      for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)):
+        diff = int((ca.numpy().view(np.uint16) != cb.numpy().view(np.uint16)).sum())
+        assert diff == 0, f"block {i}"
+    for m in (a, b): m.decode_step(); m.check_state()
+    diff = int((a.logits().view(np.uint32) != b.logits().view(np.uint32)).sum())
+    assert diff == 0

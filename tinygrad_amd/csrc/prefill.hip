@@ -7,7 +7,7 @@
 #include "qgemm_rows.h"
 #include "decode.h"
 #include "moe_gate.h"
-#include <string.h>
+#include "prefill.h"
 
 int tga_rows_fmt(int ggml_type, int64_t K);                                              // qgemm_rows.hip
 int64_t tga_rows_row_bytes(int fmt, int64_t K);
@@ -277,13 +277,17 @@ __global__ __launch_bounds__(512) void rows_group_kernel(const int* __restrict__
   }
 }
 
+int pf_gate_group(const float* logits, int R, int E, int k, int gating, int norm_topk, float scale, int* sel, float* probs, int* counts, int* place, int tt, int* off, int2* tiles, int* n_tiles,
+                  int* row_tok, int* row_dst, hipStream_t s) {
+  rows_gate_kernel<<<(unsigned)((R + 3) / 4), 256, 0, s>>>(logits, R, E, k, gating, norm_topk, scale, sel, probs, counts, place);
+  TGA_LAUNCH_CHECK();
+  const int64_t gb = ((int64_t)R * k + 511) / 512;
+  rows_group_kernel<<<(unsigned)(gb < 64 ? gb : 64), 512, 0, s>>>(counts, sel, place, R, E, k, tt, off, tiles, n_tiles, row_tok, row_dst);
+  TGA_LAUNCH_CHECK();
+  return 0;
+}
+
 // ------------------------------------------------------------------------------------------------ the step
-// Indices of the int64 tables a caller passes (pointers as integers)
-enum { PM_NBLOCKS, PM_DIM, PM_HEADS, PM_KV, PM_HD, PM_MAXCTX, PM_EMB, PM_EMB_TYPE, PM_ROPE, PM_EXPERTS, PM_TOPK, PM_GATING, PM_NORM_TOPK, PM_QKNORM, PM_HIDDEN, PM_DENSE_HIDDEN, PM_EPS_BITS, PM_SCALE_BITS, PM_COUNT };
-enum { PB_ATTN_NORM, PB_FFN_NORM, PB_QN, PB_KN, PB_CK, PB_CV, PB_MOE, PB_WQ, PB_WK, PB_WV, PB_WO, PB_GATE, PB_UP, PB_DOWN, PB_ROUTER, PB_TQ, PB_TK, PB_TV, PB_TO, PB_TGATE, PB_TDOWN, PB_COUNT };
-
-static float bits_f(int64_t b) { uint32_t u = (uint32_t)b; float f; memcpy(&f, &u, 4); return f; }
-
 #define PF_PART ((size_t)64 << 20)            // partial tiles of a split K
 
 struct PfWs { size_t x, xn, q, k, v, qh, ql, attn, act, part, logits, sel, probs, place, counts, off, tiles, ntiles, row_tok, row_dst, act_e, y_e, total; };
@@ -394,8 +398,6 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
     }
     float* logits = (float*)(ws + w.logits); int* counts = (int*)(ws + w.counts); int* sel = (int*)(ws + w.sel); int* place = (int*)(ws + w.place);
     { const void* wr[1] = {(const void*)b[PB_ROUTER]}; void* yr[1] = {logits}; const int64_t nr[1] = {E}; PF_DO(linear(TGA_F16, 1, wr, yr, nr, xn, TGA_F32, dim, 0, nullptr)); }
-    rows_gate_kernel<<<(unsigned)((R + 3) / 4), 256, 0, s>>>(logits, (int)R, (int)E, (int)k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), sel, (float*)(ws + w.probs), counts, place);
-    TGA_LAUNCH_CHECK();
     // Rows of an expert's tile, us a block with 32 / 64 / 128 (D 2048, H 1024, 64 experts, top 8 | H 1024, 16, top 8 | H 1536, 32, top 8): 24 rows per expert 189 / 185 / 226 | 107 / 112 / 125 | 159 / 152 / 186,
     // 32: 213 / 196 / 236 | 119 / 114 / 127 | 174 / 157 / 191, 80: 319 / 307 / 285 | 142 / 140 / 140 | 245 / 236 / 218, 104: 373 / 338 / 344 | 162 / 146 / 147 | 279 / 243 / 231, 160: 496 / 447 / 474 | 194 / 174 / 183 |
     // 350 / 314 / 332, 255: 712 / 632 / 630 | 243 / 222 / 232 | 484 / 426 / 427, 510: - | 377 / 338 / 337 | 860 / 738 / 712, 1000: - | 660 / 578 / 561; D 1024, H 512, 8 experts, top 4: 128 rows
@@ -404,9 +406,7 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
     const int tt = avg <= 32 ? 32 : avg <= 96 ? 64 : 128;
     const int64_t max_tiles = R * k / tt + (R * k < E ? R * k : E);
     int2* tiles = (int2*)(ws + w.tiles); int* nt = (int*)(ws + w.ntiles); int* off = (int*)(ws + w.off); int* row_tok = (int*)(ws + w.row_tok); int* row_dst = (int*)(ws + w.row_dst);
-    const int64_t gb = (R * k + 511) / 512;
-    rows_group_kernel<<<(unsigned)(gb < 64 ? gb : 64), 512, 0, s>>>(counts, sel, place, (int)R, (int)E, (int)k, tt, off, tiles, nt, row_tok, row_dst);
-    TGA_LAUNCH_CHECK();
+    PF_DO(pf_gate_group(logits, (int)R, (int)E, (int)k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), sel, (float*)(ws + w.probs), counts, place, tt, off, tiles, nt, row_tok, row_dst, s));
     const int64_t hid = m[PM_HIDDEN];
     PF_DO(pf_experts((int)b[PB_TGATE], (const void*)b[PB_GATE], (const void*)b[PB_UP], hid, dim, xn, ws + w.act_e, 0, tt, max_tiles, tiles, nt, off, row_tok, nullptr, s));
     PF_DO(pf_experts((int)b[PB_TDOWN], (const void*)b[PB_DOWN], nullptr, dim, hid, (const uint16_t*)(ws + w.act_e), ws + w.y_e, 1, tt, max_tiles, tiles, nt, off, nullptr, row_dst, s));

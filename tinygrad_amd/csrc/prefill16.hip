@@ -1,0 +1,644 @@
+// Prefill steps of many rows whose sums run in the order of the steps of sixteen rows (and of eight and four): every row of the keys, values and residuals has the bits those steps give it.
+// An MoE model's expert choices at near-ties turn with the last bit of a sum, so its prompts keep that order (model.py:110-135, 464); what changes is that a weight matrix is read once for all rows
+// of the prompt and not once for every sixteen (or, the experts', once for every token and slot).  Served: dense fp16 weights, MXFP4 experts, whole-row q / k norms, at most 4096 values in a row
+// of the dense linears and 2048 in one of the experts' (prefill16_ok below); other models take the steps of sixteen.
+// Orders that are kept, per output of a row:
+//   dense linears (qgemm_wp.hip, qgemm_dma.hip, qgemm.hip)  steps of 256 values dealt to 8 (K a multiple of 1024) or 4 waves, two chains of matrix-core products per wave, waves summed in order
+//   attention     (attn_decode_kernel, norm over whole rows) float32, partials per 64 positions from runs of lanes, merged in order
+//   router        (moe_router_kernel)                        lanes' chains of dot2 over 16-byte pieces, then the tree over the wave
+//   experts       (qgemv1.h)                                 a chain of sixteen dot2 per unit of 32 weights, its scale, then the tree over the units of the row
+#include "qfmt.h"
+#include "prefill.h"
+#include "decode.h"
+#include <type_traits>
+
+typedef _Float16 v8f16 __attribute__((ext_vector_type(8)));
+typedef _Float16 v4f16 __attribute__((ext_vector_type(4)));
+typedef float v4f32 __attribute__((ext_vector_type(4)));
+typedef float v16f32 __attribute__((ext_vector_type(16)));
+
+// ------------------------------------------------------------------------------------------------ the dense linears
+// 64 weight rows x 64 activation rows per workgroup, wave = 32 x 32.  K in steps of 256 values, staged whole by requests that write LDS themselves (two workgroups of 64 KB per CU: one loads while
+// the other multiplies); row pieces of 16 bytes XORed with the row.  A step's operands are those of the sixteen-row kernels: lane 16 g + r holds the values 64 g + 8 v .. + 7 of row r for product v;
+// products of even and odd v form two chains per part, parts (the steps of one wave there: p, p + nw, ...) are summed in order.
+struct X16Gemm { const uint16_t* w[3]; float* y[3]; const float* resid; const uint16_t* x; int n[3]; int nseg, M, K, nw, ntiles; };
+__global__ __launch_bounds__(256, 2) void x16_gemm_kernel(const X16Gemm a) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[65536];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, r = lane & 15;
+  const int mt = (a.M + 63) >> 6, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+  int nt = (idx / mt) * 8 + xcd;                                          // (the row tiles of a weight tile on one XCD)
+  const int m0 = (idx % mt) * 64;
+  if (nt >= a.ntiles) return;
+  int seg = 0;
+  if (a.nseg > 1 && nt >= (a.n[0] >> 6)) { nt -= a.n[0] >> 6; seg = 1; if (nt >= (a.n[1] >> 6)) { nt -= a.n[1] >> 6; seg = 2; } }
+  const uint16_t* w = (seg == 0 ? a.w[0] : seg == 1 ? a.w[1] : a.w[2]) + (size_t)nt * 64 * a.K;
+  const int n = seg == 0 ? a.n[0] : seg == 1 ? a.n[1] : a.n[2];
+  float* y = seg == 0 ? a.y[0] : seg == 1 ? a.y[1] : a.y[2];
+  // request i of a wave fills 1 KB: rows 2 (wave + 4 i), + 1 of a 64-row tile
+  const uint16_t* src[16];
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int row = 2 * (wave + 4 * (i & 7)) + (lane >> 5), piece = (lane & 31) ^ (row & 15);
+    const int xr = min(m0 + row, a.M - 1);
+    src[i] = (i < 8 ? w + (size_t)row * a.K : a.x + (size_t)xr * a.K) + 8 * piece;
+  }
+  const int wr0 = (wave & 1) * 32, xr0 = (wave >> 1) * 32, nsteps = a.K >> 8;
+  v4f32 c0[2][2], c1[2][2], tot[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) { c0[i][j] = c1[i][j] = tot[i][j] = v4f32{0.f, 0.f, 0.f, 0.f}; }
+  for (int p = 0; p < a.nw && p < nsteps; p++) {
+    for (int s = p; s < nsteps; s += a.nw) {
+      __syncthreads();                                                    // everyone is done with the step before
+#pragma unroll
+      for (int i = 0; i < 16; i++)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + 256 * s), (__attribute__((address_space(3))) void*)(lds + (i < 8 ? 0 : 32768) + (wave + 4 * (i & 7)) * 1024), 16, 0, 0);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+#pragma unroll
+      for (int v = 0; v < 8; v++) {
+        v8f16 wa[2], xb[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          wa[i] = *(const v8f16*)(lds + (wr0 + 16 * i + r) * 512 + (((8 * g + v) ^ r) << 4));
+          xb[i] = *(const v8f16*)(lds + 32768 + (xr0 + 16 * i + r) * 512 + (((8 * g + v) ^ r) << 4));
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) {
+            if (v & 1) c1[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa[i], xb[j], c1[i][j], 0, 0, 0);
+            else c0[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa[i], xb[j], c0[i][j], 0, 0, 0);
+          }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) { const v4f32 part = c0[i][j] + c1[i][j]; tot[i][j] += part; c0[i][j] = c1[i][j] = v4f32{0.f, 0.f, 0.f, 0.f}; }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const int row = m0 + xr0 + 16 * j + r;
+      if (row >= a.M) continue;
+      const size_t o = (size_t)row * n + nt * 64 + wr0 + 16 * i + 4 * g;
+      v4f32 v = tot[i][j];
+      if (a.resid) v += *(const v4f32*)(a.resid + o);
+      *(v4f32*)(y + o) = v;
+    }
+}
+
+// ------------------------------------------------------------------------------------------------ the first norm of the steps of eight and four rows
+// Those steps fold the first block's attn_norm into their q / k / v launch (qgemm_wp.hip / qgemm_dma.hip), whose waves sum the squares of 256 values each: lane l of wave w the values 256 w + 4 l .. + 3
+__global__ __launch_bounds__(1024) void x16_fold_norm_kernel(const float* __restrict__ x, const float* __restrict__ w, int K, float eps, uint16_t* __restrict__ out) {
+  __shared__ float nsum[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = K >> 8;
+  x += (size_t)blockIdx.x * K; out += (size_t)blockIdx.x * K;
+  f32x4 f = {0.f, 0.f, 0.f, 0.f}, nw4 = {0.f, 0.f, 0.f, 0.f};
+  if (wave < nw) { f = ((const f32x4*)x)[tid]; nw4 = ((const f32x4*)w)[tid]; }
+  float ps = 0.f;
+  ps += f.x * f.x + f.y * f.y + f.z * f.z + f.w * f.w;
+  ps = wave_sum(ps);
+  if (lane == 0) nsum[wave] = ps;
+  __syncthreads();
+  float t = 0.f;
+  for (int i = 0; i < nw; i++) t += nsum[i];
+  const float sc = 1.0f / sqrtf(t / (float)K + eps);
+  if (wave < nw) {
+    f.x = (f.x * sc) * nw4.x; f.y = (f.y * sc) * nw4.y; f.z = (f.z * sc) * nw4.z; f.w = (f.w * sc) * nw4.w;
+    ((u32x2*)out)[tid] = u32x2{f2h_bits(f.x) | (f2h_bits(f.y) << 16), f2h_bits(f.z) | (f2h_bits(f.w) << 16)};
+  }
+}
+
+// ------------------------------------------------------------------------------------------------ q / k norm over whole rows, rotation, append
+// One workgroup per row; the sums of squares as attn_decode_kernel forms them (four 16-byte pieces per thread, waves in order).  q leaves rotated in float32.
+__device__ __forceinline__ float x16_rope_lo(float x1, float x2, float c, float s) { return __builtin_fmaf(x1, c, -(x2 * s)); }
+__device__ __forceinline__ float x16_rope_hi(float x1, float x2, float c, float s) { return __builtin_fmaf(x2, c, x1 * s); }
+struct X16Rope { const float* q; const float* k; const float* v; const float* qn; const float* kn; const float* rope; float* qr; uint16_t* ck; uint16_t* cv; int* zero; int H, KV, hd, max_ctx, pos0, n_zero; float eps; };
+__global__ __launch_bounds__(256) void x16_rope_kernel(const X16Rope a) {
+  __shared__ float red[8];
+  const int row = blockIdx.x, pos = a.pos0 + row, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = a.hd >> 1;
+  const int nq = a.H * a.hd, nk = a.KV * a.hd;
+  if (row == 0) for (int i = tid; i < a.n_zero; i += 256) a.zero[i] = 0;
+  const float* q = a.q + (size_t)row * nq; const float* k = a.k + (size_t)row * nk; const float* v = a.v + (size_t)row * nk;
+  const int n4q = nq >> 2, n4k = nk >> 2;
+  f32x4 nq4[4], nk4[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    const int i = tid + 256 * t;
+    nq4[t] = ((const f32x4*)q)[i < n4q ? i : n4q - 1]; nk4[t] = ((const f32x4*)k)[i < n4k ? i : n4k - 1];
+  }
+  float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    const int i = tid + 256 * t;
+    const f32x4 x = nq4[t], y = nk4[t];
+    s0 += i < n4q ? x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w : 0.f;
+    s1 += i < n4k ? y.x * y.x + y.y * y.y + y.z * y.z + y.w * y.w : 0.f;
+  }
+  s0 = wave_sum(s0); s1 = wave_sum(s1);
+  if (lane == 0) { red[wave] = s0; red[4 + wave] = s1; }
+  __syncthreads();
+  const float qscale = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)(a.H * a.hd) + a.eps);
+  const float kscale = 1.0f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)(a.KV * a.hd) + a.eps);
+  const size_t cstep = (size_t)a.max_ctx * a.hd, crow = (size_t)pos * a.hd;
+  for (int e = 4 * tid; e < nk; e += 1024) {
+    const int hh = e / a.hd;
+    const f32x4 x = *(const f32x4*)(v + e);
+    *(u32x2*)(a.cv + crow + hh * cstep + (e - hh * a.hd)) = u32x2{f2h_bits(x.x) | (f2h_bits(x.y) << 16), f2h_bits(x.z) | (f2h_bits(x.w) << 16)};
+  }
+  const bool live = lane < half;
+  const int i = live ? lane : half - 1;
+  const float c = a.rope[(size_t)pos * a.hd + i], s = a.rope[(size_t)pos * a.hd + half + i];
+#pragma unroll 4
+  for (int h = wave; h < a.H + a.KV; h += 4) {
+    const bool isq = h < a.H;
+    const int o = (isq ? h : h - a.H) * a.hd;
+    const float* src = isq ? q + o : k + o; const float* wn = isq ? a.qn + o : a.kn + o;
+    const float sc = isq ? qscale : kscale;
+    const float x1 = (src[i] * sc) * wn[i], x2 = (src[half + i] * sc) * wn[half + i];
+    float lo = x16_rope_lo(x1, x2, c, s), hi = x16_rope_hi(x1, x2, c, s);
+    asm volatile("" : "+v"(lo), "+v"(hi));                                // (float32 values before they are rounded to fp16, as there)
+    if (!live) continue;
+    if (isq) { float* d = a.qr + (size_t)row * nq + o; d[i] = lo; d[half + i] = hi; }
+    else { uint16_t* d = a.ck + crow + (h - a.H) * cstep; d[i] = (uint16_t)f2h_bits(lo); d[half + i] = (uint16_t)f2h_bits(hi); }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------ attention
+// The arithmetic of attn_decode_kernel (float32 products and sums, runs of HD8 lanes per row of keys, partials of 64 positions), with a workgroup's 64 keys and values in registers for the rows of a
+// chunk: workgroup = (kv head, 64 positions, X16_ROWS rows); four (row, query head) pairs at a time.
+#define X16_ROWS 32
+struct X16Attn { const float* qr; const uint16_t* ck; const uint16_t* cv; float* part; uint16_t* out; int H, KV, max_ctx, P, pos0, nsplit; float scale; };
+
+template <int HD8>
+__device__ __forceinline__ float x16_run_sum(float v) {
+  v = dpp_add<0xB1>(v); v = dpp_add<0x4E>(v); v = dpp_add<0x141>(v);
+  if constexpr (HD8 >= 16) v = dpp_add<0x140>(v);
+  return v;
+}
+
+template <int HD8>
+__global__ __launch_bounds__(256) void x16_attn_kernel(const X16Attn a) {
+  constexpr int HD = HD8 * 8, RPI = 64 / HD8, NVI = 16 / RPI, NGRP = 4 * RPI, CSTR = HD + 4;
+  __shared__ float comb[4 * NGRP * CSTR];
+  const int kvh = blockIdx.x, split = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = a.H / a.KV, vr = lane / HD8, vp = lane % HD8;
+  const int row_end = min((int)(blockIdx.z + 1) * X16_ROWS, a.P), row_first = max((int)blockIdx.z * X16_ROWS, split * 64 - a.pos0);      // (rows that see a position of the split)
+  if (row_first >= row_end) return;
+  const int p0 = split * 64 + wave * 16, last = a.pos0 + a.P - 1;
+  u32x4 kt[NVI], vt[NVI];
+  {
+    const uint16_t* kb = a.ck + (size_t)kvh * a.max_ctx * HD + vp * 8; const uint16_t* vb = a.cv + (size_t)kvh * a.max_ctx * HD + vp * 8;
+#pragma unroll
+    for (int i = 0; i < NVI; i++) {
+      const int rc = min(p0 + i * RPI + vr, last);                         // (beyond the rows appended so far: masked below, but 0 times what lies there has to be 0)
+      kt[i] = *(const u32x4*)(kb + (size_t)rc * HD); vt[i] = *(const u32x4*)(vb + (size_t)rc * HD);
+    }
+  }
+  const int np = (row_end - row_first) * group;
+  f32x4 qa[4], qb[4];
+  auto fetch = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int hh = 0; hh < 4; hh++) {
+      const int p = min(b + hh, np - 1), row = row_first + p / group, head = kvh * group + p % group;
+      const float* s = a.qr + ((size_t)row * a.H + head) * HD + vp * 8;
+      qa[hh] = *(const f32x4*)s; qb[hh] = *(const f32x4*)(s + 4);
+    }
+  };
+  fetch(0);
+  for (int b = 0; b < np; b += 4) {
+    f32x4 q0[4], q1[4];
+#pragma unroll
+    for (int hh = 0; hh < 4; hh++) { q0[hh] = qa[hh]; q1[hh] = qb[hh]; }
+    fetch(b + 4);                                                          // (past the end: the last pair again)
+#pragma unroll
+    for (int hh = 0; hh < 4; hh++) {
+      if (b + hh < np) {
+        const int pos = a.pos0 + row_first + (b + hh) / group;
+        const float qq[8] = {q0[hh].x, q0[hh].y, q0[hh].z, q0[hh].w, q1[hh].x, q1[hh].y, q1[hh].z, q1[hh].w};
+        float sc[NVI];
+        float m = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < NVI; i++) {
+          const u32x4 kk = kt[i];
+          const half2_t k0 = as_h2(kk.x), k1 = as_h2(kk.y), k2 = as_h2(kk.z), k3 = as_h2(kk.w);
+          float t = qq[0] * (float)k0.x; t += qq[1] * (float)k0.y; t += qq[2] * (float)k1.x; t += qq[3] * (float)k1.y;
+          t += qq[4] * (float)k2.x; t += qq[5] * (float)k2.y; t += qq[6] * (float)k3.x; t += qq[7] * (float)k3.y;
+          t = x16_run_sum<HD8>(t);
+          sc[i] = (p0 + i * RPI + vr <= pos) ? t * a.scale : -INFINITY;
+          m = fmaxf(m, sc[i]);
+        }
+        float l = 0.f;
+        f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NVI; i++) {
+          const float pj = (p0 + i * RPI + vr <= pos) ? __expf(sc[i] - m) : 0.f;
+          l += pj;
+          const u32x4 vv = vt[i];
+          const half2_t v0 = as_h2(vv.x), v1 = as_h2(vv.y), v2 = as_h2(vv.z), v3 = as_h2(vv.w);
+          o0.x += pj * (float)v0.x; o0.y += pj * (float)v0.y; o0.z += pj * (float)v1.x; o0.w += pj * (float)v1.y;
+          o1.x += pj * (float)v2.x; o1.y += pj * (float)v2.y; o1.z += pj * (float)v3.x; o1.w += pj * (float)v3.y;
+        }
+        float* cw = comb + (size_t)(hh * NGRP + wave * RPI + vr) * CSTR;
+        *(f32x4*)(cw + vp * 8) = o0; *(f32x4*)(cw + vp * 8 + 4) = o1;
+        if (vp == 0) { cw[HD] = m; cw[HD + 1] = l; }
+      }
+    }
+    __syncthreads();
+    if (b + wave < np) {
+      const int row = row_first + (b + wave) / group, head = kvh * group + (b + wave) % group;
+      const float* cb = comb + (size_t)wave * NGRP * CSTR;
+      float m = -INFINITY;
+#pragma unroll
+      for (int g = 0; g < NGRP; g++) m = fmaxf(m, cb[g * CSTR + HD]);
+      float l = 0.f, od[HD / 64];
+#pragma unroll
+      for (int j = 0; j < HD / 64; j++) od[j] = 0.f;
+#pragma unroll
+      for (int g = 0; g < NGRP; g++) {
+        const float mg = cb[g * CSTR + HD];
+        const float wg = mg == -INFINITY ? 0.f : __expf(mg - m);
+        l += wg * cb[g * CSTR + HD + 1];
+#pragma unroll
+        for (int j = 0; j < HD / 64; j++) od[j] += wg * cb[g * CSTR + lane + 64 * j];
+      }
+      float* po = a.part + (((size_t)row * a.H + head) * a.nsplit + split) * (HD + 2);
+#pragma unroll
+      for (int j = 0; j < HD / 64; j++) po[lane + 64 * j] = od[j];
+      if (lane == 0) { po[HD] = m; po[HD + 1] = l; }
+    }
+    __syncthreads();
+  }
+}
+
+// The partials of a (row, head) merged as attn_merge_kernel does (at most HD splits)
+template <int HD>
+__global__ __launch_bounds__(HD) void x16_merge_kernel(const X16Attn a) {
+  constexpr int FB = 24, NB = 16;
+  const int head = blockIdx.x, row = blockIdx.y, d = threadIdx.x;
+  __shared__ float sw[HD];
+  __shared__ float red[2 * (HD / 64)];
+  const float* ph = a.part + ((size_t)row * a.H + head) * a.nsplit * (HD + 2);
+  const int ns = ((a.pos0 + row) >> 6) + 1;                                // (at most nsplit)
+  const int spc = d < ns ? d : ns - 1;
+  const float mv = ph[(size_t)spc * (HD + 2) + HD], lv = ph[(size_t)spc * (HD + 2) + HD + 1];
+  float v[FB];
+#pragma unroll
+  for (int j = 0; j < FB; j++) v[j] = ph[(size_t)(j < ns ? j : ns - 1) * (HD + 2) + d];
+  float m = wave_max(d < ns ? mv : -INFINITY), l = 0.f;
+  if constexpr (HD > 64) {
+    if ((d & 63) == 0) red[d >> 6] = m;
+    __syncthreads();
+    m = red[0];
+#pragma unroll
+    for (int i = 1; i < HD / 64; i++) m = fmaxf(m, red[i]);
+  }
+  const float e = d < ns ? __expf(mv - m) : 0.f;
+  if (d < ns) sw[d] = e;
+  l = d < ns ? lv * e : 0.f;
+  l = wave_sum(l);
+  if constexpr (HD > 64) {
+    if ((d & 63) == 0) red[HD / 64 + (d >> 6)] = l;
+    __syncthreads();
+    l = 0.f;
+#pragma unroll
+    for (int i = 0; i < HD / 64; i++) l += red[HD / 64 + i];
+  } else __syncthreads();
+  float o = 0.f;
+#pragma unroll
+  for (int j = 0; j < FB; j++) o += j < ns ? v[j] * sw[j] : 0.f;
+  for (int s0 = FB; s0 < ns; s0 += NB) {
+    float w[NB];
+#pragma unroll
+    for (int j = 0; j < NB; j++) w[j] = ph[(size_t)min(s0 + j, ns - 1) * (HD + 2) + d];
+#pragma unroll
+    for (int j = 0; j < NB; j++) o += s0 + j < ns ? w[j] * sw[s0 + j] : 0.f;
+  }
+  o *= 1.0f / l;
+  asm volatile("" : "+v"(o));                                             // (a float32 value before it is rounded to fp16, as there)
+  a.out[((size_t)row * a.H + head) * HD + d] = (uint16_t)f2h_bits(o);
+}
+
+// ------------------------------------------------------------------------------------------------ ffn_norm and router logits
+// The arithmetic of moe_router_kernel, RT rows per workgroup: normalised once, the router's rows read once for all of them.  The normalised rows leave as the experts read them: the sixteen pairs
+// (value j, value j + 16) of a unit of 32 behind each other.  inf: set where a normalised value is not finite in fp16 (the experts' kernel then keeps products with padding apart).
+struct X16Router { const float* x; const float* nw; const uint16_t* wr; uint16_t* xs; float* logits; int* inf; int R, dim, E; float eps; };
+template <int RT>
+__global__ __launch_bounds__(256) void x16_router_kernel(const X16Router a) {
+  __shared__ __attribute__((aligned(16))) uint16_t xn[RT][2048];
+  __shared__ float red[RT][4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), np = a.dim >> 3, r0 = blockIdx.x * RT;
+  const bool have = tid < np;                                              // (dim <= 2048: a piece of 8 values per thread)
+  const int p = have ? tid : np - 1;
+  f32x4 xa[RT][2];
+#pragma unroll
+  for (int t = 0; t < RT; t++) { const float* x = a.x + (size_t)min(r0 + t, a.R - 1) * a.dim; xa[t][0] = ((const f32x4*)x)[2 * p]; xa[t][1] = ((const f32x4*)x)[2 * p + 1]; }
+  const f32x4 w0 = ((const f32x4*)a.nw)[2 * p], w1 = ((const f32x4*)a.nw)[2 * p + 1];
+#pragma unroll
+  for (int t = 0; t < RT; t++) {
+    float s = 0.f;
+    if (have) {
+#pragma unroll
+      for (int h = 0; h < 2; h++) s += xa[t][h].x * xa[t][h].x + xa[t][h].y * xa[t][h].y + xa[t][h].z * xa[t][h].z + xa[t][h].w * xa[t][h].w;
+    }
+    s = wave_sum(s);
+    if (lane == 0) red[t][wave] = s;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < RT; t++) {
+    const float nscale = 1.0f / sqrtf((red[t][0] + red[t][1] + red[t][2] + red[t][3]) / (float)a.dim + a.eps);
+    if (have) {
+      float v[8] = {xa[t][0].x, xa[t][0].y, xa[t][0].z, xa[t][0].w, xa[t][1].x, xa[t][1].y, xa[t][1].z, xa[t][1].w};
+      const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+      for (int i = 0; i < 8; i++) v[i] = (v[i] * nscale) * w[i];
+      *(u32x4*)(&xn[t][8 * p]) = u32x4{f2h_bits(v[0]) | (f2h_bits(v[1]) << 16), f2h_bits(v[2]) | (f2h_bits(v[3]) << 16), f2h_bits(v[4]) | (f2h_bits(v[5]) << 16), f2h_bits(v[6]) | (f2h_bits(v[7]) << 16)};
+    }
+  }
+  __syncthreads();
+  bool bad = false;
+#pragma unroll
+  for (int t = 0; t < RT; t++)
+    if (r0 + t < a.R)
+      for (int d = tid; d < (a.dim >> 1); d += 256) {
+        const int e = 32 * (d >> 4) + (d & 15);
+        const uint32_t lo = xn[t][e], hi = xn[t][e + 16];
+        bad = bad || (lo & 0x7c00) == 0x7c00 || (hi & 0x7c00) == 0x7c00;
+        ((uint32_t*)(a.xs + (size_t)(r0 + t) * a.dim))[d] = lo | (hi << 16);
+      }
+  if (bad) *a.inf = 1;                                                     // (whoever writes it writes the same)
+  for (int e = wave; e < a.E; e += 4) {
+    const uint16_t* wrow = a.wr + (size_t)e * a.dim;
+    u32x4 wv[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) { const int q = lane + 64 * j; wv[j] = *(const u32x4*)(wrow + 8 * (q < np ? q : np - 1)); }
+#pragma unroll
+    for (int t = 0; t < RT; t++) {
+      float acc = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int q = lane + 64 * j;
+        if (q < np) { const u32x4 xv = *(const u32x4*)(&xn[t][8 * q]); acc = dot2(wv[j].w, xv.w, dot2(wv[j].z, xv.z, dot2(wv[j].y, xv.y, dot2(wv[j].x, xv.x, acc)))); }
+      }
+      acc = wave_sum(acc);
+      if (lane == 0 && r0 + t < a.R) a.logits[(size_t)(r0 + t) * a.E + e] = acc;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------ the experts
+// An expert's MXFP4 weights against the rows of all its assignments, each result with the bits of the expert GEMV (qgemv1.h): per unit of 32 weights a chain of sixteen dot2 from zero, times the
+// block's scale, then the tree over the units (pairs of neighbours first).  v_dot2_f32_f16 rounds the sum of two products and the addend once, and so does a matrix-core product whose other products
+// are zeros: v_mfma_f32_16x16x4_4b_f16 with two of its four values zero is 2048 dot2 in 32 cycles where the vector unit takes 256 (bits compared over normal, subnormal and huge values, sums
+// from zero and not; with all four values in use they differ, so the matrix cores run at a quarter of their fp16 rate here).
+// A workgroup owns 64 weight rows of one expert (SwiGLU: 32 of gate and the same 32 of up) and walks the expert's rows in tiles of sixteen; wave w holds units w UPW .. of the rows in registers for
+// the whole walk, so the weights are read once.  Lane 16 b + c supplies column c of block b; the sixteen rows of the tile are the other operand, the same for the four blocks.  The waves'
+// partial sums meet in LDS, where the upper levels of the tree are formed.
+// The zeros sit in the weight operand (the pair beside a weight pair).  Where a row holds values that are not finite (inf), the pair beside an activation pair is zero too: 0 x infinity would be NaN.
+struct X16Expert { const uint8_t* w[2]; const uint16_t* x; void* y; const int* off; const int* row_tok; const int* row_dst; int* inf; long long estride, row_bytes; int K, N, ngroups; };
+
+template <bool SW, int UPW>
+__global__ __launch_bounds__(512) void x16_expert_kernel(const X16Expert a) {
+  constexpr int ND = (17 * UPW + 3) / 4;                                   // dwords of a lane's run of a weight row
+  __shared__ float part[2][8][16][64];
+  const int e = blockIdx.x / a.ngroups, grp = blockIdx.x % a.ngroups;
+  const int first = a.off[e], cnt = a.off[e + 1] - first;
+  if (cnt <= 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), blk = lane >> 4, c = lane & 15;
+  const int nw = blockDim.x >> 6;                                          // (K = 32 UPW nw)
+  const int col = SW ? grp * 32 + (blk & 1) * 16 + c : grp * 64 + lane;
+  uint32_t raw[ND];
+  {
+    const uint8_t* p = (SW && blk >= 2 ? a.w[1] : a.w[0]) + e * a.estride + (long long)col * a.row_bytes + 17 * UPW * wave;      // (4-byte aligned: K is a multiple of 256)
+#pragma unroll
+    for (int i = 0; i < ND / 4; i++) { const u32x4 v = ld16(p + 16 * i); raw[4 * i] = v.x; raw[4 * i + 1] = v.y; raw[4 * i + 2] = v.z; raw[4 * i + 3] = v.w; }
+#pragma unroll
+    for (int i = ND / 4 * 4; i < ND; i++) raw[i] = ld4(p + 4 * i);
+  }
+  for (int w = nw + wave; w < 8; w += nw) {                                // (units beyond the row are zeros of the tree)
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) part[b][w][i][lane] = 0.f;
+  }
+  const int ntile = (cnt + 15) >> 4;
+  u32x4 xq[2][4];
+  const uint16_t* xrow;
+  auto row_of = [&](int t) __attribute__((always_inline)) {
+    const int rr = first + min(16 * t + c, cnt - 1);
+    return a.x + (size_t)(SW ? a.row_tok[rr] : rr) * a.K + 32 * UPW * wave;
+  };
+  auto fetch = [&](u32x4 (&d)[4], const uint16_t* p, int u) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) d[i] = *(const u32x4*)(p + 32 * u + 8 * i);
+  };
+  xrow = row_of(0);
+  fetch(xq[0], xrow, 0);
+  const bool inf = *a.inf != 0;
+  u32x2 wz[16];
+#pragma unroll
+  for (int j = 0; j < 16; j++) wz[j] = u32x2{0u, 0u};
+  auto byte_dword = [&](int o) __attribute__((always_inline)) { return (o & 3) ? __builtin_amdgcn_alignbit(raw[(o >> 2) + 1], raw[o >> 2], 8 * (o & 3)) : raw[o >> 2]; };
+  // one unit: the chain, the scale
+  auto unit = [&](int u, const u32x4 (&x)[4], float (&leaf)[16], auto inf_tag) __attribute__((always_inline)) {
+    const int o = 17 * u;
+    const uint32_t eb = (raw[o >> 2] >> (8 * (o & 3))) & 0xffu;
+    const uint32_t s02 = eb ? (eb << 23) : 0x00400000u;
+    uint32_t q[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) q[t] = byte_dword(o + 1 + 4 * t);
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      wz[4 * t + 0].x = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[t], 1.0f, 0));
+      wz[4 * t + 1].y = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[t], 1.0f, 1));
+      wz[4 * t + 2].x = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[t], 1.0f, 2));
+      wz[4 * t + 3].y = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[t], 1.0f, 3));
+    }
+    v16f32 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+      u32x2 xa = (j & 2) ? u32x2{x[j >> 2].z, x[j >> 2].w} : u32x2{x[j >> 2].x, x[j >> 2].y};
+      if constexpr (decltype(inf_tag)::value) xa = (j & 1) ? u32x2{0u, xa.y} : u32x2{xa.x, 0u};
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xa), __builtin_bit_cast(v4f16, wz[j]), acc, 0, 0, 0);
+    }
+    // the scales of the four blocks' column c
+    const auto h = __builtin_amdgcn_permlane32_swap(s02, s02, false, false);
+    const auto l0 = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false), l1 = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+    const uint32_t su[4] = {l0[0], l0[1], l1[0], l1[1]};                  // (a bit cast of an element of such a pair takes the first)
+    const float sb[4] = {__builtin_bit_cast(float, su[0]), __builtin_bit_cast(float, su[1]), __builtin_bit_cast(float, su[2]), __builtin_bit_cast(float, su[3])};
+#pragma unroll
+    for (int i = 0; i < 16; i++) leaf[i] = __builtin_fmaf(sb[i >> 2], acc[i], 0.f);
+  };
+  for (int t = 0; t < ntile; t++) {
+    const uint16_t* xnext = row_of(t + 1 < ntile ? t + 1 : t);
+    float st[3][16], leaf[16];                                             // sums of 1, 2 and 4 units that wait for their neighbour
+    auto walk = [&](auto tag) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < UPW; u++) {
+        if (u + 1 < UPW) fetch(xq[(u + 1) & 1], xrow, u + 1); else fetch(xq[(u + 1) & 1], xnext, 0);
+        unit(u, xq[u & 1], leaf, tag);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          float v = leaf[i];
+          if (u & 1) { v = st[0][i] + v; if (u & 2) { v = st[1][i] + v; if (u & 4) v = st[2][i] + v; else st[2][i] = v; } else st[1][i] = v; }
+          else st[0][i] = v;
+          if (u == UPW - 1) leaf[i] = v;
+        }
+      }
+    };
+    static_assert(UPW == 4 || UPW == 8, "whole subtrees");
+    if (inf) walk(std::true_type{}); else walk(std::false_type{});
+    xrow = xnext;
+    float (*pt)[16][64] = part[t & 1];
+#pragma unroll
+    for (int i = 0; i < 16; i++) pt[wave][i][lane] = leaf[i];
+    __syncthreads();                                                       // (the set of the tile before last is rewritten behind the next barrier only: its readers have passed this one)
+    // register 4 b + i of lane l is row 4 (l / 16) + i of column l % 16 of block b
+    for (int o = tid; o < 512; o += blockDim.x) {
+      const int l = o & 63, h = (o >> 6) & 1, i = o >> 7, row = 4 * (l >> 4) + i;
+      if (16 * t + row >= cnt) continue;
+      float s[2];
+#pragma unroll
+      for (int z = 0; z < 2; z++) {
+        const int rg = 4 * (h + 2 * z) + i;
+        s[z] = ((pt[0][rg][l] + pt[1][rg][l]) + (pt[2][rg][l] + pt[3][rg][l])) + ((pt[4][rg][l] + pt[5][rg][l]) + (pt[6][rg][l] + pt[7][rg][l]));
+      }
+      const int rr = first + 16 * t + row, cc = l & 15;
+      if constexpr (SW) {
+        float v = silu_f(s[0]) * s[1];
+        asm volatile("" : "+v"(v));                                       // (rounded to float32 first, as there)
+        const uint32_t hb = __builtin_bit_cast(uint16_t, (_Float16)v);
+        if ((hb & 0x7c00) == 0x7c00) a.inf[1] = 1;
+        ((uint16_t*)a.y)[(size_t)rr * a.N + grp * 32 + 2 * cc + h] = (uint16_t)hb;
+      } else {
+        float* y = (float*)a.y + (size_t)a.row_dst[rr] * a.N + grp * 64 + cc;
+        y[16 * h] = s[0]; y[16 * (h + 2)] = s[1];
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------ the step
+struct X16Ws { size_t x, xn, q, k, v, qr, attn, part, logits, sel, probs, place, counts, off, tiles, ntiles, row_tok, row_dst, xs, act, y, inf, total; };
+static X16Ws x16_layout(const int64_t* m, int64_t R, int64_t nsplit) {
+  X16Ws w = {}; size_t o = 0;
+  auto take = [&](size_t n) { const size_t at = o; o += (n + 255) & ~(size_t)255; return at; };
+  const int64_t dim = m[PM_DIM], nq = m[PM_HEADS] * m[PM_HD], nk = m[PM_KV] * m[PM_HD], E = m[PM_EXPERTS], k = m[PM_TOPK];
+  w.x = take(R * dim * 4); w.xn = take(R * dim * 2); w.q = take(R * nq * 4); w.k = take(R * nk * 4); w.v = take(R * nk * 4); w.qr = take(R * nq * 4); w.attn = take(R * nq * 2);
+  w.part = take(R * m[PM_HEADS] * nsplit * (m[PM_HD] + 2) * 4);
+  w.logits = take(R * E * 4); w.sel = take(R * k * 4); w.probs = take(R * k * 4); w.place = take(R * k * 4); w.counts = take((E + 2) * 4); w.inf = w.counts + E * 4; w.off = take((E + 1) * 4);
+  w.tiles = take((R * k / 16 + E + 1) * 8); w.ntiles = take(4); w.row_tok = take(R * k * 4); w.row_dst = take(R * k * 4); w.xs = take(R * dim * 2);
+  w.act = take(R * k * m[PM_HIDDEN] * 2); w.y = take(R * k * dim * 4);
+  w.total = o;
+  return w;
+}
+
+// steps of 256 values go to eight waves in qgemm_wp.hip and qgemm_dma.hip (K a multiple of 1024), to four in qgemm.hip
+static int x16_waves(int64_t K) { return K % 1024 == 0 ? 8 : 4; }
+static bool x16_dense(int64_t type, int64_t w, int64_t n, int64_t K) { return type == GGML_F16 && w % 16 == 0 && n > 0 && n % 64 == 0 && K >= 512 && K <= 4096 && K % 256 == 0; }
+static bool prefill16_ok(const int64_t* m, const int64_t* blocks) {
+  const int64_t dim = m[PM_DIM], H = m[PM_HEADS], KV = m[PM_KV], hd = m[PM_HD], E = m[PM_EXPERTS], k = m[PM_TOPK], hid = m[PM_HIDDEN];
+  if (!(hd == 64 || hd == 128) || KV <= 0 || H % KV || H * hd > 4096 || m[PM_QKNORM] != H * hd || m[PM_QKNORM] == hd || E < 1 || E > 512 || k < 1 || k > 64 || k > E || m[PM_GATING] < 1 || m[PM_GATING] > 4) return false;
+  if (dim > 2048 || dim % 256 || hid > 2048 || hid % 256 || hid < 256 || (m[PM_MAXCTX] + 63) / 64 > hd) return false;
+  for (int64_t i = 0; i < m[PM_NBLOCKS]; i++) {
+    const int64_t* b = blocks + i * PB_COUNT;
+    if (!b[PB_MOE] || !b[PB_QN] || !b[PB_KN] || b[PB_TGATE] != GGML_MXFP4 || b[PB_TDOWN] != GGML_MXFP4) return false;
+    if (!x16_dense(b[PB_TQ], b[PB_WQ], H * hd, dim) || !x16_dense(b[PB_TK], b[PB_WK], KV * hd, dim) || !x16_dense(b[PB_TV], b[PB_WV], KV * hd, dim) || !x16_dense(b[PB_TO], b[PB_WO], dim, H * hd)) return false;
+    if ((b[PB_GATE] | b[PB_UP] | b[PB_DOWN]) % 4 || (b[PB_ROUTER] | b[PB_ATTN_NORM] | b[PB_FFN_NORM] | b[PB_QN] | b[PB_KN] | b[PB_CK] | b[PB_CV]) % 16) return false;
+  }
+  return true;
+}
+
+static int x16_linear(int nseg, const int64_t* w, float* const* y, const int64_t* n, const uint16_t* x, int64_t M, int64_t K, const float* resid, hipStream_t s) {
+  X16Gemm a = {};
+  for (int i = 0; i < nseg; i++) { a.w[i] = (const uint16_t*)w[i]; a.y[i] = y[i]; a.n[i] = (int)n[i]; a.ntiles += (int)(n[i] / 64); }
+  a.resid = resid; a.x = x; a.nseg = nseg; a.M = (int)M; a.K = (int)K; a.nw = x16_waves(K);
+  x16_gemm_kernel<<<(unsigned)((a.ntiles + 7) / 8 * 8 * ((M + 63) / 64)), 256, 0, s>>>(a);
+  TGA_LAUNCH_CHECK();
+  return 0;
+}
+
+template <bool SW>
+static int x16_experts(const X16Expert& e, int64_t E, int64_t K, int64_t N, hipStream_t s) {
+  X16Expert a = e;
+  a.row_bytes = K / 32 * 17; a.estride = a.row_bytes * N; a.K = (int)K; a.N = (int)N; a.ngroups = (int)(SW ? N / 32 : N / 64);
+  // the tree has 64 leaves for rows of more than 32 units (qgemv1.h: a wave), else 32 (half a wave); eight subtrees either way
+  const int upw = K > 1024 ? 8 : 4;
+  const unsigned grid = (unsigned)(E * a.ngroups), nt = (unsigned)(K / 32 / upw * 64);
+  if (upw == 8) x16_expert_kernel<SW, 8><<<grid, nt, 0, s>>>(a); else x16_expert_kernel<SW, 4><<<grid, nt, 0, s>>>(a);
+  TGA_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" {
+
+int tga_prefill16_plan(const int64_t* m, const int64_t* blocks, int64_t rows, int64_t end, int* ok, int64_t* nbytes) {
+  TGA_REQUIRE(m && blocks && ok && nbytes && rows >= 1 && end >= rows, "tga_prefill16_plan: null pointer or no rows");
+  *ok = prefill16_ok(m, blocks);
+  *nbytes = *ok ? (int64_t)x16_layout(m, rows, (end + 63) / 64).total : 0;
+  return 0;
+}
+
+int tga_prefill16_step(const int64_t* m, const int64_t* blocks, const int32_t* tokens, int64_t P, int64_t tail, int64_t pos0, void* workspace, void* state, void* stream) {
+  TGA_REQUIRE(m && blocks && tokens && workspace && state && P >= 1 && tail >= 0 && tail <= P && pos0 >= 0 && pos0 + P <= m[PM_MAXCTX], "tga_prefill16_step: null pointer or rows beyond the cache");
+  TGA_REQUIRE(prefill16_ok(m, blocks), "tga_prefill16_step: a model outside the range (tga_prefill16_plan says which are inside)");
+  const int64_t R = P, dim = m[PM_DIM], H = m[PM_HEADS], KV = m[PM_KV], hd = m[PM_HD], nq = H * hd, nk = KV * hd, E = m[PM_EXPERTS], k = m[PM_TOPK], hid = m[PM_HIDDEN], nsplit = (pos0 + P + 63) / 64;
+  TGA_REQUIRE(R <= 4096 && R * k <= (1 << 20), "tga_prefill16_step: %lld rows are more than a step takes", (long long)R);
+  const X16Ws w = x16_layout(m, R, nsplit);
+  uint8_t* ws = (uint8_t*)workspace;
+  float* x = (float*)(ws + w.x); uint16_t* xn = (uint16_t*)(ws + w.xn); float* q = (float*)(ws + w.q); float* kk = (float*)(ws + w.k); float* v = (float*)(ws + w.v); uint16_t* attn = (uint16_t*)(ws + w.attn);
+  float* logits = (float*)(ws + w.logits); float* probs = (float*)(ws + w.probs); float* ye = (float*)(ws + w.y); int* off = (int*)(ws + w.off);
+  int* row_tok = (int*)(ws + w.row_tok); int* row_dst = (int*)(ws + w.row_dst); int* inf = (int*)(ws + w.inf);
+  hipStream_t s = (hipStream_t)stream;
+  const float eps = bits_f(m[PM_EPS_BITS]);
+  int rc;
+#define PF_DO(call) do { if ((rc = (call))) return rc; } while (0)
+  PF_DO(tga_embed_rows((const void*)m[PM_EMB], (int)m[PM_EMB_TYPE], (int)dim, tokens, (int)R, state, x, stream));
+  for (int64_t bi = 0; bi < m[PM_NBLOCKS]; bi++) {
+    const int64_t* b = blocks + bi * PB_COUNT;
+    const float* an = (const float*)b[PB_ATTN_NORM];
+    if (bi) PF_DO(tga_moe_combine_rmsnorm_rows(ye, probs, x, an, (int)R, (int)k, (int)dim, eps, xn, nullptr, stream));
+    else {
+      const int64_t folded = dim % 1024 == 0 ? tail : 0;
+      if (R > folded) PF_DO(tga_rmsnorm_rows(x, an, (int)(R - folded), (int)dim, eps, xn, nullptr, 0, stream));
+      if (folded) { x16_fold_norm_kernel<<<(unsigned)folded, 1024, 0, s>>>(x + (R - folded) * dim, an, (int)dim, eps, xn + (R - folded) * dim); TGA_LAUNCH_CHECK(); }
+    }
+    { const int64_t wt[3] = {b[PB_WQ], b[PB_WK], b[PB_WV]}, n[3] = {nq, nk, nk}; float* const y[3] = {q, kk, v}; PF_DO(x16_linear(3, wt, y, n, xn, R, dim, nullptr, s)); }
+    X16Rope ra;
+    ra.q = q; ra.k = kk; ra.v = v; ra.qn = (const float*)b[PB_QN]; ra.kn = (const float*)b[PB_KN]; ra.rope = (const float*)m[PM_ROPE]; ra.qr = (float*)(ws + w.qr); ra.ck = (uint16_t*)b[PB_CK]; ra.cv = (uint16_t*)b[PB_CV];
+    ra.zero = (int*)(ws + w.counts); ra.n_zero = (int)E + 2; ra.H = (int)H; ra.KV = (int)KV; ra.hd = (int)hd; ra.max_ctx = (int)m[PM_MAXCTX]; ra.pos0 = (int)pos0; ra.eps = eps;
+    x16_rope_kernel<<<(unsigned)R, 256, 0, s>>>(ra);
+    TGA_LAUNCH_CHECK();
+    if (bi + 1 == m[PM_NBLOCKS]) break;                                   // the last block's keys and values are in the cache; what follows them there is read by nobody
+    X16Attn aa;
+    aa.qr = ra.qr; aa.ck = ra.ck; aa.cv = ra.cv; aa.part = (float*)(ws + w.part); aa.out = attn; aa.H = (int)H; aa.KV = (int)KV; aa.max_ctx = ra.max_ctx; aa.P = (int)P; aa.pos0 = (int)pos0; aa.nsplit = (int)nsplit;
+    aa.scale = 1.0f / sqrtf((float)hd);
+    const dim3 ag((unsigned)KV, (unsigned)nsplit, (unsigned)((P + X16_ROWS - 1) / X16_ROWS)), mg((unsigned)H, (unsigned)R);
+    if (hd == 64) x16_attn_kernel<8><<<ag, 256, 0, s>>>(aa); else x16_attn_kernel<16><<<ag, 256, 0, s>>>(aa);
+    TGA_LAUNCH_CHECK();
+    if (hd == 64) x16_merge_kernel<64><<<mg, 64, 0, s>>>(aa); else x16_merge_kernel<128><<<mg, 128, 0, s>>>(aa);
+    TGA_LAUNCH_CHECK();
+    { const int64_t wt[1] = {b[PB_WO]}, n[1] = {dim}; float* const y[1] = {x}; PF_DO(x16_linear(1, wt, y, n, attn, R, nq, x, s)); }
+    X16Router rt;
+    rt.x = x; rt.nw = (const float*)b[PB_FFN_NORM]; rt.wr = (const uint16_t*)b[PB_ROUTER]; rt.xs = (uint16_t*)(ws + w.xs); rt.logits = logits; rt.inf = inf; rt.R = (int)R; rt.dim = (int)dim; rt.E = (int)E; rt.eps = eps;
+    x16_router_kernel<2><<<(unsigned)((R + 1) / 2), 256, 0, s>>>(rt);
+    TGA_LAUNCH_CHECK();
+    PF_DO(pf_gate_group(logits, (int)R, (int)E, (int)k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), (int*)(ws + w.sel), probs, (int*)(ws + w.counts), (int*)(ws + w.place), 16, off,
+                        (int2*)(ws + w.tiles), (int*)(ws + w.ntiles), row_tok, row_dst, s));
+    X16Expert ea = {};
+    ea.off = off; ea.row_tok = row_tok; ea.row_dst = row_dst; ea.inf = inf;
+    ea.w[0] = (const uint8_t*)b[PB_GATE]; ea.w[1] = (const uint8_t*)b[PB_UP]; ea.x = rt.xs; ea.y = ws + w.act;
+    PF_DO(x16_experts<true>(ea, E, dim, hid, s));
+    ea.w[0] = (const uint8_t*)b[PB_DOWN]; ea.w[1] = nullptr; ea.x = (const uint16_t*)(ws + w.act); ea.y = ye; ea.inf = inf + 1;
+    PF_DO(x16_experts<false>(ea, E, hid, dim, s));
+  }
+#undef PF_DO
+  return 0;
+}
+
+}  // extern "C"

@@ -57,6 +57,7 @@ MANY_ROWS = 2048                   # rows of a prefill step at most (its buffers
 # Fewer rows are one step of the small-batch kernels.  Lockstep prompts, one step of many rows against so many lockstep steps (eight blocks of the 8B architecture, Q8_0 / Q4_0 / Q4_K_M): 16 sequences of two
 # positions 1079 against 1534 / 988 against 1336 / 1132 against 1619 us, 8 of three 1059 against 2038 / 956 against 1795 / 1129 against 2234, 4 of five 1018 against 3073 / 944 against 2655 / 1097 against 3349
 MANY_ROWS_MIN = 17
+ROWS16, ROWS16_MIN, ROWS16_BYTES = 1024, 16, 1 << 29     # prefill_rows16: rows of a step at most (a multiple of sixteen) and at least, bytes of its buffers from which on it takes fewer
 
 def precompute_freqs_cis(dim: int, end: int, theta: float) -> np.ndarray:
   """tinygrad/llm/model.py:16-19 in float32: cat(cos(pos * f), sin(pos * f)), f = 1 / theta^(2i/dim)."""
@@ -536,6 +537,10 @@ class Transformer:
     # only, so the same values are written again - instead of a ladder of smaller steps and up to three single ones (seven steps, a tenth of a 1023-position prefill).
     # MoE models keep the ladder (one step each of 8 and / or 4 positions, then single ones).
     overlap = not self.config.num_experts
+    # MoE models: the rows of the ladder's steps of sixteen, eight and four positions together, each with the bits its step gives it, where the model is in the range of tga_prefill16_step
+    if B == 16 and self.config.num_experts and len(tokens) - 1 - start >= ROWS16_MIN:
+      if self._chunker is None or self._chunker.batch != B: self._chunker = BatchedTransformer(self.config, self._state_dict, B, max_new=1, chunk_of=self)
+      start += self._chunker.prefill_rows16(tokens, start)
     for b in [B] + [t for t in (64, 32, 16, 8, 4) if t < B]:
       total = len(tokens) - 1 - start
       if not 2 <= b <= 128 or total < b: continue
@@ -748,6 +753,37 @@ class BatchedTransformer:
     self.state.copyin(st)
     self._owner_stream.synchronize()
     self._prefill_many_rows(np.array(tokens[start:start + n], np.int32)[None, :], start)
+    self.stream.synchronize()
+    self.check_state()
+    return n
+
+  def prefill_rows16(self, tokens: list[int], start: int) -> int:
+    """Chunked prefill for `chunk_of`, an MoE model: the rows of the steps of sixteen positions from start on, and of the one step each of eight and four behind them, all together and with the bits
+    of those steps (csrc/prefill16.hip).  Returns the number of positions done: none for models outside that kernel's range and where there is no memory for its buffers."""
+    c = self.config
+    if not self.chunked or self._rows_tables is None or self.expert_path != "jobs": return 0
+    if not (0 <= start < len(tokens) < c.max_context): raise ValueError(f"positions from {start} outside the prompt of {len(tokens)} tokens")
+    if min(tokens) < 0 or max(tokens) >= c.vocab_size: raise ValueError(f"token id outside the vocabulary of {c.vocab_size}")
+    total = len(tokens) - 1 - start
+    n, tail = total // 4 * 4, total // 4 * 4 % 16
+    ok, need = ctypes.c_int(0), ctypes.c_int64(0)
+    def plan(rows): rt.check(rt.lib().tga_prefill16_plan(*self._rows_tables, rows, start + n, ctypes.byref(ok), ctypes.byref(need))); return need.value
+    per = min(n, ROWS16)
+    while plan(per) > ROWS16_BYTES and per > 64: per = per // 32 * 16
+    if not ok.value: return 0
+    try:
+      if self._rows_ws is None or self._rows_ws.nbytes < need.value: self._rows_ws = Buffer((need.value,), np.uint8)
+      if self._rows_tok is None or self._rows_tok.nbytes < 4 * n: self._rows_tok = Buffer((4 * n,), np.uint8)
+    except RuntimeError as e:
+      if "HIP Error 2," not in str(e): raise
+      return 0
+    st = np.zeros(16, np.int32); st[0], st[3], st[5] = start, len(tokens), c.vocab_size
+    self.state.copyin(st)
+    self._rows_tok.view(0, (n,), np.int32).copyin(np.array(tokens[start:start + n], np.int32))
+    self._owner_stream.synchronize()
+    for i in range(0, n, per):
+      m = min(per, n - i)
+      rt.check(rt.lib().tga_prefill16_step(*self._rows_tables, self._rows_tok.ptr + 4 * i, m, max(0, m - max(0, n - tail - i)), start + i, self._rows_ws.ptr, self.state.ptr, self.stream.handle))
     self.stream.synchronize()
     self.check_state()
     return n
