@@ -10,7 +10,7 @@
 #include "qfmt.h"
 #include "prefill.h"
 #include "decode.h"
-#include <type_traits>
+#include <utility>
 
 typedef _Float16 v8f16 __attribute__((ext_vector_type(8)));
 typedef _Float16 v4f16 __attribute__((ext_vector_type(4)));
@@ -325,8 +325,8 @@ __global__ __launch_bounds__(HD) void x16_merge_kernel(const X16Attn a) {
 
 // ------------------------------------------------------------------------------------------------ ffn_norm and router logits
 // The arithmetic of moe_router_kernel, RT rows per workgroup: normalised once, the router's rows read once for all of them.  The normalised rows leave as the experts read them: the sixteen pairs
-// (value j, value j + 16) of a unit of 32 behind each other.  inf: set where a normalised value is not finite in fp16 (the experts' kernel then keeps products with padding apart).
-struct X16Router { const float* x; const float* nw; const uint16_t* wr; uint16_t* xs; float* logits; int* inf; int R, dim, E; float eps; };
+// (value j, value j + 16) of a unit of 32 behind each other.
+struct X16Router { const float* x; const float* nw; const uint16_t* wr; uint16_t* xs; float* logits; int R, dim, E; float eps; };
 template <int RT>
 __global__ __launch_bounds__(256) void x16_router_kernel(const X16Router a) {
   __shared__ __attribute__((aligned(16))) uint16_t xn[RT][2048];
@@ -361,17 +361,14 @@ __global__ __launch_bounds__(256) void x16_router_kernel(const X16Router a) {
     }
   }
   __syncthreads();
-  bool bad = false;
 #pragma unroll
   for (int t = 0; t < RT; t++)
     if (r0 + t < a.R)
       for (int d = tid; d < (a.dim >> 1); d += 256) {
         const int e = 32 * (d >> 4) + (d & 15);
         const uint32_t lo = xn[t][e], hi = xn[t][e + 16];
-        bad = bad || (lo & 0x7c00) == 0x7c00 || (hi & 0x7c00) == 0x7c00;
         ((uint32_t*)(a.xs + (size_t)(r0 + t) * a.dim))[d] = lo | (hi << 16);
       }
-  if (bad) *a.inf = 1;                                                     // (whoever writes it writes the same)
   for (int e = wave; e < a.E; e += 4) {
     const uint16_t* wrow = a.wr + (size_t)e * a.dim;
     u32x4 wv[4];
@@ -396,143 +393,234 @@ __global__ __launch_bounds__(256) void x16_router_kernel(const X16Router a) {
 // block's scale, then the tree over the units (pairs of neighbours first).  v_dot2_f32_f16 rounds the sum of two products and the addend once, and so does a matrix-core product whose other products
 // are zeros: v_mfma_f32_16x16x4_4b_f16 with two of its four values zero is 2048 dot2 in 32 cycles where the vector unit takes 256 (bits compared over normal, subnormal and huge values, sums
 // from zero and not; with all four values in use they differ, so the matrix cores run at a quarter of their fp16 rate here).
-// A workgroup owns 64 weight rows of one expert (SwiGLU: 32 of gate and the same 32 of up) and walks the expert's rows in tiles of sixteen; wave w holds units w UPW .. of the rows in registers for
-// the whole walk, so the weights are read once.  Lane 16 b + c supplies column c of block b; the sixteen rows of the tile are the other operand, the same for the four blocks.  The waves'
-// partial sums meet in LDS, where the upper levels of the tree are formed.
-// The zeros sit in the weight operand (the pair beside a weight pair).  Where a row holds values that are not finite (inf), the pair beside an activation pair is zero too: 0 x infinity would be NaN.
-struct X16Expert { const uint8_t* w[2]; const uint16_t* x; void* y; const int* off; const int* row_tok; const int* row_dst; int* inf; long long estride, row_bytes; int K, N, ngroups; };
+// An item is 64 weight rows of one expert (SwiGLU: 32 of gate and the same 32 of up) and all of the expert's rows, in tiles of sixteen.  Workgroups stay for the whole launch and share the tiles of all
+// items evenly, each a contiguous run of them (an item may be cut); wave w holds units 8 w .. of the item's weight rows in registers, so weights are read once per item, and touches those of the next item at
+// the first tile of this one (they wait in the XCD's L2; a second set of registers does not fit).  Lane 16 b + c supplies column c of block b; the sixteen rows of the tile are the other operand, the same for the four blocks, brought to LDS by requests of the wave itself,
+// two runs of four units ahead, across items.  The waves' partial sums meet in LDS, where the upper levels of the tree are formed.
+// The zeros sit in the weight operand (the pair beside a weight pair), so where a row holds an infinity its results are NaN, which the expert GEMV's are from the first zero weight on: of 2048 values
+// and more, behind the next norm the whole row is NaN either way.
+#define X16_RUN 4096                     // bytes of LDS for four units of a tile's sixteen rows
+struct X16Expert { const uint8_t* w[2]; const uint16_t* x; void* y; const int* off; const int2* tiles; const int* n_tiles; long long estride, row_bytes; int K, N, ngroups; };
 
-template <bool SW, int UPW>
-__global__ __launch_bounds__(512) void x16_expert_kernel(const X16Expert a) {
-  constexpr int ND = (17 * UPW + 3) / 4;                                   // dwords of a lane's run of a weight row
-  __shared__ float part[2][8][16][64];
-  const int e = blockIdx.x / a.ngroups, grp = blockIdx.x % a.ngroups;
-  const int first = a.off[e], cnt = a.off[e + 1] - first;
-  if (cnt <= 0) return;
+// (units as calls with constants: a loop is unrolled too late for its arrays to become registers)
+template <class F, int... I> __device__ __forceinline__ void x16_each(F& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+
+// NS: subtrees of eight units, the waves of a workgroup at most (a tree of 32 or 64 leaves)
+template <bool SW, int NS>
+__global__ __launch_bounds__(64 * NS, 2) void x16_expert_kernel(const X16Expert a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t ring[];           // [wave][3 runs][16 rows of 256 bytes]
+  __shared__ float part[NS][16][64];
+  __shared__ uint32_t touched[NS][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), blk = lane >> 4, c = lane & 15;
-  const int nw = blockDim.x >> 6;                                          // (K = 32 UPW nw)
-  const int col = SW ? grp * 32 + (blk & 1) * 16 + c : grp * 64 + lane;
-  uint32_t raw[ND];
-  {
-    const uint8_t* p = (SW && blk >= 2 ? a.w[1] : a.w[0]) + e * a.estride + (long long)col * a.row_bytes + 17 * UPW * wave;      // (4-byte aligned: K is a multiple of 256)
+  const int nw = blockDim.x >> 6;                                          // (K = 256 nw)
+  const int ntiles = *a.n_tiles;
+  // this workgroup's tiles: of the sequence (expert, item, tile) those from s0 on, neighbouring runs on one XCD
+  const long long total = (long long)ntiles * a.ngroups;
+  const unsigned nwg = gridDim.x, turn = (blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3);      // (nwg is a multiple of 8)
+  const int s0 = (int)(total * turn / nwg);
+  int left = (int)(total * (turn + 1) / nwg) - s0;
+  if (left <= 0) return;
+  struct Item { int e, grp, tf, nt, first, cnt; };                         // tf: the expert's first tile in the list
+  auto expert_at = [&](int tile, Item& it) __attribute__((always_inline)) {
+    it.e = a.tiles[tile].x; it.tf = tile - (a.tiles[tile].y >> 4); it.first = a.off[it.e]; it.cnt = a.off[it.e + 1] - it.first; it.nt = (it.cnt + 15) >> 4;
+  };
+  auto item_behind = [&](const Item& it) __attribute__((always_inline)) {
+    Item n = it;
+    if (it.grp + 1 < a.ngroups) n.grp = it.grp + 1;
+    else if (it.tf + it.nt < ntiles) { expert_at(it.tf + it.nt, n); n.grp = 0; }
+    return n;                                                              // (behind the last: the last again)
+  };
+  Item it, nx;
+  expert_at(s0 / a.ngroups, it);
+  int t = s0 - it.tf * a.ngroups;
+  it.grp = t / it.nt; t -= it.grp * it.nt;
+  nx = item_behind(it);
+  uint32_t raw[34];
+  auto weights_of = [&](const Item& i) __attribute__((always_inline)) {
+    const int col = SW ? i.grp * 32 + (blk & 1) * 16 + c : i.grp * 64 + lane;
+    return (SW && blk >= 2 ? a.w[1] : a.w[0]) + i.e * a.estride + (long long)col * a.row_bytes + 136 * wave;      // (4-byte aligned: K is a multiple of 256)
+  };
+  auto load = [&](const Item& i) __attribute__((always_inline)) {
+    const uint8_t* p = weights_of(i);
 #pragma unroll
-    for (int i = 0; i < ND / 4; i++) { const u32x4 v = ld16(p + 16 * i); raw[4 * i] = v.x; raw[4 * i + 1] = v.y; raw[4 * i + 2] = v.z; raw[4 * i + 3] = v.w; }
+    for (int q = 0; q < 8; q++) { const u32x4 v = ld16(p + 16 * q); raw[4 * q] = v.x; raw[4 * q + 1] = v.y; raw[4 * q + 2] = v.z; raw[4 * q + 3] = v.w; }
+    u32x2 v; __builtin_memcpy(&v, p + 128, 8); raw[32] = v.x; raw[33] = v.y;
+    __builtin_amdgcn_s_waitcnt(0x0f70);                                    // (vmcnt 0: what is counted behind it are requests into LDS and stores)
+  };
+  load(it);
+  uint8_t* rw = ring + wave * (3 * X16_RUN);
+  for (int w = nw + wave; w < NS; w += nw) {                               // (units beyond the row are zeros of the tree)
 #pragma unroll
-    for (int i = ND / 4 * 4; i < ND; i++) raw[i] = ld4(p + 4 * i);
+    for (int i = 0; i < 16; i++) part[w][i][lane] = 0.f;
   }
-  for (int w = nw + wave; w < 8; w += nw) {                                // (units beyond the row are zeros of the tree)
+  // a wave's request: its values of four units, 256 bytes of each of the tile's sixteen rows, four rows per instruction, pieces of 16 bytes XORed with the row
+  uint32_t src[4];
+  auto point = [&](const Item& i, int tile) __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int i = 0; i < 16; i++) part[b][w][i][lane] = 0.f;
-  }
-  const int ntile = (cnt + 15) >> 4;
-  u32x4 xq[2][4];
-  const uint16_t* xrow;
-  auto row_of = [&](int t) __attribute__((always_inline)) {
-    const int rr = first + min(16 * t + c, cnt - 1);
-    return a.x + (size_t)(SW ? a.row_tok[rr] : rr) * a.K + 32 * UPW * wave;
+    for (int q = 0; q < 4; q++) src[q] = (uint32_t)(i.first + min(16 * tile + 4 * q + blk, i.cnt - 1)) * (uint32_t)(2 * a.K) + 512 * wave + (((c ^ blk) ^ (4 * q)) << 4);
   };
-  auto fetch = [&](u32x4 (&d)[4], const uint16_t* p, int u) __attribute__((always_inline)) {
+  auto request = [&](int half, int slot) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) d[i] = *(const u32x4*)(p + 32 * u + 8 * i);
+    for (int q = 0; q < 4; q++)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((const char*)a.x + (src[q] + 256 * half)), (__attribute__((address_space(3))) void*)(rw + slot * X16_RUN + q * 1024), 16, 0, 0);
   };
-  xrow = row_of(0);
-  fetch(xq[0], xrow, 0);
-  const bool inf = *a.inf != 0;
-  u32x2 wz[16];
+  point(it, t);
+  request(0, 0); request(1, 1);
+  u32x4 x[2][4];
+  auto read_x = [&](u32x4 (&d)[4], int slot, int u) __attribute__((always_inline)) {
 #pragma unroll
-  for (int j = 0; j < 16; j++) wz[j] = u32x2{0u, 0u};
-  auto byte_dword = [&](int o) __attribute__((always_inline)) { return (o & 3) ? __builtin_amdgcn_alignbit(raw[(o >> 2) + 1], raw[o >> 2], 8 * (o & 3)) : raw[o >> 2]; };
-  // one unit: the chain, the scale
-  auto unit = [&](int u, const u32x4 (&x)[4], float (&leaf)[16], auto inf_tag) __attribute__((always_inline)) {
-    const int o = 17 * u;
-    const uint32_t eb = (raw[o >> 2] >> (8 * (o & 3))) & 0xffu;
-    const uint32_t s02 = eb ? (eb << 23) : 0x00400000u;
-    uint32_t q[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++) q[t] = byte_dword(o + 1 + 4 * t);
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      wz[4 * t + 0].x = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[t], 1.0f, 0));
-      wz[4 * t + 1].y = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[t], 1.0f, 1));
-      wz[4 * t + 2].x = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[t], 1.0f, 2));
-      wz[4 * t + 3].y = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(q[t], 1.0f, 3));
-    }
-    v16f32 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-      u32x2 xa = (j & 2) ? u32x2{x[j >> 2].z, x[j >> 2].w} : u32x2{x[j >> 2].x, x[j >> 2].y};
-      if constexpr (decltype(inf_tag)::value) xa = (j & 1) ? u32x2{0u, xa.y} : u32x2{xa.x, 0u};
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xa), __builtin_bit_cast(v4f16, wz[j]), acc, 0, 0, 0);
-    }
-    // the scales of the four blocks' column c
-    const auto h = __builtin_amdgcn_permlane32_swap(s02, s02, false, false);
-    const auto l0 = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false), l1 = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
-    const uint32_t su[4] = {l0[0], l0[1], l1[0], l1[1]};                  // (a bit cast of an element of such a pair takes the first)
-    const float sb[4] = {__builtin_bit_cast(float, su[0]), __builtin_bit_cast(float, su[1]), __builtin_bit_cast(float, su[2]), __builtin_bit_cast(float, su[3])};
-#pragma unroll
-    for (int i = 0; i < 16; i++) leaf[i] = __builtin_fmaf(sb[i >> 2], acc[i], 0.f);
+    for (int q = 0; q < 4; q++) d[q] = *(const u32x4*)(ring + (((uint32_t)(wave * 3 + slot) * X16_RUN + c * 272) ^ (64 * u + 16 * q)));      // (c * 256 + 16 c: the low eight bits are the row's)
   };
-  for (int t = 0; t < ntile; t++) {
-    const uint16_t* xnext = row_of(t + 1 < ntile ? t + 1 : t);
+  asm volatile("s_waitcnt vmcnt(4)" ::: "memory");                        // run 0 has landed
+  read_x(x[0], 0, 0);
+  // operands with their zero in place: pairs of even and of odd products
+  u32x2 we[2] = {u32x2{0u, 0u}, u32x2{0u, 0u}}, wo[2] = {u32x2{0u, 0u}, u32x2{0u, 0u}};
+#pragma unroll
+  for (int i = 0; i < 2; i++) asm volatile("" : "+v"(we[i]), "+v"(wo[i]));
+  int slot = 0;
+  bool fresh = true;                                                       // the first tile on these weights: the next item's are touched
+  for (;;) {
+    const bool same = t + 1 < it.nt;
     float st[3][16], leaf[16];                                             // sums of 1, 2 and 4 units that wait for their neighbour
-    auto walk = [&](auto tag) __attribute__((always_inline)) {
+    auto unit = [&](auto u_) __attribute__((always_inline)) {
+      constexpr int u = decltype(u_)::value;
+      const int nslot = slot == 2 ? 0 : slot + 1;
+      if constexpr (u == 0) { if (same) point(it, t + 1); else point(nx, 0); }
+      if constexpr (u % 4 == 0) request(u / 4, slot == 0 ? 2 : slot - 1);  // (the run after the next one goes where the one before this was read from)
+      if constexpr (u == 0) {
+        if (fresh) {                                                       // both ends of the lane's run, into LDS that nobody reads
+          const uint8_t* p = weights_of(nx);
 #pragma unroll
-      for (int u = 0; u < UPW; u++) {
-        if (u + 1 < UPW) fetch(xq[(u + 1) & 1], xrow, u + 1); else fetch(xq[(u + 1) & 1], xnext, 0);
-        unit(u, xq[u & 1], leaf, tag);
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-          float v = leaf[i];
-          if (u & 1) { v = st[0][i] + v; if (u & 2) { v = st[1][i] + v; if (u & 4) v = st[2][i] + v; else st[2][i] = v; } else st[1][i] = v; }
-          else st[0][i] = v;
-          if (u == UPW - 1) leaf[i] = v;
+          for (int z = 0; z < 2; z++) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p + 132 * z), (__attribute__((address_space(3))) void*)touched[wave], 4, 0, 0);
         }
       }
-    };
-    static_assert(UPW == 4 || UPW == 8, "whole subtrees");
-    if (inf) walk(std::true_type{}); else walk(std::false_type{});
-    xrow = xnext;
-    float (*pt)[16][64] = part[t & 1];
+      if constexpr (u % 4 == 3) {
+        // the next run has landed; behind it the run requested last and, at a first tile, the two touches may be on their way
+        if (fresh) asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        read_x(x[(u + 1) & 1], nslot, 0);
+      } else read_x(x[(u + 1) & 1], slot, (u & 3) + 1);
+      constexpr int o = 17 * u;
 #pragma unroll
-    for (int i = 0; i < 16; i++) pt[wave][i][lane] = leaf[i];
-    __syncthreads();                                                       // (the set of the tile before last is rewritten behind the next barrier only: its readers have passed this one)
+      for (int i = o / 4; i <= (o + 16) / 4; i++) asm volatile("" : "+v"(raw[i]));      // (decoded here and anew for every tile: decoded ahead, they do not fit the registers)
+      auto dword_at = [&](int b) __attribute__((always_inline)) { return (b & 3) ? __builtin_amdgcn_alignbit(raw[(b >> 2) + 1], raw[b >> 2], 8 * (b & 3)) : raw[b >> 2]; };
+      const uint32_t eb = (raw[o >> 2] >> (8 * (o & 3))) & 0xffu;
+      const uint32_t s02 = eb ? (eb << 23) : 0x00400000u;
+      v16f32 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const uint32_t w = dword_at(o + 1 + 4 * q);
+        const u32x2 xl = {x[u & 1][q].x, x[u & 1][q].y}, xh = {x[u & 1][q].z, x[u & 1][q].w};
+        we[0].x = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0));
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xl), __builtin_bit_cast(v4f16, we[0]), acc, 0, 0, 0);
+        wo[0].y = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1));
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xl), __builtin_bit_cast(v4f16, wo[0]), acc, 0, 0, 0);
+        we[1].x = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2));
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xh), __builtin_bit_cast(v4f16, we[1]), acc, 0, 0, 0);
+        wo[1].y = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3));
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xh), __builtin_bit_cast(v4f16, wo[1]), acc, 0, 0, 0);
+        asm volatile("" : "+v"(we[0]), "+v"(wo[0]), "+v"(we[1]), "+v"(wo[1]));     // (their other halves are no constants to the compiler, which set them anew for every product)
+      }
+      // the scales of the four blocks' column c
+      const auto h = __builtin_amdgcn_permlane32_swap(s02, s02, false, false);
+      const auto l0 = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false), l1 = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+      const uint32_t su[4] = {l0[0], l0[1], l1[0], l1[1]};                // (a bit cast of an element of such a pair takes the first)
+      const float sb[4] = {__builtin_bit_cast(float, su[0]), __builtin_bit_cast(float, su[1]), __builtin_bit_cast(float, su[2]), __builtin_bit_cast(float, su[3])};
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        float v = __builtin_fmaf(sb[i >> 2], acc[i], 0.f);
+        if constexpr (u & 1) { v = st[0][i] + v; if constexpr (u & 2) { v = st[1][i] + v; if constexpr (u & 4) leaf[i] = st[2][i] + v; else st[2][i] = v; } else st[1][i] = v; }
+        else st[0][i] = v;
+      }
+      if constexpr (u % 4 == 3) slot = nslot;
+    };
+    x16_each(unit, std::make_integer_sequence<int, 8>{});
+    // (barriers of their own: __syncthreads would wait for the requests in flight)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");         // everyone has summed the tile before
+#pragma unroll
+    for (int i = 0; i < 16; i++) part[wave][i][lane] = leaf[i];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     // register 4 b + i of lane l is row 4 (l / 16) + i of column l % 16 of block b
     for (int o = tid; o < 512; o += blockDim.x) {
-      const int l = o & 63, h = (o >> 6) & 1, i = o >> 7, row = 4 * (l >> 4) + i;
-      if (16 * t + row >= cnt) continue;
+      const int l = o & 63, h = (o >> 6) & 1, i = o >> 7, row = 16 * t + 4 * (l >> 4) + i, cc = l & 15;
+      if (row >= it.cnt) continue;
       float s[2];
 #pragma unroll
       for (int z = 0; z < 2; z++) {
         const int rg = 4 * (h + 2 * z) + i;
-        s[z] = ((pt[0][rg][l] + pt[1][rg][l]) + (pt[2][rg][l] + pt[3][rg][l])) + ((pt[4][rg][l] + pt[5][rg][l]) + (pt[6][rg][l] + pt[7][rg][l]));
+        s[z] = (part[0][rg][l] + part[1][rg][l]) + (part[2][rg][l] + part[3][rg][l]);
+        if constexpr (NS == 8) s[z] += (part[4][rg][l] + part[5][rg][l]) + (part[6][rg][l] + part[7][rg][l]);
       }
-      const int rr = first + 16 * t + row, cc = l & 15;
       if constexpr (SW) {
         float v = silu_f(s[0]) * s[1];
         asm volatile("" : "+v"(v));                                       // (rounded to float32 first, as there)
-        const uint32_t hb = __builtin_bit_cast(uint16_t, (_Float16)v);
-        if ((hb & 0x7c00) == 0x7c00) a.inf[1] = 1;
-        ((uint16_t*)a.y)[(size_t)rr * a.N + grp * 32 + 2 * cc + h] = (uint16_t)hb;
+        ((uint16_t*)a.y)[(size_t)(it.first + row) * a.N + it.grp * 32 + 2 * cc + h] = (uint16_t)f2h_bits(v);
       } else {
-        float* y = (float*)a.y + (size_t)a.row_dst[rr] * a.N + grp * 64 + cc;
+        float* y = (float*)a.y + (size_t)(it.first + row) * a.N + it.grp * 64 + cc;
         y[16 * h] = s[0]; y[16 * (h + 2)] = s[1];
       }
     }
+    if (--left == 0) break;
+    if (same) { t++; fresh = false; continue; }
+    t = 0; fresh = true; it = nx; nx = item_behind(it);
+    load(it);
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                        // (the last requests are read by nobody: they have arrived before the workgroup's LDS is given to another)
+}
+
+// The normalised rows in the order of the experts' rows
+__global__ __launch_bounds__(256) void x16_gather_kernel(const uint16_t* __restrict__ x, const int* __restrict__ row_tok, int K, uint16_t* __restrict__ out) {
+  const u32x4* s = (const u32x4*)(x + (size_t)row_tok[blockIdx.x] * K); u32x4* d = (u32x4*)(out + (size_t)blockIdx.x * K);
+  for (int i = threadIdx.x; i < (K >> 3); i += 256) d[i] = s[i];
+}
+
+// The weighted sum of a row's experts + residual and the norm behind it, as rmsnorm_kernel<true> (rows of at most 2048 values), over results in the order of the experts' rows
+__global__ __launch_bounds__(1024) void x16_combine_kernel(float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ probs, const int* __restrict__ sel, const int* __restrict__ place,
+                                                           const int* __restrict__ off, const float* __restrict__ w, int k, int dim, float eps, uint16_t* __restrict__ out) {
+  __shared__ float red[16];
+  __shared__ float pp[64]; __shared__ int at[64];
+  const int row = blockIdx.x, tid = threadIdx.x;
+  if (tid < k) { pp[tid] = probs[(size_t)row * k + tid]; at[tid] = off[sel[(size_t)row * k + tid]] + place[(size_t)row * k + tid]; }
+  __syncthreads();
+  x += (size_t)row * dim; out += (size_t)row * dim;
+  const int e0 = tid, e1 = tid + 1024;
+  auto value = [&](int e) {
+    float v = x[e];
+    for (int j0 = 0; j0 < k; j0 += 8) {
+      float yy[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) yy[i] = y[(size_t)at[j0 + i < k ? j0 + i : k - 1] * dim + e];
+#pragma unroll
+      for (int i = 0; i < 8; i++) if (j0 + i < k) v += pp[j0 + i] * yy[i];
+    }
+    x[e] = v;
+    return v;
+  };
+  float v0 = 0.f, v1 = 0.f, w0 = 0.f, w1 = 0.f;
+  if (e0 < dim) { v0 = value(e0); w0 = w[e0]; }
+  if (e1 < dim) { v1 = value(e1); w1 = w[e1]; }
+  float s = v0 * v0 + v1 * v1;
+  s = wave_sum(s);
+  if ((tid & 63) == 0) red[tid >> 6] = s;
+  __syncthreads();
+  float tot = 0.f;
+  for (int i = 0; i < 16; i++) tot += red[i];
+  const float scale = 1.0f / sqrtf(tot / (float)dim + eps);
+  float o0 = (v0 * scale) * w0, o1 = (v1 * scale) * w1;
+  asm volatile("" : "+v"(o0), "+v"(o1));
+  if (e0 < dim) out[e0] = (uint16_t)f2h_bits(o0);
+  if (e1 < dim) out[e1] = (uint16_t)f2h_bits(o1);
 }
 
 // ------------------------------------------------------------------------------------------------ the step
-struct X16Ws { size_t x, xn, q, k, v, qr, attn, part, logits, sel, probs, place, counts, off, tiles, ntiles, row_tok, row_dst, xs, act, y, inf, total; };
+struct X16Ws { size_t x, xn, q, k, v, qr, attn, part, logits, sel, probs, place, counts, off, tiles, ntiles, row_tok, row_dst, xs, xe, act, y, total; };
 static X16Ws x16_layout(const int64_t* m, int64_t R, int64_t nsplit) {
   X16Ws w = {}; size_t o = 0;
   auto take = [&](size_t n) { const size_t at = o; o += (n + 255) & ~(size_t)255; return at; };
   const int64_t dim = m[PM_DIM], nq = m[PM_HEADS] * m[PM_HD], nk = m[PM_KV] * m[PM_HD], E = m[PM_EXPERTS], k = m[PM_TOPK];
   w.x = take(R * dim * 4); w.xn = take(R * dim * 2); w.q = take(R * nq * 4); w.k = take(R * nk * 4); w.v = take(R * nk * 4); w.qr = take(R * nq * 4); w.attn = take(R * nq * 2);
   w.part = take(R * m[PM_HEADS] * nsplit * (m[PM_HD] + 2) * 4);
-  w.logits = take(R * E * 4); w.sel = take(R * k * 4); w.probs = take(R * k * 4); w.place = take(R * k * 4); w.counts = take((E + 2) * 4); w.inf = w.counts + E * 4; w.off = take((E + 1) * 4);
-  w.tiles = take((R * k / 16 + E + 1) * 8); w.ntiles = take(4); w.row_tok = take(R * k * 4); w.row_dst = take(R * k * 4); w.xs = take(R * dim * 2);
+  w.logits = take(R * E * 4); w.sel = take(R * k * 4); w.probs = take(R * k * 4); w.place = take(R * k * 4); w.counts = take(E * 4); w.off = take((E + 1) * 4);
+  w.tiles = take((R * k / 16 + E + 1) * 8); w.ntiles = take(4); w.row_tok = take(R * k * 4); w.row_dst = take(R * k * 4); w.xs = take(R * dim * 2); w.xe = take(R * k * dim * 2);
   w.act = take(R * k * m[PM_HIDDEN] * 2); w.y = take(R * k * dim * 4);
   w.total = o;
   return w;
@@ -564,13 +652,18 @@ static int x16_linear(int nseg, const int64_t* w, float* const* y, const int64_t
 }
 
 template <bool SW>
-static int x16_experts(const X16Expert& e, int64_t E, int64_t K, int64_t N, hipStream_t s) {
+static int x16_experts(const X16Expert& e, int64_t K, int64_t N, hipStream_t s) {
   X16Expert a = e;
   a.row_bytes = K / 32 * 17; a.estride = a.row_bytes * N; a.K = (int)K; a.N = (int)N; a.ngroups = (int)(SW ? N / 32 : N / 64);
-  // the tree has 64 leaves for rows of more than 32 units (qgemv1.h: a wave), else 32 (half a wave); eight subtrees either way
-  const int upw = K > 1024 ? 8 : 4;
-  const unsigned grid = (unsigned)(E * a.ngroups), nt = (unsigned)(K / 32 / upw * 64);
-  if (upw == 8) x16_expert_kernel<SW, 8><<<grid, nt, 0, s>>>(a); else x16_expert_kernel<SW, 4><<<grid, nt, 0, s>>>(a);
+  // The tree has 64 leaves for rows of more than 32 units (qgemv1.h: a wave), else 32 (half a wave).  Two workgroups of four waves per CU or one of eight
+  const int nw = (int)(K / 256), ns = nw > 4 ? 8 : 4;
+  auto kern = ns == 4 ? x16_expert_kernel<SW, 4> : x16_expert_kernel<SW, 8>;
+  static const hipError_t configured = [] {
+    const hipError_t r = hipFuncSetAttribute((const void*)x16_expert_kernel<SW, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 3 * X16_RUN);
+    return r != hipSuccess ? r : hipFuncSetAttribute((const void*)x16_expert_kernel<SW, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 8 * 3 * X16_RUN);
+  }();
+  TGA_HIP(configured);
+  kern<<<ns == 4 ? 512 : 256, 64 * nw, nw * 3 * X16_RUN, s>>>(a);
   TGA_LAUNCH_CHECK();
   return 0;
 }
@@ -588,12 +681,12 @@ int tga_prefill16_step(const int64_t* m, const int64_t* blocks, const int32_t* t
   TGA_REQUIRE(m && blocks && tokens && workspace && state && P >= 1 && tail >= 0 && tail <= P && pos0 >= 0 && pos0 + P <= m[PM_MAXCTX], "tga_prefill16_step: null pointer or rows beyond the cache");
   TGA_REQUIRE(prefill16_ok(m, blocks), "tga_prefill16_step: a model outside the range (tga_prefill16_plan says which are inside)");
   const int64_t R = P, dim = m[PM_DIM], H = m[PM_HEADS], KV = m[PM_KV], hd = m[PM_HD], nq = H * hd, nk = KV * hd, E = m[PM_EXPERTS], k = m[PM_TOPK], hid = m[PM_HIDDEN], nsplit = (pos0 + P + 63) / 64;
-  TGA_REQUIRE(R <= 4096 && R * k <= (1 << 20), "tga_prefill16_step: %lld rows are more than a step takes", (long long)R);
+  TGA_REQUIRE(R <= 4096 && R * k <= 65536, "tga_prefill16_step: %lld rows are more than a step takes", (long long)R);
   const X16Ws w = x16_layout(m, R, nsplit);
   uint8_t* ws = (uint8_t*)workspace;
   float* x = (float*)(ws + w.x); uint16_t* xn = (uint16_t*)(ws + w.xn); float* q = (float*)(ws + w.q); float* kk = (float*)(ws + w.k); float* v = (float*)(ws + w.v); uint16_t* attn = (uint16_t*)(ws + w.attn);
   float* logits = (float*)(ws + w.logits); float* probs = (float*)(ws + w.probs); float* ye = (float*)(ws + w.y); int* off = (int*)(ws + w.off);
-  int* row_tok = (int*)(ws + w.row_tok); int* row_dst = (int*)(ws + w.row_dst); int* inf = (int*)(ws + w.inf);
+  int* row_tok = (int*)(ws + w.row_tok); int* sel = (int*)(ws + w.sel); int* place = (int*)(ws + w.place); int2* tiles = (int2*)(ws + w.tiles); int* nt = (int*)(ws + w.ntiles);
   hipStream_t s = (hipStream_t)stream;
   const float eps = bits_f(m[PM_EPS_BITS]);
   int rc;
@@ -602,7 +695,7 @@ int tga_prefill16_step(const int64_t* m, const int64_t* blocks, const int32_t* t
   for (int64_t bi = 0; bi < m[PM_NBLOCKS]; bi++) {
     const int64_t* b = blocks + bi * PB_COUNT;
     const float* an = (const float*)b[PB_ATTN_NORM];
-    if (bi) PF_DO(tga_moe_combine_rmsnorm_rows(ye, probs, x, an, (int)R, (int)k, (int)dim, eps, xn, nullptr, stream));
+    if (bi) { x16_combine_kernel<<<(unsigned)R, 1024, 0, s>>>(x, ye, probs, sel, place, off, an, (int)k, (int)dim, eps, xn); TGA_LAUNCH_CHECK(); }
     else {
       const int64_t folded = dim % 1024 == 0 ? tail : 0;
       if (R > folded) PF_DO(tga_rmsnorm_rows(x, an, (int)(R - folded), (int)dim, eps, xn, nullptr, 0, stream));
@@ -611,7 +704,7 @@ int tga_prefill16_step(const int64_t* m, const int64_t* blocks, const int32_t* t
     { const int64_t wt[3] = {b[PB_WQ], b[PB_WK], b[PB_WV]}, n[3] = {nq, nk, nk}; float* const y[3] = {q, kk, v}; PF_DO(x16_linear(3, wt, y, n, xn, R, dim, nullptr, s)); }
     X16Rope ra;
     ra.q = q; ra.k = kk; ra.v = v; ra.qn = (const float*)b[PB_QN]; ra.kn = (const float*)b[PB_KN]; ra.rope = (const float*)m[PM_ROPE]; ra.qr = (float*)(ws + w.qr); ra.ck = (uint16_t*)b[PB_CK]; ra.cv = (uint16_t*)b[PB_CV];
-    ra.zero = (int*)(ws + w.counts); ra.n_zero = (int)E + 2; ra.H = (int)H; ra.KV = (int)KV; ra.hd = (int)hd; ra.max_ctx = (int)m[PM_MAXCTX]; ra.pos0 = (int)pos0; ra.eps = eps;
+    ra.zero = (int*)(ws + w.counts); ra.n_zero = (int)E; ra.H = (int)H; ra.KV = (int)KV; ra.hd = (int)hd; ra.max_ctx = (int)m[PM_MAXCTX]; ra.pos0 = (int)pos0; ra.eps = eps;
     x16_rope_kernel<<<(unsigned)R, 256, 0, s>>>(ra);
     TGA_LAUNCH_CHECK();
     if (bi + 1 == m[PM_NBLOCKS]) break;                                   // the last block's keys and values are in the cache; what follows them there is read by nobody
@@ -625,17 +718,19 @@ int tga_prefill16_step(const int64_t* m, const int64_t* blocks, const int32_t* t
     TGA_LAUNCH_CHECK();
     { const int64_t wt[1] = {b[PB_WO]}, n[1] = {dim}; float* const y[1] = {x}; PF_DO(x16_linear(1, wt, y, n, attn, R, nq, x, s)); }
     X16Router rt;
-    rt.x = x; rt.nw = (const float*)b[PB_FFN_NORM]; rt.wr = (const uint16_t*)b[PB_ROUTER]; rt.xs = (uint16_t*)(ws + w.xs); rt.logits = logits; rt.inf = inf; rt.R = (int)R; rt.dim = (int)dim; rt.E = (int)E; rt.eps = eps;
+    rt.x = x; rt.nw = (const float*)b[PB_FFN_NORM]; rt.wr = (const uint16_t*)b[PB_ROUTER]; rt.xs = (uint16_t*)(ws + w.xs); rt.logits = logits; rt.R = (int)R; rt.dim = (int)dim; rt.E = (int)E; rt.eps = eps;
     x16_router_kernel<2><<<(unsigned)((R + 1) / 2), 256, 0, s>>>(rt);
     TGA_LAUNCH_CHECK();
-    PF_DO(pf_gate_group(logits, (int)R, (int)E, (int)k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), (int*)(ws + w.sel), probs, (int*)(ws + w.counts), (int*)(ws + w.place), 16, off,
-                        (int2*)(ws + w.tiles), (int*)(ws + w.ntiles), row_tok, row_dst, s));
+    PF_DO(pf_gate_group(logits, (int)R, (int)E, (int)k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), sel, probs, (int*)(ws + w.counts), place, 16, off, tiles, nt, row_tok, (int*)(ws + w.row_dst), s));
+    uint16_t* xe = (uint16_t*)(ws + w.xe);
+    x16_gather_kernel<<<(unsigned)(R * k), 256, 0, s>>>(rt.xs, row_tok, (int)dim, xe);
+    TGA_LAUNCH_CHECK();
     X16Expert ea = {};
-    ea.off = off; ea.row_tok = row_tok; ea.row_dst = row_dst; ea.inf = inf;
-    ea.w[0] = (const uint8_t*)b[PB_GATE]; ea.w[1] = (const uint8_t*)b[PB_UP]; ea.x = rt.xs; ea.y = ws + w.act;
-    PF_DO(x16_experts<true>(ea, E, dim, hid, s));
-    ea.w[0] = (const uint8_t*)b[PB_DOWN]; ea.w[1] = nullptr; ea.x = (const uint16_t*)(ws + w.act); ea.y = ye; ea.inf = inf + 1;
-    PF_DO(x16_experts<false>(ea, E, hid, dim, s));
+    ea.off = off; ea.tiles = tiles; ea.n_tiles = nt;
+    ea.w[0] = (const uint8_t*)b[PB_GATE]; ea.w[1] = (const uint8_t*)b[PB_UP]; ea.x = xe; ea.y = ws + w.act;
+    PF_DO(x16_experts<true>(ea, dim, hid, s));
+    ea.w[0] = (const uint8_t*)b[PB_DOWN]; ea.w[1] = nullptr; ea.x = (const uint16_t*)(ws + w.act); ea.y = ye;
+    PF_DO(x16_experts<false>(ea, hid, dim, s));
   }
 #undef PF_DO
   return 0;
