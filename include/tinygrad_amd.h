@@ -39,6 +39,8 @@ extern "C" {
 const char* tga_last_error(void);
 int tga_init(int device);                                  /* hipSetDevice + kernel attribute set-up; ops_hip.py:14-20.  Also allocates, once per device, the 160 MB workspace of the 17 .. 128 row linears */
 int tga_device_name(char* buf, size_t len);
+int tga_host_malloc(void** ptr, size_t nbytes);            /* pinned host memory that kernels can write (hipHostMalloc) */
+int tga_host_free(void* ptr);
 int tga_malloc(void** ptr, size_t nbytes);                 /* ops_hip.py:60-62; served from freed blocks of the same size class where one is kept; refused while the thread captures a stream, whoever opened the capture (as hipMalloc is) */
 int tga_free(void* ptr);                                   /* ops_hip.py:63; keeps the block for later requests (at most 4 GiB per device, blocks of at most 1 GiB): it is handed out again only after a wait for the device; a block freed before is an error */
 int tga_trim(void);                                        /* gives every kept block back to the runtime; refused while the thread captures */
@@ -241,6 +243,10 @@ int tga_rmsnorm_qlinear_multi_touch(const float* norm_weight, float norm_eps, in
  * while state.pos + 1 < state.n_prompt the next input token is prompt[pos + 1]; otherwise the argmax token is stored at
  * out_tokens[state.step] and fed back.  scratch_v / scratch_i: 256 floats / 256 int32. */
 int tga_argmax_step(const float* logits, int n, float* scratch_v, int* scratch_i, void* state, const int* prompt, int* out_tokens, int max_tokens, void* stream);
+/* The same, and the next token and state.error also go to host[0], host[1] (pinned memory of tga_host_malloc: readable once the stream has been waited for). */
+int tga_argmax_step_host(const float* logits, int n, float* scratch_v, int* scratch_i, void* state, const int* prompt, int* out_tokens, int max_tokens, int* host, void* stream);
+/* The decode record of a sequence that starts at position pos with this input token (every other field 0), in stream order. */
+int tga_decode_begin(void* state, int pos, int token, int n_prompt, int vocab, void* stream);
 /* prompt step that skips the output projection: token = prompt[pos + 1], pos += 1. */
 int tga_advance_prompt(void* state, const int* prompt, void* stream);
 

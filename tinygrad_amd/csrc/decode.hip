@@ -837,7 +837,7 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(const float* __rest
 // Final reduce and the loop bookkeeping of Transformer.generate (tinygrad/llm/model.py:475-484) kept on the device: while
 // prompt tokens remain the next input is prompt[pos + 1]; afterwards the argmax token is appended to out_tokens and fed back.
 __global__ __launch_bounds__(256) void argmax_final_kernel(const float* __restrict__ pv, const int* __restrict__ pi, int np, DecodeState* st,
-                                                           const int* __restrict__ prompt, int* __restrict__ out_tokens, int max_tokens) {
+                                                           const int* __restrict__ prompt, int* __restrict__ out_tokens, int max_tokens, int* host) {
   __shared__ float sv[256]; __shared__ int si[256];
   float best = -INFINITY; int bi = 0;
   for (int i = threadIdx.x; i < np; i += 256) {
@@ -862,7 +862,13 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const float* __restri
       st->token = tok; st->step += 1;
     }
     st->pos = next;
+    if (host) { host[0] = st->token; host[1] = st->error; }               // (pinned host memory: what the loop reads of a step costs no copy)
   }
+}
+// The record of a sequence that starts at pos with this token (arguments instead of a copy from the host: 15 us of it per sequence)
+__global__ void decode_begin_kernel(int* st, int pos, int token, int n_prompt, int vocab) {
+  const int i = threadIdx.x;
+  st[i] = i == 0 ? pos : i == 1 ? token : i == 3 ? n_prompt : i == 5 ? vocab : 0;
 }
 // Prompt step without sampling (no lm-head was run): feed prompt[pos + 1] and advance.
 __global__ void advance_prompt_kernel(DecodeState* st, const int* __restrict__ prompt) {
@@ -1178,13 +1184,23 @@ int tga_attention_decode(const float* q, const float* k, const float* v, void* c
                                      out_f16, out_f32, stage_type, stream);
 }
 
-int tga_argmax_step(const float* logits, int n, float* scratch_v, int* scratch_i, void* state, const int* prompt, int* out_tokens, int max_tokens, void* stream) {
+int tga_argmax_step_host(const float* logits, int n, float* scratch_v, int* scratch_i, void* state, const int* prompt, int* out_tokens, int max_tokens, int* host, void* stream) {
   TGA_REQUIRE(logits && scratch_v && scratch_i && state && prompt, "tga_argmax_step: null pointer");
   TGA_REQUIRE(n > 0, "tga_argmax_step: n=%d", n);
   const int np = 256;
   argmax_partial_kernel<<<np, 256, 0, (hipStream_t)stream>>>(logits, n, scratch_v, scratch_i);
   TGA_LAUNCH_CHECK();
-  argmax_final_kernel<<<1, 256, 0, (hipStream_t)stream>>>(scratch_v, scratch_i, np, (DecodeState*)state, prompt, out_tokens, max_tokens);
+  argmax_final_kernel<<<1, 256, 0, (hipStream_t)stream>>>(scratch_v, scratch_i, np, (DecodeState*)state, prompt, out_tokens, max_tokens, host);
+  TGA_LAUNCH_CHECK();
+  return 0;
+}
+int tga_argmax_step(const float* logits, int n, float* scratch_v, int* scratch_i, void* state, const int* prompt, int* out_tokens, int max_tokens, void* stream) {
+  return tga_argmax_step_host(logits, n, scratch_v, scratch_i, state, prompt, out_tokens, max_tokens, nullptr, stream);
+}
+
+int tga_decode_begin(void* state, int pos, int token, int n_prompt, int vocab, void* stream) {
+  TGA_REQUIRE(state, "tga_decode_begin: null pointer");
+  decode_begin_kernel<<<1, 16, 0, (hipStream_t)stream>>>((int*)state, pos, token, n_prompt, vocab);
   TGA_LAUNCH_CHECK();
   return 0;
 }

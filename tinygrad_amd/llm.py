@@ -359,6 +359,7 @@ class _Shared:
     self.rope = Buffer.from_numpy(rope_table(c.head_dim, c.rope_dim or c.head_dim, c.max_context, c.rope_theta))
     self.prompt = Buffer((c.max_context,), np.int32).zero_()
     self.out_tokens = Buffer((max(1, max_new),), np.int32).zero_()
+    self.host = rt.HostInts(16)                                          # the last decode step's token and state.error, written by its last launch
 
 class Transformer:
   def __init__(self, config: TransformerConfig, state_dict: dict, max_new: int = 4096):
@@ -416,7 +417,7 @@ class Transformer:
       else:
         rt.check(L.tga_rmsnorm(x.ptr, self.output_norm.ptr, c.dim, c.norm_eps, s.xn.ptr, None, 0, st))
         self.output(s.xn, out=s.logits, stream=st)
-      rt.check(L.tga_argmax_step(s.logits.ptr, c.vocab_size, s.am_v.ptr, s.am_i.ptr, s.state.ptr, s.prompt.ptr, s.out_tokens.ptr, self.max_new, st))
+      rt.check(L.tga_argmax_step_host(s.logits.ptr, c.vocab_size, s.am_v.ptr, s.am_i.ptr, s.state.ptr, s.prompt.ptr, s.out_tokens.ptr, self.max_new, s.host.ptr, st))
     else:
       rt.check(L.tga_advance_prompt(s.state.ptr, s.prompt.ptr, st))
 
@@ -497,6 +498,8 @@ class Transformer:
   def get_start_pos(self, tokens: list[int]) -> int:
     """How many leading positions of the KV cache can be kept for this prompt (Transformer.get_start_pos, model.py:455-462): the longest common
     prefix of tokens[:-1] and the tokens whose keys and values the cache holds."""
+    n = min(len(tokens) - 1, len(self._cached_tokens))
+    if n > 0 and isinstance(tokens, list) and tokens[:n] == self._cached_tokens[:n]: return n
     n = 0
     for a, b in zip(tokens[:-1], self._cached_tokens):
       if a != b: break
@@ -509,12 +512,15 @@ class Transformer:
     if not 1 <= len(tokens) < c.max_context: raise ValueError(f"prompt of {len(tokens)} tokens does not fit max_context {c.max_context}")
     if min(tokens) < 0 or max(tokens) >= c.vocab_size: raise ValueError(f"token id outside the vocabulary of {c.vocab_size}")
     if not 0 <= start_pos < len(tokens): raise ValueError(f"start position {start_pos} outside the prompt of {len(tokens)} tokens")
-    prompt = np.zeros(c.max_context, dtype=np.int32); prompt[:len(tokens)] = tokens
-    s.prompt.copyin(prompt)
-    st = np.zeros(16, dtype=np.int32); st[0], st[1], st[3], st[5] = start_pos, tokens[start_pos], len(tokens), c.vocab_size
-    s.state.copyin(st)
-    self._n_prompt, self._steps_done = len(tokens), start_pos
     self._cached_tokens = list(tokens[:start_pos])
+    self._start(tokens, start_pos)
+
+  def _start(self, tokens: list[int], start_pos: int):
+    """reset() behind its checks, with the list of cached tokens already cut to start_pos."""
+    c, s = self.config, self.s
+    if start_pos < len(tokens) - 1: s.prompt.view(0, (len(tokens),), np.int32).copyin(np.array(tokens, dtype=np.int32))     # (nothing reads the prompt from its last token on)
+    rt.check(rt.lib().tga_decode_begin(s.state.ptr, start_pos, int(tokens[start_pos]), len(tokens), c.vocab_size, self.stream.handle))
+    self._n_prompt, self._steps_done = len(tokens), start_pos
 
   def prefill(self, tokens: list[int], use_graph: bool = True, reuse_cache: bool = True, on_block=None):
     """Feeds all but the last prompt token (KV cache fill); the last one is consumed by the first decode step.  Like the reference's generate
@@ -522,7 +528,8 @@ class Transformer:
     on_block(i) after the launches of block i of every position (see _step)."""
     start = self.get_start_pos(tokens) if reuse_cache else 0
     self.prefill_steps = len(tokens) - 1 - start                        # (positions the last call actually computed)
-    self._cached_tokens = self._cached_tokens[:start]                   # the rows from here on are about to be overwritten: if a step below raises, they are not claimed
+    reused = start
+    del self._cached_tokens[start:]                                     # the rows from here on are about to be overwritten: if a step below raises, they are not claimed
     B = self.prefill_chunk if on_block is None else 1
     # From MANY_ROWS_MIN positions on, and with the chunk size left at its largest, the positions are steps of many rows: one pass over the weights for (nearly) any prompt
     n_rows = len(tokens) - 1 - start
@@ -554,14 +561,18 @@ class Transformer:
       if overlap:
         if start < len(tokens) - 1: chunker.prefill_chunks(tokens, len(tokens) - 1 - b, 1, use_graph); start = len(tokens) - 1
         break
-    self.reset(tokens, start)
+    # (reset()'s checks; the reused tokens are ones that have passed them)
+    if not 1 <= len(tokens) < self.config.max_context: raise ValueError(f"prompt of {len(tokens)} tokens does not fit max_context {self.config.max_context}")
+    rest = tokens[reused:] if reused else tokens
+    if min(rest) < 0 or max(rest) >= self.config.vocab_size: raise ValueError(f"token id outside the vocabulary of {self.config.vocab_size}")
+    self._start(tokens, start)
     for _ in range(len(tokens) - 1 - start):
       if use_graph and on_block is None: self._graph(False).launch()
       else: self._step(False, on_block)
     self._steps_done = len(tokens) - 1
-    self._cached_tokens = list(tokens[:-1])
+    if len(self._cached_tokens) != len(tokens) - 1: self._cached_tokens = list(tokens[:-1])
     self._last_input = tokens[-1]
-    self.stream.synchronize()
+    if start < len(tokens) - 1: self.stream.synchronize()
 
   def decode_step(self, use_graph: bool = True, sync: bool = True, on_block=None):
     """One token.  The position it occupies must exist in the KV cache and the rotation table: like the reference's generate loop
@@ -577,12 +588,13 @@ class Transformer:
     """Greedy decoding (temperature 0): yields one token id per step, like Transformer.generate (model.py:464-484), and like it stops when
     the context is full (model.py:475)."""
     self.prefill(tokens, use_graph)
+    err = 1                                                             # (no step: the record itself is read)
     for i in range(min(max_new_tokens, self.config.max_context - len(tokens), self.max_new)):
       self.decode_step(use_graph, sync=True)                          # the reference syncs once per token too (out.item(), model.py:482)
-      tok = int(self.s.out_tokens.view(4 * i, (1,), np.int32).numpy()[0])
+      tok, err = self.s.host.values[0], self.s.host.values[1]
       self._last_input = tok                                          # (model.py:483: the cache then holds tokens[:-1])
       yield tok
-    self.check_state()
+    if err: self.check_state()                                          # (the last step has written the flags of all before it)
 
   def logits(self) -> np.ndarray: return self.s.logits.numpy().reshape(-1)
 
@@ -645,12 +657,14 @@ class BatchedTransformer:
         b["cache_k"] = Buffer((B, c.n_kv_heads, c.max_context, c.head_dim), f16).zero_()
         b["cache_v"] = Buffer((B, c.n_kv_heads, c.max_context, c.head_dim), f16).zero_()
       self.blk.append(b)
-    self.state = Buffer((16,), np.int32).zero_()
-    self.tokens = Buffer((B,), np.int32).zero_()
+    # state | tokens | prompts in one allocation: a batch of prompts starts with one copy
+    nt, np_ = (B + 15) // 16 * 16, (B if chunk_of is None else 1) * c.max_context
+    self._io = Buffer((16 + nt + np_,), np.int32).zero_()
+    self.state, self.tokens = self._io.view(0, (16,), np.int32), self._io.view(64, (B,), np.int32)
+    self.prompts = self._io.view(64 + 4 * nt, (B if chunk_of is None else 1, c.max_context), np.int32)
     if c.num_experts: self.job_flags = Buffer((1,), np.int32).zero_()
     self.logits_buf = Buffer((B, c.vocab_size), f32) if chunk_of is None else None
     self.rope = Buffer.from_numpy(rope_table(c.head_dim, c.rope_dim or c.head_dim, c.max_context, c.rope_theta)) if chunk_of is None else chunk_of.s.rope
-    self.prompts = Buffer((B if chunk_of is None else 1, c.max_context), np.int32).zero_()
     self.out_tokens = Buffer((max(1, max_new), B), np.int32).zero_()
     self.stream = rt.Stream()
     self._graphs, self._steps_done = {}, 0
@@ -951,15 +965,16 @@ class BatchedTransformer:
     if len(prompts) != B or any(len(p) != n for p in prompts): raise ValueError(f"need {B} prompts of equal length")
     if not 1 <= n < c.max_context: raise ValueError(f"prompt of {n} tokens does not fit max_context {c.max_context}")
     if min(map(min, prompts)) < 0 or max(map(max, prompts)) >= c.vocab_size: raise ValueError(f"token id outside the vocabulary of {c.vocab_size}")
-    pr = np.zeros((B, c.max_context), np.int32); pr[:, :n] = np.array(prompts, np.int32)
-    self.prompts.copyin(pr)
+    io = np.zeros(self._io.shape, np.int32)
+    st, pr = io[:16], io[16 + (B + 15) // 16 * 16:].reshape(B, c.max_context)
+    pr[:, :n] = np.array(prompts, np.int32)
     # all but the last position of every prompt: as steps of many rows (sequences x positions) where the model is in their range and there are rows enough, else step by step
     many = self.many_rows and self._rows_tables is not None and on_block is None and B * (n - 1) >= MANY_ROWS_MIN and self.expert_path == "jobs"     # (a chosen expert path runs every step)
     many = many and self._rows_reserve(B, n - 1)
     done = n - 1 if many else 0
-    self.tokens.copyin(np.ascontiguousarray(pr[:, done]))
-    st = np.zeros(16, np.int32); st[0], st[3], st[5] = done, n, c.vocab_size
-    self.state.copyin(st)
+    st[0], st[3], st[5] = done, n, c.vocab_size
+    io[16:16 + B] = pr[:, done]
+    self._io.copyin(io)
     if many: self._prefill_many_rows(pr[:, :n - 1], 0)
     for _ in range(n - 1 - done):
       if use_graph and on_block is None: self._graph(False).launch()

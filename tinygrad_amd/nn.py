@@ -2,7 +2,7 @@
 that stays in its packed GGUF block layout.  The weight operand is the raw tensor byte range from the GGUF file buffer
 (tinygrad/llm/gguf.py:144-148: rows = out_features, quant blocks along in_features); nothing is repacked or dequantized to memory."""
 from __future__ import annotations
-import ctypes
+import ctypes, math
 import numpy as np
 from tinygrad_amd import runtime as rt
 from tinygrad_amd.runtime import Buffer, GGML_QUANT
@@ -23,7 +23,7 @@ class QuantLinear:
   def __call__(self, x: Buffer, out: Buffer | None = None, out_dtype=None, stream=None) -> Buffer:
     """x: (..., in_features) float16 or float32 with at most 8 rows (up to 16 for prefill chunks).  Returns (rows, out_features); the caller may pass `out`."""
     assert x.shape[-1] == self.in_features, f"{x.shape} vs in_features {self.in_features}"
-    m = int(np.prod(x.shape[:-1], dtype=np.int64)) if len(x.shape) > 1 else 1
+    m = x.shape[0] if len(x.shape) == 2 else math.prod(x.shape[:-1])
     assert 1 <= m <= 128, f"batch of {m} rows is outside the range 1..128"
     if out is None: out = Buffer((*x.shape[:-1], self.out_features), out_dtype or x.dtype)
     assert out.nbytes == m * self.out_features * out.dtype.itemsize

@@ -3,7 +3,7 @@
 Mirrors the reference's HIP device glue (tinygrad/runtime/ops_hip.py:9-70): a non-zero status becomes RuntimeError with the
 library's message, buffers are explicit device allocations owned by the Python side."""
 from __future__ import annotations
-import ctypes, os, pathlib
+import ctypes, math, os, pathlib
 import numpy as np
 
 F32, F16, Q4_0, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4 = 0, 1, 2, 8, 12, 13, 14, 39
@@ -90,6 +90,8 @@ def _declare(lib):
     "tga_attention_decode_split": [vp, vp, vp, vp, vp, vp, vp, i, i, i, i, vp, vp],
     "tga_attention_decode_split_normed": [vp, vp, vp, vp, vp, ctypes.c_float, i, vp, vp, vp, vp, i, i, i, i, vp, vp],
     "tga_attn_merge_qlinear": [i, vp, vp, i64, i64, vp, vp, i, i, vp],
+    "tga_argmax_step_host": [vp, i, vp, vp, vp, vp, vp, i, vp, vp], "tga_decode_begin": [vp, i, i, i, i, vp],
+    "tga_host_malloc": [ctypes.POINTER(vp), ctypes.c_size_t], "tga_host_free": [vp],
     "tga_argmax_step": [vp, i, vp, vp, vp, vp, vp, i, vp],
     "tga_advance_prompt": [vp, vp, vp],
     "tga_copy_kernel": [vp, vp, ctypes.c_size_t, vp],
@@ -133,9 +135,9 @@ def synchronize() -> None: check(lib().tga_sync())
 class Buffer:
   """A device allocation plus the (shape, dtype) the host side attaches to it.  dtype is a numpy dtype."""
   def __init__(self, shape, dtype=np.uint8, ptr: int | None = None, owner=None):
-    self.shape = tuple(int(s) for s in (shape if isinstance(shape, (tuple, list)) else (shape,)))
+    self.shape = tuple(map(int, shape)) if isinstance(shape, (tuple, list)) else (int(shape),)
     self.dtype = np.dtype(dtype)
-    self.nbytes = int(np.prod(self.shape, dtype=np.int64)) * self.dtype.itemsize
+    self.nbytes = math.prod(self.shape) * self.dtype.itemsize
     self._owner = owner
     if ptr is None:
       p = ctypes.c_void_p()
@@ -174,6 +176,15 @@ class Buffer:
   def zero_(self, stream=None) -> "Buffer":
     if self.nbytes: check(lib().tga_memset(self.ptr, 0, self.nbytes, stream))
     return self
+
+class HostInts:
+  """n pinned int32 that kernels write and the host reads without a copy (once the stream that ran them has been waited for)."""
+  def __init__(self, n: int):
+    p = ctypes.c_void_p(); check(lib().tga_host_malloc(ctypes.byref(p), 4 * n)); self.ptr = p.value
+    self.values = (ctypes.c_int32 * n).from_address(self.ptr)
+    for j in range(n): self.values[j] = 0
+  def __del__(self):
+    if getattr(self, "ptr", None) and _lib is not None: _lib.tga_host_free(ctypes.c_void_p(self.ptr)); self.ptr = None
 
 class Stream:
   def __init__(self):
@@ -235,8 +246,12 @@ class CommandList:
   def __del__(self):
     if getattr(self, "handle", None) and _lib is not None: _lib.tga_cmdlist_destroy(ctypes.c_void_p(self.handle)); self.handle = None
 
+_CODES: dict = {}                                             # (filled below: the codes of the two activation types, by dtype)
 def dtype_code(dt) -> int:
+  c = _CODES.get(dt)
+  if c is not None: return c
   dt = np.dtype(dt)
   if dt == np.float32: return F32
   if dt == np.float16: return F16
   raise TypeError(f"unsupported activation dtype {dt}")
+_CODES.update({np.dtype(np.float32): F32, np.dtype(np.float16): F16})
