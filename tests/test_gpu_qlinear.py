@@ -531,6 +531,27 @@ def test_sixteen_and_more_rows_segments_residual_and_swiglu(gpu, m):
     a, b = refs[1], ol.linear_f64(x.astype(np.float32), ol.weight_f32(g[1].blocks.numpy(), ns[1], k, t))
     assert ol.rel_err(out.numpy(), a / (1 + np.exp(-a)) * b) <= TOL, (t, k)
 
+@pytest.mark.parametrize("n,k,m,f32", [(16, 4096, 3, False), (16, 2048, 16, True), (4112, 4096, 16, False), (4112, 2048, 5, True), (12304, 4096, 9, True), (12304, 2048, 8, False), (20480, 4096, 4, False)])
+def test_small_batch_of_superblocks_that_start_off_a_piece(gpu, n, k, m, f32):
+  """Q6_K on the wave-private rings (qgemm_wp.hip), a step of a wave at a time: one row group, one workgroup with a group more than the others (2 or 1 ring positions per group, so rings that
+  never fill and rings that wrap), the plain and the residual epilogue, against the float64 anchor; twice, to see that a launch leaves nothing behind."""
+  from tinygrad_amd.nn import QuantLinear, qlinear_multi
+  rng = np.random.default_rng(5 + n + k + m)
+  w = synth.random_blocks(rng, 14, n, k)
+  x = synth.activations(rng, m, k, np.float32 if f32 else np.float16)
+  ref = ol.linear_f64(x.astype(np.float16).astype(np.float32), ol.weight_f32(w, n, k, 14))       # (the kernel rounds float32 rows to fp16 operands)
+  lin = QuantLinear(gpu.Buffer.from_numpy(w), 14, n, k)
+  xb = gpu.Buffer.from_numpy(x)
+  for rep in range(2):
+    out = gpu.Buffer((m, n), np.float32)
+    gpu.check(gpu.lib().tga_memset(out.ptr, 0xFF, out.nbytes, None))
+    lin(xb, out=out)
+    assert ol.rel_err(out.numpy(), ref) <= TOL, rep
+    res = rng.standard_normal((m, n)).astype(np.float32)
+    rb = gpu.Buffer.from_numpy(res)
+    qlinear_multi([lin], xb, [rb], epilogue=1, resid=[rb])
+    assert ol.rel_err(rb.numpy(), res + ref) <= TOL, rep
+
 @pytest.mark.parametrize("t,k,m,f32", [(8, 4096, 2, False), (8, 4096, 3, True), (8, 2048, 5, False), (8, 4096, 8, True), (8, 2048, 9, True), (8, 4096, 13, False), (8, 4096, 16, True), (8, 2048, 16, False),
                                        (1, 2048, 2, False), (1, 2048, 4, True), (1, 2048, 8, False), (1, 2048, 11, True), (1, 2048, 16, False),
                                        (2, 4096, 8, False), (2, 2048, 16, True), (12, 4096, 6, True), (12, 2048, 16, False), (13, 4096, 8, False), (13, 2048, 3, True),

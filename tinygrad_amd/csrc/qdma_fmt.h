@@ -70,6 +70,7 @@ template <> struct DmaFmt<GGML_Q6_K> {
   static constexpr int PAD = 2;                          // pitches of 107 and 55 pieces = 428 and 220 dwords = 44 and 28 mod 64: sixteen rows on sixteen different bank quads
   // Slots of 16 units (K beyond 4096, an even number of slots): 4 superblocks = 840 bytes start 8 bytes off a 16-byte boundary in every second slot.  A stage
   // (1680 bytes of a row) is fetched as two windows of 53 aligned pieces, [0, 848) and [832, 1680): the second slot's units start 8 bytes into its window.
+  static constexpr int slot_bytes(int su) { return su / 4 * 210; }
   static constexpr int pieces(int su) { return su == 32 ? 105 : 53; }
   static constexpr int second_off(int su) { return su == 32 ? 1680 : 832; }
   static constexpr int stage_stride(int su) { return su / 4 * 210 * 2; }

@@ -84,6 +84,9 @@ __device__ __forceinline__ half2_t h2_splat_f(float f) { const _Float16 v = (_Fl
 // A constant the compiler must keep in a VGPR: VOP3 forms such as v_and_or_b32 / v_perm_b32 accept a single scalar
 // operand and no literal on this ISA, so (x & MASK) | BIAS only becomes one instruction when BIAS already lives in a VGPR.
 __device__ __forceinline__ uint32_t vgpr_const(uint32_t c) { asm("" : "+v"(c)); return c; }
+// (a & m) | c as one instruction, the mask in a scalar register (sgpr_const): of a chain of two the compiler makes two ands and an or3
+__device__ __forceinline__ uint32_t sgpr_const(uint32_t c) { asm("" : "+s"(c)); return c; }
+__device__ __forceinline__ uint32_t and_or_s(uint32_t a, uint32_t m, uint32_t c) { uint32_t o; asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(o) : "v"(a), "s"(m), "v"(c)); return o; }
 
 // ------------------------------------------------------------------------------------------------ Q4_0 (gguf.py:46)
 template <> struct Fmt<GGML_Q4_0> {
@@ -449,21 +452,21 @@ template <> struct Fmt<GGML_Q6_K> {
     return 256 * (u >> 2) + 128 * ((u >> 1) & 1) + 32 * (k >> 3) + 16 * (u & 1) + 2 * (k & 7);
   }
   // wv[8j + 2t + {0,1}] = even / odd pairs of dword t of group j; value 1024 + 6-bit q
-  static constexpr int NKC = 1;
-  static __device__ __forceinline__ void consts(uint32_t* kc) { kc[0] = vgpr_const(0x64006400u); }
+  static constexpr int NKC = 3;
+  static __device__ __forceinline__ void consts(uint32_t* kc) { kc[0] = vgpr_const(0x64006400u); kc[1] = sgpr_const(0x000F000Fu); kc[2] = sgpr_const(0x00300030u); }
   static __device__ __forceinline__ void decode(const Raw& r, uint32_t* wv, const uint32_t* kc) {
-    const uint32_t K64 = kc[0];
+    const uint32_t K64 = kc[0], LO = kc[1], HI = kc[2];
 #pragma unroll
     for (int t = 0; t < 4; t++) {
       const uint32_t A = r.a[t], B = r.b[t], H = r.h[t];
-      wv[0 + 2 * t]      = and_or(H << 4, 0x00300030u, and_or(A, 0x000F000Fu, K64));
-      wv[0 + 2 * t + 1]  = and_or(H >> 4, 0x00300030u, and_or(A >> 8, 0x000F000Fu, K64));
-      wv[8 + 2 * t]      = and_or(H << 2, 0x00300030u, and_or(B, 0x000F000Fu, K64));
-      wv[8 + 2 * t + 1]  = and_or(H >> 6, 0x00300030u, and_or(B >> 8, 0x000F000Fu, K64));
-      wv[16 + 2 * t]     = and_or(H, 0x00300030u, and_or(A >> 4, 0x000F000Fu, K64));
-      wv[16 + 2 * t + 1] = and_or(H >> 8, 0x00300030u, and_or(A >> 12, 0x000F000Fu, K64));
-      wv[24 + 2 * t]     = and_or(H >> 2, 0x00300030u, and_or(B >> 4, 0x000F000Fu, K64));
-      wv[24 + 2 * t + 1] = and_or(H >> 10, 0x00300030u, and_or(B >> 12, 0x000F000Fu, K64));
+      wv[0 + 2 * t]      = and_or_s(H << 4, HI, and_or_s(A, LO, K64));
+      wv[0 + 2 * t + 1]  = and_or_s(H >> 4, HI, and_or_s(A >> 8, LO, K64));
+      wv[8 + 2 * t]      = and_or_s(H << 2, HI, and_or_s(B, LO, K64));
+      wv[8 + 2 * t + 1]  = and_or_s(H >> 6, HI, and_or_s(B >> 8, LO, K64));
+      wv[16 + 2 * t]     = and_or_s(H, HI, and_or_s(A >> 4, LO, K64));
+      wv[16 + 2 * t + 1] = and_or_s(H >> 8, HI, and_or_s(A >> 12, LO, K64));
+      wv[24 + 2 * t]     = and_or_s(H >> 2, HI, and_or_s(B >> 4, LO, K64));
+      wv[24 + 2 * t + 1] = and_or_s(H >> 10, HI, and_or_s(B >> 12, LO, K64));
     }
   }
   // xv[2j + t/2] = {E(t), O(t), E(t+1), O(t+1)} (t even), E/O = even/odd element pairs of dword t of group j

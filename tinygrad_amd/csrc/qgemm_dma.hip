@@ -457,7 +457,7 @@ static int launch_qd(QArgs a, int M, hipStream_t s) {
 // 16 rows at a 16-byte aligned address (8 rows for the SwiGLU pair);
 // Q4_0 / Q8_0 / Q4_1 / Q5_0 / Q5_1 block pairs: K = 1024, 2048, 3072 or 4096 (larger multiples of 1024 for one matrix); Q4_K / Q5_K: K = 2048 or 4096 (Q5_K: and 1024, 3072), larger
 // multiples of 1024 for one matrix; Q6_K: one matrix, K a multiple of 2048; fp16 weights: K <= 4096, no SwiGLU pair.
-int tga_qgemm_wp_dispatch(int fmt, const QArgs& a, int M, hipStream_t s);   // qgemm_wp.hip: the same call on wave-private rings (Q8_0, K = 2048 / 4096), -1 outside its range
+int tga_qgemm_wp_dispatch(int fmt, const QArgs& a, int M, hipStream_t s);   // qgemm_wp.hip: the same call on wave-private rings (K = 2048 / 4096), -1 outside its range
 // what both kernels ask of a call: 2 <= M <= 16, every matrix whole row groups at a 16-byte aligned address, float32 rows where a norm folds in
 static bool qd_call_ok(const QArgs& a, int M) {
   if (M < 2 || M > 16 || a.nseg < 1 || a.nseg > 3 || a.epilogue > 2 || a.sel || a.x_staged || a.y_stage_fmt) return false;

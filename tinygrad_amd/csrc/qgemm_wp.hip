@@ -1,4 +1,4 @@
-// Small-batch GEMM over Q4_0 / Q8_0 / Q4_1 / Q5_0 / Q5_1 block pairs, Q4_K / Q5_K superblocks (K = 2048 or 4096) and fp16 weights (K = 2048), 2 <= M <= 16 activation rows, with the weights streamed into LDS by direct-to-LDS loads into rings
+// Small-batch GEMM over Q4_0 / Q8_0 / Q4_1 / Q5_0 / Q5_1 block pairs, Q4_K / Q5_K / Q6_K superblocks (K = 2048 or 4096) and fp16 weights (K = 2048), 2 <= M <= 16 activation rows, with the weights streamed into LDS by direct-to-LDS loads into rings
 // that belong to ONE WAVE each: the same call sites and arithmetic as qgemm_dma.hip (x.linear(W.T) over a lazily dequantized weight: tinygrad/nn/__init__.py:177,
 // tinygrad/mixin/op.py:367-392; a unit is decoded once into fp16 weights - the reference's fp16 weight cast, tinygrad/llm/model.py:376 - and
 // v_mfma_f32_16x16x32_f16 multiplies it with all activation rows), without a workgroup barrier in the loop.
@@ -38,11 +38,18 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
   using DF = DmaFmt<T_>;
   typedef typename F::Raw Raw;
   static_assert(!(MS && SW), "the SwiGLU pair is not combined with the q / k / v walk");
-  constexpr int SLICE = DF::slot_bytes(UPW);             // bytes of one row that a wave owns
+  // A ring position holds a wave's run of a row group or, Q6_K, one step of it: a superblock of 210 bytes per row, fetched as the fourteen aligned pieces that hold it.  Its ring of four steps is
+  // 120 KB a CU (three from nine rows on); whole runs (two positions of 420 bytes per row) would be 121 KB with half of it idle while the other half is decoded, and their second superblock starts off a piece.
+  // A lane's operands of the next step are read from LDS while this step is decoded, so a position is requested into again one step earlier.  128256 x 4096, 4 / 8 / 16 rows (us):
+  // barrier kernel 121 / 130 / 136, this ring 113 / 115 / 115, with the operands one step ahead 109 / 110 / 110, with single-instruction masks in the decode (qfmt.h) 104 / 105 / 107;
+  // 14336 x 4096, 4 / 16 rows: 21.4 / 23.3 -> 19.7 / 19.8.  What is left is the decode: 250 vector instructions per superblock, two waves a SIMD.
+  constexpr bool BYSTEP = T_ == GGML_Q6_K;
+  constexpr int NST = UPW / 4;                           // steps (4 units x 16 rows) of a wave per row group
+  constexpr int IPG = BYSTEP ? NST : 1;                  // ring positions per row group
+  constexpr int SLICE = BYSTEP ? 14 * 16 : DF::slot_bytes(UPW);   // bytes of one row in a ring position
   static_assert(SLICE % 16 == 0 && UPW % 4 == 0, "a wave's run of a row is whole 16-byte pieces and whole steps of four units");
   constexpr int PR = SLICE / 16, PP = PR + (PR % 2 == 0 ? 1 : 0);   // pieces per row, and with the pad piece: an odd pitch in pieces puts sixteen rows on sixteen different bank quads
   constexpr int PIECES = 16 * PP, NI = (PIECES + 63) / 64, REM = PIECES - 64 * (NI - 1), STAGE = PIECES * 16, PITCH = PP * 16;
-  constexpr int NST = UPW / 4;                           // steps (4 units x 16 rows) of a wave per row group
   constexpr int GR = SW ? 8 : 16;                        // output rows per row group
   extern __shared__ u32x4 lds[];
   __shared__ __attribute__((aligned(16))) float part[2][WP_NW][256];   // [tile set][wave][16 c + 4 (g ^ (c >> 2)) + i]: lane (g, c) keeps rows 4 g .. 4 g + 3 of column c as one 16-byte piece (the swizzle spreads a quarter wave over all banks)
@@ -62,6 +69,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
   auto rows_of = [&](int sg) -> long long { return !MS ? a.n[0] : sg == 0 ? a.n[0] : sg == 1 ? a.n[1] : a.n[2]; };
   auto w_of = [&](int sg) -> const uint8_t* { return !MS ? a.w[0] : sg == 0 ? a.w[0] : sg == 1 ? a.w[1] : a.w[2]; };
   const long long G = ((long long)blockIdx.x < ngroups) ? (ngroups - blockIdx.x + gridDim.x - 1) / gridDim.x : 0;   // row groups of this workgroup: every wave walks all of them
+  const long long items = G * IPG;
   __syncthreads();                                       // (the counters are set)
   if (G == 0) return;
 
@@ -74,12 +82,14 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
     int rr = sigma / PP, q = sigma - rr * PP;
     rr = rr < 16 ? rr : 15; q = q < PR ? q : PR - 1;
     from_up[i] = SW && rr >= 8;
-    doff[i] = (long long)(SW ? (rr & 7) : rr) * a.row_bytes + (long long)wave * SLICE + q * 16;
+    doff[i] = (long long)(SW ? (rr & 7) : rr) * a.row_bytes + (BYSTEP ? 0 : (long long)wave * SLICE) + q * 16;
   }
-  auto issue = [&](long long j, int slot) {
+  auto step_byte = [&](int ss) { return 210 * (wave * NST + ss); };      // (BYSTEP) where the superblock of step ss starts in a row
+  auto issue = [&](long long k, int slot) {
+    const long long j = IPG == 1 ? k : k / IPG;
     const long long grp = (long long)blockIdx.x + j * gridDim.x;
     int sg; long long l0; seg_of(grp * GR, sg, l0);
-    const long long goff = l0 * a.row_bytes;
+    const long long goff = l0 * a.row_bytes + (BYSTEP ? step_byte((int)(k % IPG)) & ~15 : 0);
     const uint8_t* base = w_of(sg) + goff;
     const uint8_t* base_up = SW ? a.w[1] + goff : base;
     char* dst = ringw + slot * STAGE;
@@ -123,7 +133,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
       // activations of the wave that starts last wait behind the weight misses of the seven that started first (its operands were ready 2 us after theirs)
       asm volatile("s_barrier" ::: "memory");
       int issued = 0;
-      for (int k = 0; k < NB - 1; k++) if (k < G) { issue(k, k); issued++; }
+      for (int k = 0; k < NB - 1; k++) if (k < items) { issue(k, k); issued++; }
       qd_wait_vm(issued * NI);
       float sc[NORM ? NV : 1];
       if constexpr (NORM) {
@@ -220,16 +230,17 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
   };
 
   int slot = 0;
+  Raw ahead;
+  if constexpr (BYSTEP) {                                               // position 0 has landed and is read; the prologue has requested NB - 1 positions, the last one follows
+    static_assert(NB == 3 || NB == 4, "ring of three or four steps");
+    if (NB == 4 && items >= 3) wp_wait_vm<2 * NI>(); else if (items >= 2) wp_wait_vm<NI>(); else wp_wait_vm<0>();
+    ahead = DF::from_lds(ringw + r * PITCH + (step_byte(0) & 15), g);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (items >= NB) issue(NB - 1, NB - 1);
+  }
   for (long long j = 0; j < G; j++) {
-    const long long after = G - 1 - j;
-    // this wave's pieces of group j have landed (later groups, and the stores of a sum, may be in flight)
-    if constexpr (NB == 2) wp_wait_vm<0>();
-    else { static_assert(NB == 3 && NI <= 24, "ring of two or three groups"); if (after >= 1) wp_wait_vm<NI>(); else wp_wait_vm<0>(); }
-    if (j + NB - 1 < G) issue(j + NB - 1, slot == 0 ? NB - 1 : slot - 1);
     v4f32 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ss = 0; ss < NST; ss++) {
-      const Raw buf = DF::from_lds(ringw + slot * STAGE + r * PITCH, 4 * ss + g);
+    auto multiply = [&](const Raw& buf, int ss) __attribute__((always_inline)) {
       uint32_t wv[F::NWV];
       F::decode(buf, wv, kc);
       F::to_f16(buf, wv);
@@ -239,9 +250,33 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
         if (v & 1) acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8f16, av), __builtin_bit_cast(v8f16, bfrag[ss][v]), acc1, 0, 0, 0);
         else acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8f16, av), __builtin_bit_cast(v8f16, bfrag[ss][v]), acc0, 0, 0, 0);
       }
+    };
+    if constexpr (BYSTEP) {
+      // the step behind this one is read from LDS while this one is decoded, so its ring position is requested into again at once
+#pragma unroll
+      for (int ss = 0; ss < NST; ss++) {
+        const long long k = j * NST + ss, after = items - 1 - k;
+        const int nslot = slot + 1 == NB ? 0 : slot + 1;
+        // position k has been read; behind position k + 1 at most NB - 2 are on their way (behind the last one a position of earlier steps is read and dropped)
+        if (NB == 4 && after >= 3) wp_wait_vm<2 * NI>(); else if (after >= 2) wp_wait_vm<NI>(); else wp_wait_vm<0>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const Raw next = DF::from_lds(ringw + nslot * STAGE + r * PITCH + (step_byte((ss + 1) % NST) & 15), g);
+        if (after >= NB) issue(k + NB, slot);
+        multiply(ahead, ss);
+        ahead = next;
+        slot = nslot;
+      }
+    } else {
+      const long long after = G - 1 - j;
+      // this wave's pieces of group j have landed (later groups, and the stores of a sum, may be in flight)
+      static_assert(BYSTEP || NB == 2 || (NB == 3 && NI <= 24), "ring of two or three groups");
+      if (NB == 3 && after >= 1) wp_wait_vm<NI>(); else wp_wait_vm<0>();
+      if (j + NB - 1 < G) issue(j + NB - 1, slot == 0 ? NB - 1 : slot - 1);
+#pragma unroll
+      for (int ss = 0; ss < NST; ss++) multiply(DF::from_lds(ringw + slot * STAGE + r * PITCH, 4 * ss + g), ss);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // every read of this ring position is done: the next pass requests into it
+      slot = slot + 1 == NB ? 0 : slot + 1;
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // every read of this ring position is done: the next pass requests into it
-    slot = slot + 1 == NB ? 0 : slot + 1;
     // the tile set of this group: free once the group two before it has been summed
     const int p = (int)(j & 1);
     const unsigned turn = (unsigned)(j >> 1);
@@ -274,7 +309,7 @@ static int wp_cu_count() {
 template <int T, bool MS, bool SW, int UPW, int NB>
 static int launch_wp_k(const QArgs& a, int M, hipStream_t s) {
   using DF = DmaFmt<T>;
-  constexpr int SLICE = DF::slot_bytes(UPW), PR = SLICE / 16, PP = PR + (PR % 2 == 0 ? 1 : 0), STAGE = 16 * PP * 16;
+  constexpr int SLICE = T == GGML_Q6_K ? 14 * 16 : DF::slot_bytes(UPW), PR = SLICE / 16, PP = PR + (PR % 2 == 0 ? 1 : 0), STAGE = 16 * PP * 16;
   const int xb = (M > 8 ? 16 : M > 4 ? 8 : 4) * 512;                   // the activations' way through LDS: behind the ring positions that are requested first
   int ring_w = NB * STAGE; if ((NB - 1) * STAGE + xb > ring_w) ring_w = (NB - 1) * STAGE + xb;
   const size_t lds = (size_t)WP_NW * ring_w;
@@ -302,10 +337,15 @@ template <int T, int UPW>
 static int launch_wp_u(const QArgs& a, int M, hipStream_t s) {
   // three groups in flight per wave where the ring holds them, else two
   int rc;
+  if constexpr (T == GGML_Q6_K) {                                      // (one matrix, plain or residual epilogue, as on the barrier kernel; from nine rows on the activations' way through LDS leaves room for three steps)
+    if (a.epilogue == 2 || a.nseg > 1) return -1;
+    rc = launch_wp_k<T, false, false, UPW, 4>(a, M, s); return rc >= 0 ? rc : launch_wp_k<T, false, false, UPW, 3>(a, M, s);
+  } else {
   if constexpr (T != GGML_F16) { if (a.epilogue == 2) { rc = launch_wp_k<T, false, true, UPW, 3>(a, M, s); return rc >= 0 ? rc : launch_wp_k<T, false, true, UPW, 2>(a, M, s); } }
   if (a.epilogue == 2) return -1;
   if (a.nseg > 1) { rc = launch_wp_k<T, true, false, UPW, 3>(a, M, s); return rc >= 0 ? rc : launch_wp_k<T, true, false, UPW, 2>(a, M, s); }
   rc = launch_wp_k<T, false, false, UPW, 3>(a, M, s); return rc >= 0 ? rc : launch_wp_k<T, false, false, UPW, 2>(a, M, s);
+  }
 }
 
 template <int T>
@@ -320,7 +360,7 @@ static int launch_wp(QArgs a, int M, hipStream_t s) {
 }
 
 // Called by tga_qgemm_dma_dispatch with a call it has checked (2 <= M <= 16, matrices of whole row groups at 16-byte aligned addresses, float32 rows where a norm
-// folds in).  Returns -1 outside this kernel's range (K other than 2048 / 4096, Q6_K and the formats that are not block pairs, a ring that does not fit LDS,
+// folds in).  Returns -1 outside this kernel's range (K other than 2048 / 4096, Q6_K in several matrices or as a SwiGLU pair, a ring that does not fit LDS,
 // outputs that are not 16-byte aligned).
 int tga_qgemm_wp_dispatch(int fmt, const QArgs& a, int M, hipStream_t s) {
   static const bool off = getenv("TGA_WP") && atoi(getenv("TGA_WP")) == 0;      // (for A / B runs against the barrier kernel)
@@ -339,6 +379,7 @@ int tga_qgemm_wp_dispatch(int fmt, const QArgs& a, int M, hipStream_t s) {
     case GGML_Q4_1: return launch_wp<GGML_Q4_1>(a, M, s);
     case GGML_Q5_0: return launch_wp<GGML_Q5_0>(a, M, s);
     case GGML_Q5_1: return launch_wp<GGML_Q5_1>(a, M, s);
+    case GGML_Q6_K: return launch_wp<GGML_Q6_K>(a, M, s);
     case GGML_F16: return launch_wp<GGML_F16>(a, M, s);
   }
   return -1;
