@@ -286,6 +286,23 @@ def _single_steps(moe, inp, logits, k, gate_up, b_gate_up, down, b_down):
   z = moe.add_expert_bias(moe.grouped_mx_gemm(y, down, r.off, routed_only=True, counts=r.counts), b_down, r.off)
   return moe.combine(z, r, inp.shape[0], k).numpy()
 
+@pytest.mark.parametrize("T,D,I,E,k,skew", [(1, 256, 256, 3, 1, 0), (5, 768, 256, 70, 8, 1), (33, 2048, 768, 5, 3, 1), (40, 1280, 512, 20, 4, 0), (130, 256, 768, 4, 4, 0), (600, 1024, 256, 9, 2, 2), (900, 512, 512, 12, 2, 0),
+                                            (2600, 256, 768, 40, 2, 1), (6000, 256, 256, 80, 2, 0), (3100, 768, 512, 65, 4, 0), (700, 1536, 512, 512, 8, 1)])
+def test_moe_feed_forward_at_every_tile_height(gpu, T, D, I, E, k, skew):
+  """Tiles of 16, 32, 64, 128 and 256 rows (by the rows per expert; 256 where the counts, on the device, make them half the rounds), reductions of 2, 4, 6, 8, 10, 12 and 16 steps of 128 (scales
+  are fetched four steps at a time, a last pair on its own), experts of no rows, of one, of several tiles and with a remainder, more experts than lanes: bits of the single steps, twice."""
+  from tinygrad_amd import moe
+  rng = np.random.default_rng(T + D + I + E)
+  B = gpu.Buffer.from_numpy
+  inp = moe.to_bf16_bits(rng.standard_normal((T, D)).astype(np.float32))
+  logits = (rng.standard_normal((T, E)) + skew * np.linspace(0, 3, E)).astype(np.float32)
+  def weight(n, kk): return moe.quantize_mxfp8(B(moe.to_bf16_bits((rng.standard_normal((E * n, kk), dtype=np.float32) * np.float32(kk ** -0.5)))))[:2]
+  (gq, ge), (dq, de) = weight(2 * I, D), weight(D, I)
+  args = (B(inp), B(logits), k, (gq.view(0, (E, 2 * I, D), np.uint8), ge.view(0, (E, 2 * I, D // 32), np.uint8)), B((rng.standard_normal((E, 2 * I)) * 0.1).astype(np.float32)),
+          (dq.view(0, (E, D, I), np.uint8), de.view(0, (E, D, I // 32), np.uint8)), B((rng.standard_normal((E, D)) * 0.1).astype(np.float32)))
+  ref = _single_steps(moe, *args)
+  for _ in range(2): assert (moe.moe_feed_forward(*args).numpy() != ref).sum() == 0
+
 @pytest.mark.parametrize("case", ["random", "masked", "fewer than k", "tiny"])
 def test_moe_feed_forward_has_the_bits_of_the_single_steps(gpu, case):
   """Random rows; logits masked with -inf so that exactly k, or fewer than k, experts are left (the surplus picks weigh nothing); gate values whose sigmoid is a subnormal number."""

@@ -7,14 +7,16 @@
 // (+ a fill of the expert counters in front when more than one workgroup routes).  The values are those of route -> dispatch -> quantize_mxfp8 -> grouped_mx_gemm ->
 // add_expert_bias -> swiglu -> quantize_mxfp8 -> grouped_mx_gemm -> add_expert_bias -> combine: every rounding to bf16 and to E4M3 sits where it sits there.  What
 // is gone are the passes between them (T = 4096, k = 8, E = 128, D = 2048, I = 768: dispatch, two quantisations, two bias adds, SwiGLU over 65536 padded rows) and the
-// padding of every expert's rows to 256, and the host work of eleven entry points.  MI355X, back to back: T = 2000, k = 8, E = 64, D = 2048, I = 512 2480 (single passes:
-// 810) -> 186 us; T = 32, k = 8, E = 64, I = 768 840 (single) -> 81 us; the benchmark's T = 4096, E = 128, I = 768 1340 (single) -> 406 us.
+// padding of every expert's rows to 256, and the host work of eleven entry points.  MI355X, back to back: T = 2000, k = 8, E = 64, D = 2048, I = 512, popularity
+// by 1 / rank^1.1: 2480 (single passes: 810) -> 182 -> 150 us; T = 32, k = 8, E = 64, I = 768: 840 (single) -> 77 -> 67 us; T = 4096, E = 128, I = 768: 1340 (single) -> 406 -> 370 us.  The second step of
+// each: operands by direct-to-LDS loads instead of through registers, scales sixteen bytes a row, lower tiles, routing workgroups of 16 tokens.
 #include "mxfp8.h"
 #include "host.h"
+#include <type_traits>
 
 #define FFN_MAX_E 512             // experts (their counts and offsets sit in LDS)
 #define FFN_MAX_K 64              // experts per token
-#define FFN_BN 256                // weight rows of a tile
+#define FFN_TALL_STAGE (512 * 132)
 
 struct FfnArgs {
   const uint16_t* x; const float* logits; const uint8_t* w[2]; const uint8_t* we8[2]; const float* bias[2];
@@ -27,11 +29,12 @@ struct FfnArgs {
   float* weights;                 // [T][k]
   uint16_t* out;
   int nq_blocks;                  // workgroups of moe_prep_kernel that quantise
+  int prep_tokens;                // tokens of a routing workgroup
   int one_route_block;
 };
 
 // ---------------------------------------------------------------------------------------------------- routing + quantisation of the input
-#define PREP_TOKENS 64            // tokens of a routing workgroup: sixteen waves of four
+#define PREP_TOKENS 64            // most tokens of a routing workgroup of sixteen waves
 
 template <int CTRL, int ROW_MASK> __device__ __forceinline__ uint32_t dpp_umax(uint32_t v) {
   const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xF, false);
@@ -96,7 +99,7 @@ __global__ __launch_bounds__(1024) void moe_prep_kernel(const FfnArgs a) {
   }
   __shared__ int ids[PREP_TOKENS * FFN_MAX_K];
   __shared__ int hist[FFN_MAX_E], base[FFN_MAX_E];
-  const int t0 = ((int)blockIdx.x - a.nq_blocks) * PREP_TOKENS, nt = min(PREP_TOKENS, a.T - t0), n = nt * a.k;
+  const int t0 = ((int)blockIdx.x - a.nq_blocks) * a.prep_tokens, nt = min(a.prep_tokens, a.T - t0), n = nt * a.k;
   for (int e = threadIdx.x; e < a.E; e += 1024) hist[e] = 0;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int i = wave; i < nt; i += 16) route_token<NV>(a, t0 + i, lane, ids + i * a.k);
@@ -124,14 +127,21 @@ __global__ __launch_bounds__(1024) void moe_prep_kernel(const FfnArgs a) {
 }
 __global__ __launch_bounds__(512) void moe_zero_counts_kernel(int* counts, int E) { if ((int)threadIdx.x < E) counts[threadIdx.x] = 0; }
 
-// Exclusive prefix sums over the experts' counts and over their tiles by the first wave of a workgroup: off[e] = first row, tile[e] = first tile (off[E], tile[E]: the totals)
+// Exclusive prefix sums over the experts' counts and over their tiles of bm rows, by the first wave of a workgroup: off[e] = first row, tile[e] = first tile (off[E], tile[E]: the totals).
+// COUNTS: counts are given; otherwise off[] is there and gives them.
+template <bool COUNTS>
 __device__ __forceinline__ void ffn_offsets(const int* __restrict__ counts, int E, int bm, int tiles_n, int* off, int* tile) {
   const int lane = threadIdx.x;
   if (lane < 64) {
     constexpr int PER = FFN_MAX_E / 64;
     int c[PER], so = 0, st = 0;
 #pragma unroll
-    for (int i = 0; i < PER; i++) { const int e = lane * PER + i; c[i] = e < E ? counts[e] : 0; so += c[i]; st += (c[i] + bm - 1) / bm * tiles_n; }
+    for (int i = 0; i < PER; i++) {                                       // (one wait for all of them)
+      const int e = lane * PER + i, k = min(e, E - 1), v = COUNTS ? counts[k] : off[k + 1] - off[k];
+      c[i] = e < E ? v : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < PER; i++) { so += c[i]; st += (c[i] + bm - 1) / bm * tiles_n; }
     int io = so, it = st;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) { const int uo = __shfl_up(io, o), ut = __shfl_up(it, o); if (lane >= o) { io += uo; it += ut; } }
@@ -139,37 +149,108 @@ __device__ __forceinline__ void ffn_offsets(const int* __restrict__ counts, int 
 #pragma unroll
     for (int i = 0; i < PER; i++) {
       const int e = lane * PER + i;
-      if (e <= E) { off[e] = io; if (tile) tile[e] = it; }
+      if (e <= E) { if (COUNTS) off[e] = io; if (tile) tile[e] = it; }
       io += c[i]; it += (c[i] + bm - 1) / bm * tiles_n;
-      if (e == E - 1) { off[E] = io; if (tile) tile[E] = it; }
+      if (e == E - 1) { if (COUNTS) off[E] = io; if (tile) tile[E] = it; }
     }
   }
 }
 
 // ---------------------------------------------------------------------------------------------------- the two products
-// Tile of BM rows x 256 weight rows, K steps of 128, WM x 4 waves of (BM / WM) x 64, operands in LDS in the order the scaled MFMA consumes (mxfp8.h), weights as the A
-// operand, so a lane holds four consecutive output columns of one row.  The 16-row sub-tiles are dealt to the WM waves alternately and only those that hold rows are
-// multiplied.  A workgroup walks tiles b, b + gridDim.x, ...: consecutive tiles of an expert share its weight or activation rows, and the workgroups of an XCD (b % 8) take a
-// contiguous run of tiles.  The first step of the next tile is fetched during the last step of this one.
-// UP: gate/up (rows gathered by token, epilogue bias + clamped interleaved SwiGLU + quantisation) or down (compact rows, epilogue bias).
+// The tile of BM x BN that a workgroup is at: expert, rows [m0, m0 + valid) of it from compact row row0 on, columns [BN tn, ...), first weight row
 struct FfnCur { uint32_t boff; int e, m0, tn, valid, row0; };
+template <int BM, int BN>
+__device__ __forceinline__ void ffn_find(int E, int N, int tiles_n, const int* s_off, const int* s_tile, int tile, FfnCur& c) {
+  const int lane = threadIdx.x & 63;
+  int n = 0;                                                             // the expert whose tiles hold this one: the last that starts at or in front of it
+  for (int e = 0; e < E; e += 64) n += __popcll(__ballot(e + lane < E && s_tile[e + lane] <= tile));
+  const int lo = n - 1;
+  const int i = tile - __builtin_amdgcn_readfirstlane(s_tile[lo]), tm = i / tiles_n, off = __builtin_amdgcn_readfirstlane(s_off[lo]);
+  c.e = lo; c.tn = i - tm * tiles_n; c.m0 = tm * BM; c.valid = min(__builtin_amdgcn_readfirstlane(s_off[lo + 1]) - off - c.m0, BM);
+  c.row0 = off + c.m0;
+  c.boff = ((uint32_t)lo * (uint32_t)N + (uint32_t)c.tn * BN);
+}
 
-template <int BM, int WM, bool UP>
-__global__ __launch_bounds__(256 * WM) void ffn_gemm_kernel(const FfnArgs a) {
-  constexpr int NT = 256 * WM, RS = BM / 16 / WM;                        // threads, 16-row sub-tiles of a wave
-  constexpr int PA = BM * 8 / NT, PB = FFN_BN * 8 / NT, NS = (BM + FFN_BN + NT - 1) / NT;   // 16-byte pieces and scale dwords per thread and step
-  static_assert(PA >= 1 && RS >= 1, "tile too small");
-  constexpr int STAGE = (BM + FFN_BN) * 132;
+// fminf / fmaxf of values that are no signalling NaN (bf16 results of a conversion): one instruction, where the functions quieten their arguments first
+__device__ __forceinline__ float min_q(float a, float b) { float o; asm("v_min_f32 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b)); return o; }
+__device__ __forceinline__ float max_q(float a, float b) { float o; asm("v_max_f32 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b)); return o; }
+__device__ __forceinline__ float max3_abs(float m, float a, float b) { float o; asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(o) : "v"(m), "v"(a), "v"(b)); return o; }
+
+// The result of a tile: lane = row r16 of sub-tile WM i + wm, columns 4 kg .. 4 kg + 3 of n sub-tile j.  slab: 16 rows of 144 bytes of LDS that are this wave's; b: the bias of its 64 columns.
+template <int RS, int WM, int BN, bool UP>
+__device__ __forceinline__ void ffn_epilogue(const FfnArgs& a, const FfnCur& c, const v4f32 (&acc)[RS][4], int nsub, int wm, int wn, uint8_t* slab, const float* b) {
+  const int lane = threadIdx.x & 63, r16 = lane & 15, kg = lane >> 4, row0 = c.row0;
+  const float limit = __builtin_canonicalizef(a.limit);
+  f32x4 bias[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    bias[j] = *(const f32x4*)(b + 16 * j + 4 * kg);
+#pragma unroll
+    for (int i = 0; i < 4; i++) bias[j][i] = bf16_to_f(f_to_bf16(bias[j][i]));
+  }
+#pragma unroll
+  for (int i = 0; i < RS; i++) {
+    if (i >= nsub) break;
+    const int r0 = 16 * (WM * i + wm);                                // first row of the sub-tile
+    if constexpr (UP) {
+      float y[8], amax = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        // h = bf16(acc); h = bf16(h + bf16(bias)); then gate and up are neighbouring columns
+        const uint32_t h01 = pack_bf16x2(acc[i][j][0], acc[i][j][1]), h23 = pack_bf16x2(acc[i][j][2], acc[i][j][3]);
+        const uint32_t g01 = pack_bf16x2(bf16_lo(h01) + bias[j][0], bf16_hi(h01) + bias[j][1]), g23 = pack_bf16x2(bf16_lo(h23) + bias[j][2], bf16_hi(h23) + bias[j][3]);
+        const float gl0 = min_q(bf16_lo(g01), limit), gl1 = min_q(bf16_lo(g23), limit);
+        const float li0 = min_q(max_q(bf16_hi(g01), -limit), limit), li1 = min_q(max_q(bf16_hi(g23), -limit), limit);
+        const uint32_t ag = pack_bf16x2(1.702f * gl0, 1.702f * gl1);
+        const uint32_t sg = pack_bf16x2(mx_sigmoid_bf16(bf16_lo(ag)), mx_sigmoid_bf16(bf16_hi(ag)));
+        const uint32_t p = pack_bf16x2(gl0 * bf16_lo(sg), gl1 * bf16_hi(sg)), q = pack_bf16x2(li0 + 1.0f, li1 + 1.0f);
+        const uint32_t o = pack_bf16x2(bf16_lo(p) * bf16_lo(q), bf16_hi(p) * bf16_hi(q));
+        y[2 * j] = bf16_lo(o); y[2 * j + 1] = bf16_hi(o);
+        amax = max3_abs(amax, y[2 * j], y[2 * j + 1]);
+      }
+      amax = fmaxf(amax, __shfl_xor(amax, 16)); amax = fmaxf(amax, __shfl_xor(amax, 32));     // the wave's 64 columns are one block of 32 results
+      const int e = mx_e8(amax);
+      const float sc = mx_scale(e);
+#pragma unroll
+      for (int j = 0; j < 4; j++) *(uint16_t*)(slab + r16 * 40 + 8 * j + 2 * kg) = (uint16_t)e4m3x2(y[2 * j] * sc, y[2 * j + 1] * sc);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const u32x2 o = *(const u32x2*)(slab + r16 * 40 + 8 * kg);
+      if (r0 + r16 < c.valid) {
+        const size_t row = (size_t)(row0 + r0 + r16);
+        *(u32x2*)(a.yq + row * a.I + c.tn * (BN / 2) + wn * 32 + 8 * kg) = o;
+        if (kg == 0) a.ye8[row * (a.I / 32) + c.tn * (BN / 64) + wn] = (uint8_t)e;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const uint32_t h01 = pack_bf16x2(acc[i][j][0], acc[i][j][1]), h23 = pack_bf16x2(acc[i][j][2], acc[i][j][3]);
+        *(u32x2*)(slab + r16 * 144 + 32 * j + 8 * kg) = u32x2{pack_bf16x2(bf16_lo(h01) + bias[j][0], bf16_hi(h01) + bias[j][1]), pack_bf16x2(bf16_lo(h23) + bias[j][2], bf16_hi(h23) + bias[j][3])};
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const int rr = lane >> 3, rc = lane & 7;
+#pragma unroll
+      for (int p = 0; p < 2; p++) {
+        const u32x4 o = *(const u32x4*)(slab + (rr + 8 * p) * 144 + 16 * rc);
+        if (r0 + rr + 8 * p < c.valid) *(u32x4*)(a.z + (size_t)(row0 + r0 + rr + 8 * p) * a.D + c.tn * BN + wn * 64 + 8 * rc) = o;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+  }
+}
+
+// Tiles of 256 x 256, two steps in LDS, the next one through registers: half as many tiles as above, each 1.6 times as long.
+template <bool UP>
+__device__ __forceinline__ void ffn_tall(const FfnArgs& a, uint8_t* smem, int* s_row, const int* s_off, const int* s_tile) {
+  constexpr int BM = 256, BN = 256, WM = 2, NT = 512, RS = 8;            // threads, 16-row sub-tiles of a wave
+  constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT, NS = (BM + BN + NT - 1) / NT;   // 16-byte pieces and scale dwords per thread and step
+  constexpr int STAGE = FFN_TALL_STAGE;
   constexpr int RPT = NT / 8;                                            // rows between a thread's pieces
-  __shared__ __attribute__((aligned(16))) uint8_t smem[2 * STAGE];
-  __shared__ int s_off[FFN_MAX_E + 1], s_tile[FFN_MAX_E + 1], s_row[2][BM];   // s_row: operand rows of the tile being multiplied and of the next one
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3, r16 = lane & 15, kg = lane >> 4;
-  const int N = UP ? 2 * a.I : a.D, K = UP ? a.D : a.I, KB = K / 32, nsteps = K / 128, tiles_n = N / FFN_BN;
+  const int N = UP ? 2 * a.I : a.D, K = UP ? a.D : a.I, KB = K / 32, nsteps = K / 128, tiles_n = N / BN;
   const uint8_t* __restrict__ A = UP ? a.xq : a.yq; const uint8_t* __restrict__ Ae = UP ? a.xe8 : a.ye8;
   const uint8_t* __restrict__ B = a.w[UP ? 0 : 1]; const uint8_t* __restrict__ Be = a.we8[UP ? 0 : 1];
-  ffn_offsets(a.counts, a.E, BM, tiles_n, s_off, s_tile);
-  __syncthreads();
   const int ntiles = __builtin_amdgcn_readfirstlane(s_tile[a.E]);
   const int per = (ntiles + 7) >> 3;                                     // tiles of an XCD's run
   const int first = ((int)blockIdx.x & 7) * per, last = min(first + per, ntiles), step_wg = (int)(gridDim.x + 7 - (blockIdx.x & 7)) >> 3;
@@ -185,16 +266,11 @@ __global__ __launch_bounds__(256 * WM) void ffn_gemm_kernel(const FfnArgs a) {
   const int f0 = ((16 * kg + (r16 ^ kg)) << 4), f1 = 1024 + ((16 * kg + (r16 ^ (kg + 4))) << 4);
 
   auto setup = [&](int tile, FfnCur& c, int which) __attribute__((always_inline)) {
-    int lo = 0, hi = a.E;                                                // the expert whose tiles hold this one
-    while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (__builtin_amdgcn_readfirstlane(s_tile[mid]) <= tile) lo = mid; else hi = mid; }
-    const int i = tile - __builtin_amdgcn_readfirstlane(s_tile[lo]), tm = i / tiles_n, off = __builtin_amdgcn_readfirstlane(s_off[lo]);
-    c.e = lo; c.tn = i - tm * tiles_n; c.m0 = tm * BM; c.valid = min(__builtin_amdgcn_readfirstlane(s_off[lo + 1]) - off - c.m0, BM);
-    c.row0 = off + c.m0;
-    c.boff = ((uint32_t)lo * (uint32_t)N + (uint32_t)c.tn * FFN_BN);     // first weight row
-    if (tid < BM) { const int r = min(tid, c.valid - 1); s_row[which][tid] = UP ? a.row_tok[(size_t)lo * a.T + c.m0 + r] : c.row0 + r; }   // rows beyond the expert's repeat its last one (their results are dropped)
+    ffn_find<BM, BN>(a.E, N, tiles_n, s_off, s_tile, tile, c);
+    if (tid < BM) { const int r = min(tid, c.valid - 1); s_row[which * BM + tid] = UP ? a.row_tok[(size_t)c.e * a.T + c.m0 + r] : c.row0 + r; }   // rows beyond the expert's repeat its last one (their results are dropped)
   };
   u32x4 va[PA], vb[PB]; uint32_t vs[NS];
-  auto load_a = [&](int which, int s, int j) __attribute__((always_inline)) { va[j] = *(const u32x4*)(A + (size_t)(uint32_t)s_row[which][cpy_r + RPT * j] * K + (uint32_t)(s * 128 + cpy_c * 16)); };
+  auto load_a = [&](int which, int s, int j) __attribute__((always_inline)) { va[j] = *(const u32x4*)(A + (size_t)(uint32_t)s_row[which * BM + cpy_r + RPT * j] * K + (uint32_t)(s * 128 + cpy_c * 16)); };
   auto load_b = [&](const FfnCur& c, int s, int j) __attribute__((always_inline)) {
     vb[j] = *(const u32x4*)(B + (size_t)(c.boff + RPT * j) * K + (uint32_t)cpy_r * (uint32_t)K + (uint32_t)(s * 128 + cpy_c * 16));
   };
@@ -202,7 +278,7 @@ __global__ __launch_bounds__(256 * WM) void ffn_gemm_kernel(const FfnArgs a) {
 #pragma unroll
     for (int j = 0; j < NS; j++) {
       const int i = tid + NT * j;
-      const uint8_t* p = i < BM ? Ae + (size_t)(uint32_t)s_row[which][i] * KB : Be + (size_t)(c.boff + (uint32_t)min(i - BM, FFN_BN - 1)) * KB;
+      const uint8_t* p = i < BM ? Ae + (size_t)(uint32_t)s_row[which * BM + i] * KB : Be + (size_t)(c.boff + (uint32_t)min(i - BM, BN - 1)) * KB;
       vs[j] = *(const uint32_t*)(p + 4 * s);
     }
   };
@@ -210,7 +286,7 @@ __global__ __launch_bounds__(256 * WM) void ffn_gemm_kernel(const FfnArgs a) {
   auto store_b = [&](uint8_t* st, int j) __attribute__((always_inline)) { *(u32x4*)(st + lds_b[j]) = vb[j]; };
   auto store_s = [&](uint8_t* st) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < NS; j++) { const int i = tid + NT * j; if (i < BM + FFN_BN) ((uint32_t*)(st + (BM + FFN_BN) * 128))[i] = vs[j]; }
+    for (int j = 0; j < NS; j++) { const int i = tid + NT * j; if (i < BM + BN) ((uint32_t*)(st + (BM + BN) * 128))[i] = vs[j]; }
   };
 
   FfnCur cur, nxt;
@@ -254,7 +330,7 @@ __global__ __launch_bounds__(256 * WM) void ffn_gemm_kernel(const FfnArgs a) {
       for (int j = 0; j < PB; j++) load_b(src, ls, j);
       __builtin_amdgcn_sched_barrier(0);
       const uint8_t* As = st; const uint8_t* Bs = st + BM * 128 + wn * 4 * 2048;
-      const uint32_t* sA = (const uint32_t*)(st + (BM + FFN_BN) * 128) + r16; const uint32_t* sB = sA + BM + wn * 64;
+      const uint32_t* sA = (const uint32_t*)(st + (BM + BN) * 128) + r16; const uint32_t* sB = sA + BM + wn * 64;
       if (nsub > 0) {
         v8i32 bf[4]; int sb[4];
 #pragma unroll
@@ -289,70 +365,235 @@ __global__ __launch_bounds__(256 * WM) void ffn_gemm_kernel(const FfnArgs a) {
       store_s(st2);
       __syncthreads();
     }
-    // ---- epilogue: lane = row r16 of sub-tile WM i + wm, columns 4 kg .. 4 kg + 3 of n sub-tile j.  The stage the last step was read from is idle: wave-private slabs.
-    {
-      uint8_t* slab = smem + ((par + nsteps - 1) & 1) * STAGE + wave * 2304;   // 16 rows of 144 bytes
-      const int row0 = cur.row0;
-      f32x4 bias[4];
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        bias[j] = *(const f32x4*)(a.bias[UP ? 0 : 1] + (size_t)cur.e * N + cur.tn * FFN_BN + wn * 64 + 16 * j + 4 * kg);
-#pragma unroll
-        for (int c = 0; c < 4; c++) bias[j][c] = bf16_to_f(f_to_bf16(bias[j][c]));
-      }
-#pragma unroll
-      for (int i = 0; i < RS; i++) {
-        if (i >= nsub) break;
-        const int r0 = 16 * (WM * i + wm);                                // first row of the sub-tile
-        if constexpr (UP) {
-          float y[8], amax = 0.f;
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            // h = bf16(acc); h = bf16(h + bf16(bias)); then gate and up are neighbouring columns
-            const uint32_t h01 = pack_bf16x2(acc[i][j][0], acc[i][j][1]), h23 = pack_bf16x2(acc[i][j][2], acc[i][j][3]);
-            const uint32_t g01 = pack_bf16x2(bf16_lo(h01) + bias[j][0], bf16_hi(h01) + bias[j][1]), g23 = pack_bf16x2(bf16_lo(h23) + bias[j][2], bf16_hi(h23) + bias[j][3]);
-            const float gl0 = fminf(bf16_lo(g01), a.limit), gl1 = fminf(bf16_lo(g23), a.limit);
-            const float li0 = fminf(fmaxf(bf16_hi(g01), -a.limit), a.limit), li1 = fminf(fmaxf(bf16_hi(g23), -a.limit), a.limit);
-            const uint32_t ag = pack_bf16x2(1.702f * gl0, 1.702f * gl1);
-            const uint32_t sg = pack_bf16x2(mx_sigmoid_bf16(bf16_lo(ag)), mx_sigmoid_bf16(bf16_hi(ag)));
-            const uint32_t p = pack_bf16x2(gl0 * bf16_lo(sg), gl1 * bf16_hi(sg)), q = pack_bf16x2(li0 + 1.0f, li1 + 1.0f);
-            const uint32_t o = pack_bf16x2(bf16_lo(p) * bf16_lo(q), bf16_hi(p) * bf16_hi(q));
-            y[2 * j] = bf16_lo(o); y[2 * j + 1] = bf16_hi(o);
-            amax = fmaxf(amax, fmaxf(fabsf(y[2 * j]), fabsf(y[2 * j + 1])));
-          }
-          amax = fmaxf(amax, __shfl_xor(amax, 16)); amax = fmaxf(amax, __shfl_xor(amax, 32));     // the wave's 64 columns are one block of 32 results
-          const int e = mx_e8(amax);
-          const float sc = mx_scale(e);
-#pragma unroll
-          for (int j = 0; j < 4; j++) *(uint16_t*)(slab + r16 * 40 + 8 * j + 2 * kg) = (uint16_t)e4m3x2(y[2 * j] * sc, y[2 * j + 1] * sc);
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          const u32x2 o = *(const u32x2*)(slab + r16 * 40 + 8 * kg);
-          if (r0 + r16 < cur.valid) {
-            const size_t row = (size_t)(row0 + r0 + r16);
-            *(u32x2*)(a.yq + row * a.I + cur.tn * 128 + wn * 32 + 8 * kg) = o;
-            if (kg == 0) a.ye8[row * (a.I / 32) + cur.tn * 4 + wn] = (uint8_t)e;
-          }
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const uint32_t h01 = pack_bf16x2(acc[i][j][0], acc[i][j][1]), h23 = pack_bf16x2(acc[i][j][2], acc[i][j][3]);
-            *(u32x2*)(slab + r16 * 144 + 32 * j + 8 * kg) = u32x2{pack_bf16x2(bf16_lo(h01) + bias[j][0], bf16_hi(h01) + bias[j][1]), pack_bf16x2(bf16_lo(h23) + bias[j][2], bf16_hi(h23) + bias[j][3])};
-          }
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          const int rr = lane >> 3, rc = lane & 7;
-#pragma unroll
-          for (int p = 0; p < 2; p++) {
-            const u32x4 o = *(const u32x4*)(slab + (rr + 8 * p) * 144 + 16 * rc);
-            if (r0 + rr + 8 * p < cur.valid) *(u32x4*)(a.z + (size_t)(row0 + r0 + rr + 8 * p) * N + cur.tn * FFN_BN + wn * 64 + 8 * rc) = o;
-          }
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        }
-      }
-    }
+    // the stage the last step was read from is idle: wave-private slabs
+    ffn_epilogue<RS, WM, BN, UP>(a, cur, acc, nsub, wm, wn, smem + ((par + nsteps - 1) & 1) * STAGE + wave * 2304, a.bias[UP ? 0 : 1] + (size_t)cur.e * N + cur.tn * BN + wn * 64);
     if (!more) break;
     __syncthreads();                                                      // the slabs are free before any wave's next step writes that stage
     par = (par + nsteps) & 1; cur = nxt; t = tnext; which ^= 1;
+  }
+}
+
+// Tile of BM rows x 64 WN weight rows, K steps of 128, WM x WN waves of (BM / WM) x 64, weights as the A operand of the scaled MFMA, so a lane holds four consecutive
+// output columns of one row.  The 16-row sub-tiles are dealt to the WM waves alternately and only those that hold rows are multiplied.  A workgroup walks tiles b,
+// b + gridDim.x, ...: consecutive tiles of an expert share its weight or activation rows, and the workgroups of an XCD (b % 8) take a contiguous run of tiles.
+// Operands go to a ring of NB steps in LDS by direct-to-LDS loads, NB - 1 steps ahead of the multiplication and across tile borders: one barrier per step, no registers in between.
+// A step's region: rows of 128 bytes, 16-byte chunk c of row R at chunk c ^ (R & 7) (a request covers eight whole rows, a read of sixteen rows meets each bank group once
+// per eight lanes).  Scales come four steps at a time, sixteen bytes a row: a dword a row and step was 64 cache lines a request, a fifth of the time.  Rows beyond the expert's repeat its last one.
+// UP: gate/up (rows gathered by token, epilogue bias + clamped interleaved SwiGLU + quantisation) or down (compact rows, epilogue bias).
+// Measured (us, gate/up + down): 16000 rows of 64 experts skewed, D 2048, I 512, tiles of 128: 97.5 + 52.7 (tiles of 256 through registers) -> 79 + 42; 256 rows of 64 experts, I 768, tiles of 16:
+// 42.1 + 23.3 -> 35.8 + 20.2, which is 4.6 TB/s of weights.  What bounds the first: a step is 1.4 us of which 0.45 are products (eight waves read 128 KB of LDS, then multiply, in one phase;
+// two groups of waves half a step apart with a barrier each half: 77 + 44, not kept), the epilogue's 400 vector instructions per sub-tile 6 us a tile, and 2.4 rounds of tiles on 256 CUs.
+__device__ __forceinline__ const uint8_t* scalar_ptr(const uint8_t* p) {
+  const uint64_t v = (uint64_t)(uintptr_t)p;
+  uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  asm("" : "+s"(lo), "+s"(hi));
+  return (const uint8_t*)(uintptr_t)(((uint64_t)hi << 32) | lo);
+}
+template <int N> __device__ __forceinline__ void ffn_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
+
+template <int BM, int WM, int WN, int NB, bool UP>
+__global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a) {
+  constexpr int NW = WM * WN, BN = 64 * WN, RS = BM / 16 / WM;          // waves, weight rows of a tile, 16-row sub-tiles of a wave
+  constexpr int IA = BM / 8 / NW, IB = BN / 8 / NW, SI = (BM + BN + 63) / 64, IS = (SI + NW - 1) / NW, NI = IA + IB;   // requests of a wave: eight rows of operands a step, 64 rows' scales of four steps
+  constexpr int STAGE = (BM + BN) * 128;
+  static_assert(IA * 8 * NW == BM && IB * 8 * NW == BN && RS >= 1 && (NB == 2 || NB == 3) && STAGE >= NW * 2304, "tile shape");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];        // NB steps, the scales of up to four steps, the experts' first rows and tiles
+  __shared__ __attribute__((aligned(16))) float s_bias[2][BN];          // of the tile multiplied and the one requested
+  __shared__ __attribute__((aligned(16))) int s_ids[UP ? NW : 1][UP ? 8 * IA + 64 * IS : 1];   // tokens of the rows this wave requests: operands, scales (its own: no barrier between their arrival and their use)
+  uint8_t* const scales = smem + NB * STAGE;
+  int* const s_off = (int*)(scales + (BM + BN) * 16); int* const s_tile = s_off + a.E + 1;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN, r16 = lane & 15, kg = lane >> 4;
+  const int N = UP ? 2 * a.I : a.D, K = UP ? a.D : a.I, KB = K / 32, nsteps = K / 128, tiles_n = N / BN;
+  const uint8_t* __restrict__ A = UP ? a.xq : a.yq; const uint8_t* __restrict__ Ae = UP ? a.xe8 : a.ye8;
+  const uint8_t* __restrict__ B = a.w[UP ? 0 : 1]; const uint8_t* __restrict__ Be = a.we8[UP ? 0 : 1];
+  ffn_offsets<true>(a.counts, a.E, BM, tiles_n, s_off, s_tile);
+  __syncthreads();
+  const int ntiles = __builtin_amdgcn_readfirstlane(s_tile[a.E]);
+  if constexpr (BM == 128) {
+    const int grid = (int)gridDim.x, rounds = (ntiles + grid - 1) / grid;
+    if (rounds > 1) {                                                     // tall tiles where they halve the rounds of the launch: see the dispatch
+      int tall = 0;
+      for (int e = 0; e < a.E; e += 64) tall += e + lane < a.E ? (s_off[e + lane + 1] - s_off[e + lane] + 255) >> 8 : 0;
+#pragma unroll
+      for (int o = 32; o; o >>= 1) tall += __shfl_xor(tall, o);
+      tall = __builtin_amdgcn_readfirstlane(tall) * tiles_n;
+      if (2 * ((tall + grid - 1) / grid) <= rounds) {
+        __syncthreads();                                                  // (every wave has read the tiles)
+        ffn_offsets<false>(nullptr, a.E, 256, tiles_n, s_off, s_tile);
+        __syncthreads();
+        ffn_tall<UP>(a, smem, (int*)(smem + 2 * FFN_TALL_STAGE), s_off, s_tile);
+        return;
+      }
+    }
+  }
+  const int per = (ntiles + 7) >> 3;                                     // tiles of an XCD's run
+  const int first = ((int)blockIdx.x & 7) * per, last = min(first + per, ntiles), step_wg = (int)(gridDim.x + 7 - (blockIdx.x & 7)) >> 3;
+  int t = first + ((int)blockIdx.x >> 3);
+  if (t >= last) return;
+  const long long total = (long long)((last - t + step_wg - 1) / step_wg) * nsteps;   // steps of this workgroup
+
+  auto find = [&](int tile, FfnCur& c) __attribute__((always_inline)) { ffn_find<BM, BN>(a.E, N, tiles_n, s_off, s_tile, tile, c); };
+
+  // ---- the requesting side: where it is, and this lane's addresses in that tile
+  int rt_ = t, rs_ = 0, rslot = 0, rn = 0;                               // tile, step, ring position, tiles begun
+  FfnCur rc_;                                                            // the tile that begins next
+  const uint8_t* pa[IA]; const uint8_t* ps[IS]; const uint8_t* pb = nullptr;
+  uint32_t boff_lane[IB];
+#pragma unroll
+  for (int i = 0; i < IB; i++) boff_lane[i] = (uint32_t)(8 * i + (lane >> 3)) * (uint32_t)K + (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
+  // UP: the tokens of a tile's rows, requested when the tile before it begins (a load whose result is waited for would wait for everything requested in front of it)
+  auto request_ids = [&]() __attribute__((always_inline)) {
+    const int* tok = a.row_tok + (size_t)rc_.e * a.T + rc_.m0;
+    int* to = &s_ids[UP ? wave : 0][0];
+    if (lane < 8 * IA) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(tok + min(8 * IA * wave + lane, rc_.valid - 1)), (__attribute__((address_space(3))) void*)to, 4, 0, 0);
+#pragma unroll
+    for (int i = 0; i < IS; i++)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(tok + min(64 * min(wave * IS + i, SI - 1) + lane, rc_.valid - 1)), (__attribute__((address_space(3))) void*)(to + 8 * IA + 64 * i), 4, 0, 0);
+  };
+  auto begin = [&]() __attribute__((always_inline)) {
+    const FfnCur c = rc_;
+    // (read by inline assembly, its wait with it: in front of a plain read the compiler would wait for all requests in flight.  At rn = 0 they are waited for; later the wait of a step
+    // behind the one they were requested at is behind this wave: a tile has at least two steps.)
+    if constexpr (UP) { if (rn == 0) ffn_wait_vm<0>(); }
+    const uint32_t ids = (uint32_t)(uintptr_t)&s_ids[UP ? wave : 0][0];
+    auto row_of = [&](int r, int at) __attribute__((always_inline)) {     // row r of the tile, entry `at` of the list
+      int id = c.row0 + min(r, c.valid - 1);
+      if constexpr (UP) asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(id) : "v"(ids + 4u * (uint32_t)at) : "memory");
+      return (size_t)(uint32_t)id;
+    };
+#pragma unroll
+    for (int i = 0; i < IA; i++) pa[i] = A + row_of(8 * (wave * IA + i) + (lane >> 3), 8 * i + (lane >> 3)) * K + (((lane & 7) ^ (lane >> 3)) << 4);
+    pb = B + ((size_t)c.boff + (size_t)(wave * IB) * 8) * K;
+#pragma unroll
+    for (int i = 0; i < IS; i++) {
+      const int r = 64 * min(wave * IS + i, SI - 1) + lane;              // (the last waves repeat the last request)
+      const uint8_t* in_a = Ae + row_of(r, 8 * IA + 64 * i + lane) * KB;
+      const uint8_t* in_b = Be + ((size_t)c.boff + (size_t)min(max(r - BM, 0), BN - 1)) * KB;
+      ps[i] = r < BM ? in_a : in_b;
+    }
+    if (wave < WN) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a.bias[UP ? 0 : 1] + (size_t)c.e * N + (size_t)c.tn * BN + 64 * wave + lane),
+                                                    (__attribute__((address_space(3))) void*)&s_bias[rn & 1][64 * wave], 4, 0, 0);
+    rn++;
+    if (rt_ + step_wg < last) { find(rt_ + step_wg, rc_); if constexpr (UP) request_ids(); }
+  };
+  // The scales of steps q .. q + 3 (a tile's last steps may be two), sixteen bytes a row.  A row's last eight bytes come with the eight in front of them; rows of eight bytes (K = 256) as two dwords,
+  // each in a plane of its own.
+  auto request_scales = [&](int q) __attribute__((always_inline)) {
+    const int at = min(4 * q, KB - 16);
+#pragma unroll
+    for (int i = 0; i < IS; i++) {
+      const int u = min(wave * IS + i, SI - 1);
+      if ((BM + BN) % 64 == 0 || 64 * u + lane < BM + BN) {
+        if (at >= 0) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(ps[i] + at), (__attribute__((address_space(3))) void*)(scales + u * 1024), 16, 0, 0);
+        else {
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)ps[i], (__attribute__((address_space(3))) void*)(scales + u * 256), 4, 0, 0);
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(ps[i] + 4), (__attribute__((address_space(3))) void*)(scales + (BM + BN) * 4 + u * 256), 4, 0, 0);
+        }
+      }
+    }
+  };
+  // a step of the tile that is requested; q >= 0: the scales from that step on in front of it
+  auto request = [&](int q) __attribute__((always_inline)) {
+    if (rs_ == 0) begin();
+    if (q >= 0) request_scales(q);
+    uint8_t* st = smem + rslot * STAGE;
+#pragma unroll
+    for (int i = 0; i < IA; i++) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)pa[i], (__attribute__((address_space(3))) void*)(st + (wave * IA + i) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < IB; i++)                                         // (scalar base + the lane's offset: no vector address arithmetic)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(scalar_ptr(pb) + boff_lane[i]), (__attribute__((address_space(3))) void*)(st + BM * 128 + (wave * IB + i) * 1024), 16, 0, 0);
+    pb += 128;
+#pragma unroll
+    for (int i = 0; i < IA; i++) pa[i] += 128;
+    rslot = rslot + 1 == NB ? 0 : rslot + 1;
+    if (++rs_ == nsteps) { rs_ = 0; rt_ += step_wg; }
+  };
+
+  FfnCur cur;
+  find(t, cur);
+  rc_ = cur;
+  if constexpr (UP) request_ids();
+  for (int i = 0; i < NB - 1; i++) request(i == 0 ? 0 : -1);             // (a tile has at least two steps)
+  const int f0 = r16 * 128 + ((kg ^ (r16 & 7)) << 4), f1 = f0 ^ 64;
+  int slot = 0, cn = 0, stores = 0;                                      // stores: of the last tile's epilogue, at least
+  const uint32_t pick = (uint32_t)(kg | (kg + 4) << 8) | 0x0C0C0000u;    // v_perm: byte kg of two dwords
+  long long left = total;                                                // steps not yet multiplied
+  while (true) {
+    v4f32 acc[RS][4];
+#pragma unroll
+    for (int i = 0; i < RS; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[i][j] = v4f32{0.f, 0.f, 0.f, 0.f};
+    const int nsub = (((cur.valid + 15) >> 4) - wm + WM - 1) / WM;        // sub-tiles wm, wm + WM, ... of this wave that hold rows
+    uint8_t* st = smem;
+    uint32_t sca[RS], scb[4];                                             // this lane's scale bytes of the steps ahead
+    for (int s = 0; s < nsteps; s++) {
+      // This wave's requests of the step have landed, and so have the others'.  What was requested behind it may be in flight: the next step (NB = 3), the scales in front of that one, the stores
+      // of the tile before.
+      left--;
+      if (NB == 2 || left == 0) ffn_wait_vm<0>();
+      else if (s < 2) { if (stores >= 8) ffn_wait_vm<NI + 8>(); else if (stores >= 6) ffn_wait_vm<NI + 6>(); else if (stores >= 4) ffn_wait_vm<NI + 4>(); else if (stores >= 2) ffn_wait_vm<NI + 2>(); else ffn_wait_vm<NI>(); }
+      else if ((s & 3) == 3) ffn_wait_vm<NI + IS>();
+      else ffn_wait_vm<NI>();
+      asm volatile("s_barrier" ::: "memory");
+      // Into the position of the step before, which every wave has read; the scales of the next four steps once every wave has those of this group (read at its first step)
+      const int p4 = s & ~3, len = min(4, nsteps - p4), q = p4 + len;
+      if (left >= NB - 1) request(s - p4 != max(1, len - (NB - 1)) ? -1 : q < nsteps ? q : t + step_wg < last ? 0 : -1);
+      st = smem + slot * STAGE;
+      slot = slot + 1 == NB ? 0 : slot + 1;
+      if (s == p4) {
+        auto bytes = [&](int row) __attribute__((always_inline)) {       // byte i: the scale of step s + i of this lane's block
+          u32x4 d;
+          if (KB == 8) d = u32x4{((const uint32_t*)scales)[row], ((const uint32_t*)scales)[BM + BN + row], 0u, 0u}; else d = *(const u32x4*)(scales + row * 16);
+          const uint32_t lo = __builtin_amdgcn_perm(d.y, d.x, pick), hi = __builtin_amdgcn_perm(d.w, d.z, pick);
+          return KB != 8 && len == 2 ? hi : lo | (hi << 16);
+        };
+#pragma unroll
+        for (int j = 0; j < 4; j++) scb[j] = bytes(BM + wn * 64 + 16 * j + r16);
+#pragma unroll
+        for (int i = 0; i < RS; i++) sca[i] = bytes(16 * (WM * i + wm) + r16);
+      }
+      const uint8_t* As = st; const uint8_t* Bs = st + BM * 128 + wn * 4 * 2048;
+      auto multiply = [&](auto full_tag) __attribute__((always_inline)) {
+        constexpr bool FULL = decltype(full_tag)::value;                  // every sub-tile holds rows: no branches between the products
+        v8i32 bf[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const u32x4 y0 = *(const u32x4*)(Bs + j * 2048 + f0), y1 = *(const u32x4*)(Bs + j * 2048 + f1);
+          bf[j] = v8i32{(int)y0.x, (int)y0.y, (int)y0.z, (int)y0.w, (int)y1.x, (int)y1.y, (int)y1.z, (int)y1.w};
+        }
+        auto frag = [&](int i, v8i32& af) __attribute__((always_inline)) {
+          const uint8_t* p = As + (WM * i + wm) * 2048;
+          const u32x4 x0 = *(const u32x4*)(p + f0), x1 = *(const u32x4*)(p + f1);
+          af = v8i32{(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
+        };
+        v8i32 af[2];
+        frag(0, af[0]);
+#pragma unroll
+        for (int i = 0; i < RS; i++) {
+          if (i + 1 < (FULL ? RS : nsub)) frag(i + 1, af[(i + 1) & 1]);
+          if (FULL || i < nsub) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[j], af[i & 1], acc[i][j], 0, 0, 0, (int)scb[j], 0, (int)sca[i]);
+          }
+        }
+      };
+      if (RS <= 4 && nsub == RS) multiply(std::true_type{}); else if (nsub > 0) multiply(std::false_type{});
+#pragma unroll
+      for (int j = 0; j < 4; j++) scb[j] >>= 8;
+#pragma unroll
+      for (int i = 0; i < RS; i++) sca[i] >>= 8;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // every read of this position is done: behind the next barrier it is requested into
+    }
+    // ---- epilogue: the position the last step was read from is idle until the next barrier
+    asm volatile("s_barrier" ::: "memory");
+    ffn_epilogue<RS, WM, BN, UP>(a, cur, acc, nsub, wm, wn, st + wave * 2304, &s_bias[cn & 1][wn * 64]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                    // the slab has been read
+    stores = nsub > 0 ? (UP ? 2 : 1) * nsub : 0;                         // (every sub-tile stores at least its first row)
+    t += step_wg; cn++;
+    if (t >= last) break;
+    find(t, cur);
   }
 }
 
@@ -360,7 +601,7 @@ __global__ __launch_bounds__(256 * WM) void ffn_gemm_kernel(const FfnArgs a) {
 __global__ __launch_bounds__(256) void moe_combine_kernel(const FfnArgs a) {
   __shared__ int s_off[FFN_MAX_E + 1];
   __shared__ int s_row[FFN_MAX_K]; __shared__ float s_w[FFN_MAX_K];
-  ffn_offsets(a.counts, a.E, 1, 1, s_off, nullptr);
+  ffn_offsets<true>(a.counts, a.E, 1, 1, s_off, nullptr);
   __syncthreads();
   for (int t = blockIdx.x; t < a.T; t += gridDim.x) {
     if ((int)threadIdx.x < a.k) {
@@ -399,6 +640,23 @@ static FfnLayout ffn_layout(long long T, long long D, long long I, long long E, 
   return l;
 }
 
+template <int BM, int WM, int WN, int NB>
+static hipError_t launch_ffn(const FfnArgs& a, int grid, hipStream_t s) {
+  constexpr int ring = (BM + 64 * WN) * (128 * NB + 16), most = ring + 8 * (FFN_MAX_E + 1);
+  const int lds = ring + 8 * (a.E + 1);
+  auto up = ffn_gemm_kernel<BM, WM, WN, NB, true>; auto down = ffn_gemm_kernel<BM, WM, WN, NB, false>;
+  static const hipError_t configured = [&] {
+    const hipError_t e = hipFuncSetAttribute((const void*)up, hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    return e != hipSuccess ? e : hipFuncSetAttribute((const void*)down, hipFuncAttributeMaxDynamicSharedMemorySize, most);
+  }();
+  if (configured != hipSuccess) return configured;
+  up<<<grid, 64 * WM * WN, lds, s>>>(a);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  down<<<grid, 64 * WM * WN, lds, s>>>(a);
+  return hipGetLastError();
+}
+
 extern "C" {
 
 // bytes of workspace tga_moe_feed_forward needs; 0 when the sizes are outside its range (the caller then runs the single steps)
@@ -429,7 +687,10 @@ int tga_moe_feed_forward(const void* x_bf16, const float* logits, int64_t T, int
   hipStream_t s = (hipStream_t)stream;
   const long long n8 = T * (D / 8), qb = (n8 + 1023) / 1024;
   a.nq_blocks = (int)(qb < 448 ? qb : 448);
-  const int route_blocks = (int)((T + PREP_TOKENS - 1) / PREP_TOKENS);
+  // one workgroup needs no shared counters; beyond, a token per wave, until there are so many workgroups that they queue for the counters (the whole call, T = 2000, 64 experts: 155 -> 150 us with
+  // 16 tokens a workgroup instead of 64, 32: 150.3; 1600 tokens, 32 experts: 71.5 -> 65.4; 8000 tokens, 80 experts: 75.1 -> 77.9)
+  a.prep_tokens = T <= 64 || T > 4096 ? 64 : T > 2048 ? 32 : 16;
+  const int route_blocks = (int)((T + a.prep_tokens - 1) / a.prep_tokens);
   a.one_route_block = route_blocks == 1;
   if (!a.one_route_block) { moe_zero_counts_kernel<<<1, 512, 0, s>>>(a.counts, n_experts); TGA_LAUNCH_CHECK(); }
   const dim3 pg(a.nq_blocks + route_blocks);
@@ -438,17 +699,18 @@ int tga_moe_feed_forward(const void* x_bf16, const float* logits, int64_t T, int
   else moe_prep_kernel<FFN_MAX_E / 64><<<pg, 1024, 0, s>>>(a);
   TGA_LAUNCH_CHECK();
   static const int n_cu = [] { int dev = 0, n = 0; return (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) ? n : 256; }();
-  // Tiles of 32 or 256 rows by the rows per expert, us of the call (32 / 256): 64 experts, D 2048, I 512, even popularity: 16 rows 61.5 / 65.8, 24 71.3 / 67.1, 40 71.7 / 70.1, 48 90.0 / 72.3, 128 125 / 93,
-  // 200 181 / 114; popularity by 1 / rank^1.1: 16 67.5 / 74.6, 48 73.2 / 110, 64 91.7 / 132, 128 126 / 150, 200 185 / 167.  128 experts, I 768: even 32 189 / 182, 48 221 / 192, 128 349 / 231; skewed 32
-  // 191 / 219, 48 229 / 235, 64 238 / 242, 96 304 / 271.  16 experts, D 1536, I 768: 48 45.0 / 50.7, 128 53.2 / 64.9, 200 71.6 / 77.5 even, 46.0 / 68.0, 52.5 / 75.7, 72.1 / 78.5 skewed.  At 48 the even
-  // popularity gains; where it is skewed, or the experts are few, 32 rows stay better up to 128 and more, but the host does not know the counts.
-  const bool small = T * k < 48ll * n_experts;
-  if (small) {
-    ffn_gemm_kernel<32, 1, true><<<2 * n_cu, 256, 0, s>>>(a); TGA_LAUNCH_CHECK();
-    ffn_gemm_kernel<32, 1, false><<<2 * n_cu, 256, 0, s>>>(a); TGA_LAUNCH_CHECK();
+  // Tile height by the rows per expert r, us of the call (heights 16 / 32 / 64 / 128; MI355X).  64 experts, D 2048, I 512, k 8, even popularity: r = 2 50.5 / 52.0 / 51.8 / 51.2, 8 61.4 / 62.4 / 62.7 / 61.9,
+  // 32 86.6 / 69.5 / 68.4 / 69.5, 48 - / 87 / 80 / 73, 64 126 / 90 / 89 / 76, 128 199 / 125 / 119 / 112, 200 271 / 164 / 155 / 119; popularity by 1 / rank^1.1: 2 45.9 / 46.5 / 49.2 / 48.1, 16 82 / 67 / 84 / 73,
+  // 32 89 / 83 / 83 / 94, 64 127 / 90 / 92 / 100, 128 202 / 127 / 119 / 115, 200 278 / 166 / 150 / 146.  16 experts, D 1536, I 768, k 4 (few tiles: lower ones fill the chip): 16 35.2 / 33.3 / 36.3 / 40.9,
+  // 64 49.9 / 37.9 / 40.0 / 47.3, 128 66 / 53.7 / 43.1 / 51.5, 200 86 / 60.9 / 60.1 / 53.3.  Where even popularity makes 128 rows two rounds of the launch and 256 one, the device takes 256 (64 experts, r = 128 / 160: 112 -> 100, 112 -> 106): it has the counts.
+  if (T * k < 6ll * n_experts) {
+    TGA_HIP((launch_ffn<16, 1, 2, 2>(a, 4 * n_cu, s)));
+  } else if (T * k < 48ll * n_experts) {
+    TGA_HIP((launch_ffn<32, 2, 2, 2>(a, 3 * n_cu, s)));
+  } else if (4 * (n_experts * ((T * k + 128ll * n_experts - 1) / (128ll * n_experts)) * (2 * I / 256)) < 3 * n_cu) {
+    TGA_HIP((launch_ffn<64, 2, 2, 2>(a, 2 * n_cu, s)));
   } else {
-    ffn_gemm_kernel<256, 2, true><<<n_cu, 512, 0, s>>>(a); TGA_LAUNCH_CHECK();
-    ffn_gemm_kernel<256, 2, false><<<n_cu, 512, 0, s>>>(a); TGA_LAUNCH_CHECK();
+    TGA_HIP((launch_ffn<128, 2, 4, 3>(a, n_cu, s)));
   }
   moe_combine_kernel<<<(unsigned)(T < 2048 ? T : 2048), 256, 0, s>>>(a);
   TGA_LAUNCH_CHECK();

@@ -36,7 +36,7 @@ __device__ __forceinline__ uint32_t e4m3x4(float a, float b, float c, float d) {
 __device__ __forceinline__ uint32_t e4m3x2(float a, float b) { return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(mx_clamp(a), mx_clamp(b), 0, false) & 0xFFFFu; }
 // 1 / (1 + exp(-x)) of a bf16 value on its way to bf16.  The scaling by 2^-24 keeps the reciprocal out of the subnormal numbers, which v_rcp_f32 flushes to zero (x = -87.5 .. -88.5); after the
 // rounding to bf16 the result is that of expf and a rounded division for all 2^16 inputs (enumerated), in a fifth of the operations.
-__device__ __forceinline__ float mx_sigmoid_bf16(float x) { return __builtin_amdgcn_rcpf((1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x)) * 0x1p-24f) * 0x1p-24f; }
+__device__ __forceinline__ float mx_sigmoid_bf16(float x) { return __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_amdgcn_exp2f(-1.4426950408889634f * x), 0x1p-24f, 0x1p-24f)) * 0x1p-24f; }
 
 __device__ __forceinline__ float quad_max(float v) {                    // over the four lanes of a quad
   v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true)));     // quad_perm [1,0,3,2]
