@@ -80,3 +80,26 @@ def test_synth_q4_k_writer_produces_valid_blocks(gpu):
   w = og.ggml_data_to_tensor(buf.numpy(), n, 12)
   assert np.isfinite(w).all() and np.abs(w).max() <= amp * 1.1 and w.std() > amp * 0.4
   assert _gpu_dequant(gpu, buf.numpy(), n, 12).tobytes() == w.tobytes()
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("f16", [True, False])
+def test_large_results_are_those_of_their_parts(gpu, t, f16):
+  """Results of 16 MB and more leave past the caches: the bits of the same blocks in runs below that, at the smallest such size, one block more, and (fp16) an output that starts two bytes
+  off a dword; the bytes around it stay."""
+  nel, nby = GGML_QUANT[t]
+  n = (16 << 20) // (2 if f16 else 4) + nel
+  n -= n % nel
+  rng = np.random.default_rng(t)
+  data = np.tile(synth.random_blocks(rng, t, 64, 1024), -(-n // 65536))[:n // nel * nby]
+  src, sz, L = gpu.Buffer.from_numpy(data), 2 if f16 else 4, gpu.lib()
+  half = n // nel // 2
+  ref = gpu.Buffer((n * sz,), np.uint8)
+  for b0, nb in ((0, half), (half, n // nel - half)):
+    gpu.check(L.tga_dequant(t, src.ptr + b0 * nby, nb * nel, ref.ptr + b0 * nel * sz, gpu.dtype_code(np.float16 if f16 else np.float32), None))
+  ref = ref.numpy()
+  for off in ((16, 18) if f16 else (16,)):
+    out = gpu.Buffer((n * sz + 64,), np.uint8)
+    gpu.check(L.tga_memset(out.ptr, 0xAB, out.nbytes, None))
+    gpu.check(L.tga_dequant(t, src.ptr, n, out.ptr + off, gpu.dtype_code(np.float16 if f16 else np.float32), None))
+    got = out.numpy()
+    assert (got[off:off + n * sz] != ref).sum() == 0 and (got[:off] == 0xAB).all() and (got[off + n * sz:] == 0xAB).all(), off

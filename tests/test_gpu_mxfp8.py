@@ -238,6 +238,26 @@ def test_quantize_rows_of_any_length(gpu, rows, K):
     assert (packed is None) == (K % 128 != 0)
     if packed is not None: np.testing.assert_array_equal(packed.numpy(), re8.reshape(rows, K // 128, 4).view(np.uint32)[..., 0].T)
 
+def test_large_quantized_results_are_those_of_their_parts(gpu):
+  """Results of 16 MB and more leave past the caches: rows of float32, of bf16, of the fused SwiGLU and of the transposed form against the same rows in parts below that."""
+  from tinygrad_amd import moe
+  rows, K = 4100, 4096
+  rng = np.random.default_rng(9)
+  x = rng.standard_normal((rows, K), dtype=np.float32) * np.exp2(rng.integers(-20, 12, size=(rows, 1))).astype(np.float32)
+  bits, up = moe.to_bf16_bits(x), moe.to_bf16_bits(x[::-1])
+  B = gpu.Buffer.from_numpy
+  for whole, part in ((lambda: moe.quantize_mxfp8(B(x)), lambda a, b: moe.quantize_mxfp8(B(x[a:b]))), (lambda: moe.quantize_mxfp8(B(bits)), lambda a, b: moe.quantize_mxfp8(B(bits[a:b]))),
+                      (lambda: moe.fused_silu_mul_quantize_mxfp8(B(bits), B(up)), lambda a, b: moe.fused_silu_mul_quantize_mxfp8(B(bits[a:b]), B(up[a:b])))):
+    q, e8, packed = (b.numpy() for b in whole())
+    for a, b in ((0, 2050), (2050, rows)):
+      rq, re8, rp = (v.numpy() for v in part(a, b))
+      assert (q[a:b] != rq).sum() == 0 and (e8[a:b] != re8).sum() == 0 and (packed[:, a:b] != rp).sum() == 0
+  g = bits[:4096]                                                      # (columns of the source are rows of the result)
+  q, e8, packed = (b.numpy() for b in moe.transpose_quantize_mxfp8(B(g)))
+  for a, b in ((0, 2048), (2048, K)):
+    rq, re8, rp = (v.numpy() for v in moe.transpose_quantize_mxfp8(B(np.ascontiguousarray(g[:, a:b]))))
+    assert (q[a:b] != rq).sum() == 0 and (e8[a:b] != re8).sum() == 0 and (packed[:, a:b] != rp).sum() == 0
+
 @pytest.mark.parametrize("M,N", [(32, 64), (96, 128), (128, 64), (160, 192), (512, 256)])
 def test_transpose_quantize_of_ragged_row_counts(gpu, M, N):
   """Row counts that end inside a 128-row tile (no packed scales there) against quantize_mxfp8 of the transposed matrix, bit for bit."""

@@ -1,12 +1,13 @@
 // Block dequant kernels: bit-exact restatement of ggml_data_to_tensor (tinygrad/llm/gguf.py:23-119) for Q4_0 (:46), Q4_1 (:47-49), Q5_0 / Q5_1 (:50-55), Q8_0 (:56),
 // Q4_K / Q5_K (:57-67), Q6_K (:68-72), IQ3_XXS / IQ3_S / IQ2_S (:73-95), IQ4_XS (:96-104), MXFP4 (:105-114) and Q1_0 (:115-118).  One thread produces the
 // consecutive results of one 16-byte store: eight fp16, which share their sub-block's header, or four fp32.  What bounds it is the number of requests, not their bytes: one per header field and
-// one per four codes, whatever the block's alignment, where a byte at a time took twice as many (14336 x 4096 to fp16, back to back: Q4_K 43 -> 25 us, 5.9 TB/s; Q4_0 28.5 -> 22.7; MXFP4 50 -> 29;
-// eight fp32 per thread are two stores with gaps between lanes: Q4_0 43 us, four 38).
+// one per four codes, whatever the block's alignment, where a byte at a time took twice as many (14336 x 4096 to fp16, back to back into one buffer: Q4_K 43 -> 25 us; Q4_0 28.5 -> 22.7; MXFP4 50 -> 29;
+// eight fp32 per thread are two stores with gaps between lanes: Q4_0 43 us, four 38).  Into memory that no cache holds, with stores past the caches: Q4_K 42.4 -> 24.7 us (6.1 TB/s), Q4_0 32.3 -> 21.7,
+// Q6_K 36.1 -> 34.8, MXFP4 49.3 -> 41.6, Q4_K to fp32 70.6 -> 39.3.
 #include "deq.h"
 #include "host.h"
 
-template <int T, bool F16>
+template <int T, bool F16, bool PAST>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ blocks, uint8_t* __restrict__ out, int64_t nv) {
   constexpr int V = F16 ? 8 : 4;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nv; i += (int64_t)gridDim.x * 256) {
@@ -20,10 +21,11 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
 #pragma unroll
       for (int q = 0; q < 8; q++) asm volatile("" : "+v"(o[q]));
       const u32x4 v = {f2h_bits(o[0]) | (f2h_bits(o[1]) << 16), f2h_bits(o[2]) | (f2h_bits(o[3]) << 16), f2h_bits(o[4]) | (f2h_bits(o[5]) << 16), f2h_bits(o[6]) | (f2h_bits(o[7]) << 16)};
-      __builtin_memcpy(out + 16 * i, &v, 16);                              // (a store that asks for no more alignment than two of four values did)
+      typedef u32x4 any_u32x4 __attribute__((aligned(2)));                 // (a store that asks for no more alignment than two of four values did)
+      store_result<PAST, any_u32x4>(v, (any_u32x4*)(out + 16 * i));
     } else {
       const f32x4 v = {o[0], o[1], o[2], o[3]};
-      ((f32x4*)out)[i] = v;
+      store_result<PAST>(v, (f32x4*)out + i);
     }
   }
 }
@@ -31,10 +33,11 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
 template <int T> static int launch_dequant(const void* blocks, int64_t n, void* out, int out_dtype, hipStream_t s) {
   TGA_REQUIRE(n % Deq<T>::NEL == 0, "tga_dequant: n=%lld is not a multiple of the block size %d", (long long)n, Deq<T>::NEL);
   if (n == 0) return 0;
+  const bool past = n * (out_dtype == TGA_F32 ? 4 : 2) >= TGA_PAST_BYTES;
   const int64_t nv = n / (out_dtype == TGA_F32 ? 4 : 8);
   const int grid = (int)((nv + 255) / 256 < 65536 ? (nv + 255) / 256 : 65536);
-  if (out_dtype == TGA_F32) dequant_kernel<T, false><<<grid, 256, 0, s>>>((const uint8_t*)blocks, (uint8_t*)out, nv);
-  else dequant_kernel<T, true><<<grid, 256, 0, s>>>((const uint8_t*)blocks, (uint8_t*)out, nv);
+  auto kern = out_dtype == TGA_F32 ? (past ? dequant_kernel<T, false, true> : dequant_kernel<T, false, false>) : (past ? dequant_kernel<T, true, true> : dequant_kernel<T, true, false>);
+  kern<<<grid, 256, 0, s>>>((const uint8_t*)blocks, (uint8_t*)out, nv);
   TGA_LAUNCH_CHECK();
   return 0;
 }

@@ -11,7 +11,7 @@
 // ------------------------------------------------------------------------------------------------ quantize_mxfp8
 // A block of 32 values: e8 = clamp(floor(log2(max(amax, 1e-38))) + 127, 0, 254), q = e4m3(clamp(x * 2^(127 - e8), +-448)).  Four neighbouring lanes hold a block, eight
 // values each: every load and store of a wave covers one contiguous span (a thread per block read 16 bytes of every 64, and converted in ~30 operations per value
-// what v_cvt_pk_fp8_f32 converts two at a time: 16384 x 4096 bf16 rows 59 us; now 46 us for the whole call, 4.5 TB/s where a large copy moves 5.0), the block maximum takes two quad permutations.
+// what v_cvt_pk_fp8_f32 converts two at a time: 16384 x 4096 bf16 rows 59 us; 46 us for the whole call; 43.7 -> 39.3 with results past the caches, 5.2 TB/s), the block maximum takes two quad permutations.
 // Also writes the packed scales of mx_pack: packed[k / 128][row] = 4 consecutive e8 bytes (little-endian), one dword per sixteen lanes.
 // MODE 0: x float32; 1: x bf16; 2: fused SwiGLU producer, value = w1 * sigmoid(w1) * w3 in float32 from two bf16 tensors x (= x_w1)
 // and x2 (= x_w3), sigmoid as 1 / (1 + exp2(-w1 * log2(e)))  (extra/llama_kernels/fused_silu_mul_quantize_mxfp8/__init__.py:33-36)
@@ -19,11 +19,11 @@ __device__ __forceinline__ void bf16x8(const u32x4 w, float* o) {
 #pragma unroll
   for (int i = 0; i < 4; i++) { o[2 * i] = bf16_lo(w[i]); o[2 * i + 1] = bf16_hi(w[i]); }
 }
-template <int MODE>
+template <int MODE, bool PAST>
 __global__ __launch_bounds__(256) void quantize_mxfp8_kernel(const void* __restrict__ x, const void* __restrict__ x2, const long long rows, const int K, uint8_t* __restrict__ q,
                                                              uint8_t* __restrict__ e8, uint8_t* __restrict__ packed) {
   const long long n8 = rows * (K / 8), stride = (long long)gridDim.x * 256;             // pieces of eight values
-  constexpr int U = MODE == 1 ? 4 : 2;                                                   // pieces per thread and trip: their loads go out together
+  constexpr int U = 2;                                                                   // pieces per thread and trip: their loads go out together (four of bf16: 41.0 against 39.3 us)
   for (long long p0 = (long long)blockIdx.x * 256 + threadIdx.x; p0 < n8; p0 += U * stride) {
     u32x4 a[U], b[U];
 #pragma unroll
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256) void quantize_mxfp8_kernel(const void* __restr
       for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v[i]));
       const int e = mx_e8(quad_max(amax));
       const float s = mx_scale(e);
-      ((u32x2*)q)[p] = u32x2{e4m3x4(v[0] * s, v[1] * s, v[2] * s, v[3] * s), e4m3x4(v[4] * s, v[5] * s, v[6] * s, v[7] * s)};
+      store_result<PAST>(u32x2{e4m3x4(v[0] * s, v[1] * s, v[2] * s, v[3] * s), e4m3x4(v[4] * s, v[5] * s, v[6] * s, v[7] * s)}, (u32x2*)q + p);
       const int lane = threadIdx.x & 63;
       if ((lane & 3) == 0) e8[p >> 2] = (uint8_t)e;
       if (packed) {                                                                      // (K % 128 == 0: the sixteen lanes of a dword sit in one row)
@@ -67,6 +67,7 @@ __global__ __launch_bounds__(256) void quantize_mxfp8_kernel(const void* __restr
 // tensor: g (M, N) bf16 -> q (N, M), e8 (N, M / 32), packed (M / 128, N).  One workgroup takes 128 rows x 64 columns of g through LDS (row-wise 16-byte loads).  A thread
 // reads two neighbouring columns at once (one dword per row), sixteen rows of them; a block is the sixteen rows of two threads eight lanes apart in the row
 // run index, and the eight runs of a column fill one 128-byte line of q.
+template <bool PAST>
 __global__ __launch_bounds__(256) void transpose_quantize_mxfp8_kernel(const uint16_t* __restrict__ g, int M, int N, uint8_t* __restrict__ q,
                                                                        uint8_t* __restrict__ e8, uint8_t* __restrict__ packed) {
   __shared__ uint32_t tile[128][33];                        // 132-byte rows: the column reads of eight 16-row runs fall on different banks
@@ -75,7 +76,7 @@ __global__ __launch_bounds__(256) void transpose_quantize_mxfp8_kernel(const uin
   for (int p = 0; p < 4; p++) {
     const int r = p * 32 + (t >> 3), c4 = (t & 7) * 4;
     u32x4 w = {0, 0, 0, 0};
-    if (m0 + r < M) w = *(const u32x4*)(g + (size_t)(m0 + r) * N + n0 + 2 * c4);
+    if (m0 + r < M) w = __builtin_nontemporal_load((const u32x4*)(g + (size_t)(m0 + r) * N + n0 + 2 * c4));     // (128 bytes of a row: used once)
 #pragma unroll
     for (int i = 0; i < 4; i++) tile[r][c4 + i] = w[i];
   }
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(256) void transpose_quantize_mxfp8_kernel(const uin
     for (int i = 0; i < 4; i++) o[i] = e4m3x4(v[4 * i] * s, v[4 * i + 1] * s, v[4 * i + 2] * s, v[4 * i + 3] * s);
     const int kb = (m0 >> 5) + (run >> 1);
     if (live) {
-      *(u32x4*)(q + n * M + m0 + run * 16) = o;
+      store_result<PAST>(o, (u32x4*)(q + n * M + m0 + run * 16));
       if (!(run & 1)) e8[n * (M / 32) + kb] = (uint8_t)e;
     }
     if (packed) {                                           // (M % 128 == 0: every run is live)
@@ -494,10 +495,10 @@ __global__ __launch_bounds__(256) void add_expert_bias_kernel(uint16_t* __restri
   }
 }
 
-// workgroups for n8 pieces of eight values, u per thread and trip: one trip each up to 8192 workgroups
-static int quantize_grid(long long n8, int u) {
-  const long long full = (n8 + 255) / 256, want = (full + u - 1) / u;
-  return (int)(want < 512 ? (full < 512 ? full : 512) : want < 8192 ? want : 8192);
+// workgroups for n8 pieces of eight values, two per thread and trip: one trip each up to 65536 workgroups
+static int quantize_grid(long long n8) {
+  const long long full = (n8 + 255) / 256, want = (full + 1) / 2;
+  return (int)(want < 512 ? (full < 512 ? full : 512) : want < 65536 ? want : 65536);
 }
 
 extern "C" {
@@ -507,9 +508,10 @@ int tga_quantize_mxfp8(const void* x, int x_is_bf16, int64_t rows, int64_t K, vo
   TGA_REQUIRE(rows >= 0 && K > 0 && K % 32 == 0, "tga_quantize_mxfp8: K=%lld must be a positive multiple of 32", (long long)K);
   TGA_REQUIRE(!packed || K % 128 == 0, "tga_quantize_mxfp8: packed scales need K %% 128 == 0");
   if (rows == 0) return 0;
-  const int grid = quantize_grid(rows * (K / 8), x_is_bf16 ? 4 : 2);
-  if (x_is_bf16) quantize_mxfp8_kernel<1><<<grid, 256, 0, (hipStream_t)stream>>>(x, nullptr, rows, (int)K, (uint8_t*)q, (uint8_t*)e8, (uint8_t*)packed);
-  else quantize_mxfp8_kernel<0><<<grid, 256, 0, (hipStream_t)stream>>>(x, nullptr, rows, (int)K, (uint8_t*)q, (uint8_t*)e8, (uint8_t*)packed);
+  const int grid = quantize_grid(rows * (K / 8));
+  const bool past = rows * K >= TGA_PAST_BYTES;
+  auto kern = x_is_bf16 ? (past ? quantize_mxfp8_kernel<1, true> : quantize_mxfp8_kernel<1, false>) : (past ? quantize_mxfp8_kernel<0, true> : quantize_mxfp8_kernel<0, false>);
+  kern<<<grid, 256, 0, (hipStream_t)stream>>>(x, nullptr, rows, (int)K, (uint8_t*)q, (uint8_t*)e8, (uint8_t*)packed);
   TGA_LAUNCH_CHECK();
   return 0;
 }
@@ -519,8 +521,9 @@ int tga_silu_mul_quantize_mxfp8(const void* x_w1_bf16, const void* x_w3_bf16, in
   TGA_REQUIRE(rows >= 0 && K > 0 && K % 32 == 0, "tga_silu_mul_quantize_mxfp8: K=%lld must be a positive multiple of 32", (long long)K);
   TGA_REQUIRE(!packed || K % 128 == 0, "tga_silu_mul_quantize_mxfp8: packed scales need K %% 128 == 0");
   if (rows == 0) return 0;
-  const int grid = quantize_grid(rows * (K / 8), 2);
-  quantize_mxfp8_kernel<2><<<grid, 256, 0, (hipStream_t)stream>>>(x_w1_bf16, x_w3_bf16, rows, (int)K, (uint8_t*)q, (uint8_t*)e8, (uint8_t*)packed);
+  const int grid = quantize_grid(rows * (K / 8));
+  auto kern = rows * K >= TGA_PAST_BYTES ? quantize_mxfp8_kernel<2, true> : quantize_mxfp8_kernel<2, false>;
+  kern<<<grid, 256, 0, (hipStream_t)stream>>>(x_w1_bf16, x_w3_bf16, rows, (int)K, (uint8_t*)q, (uint8_t*)e8, (uint8_t*)packed);
   TGA_LAUNCH_CHECK();
   return 0;
 }
@@ -530,7 +533,8 @@ int tga_transpose_quantize_mxfp8(const void* g_bf16, int64_t M, int64_t N, void*
   TGA_REQUIRE(M > 0 && N > 0 && M % 32 == 0 && N % 64 == 0, "tga_transpose_quantize_mxfp8: M=%lld must be a multiple of 32 and N=%lld of 64", (long long)M, (long long)N);
   TGA_REQUIRE(!packed || M % 128 == 0, "tga_transpose_quantize_mxfp8: packed scales need M %% 128 == 0");
   TGA_REQUIRE(M < (1ll << 31) && N < (1ll << 31) && (M + 127) / 128 <= 65535, "tga_transpose_quantize_mxfp8: matrix too large");
-  transpose_quantize_mxfp8_kernel<<<dim3((unsigned)(N / 64), (unsigned)((M + 127) / 128)), 256, 0, (hipStream_t)stream>>>((const uint16_t*)g_bf16, (int)M, (int)N, (uint8_t*)q, (uint8_t*)e8,
+  auto kern = M * N >= TGA_PAST_BYTES ? transpose_quantize_mxfp8_kernel<true> : transpose_quantize_mxfp8_kernel<false>;
+  kern<<<dim3((unsigned)(N / 64), (unsigned)((M + 127) / 128)), 256, 0, (hipStream_t)stream>>>((const uint16_t*)g_bf16, (int)M, (int)N, (uint8_t*)q, (uint8_t*)e8,
                                                                                                                         (uint8_t*)packed);
   TGA_LAUNCH_CHECK();
   return 0;
