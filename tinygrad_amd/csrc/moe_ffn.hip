@@ -8,7 +8,7 @@
 // add_expert_bias -> swiglu -> quantize_mxfp8 -> grouped_mx_gemm -> add_expert_bias -> combine: every rounding to bf16 and to E4M3 sits where it sits there.  What
 // is gone are the passes between them (T = 4096, k = 8, E = 128, D = 2048, I = 768: dispatch, two quantisations, two bias adds, SwiGLU over 65536 padded rows) and the
 // padding of every expert's rows to 256, and the host work of eleven entry points.  MI355X, back to back: T = 2000, k = 8, E = 64, D = 2048, I = 512, popularity
-// by 1 / rank^1.1: 2480 (single passes: 810) -> 182 -> 150 us; T = 32, k = 8, E = 64, I = 768: 840 (single) -> 77 -> 67 us; T = 4096, E = 128, I = 768: 1340 (single) -> 406 -> 370 us.  The second step of
+// by 1 / rank^1.1: 2480 (single passes: 810) -> 182 -> 150 us; T = 32, k = 8, E = 64, I = 768: 840 (single) -> 77 -> 62 us; T = 4096, E = 128, I = 768: 1340 (single) -> 406 -> 370 us.  The second step of
 // each: operands by direct-to-LDS loads instead of through registers, scales sixteen bytes a row, lower tiles, routing workgroups of 16 tokens.
 #include "mxfp8.h"
 #include "host.h"
@@ -379,9 +379,9 @@ __device__ __forceinline__ void ffn_tall(const FfnArgs& a, uint8_t* smem, int* s
 // Operands go to a ring of NB steps in LDS by direct-to-LDS loads, NB - 1 steps ahead of the multiplication and across tile borders: one barrier per step, no registers in between.
 // A step's region: rows of 128 bytes, 16-byte chunk c of row R at chunk c ^ (R & 7) (a request covers eight whole rows, a read of sixteen rows meets each bank group once
 // per eight lanes).  Scales come four steps at a time, sixteen bytes a row: a dword a row and step was 64 cache lines a request, a fifth of the time.  Rows beyond the expert's repeat its last one.
-// UP: gate/up (rows gathered by token, epilogue bias + clamped interleaved SwiGLU + quantisation) or down (compact rows, epilogue bias).
+// UP: gate/up (rows gathered by token, epilogue bias + clamped interleaved SwiGLU + quantisation) or down (compact rows, epilogue bias).  ONCE: weights requested past the caches.
 // Measured (us, gate/up + down): 16000 rows of 64 experts skewed, D 2048, I 512, tiles of 128: 97.5 + 52.7 (tiles of 256 through registers) -> 79 + 42; 256 rows of 64 experts, I 768, tiles of 16:
-// 42.1 + 23.3 -> 35.8 + 20.2, which is 4.6 TB/s of weights.  What bounds the first: a step is 1.4 us of which 0.45 are products (eight waves read 128 KB of LDS, then multiply, in one phase;
+// 42.1 + 23.3 -> 35.8 + 20.2, past the caches 31.5 + 19.1: 5.2 TB/s of weights.  What bounds the first: a step is 1.4 us of which 0.45 are products (eight waves read 128 KB of LDS, then multiply, in one phase;
 // two groups of waves half a step apart with a barrier each half: 77 + 44, not kept), the epilogue's 400 vector instructions per sub-tile 6 us a tile, and 2.4 rounds of tiles on 256 CUs.
 __device__ __forceinline__ const uint8_t* scalar_ptr(const uint8_t* p) {
   const uint64_t v = (uint64_t)(uintptr_t)p;
@@ -391,7 +391,7 @@ __device__ __forceinline__ const uint8_t* scalar_ptr(const uint8_t* p) {
 }
 template <int N> __device__ __forceinline__ void ffn_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
 
-template <int BM, int WM, int WN, int NB, bool UP>
+template <int BM, int WM, int WN, int NB, bool UP, bool ONCE>
 __global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a) {
   constexpr int NW = WM * WN, BN = 64 * WN, RS = BM / 16 / WM;          // waves, weight rows of a tile, 16-row sub-tiles of a wave
   constexpr int IA = BM / 8 / NW, IB = BN / 8 / NW, SI = (BM + BN + 63) / 64, IS = (SI + NW - 1) / NW, NI = IA + IB;   // requests of a wave: eight rows of operands a step, 64 rows' scales of four steps
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a)
     for (int i = 0; i < IA; i++) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)pa[i], (__attribute__((address_space(3))) void*)(st + (wave * IA + i) * 1024), 16, 0, 0);
 #pragma unroll
     for (int i = 0; i < IB; i++)                                         // (scalar base + the lane's offset: no vector address arithmetic)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(scalar_ptr(pb) + boff_lane[i]), (__attribute__((address_space(3))) void*)(st + BM * 128 + (wave * IB + i) * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(scalar_ptr(pb) + boff_lane[i]), (__attribute__((address_space(3))) void*)(st + BM * 128 + (wave * IB + i) * 1024), 16, 0, ONCE ? 2 : 0);
     pb += 128;
 #pragma unroll
     for (int i = 0; i < IA; i++) pa[i] += 128;
@@ -640,11 +640,11 @@ static FfnLayout ffn_layout(long long T, long long D, long long I, long long E, 
   return l;
 }
 
-template <int BM, int WM, int WN, int NB>
+template <int BM, int WM, int WN, int NB, bool ONCE>
 static hipError_t launch_ffn(const FfnArgs& a, int grid, hipStream_t s) {
   constexpr int ring = (BM + 64 * WN) * (128 * NB + 16), most = ring + 8 * (FFN_MAX_E + 1);
   const int lds = ring + 8 * (a.E + 1);
-  auto up = ffn_gemm_kernel<BM, WM, WN, NB, true>; auto down = ffn_gemm_kernel<BM, WM, WN, NB, false>;
+  auto up = ffn_gemm_kernel<BM, WM, WN, NB, true, ONCE>; auto down = ffn_gemm_kernel<BM, WM, WN, NB, false, ONCE>;
   static const hipError_t configured = [&] {
     const hipError_t e = hipFuncSetAttribute((const void*)up, hipFuncAttributeMaxDynamicSharedMemorySize, most);
     return e != hipSuccess ? e : hipFuncSetAttribute((const void*)down, hipFuncAttributeMaxDynamicSharedMemorySize, most);
@@ -703,14 +703,17 @@ int tga_moe_feed_forward(const void* x_bf16, const float* logits, int64_t T, int
   // 32 86.6 / 69.5 / 68.4 / 69.5, 48 - / 87 / 80 / 73, 64 126 / 90 / 89 / 76, 128 199 / 125 / 119 / 112, 200 271 / 164 / 155 / 119; popularity by 1 / rank^1.1: 2 45.9 / 46.5 / 49.2 / 48.1, 16 82 / 67 / 84 / 73,
   // 32 89 / 83 / 83 / 94, 64 127 / 90 / 92 / 100, 128 202 / 127 / 119 / 115, 200 278 / 166 / 150 / 146.  16 experts, D 1536, I 768, k 4 (few tiles: lower ones fill the chip): 16 35.2 / 33.3 / 36.3 / 40.9,
   // 64 49.9 / 37.9 / 40.0 / 47.3, 128 66 / 53.7 / 43.1 / 51.5, 200 86 / 60.9 / 60.1 / 53.3.  Where even popularity makes 128 rows two rounds of the launch and 256 one, the device takes 256 (64 experts, r = 128 / 160: 112 -> 100, 112 -> 106): it has the counts.
+  // Low tiles read a weight about once.  Where the layer's weights are also more than half of the 256 MB behind the L2s, so that they are not there again at the next call, the requests pass them by:
+  // 32 tokens of 64 experts, I 768 67.7 -> 61.9 us, r = 4, I 512 56.5 -> 51.1, r = 24 64.7 -> 61.7; of 57 MB that are still there 32.4 -> 36.1.
+  const bool once = 3ll * n_experts * I * D >= (128ll << 20);
   if (T * k < 6ll * n_experts) {
-    TGA_HIP((launch_ffn<16, 1, 2, 2>(a, 4 * n_cu, s)));
+    TGA_HIP((once ? launch_ffn<16, 1, 2, 2, true>(a, 4 * n_cu, s) : launch_ffn<16, 1, 2, 2, false>(a, 4 * n_cu, s)));
   } else if (T * k < 48ll * n_experts) {
-    TGA_HIP((launch_ffn<32, 2, 2, 2>(a, 3 * n_cu, s)));
+    TGA_HIP((once ? launch_ffn<32, 2, 2, 2, true>(a, 3 * n_cu, s) : launch_ffn<32, 2, 2, 2, false>(a, 3 * n_cu, s)));
   } else if (4 * (n_experts * ((T * k + 128ll * n_experts - 1) / (128ll * n_experts)) * (2 * I / 256)) < 3 * n_cu) {
-    TGA_HIP((launch_ffn<64, 2, 2, 2>(a, 2 * n_cu, s)));
+    TGA_HIP((launch_ffn<64, 2, 2, 2, false>(a, 2 * n_cu, s)));
   } else {
-    TGA_HIP((launch_ffn<128, 2, 4, 3>(a, n_cu, s)));
+    TGA_HIP((launch_ffn<128, 2, 4, 3, false>(a, n_cu, s)));
   }
   moe_combine_kernel<<<(unsigned)(T < 2048 ? T : 2048), 256, 0, s>>>(a);
   TGA_LAUNCH_CHECK();

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(QD_NW * 64) void qgemm_dma_kernel(const QArgs args,
     for (int i = 0; i < IMAX; i++) {
       const int j = wave + QD_NW * i;
       if (j < NI2)                                                     // (the same for the whole wave)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((from_up[i] ? base_up : base) + (two ? doff[i] : doff_odd[i])), (__attribute__((address_space(3))) void*)(dst + j * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((from_up[i] ? base_up : base) + (two ? doff[i] : doff_odd[i])), (__attribute__((address_space(3))) void*)(dst + j * 1024), 16, 0, T_ == GGML_Q6_K ? 0 : 2);     // (past the caches: see qgemm_wp.hip)
     }
     if (++ist == spg) { ist = 0; ij++; }
     islot = islot + 1 == nb ? 0 : islot + 1;
