@@ -349,7 +349,7 @@ template <> struct Fmt<GGML_F16> {
   static __device__ __forceinline__ Raw load_nu(const uint8_t* row, int u, int nu) {
     const uint8_t* p = row + 16 * u; Raw r;
 #pragma unroll
-    for (int i = 0; i < 8; i++) r.q[i] = ld16_a4(p + (size_t)16 * nu * i);
+    for (int i = 0; i < 8; i++) r.q[i] = __builtin_nontemporal_load((const TGA_GLOBAL u32x4_a4*)(p + (size_t)16 * nu * i));   // (whole lines per request, read once: past the caches)
     return r;
   }
   static __device__ __forceinline__ int xoff(int u, int k) { return 64 * u + 2 * k; }
