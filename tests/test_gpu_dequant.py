@@ -103,3 +103,21 @@ def test_large_results_are_those_of_their_parts(gpu, t, f16):
     gpu.check(L.tga_dequant(t, src.ptr, n, out.ptr + off, gpu.dtype_code(np.float16 if f16 else np.float32), None))
     got = out.numpy()
     assert (got[off:off + n * sz] != ref).sum() == 0 and (got[:off] == 0xAB).all() and (got[off + n * sz:] == 0xAB).all(), off
+
+@pytest.mark.parametrize("t", TYPES)
+def test_ragged_last_workgroups_and_unaligned_blocks(gpu, t):
+  """One block, a block less and more than a workgroup's run of 2048 or 4096 values, and block bytes that start two past a 16-byte boundary: the
+  oracle's bits in float32 and their cast in fp16, the byte behind the result untouched."""
+  nel, nby = GGML_QUANT[t]
+  rng = np.random.default_rng(100 + t)
+  for nb in sorted({1, 2048 // nel - 1, 2048 // nel + 1, 4096 // nel - 1, 4096 // nel, 4096 // nel + 1, 3 * 4096 // nel + 2} - {0}):
+    data = synth.random_blocks(rng, t, 1, nb * nel)
+    ref = og.ggml_data_to_tensor(data, nb * nel, t)
+    for at in (0, 2):
+      src = gpu.Buffer.from_numpy(np.concatenate([np.zeros(at, np.uint8), data]))
+      for f16, sz in ((True, 2), (False, 4)):
+        out = gpu.Buffer((nb * nel * sz + 16,), np.uint8)
+        gpu.check(gpu.lib().tga_memset(out.ptr, 0xAB, out.nbytes, None))
+        gpu.check(gpu.lib().tga_dequant(t, src.ptr + at, nb * nel, out.ptr, gpu.dtype_code(np.float16 if f16 else np.float32), None))
+        got, exp = out.numpy(), (ref.astype(np.float16) if f16 else ref)
+        assert got[:nb * nel * sz].tobytes() == exp.tobytes() and (got[nb * nel * sz:] == 0xAB).all(), (nb, at, f16)
