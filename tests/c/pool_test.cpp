@@ -45,6 +45,9 @@ static hipError_t hipFree(void* p) {
   g_live.erase(p); g_used -= g_size[p]; g_waits++;                          // (waits for the device)
   return hipSuccess;
 }
+enum { hipHostMallocDefault = 0 };
+static hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
+static hipError_t hipHostFree(void* p) { return hipFree(p); }
 [[maybe_unused]] static hipError_t hipDeviceSynchronize() { if (hipError_t e = refused()) return e; if (g_other_capture) { g_capture_broken = true; return hipErrorStreamCaptureUnsupported; } g_waits++; return hipSuccess; }
 static hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 [[maybe_unused]] static hipError_t hipGetLastError() { return hipSuccess; }
@@ -145,9 +148,20 @@ static void full_of_other_blocks() {
   }
   CHECK(g_pools[0].kept <= POOL_BYTES);
 }
+static void pinned_freed_in_a_capture() {
+  for (int own = 0; own < 2; own++) {                                       // (a capture that something else opened, and one of the library's)
+    void *a, *b; CHECK(!pinned_malloc(&a, 64)); CHECK(!pinned_malloc(&b, 64));
+    t_captures = own; g_capturing = true;
+    CHECK(!pinned_free(a)); CHECK(pinned_free(a) != 0); CHECK(!g_capture_broken && g_live.count(a));
+    if (own) { void* c = nullptr; CHECK(pinned_malloc(&c, 64) != 0 && !c); CHECK(!g_capture_broken); }
+    t_captures = 0; g_capturing = false;
+    void* c; CHECK(!pinned_malloc(&c, 64)); CHECK(!g_live.count(a));
+    CHECK(!pinned_free(b)); CHECK(!pinned_free(c)); CHECK(!pool_give_back()); CHECK(g_live.empty());
+  }
+}
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}, {"capture_of_its_own", capture_of_its_own}, {"classes_hold_little_more", classes_hold_little_more}, {"no_host_memory", no_host_memory}, {"full_of_other_blocks", full_of_other_blocks}};
+  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}, {"capture_of_its_own", capture_of_its_own}, {"classes_hold_little_more", classes_hold_little_more}, {"no_host_memory", no_host_memory}, {"full_of_other_blocks", full_of_other_blocks}, {"pinned_freed_in_a_capture", pinned_freed_in_a_capture}};
   CHECK(argc == 2 && tests.count(argv[1]));
   tests.at(argv[1])();
   puts("ok");

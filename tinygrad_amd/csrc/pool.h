@@ -131,10 +131,29 @@ static int pool_free_(void* ptr) {
   p.kept += cls; p.dirty += cls; it->second.out = false;
   return 0;
 }
+// Pinned host memory: a block that is given back waits in a list, without a call to the runtime (an hipHostFree would end a capture of its thread, and a model may be collected during one), for the
+// next request or tga_trim(); the list holds no more than what was in use at a time since the last request.
+static std::vector<void*> g_pinned_freed;
+static int pinned_release() { while (!g_pinned_freed.empty()) { void* q = g_pinned_freed.back(); g_pinned_freed.pop_back(); TGA_HIP(hipHostFree(q)); } return 0; }
+static int pinned_malloc_(void** ptr, size_t n) {
+  TGA_REQUIRE(!t_captures, "tga_host_malloc: not while this thread captures a stream");
+  TGA_HIP(hipFree(nullptr));                                                          // (as in pool_malloc_)
+  std::lock_guard<std::mutex> lock(g_pool_mutex);
+  if (const int rc = pinned_release()) return rc;
+  TGA_HIP(hipHostMalloc(ptr, n, hipHostMallocDefault));
+  return 0;
+}
+static int pinned_free_(void* ptr) {
+  std::lock_guard<std::mutex> lock(g_pool_mutex);
+  for (void* q : g_pinned_freed) TGA_REQUIRE(q != ptr, "tga_host_free: the block has been freed before");
+  g_pinned_freed.push_back(ptr);
+  return 0;
+}
 static int pool_give_back_() {
   TGA_REQUIRE(!t_captures, "tga_trim: not while this thread captures a stream");
   if (const int rc = pool_free_large()) return rc;
   std::lock_guard<std::mutex> lock(g_pool_mutex);
+  if (const int rc = pinned_release()) return rc;
   return pool_trim();
 }
 // (the lists may throw where the host has no memory left: an error at the C entries)
@@ -144,3 +163,5 @@ template <typename F> static int pool_guarded(const char* who, F f) {
 static int pool_malloc(void** ptr, size_t n) { return pool_guarded("tga_malloc", [&] { return pool_malloc_(ptr, n); }); }
 static int pool_free(void* ptr) { return pool_guarded("tga_free", [&] { return pool_free_(ptr); }); }
 static int pool_give_back() { return pool_guarded("tga_trim", [] { return pool_give_back_(); }); }
+static int pinned_malloc(void** ptr, size_t n) { return pool_guarded("tga_host_malloc", [&] { return pinned_malloc_(ptr, n); }); }
+static int pinned_free(void* ptr) { return pool_guarded("tga_host_free", [&] { return pinned_free_(ptr); }); }

@@ -44,8 +44,8 @@ int tga_malloc(void** ptr, size_t nbytes) {
 }
 int tga_free(void* ptr) { return ptr ? pool_free(ptr) : 0; }
 int tga_trim(void) { return pool_give_back(); }
-int tga_host_malloc(void** ptr, size_t nbytes) { TGA_REQUIRE(ptr && nbytes, "tga_host_malloc: null pointer or no bytes"); TGA_HIP(hipHostMalloc(ptr, nbytes, hipHostMallocDefault)); return 0; }
-int tga_host_free(void* ptr) { if (ptr) TGA_HIP(hipHostFree(ptr)); return 0; }
+int tga_host_malloc(void** ptr, size_t nbytes) { TGA_REQUIRE(ptr && nbytes, "tga_host_malloc: null pointer or no bytes"); return pinned_malloc(ptr, nbytes); }
+int tga_host_free(void* ptr) { return ptr ? pinned_free(ptr) : 0; }
 int tga_memcpy_h2d(void* dst, const void* src, size_t n) { TGA_HIP(hipMemcpy(dst, src, n, hipMemcpyHostToDevice)); return 0; }
 int tga_memcpy_d2h(void* dst, const void* src, size_t n) { TGA_HIP(hipMemcpy(dst, src, n, hipMemcpyDeviceToHost)); return 0; }
 int tga_memcpy_d2d(void* dst, const void* src, size_t n, void* stream) {
