@@ -28,10 +28,10 @@ def test_bits_of_the_steps_of_sixteen_rows(gpu, monkeypatch, name, n, rows):
   for p in (prompt, prompt[:n // 2] + [7] * 40):
     monkeypatch.setattr(llm, "ROWS16", rows); monkeypatch.setattr(llm, "ROWS16_MIN", 1)
     a.prefill(p)
-    assert a._chunker._rows_ws is not None and a._chunker.x is None        # (no step of sixteen was run)
+    assert a._chunker._rows16_ws is not None and a._chunker.x is None        # (no step of sixteen was run)
     monkeypatch.setattr(llm, "ROWS16_MIN", 1 << 30)
     b.prefill(p)
-    assert b._chunker is None or b._chunker._rows_ws is None
+    assert b._chunker is None or b._chunker._rows16_ws is None
     for i, (ba, bb) in enumerate(zip(a.blk, b.blk)):
       for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)):
         diff = int((ca.numpy().view(np.uint16) != cb.numpy().view(np.uint16)).sum())

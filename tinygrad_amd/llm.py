@@ -682,6 +682,7 @@ class BatchedTransformer:
       if ok and c.dim % 256 == 0 and c.hidden_dim % 256 == 0 and nq % 256 == 0:
         self.rows64 = 2 if B <= 32 else 4 if B <= 64 else 8             # column groups of sixteen rows in the layout
     self._rows_tables, self._rows_ws, self._rows_tok = self._many_rows_tables(), None, None
+    self._rows16_ws, self._rows16_tok = None, None                       # (prefill_rows16's)
     self.many_rows = not c.num_experts                                  # lockstep prompts as steps of many rows (see Transformer.many_rows)
     self.x = None
     if not self.chunked: self._alloc_step()
@@ -786,18 +787,18 @@ class BatchedTransformer:
     while plan(per) > ROWS16_BYTES and per > 64: per = per // 32 * 16
     if not ok.value: return 0
     try:
-      if self._rows_ws is None or self._rows_ws.nbytes < need.value: self._rows_ws = Buffer((need.value,), np.uint8)
-      if self._rows_tok is None or self._rows_tok.nbytes < 4 * n: self._rows_tok = Buffer((4 * n,), np.uint8)
+      if self._rows16_ws is None or self._rows16_ws.nbytes < need.value: self._rows16_ws = Buffer((need.value,), np.uint8)
+      if self._rows16_tok is None or self._rows16_tok.nbytes < 4 * n: self._rows16_tok = Buffer((4 * n,), np.uint8)
     except RuntimeError as e:
       if "HIP Error 2," not in str(e): raise
       return 0
     st = np.zeros(16, np.int32); st[0], st[3], st[5] = start, len(tokens), c.vocab_size
     self.state.copyin(st)
-    self._rows_tok.view(0, (n,), np.int32).copyin(np.array(tokens[start:start + n], np.int32))
+    self._rows16_tok.view(0, (n,), np.int32).copyin(np.array(tokens[start:start + n], np.int32))
     self._owner_stream.synchronize()
     for i in range(0, n, per):
       m = min(per, n - i)
-      rt.check(rt.lib().tga_prefill16_step(*self._rows_tables, self._rows_tok.ptr + 4 * i, m, max(0, m - max(0, n - tail - i)), start + i, self._rows_ws.ptr, self.state.ptr, self.stream.handle))
+      rt.check(rt.lib().tga_prefill16_step(*self._rows_tables, self._rows16_tok.ptr + 4 * i, m, max(0, m - max(0, n - tail - i)), start + i, self._rows16_ws.ptr, self.state.ptr, self.stream.handle))
     self.stream.synchronize()
     self.check_state()
     return n
