@@ -170,8 +170,9 @@ __global__ __launch_bounds__(256) void x16_rope_kernel(const X16Rope a) {
 
 // ------------------------------------------------------------------------------------------------ attention
 // The arithmetic of attn_decode_kernel (float32 products and sums, runs of HD8 lanes per row of keys, partials of 64 positions), with a workgroup's 64 keys and values in registers for the rows of a
-// chunk: workgroup = (kv head, 64 positions, X16_ROWS rows); four (row, query head) pairs at a time.
-#define X16_ROWS 32
+// chunk: workgroup = (kv head, 64 positions, X16_ROWS rows); four (row, query head) pairs at a time.  Three workgroups fit a CU (157 registers; with
+// 128 they spill: 78 us): of 512 rows and 16 heads 1152 workgroups of 32 rows, 1.5 rounds of the chip, or 2304 of 16, three: 60.5 -> 56.7 us.
+#define X16_ROWS 16
 struct X16Attn { const float* qr; const uint16_t* ck; const uint16_t* cv; float* part; uint16_t* out; int H, KV, max_ctx, P, pos0, nsplit; float scale; };
 
 template <int HD8>
