@@ -552,6 +552,40 @@ def test_small_batch_of_superblocks_that_start_off_a_piece(gpu, n, k, m, f32):
     qlinear_multi([lin], xb, [rb], epilogue=1, resid=[rb])
     assert ol.rel_err(rb.numpy(), res + ref) <= TOL, rep
 
+@pytest.mark.parametrize("n,k,m", [(16, 4096, 3), (4112, 4096, 8), (8208, 4096, 16), (16, 2048, 3), (4096, 2048, 4), (4112, 2048, 9), (12304, 2048, 16)])
+def test_order_of_sums_of_small_batch_q6_k(gpu, n, k, m):
+  """Wave w of a workgroup has the superblocks w % 4 and w % 4 + 4, of the second eight from wave 4 on, and the waves' sums are added in order (qgemm_dma.hip and qgemm_wp.hip alike).  One weight per
+  superblock is not zero, its product has 13 bits, and the exponents of a wave's two products lie within eleven of each other: they are added exactly, only the sum over the waves rounds, and the
+  bits of every result are known."""
+  rng = np.random.default_rng(n + k + m)
+  nsb = k // 256
+  blocks = np.zeros((n, nsb, 210), np.uint8)
+  blocks[..., 128:192], blocks[..., 208:] = 0xAA, np.array([1.0], np.float16).view(np.uint8)      # (every code 32, which is zero)
+  e, code, shift = rng.integers(0, 256, (n, nsb)), rng.integers(1, 32, (n, nsb)) * rng.choice([-1, 1], (n, nsb)), rng.integers(0, 5, (n, nsb))
+  h, j, l, q = e >> 7, (e >> 5) & 3, e & 31, code + 32
+  i0, i1 = np.indices((n, nsb))
+  blocks[i0, i1, 64 * h + 32 * (j & 1) + l] = (q & 15) << (4 * (j >> 1))
+  blocks[i0, i1, 128 + 32 * h + l] = 0xAA & ~(3 << (2 * j)) | (q >> 4) << (2 * j)
+  blocks[i0, i1, 192 + 8 * h + 2 * j + (l >> 4)] = 1 << shift
+  sb = np.arange(nsb)
+  wave, base = sb % 4 + 4 * (sb // 8), rng.choice([-14, -7, 0, 2], (m, nsb // 2))
+  x = ((2 * rng.integers(0, 128, (m, k)) + 1) * 2.0 ** (rng.integers(0, 7, (m, k)) + np.repeat(base[:, wave], 256, axis=1)) * rng.choice([-1, 1], (m, k))).astype(np.float16)
+  w = ol.weight_f32(blocks.reshape(-1), n, k, 14).reshape(n, nsb, 256)
+  assert ((w != 0).sum(-1) == 1).all() and (w[i0, i1, e] == code * 2.0 ** shift).all()
+  y = w[i0, i1, e].astype(np.float64) * x.astype(np.float64).reshape(m, nsb, 256)[:, i1, e]      # (m, n, superblocks)
+  def total(pairs):
+    v = np.zeros((m, n), np.float32)
+    for a, b in pairs: v += (y[..., a] + y[..., b]).astype(np.float32)
+    return v
+  pairs = [(8 * (wv >> 2) + (wv & 3), 8 * (wv >> 2) + (wv & 3) + 4) for wv in range(nsb // 2)]
+  assert all(((y[..., a] + y[..., b]).astype(np.float32) == y[..., a] + y[..., b]).all() for a, b in pairs)
+  ref = total(pairs)
+  assert (ref != total([(2 * wv, 2 * wv + 1) for wv in range(nsb // 2)])).mean() > 0.02          # (neighbours on one wave give other bits)
+  from tinygrad_amd.nn import QuantLinear
+  for act in (x, x.astype(np.float32)):
+    got = QuantLinear(gpu.Buffer.from_numpy(blocks), 14, n, k)(gpu.Buffer.from_numpy(act), out_dtype=np.float32).numpy()
+    np.testing.assert_array_equal(got, ref)
+
 @pytest.mark.parametrize("t,k,m,f32", [(8, 4096, 2, False), (8, 4096, 3, True), (8, 2048, 5, False), (8, 4096, 8, True), (8, 2048, 9, True), (8, 4096, 13, False), (8, 4096, 16, True), (8, 2048, 16, False),
                                        (1, 2048, 2, False), (1, 2048, 4, True), (1, 2048, 8, False), (1, 2048, 11, True), (1, 2048, 16, False),
                                        (2, 4096, 8, False), (2, 2048, 16, True), (12, 4096, 6, True), (12, 2048, 16, False), (13, 4096, 8, False), (13, 2048, 3, True),

@@ -31,7 +31,7 @@ __device__ __forceinline__ unsigned wp_lds_add(unsigned* p, unsigned d) { unsign
 __device__ __forceinline__ void wp_lds_poke(unsigned* p, unsigned d) { asm volatile("ds_write_b32 %0, %1" :: "v"(wp_lds_addr(p)), "v"(d) : "memory"); }
 template <int N> __device__ __forceinline__ void wp_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
 
-template <int T_, bool MS, bool SW, int UPW, int NB>
+template <int T_, bool MS, bool SW, int UPW, int NB, int TEAMS>
 __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, const int M, const int ring_w) {
   const QArgs a = args;
   using F = Fmt<T_>;
@@ -39,11 +39,14 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
   typedef typename F::Raw Raw;
   static_assert(!(MS && SW), "the SwiGLU pair is not combined with the q / k / v walk");
   // A ring position holds a wave's run of a row group or, Q6_K, one step of it: a superblock of 210 bytes per row, fetched as the fourteen aligned pieces that hold it.  Its ring of four steps is
-  // 120 KB a CU (three from nine rows on); whole runs (two positions of 420 bytes per row) would be 121 KB with half of it idle while the other half is decoded, and their second superblock starts off a piece.
-  // A lane's operands of the next step are read from LDS while this step is decoded, so a position is requested into again one step earlier.  128256 x 4096, 4 / 8 / 16 rows (us):
-  // barrier kernel 121 / 130 / 136, this ring 113 / 115 / 115, with the operands one step ahead 109 / 110 / 110, with single-instruction masks in the decode (qfmt.h) 104 / 105 / 107;
-  // 14336 x 4096, 4 / 16 rows: 21.4 / 23.3 -> 19.7 / 19.8.  What is left is the decode: 250 vector instructions per superblock, two waves a SIMD.
+  // 120 KB a CU (three from nine rows on).  A lane's operands of the next step are read from LDS while this step is decoded, so a position is requested into again one step earlier.
+  // The sums run as on the barrier kernel (qgemm_dma.hip), whose bits results have: wave w has the superblocks w % 4 and w % 4 + 4, of the second eight from wave 4 on.  Rows of eight superblocks are
+  // four waves' (TEAMS = 2: waves 4 - 7 take every second row group).  128256 x 4096, 4 / 8 / 16 rows, calls back to back (us): barrier kernel 121 / 128 / 133, this ring 101 / 102 / 105 (106 / 108 / 111
+  // on another box); 14336 x 4096 20.0 / 20.4 / 21.4 -> 18.2 / 18.7 / 18.6; 8192 x 2048 9.5 / 9.8 / 10.7 -> 8.0 / 8.4 / 9.4 (with a superblock for each of eight waves, in another order of sums:
+  // 7.9 / 8.1 / 8.5).  What is left is the decode: 250 vector instructions per superblock, two waves a SIMD.
   constexpr bool BYSTEP = T_ == GGML_Q6_K;
+  static_assert(BYSTEP ? UPW == 8 : TEAMS == 1, "Q6_K: two superblocks a wave");
+  constexpr int TW = WP_NW / TEAMS;                      // waves that share a row group
   constexpr int NST = UPW / 4;                           // steps (4 units x 16 rows) of a wave per row group
   constexpr int IPG = BYSTEP ? NST : 1;                  // ring positions per row group
   constexpr int SLICE = BYSTEP ? 14 * 16 : DF::slot_bytes(UPW);   // bytes of one row in a ring position
@@ -54,11 +57,11 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
   extern __shared__ u32x4 lds[];
   __shared__ __attribute__((aligned(16))) float part[2][WP_NW][256];   // [tile set][wave][16 c + 4 (g ^ (c >> 2)) + i]: lane (g, c) keeps rows 4 g .. 4 g + 3 of column c as one 16-byte piece (the swizzle spreads a quarter wave over all banks)
   __shared__ float nsum[WP_NW][16];
-  __shared__ unsigned cnt[2], done[2];
+  __shared__ unsigned cnt[2 * TEAMS], done[2 * TEAMS];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = lane & 15, g = lane >> 4;
+  const int r = lane & 15, g = lane >> 4, team = TEAMS == 1 ? 0 : wave / TW;
   char* ringw = (char*)lds + (size_t)wave * ring_w;
-  if (threadIdx.x < 2) { cnt[threadIdx.x] = 0u; done[threadIdx.x] = 0u; }
+  if (threadIdx.x < 2 * TEAMS) { cnt[threadIdx.x] = 0u; done[threadIdx.x] = 0u; }
   uint32_t kc[F::NKC];
   F::consts(kc);
   const long long ngroups = (SW ? a.n[0] : a.ntot) / GR;
@@ -69,7 +72,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
   auto rows_of = [&](int sg) -> long long { return !MS ? a.n[0] : sg == 0 ? a.n[0] : sg == 1 ? a.n[1] : a.n[2]; };
   auto w_of = [&](int sg) -> const uint8_t* { return !MS ? a.w[0] : sg == 0 ? a.w[0] : sg == 1 ? a.w[1] : a.w[2]; };
   const long long G = ((long long)blockIdx.x < ngroups) ? (ngroups - blockIdx.x + gridDim.x - 1) / gridDim.x : 0;   // row groups of this workgroup: every wave walks all of them
-  const long long items = G * IPG;
+  const long long GT = (G - team + TEAMS - 1) / TEAMS, items = GT * IPG;         // ... and of this team
   __syncthreads();                                       // (the counters are set)
   if (G == 0) return;
 
@@ -84,12 +87,13 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
     from_up[i] = SW && rr >= 8;
     doff[i] = (long long)(SW ? (rr & 7) : rr) * a.row_bytes + (BYSTEP ? 0 : (long long)wave * SLICE) + q * 16;
   }
-  auto step_byte = [&](int ss) { return 210 * (wave * NST + ss); };      // (BYSTEP) where the superblock of step ss starts in a row
+  auto unit0 = [&](int ss) { return BYSTEP ? 4 * ((TEAMS == 1 ? 8 * (wave >> 2) : 0) + (wave & 3) + 4 * ss) : wave * UPW + 4 * ss; };      // the first of the four units of step ss
+  auto step_byte = [&](int ss) { return unit0(ss) / 4 * 210; };          // (BYSTEP) where its superblock starts in a row
   // (weights pass the caches by (2): they are read once per launch and a model's do not come round again in time.  Eight rows, memory cold: Q8_0 14336 x 4096 16.2 -> 14.8 us, 4096 x 14336 18.2 -> 16.0,
   // 4096 x 4096 7.9 -> 7.1, Q4_K 14336 x 4096 15.5 -> 14.7, Q4_0 13.3 -> 12.4, fp16 4096 x 4096 10.8 -> 10.0; the same bytes still behind the L2s from call to call: 14.0 -> 14.4, 15.4 -> 15.3, 6.8 -> 6.6.
   // Q6_K's windows share lines between requests: 103 -> 106 on the lm-head, so they stay)
   auto issue = [&](long long k, int slot) {
-    const long long j = IPG == 1 ? k : k / IPG;
+    const long long j = team + TEAMS * (IPG == 1 ? k : k / IPG);
     const long long grp = (long long)blockIdx.x + j * gridDim.x;
     int sg; long long l0; seg_of(grp * GR, sg, l0);
     const long long goff = l0 * a.row_bytes + (BYSTEP ? step_byte((int)(k % IPG)) & ~15 : 0);
@@ -103,7 +107,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
     }
   };
 
-  // ---- this lane's activation operands (lane (g, c): the eight vectors of unit wave UPW + 4 ss + g of row c, zeros for c >= M): requested first, the weights second
+  // ---- this lane's activation operands (lane (g, c): the eight vectors of unit unit0(ss) + g of row c, zeros for c >= M): requested first, the weights second
   // (loads return in issue order), turned into the operand layout through the part of the wave's ring that the first groups do not use yet.  As in qgemm_dma.hip the
   // requests are inline assembly and their wait is counted by hand: a compiler-placed wait would also cover the weight pieces behind them.
   u32x4 bfrag[NST][F::XV];
@@ -122,7 +126,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
 #pragma unroll
         for (int v = 0; v < NV; v++) {
           const int row = F32 ? v : 2 * v + (lane >> 5);
-          const int uc = wave * UPW + 4 * ss;
+          const int uc = unit0(ss);
           const char* ptr = F32 ? (const char*)((const float*)a.x + (long long)(row < M ? row : 0) * a.K + 64 * uc + 4 * lane)
                                 : (const char*)((const uint16_t*)a.x + (long long)(row < M ? row : 0) * a.K + 64 * uc + 8 * (lane & 31));
           asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(xq[ss][v]) : "v"(ptr) : "memory");
@@ -130,7 +134,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
       u32x4 nwq[NORM ? NST : 1];                         // the norm weight of the step's columns (this lane: 4 values)
       if constexpr (NORM) {
 #pragma unroll
-        for (int ss = 0; ss < NST; ss++) { const float* ptr = a.norm_w + 64 * (wave * UPW + 4 * ss) + 4 * lane; asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(nwq[ss]) : "v"(ptr) : "memory"); }
+        for (int ss = 0; ss < NST; ss++) { const float* ptr = a.norm_w + 64 * unit0(ss) + 4 * lane; asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(nwq[ss]) : "v"(ptr) : "memory"); }
       }
       // every wave's activation requests are in the CU's queue before any weight request: a CU returns vector-memory data in request order, and without this the
       // activations of the wave that starts last wait behind the weight misses of the seven that started first (its operands were ready 2 us after theirs)
@@ -164,7 +168,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
         for (int v = 0; v < NV; v++) {
           float t = 0.f;
 #pragma unroll
-          for (int w = 0; w < WP_NW; w++) t += nsum[w][v];
+          for (int w = 0; w < TW; w++) t += nsum[team * TW + w][v];
           sc[v] = 1.0f / sqrtf(t / (float)a.K + a.norm_eps);
         }
       }
@@ -225,7 +229,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
         const long long o = (long long)c * nrows + l0 + 4 * g;
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < WP_NW; w++) v += *(const f32x4*)&part[p][w][16 * c + 4 * (g ^ (c >> 2))];
+        for (int w = 0; w < TW; w++) v += *(const f32x4*)&part[p][team * TW + w][16 * c + 4 * (g ^ (c >> 2))];
         if (rb) v += *(const f32x4*)(rb + o);
         store4(yb, o, v);
       }
@@ -241,7 +245,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (items >= NB) issue(NB - 1, NB - 1);
   }
-  for (long long j = 0; j < G; j++) {
+  for (long long i = 0; i < GT; i++) {                                  // (row group `team + TEAMS i` of this workgroup)
     v4f32 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
     auto multiply = [&](const Raw& buf, int ss) __attribute__((always_inline)) {
       uint32_t wv[F::NWV];
@@ -258,7 +262,7 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
       // the step behind this one is read from LDS while this one is decoded, so its ring position is requested into again at once
 #pragma unroll
       for (int ss = 0; ss < NST; ss++) {
-        const long long k = j * NST + ss, after = items - 1 - k;
+        const long long k = i * NST + ss, after = items - 1 - k;
         const int nslot = slot + 1 == NB ? 0 : slot + 1;
         // position k has been read; behind position k + 1 at most NB - 2 are on their way (behind the last one a position of earlier steps is read and dropped)
         if (NB == 4 && after >= 3) wp_wait_vm<2 * NI>(); else if (after >= 2) wp_wait_vm<NI>(); else wp_wait_vm<0>();
@@ -270,32 +274,32 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
         slot = nslot;
       }
     } else {
-      const long long after = G - 1 - j;
+      const long long after = GT - 1 - i;
       // this wave's pieces of group j have landed (later groups, and the stores of a sum, may be in flight)
       static_assert(BYSTEP || NB == 2 || (NB == 3 && NI <= 24), "ring of two or three groups");
       if (NB == 3 && after >= 1) wp_wait_vm<NI>(); else wp_wait_vm<0>();
-      if (j + NB - 1 < G) issue(j + NB - 1, slot == 0 ? NB - 1 : slot - 1);
+      if (i + NB - 1 < GT) issue(i + NB - 1, slot == 0 ? NB - 1 : slot - 1);
 #pragma unroll
       for (int ss = 0; ss < NST; ss++) multiply(DF::from_lds(ringw + slot * STAGE + r * PITCH, 4 * ss + g), ss);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // every read of this ring position is done: the next pass requests into it
       slot = slot + 1 == NB ? 0 : slot + 1;
     }
     // the tile set of this group: free once the group two before it has been summed
-    const int p = (int)(j & 1);
-    const unsigned turn = (unsigned)(j >> 1);
-    if (j >= 2) for (int n = 0; wp_lds_peek(&done[p]) != turn && n < WP_SPIN; n++) __builtin_amdgcn_s_sleep(1);
+    const int p = (int)(i & 1), tp = 2 * team + p;
+    const unsigned turn = (unsigned)(i >> 1);
+    if (i >= 2) for (int n = 0; wp_lds_peek(&done[tp]) != turn && n < WP_SPIN; n++) __builtin_amdgcn_s_sleep(1);
     *(f32x4*)&part[p][wave][16 * r + 4 * (g ^ (r >> 2))] = f32x4{acc0[0] + acc1[0], acc0[1] + acc1[1], acc0[2] + acc1[2], acc0[3] + acc1[3]};
     // (no wait between the tile and the count: LDS executes a wave's operations in order)
-    if (wave != (int)(j & 7)) {
-      if (lane == 0) asm volatile("ds_add_u32 %0, %1" :: "v"(wp_lds_addr(&cnt[p])), "v"(1u) : "memory");   // counted in; nothing to wait for
+    if (wave - team * TW != (int)(i & (TW - 1))) {
+      if (lane == 0) asm volatile("ds_add_u32 %0, %1" :: "v"(wp_lds_addr(&cnt[tp])), "v"(1u) : "memory");   // counted in; nothing to wait for
     } else {
-      // this wave sums group j: the role rotates, so that the wave that arrives last is not the one that falls further behind; the others are ahead of it
+      // this wave sums the group: the role rotates, so that the wave that arrives last is not the one that falls further behind; the others are ahead of it
       // and wait for nobody, so the (bounded) wait below ends
-      if (lane == 0) asm volatile("ds_add_u32 %0, %1" :: "v"(wp_lds_addr(&cnt[p])), "v"(1u) : "memory");
-      for (int n = 0; wp_lds_peek(&cnt[p]) != WP_NW && n < WP_SPIN; n++) __builtin_amdgcn_s_sleep(1);
-      reduce_store(((long long)blockIdx.x + j * gridDim.x) * GR, p);
+      if (lane == 0) asm volatile("ds_add_u32 %0, %1" :: "v"(wp_lds_addr(&cnt[tp])), "v"(1u) : "memory");
+      for (int n = 0; wp_lds_peek(&cnt[tp]) != TW && n < WP_SPIN; n++) __builtin_amdgcn_s_sleep(1);
+      reduce_store(((long long)blockIdx.x + (team + TEAMS * i) * gridDim.x) * GR, p);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // the tiles have been read
-      if (lane == 0) { wp_lds_poke(&cnt[p], 0u); wp_lds_poke(&done[p], turn + 1u); }
+      if (lane == 0) { wp_lds_poke(&cnt[tp], 0u); wp_lds_poke(&done[tp], turn + 1u); }
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -309,7 +313,7 @@ static int wp_cu_count() {
 
 #define WP_STATIC_LDS (2 * WP_NW * 256 * 4 + WP_NW * 16 * 4 + 64)
 
-template <int T, bool MS, bool SW, int UPW, int NB>
+template <int T, bool MS, bool SW, int UPW, int NB, int TEAMS = 1>
 static int launch_wp_k(const QArgs& a, int M, hipStream_t s) {
   using DF = DmaFmt<T>;
   constexpr int SLICE = T == GGML_Q6_K ? 14 * 16 : DF::slot_bytes(UPW), PR = SLICE / 16, PP = PR + (PR % 2 == 0 ? 1 : 0), STAGE = 16 * PP * 16;
@@ -317,7 +321,7 @@ static int launch_wp_k(const QArgs& a, int M, hipStream_t s) {
   int ring_w = NB * STAGE; if ((NB - 1) * STAGE + xb > ring_w) ring_w = (NB - 1) * STAGE + xb;
   const size_t lds = (size_t)WP_NW * ring_w;
   if (lds + WP_STATIC_LDS > (size_t)QD_LDS_CU) return -1;
-  auto kern = qgemm_wp_kernel<T, MS, SW, UPW, NB>;
+  auto kern = qgemm_wp_kernel<T, MS, SW, UPW, NB, TEAMS>;
   static int static_lds = 0;
   static const hipError_t configured = [&]() {
     hipFuncAttributes fa;
@@ -336,13 +340,13 @@ static int launch_wp_k(const QArgs& a, int M, hipStream_t s) {
   return 0;
 }
 
-template <int T, int UPW>
+template <int T, int UPW, int TEAMS = 1>
 static int launch_wp_u(const QArgs& a, int M, hipStream_t s) {
   // three groups in flight per wave where the ring holds them, else two
   int rc;
   if constexpr (T == GGML_Q6_K) {                                      // (one matrix, plain or residual epilogue, as on the barrier kernel; from nine rows on the activations' way through LDS leaves room for three steps)
     if (a.epilogue == 2 || a.nseg > 1) return -1;
-    rc = launch_wp_k<T, false, false, UPW, 4>(a, M, s); return rc >= 0 ? rc : launch_wp_k<T, false, false, UPW, 3>(a, M, s);
+    rc = launch_wp_k<T, false, false, UPW, 4, TEAMS>(a, M, s); return rc >= 0 ? rc : launch_wp_k<T, false, false, UPW, 3, TEAMS>(a, M, s);
   } else {
   if constexpr (T != GGML_F16) { if (a.epilogue == 2) { rc = launch_wp_k<T, false, true, UPW, 3>(a, M, s); return rc >= 0 ? rc : launch_wp_k<T, false, true, UPW, 2>(a, M, s); } }
   if (a.epilogue == 2) return -1;
@@ -358,7 +362,7 @@ static int launch_wp(QArgs a, int M, hipStream_t s) {
   a.row_bytes = (long long)(a.K / F::BW) * F::BB;
   if (a.K % F::UW != 0 || a.row_bytes % 16 != 0) return -1;
   if constexpr (T != GGML_F16) { if (a.nu == 64) return launch_wp_u<T, 8>(a, M, s); }       // (fp16 rows of 4096 values: a ring of two groups does not fit, and its operands would spill)
-  if (a.nu == 32) return launch_wp_u<T, 4>(a, M, s);
+  if (a.nu == 32) { if constexpr (T == GGML_Q6_K) return launch_wp_u<T, 8, 2>(a, M, s); else return launch_wp_u<T, 4>(a, M, s); }
   return -1;
 }
 
