@@ -552,6 +552,14 @@ def test_small_batch_of_superblocks_that_start_off_a_piece(gpu, n, k, m, f32):
     qlinear_multi([lin], xb, [rb], epilogue=1, resid=[rb])
     assert ol.rel_err(rb.numpy(), res + ref) <= TOL, rep
 
+@pytest.mark.parametrize("n,k,m", [(4099, 1024, 1), (8192, 2048, 1), (33000, 4096, 1), (4099, 14336, 1), (16400, 4096, 2)])
+def test_equal_rows_of_q6_k_have_equal_results(gpu, n, k, m):
+  """The bits of a row do not hang on where it lies in the matrix (the rows of a wave, the steps of its loop): rows of the same bytes give the same float32."""
+  rng = np.random.default_rng(n + k)
+  w = np.tile(synth.random_blocks(rng, 14, 3, k).reshape(3, -1), (n // 3 + 1, 1))[:n]
+  y = _run(gpu, 14, np.ascontiguousarray(w).reshape(-1), synth.activations(rng, m, k, np.float16), n, k)
+  for i in range(3): assert (y[:, i::3].view(np.uint32) == y[:, i:i + 1].view(np.uint32)).all()
+
 @pytest.mark.parametrize("n,k,m", [(16, 4096, 3), (4112, 4096, 8), (8208, 4096, 16), (16, 2048, 3), (4096, 2048, 4), (4112, 2048, 9), (12304, 2048, 16)])
 def test_order_of_sums_of_small_batch_q6_k(gpu, n, k, m):
   """Wave w of a workgroup has the superblocks w % 4 and w % 4 + 4, of the second eight from wave 4 on, and the waves' sums are added in order (qgemm_dma.hip and qgemm_wp.hip alike).  One weight per

@@ -486,7 +486,8 @@ template <> struct Fmt<GGML_Q6_K> {
     const int g8 = (r.d & 1) * 8;   // scales 8h + 2j + g live in bytes g, g+2 of sc0 (j = 0, 1) and sc1 (j = 2, 3)
     const float s0 = (float)(int)(int8_t)(r.sc0 >> g8), s1 = (float)(int)(int8_t)(r.sc0 >> (16 + g8));
     const float s2 = (float)(int)(int8_t)(r.sc1 >> g8), s3 = (float)(int)(int8_t)(r.sc1 >> (16 + g8));
-    return h2f_bits(r.d >> 16) * (s0 * a[0] + s1 * a[1] + s2 * a[2] + s3 * a[3]);
+    // (in a stated order: left to itself the compiler rounded s0 a[0] before the addition at some positions of an unrolled loop and s1 a[1] at others, and a row's last bit hung on where it lay)
+    return h2f_bits(r.d >> 16) * __builtin_fmaf(s3, a[3], __builtin_fmaf(s2, a[2], __builtin_fmaf(s0, a[0], s1 * a[1])));
   }
   static __device__ __forceinline__ void to_f16(const Raw& r, uint32_t* wv) {
     const int g8 = (r.d & 1) * 8;
