@@ -39,3 +39,27 @@ def test_bits_of_the_steps_of_sixteen_rows(gpu, monkeypatch, name, n, rows):
     for m in (a, b): m.decode_step(); m.check_state()
     diff = int((a.logits().view(np.uint32) != b.logits().view(np.uint32)).sum())
     assert diff == 0
+
+@pytest.mark.parametrize("name", ["1536x768", "512x256"])
+@pytest.mark.parametrize("n,at", [(40, 21), (100, 70), (333, 200)])
+def test_values_that_are_not_finite_stay_with_later_positions(gpu, name, n, at):
+  """A token whose value in one column leaves the fp16 range: the keys and values of the positions in front of it are those of a prompt that has another token there, in every block."""
+  from tinygrad_amd.llm import Transformer, TransformerConfig, synth_state_moe
+  cfg = dict(CONFIGS[name], num_blocks=3)
+  c = TransformerConfig(max_context=384, **cfg)
+  sd = synth_state_moe(c, seed=n)
+  def edit(key, f):
+    b, _, shape = sd[key]
+    w = b.numpy().view(np.float16).reshape(shape); f(w); b.copyin(w.view(np.uint8).reshape(b.shape).view(b.dtype))
+  def column(w): w[:, 0] = 0; w[5, 0] = 100
+  def row(w): w[0, 0] = 60000
+  edit("token_embd.weight", column); edit("blk.0.attn_v.weight", row)            # (only token 5 has anything in column 0, and 60000 times that is infinite)
+  prompt = np.random.default_rng(n).integers(6, cfg["vocab_size"], size=n).tolist()
+  other = prompt[:at] + [5] + prompt[at + 1:]
+  a, b = Transformer(c, sd, max_new=8), Transformer(c, sd, max_new=8)
+  a.prefill(other); b.prefill(prompt)
+  assert a._chunker._rows16_ws is not None and np.isinf(a.blk[0].cache_v.numpy()[0, at, 0])
+  for ba, bb in zip(a.blk, b.blk):
+    for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)):
+      ca, cb = ca.numpy()[:, :at], cb.numpy()[:, :at]
+      assert np.isfinite(cb).all(); np.testing.assert_array_equal(ca.view(np.uint16), cb.view(np.uint16))

@@ -170,8 +170,9 @@ __global__ __launch_bounds__(256) void x16_rope_kernel(const X16Rope a) {
 
 // ------------------------------------------------------------------------------------------------ attention
 // The arithmetic of attn_decode_kernel (float32 products and sums, runs of HD8 lanes per row of keys, partials of 64 positions), with a workgroup's 64 keys and values in registers for the rows of a
-// chunk: workgroup = (kv head, 64 positions, X16_ROWS rows); four (row, query head) pairs at a time.  Three workgroups fit a CU (157 registers; with
-// 128 they spill: 78 us): of 512 rows and 16 heads 1152 workgroups of 32 rows, 1.5 rounds of the chip, or 2304 of 16, three: 60.5 -> 56.7 us.
+// chunk: workgroup = (kv head, 64 positions, X16_ROWS rows); four (row, query head) pairs at a time.  Three workgroups fit a CU (153 registers; with
+// 128 they spill: 78 us): of 512 rows and 16 heads 1152 workgroups of 32 rows, 1.5 rounds of the chip, or 2304 of 16, three: 60.5 -> 56.7 us.  Values behind a row's position are dropped by selects:
+// 57.4 -> 62.5 us; a path of its own for tiles that hold a value that is not finite takes registers or hoisted conversions from the other one (61.5 .. 70.9 us).
 #define X16_ROWS 16
 struct X16Attn { const float* qr; const uint16_t* ck; const uint16_t* cv; float* part; uint16_t* out; int H, KV, max_ctx, P, pos0, nsplit; float scale; };
 
@@ -239,7 +240,8 @@ __global__ __launch_bounds__(256) void x16_attn_kernel(const X16Attn a) {
         for (int i = 0; i < NVI; i++) {
           const float pj = (p0 + i * RPI + vr <= pos) ? __expf(sc[i] - m) : 0.f;
           l += pj;
-          const u32x4 vv = vt[i];
+          u32x4 vv = vt[i];
+          if (p0 + i * RPI + vr > pos) vv = u32x4{0u, 0u, 0u, 0u};         // (a later position's: 0 times a value that is not finite would reach this row)
           const half2_t v0 = as_h2(vv.x), v1 = as_h2(vv.y), v2 = as_h2(vv.z), v3 = as_h2(vv.w);
           o0.x += pj * (float)v0.x; o0.y += pj * (float)v0.y; o0.z += pj * (float)v1.x; o0.w += pj * (float)v1.y;
           o1.x += pj * (float)v2.x; o1.y += pj * (float)v2.y; o1.z += pj * (float)v3.x; o1.w += pj * (float)v3.y;
