@@ -40,6 +40,32 @@ def test_bits_of_the_steps_of_sixteen_rows(gpu, monkeypatch, name, n, rows):
     diff = int((a.logits().view(np.uint32) != b.logits().view(np.uint32)).sum())
     assert diff == 0
 
+def _same_bits(a, b, n):
+  for i, (ba, bb) in enumerate(zip(a.blk, b.blk)):
+    for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): assert (ca.numpy().view(np.uint16)[:, :n - 1] == cb.numpy().view(np.uint16)[:, :n - 1]).all(), f"block {i}"
+  for m in (a, b): m.decode_step(); m.check_state()
+  assert (a.logits().view(np.uint32) == b.logits().view(np.uint32)).all()
+
+@pytest.mark.parametrize("name", list(CONFIGS))
+def test_bits_with_norm_weights_of_any_value(gpu, monkeypatch, name):
+  """Norm weights that are no powers of two (the synthetic models' are 1): a normalised value is rounded where the steps of sixteen, eight and four rows round it."""
+  from tinygrad_amd import llm
+  from tinygrad_amd.llm import Transformer, TransformerConfig, synth_state_moe
+  cfg, rng, n = CONFIGS[name], np.random.default_rng(37), 350
+  c = TransformerConfig(max_context=384, **cfg)
+  sd = synth_state_moe(c, seed=37)
+  for key, (b, _, shape) in sd.items():
+    if key.endswith("norm.weight"): b.view(0, shape, np.float32).copyin((rng.uniform(0.3, 3, shape) * rng.choice([-1, 1], shape)).astype(np.float32))
+  for m in (n, n - 26, 140):                                                        # (349, 323 and 139 positions: behind the steps of sixteen 8 + 4 + 1, 3 and 8 + 3)
+    prompt = rng.integers(0, cfg["vocab_size"], size=m).tolist()
+    a, b = Transformer(c, sd, max_new=8), Transformer(c, sd, max_new=8)
+    monkeypatch.setattr(llm, "ROWS16_MIN", 16)
+    a.prefill(prompt)
+    monkeypatch.setattr(llm, "ROWS16_MIN", 1 << 30)
+    b.prefill(prompt)
+    assert a._chunker._rows16_ws is not None and b._chunker._rows16_ws is None
+    _same_bits(a, b, m)
+
 @pytest.mark.parametrize("name", ["1536x768", "512x256"])
 @pytest.mark.parametrize("n,at", [(40, 21), (100, 70), (333, 200)])
 def test_values_that_are_not_finite_stay_with_later_positions(gpu, name, n, at):

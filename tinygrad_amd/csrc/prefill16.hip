@@ -359,7 +359,7 @@ __global__ __launch_bounds__(1024) void x16_router_kernel(const X16Router a) {
       float v[8] = {xa[t][0].x, xa[t][0].y, xa[t][0].z, xa[t][0].w, xa[t][1].x, xa[t][1].y, xa[t][1].z, xa[t][1].w};
       const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
-      for (int i = 0; i < 8; i++) v[i] = (v[i] * nscale) * w[i];
+      for (int i = 0; i < 8; i++) { v[i] = (v[i] * nscale) * w[i]; asm volatile("" : "+v"(v[i])); }      // (a float32 value before it is rounded to fp16, as there: one instruction would round once)
       *(u32x4*)(&xn[t][8 * p]) = u32x4{f2h_bits(v[0]) | (f2h_bits(v[1]) << 16), f2h_bits(v[2]) | (f2h_bits(v[3]) << 16), f2h_bits(v[4]) | (f2h_bits(v[5]) << 16), f2h_bits(v[6]) | (f2h_bits(v[7]) << 16)};
     }
   }
