@@ -46,6 +46,55 @@ def _same_bits(a, b, n):
   for m in (a, b): m.decode_step(); m.check_state()
   assert (a.logits().view(np.uint32) == b.logits().view(np.uint32)).all()
 
+# the rest of the range: attention rows of other widths than the residual's (attn_output over 9, 10, 12 and 16 steps of 256, dealt to four and to eight waves), and contexts of more than 24 splits
+WIDE = {f"{h}x{hd}": dict(num_blocks=2, dim=512, hidden_dim=256, n_heads=h, n_kv_heads=kv, head_dim=hd, qk_norm=h * hd, num_experts=16, num_experts_per_tok=2, **BASE)
+        for h, kv, hd in ((18, 6, 128), (40, 8, 64), (24, 24, 128), (32, 8, 128))}
+LONG = {f"long-{h}x{hd}": dict(num_blocks=2, dim=512, hidden_dim=256, n_heads=h, n_kv_heads=h // 2, head_dim=hd, qk_norm=h * hd, num_experts=16, num_experts_per_tok=2, **BASE) for h, hd in ((8, 64), (4, 128))}
+
+@pytest.mark.parametrize("name,n", [(name, 95) for name in WIDE] + [(name, 1667) for name in LONG])
+def test_bits_over_the_rest_of_the_range(gpu, monkeypatch, name, n):
+  """94 positions of wide attention rows; 1666 positions (27 splits of 64, two steps: 1024 rows and 642 with the tail of eight)."""
+  from tinygrad_amd import llm
+  a, b = _models({**WIDE, **LONG}[name], 5 + n, 128 if n < 128 else 2048)
+  prompt = np.random.default_rng(n).integers(0, BASE["vocab_size"], size=n).tolist()
+  a.prefill(prompt)
+  assert a._chunker._rows16_ws is not None and a._chunker.x is None
+  monkeypatch.setattr(llm, "ROWS16_MIN", 1 << 30)
+  b.prefill(prompt)
+  assert b._chunker._rows16_ws is None
+  _same_bits(a, b, n)
+
+def test_bits_of_steps_that_memory_cuts(gpu, monkeypatch):
+  """Buffers bounded to less than a prompt's rows need (steps of fewer rows, a multiple of sixteen each), and no memory for them at all (the steps of sixteen)."""
+  from tinygrad_amd import llm
+  n = 300
+  prompt = np.random.default_rng(n).integers(0, BASE["vocab_size"], size=n).tolist()
+  a, b = _models(CONFIGS["512x256"], n, 384)
+  c, d = _models(CONFIGS["512x256"], n, 384)
+  real, sizes = llm.Buffer, []
+  class Counted(real):
+    def __init__(self, shape, *args, **kw):
+      sizes.append(int(np.prod(shape))); super().__init__(shape, *args, **kw)
+  monkeypatch.setattr(llm, "ROWS16_BYTES", 1 << 20); monkeypatch.setattr(llm, "Buffer", Counted)
+  a.prefill(prompt)
+  monkeypatch.setattr(llm, "Buffer", real)
+  ws = a._chunker._rows16_ws
+  assert ws is not None and a._chunker.x is None and ws.nbytes in sizes
+  monkeypatch.setattr(llm, "ROWS16_BYTES", 1 << 29)
+  c.prefill(prompt)
+  assert ws.nbytes < c._chunker._rows16_ws.nbytes // 2
+  def none(shape, *args, **kw):
+    if int(np.prod(shape)) == c._chunker._rows16_ws.nbytes: raise RuntimeError("HIP Error 2, out of memory")
+    return real(shape, *args, **kw)
+  monkeypatch.setattr(llm, "Buffer", none)
+  d.prefill(prompt)
+  monkeypatch.setattr(llm, "Buffer", real)
+  assert d._chunker._rows16_ws is None and d._chunker.x is not None
+  monkeypatch.setattr(llm, "ROWS16_MIN", 1 << 30)
+  for m in (a, c, d):
+    b.prefill(prompt)
+    _same_bits(m, b, n)
+
 @pytest.mark.parametrize("name", list(CONFIGS))
 def test_bits_with_norm_weights_of_any_value(gpu, monkeypatch, name):
   """Norm weights that are no powers of two (the synthetic models' are 1): a normalised value is rounded where the steps of sixteen, eight and four rows round it."""
@@ -65,6 +114,31 @@ def test_bits_with_norm_weights_of_any_value(gpu, monkeypatch, name):
     b.prefill(prompt)
     assert a._chunker._rows16_ws is not None and b._chunker._rows16_ws is None
     _same_bits(a, b, m)
+
+@pytest.mark.parametrize("name", list(CONFIGS))
+def test_expert_products_of_values_of_every_size(gpu, monkeypatch, name):
+  """The experts' products are matrix-core products of two values with zeros beside them, in place of v_dot2_f32_f16: the bits over activations from subnormal fp16 numbers to 2^13 in one sum (norm
+  weights of 2^-24 .. 2^12, both signs) and over hidden values as far apart (block scales of 2^-26 .. 2^-14)."""
+  from tinygrad_amd import llm
+  from tinygrad_amd.llm import Transformer, TransformerConfig, synth_state_moe
+  cfg, rng = CONFIGS[name], np.random.default_rng(31)
+  c = TransformerConfig(max_context=192, **cfg)
+  sd = synth_state_moe(c, seed=31)
+  for i in range(c.num_blocks):
+    w = (2.0 ** rng.uniform(-24, 12, c.dim) * rng.choice([-1, 1], c.dim)).astype(np.float32)
+    sd[f"blk.{i}.ffn_norm.weight"][0].view(0, (c.dim,), np.float32).copyin(w)
+    for nm in ("gate", "up"):
+      b = sd[f"blk.{i}.ffn_{nm}_exps.weight"][0]
+      raw = b.numpy().view(np.uint8).reshape(-1, 17)
+      raw[:, 0] = 127 - rng.integers(14, 27, len(raw) // (c.dim // 32)).repeat(c.dim // 32)      # (a scale for each row: rows of the hidden layer lie apart)
+      b.copyin(raw.reshape(b.shape))
+  prompt = rng.integers(0, cfg["vocab_size"], size=125).tolist()
+  a, b = Transformer(c, sd, max_new=8), Transformer(c, sd, max_new=8)
+  a.prefill(prompt)
+  monkeypatch.setattr(llm, "ROWS16_MIN", 1 << 30)
+  b.prefill(prompt)
+  assert a._chunker._rows16_ws is not None and b._chunker._rows16_ws is None and np.isfinite(b.blk[-1].cache_v.numpy()).all()
+  _same_bits(a, b, 125)
 
 @pytest.mark.parametrize("name", ["1536x768", "512x256"])
 @pytest.mark.parametrize("n,at", [(40, 21), (100, 70), (333, 200)])
