@@ -307,9 +307,9 @@ def _single_steps(moe, inp, logits, k, gate_up, b_gate_up, down, b_down):
   return moe.combine(z, r, inp.shape[0], k).numpy()
 
 @pytest.mark.parametrize("T,D,I,E,k,skew", [(1, 256, 256, 3, 1, 0), (5, 768, 256, 70, 8, 1), (33, 2048, 768, 5, 3, 1), (40, 1280, 512, 20, 4, 0), (130, 256, 768, 4, 4, 0), (600, 1024, 256, 9, 2, 2), (900, 512, 512, 12, 2, 0),
-                                            (2600, 256, 768, 40, 2, 1), (6000, 256, 256, 80, 2, 0), (3100, 768, 512, 65, 4, 0), (700, 1536, 512, 512, 8, 1)])
+                                            (2600, 256, 768, 40, 2, 1), (4128, 4096, 256, 4, 4, 0), (6000, 256, 256, 80, 2, 0), (3100, 768, 512, 65, 4, 0), (700, 1536, 512, 512, 8, 1)])
 def test_moe_feed_forward_at_every_tile_height(gpu, T, D, I, E, k, skew):
-  """Tiles of 16, 32, 64, 128 and 256 rows (by the rows per expert; 256 where the counts, on the device, make them half the rounds), reductions of 2, 4, 6, 8, 10, 12 and 16 steps of 128 (scales
+  """Tiles of 16, 32, 64, 128 and 256 rows (by the rows per expert; 256 where the counts, on the device, make them five ninths of the rounds or fewer: 9 / 5 rounds of the down product of 4 x 4128 rows), reductions of 2, 4, 6, 8, 10, 12 and 16 steps of 128 (scales
   are fetched four steps at a time, a last pair on its own), experts of no rows, of one, of several tiles and with a remainder, more experts than lanes: bits of the single steps, twice."""
   from tinygrad_amd import moe
   rng = np.random.default_rng(T + D + I + E)

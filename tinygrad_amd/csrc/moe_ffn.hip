@@ -128,30 +128,38 @@ __global__ __launch_bounds__(1024) void moe_prep_kernel(const FfnArgs a) {
 __global__ __launch_bounds__(512) void moe_zero_counts_kernel(int* counts, int E) { if ((int)threadIdx.x < E) counts[threadIdx.x] = 0; }
 
 // Exclusive prefix sums over the experts' counts and over their tiles of bm rows, by the first wave of a workgroup: off[e] = first row, tile[e] = first tile (off[E], tile[E]: the totals).
-// COUNTS: counts are given; otherwise off[] is there and gives them.
-template <bool COUNTS>
-__device__ __forceinline__ void ffn_offsets(const int* __restrict__ counts, int E, int bm, int tiles_n, int* off, int* tile) {
+// tall: tiles of 256 rows instead, and *tall = 1, where their rounds of a launch of `grid` workgroups are at most five ninths of those of bm rows (see the dispatch); otherwise *tall = 0.
+__device__ __forceinline__ void ffn_offsets(const int* __restrict__ counts, int E, int bm, int tiles_n, int* off, int* tile, int* tall = nullptr, int grid = 1) {
   const int lane = threadIdx.x;
   if (lane < 64) {
     constexpr int PER = FFN_MAX_E / 64;
-    int c[PER], so = 0, st = 0;
+    int c[PER], so = 0, st = 0, st2 = 0;
 #pragma unroll
     for (int i = 0; i < PER; i++) {                                       // (one wait for all of them)
-      const int e = lane * PER + i, k = min(e, E - 1), v = COUNTS ? counts[k] : off[k + 1] - off[k];
+      const int e = lane * PER + i, v = counts[min(e, E - 1)];
       c[i] = e < E ? v : 0;
     }
 #pragma unroll
-    for (int i = 0; i < PER; i++) { so += c[i]; st += (c[i] + bm - 1) / bm * tiles_n; }
-    int io = so, it = st;
+    for (int i = 0; i < PER; i++) { so += c[i]; st += (c[i] + bm - 1) / bm * tiles_n; if (tall) st2 += (c[i] + 255) / 256 * tiles_n; }
+    int io = so, it = st, it2 = st2;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) { const int uo = __shfl_up(io, o), ut = __shfl_up(it, o); if (lane >= o) { io += uo; it += ut; } }
+    for (int o = 1; o < 64; o <<= 1) {
+      const int uo = __shfl_up(io, o), ut = __shfl_up(it, o), u2 = tall ? __shfl_up(it2, o) : 0;
+      if (lane >= o) { io += uo; it += ut; it2 += u2; }
+    }
+    if (tall) {
+      const int n = __builtin_amdgcn_readlane(it, 63), n2 = __builtin_amdgcn_readlane(it2, 63);
+      const bool take = 9 * ((n2 + grid - 1) / grid) <= 5 * ((n + grid - 1) / grid);
+      if (take) { bm = 256; it = it2; st = st2; }
+      if (lane == 0) *tall = take;
+    }
     io -= so; it -= st;
 #pragma unroll
     for (int i = 0; i < PER; i++) {
       const int e = lane * PER + i;
-      if (e <= E) { if (COUNTS) off[e] = io; if (tile) tile[e] = it; }
+      if (e <= E) { off[e] = io; if (tile) tile[e] = it; }
       io += c[i]; it += (c[i] + bm - 1) / bm * tiles_n;
-      if (e == E - 1) { if (COUNTS) off[E] = io; if (tile) tile[E] = it; }
+      if (e == E - 1) { off[E] = io; if (tile) tile[E] = it; }
     }
   }
 }
@@ -257,12 +265,7 @@ __device__ __forceinline__ void ffn_tall(const FfnArgs& a, uint8_t* smem, int* s
   int t = first + ((int)blockIdx.x >> 3);
   if (t >= last) return;
 
-  const int cpy_c = tid & 7, cpy_r = tid >> 3;
-  int lds_a[PA], lds_b[PB];
-#pragma unroll
-  for (int j = 0; j < PA; j++) lds_a[j] = gg_slot_off(cpy_r + RPT * j, cpy_c);
-#pragma unroll
-  for (int j = 0; j < PB; j++) lds_b[j] = BM * 128 + gg_slot_off(cpy_r + RPT * j, cpy_c);
+  const int cpy_c = tid & 7, cpy_r = tid >> 3, slot0 = gg_slot_off(cpy_r, cpy_c);     // (RPT rows further on: RPT * 128 bytes)
   const int f0 = ((16 * kg + (r16 ^ kg)) << 4), f1 = 1024 + ((16 * kg + (r16 ^ (kg + 4))) << 4);
 
   auto setup = [&](int tile, FfnCur& c, int which) __attribute__((always_inline)) {
@@ -282,8 +285,8 @@ __device__ __forceinline__ void ffn_tall(const FfnArgs& a, uint8_t* smem, int* s
       vs[j] = *(const uint32_t*)(p + 4 * s);
     }
   };
-  auto store_a = [&](uint8_t* st, int j) __attribute__((always_inline)) { *(u32x4*)(st + lds_a[j]) = va[j]; };
-  auto store_b = [&](uint8_t* st, int j) __attribute__((always_inline)) { *(u32x4*)(st + lds_b[j]) = vb[j]; };
+  auto store_a = [&](uint8_t* st, int j) __attribute__((always_inline)) { *(u32x4*)(st + slot0 + RPT * 128 * j) = va[j]; };
+  auto store_b = [&](uint8_t* st, int j) __attribute__((always_inline)) { *(u32x4*)(st + BM * 128 + slot0 + RPT * 128 * j) = vb[j]; };
   auto store_s = [&](uint8_t* st) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NS; j++) { const int i = tid + NT * j; if (i < BM + BN) ((uint32_t*)(st + (BM + BN) * 128))[i] = vs[j]; }
@@ -407,26 +410,13 @@ __global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a)
   const int N = UP ? 2 * a.I : a.D, K = UP ? a.D : a.I, KB = K / 32, nsteps = K / 128, tiles_n = N / BN;
   const uint8_t* __restrict__ A = UP ? a.xq : a.yq; const uint8_t* __restrict__ Ae = UP ? a.xe8 : a.ye8;
   const uint8_t* __restrict__ B = a.w[UP ? 0 : 1]; const uint8_t* __restrict__ Be = a.we8[UP ? 0 : 1];
-  ffn_offsets<true>(a.counts, a.E, BM, tiles_n, s_off, s_tile);
-  __syncthreads();
+  if constexpr (BM == 128) {                                             // tall tiles where they nearly halve the rounds of the launch: see the dispatch
+    __shared__ int s_tall;
+    ffn_offsets(a.counts, a.E, BM, tiles_n, s_off, s_tile, &s_tall, (int)gridDim.x);
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_tall)) { ffn_tall<UP>(a, smem, (int*)(smem + 2 * FFN_TALL_STAGE), s_off, s_tile); return; }
+  } else { ffn_offsets(a.counts, a.E, BM, tiles_n, s_off, s_tile); __syncthreads(); }
   const int ntiles = __builtin_amdgcn_readfirstlane(s_tile[a.E]);
-  if constexpr (BM == 128) {
-    const int grid = (int)gridDim.x, rounds = (ntiles + grid - 1) / grid;
-    if (rounds > 1) {                                                     // tall tiles where they halve the rounds of the launch: see the dispatch
-      int tall = 0;
-      for (int e = 0; e < a.E; e += 64) tall += e + lane < a.E ? (s_off[e + lane + 1] - s_off[e + lane] + 255) >> 8 : 0;
-#pragma unroll
-      for (int o = 32; o; o >>= 1) tall += __shfl_xor(tall, o);
-      tall = __builtin_amdgcn_readfirstlane(tall) * tiles_n;
-      if (2 * ((tall + grid - 1) / grid) <= rounds) {
-        __syncthreads();                                                  // (every wave has read the tiles)
-        ffn_offsets<false>(nullptr, a.E, 256, tiles_n, s_off, s_tile);
-        __syncthreads();
-        ffn_tall<UP>(a, smem, (int*)(smem + 2 * FFN_TALL_STAGE), s_off, s_tile);
-        return;
-      }
-    }
-  }
   const int per = (ntiles + 7) >> 3;                                     // tiles of an XCD's run
   const int first = ((int)blockIdx.x & 7) * per, last = min(first + per, ntiles), step_wg = (int)(gridDim.x + 7 - (blockIdx.x & 7)) >> 3;
   int t = first + ((int)blockIdx.x >> 3);
@@ -601,7 +591,7 @@ __global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a)
 __global__ __launch_bounds__(256) void moe_combine_kernel(const FfnArgs a) {
   __shared__ int s_off[FFN_MAX_E + 1];
   __shared__ int s_row[FFN_MAX_K]; __shared__ float s_w[FFN_MAX_K];
-  ffn_offsets<true>(a.counts, a.E, 1, 1, s_off, nullptr);
+  ffn_offsets(a.counts, a.E, 1, 1, s_off, nullptr);
   __syncthreads();
   for (int t = blockIdx.x; t < a.T; t += gridDim.x) {
     if ((int)threadIdx.x < a.k) {
@@ -702,7 +692,10 @@ int tga_moe_feed_forward(const void* x_bf16, const float* logits, int64_t T, int
   // Tile height by the rows per expert r, us of the call (heights 16 / 32 / 64 / 128; MI355X).  64 experts, D 2048, I 512, k 8, even popularity: r = 2 50.5 / 52.0 / 51.8 / 51.2, 8 61.4 / 62.4 / 62.7 / 61.9,
   // 32 86.6 / 69.5 / 68.4 / 69.5, 48 - / 87 / 80 / 73, 64 126 / 90 / 89 / 76, 128 199 / 125 / 119 / 112, 200 271 / 164 / 155 / 119; popularity by 1 / rank^1.1: 2 45.9 / 46.5 / 49.2 / 48.1, 16 82 / 67 / 84 / 73,
   // 32 89 / 83 / 83 / 94, 64 127 / 90 / 92 / 100, 128 202 / 127 / 119 / 115, 200 278 / 166 / 150 / 146.  16 experts, D 1536, I 768, k 4 (few tiles: lower ones fill the chip): 16 35.2 / 33.3 / 36.3 / 40.9,
-  // 64 49.9 / 37.9 / 40.0 / 47.3, 128 66 / 53.7 / 43.1 / 51.5, 200 86 / 60.9 / 60.1 / 53.3.  Where even popularity makes 128 rows two rounds of the launch and 256 one, the device takes 256 (64 experts, r = 128 / 160: 112 -> 100, 112 -> 106): it has the counts.
+  // 64 49.9 / 37.9 / 40.0 / 47.3, 128 66 / 53.7 / 43.1 / 51.5, 200 86 / 60.9 / 60.1 / 53.3.  Where 256 rows make at most five ninths of the rounds that 128 make, each launch takes them on the device, which has
+  // the counts.  gate/up or down alone, rounds 128 / 256, us of 128 / 256: 2 / 1 rounds 57.1 / 45.3 (64 experts, r = 128), 58.0 / 55.5 (8, r = 1024), 56.0 / 52.8 (16, r = 512); 4 / 2 89.3 / 84.9 and 45.7 / 43.5
+  // (16, r = 1000), 116 / 109 (8, r = 4096); 8 / 4 70.6 / 67.7 (8, r = 4096); 9 / 5 76.7 / 74.7 (16, r = 2048), 57.2 / 55.2 (32, r = 1024); 5 / 3 137 / 132 (16, r = 2048, even) but 141 / 151 (skewed), 134 / 148 (32),
+  // 46.8 / 50.3 (64, r = 250); 3 / 2 82 / 101 (8, r = 2048), 50 / 64; 8 / 5 53.8 / 54.1.  Against tiles of 256 for all of them: the call of 16 experts, r = 2048, even, 232 -> 240, skewed 256 -> 243.
   // Low tiles read a weight about once.  Where the layer's weights are also more than half of the 256 MB behind the L2s, so that they are not there again at the next call, the requests pass them by:
   // 32 tokens of 64 experts, I 768 67.7 -> 61.9 us, r = 4, I 512 56.5 -> 51.1, r = 24 64.7 -> 61.7; of 57 MB that are still there 32.4 -> 36.1.
   const bool once = 3ll * n_experts * I * D >= (128ll << 20);
