@@ -630,20 +630,31 @@ static FfnLayout ffn_layout(long long T, long long D, long long I, long long E, 
   return l;
 }
 
+// per_cu: workgroups of a CU, at most; each launch has as many as its LDS leaves room for (16-row tiles: three of gate/up, whose rows' tokens sit in LDS, and four of down up to 90 experts).  With four for
+// both, a quarter of gate/up's tiles beyond 768 began when others had ended: 80 experts, I 768, 32 / 56 tokens 93.5 -> 90.7 / 97.7 -> 94.2 us, 128 experts (down: three), I 512 / 768, 64 tokens 110 -> 101 / 132 -> 123, up to 768 tiles the same.
 template <int BM, int WM, int WN, int NB, bool ONCE>
-static hipError_t launch_ffn(const FfnArgs& a, int grid, hipStream_t s) {
+static hipError_t launch_ffn(const FfnArgs& a, int n_cu, int per_cu, hipStream_t s) {
   constexpr int ring = (BM + 64 * WN) * (128 * NB + 16), most = ring + 8 * (FFN_MAX_E + 1);
   const int lds = ring + 8 * (a.E + 1);
   auto up = ffn_gemm_kernel<BM, WM, WN, NB, true, ONCE>; auto down = ffn_gemm_kernel<BM, WM, WN, NB, false, ONCE>;
+  static int own[2];                                                     // LDS of the kernels' own
   static const hipError_t configured = [&] {
-    const hipError_t e = hipFuncSetAttribute((const void*)up, hipFuncAttributeMaxDynamicSharedMemorySize, most);
-    return e != hipSuccess ? e : hipFuncSetAttribute((const void*)down, hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    const void* k[2] = {(const void*)up, (const void*)down};
+    for (int i = 0; i < 2; i++) {
+      hipFuncAttributes fa;
+      hipError_t e = hipFuncGetAttributes(&fa, k[i]);
+      if (e == hipSuccess) e = hipFuncSetAttribute(k[i], hipFuncAttributeMaxDynamicSharedMemorySize, most);
+      if (e != hipSuccess) return e;
+      own[i] = (int)fa.sharedSizeBytes;
+    }
+    return hipSuccess;
   }();
   if (configured != hipSuccess) return configured;
-  up<<<grid, 64 * WM * WN, lds, s>>>(a);
+  auto grid = [&](int i) { const int fit = 160 * 1024 / ((lds + own[i] + 1279) / 1280 * 1280); return n_cu * (fit < 1 ? 1 : fit < per_cu ? fit : per_cu); };      // (LDS is handed out in pieces of 1280 bytes)
+  up<<<grid(0), 64 * WM * WN, lds, s>>>(a);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  down<<<grid, 64 * WM * WN, lds, s>>>(a);
+  down<<<grid(1), 64 * WM * WN, lds, s>>>(a);
   return hipGetLastError();
 }
 
@@ -700,13 +711,13 @@ int tga_moe_feed_forward(const void* x_bf16, const float* logits, int64_t T, int
   // 32 tokens of 64 experts, I 768 67.7 -> 61.9 us, r = 4, I 512 56.5 -> 51.1, r = 24 64.7 -> 61.7; of 57 MB that are still there 32.4 -> 36.1.
   const bool once = 3ll * n_experts * I * D >= (128ll << 20);
   if (T * k < 6ll * n_experts) {
-    TGA_HIP((once ? launch_ffn<16, 1, 2, 2, true>(a, 4 * n_cu, s) : launch_ffn<16, 1, 2, 2, false>(a, 4 * n_cu, s)));
+    TGA_HIP((once ? launch_ffn<16, 1, 2, 2, true>(a, n_cu, 4, s) : launch_ffn<16, 1, 2, 2, false>(a, n_cu, 4, s)));
   } else if (T * k < 48ll * n_experts) {
-    TGA_HIP((once ? launch_ffn<32, 2, 2, 2, true>(a, 3 * n_cu, s) : launch_ffn<32, 2, 2, 2, false>(a, 3 * n_cu, s)));
+    TGA_HIP((once ? launch_ffn<32, 2, 2, 2, true>(a, n_cu, 3, s) : launch_ffn<32, 2, 2, 2, false>(a, n_cu, 3, s)));
   } else if (4 * (n_experts * ((T * k + 128ll * n_experts - 1) / (128ll * n_experts)) * (2 * I / 256)) < 3 * n_cu) {
-    TGA_HIP((launch_ffn<64, 2, 2, 2, false>(a, 2 * n_cu, s)));
+    TGA_HIP((launch_ffn<64, 2, 2, 2, false>(a, n_cu, 2, s)));
   } else {
-    TGA_HIP((launch_ffn<128, 2, 4, 3, false>(a, n_cu, s)));
+    TGA_HIP((launch_ffn<128, 2, 4, 3, false>(a, n_cu, 1, s)));
   }
   moe_combine_kernel<<<(unsigned)(T < 2048 ? T : 2048), 256, 0, s>>>(a);
   TGA_LAUNCH_CHECK();
