@@ -40,7 +40,7 @@ const char* tga_last_error(void);
 int tga_init(int device);                                  /* hipSetDevice + kernel attribute set-up; ops_hip.py:14-20.  Also allocates, once per device, the 160 MB workspace of the 17 .. 128 row linears */
 int tga_device_name(char* buf, size_t len);
 int tga_host_malloc(void** ptr, size_t nbytes);            /* pinned host memory that kernels can write (hipHostMalloc); refused while the thread captures a stream */
-int tga_host_free(void* ptr);                              /* may be called during a capture: the block goes back to the runtime with the next tga_host_malloc or tga_trim */
+int tga_host_free(void* ptr);                              /* may be called during a capture: the block goes back to the runtime with the next tga_host_malloc or tga_trim; a pointer that is no such block, or freed before, is an error */
 int tga_malloc(void** ptr, size_t nbytes);                 /* ops_hip.py:60-62; served from freed blocks of the same size class where one is kept; refused while the thread captures a stream, whoever opened the capture (as hipMalloc is) */
 int tga_free(void* ptr);                                   /* ops_hip.py:63; keeps the block for later requests (at most 4 GiB per device, blocks of at most 1 GiB): it is handed out again only after a wait for the device; a block freed before is an error */
 int tga_trim(void);                                        /* gives every kept block back to the runtime; refused while the thread captures */

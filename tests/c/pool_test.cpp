@@ -159,9 +159,15 @@ static void pinned_freed_in_a_capture() {
     CHECK(!pinned_free(b)); CHECK(!pinned_free(c)); CHECK(!pool_give_back()); CHECK(g_live.empty());
   }
 }
+static void pinned_of_someone_else() {
+  void *a, *b; int other = 0; CHECK(!pinned_malloc(&a, 64));
+  CHECK(pinned_free(&other) != 0); CHECK(pinned_free((char*)a + 4) != 0);      // (refused here and not in the next caller's request)
+  CHECK(!pinned_malloc(&b, 64)); CHECK(g_live.count(a) && g_live.count(b));
+  CHECK(!pinned_free(a)); CHECK(!pinned_free(b)); CHECK(!pool_give_back()); CHECK(g_live.empty());
+}
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}, {"capture_of_its_own", capture_of_its_own}, {"classes_hold_little_more", classes_hold_little_more}, {"no_host_memory", no_host_memory}, {"full_of_other_blocks", full_of_other_blocks}, {"pinned_freed_in_a_capture", pinned_freed_in_a_capture}};
+  const std::map<std::string, void (*)()> tests = {{"freed_twice", freed_twice}, {"waits_before_handing_out", waits_before_handing_out}, {"capture_opened_elsewhere", capture_opened_elsewhere}, {"capture_of_another_thread", capture_of_another_thread}, {"a_free_that_fails", a_free_that_fails}, {"capture_of_its_own", capture_of_its_own}, {"classes_hold_little_more", classes_hold_little_more}, {"no_host_memory", no_host_memory}, {"full_of_other_blocks", full_of_other_blocks}, {"pinned_freed_in_a_capture", pinned_freed_in_a_capture}, {"pinned_of_someone_else", pinned_of_someone_else}};
   CHECK(argc == 2 && tests.count(argv[1]));
   tests.at(argv[1])();
   puts("ok");

@@ -11,7 +11,7 @@ def program(tmp_path_factory):
   assert r.returncode == 0, r.stderr
   return exe
 
-@pytest.mark.parametrize("case", ["freed_twice", "waits_before_handing_out", "capture_opened_elsewhere", "capture_of_another_thread", "a_free_that_fails", "capture_of_its_own", "classes_hold_little_more", "no_host_memory", "full_of_other_blocks", "pinned_freed_in_a_capture"])
+@pytest.mark.parametrize("case", ["freed_twice", "waits_before_handing_out", "capture_opened_elsewhere", "capture_of_another_thread", "a_free_that_fails", "capture_of_its_own", "classes_hold_little_more", "no_host_memory", "full_of_other_blocks", "pinned_freed_in_a_capture", "pinned_of_someone_else"])
 def test_pool(program, case):
   r = subprocess.run([str(program), case], capture_output=True, text=True, timeout=60)
   assert r.returncode == 0, r.stdout + r.stderr

@@ -1,5 +1,6 @@
 // Device allocations behind tga_malloc / tga_free (included by runtime.hip, and on the host by the test of its rules, which brings functions of its own under the names of the runtime's).
 #pragma once
+#include <algorithm>
 #include <exception>
 #include <map>
 #include <mutex>
@@ -133,7 +134,7 @@ static int pool_free_(void* ptr) {
 }
 // Pinned host memory: a block that is given back waits in a list, without a call to the runtime (an hipHostFree would end a capture of its thread, and a model may be collected during one), for the
 // next request or tga_trim(); the list holds no more than what was in use at a time since the last request.
-static std::vector<void*> g_pinned_freed;
+static std::vector<void*> g_pinned, g_pinned_freed;                                   // in use; given back
 static int pinned_release() { while (!g_pinned_freed.empty()) { void* q = g_pinned_freed.back(); g_pinned_freed.pop_back(); TGA_HIP(hipHostFree(q)); } return 0; }
 static int pinned_malloc_(void** ptr, size_t n) {
   TGA_REQUIRE(!t_captures, "tga_host_malloc: not while this thread captures a stream");
@@ -141,12 +142,15 @@ static int pinned_malloc_(void** ptr, size_t n) {
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   if (const int rc = pinned_release()) return rc;
   TGA_HIP(hipHostMalloc(ptr, n, hipHostMallocDefault));
+  try { g_pinned.push_back(*ptr); } catch (...) { (void)hipHostFree(*ptr); *ptr = nullptr; throw; }
   return 0;
 }
 static int pinned_free_(void* ptr) {
   std::lock_guard<std::mutex> lock(g_pool_mutex);
-  for (void* q : g_pinned_freed) TGA_REQUIRE(q != ptr, "tga_host_free: the block has been freed before");
+  const auto it = std::find(g_pinned.begin(), g_pinned.end(), ptr);
+  TGA_REQUIRE(it != g_pinned.end(), "tga_host_free: no block of tga_host_malloc, or one that has been freed before");      // (in the list it would fail the next caller's request)
   g_pinned_freed.push_back(ptr);
+  g_pinned.erase(it);
   return 0;
 }
 static int pool_give_back_() {
