@@ -31,6 +31,20 @@ def test_small_model_logits_and_tokens(gpu):
   assert got == ref
   assert worst <= 1e-3
 
+def test_a_prompt_is_done_when_its_call_returns(gpu, monkeypatch):
+  """prefill() and reset() wait for what they launched - their errors are theirs and the record can be read on any stream -, also where nothing but the sequence's record is set; a sequence that
+  generate() starts is waited for once, behind its first step."""
+  model, _ = _build(gpu, SMALL, 256, seed=5)
+  prompt = list(range(200))
+  model.prefill(prompt)
+  log, L, wait = [], gpu.lib(), model.stream.synchronize
+  begin = L.tga_decode_begin
+  monkeypatch.setattr(L, "tga_decode_begin", lambda *a: (log.append("begin"), begin(*a))[1])
+  monkeypatch.setattr(model.stream, "synchronize", lambda: (log.append("wait"), wait())[1], raising=False)
+  for call in (lambda: model.prefill(prompt), lambda: model.prefill(prompt, reuse_cache=False), lambda: model.reset(prompt[:7], 3), lambda: list(model.generate(prompt, 1))):
+    log.clear(); call()
+    assert log[-2:] == ["begin", "wait"], log
+
 def test_context_and_token_guards(gpu):
   """The sequence ends at max_context like the reference's generate loop (tinygrad/llm/model.py:475), ids outside the vocabulary are refused on
   the host, and the kernels themselves refuse (flag, no access) a position or token outside their tables."""

@@ -514,9 +514,10 @@ class Transformer:
     if not 0 <= start_pos < len(tokens): raise ValueError(f"start position {start_pos} outside the prompt of {len(tokens)} tokens")
     self._cached_tokens = list(tokens[:start_pos])
     self._start(tokens, start_pos)
+    self.stream.synchronize()
 
   def _start(self, tokens: list[int], start_pos: int):
-    """reset() behind its checks, with the list of cached tokens already cut to start_pos."""
+    """reset() behind its checks, with the list of cached tokens already cut to start_pos, on self.stream: nothing waits for it here."""
     c, s = self.config, self.s
     if start_pos < len(tokens) - 1: s.prompt.view(0, (len(tokens),), np.int32).copyin(np.array(tokens, dtype=np.int32))     # (nothing reads the prompt from its last token on)
     rt.check(rt.lib().tga_decode_begin(s.state.ptr, start_pos, int(tokens[start_pos]), len(tokens), c.vocab_size, self.stream.handle))
@@ -526,6 +527,11 @@ class Transformer:
     """Feeds all but the last prompt token (KV cache fill); the last one is consumed by the first decode step.  Like the reference's generate
     (model.py:472-473) the positions whose tokens equal what the cache already holds are not recomputed.  on_block: token by token with eager launches,
     on_block(i) after the launches of block i of every position (see _step)."""
+    self._prefill(tokens, use_graph, reuse_cache, on_block)
+    self.stream.synchronize()
+
+  def _prefill(self, tokens: list[int], use_graph: bool = True, reuse_cache: bool = True, on_block=None):
+    """prefill() whose last launches may still run on self.stream when it returns: generate() waits behind its first step."""
     start = self.get_start_pos(tokens) if reuse_cache else 0
     self.prefill_steps = len(tokens) - 1 - start                        # (positions the last call actually computed)
     reused = start
@@ -572,7 +578,6 @@ class Transformer:
     self._steps_done = len(tokens) - 1
     if len(self._cached_tokens) != len(tokens) - 1: self._cached_tokens = list(tokens[:-1])
     self._last_input = tokens[-1]
-    if start < len(tokens) - 1: self.stream.synchronize()
 
   def decode_step(self, use_graph: bool = True, sync: bool = True, on_block=None):
     """One token.  The position it occupies must exist in the KV cache and the rotation table: like the reference's generate loop
@@ -587,7 +592,7 @@ class Transformer:
   def generate(self, tokens: list[int], max_new_tokens: int, use_graph: bool = True):
     """Greedy decoding (temperature 0): yields one token id per step, like Transformer.generate (model.py:464-484), and like it stops when
     the context is full (model.py:475)."""
-    self.prefill(tokens, use_graph)
+    self._prefill(tokens, use_graph)
     err = 1                                                             # (no step: the record itself is read)
     for i in range(min(max_new_tokens, self.config.max_context - len(tokens), self.max_new)):
       self.decode_step(use_graph, sync=True)                          # the reference syncs once per token too (out.item(), model.py:482)
