@@ -552,6 +552,25 @@ def test_small_batch_of_superblocks_that_start_off_a_piece(gpu, n, k, m, f32):
     qlinear_multi([lin], xb, [rb], epilogue=1, resid=[rb])
     assert ol.rel_err(rb.numpy(), res + ref) <= TOL, rep
 
+@pytest.mark.parametrize("n,k", [(8208, 4096), (16400, 2048)])
+def test_fp16_rows_through_and_past_the_caches(gpu, n, k):
+  """Launches of 64 MB of fp16 weights and more request them past the caches, smaller ones do not (one row, five on the rings and on the barrier kernel, several matrices): the bits of the two halves."""
+  from tinygrad_amd.nn import QuantLinear, qlinear_multi
+  rng = np.random.default_rng(n)
+  w = (rng.standard_normal((n, k), dtype=np.float32) * np.float32(k ** -0.5)).astype(np.float16)
+  whole, half = gpu.Buffer.from_numpy(w.view(np.uint8).reshape(-1)), n // 32 * 16
+  cut = half * k * 2
+  parts = [whole.view(0, (cut,), np.uint8), whole.view(cut, (whole.nbytes - cut,), np.uint8)]
+  assert whole.nbytes >= 64 << 20 > max(b.nbytes for b in parts)
+  lins = [QuantLinear(parts[0], 1, half, k), QuantLinear(parts[1], 1, n - half, k)]
+  for m in (1, 5):
+    x = gpu.Buffer.from_numpy(synth.activations(rng, m, k, np.float32))
+    y = QuantLinear(whole, 1, n, k)(x).numpy()
+    np.testing.assert_array_equal(y, np.concatenate([lin(x).numpy() for lin in lins], axis=1))
+    outs = [gpu.Buffer((m, lin.out_features), np.float32) for lin in lins]
+    qlinear_multi(lins, x, outs)
+    np.testing.assert_array_equal(y, np.concatenate([o.numpy() for o in outs], axis=1))
+
 @pytest.mark.parametrize("n,k,m", [(4099, 1024, 1), (8192, 2048, 1), (33000, 4096, 1), (4099, 14336, 1), (16400, 4096, 2)])
 def test_equal_rows_of_q6_k_have_equal_results(gpu, n, k, m):
   """The bits of a row do not hang on where it lies in the matrix (the rows of a wave, the steps of its loop): rows of the same bytes give the same float32."""

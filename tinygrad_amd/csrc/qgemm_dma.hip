@@ -116,11 +116,20 @@ __global__ __launch_bounds__(QD_NW * 64) void qgemm_dma_kernel(const QArgs args,
     const uint8_t* base_up = SW ? a.w[1] + goff : base;
     char* dst = ring + (size_t)islot * (2 * SLOT_BYTES);
     const bool two = 2 * ist + 1 < nslots;
+    if (T_ == GGML_F16 ? a.ntot * a.row_bytes >= QG_PAST_F16 : T_ != GGML_Q6_K) {     // (past the caches: see qgemm_wp.hip)
 #pragma unroll
-    for (int i = 0; i < IMAX; i++) {
-      const int j = wave + QD_NW * i;
-      if (j < NI2)                                                     // (the same for the whole wave)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((from_up[i] ? base_up : base) + (two ? doff[i] : doff_odd[i])), (__attribute__((address_space(3))) void*)(dst + j * 1024), 16, 0, T_ == GGML_Q6_K ? 0 : 2);     // (past the caches: see qgemm_wp.hip)
+      for (int i = 0; i < IMAX; i++) {
+        const int j = wave + QD_NW * i;
+        if (j < NI2)                                                   // (the same for the whole wave)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((from_up[i] ? base_up : base) + (two ? doff[i] : doff_odd[i])), (__attribute__((address_space(3))) void*)(dst + j * 1024), 16, 0, 2);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < IMAX; i++) {
+        const int j = wave + QD_NW * i;
+        if (j < NI2)                                                   // (the same for the whole wave)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((from_up[i] ? base_up : base) + (two ? doff[i] : doff_odd[i])), (__attribute__((address_space(3))) void*)(dst + j * 1024), 16, 0, 0);
+      }
     }
     if (++ist == spg) { ist = 0; ij++; }
     islot = islot + 1 == nb ? 0 : islot + 1;

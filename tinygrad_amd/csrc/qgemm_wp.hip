@@ -89,9 +89,11 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
   }
   auto unit0 = [&](int ss) { return BYSTEP ? 4 * ((TEAMS == 1 ? 8 * (wave >> 2) : 0) + (wave & 3) + 4 * ss) : wave * UPW + 4 * ss; };      // the first of the four units of step ss
   auto step_byte = [&](int ss) { return unit0(ss) / 4 * 210; };          // (BYSTEP) where its superblock starts in a row
-  // (weights pass the caches by (2): they are read once per launch and a model's do not come round again in time.  Eight rows, memory cold: Q8_0 14336 x 4096 16.2 -> 14.8 us, 4096 x 14336 18.2 -> 16.0,
-  // 4096 x 4096 7.9 -> 7.1, Q4_K 14336 x 4096 15.5 -> 14.7, Q4_0 13.3 -> 12.4, fp16 4096 x 4096 10.8 -> 10.0; the same bytes still behind the L2s from call to call: 14.0 -> 14.4, 15.4 -> 15.3, 6.8 -> 6.6.
-  // Q6_K's windows share lines between requests: 103 -> 106 on the lm-head, so they stay)
+  // Weights pass the caches (2): they are read once per launch and a model's do not come round again in time.  Eight rows, memory cold: Q8_0 14336 x 4096 16.2 -> 14.8 us, 4096 x 14336 18.2 -> 16.0,
+  // Q4_K 14336 x 4096 15.5 -> 14.7, Q4_0 13.3 -> 12.4.  The same matrix from call to call: within 0.3 us either way up to 16 MB, no slower beyond (kernels alone, Q8_0 K 4096, 16 / 32 / 64 MB 6.7 / 8.7 / 14.5 ->
+  // 6.6 / 8.5 / 13.4, Q4_0 8.1 / 12.2 / 17.9 -> 8.2 / 12.2 / 17.0, Q4_K 10.0 / 14.6 / 23.1 -> 9.9 / 14.4 / 22.7).  fp16 rows from QG_PAST_F16 bytes on; Q6_K's windows share lines between requests: 103 -> 106 on the
+  // lm-head, so they stay.
+  const bool past = T_ == GGML_F16 ? a.ntot * a.row_bytes >= QG_PAST_F16 : T_ != GGML_Q6_K;
   auto issue = [&](long long k, int slot) {
     const long long j = team + TEAMS * (IPG == 1 ? k : k / IPG);
     const long long grp = (long long)blockIdx.x + j * gridDim.x;
@@ -100,10 +102,16 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
     const uint8_t* base = w_of(sg) + goff;
     const uint8_t* base_up = SW ? a.w[1] + goff : base;
     char* dst = ringw + slot * STAGE;
+    if (past) {
 #pragma unroll
-    for (int i = 0; i < NI; i++) {
-      if (i + 1 < NI || REM == 64 || lane < REM)         // (the last instruction fills the rest of the stage and nothing beyond it)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((from_up[i] ? base_up : base) + doff[i]), (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, 0, T_ == GGML_Q6_K ? 0 : 2);
+      for (int i = 0; i < NI; i++)
+        if (i + 1 < NI || REM == 64 || lane < REM)       // (the last instruction fills the rest of the stage and nothing beyond it)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((from_up[i] ? base_up : base) + doff[i]), (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, 0, 2);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NI; i++)
+        if (i + 1 < NI || REM == 64 || lane < REM)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((from_up[i] ? base_up : base) + doff[i]), (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, 0, 0);
     }
   };
 

@@ -187,7 +187,7 @@ __device__ __forceinline__ void qgemv1_body(const QArgs& args, const unsigned bx
       long long rr = (EPI == 2) ? row : row + r;
       rr = rr < last ? rr : last;
       const uint8_t* rp = ((EPI == 2 && r == 1) ? base1 : base0) + rr * a.row_bytes;
-      if constexpr (T == GGML_F16) g.w[r] = F::load_nu(rp, uc, a.nu); else g.w[r] = F::load(rp, uc);
+      if constexpr (T == GGML_F16 || T == F_F16_PAST) g.w[r] = F::load_nu(rp, uc, a.nu); else g.w[r] = F::load(rp, uc);
     }
     if constexpr (EPI == 1) {
       if constexpr (WK > 1) {                                      // wave 0, lane m R + r stores row + r of activation row m
@@ -293,7 +293,7 @@ __device__ __forceinline__ void qgemv1_body(const QArgs& args, const unsigned bx
   };
   // piece i (elements 8i .. 8i+7 as 4 fp16 pairs) into LDS: unit F::unit_of(8i) at pair F::pair_of(8i) (4 consecutive pairs stay inside one unit run)
   auto put_piece = [&](int i, const u32x4& v, int m = 0) {
-    if constexpr (T == GGML_F16) *(u32x4*)(xlds + (m * a.nu + F::unit_of_nu(8 * i, a.nu)) * USTRIDE + F::pair_of_nu(8 * i, a.nu)) = v;
+    if constexpr (T == GGML_F16 || T == F_F16_PAST) *(u32x4*)(xlds + (m * a.nu + F::unit_of_nu(8 * i, a.nu)) * USTRIDE + F::pair_of_nu(8 * i, a.nu)) = v;
     else *(u32x4*)(xlds + (m * a.nu + F::unit_of(8 * i)) * USTRIDE + F::pair_of(8 * i)) = v;
   };
   auto pack8 = [](const f32x4& l, const f32x4& h) {

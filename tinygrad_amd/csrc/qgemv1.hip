@@ -5,6 +5,7 @@
 extern template int qgemv1_launch_format<F_Q4_0P>(QArgs, hipStream_t);
 extern template int qgemv1_launch_format<F_Q8_0P>(QArgs, hipStream_t);
 extern template int qgemv1_launch_format<GGML_F16>(QArgs, hipStream_t);
+extern template int qgemv1_launch_format<F_F16_PAST>(QArgs, hipStream_t);
 extern template int qgemv1_launch_format<GGML_MXFP4>(QArgs, hipStream_t);
 extern template int qgemv1_launch_format<GGML_Q6_K>(QArgs, hipStream_t);
 extern template int qgemv1_launch_format<GGML_Q4_K>(QArgs, hipStream_t);
@@ -40,7 +41,7 @@ int tga_qgemv1_dispatch(int fmt, const QArgs& a, hipStream_t s) {
     case GGML_IQ2_S: return qgemv1_launch_format<GGML_IQ2_S>(a, s);
     case GGML_Q1_0: return qgemv1_launch_format<GGML_Q1_0>(a, s);
     case GGML_MXFP4: return qgemv1_launch_format<GGML_MXFP4>(a, s);
-    case GGML_F16: return qgemv1_launch_format<GGML_F16>(a, s);
+    case GGML_F16: return (a.epilogue == 2 ? 2 : 1) * a.ntot * a.K * 2 * (a.sel ? a.xdiv_jobs : 1) >= QG_PAST_F16 ? qgemv1_launch_format<F_F16_PAST>(a, s) : qgemv1_launch_format<GGML_F16>(a, s);
   }
   return -1;
 }
