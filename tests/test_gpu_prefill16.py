@@ -140,6 +140,14 @@ def test_expert_products_of_values_of_every_size(gpu, monkeypatch, name):
   assert a._chunker._rows16_ws is not None and b._chunker._rows16_ws is None and np.isfinite(b.blk[-1].cache_v.numpy()).all()
   _same_bits(a, b, 125)
 
+def test_one_step_of_sixteen_stays_one(gpu):
+  """Sixteen to nineteen positions are one step of sixteen rows (a graph) and single ones; from twenty on, or where a row's experts have many hidden values, all rows go together."""
+  wide = dict(CONFIGS["512x256"], hidden_dim=1536, num_experts_per_tok=8, num_blocks=1)
+  for cfg, n, together in ((CONFIGS["512x256"], 17, False), (CONFIGS["512x256"], 20, False), (CONFIGS["512x256"], 21, True), (wide, 16, False), (wide, 17, True), (wide, 20, True)):
+    m = _models(cfg, n, 64)[0]
+    m.prefill(list(range(n)))
+    assert (m._chunker is not None and m._chunker._rows16_ws is not None) == together, (n, together)
+
 @pytest.mark.parametrize("name", ["1536x768", "512x256"])
 @pytest.mark.parametrize("n,at", [(40, 21), (100, 70), (333, 200)])
 def test_values_that_are_not_finite_stay_with_later_positions(gpu, name, n, at):

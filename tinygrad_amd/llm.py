@@ -57,7 +57,12 @@ MANY_ROWS = 2048                   # rows of a prefill step at most (its buffers
 # Fewer rows are one step of the small-batch kernels.  Lockstep prompts, one step of many rows against so many lockstep steps (eight blocks of the 8B architecture, Q8_0 / Q4_0 / Q4_K_M): 16 sequences of two
 # positions 1079 against 1534 / 988 against 1336 / 1132 against 1619 us, 8 of three 1059 against 2038 / 956 against 1795 / 1129 against 2234, 4 of five 1018 against 3073 / 944 against 2655 / 1097 against 3349
 MANY_ROWS_MIN = 17
-ROWS16, ROWS16_MIN, ROWS16_BYTES = 1024, 16, 1 << 29     # prefill_rows16: rows of a step at most (a multiple of sixteen) and at least, bytes of its buffers from which on it takes fewer
+# prefill_rows16: rows of a step at most (a multiple of sixteen), positions of a prompt at least, bytes of its buffers from which on it takes fewer rows.  Sixteen to nineteen positions are one step of
+# sixteen, whose launches are a graph; prefill_rows16 is faster there only where a row's experts have many hidden values (k times the width).  A prompt of 17 tokens and its first logits, prefill_rows16 / the
+# step, six blocks, us: D 2048 k 2 x 1536 1144 / 871, 4 x 1024 1050 / 877, 8 x 1024 1248 / 1088, 8 x 1536 1222 / 1330; D 1024 694 / 600 (2 x 512), 925 / 818 (8 x 1024), 877 / 936 (8 x 1536); D 512 661 / 669
+# (4 x 1024), 745 / 876 (8 x 1536).  One more step of four: 21 tokens 1277 / 1611, 1194 / 1299 (D 2048, 8 x 1024 and 2 x 1536), 704 / 958 (D 1024, 2 x 512).
+ROWS16, ROWS16_MIN, ROWS16_BYTES = 1024, 20, 1 << 29
+ROWS16_WIDE = 10240                # k times the experts' width from which on four positions fewer are enough
 
 def precompute_freqs_cis(dim: int, end: int, theta: float) -> np.ndarray:
   """tinygrad/llm/model.py:16-19 in float32: cat(cos(pos * f), sin(pos * f)), f = 1 / theta^(2i/dim)."""
@@ -551,7 +556,7 @@ class Transformer:
     # MoE models keep the ladder (one step each of 8 and / or 4 positions, then single ones).
     overlap = not self.config.num_experts
     # MoE models: the rows of the ladder's steps of sixteen, eight and four positions together, each with the bits its step gives it, where the model is in the range of tga_prefill16_step
-    if B == 16 and self.config.num_experts and len(tokens) - 1 - start >= ROWS16_MIN:
+    if B == 16 and self.config.num_experts and len(tokens) - 1 - start >= ROWS16_MIN - (4 if self.config.num_experts_per_tok * self.config.hidden_dim > ROWS16_WIDE else 0):
       if self._chunker is None or self._chunker.batch != B: self._chunker = BatchedTransformer(self.config, self._state_dict, B, max_new=1, chunk_of=self)
       start += self._chunker.prefill_rows16(tokens, start)
     for b in [B] + [t for t in (64, 32, 16, 8, 4) if t < B]:
