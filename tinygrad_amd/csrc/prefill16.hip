@@ -394,8 +394,8 @@ __global__ __launch_bounds__(1024) void x16_router_kernel(const X16Router a) {
 // ------------------------------------------------------------------------------------------------ the experts
 // An expert's MXFP4 weights against the rows of all its assignments, each result with the bits of the expert GEMV (qgemv1.h): per unit of 32 weights a chain of sixteen dot2 from zero, times the
 // block's scale, then the tree over the units (pairs of neighbours first).  v_dot2_f32_f16 rounds the sum of two products and the addend once, and so does a matrix-core product whose other products
-// are zeros: v_mfma_f32_16x16x4_4b_f16 with two of its four values zero is 2048 dot2 in 32 cycles where the vector unit takes 256 (bits compared over normal, subnormal and huge values, sums
-// from zero and not; with all four values in use they differ, so the matrix cores run at a quarter of their fp16 rate here).
+// are zeros: v_mfma_f32_16x16x4_4b_f16 with two of its four values zero is 1024 dot2 in 32 cycles where the vector unit takes 93 (16 instructions, 5.8 cycles each in a loop of nothing else; bits compared over
+// normal, subnormal and huge values, sums from zero and not; with all four values in use they differ, so the matrix cores run at an eighth of their fp16 rate here).
 // An item is 64 weight rows of one expert (SwiGLU: 32 of gate and the same 32 of up) and all of the expert's rows, in tiles of sixteen.  Workgroups stay for the whole launch and share the tiles of all
 // items evenly, each a contiguous run of them (an item may be cut); wave w holds units 8 w .. of the item's weight rows in registers, so weights are read once per item, and touches those of the next item at
 // the first tile of this one (they wait in the XCD's L2; a second set of registers does not fit).  Lane 16 b + c supplies column c of block b; the sixteen rows of the tile are the other operand, the same for the four blocks, brought to LDS by requests of the wave itself,
