@@ -37,13 +37,16 @@ def test_a_prompt_is_done_when_its_call_returns(gpu, monkeypatch):
   model, _ = _build(gpu, SMALL, 256, seed=5)
   prompt = list(range(200))
   model.prefill(prompt)
-  log, L, wait = [], gpu.lib(), model.stream.synchronize
+  log, L, stream = [], gpu.lib(), type(model.stream)
+  wait = stream.synchronize
   begin = L.tga_decode_begin
   monkeypatch.setattr(L, "tga_decode_begin", lambda *a: (log.append("begin"), begin(*a))[1])
-  monkeypatch.setattr(model.stream, "synchronize", lambda: (log.append("wait"), wait())[1], raising=False)
-  for call in (lambda: model.prefill(prompt), lambda: model.prefill(prompt, reuse_cache=False), lambda: model.reset(prompt[:7], 3), lambda: list(model.generate(prompt, 1))):
+  monkeypatch.setattr(stream, "synchronize", lambda self: (log.append("wait"), wait(self))[1])
+  for call in (lambda: model.prefill(prompt), lambda: model.reset(prompt[:7], 3), lambda: model.prefill(prompt, reuse_cache=False)):
     log.clear(); call()
     assert log[-2:] == ["begin", "wait"], log
+  log.clear(); list(model.generate(prompt, 1))                                   # (the prompt is in the cache)
+  assert log == ["begin", "wait"], log
 
 def test_context_and_token_guards(gpu):
   """The sequence ends at max_context like the reference's generate loop (tinygrad/llm/model.py:475), ids outside the vocabulary are refused on

@@ -521,22 +521,24 @@ class Transformer:
     self._start(tokens, start_pos)
     self.stream.synchronize()
 
-  def _start(self, tokens: list[int], start_pos: int):
-    """reset() behind its checks, with the list of cached tokens already cut to start_pos, on self.stream: nothing waits for it here."""
+  def _start(self, tokens: list[int], start_pos: int, stream=None):
+    """reset() behind its checks, with the list of cached tokens already cut to start_pos, on self.stream or the one given: nothing waits for it here."""
     c, s = self.config, self.s
     if start_pos < len(tokens) - 1: s.prompt.view(0, (len(tokens),), np.int32).copyin(np.array(tokens, dtype=np.int32))     # (nothing reads the prompt from its last token on)
-    rt.check(rt.lib().tga_decode_begin(s.state.ptr, start_pos, int(tokens[start_pos]), len(tokens), c.vocab_size, self.stream.handle))
+    rt.check(rt.lib().tga_decode_begin(s.state.ptr, start_pos, int(tokens[start_pos]), len(tokens), c.vocab_size, (stream or self.stream).handle))
     self._n_prompt, self._steps_done = len(tokens), start_pos
 
   def prefill(self, tokens: list[int], use_graph: bool = True, reuse_cache: bool = True, on_block=None):
     """Feeds all but the last prompt token (KV cache fill); the last one is consumed by the first decode step.  Like the reference's generate
     (model.py:472-473) the positions whose tokens equal what the cache already holds are not recomputed.  on_block: token by token with eager launches,
     on_block(i) after the launches of block i of every position (see _step)."""
-    self._prefill(tokens, use_graph, reuse_cache, on_block)
-    self.stream.synchronize()
+    if self._prefill(tokens, use_graph, reuse_cache, on_block): self.stream.synchronize()
 
   def _prefill(self, tokens: list[int], use_graph: bool = True, reuse_cache: bool = True, on_block=None):
-    """prefill() whose last launches may still run on self.stream when it returns: generate() waits behind its first step."""
+    """prefill() whose last launches may still run on self.stream when it returns True: generate() waits behind its first step."""
+    # Where the chunked steps end at the last position, the sequence's record is set behind them, on their stream and in front of their wait (a wait of its own is 13 us of a prompt)
+    begun = []
+    def begin(stream): begun.append(True); self._start(tokens, len(tokens) - 1, stream)
     start = self.get_start_pos(tokens) if reuse_cache else 0
     self.prefill_steps = len(tokens) - 1 - start                        # (positions the last call actually computed)
     reused = start
@@ -548,7 +550,7 @@ class Transformer:
       if n_rows >= B and self._chunker is None: self._chunker = BatchedTransformer(self.config, self._state_dict, B, max_new=1, chunk_of=self)
       if self._chunker is None and 16 not in self._tail_chunkers: self._tail_chunkers[16] = BatchedTransformer(self.config, self._state_dict, 16, max_new=1, chunk_of=self)
       chunker = self._chunker or self._tail_chunkers[16]
-      if chunker._rows_tables is not None: start += chunker.prefill_rows(tokens, start, n_rows)
+      if chunker._rows_tables is not None: start += chunker.prefill_rows(tokens, start, n_rows, begin)
     if B > 16 and self.config.num_experts: B = 16                       # (MoE blocks keep steps of sixteen positions: longer ones are not measured there)
     # Whole chunks as small-batch steps (model.py:476-481) of the largest size that the prompt holds (the chosen one, else 64, 32, 16, 8 or 4 positions).  Dense models: what
     # they leave is ONE more chunk that ends at the last position and computes some positions again - every row of a step depends on the cache and on its own token
@@ -558,7 +560,7 @@ class Transformer:
     # MoE models: the rows of the ladder's steps of sixteen, eight and four positions together, each with the bits its step gives it, where the model is in the range of tga_prefill16_step
     if B == 16 and self.config.num_experts and len(tokens) - 1 - start >= ROWS16_MIN - (4 if self.config.num_experts_per_tok * self.config.hidden_dim > ROWS16_WIDE else 0):
       if self._chunker is None or self._chunker.batch != B: self._chunker = BatchedTransformer(self.config, self._state_dict, B, max_new=1, chunk_of=self)
-      start += self._chunker.prefill_rows16(tokens, start)
+      start += self._chunker.prefill_rows16(tokens, start, begin)
     for b in [B] + [t for t in (64, 32, 16, 8, 4) if t < B]:
       total = len(tokens) - 1 - start
       if not 2 <= b <= 128 or total < b: continue
@@ -568,21 +570,22 @@ class Transformer:
       else:
         if b not in self._tail_chunkers: self._tail_chunkers[b] = BatchedTransformer(self.config, self._state_dict, b, max_new=1, chunk_of=self)
         chunker = self._tail_chunkers[b]
-      start += chunker.prefill_chunks(tokens, start, total // b, use_graph)
+      start += chunker.prefill_chunks(tokens, start, total // b, use_graph, begin)
       if overlap:
-        if start < len(tokens) - 1: chunker.prefill_chunks(tokens, len(tokens) - 1 - b, 1, use_graph); start = len(tokens) - 1
+        if start < len(tokens) - 1: chunker.prefill_chunks(tokens, len(tokens) - 1 - b, 1, use_graph, begin); start = len(tokens) - 1
         break
     # (reset()'s checks; the reused tokens are ones that have passed them)
     if not 1 <= len(tokens) < self.config.max_context: raise ValueError(f"prompt of {len(tokens)} tokens does not fit max_context {self.config.max_context}")
     rest = tokens[reused:] if reused else tokens
     if min(rest) < 0 or max(rest) >= self.config.vocab_size: raise ValueError(f"token id outside the vocabulary of {self.config.vocab_size}")
-    self._start(tokens, start)
+    if not begun: self._start(tokens, start)
     for _ in range(len(tokens) - 1 - start):
       if use_graph and on_block is None: self._graph(False).launch()
       else: self._step(False, on_block)
     self._steps_done = len(tokens) - 1
     if len(self._cached_tokens) != len(tokens) - 1: self._cached_tokens = list(tokens[:-1])
     self._last_input = tokens[-1]
+    return not begun
 
   def decode_step(self, use_graph: bool = True, sync: bool = True, on_block=None):
     """One token.  The position it occupies must exist in the KV cache and the rotation table: like the reference's generate loop
@@ -766,9 +769,9 @@ class BatchedTransformer:
       rt.check(rt.lib().tga_prefill_step(*self._rows_tables, self._rows_tok.ptr + 4 * at, nseq, m, pos0 + i, self._rows_ws.ptr, self.state.ptr, self.stream.handle))
       at += nseq * m
 
-  def prefill_rows(self, tokens: list[int], start: int, n: int) -> int:
+  def prefill_rows(self, tokens: list[int], start: int, n: int, begin=None) -> int:
     """Chunked prefill for `chunk_of` in steps of many rows: the positions start .. start + n - 1 of the prompt into its KV caches.  Returns the number of positions done
-    (none where there is no memory for the step's buffers)."""
+    (none where there is no memory for the step's buffers).  begin(stream): called in front of the wait for the steps, on this stream, where they end at the prompt's last position but one."""
     c = self.config
     if not self.chunked or self._rows_tables is None: raise RuntimeError("prefill_rows needs a model built with chunk_of and linears in the range of tga_prefill_step")
     if not (0 <= start and n >= 1 and start + n <= len(tokens) < c.max_context): raise ValueError(f"positions {start}+{n} outside the prompt of {len(tokens)} tokens")
@@ -778,13 +781,15 @@ class BatchedTransformer:
     self.state.copyin(st)
     self._owner_stream.synchronize()
     self._prefill_many_rows(np.array(tokens[start:start + n], np.int32)[None, :], start)
+    if begin is not None and start + n == len(tokens) - 1: begin(self.stream)
     self.stream.synchronize()
     self.check_state()
     return n
 
-  def prefill_rows16(self, tokens: list[int], start: int) -> int:
+  def prefill_rows16(self, tokens: list[int], start: int, begin=None) -> int:
     """Chunked prefill for `chunk_of`, an MoE model: the rows of the steps of sixteen positions from start on, and of the one step each of eight and four behind them, all together and with the bits
-    of those steps (csrc/prefill16.hip).  Returns the number of positions done: none for models outside that kernel's range and where there is no memory for its buffers."""
+    of those steps (csrc/prefill16.hip).  Returns the number of positions done: none for models outside that kernel's range and where there is no memory for its buffers.
+    begin: as in prefill_rows."""
     c = self.config
     if not self.chunked or self._rows_tables is None or self.expert_path != "jobs": return 0
     if not (0 <= start < len(tokens) < c.max_context): raise ValueError(f"positions from {start} outside the prompt of {len(tokens)} tokens")
@@ -809,6 +814,7 @@ class BatchedTransformer:
     for i in range(0, n, per):
       m = min(per, n - i)
       rt.check(rt.lib().tga_prefill16_step(*self._rows_tables, self._rows16_tok.ptr + 4 * i, m, max(0, m - max(0, n - tail - i)), start + i, self._rows16_ws.ptr, self.state.ptr, self.stream.handle))
+    if begin is not None and start + n == len(tokens) - 1: begin(self.stream)
     self.stream.synchronize()
     self.check_state()
     return n
@@ -948,9 +954,9 @@ class BatchedTransformer:
       self._graphs[with_head] = g
     return self._graphs[with_head]
 
-  def prefill_chunks(self, tokens: list[int], start: int, n_chunks: int, use_graph: bool = True) -> int:
+  def prefill_chunks(self, tokens: list[int], start: int, n_chunks: int, use_graph: bool = True, begin=None) -> int:
     """Chunked prefill for `chunk_of`: computes the positions start .. start + n_chunks * batch - 1 of the prompt, `batch` at a time, into its KV caches.
-    Returns the number of positions done."""
+    Returns the number of positions done.  begin: as in prefill_rows."""
     c, B = self.config, self.batch
     if not self.chunked: raise RuntimeError("prefill_chunks needs a model built with chunk_of")
     if n_chunks <= 0: return 0
@@ -966,6 +972,7 @@ class BatchedTransformer:
     for _ in range(n_chunks):
       if use_graph: self._graph(False).launch()
       else: self._step(False)
+    if begin is not None and start + n_chunks * B == len(tokens) - 1: begin(self.stream)
     self.stream.synchronize()
     self.check_state()
     return n_chunks * B
