@@ -554,14 +554,14 @@ def test_small_batch_of_superblocks_that_start_off_a_piece(gpu, n, k, m, f32):
 
 @pytest.mark.parametrize("n,k", [(8208, 4096), (16400, 2048)])
 def test_fp16_rows_through_and_past_the_caches(gpu, n, k):
-  """Launches of 64 MB of fp16 weights and more request them past the caches, smaller ones do not (one row, five on the rings and on the barrier kernel, several matrices): the bits of the two halves."""
+  """Launches of 64 MB of fp16 weights and more (several rows: 48 MB) request them past the caches, smaller ones do not (one row, five on the rings and on the barrier kernel, several matrices): the bits of the two halves."""
   from tinygrad_amd.nn import QuantLinear, qlinear_multi
   rng = np.random.default_rng(n)
   w = (rng.standard_normal((n, k), dtype=np.float32) * np.float32(k ** -0.5)).astype(np.float16)
   whole, half = gpu.Buffer.from_numpy(w.view(np.uint8).reshape(-1)), n // 32 * 16
   cut = half * k * 2
   parts = [whole.view(0, (cut,), np.uint8), whole.view(cut, (whole.nbytes - cut,), np.uint8)]
-  assert whole.nbytes >= 64 << 20 > max(b.nbytes for b in parts)
+  assert whole.nbytes >= 64 << 20 and max(b.nbytes for b in parts) < 48 << 20
   lins = [QuantLinear(parts[0], 1, half, k), QuantLinear(parts[1], 1, n - half, k)]
   for m in (1, 5):
     x = gpu.Buffer.from_numpy(synth.activations(rng, m, k, np.float32))

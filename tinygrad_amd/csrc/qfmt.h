@@ -163,12 +163,15 @@ template <> struct Fmt<GGML_Q8_0> {
 
 enum { F_Q4_0P = 1002, F_Q8_0P = 1008 };   // block-pair formats (4-byte aligned 36 / 68 byte units)
 enum { F_F16_PAST = 1001 };                // fp16 rows whose requests pass the caches (single rows)
-// fp16 weights pass the caches from so many bytes in a launch on; smaller matrices may be behind the L2s at the next call, and gain little or nothing where they are not.  us through / past the caches,
+// fp16 weights pass the caches from so many bytes in a launch on (one row; several rows); smaller matrices may be behind the L2s at the next call, and gain little or nothing where they are not.  us through / past the caches,
 // the same matrix again and again | cold: single rows, K = 4096, 4 MB 4.3 / 4.9 | 4.9 / 5.4, 16 MB 4.4 / 5.2 | 6.6 / 6.6, 32 MB 4.7 / 5.8 | 8.4 / 7.9, 48 MB 8.1 / 9.6 | 11.3 / 11.5, 64 MB 12.1 / 11.4 | 14.0 / 13.1,
 // 96 MB 16.4 / 16.2 | 20.1 / 17.8, K = 2048, 32 MB 4.6 / 6.2 | 8.5 / 8.2, 64 MB 12.2 / 11.7 | 13.8 / 13.8; eight rows, K = 4096 (barrier kernel), 4 MB 6.8 / 7.8 | 7.6 / 8.0, 16 MB 6.6 / 7.9 | 8.7 / 8.9,
 // 32 MB 7.2 / 8.9 | 10.2 / 10.3, 48 MB 10.7 / 12.5 | 14.3 / 13.9, 64 MB 13.6 / 14.0 | 15.8 / 15.1, 96 MB 18.0 / 18.9 | 21.0 / 20.0, K = 2048 (wave-private rings), 32 MB 6.5 / 7.0 | 9.9 / 9.6, 64 MB 14.3 / 13.2 | 16.1 / 15.6.
 // (Quantised blocks take longer to decode than to read: through or past is the same from call to call, so theirs pass at every size; see qgemm_wp.hip.)
+// In models: one token of fp16 weights, always past / through below 64 MB, D 4096 H 10240 488 / 480 us, D 2048 H 7168 387 / 373, H 5120 541 / 547, D 1024 193 / 170; eight sequences of D 4096 (q / k / v 48 MB)
+// always past / through below 64 MB / 32 MB 1771 / 1796 / 1776 us a step: several rows pass from 48 MB on.
 #define QG_PAST_F16 (64ll << 20)
+#define QG_PAST_F16_ROWS (48ll << 20)
 
 // Weight bytes always live in global memory: the loads name that address space, so that pointers which reach a kernel through
 // a table in memory (and carry no address space of their own) still become global_load instead of FLAT instructions.

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(QD_NW * 64) void qgemm_dma_kernel(const QArgs args,
     const uint8_t* base_up = SW ? a.w[1] + goff : base;
     char* dst = ring + (size_t)islot * (2 * SLOT_BYTES);
     const bool two = 2 * ist + 1 < nslots;
-    if (T_ == GGML_F16 ? a.ntot * a.row_bytes >= QG_PAST_F16 : T_ != GGML_Q6_K) {     // (past the caches: see qgemm_wp.hip)
+    if (T_ == GGML_F16 ? a.ntot * a.row_bytes >= QG_PAST_F16_ROWS : T_ != GGML_Q6_K) {     // (past the caches: see qgemm_wp.hip)
 #pragma unroll
       for (int i = 0; i < IMAX; i++) {
         const int j = wave + QD_NW * i;

@@ -91,9 +91,9 @@ __global__ __launch_bounds__(WP_NW * 64) void qgemm_wp_kernel(const QArgs args, 
   auto step_byte = [&](int ss) { return unit0(ss) / 4 * 210; };          // (BYSTEP) where its superblock starts in a row
   // Weights pass the caches (2): they are read once per launch and a model's do not come round again in time.  Eight rows, memory cold: Q8_0 14336 x 4096 16.2 -> 14.8 us, 4096 x 14336 18.2 -> 16.0,
   // Q4_K 14336 x 4096 15.5 -> 14.7, Q4_0 13.3 -> 12.4.  The same matrix from call to call: within 0.3 us either way up to 16 MB, no slower beyond (kernels alone, Q8_0 K 4096, 16 / 32 / 64 MB 6.7 / 8.7 / 14.5 ->
-  // 6.6 / 8.5 / 13.4, Q4_0 8.1 / 12.2 / 17.9 -> 8.2 / 12.2 / 17.0, Q4_K 10.0 / 14.6 / 23.1 -> 9.9 / 14.4 / 22.7).  fp16 rows from QG_PAST_F16 bytes on; Q6_K's windows share lines between requests: 103 -> 106 on the
+  // 6.6 / 8.5 / 13.4, Q4_0 8.1 / 12.2 / 17.9 -> 8.2 / 12.2 / 17.0, Q4_K 10.0 / 14.6 / 23.1 -> 9.9 / 14.4 / 22.7).  fp16 rows from QG_PAST_F16_ROWS bytes on; Q6_K's windows share lines between requests: 103 -> 106 on the
   // lm-head, so they stay.
-  const bool past = T_ == GGML_F16 ? a.ntot * a.row_bytes >= QG_PAST_F16 : T_ != GGML_Q6_K;
+  const bool past = T_ == GGML_F16 ? a.ntot * a.row_bytes >= QG_PAST_F16_ROWS : T_ != GGML_Q6_K;
   auto issue = [&](long long k, int slot) {
     const long long j = team + TEAMS * (IPG == 1 ? k : k / IPG);
     const long long grp = (long long)blockIdx.x + j * gridDim.x;
