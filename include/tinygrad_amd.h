@@ -410,7 +410,7 @@ int tga_qlinear_many(int ggml_type, int nseg, const void* const* w, void* const*
                      const float* resid, void* workspace, int64_t workspace_bytes, void* stream);
 int tga_rows_format_ok(int ggml_type, int64_t K, int* ok);
 /* A prefill step of any number of rows (prefill.hip; model.py:464, 476-481): positions pos0 .. pos0 + P - 1 of nseq sequences through all blocks, keys and values appended to
- * the caches.  model / blocks: tables of int64 (pointers as integers) in the order of the PM_ / PB_ enumerations there; tokens: (nseq, P) ids on the device.
+ * the caches.  model / blocks: tables of int64 (pointers as integers) in the order of the PM_ / PB_ enumerations of csrc/prefill.h; tokens: (nseq, P) ids on the device.
  * _plan: bytes of the caller's workspace for that many rows (nseq * P). */
 int tga_prefill_plan(const int64_t* model, int64_t rows, int64_t* nbytes);
 int tga_prefill_step(const int64_t* model, const int64_t* blocks, const int32_t* tokens, int64_t nseq, int64_t P, int64_t pos0, void* workspace, void* state, void* stream);

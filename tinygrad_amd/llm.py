@@ -725,7 +725,7 @@ class BatchedTransformer:
       self.xn_st, self.attn_st, self.act_st = Buffer((R, c.dim), f16).zero_(), Buffer((R, nq), f16).zero_(), Buffer((R, c.hidden_dim), f16).zero_()
 
   def _many_rows_tables(self):
-    """The tables of tga_prefill_step (csrc/prefill.hip: PM_ / PB_ enumerations), or None for a model outside its range: q / k / v biases, head sizes other than 64 and 128, a
+    """The tables of tga_prefill_step (csrc/prefill.h: PM_ / PB_ enumerations), or None for a model outside its range: q / k / v biases, head sizes other than 64 and 128, a
     shared expert, an expert selection bias, ffn_gate / ffn_up of different block types, a router that is not fp16, or block types and row lengths its linears do not take."""
     c = self.config
     def fits(l):
