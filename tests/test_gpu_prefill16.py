@@ -95,6 +95,25 @@ def test_bits_of_steps_that_memory_cuts(gpu, monkeypatch):
     b.prefill(prompt)
     _same_bits(m, b, n)
 
+@pytest.mark.parametrize("over", [dict(expert_gating_func=f, norm_topk_prob=n, routed_scaling_factor=r) for f in (1, 2, 3, 4) for n, r in ((False, 2.5), (True, 1.0), (True, 2.5))],
+                         ids=lambda o: "-".join(str(v) for v in o.values()))
+def test_bits_of_every_gating(gpu, monkeypatch, over):
+  """Softmax, sigmoid, softmax of the picked and sqrt softplus, weights normed and scaled or not; every expert's router row is there twice, so picks are ties."""
+  from tinygrad_amd import llm
+  from tinygrad_amd.llm import Transformer, TransformerConfig, synth_state_moe
+  c = TransformerConfig(max_context=192, **dict(CONFIGS["512x256"], num_experts=24, num_experts_per_tok=5, **over))
+  sd = synth_state_moe(c, seed=41)
+  for i in range(c.num_blocks):
+    r = sd[f"blk.{i}.ffn_gate_inp.weight"][0].view(0, (24, c.dim), np.float16)
+    w = r.numpy(); w[1::2] = w[::2]; r.copyin(w)
+  a, b = Transformer(c, sd, max_new=8), Transformer(c, sd, max_new=8)
+  prompt = np.random.default_rng(41).integers(0, BASE["vocab_size"], size=150).tolist()
+  a.prefill(prompt)
+  assert a._chunker._rows16_ws is not None and a._chunker.x is None
+  monkeypatch.setattr(llm, "ROWS16_MIN", 1 << 30)
+  b.prefill(prompt)
+  _same_bits(a, b, 150)
+
 @pytest.mark.parametrize("name", list(CONFIGS))
 def test_bits_with_norm_weights_of_any_value(gpu, monkeypatch, name):
   """Norm weights that are no powers of two (the synthetic models' are 1): a normalised value is rounded where the steps of sixteen, eight and four rows round it."""
