@@ -76,6 +76,36 @@ def test_wide_tiles_of_q4_0(gpu, m, n, k, epi):
   if epi == 2: refs = [refs[0] / (1 + np.exp(-refs[0])) * refs[1]]
   for o, ref in zip(outs, refs): assert ol.rel_err(o.numpy(), ref + r if epi == 1 else ref) <= (2e-4 if epi == 2 else 5e-5)
 
+@pytest.mark.parametrize("t", [2, 12], ids=["Q4_0", "Q4_K"])
+@pytest.mark.parametrize("m,n,k,epi", [(385, (16400,), 1280, 0), (513, (12304,), 1536, 0), (1023, (4112,), 2816, 1), (1025, (4096, 1040, 2064), 1280, 0), (641, (7184,), 1280, 2), (300, (4096,), 14336, 1), (2047, (6160,), 3072, 0)],
+                         ids=["one-row", "ragged", "split", "three", "swiglu", "split-eight", "rounds"])
+def test_tall_tiles(gpu, t, m, n, k, epi):
+  """The 512 x 128 tiles: last tiles of 1, 44 and 127 rows and of 16 and 32 outputs, five to fourteen steps a workgroup, odd and even, matrices that meet inside a tile, K split into unequal parts, float32 and fp16 results.
+  Weights that begin four bytes behind a sixteen-byte line take the other tiles: the same fp16 weights in another order of sums, float32 sums of K products differ by about sqrt(K) 2^-24 of their absolute sum, 5e-5
+  of the largest result at most.  So do those of the reference for Q4_0; for Q4_K, whose weights round differently now and then, the bar is that of test_many_rows_linear_at_tile_edges."""
+  from tinygrad_amd import runtime as rt
+  rng = np.random.default_rng(m + t)
+  ws = rt.Buffer((64 << 20,), np.uint8)
+  ns = n * 2 if epi == 2 else n
+  parts = [_weight(rng, rt, t, i, k) for i in ns]
+  x = synth.activations(rng, m, k, np.float16); xb = rt.Buffer.from_numpy(x)
+  r = rng.standard_normal((m, n[0])).astype(np.float32)
+  refs = [x.astype(np.float32) @ p[1].T for p in parts]
+  if epi == 2: refs = [refs[0] / (1 + np.exp(-refs[0])) * refs[1]]
+  VP = ctypes.c_void_p * len(ns)
+  for dt, off in ((np.float32, 0), (np.float32, 4), (np.float16, 0)):
+    if epi == 1 and dt == np.float16: continue
+    bufs = [rt.Buffer.from_numpy(np.concatenate([np.zeros(off, np.uint8), p[0].reshape(-1).view(np.uint8)])) for p in parts]
+    outs = [rt.Buffer.from_numpy(r) if epi == 1 else rt.Buffer((m, i), dt) for i in n]
+    rt.check(rt.lib().tga_qlinear_many(t, len(ns), VP(*[b.ptr + off for b in bufs]), VP(*[(outs[i].ptr if i < len(outs) else None) for i in range(len(ns))]), (ctypes.c_int64 * len(ns))(*ns),
+                                       xb.ptr, rt.F32 if dt == np.float32 else rt.F16, m, k, epi, outs[0].ptr if epi == 1 else None, ws.ptr, ws.nbytes, None))
+    sums = 2e-4 if epi == 2 else 5e-5
+    got = [o.numpy().astype(np.float32) for o in outs]
+    if off == 0 and dt == np.float32: tall = got
+    for o, o2, ref in zip(got, tall, refs):
+      assert ol.rel_err(o, ref + r if epi == 1 else ref) <= ((4e-3 if epi == 2 else 1e-3) if t == 12 else sums) + (5e-4 if dt == np.float16 else 0)
+      assert ol.rel_err(o, o2) <= sums + (5e-4 if dt == np.float16 else 0)
+
 DENSE = dict(num_blocks=2, dim=512, hidden_dim=768, n_heads=8, n_kv_heads=2, norm_eps=1e-5, vocab_size=512, head_dim=64, rope_theta=500000.0)
 DENSE128 = dict(num_blocks=2, dim=768, hidden_dim=512, n_heads=6, n_kv_heads=6, norm_eps=1e-5, vocab_size=512, head_dim=128, rope_theta=10000.0)
 MOE = dict(num_blocks=2, dim=256, hidden_dim=256, n_heads=4, n_kv_heads=4, norm_eps=1e-5, vocab_size=512, head_dim=64, rope_theta=10000.0, qk_norm=256, num_experts=8, num_experts_per_tok=2)

@@ -180,3 +180,23 @@ def test_wide_tiles_keep_their_requests_in_flight():
   assert _wide_findings(good[:at - 1] + good[at:])                                  # (the wait gone)
   assert _wide_findings(good[:at - 1] + [("s_waitcnt vmcnt(3)", False)] + good[at - 1:])
   assert _wide_findings(good[:9] + [("scratch_load_dword v1, off, off", False)] + good[9:])
+
+def test_tall_tiles_wait_only_by_hand():
+  """qgemm_tall_kernel (csrc/qgemm_tall.hip): its loop over K holds no spill and no wait for vector memory but the four in front of its barriers, which leave fourteen or two younger requests under way."""
+  try: hipcc = tb._hipcc()
+  except RuntimeError: pytest.skip("hipcc not found")
+  with tempfile.TemporaryDirectory() as d:
+    out = pathlib.Path(d) / "tall.s"
+    r = subprocess.run([hipcc, *tb.HIPCC_FLAGS, "--cuda-device-only", "-S", str(tb.CSRC / "qgemm_tall.hip"), "-o", str(out)], capture_output=True, text=True)
+    if r.returncode != 0: pytest.fail(f"hipcc -S failed:\n{r.stderr[-2000:]}")
+    text = out.read_text()
+  names = re.findall(r"^(_Z17qgemm_tall_kernelI\w+):", text, re.M)
+  assert len(names) == 4, names
+  for name in names:
+    lines = [l.split(";")[0].strip() for l in text[text.index("\n" + name + ":"):text.index(".set " + name + ".uses_flat_scratch")].split("\n")]
+    at = {l[:-1]: i for i, l in enumerate(lines) if re.match(r"\.LBB\d+_\d+:$", l)}
+    loops = [lines[at[m.group(1)]:i] for i, l in enumerate(lines) if (m := re.match(r"s_cbranch\w+ (\.LBB\d+_\d+)$", l)) and at.get(m.group(1), i) < i]
+    loops = [x for x in loops if sum(t.startswith("v_mfma") for t in x) == 256]
+    assert len(loops) == 1, name
+    assert [t for t in loops[0] if "vmcnt" in t] == ["s_waitcnt vmcnt(14)"] * 2 + ["s_waitcnt vmcnt(2)"] * 2, name
+    assert not any(t.startswith("scratch_") for t in loops[0]) and sum(t == "s_barrier" for t in loops[0]) == 4 and sum(" lds" in t for t in loops[0]) == 20, name

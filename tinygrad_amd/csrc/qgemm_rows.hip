@@ -1,4 +1,4 @@
-// Entry points of the many-rows linears (kernel: qgemm_rows.h).
+// Entry points of the many-rows linears (kernels: qgemm_rows.h, qgemm_tall.hip).
 #include "qgemm_rows.h"
 
 #define X(F) int tga_rows_launch_##F(const RowsArgs& a, int tt, unsigned grid, hipStream_t s);
@@ -33,7 +33,10 @@ int64_t tga_rows_row_bytes(int fmt, int64_t K) {
   }
   return 0;
 }
+int tga_rows_tall(int fmt, const RowsArgs& a, unsigned grid, hipStream_t s);             // qgemm_tall.hip
+#define ROWS_TALL 512             // the tile height that asks for it
 int tga_rows_dispatch(int fmt, const RowsArgs& a, int tt, unsigned grid, hipStream_t s) {
+  if (tt == ROWS_TALL) return tga_rows_tall(fmt, a, grid, s);
   switch (fmt) {
 #define X(F) case F: return tga_rows_launch_##F(a, tt, grid, s);
     ROWS_FORMATS(X)
@@ -134,7 +137,7 @@ static bool rows_wide(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t 
   a.ks = rows_split(a, may_split, part_bytes, 512);
   return a.K / 256 / a.ks >= 12 && (long long)a.row_tiles * a.tok_tiles * a.ks >= 320;
 }
-static int rows_plan(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t part_bytes) {
+static int rows_plan_small(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t part_bytes) {
   if (rows_wide(a, fmt, swiglu, may_split, part_bytes)) return ROWS_WIDE;
   const int wt = swiglu ? ROWS_WT / 2 : ROWS_WT;
   a.row_tiles = (int)((a.ntot + wt - 1) / wt);
@@ -148,6 +151,53 @@ static int rows_plan(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t p
   a.tok_tiles = (a.M + tt - 1) / tt;
   a.ks = rows_split(a, may_split, part_bytes, 4 * ROWS_KS);
   return tt;
+}
+
+// The 512 x 128 tiles of qgemm_tall.hip (one workgroup per CU) against the plan above (two): the choice falls by the time either takes, us, as measured on products of K 1024 .. 14336, 64 .. 2047 rows and
+// 1024 .. 28672 outputs: a round of tall tiles 9 + 5.1 a step of 256, up to 6.3 where all CUs have one (the clock falls with the power), of 256 x 128 tiles 8 + 7.8, of 128 rows 6 + 2.1 a step of 128
+// (1.65 where CUs have only one workgroup), of 64 rows 5 + 1.25 (1.05); Q4_K a sixth more in tall tiles; a split of K writes its sums and reads them.  A last round that is nearly empty costs tall tiles more
+// than it costs small ones.  us, the plan above / tall tiles: Q4_0 4096 -> 2 x 14336 (SwiGLU), 300, 508, 640, 1023, 2047 rows 128 / 92, 131 / 106, 197 / 197 (not taken), 260 / 209, 488 / 448, Q4_K
+// 135 / 106, 148 / 120, 215 / 230 (not taken), 291 / 237, 606 / 511; Q4_0 14336 -> 4096, 300, 508, 1023, 2047 rows 69 / 61, 86 / 77, 142 / 124, 257 / 217; 4096 -> 6144 of 768, 1023, 2047 rows 77 / 60, 76 / 70,
+// 134 / 100; 4096 -> 4096 of 1023 rows 57 / 59 (not taken); 2048 -> 2 x 5632 of 1023 rows 65 / 53, of 640 43 / 52 (not taken); 3072 -> 2 x 8448 of 1280 rows,
+// two rounds two thirds full, 146 / 156 (not taken); 14336 -> 4096 of 150 rows 45 / 47 (not taken).
+static double rows_split_us(const RowsArgs& a) { return a.ks == 1 ? 0. : 2. + (double)a.ks * a.M * a.ntot * 8e-6 / 6.5; }
+static double rows_us(const RowsArgs& a, int tt) {
+  const long long wg = (long long)a.row_tiles * a.tok_tiles * a.ks;
+  const double steps = (double)a.K / ROWS_KS / a.ks;
+  if (tt == ROWS_WIDE) return (double)((wg + 511) / 512) * (8. + 3.9 * steps) + rows_split_us(a);
+  if (tt == 128) return (double)((wg + 511) / 512) * (6. + (wg > 256 ? 2.1 : 1.65) * steps) + rows_split_us(a);
+  return tt == 64 ? (double)((wg + 767) / 768) * (5. + (wg > 256 ? 1.25 : 1.05) * steps) + rows_split_us(a) : 0.;
+}
+static int rows_plan(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t part_bytes) {
+  const int tt = rows_plan_small(a, fmt, swiglu, may_split, part_bytes);
+  // (whole sub-tiles of sixteen rows, requests of sixteen bytes)
+  if ((fmt != F_Q4_0P && fmt != GGML_Q4_K) || tt == 32 || a.K % 256 || a.K > (1 << 20) || a.ntot >= (1ll << 30)) return tt;
+  for (int i = 0; i < (swiglu ? 2 : a.nseg); i++) if (a.n[i] % 16 || ((uintptr_t)a.w[i] & 15)) return tt;
+  RowsArgs t = a, best = a;
+  double us = rows_us(a, tt);
+  const int wt = swiglu ? ROWS_TALL / 2 : ROWS_TALL;
+  t.row_tiles = (int)((a.ntot + wt - 1) / wt); t.tok_tiles = (a.M + 127) / 128;
+  const int steps = a.K / 256;
+  const long long tiles = (long long)t.row_tiles * t.tok_tiles, per = (tiles + 7) / 8;       // (of the 32 CUs of an XCD)
+  bool taken = false;
+  for (int least = 5; least <= 7; least += 2) {
+    t.ks = 1;
+    if (may_split && per <= 32) {
+      t.ks = (int)(32 / per);
+      if (t.ks > steps / least) t.ks = steps / least;
+      while (t.ks > 1 && (size_t)t.ks * a.M * a.ntot * 4 > part_bytes) t.ks--;
+      if (t.ks < 1) t.ks = 1;
+    }
+    const long long rounds = (per * t.ks + 31) / 32;
+    const double full = (double)(tiles * t.ks) / (double)(256 * rounds);
+    if (full < (rounds == 1 ? 0.5 : 0.7)) continue;
+    const double step = (5.1 + (full > 0.6 ? 3. * (full - 0.6) : 0.)) * (fmt == GGML_Q4_K ? 1.16 : 1.);
+    const double e = (double)rounds * (9. + step * steps / t.ks) + rows_split_us(t);
+    if (e < us) { us = e; best = t; taken = true; }
+  }
+  if (!taken) return tt;
+  a = best;
+  return ROWS_TALL;
 }
 
 // tga_qlinear_many; norm_w != nullptr (one matrix, epilogue 1 in place, fp32): also xn = fp16 RMSNorm of the result's rows
