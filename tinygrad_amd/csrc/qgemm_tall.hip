@@ -6,7 +6,9 @@
 // there.  Weights and decode stay private to the wave, so no barrier concerns them: a wave decodes 64 rows straight into its A operands (lane (r16, g) of sub-tile i: row 16 i + r16, K position
 // group g), eight weights of each sub-tile per 32 products.  Eight waves share the activations: a ring of four quarter steps of 64 values, requested two quarters ahead, one barrier per quarter
 // in front of its last products, so that the first operands of the next quarter are read behind this one's.  Requests are inline assembly: the compiler would wait for all of them at every read of LDS;
-// the waits below are counted by hand and none of the compiler's own is in the loop.
+// the waits below are counted by hand and none of the compiler's own is in the loop.  Weights that come from HBM arrive later than the two quarters for which their requests are under way, so every wave
+// touches the lines of 32 of its rows two and three steps ahead (the workgroups of neighbouring activation tiles the other 32): weights not in the caches behind the L2s, gate / up of 508 / 1023 / 2047 rows
+// 127 -> 120, 235 -> 227, 471 -> 450 us.
 // 1023 rows: gate / up 270 -> 217 us, at 2048 rows 495 -> 436; the loop keeps the matrix pipe busy in 70 % of its cycles, at a clock that its power brings down to 1.8 GHz (2.2 in the kernel above).
 #include "qgemm_rows.h"
 
@@ -76,6 +78,10 @@ template <> struct TallFmt<GGML_Q4_K> {                 // low nibbles of 32 byt
 __device__ __forceinline__ void tall_request(u32x4 r, uint32_t dst, uint32_t off, int at) {
   asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(dst), "v"(off), "s"(r), "s"(at) : "memory");
 }
+// ... four bytes a lane: what brings a line nearer
+__device__ __forceinline__ void tall_touch(u32x4 r, uint32_t dst, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" :: "s"(dst), "v"(off), "s"(r) : "memory");
+}
 __device__ __forceinline__ u32x4 tall_desc(const void* p) {                             // (as wide_desc: nothing relies on its range check)
   const uint64_t v = (uint64_t)(uintptr_t)p;
   return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v), (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) & 0xFFFFu, 0xFFFFFFFFu, 0x00027000u};
@@ -86,7 +92,7 @@ __global__ __launch_bounds__(512, 1) void qgemm_tall_kernel(const RowsArgs a) {
   using WF = TallFmt<T>;
   constexpr int QB = TALL_TT * 128, SB = 16 * WF::CH, PC = WF::CH / 16, WB = 4 * SB;    // bytes: activations of a quarter, weights of a sub-tile; pieces of a row; bytes of a wave's weights
   static_assert(SB > 2048 && SB <= 3072 && 4 * QB >= 4 * 16384 && 8 * WB >= 4 * 16384, "three requests a sub-tile; 16 KB a wave for its results");
-  __shared__ __attribute__((aligned(16))) uint8_t lds[4 * QB + 8 * WB];                 // [four quarters: 128 rows of 64 values | eight waves: 64 rows of CH bytes]
+  __shared__ __attribute__((aligned(16))) uint8_t lds[4 * QB + 8 * WB + 256];           // [four quarters: 128 rows of 64 values | eight waves: 64 rows of CH bytes | what touches bring]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
   // ---- tile: as in qgemm_rows_kernel, the workgroups of an XCD take a contiguous run, activation tiles innermost
   const int nwg = a.row_tiles * a.tok_tiles, per = (nwg + 7) >> 3, b = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
@@ -94,14 +100,16 @@ __global__ __launch_bounds__(512, 1) void qgemm_tall_kernel(const RowsArgs a) {
   const int rt = b / a.tok_tiles, t0 = (b - rt * a.tok_tiles) * TALL_TT, cnt = min(a.M - t0, TALL_TT);
   const int nsteps = a.K / 256, s0 = (int)((long long)blockIdx.y * nsteps / a.ks), s1 = (int)((long long)(blockIdx.y + 1) * nsteps / a.ks);
   // ---- this wave's rows: sub-tiles of sixteen, each in one matrix (SwiGLU: they alternate gate / up, so partner values meet in one lane); those beyond the last repeat it, their results are dropped
-  u32x4 wr[4];
+  u32x4 wr[4], tr = {};
+  const int ti = SW ? b & 1 : (b & 1) * 2;                                              // (sub-tile from which on this workgroup's touches bring 32 rows)
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     int row0 = min(SW ? rt * (TALL_WT / 2) + wave * 32 + (i >> 1) * 16 : rt * TALL_WT + wave * 64 + i * 16, (int)a.ntot - 16);
-    const uint8_t* wb = a.w[0];
+    const uint8_t* wb = a.w[0]; int n = (int)a.n[0];
     if constexpr (SW) { if (i & 1) wb = a.w[1]; }
-    else if (a.nseg > 1 && row0 >= a.n[0]) { row0 -= (int)a.n[0]; wb = a.w[1]; if (a.nseg > 2 && row0 >= a.n[1]) { row0 -= (int)a.n[1]; wb = a.w[2]; } }
+    else if (a.nseg > 1 && row0 >= n) { row0 -= n; wb = a.w[1]; n = (int)a.n[1]; if (a.nseg > 2 && row0 >= n) { row0 -= n; wb = a.w[2]; n = (int)a.n[2]; } }
     wr[i] = tall_desc(wb + (size_t)row0 * a.row_bytes);
+    if (i == ti) { tr = wr[i]; tr.z = (uint32_t)min((long long)(n - row0) * a.row_bytes, 0xFFFFFFFFll); }      // (its range ends with the matrix: 32 rows may not)
   }
   // ---- weights: a sub-tile's 16 PC pieces by three requests, the last one from its end (pieces that two of them bring are the same bytes)
   const uint32_t lbase = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)lds, wbase = lbase + 4 * QB + wave * WB;
@@ -115,6 +123,11 @@ __global__ __launch_bounds__(512, 1) void qgemm_tall_kernel(const RowsArgs a) {
     const int k = n >> 2, i = n & 3;
     if (i == 0) woff = woffset(k);
     tall_request(wr[i], wbase + i * SB + (k < 2 ? 1024 * k : SB - 1024), woff, WF::CH * s);
+  };
+  auto touch = [&](int s) __attribute__((always_inline)) {
+    int l = lane; asm volatile("" : "+v"(l));
+    const uint32_t at = (uint32_t)min(WF::CH * (s & ~1), (int)a.row_bytes - 2 * WF::CH);
+    tall_touch(tr, lbase + 4 * QB + 8 * WB, __umul24((uint32_t)((l & 15) + 16 * (s & 1)), (uint32_t)a.row_bytes) + (uint32_t)min((l >> 4) * 96, 2 * WF::CH - 4) + at);
   };
   // ---- activations: quarter c of a step = values 64 g + 16 c .. + 15 of every group g; thread: slot tid & 7 of rows tid >> 3 and + 64; slot = piece ^ row, piece 4 e + g = values 64 g + 16 c + 8 e .. + 7
   const int xr = tid >> 3, piece = (tid & 7) ^ (xr & 7);
@@ -146,7 +159,8 @@ __global__ __launch_bounds__(512, 1) void qgemm_tall_kernel(const RowsArgs a) {
   for (int n = 0; n < 12; n++) wrequest(s0, n);
 #pragma unroll
   for (int c = 0; c < 3; c++) { xrequest(c, s0, 0); xrequest(c, s0, 1); }
-  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  touch((s0 + 1) & ~1); touch((s0 + 1) | 1);
+  asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
 #pragma unroll
   for (int i = 0; i < 4; i++) uread(i);
 #pragma unroll
@@ -157,18 +171,22 @@ __global__ __launch_bounds__(512, 1) void qgemm_tall_kernel(const RowsArgs a) {
     const int sn = min(s + 1, s1 - 1);                                                  // (behind the last step the requests repeat it; nothing reads what they bring)
     // 64 groups of four products, in this order.  With each: the activations of two groups further are read and four weights of the next eight of a sub-tile are decoded.  Requests: next step's weights
     // in the first quarter (its units are read in the last one, when each sub-tile's are used up), a quarter's activations at the end of the one three before it, behind a barrier that every wave
-    // reaches when it has used the quarter which they replace.
+    // reaches when it has used the quarter which they replace, and a touch last in the first quarter, so that only the last barrier's wait has it in front.
 #pragma unroll
     for (int c = 0; c < 4; c++) {
 #pragma unroll
       for (int n = 0; n < 16; n++) {
         const int v = 2 * c + (n >> 3), j = n & 7, m = 16 * c + n;
-        if (n == 12) {                                                                  // the next quarter's activations are there: behind them two or four requests for activations, and twelve for weights in between
-          if (c < 2) asm volatile("s_waitcnt vmcnt(14)\n\ts_barrier" ::: "memory"); else asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
+        if (n == 12) {                                                                  // the next quarter's activations are there; younger are the two requests of the quarter behind it, twelve for weights, a touch
+          if (c == 0) asm volatile("s_waitcnt vmcnt(14)\n\ts_barrier" ::: "memory");
+          else if (c == 1) asm volatile("s_waitcnt vmcnt(15)\n\ts_barrier" ::: "memory");
+          else if (c == 2) asm volatile("s_waitcnt vmcnt(3)\n\ts_barrier" ::: "memory");
+          else asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
         }
         x[(m + 2) % 3] = n < 14 ? xread(c, n + 2) : xread((c + 1) & 3, n - 14);
         if (c == 0 && n < 12) wrequest(sn, n);
         if (n >= 14) xrequest((c + 3) & 3, c == 0 ? s : sn, n - 14);
+        if (c == 0 && n == 15) touch(s + 3);
         if (v == 6 && j >= 2 && !(j & 1)) uread(j / 2 - 1);
         if (v == 7 && j == 0) uread(3);
         if (v < 7) decode(v + 1, j);
