@@ -1,9 +1,9 @@
 // A prefill step of any number of rows: the positions pos0 .. pos0 + P - 1 of one or more sequences go through all blocks together (the reference's chunked prefill,
 // tinygrad/llm/model.py:464, 476-481, with the prompt as one chunk), every linear as ONE pass over its weights (qgemm_rows.h).  Per block: q / k / v -> rotation +
-// append -> attention -> attn_output (+ residual, norm) -> gate / up + SwiGLU -> down (+ residual, the next block's norm): eight launches and the sums of a split q / k / v, or for a MoE block norm -> router logits -> gating ->
+// append -> attention -> attn_output (+ residual, norm) -> gate / up + SwiGLU -> down (+ residual, the next block's norm): eight launches, or for a MoE block norm -> router logits -> gating ->
 // grouping -> selected experts' gate / up + SwiGLU -> down -> weighted sum (+ residual), model.py:110-135.  The launches are issued by one native call.
-// MI355X, prompt to first logits: 8B-arch Q4_0 of 1024 tokens 42.4 ms (steps of 128 rows, qgemm64.hip) -> 21.2; OLMoE-arch of 512 tokens, where its user asks for it, 64.0 (steps of 16 rows, an
-// expert GEMV per token and slot) -> 5.0; four 8B-arch Q4_K_M sequences of 128 tokens 333 (one lockstep step per position) -> 15.5.
+// MI355X, prompt to first logits: 8B-arch Q4_0 of 1024 tokens 42.4 ms (steps of 128 rows, qgemm64.hip) -> 18.0; OLMoE-arch of 512 tokens, where its user asks for it, 64.0 (steps of 16 rows, an
+// expert GEMV per token and slot) -> 5.0; four 8B-arch Q4_K_M sequences of 128 tokens 333 (one lockstep step per position) -> 13.3.
 #include "qgemm_rows.h"
 #include "decode.h"
 #include "moe_gate.h"
@@ -13,38 +13,43 @@ int tga_rows_fmt(int ggml_type, int64_t K);                                     
 int64_t tga_rows_row_bytes(int fmt, int64_t K);
 int tga_rows_dispatch(int fmt, const RowsArgs& a, int tt, unsigned grid, hipStream_t s);
 int tga_rows_linear(int ggml_type, int nseg, const void* const* w, void* const* y, const int64_t* n, const void* x_f16, int y_dtype, int64_t M, int64_t K, int epilogue, const float* resid,
-                    void* workspace, int64_t workspace_bytes, const float* norm_w, float norm_eps, void* xn, void* stream);
+                    void* workspace, int64_t workspace_bytes, const float* norm_w, float norm_eps, void* xn, int* parts, void* stream);
 int tga_rows_norm(float* x, const float* w, int M, int n, float eps, void* xn, void* stream);
 
 // ------------------------------------------------------------------------------------------------ rotation + append
 // One workgroup per row.  q is rotated (after its norm) and leaves as TWO fp16 values per element, the rounded value and what the rounding left over, for matrix-core
 // scores of the float32 query (rows_attn_kernel); k is rotated into the cache, v copied.  The rotation is apply_rope's (model.py:29-33) written as one rounded product and one fused multiply-add,
 // like every kernel that rotates, so a cache row has the same bits whichever path appended it.  norm: 0 none, 1 RMSNorm over the whole q / k rows (model.py:169), 2 per head (:180).
+// Rows come as the linears leave them: whole (ks 1), or as the sums of a split K, plane values apart, which are completed here in their order (a launch of its own that writes and reads them again before:
+// 1023 rows of 4096 + 2 x 1024 values, two sums each, 12.6 + 10.3 -> 14.4 us a block; 508 rows, three and eight sums, 17 -> 8.9).
+struct RopeSrc { const float* p; size_t plane; int stride, ks; };
 struct RopeArgs {
-  const float* q; const float* k; const float* v; const float* qn; const float* kn; const float* rope;
+  RopeSrc q, k, v; const float* qn; const float* kn; const float* rope;
   uint16_t* qh; uint16_t* ql; uint16_t* ck; uint16_t* cv; int* zero;      // zero: n_zero counters cleared for the launches behind this one
   int H, KV, hd, max_ctx, P, pos0, norm, n_zero; float eps;
 };
-__global__ __launch_bounds__(256) void rows_rope_kernel(const RopeArgs a) {
+__global__ __launch_bounds__(512) void rows_rope_kernel(const RopeArgs a) {
   __shared__ float red[8];
   const int r = blockIdx.x, z = r / a.P, pos = a.pos0 + r % a.P, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = a.hd >> 1;
   const int nq = a.H * a.hd, nk = a.KV * a.hd;
-  if (r == 0) for (int i = tid; i < a.n_zero; i += 256) a.zero[i] = 0;
-  const float* q = a.q + (size_t)r * nq; const float* k = a.k + (size_t)r * nk; const float* v = a.v + (size_t)r * nk;
+  if (r == 0) for (int i = tid; i < a.n_zero; i += 512) a.zero[i] = 0;
+  const float* q = a.q.p + (size_t)r * a.q.stride; const float* k = a.k.p + (size_t)r * a.k.stride; const float* v = a.v.p + (size_t)r * a.v.stride;
   const size_t crow = ((size_t)z * a.KV * a.max_ctx + pos) * a.hd, cstep = (size_t)a.max_ctx * a.hd;
 #pragma unroll 2
-  for (int e = 4 * tid; e < nk; e += 1024) {
+  for (int e = 4 * tid; e < nk; e += 2048) {
     const int hh = e / a.hd;
-    const f32x4 x = *(const f32x4*)(v + e);
+    f32x4 x = *(const f32x4*)(v + e);
+#pragma unroll 4
+    for (int p = 1; p < a.v.ks; p++) { const f32x4 y = *(const f32x4*)(v + p * a.v.plane + e); x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w; }
     *(u32x2*)(a.cv + crow + hh * cstep + (e - hh * a.hd)) = u32x2{f2h_bits(x.x) | (f2h_bits(x.y) << 16), f2h_bits(x.z) | (f2h_bits(x.w) << 16)};
   }
   float qs = 1.f, ks = 1.f;
   if (a.norm == 1) {
     float s0 = 0.f, s1 = 0.f;
-    for (int i = tid; i < (nq >> 2); i += 256) { const f32x4 x = ((const f32x4*)q)[i]; s0 += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w; }
-    for (int i = tid; i < (nk >> 2); i += 256) { const f32x4 x = ((const f32x4*)k)[i]; s1 += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w; }
+    for (int i = tid & 255; wave < 4 && i < (nq >> 2); i += 256) { const f32x4 x = ((const f32x4*)q)[i]; s0 += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w; }
+    for (int i = tid & 255; wave < 4 && i < (nk >> 2); i += 256) { const f32x4 x = ((const f32x4*)k)[i]; s1 += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w; }
     s0 = wave_sum(s0); s1 = wave_sum(s1);
-    if (lane == 0) { red[wave] = s0; red[4 + wave] = s1; }
+    if (lane == 0 && wave < 4) { red[wave] = s0; red[4 + wave] = s1; }
     __syncthreads();
     qs = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)nq + a.eps);
     ks = 1.0f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)nk + a.eps);
@@ -53,20 +58,28 @@ __global__ __launch_bounds__(256) void rows_rope_kernel(const RopeArgs a) {
   const bool live = lane < half;                                          // (half is 32 or 64)
   const int i = live ? lane : half - 1;
   const float c = rr[i], s = rr[half + i];
-  // (a wave's heads in groups of RU, whose values are requested together: a head at a time, the ten heads of a wave are ten trips to memory)
+  // (a wave's heads in groups of RU, whose values are requested together: a head at a time, each is a trip to memory)
   constexpr int RU = 5;
   const int nh = a.H + a.KV;
-  for (int h0 = wave; h0 < nh; h0 += 4 * RU) {
+  for (int h0 = wave; h0 < nh; h0 += 8 * RU) {
     float xa[RU], xb[RU];
 #pragma unroll
     for (int u = 0; u < RU; u++) {
-      const int h = min(h0 + 4 * u, nh - 1);
+      const int h = min(h0 + 8 * u, nh - 1);
       const float* src = h < a.H ? q + h * a.hd : k + (h - a.H) * a.hd;
       xa[u] = src[i]; xb[u] = src[half + i];
     }
+#pragma unroll 3
+    for (int p = 1; p < a.q.ks; p++)                                      // (q and k are of one launch where they are split)
+#pragma unroll
+      for (int u = 0; u < RU; u++) {
+        const int h = min(h0 + 8 * u, nh - 1);
+        const float* src = (h < a.H ? q + h * a.hd : k + (h - a.H) * a.hd) + p * a.q.plane;
+        xa[u] += src[i]; xb[u] += src[half + i];
+      }
 #pragma unroll
     for (int u = 0; u < RU; u++) {
-      const int h = h0 + 4 * u;
+      const int h = h0 + 8 * u;
       if (h >= nh) break;
       const bool isq = h < a.H;
       const int hh = isq ? h : h - a.H;
@@ -99,12 +112,13 @@ __global__ __launch_bounds__(256) void rows_rope_kernel(const RopeArgs a) {
 // S^T = K Q^T: keys as A operand from LDS (rows of head_dim values, 16-byte pieces XORed with the key), the rotated queries as two fp16 B operands held in registers.
 // O^T = V^T P^T: the probabilities likewise as a rounded value and its remainder (each product once more on matrix cores that are far from busy here); the eight keys a lane holds after the first product are taken as they are, and V is written to LDS transposed with its keys in that order, two keys
 // per dword, pieces XORed with the dimension.  The next tile is fetched while this one is multiplied.  flattened workgroup = (kv head, sequence) innermost: with eight
-// kv heads all readers of a head's rows run on one XCD and share its L2; the longest row tiles come first.
+// kv heads all readers of a head's rows run on one XCD and share its L2; the longest row tiles come first, in runs of as many tiles as give every CU a workgroup (cus), every second run
+// the other way round: the workgroups that share a CU have long and short tiles (1023 rows, 32 heads, two workgroups a CU: 41.4 -> 39.5 us).
 // Two fp16 values hold 22 bits and more of a query or probability, and sums are formed in few additions at their full size (remainders first, two chains per score, a tile's products from
 // zero).  Share of fp16 results that are not the rounded float64 attention, 64 and 1024 positions, heads of 64 and 128, scores of standard deviation 0.03 .. 5: 1.8e-4 .. 2.2e-3; the float32
 // kernel of eight rows and fewer: 2.4e-4 .. 2.4e-3.  (Queries beyond 65504 have no such pair, as keys beyond have no cache row.)
 #define PSCALE 32768.0f             // of probabilities on their way to two fp16 values (the remainder of 0.2 is a subnormal number already: the absolute step 2^-24)
-struct RowsAttnArgs { const uint16_t* qh; const uint16_t* ql; const uint16_t* ck; const uint16_t* cv; uint16_t* out; int H, KV, max_ctx, P, pos0, nseq, qtiles; float scale; };
+struct RowsAttnArgs { const uint16_t* qh; const uint16_t* ql; const uint16_t* ck; const uint16_t* cv; uint16_t* out; int H, KV, max_ctx, P, pos0, nseq, qtiles, cus; float scale; };
 
 template <int HD>
 __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
@@ -115,7 +129,7 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
   const int group = a.H / a.KV, kz = a.KV * a.nseq;
   int b = blockIdx.x;
   const int kvz = b % kz; b /= kz;
-  const int hh = b % group, qt = a.qtiles - 1 - b / group;
+  const int hh = b % group, rank = b / group, part = rank / a.cus, qt = a.qtiles - 1 - ((part & 1) ? min((part + 1) * a.cus, a.qtiles) - 1 - (rank - part * a.cus) : rank);
   const int kvh = kvz % a.KV, z = kvz / a.KV, head = kvh * group + hh;
   const int row_first = qt * 64, nq = a.H * HD;
   const int wrow = row_first + wave * 16;                                 // first row of this wave
@@ -358,7 +372,7 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
   // x += in . W^T, and xn = the norm that follows (norm nullptr: nothing follows)
   auto linear_norm = [&](int type, int64_t wp, const void* in, int64_t K, const float* norm) {
     const void* wt[1] = {(const void*)wp}; void* y[1] = {x}; const int64_t n[1] = {dim};
-    return tga_rows_linear(type, 1, wt, y, n, in, TGA_F32, R, K, 1, x, ws + w.part, (int64_t)PF_PART, norm, eps, xn, stream);
+    return tga_rows_linear(type, 1, wt, y, n, in, TGA_F32, R, K, 1, x, ws + w.part, (int64_t)PF_PART, norm, eps, xn, nullptr, stream);
   };
   PF_DO(tga_embed_rows((const void*)m[PM_EMB], (int)m[PM_EMB_TYPE], (int)dim, tokens, (int)R, state, x, stream));
   for (int64_t bi = 0; bi < m[PM_NBLOCKS]; bi++) {
@@ -368,26 +382,34 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
     else if (bi == 0) PF_DO(tga_rows_norm(x, (const float*)b[PB_ATTN_NORM], (int)R, (int)dim, eps, xn, stream));      // (later ones come behind the block before)
     const void* wt[3] = {(const void*)b[PB_WQ], (const void*)b[PB_WK], (const void*)b[PB_WV]};
     void* y[3] = {q, kk, v}; const int64_t n[3] = {nq, nk, nk};
+    RopeArgs ra;
+    ra.norm = !b[PB_QN] ? 0 : m[PM_QKNORM] == hd ? 2 : 1;
+    RopeSrc* const src[3] = {&ra.q, &ra.k, &ra.v};
+    int64_t used = 0;
     for (int i = 0; i < 3;) {                                             // one launch per run of equal block types
-      int j = i + 1;
+      int j = i + 1, ks = 1;
       while (j < 3 && b[PB_TQ + j] == b[PB_TQ + i]) j++;
-      PF_DO(linear((int)b[PB_TQ + i], j - i, wt + i, y + i, n + i, xn, TGA_F32, dim, 0, nullptr));
+      int64_t run = 0, at = 0;
+      for (int l = i; l < j; l++) run += n[l];
+      // (the rotation completes the sums itself where q and k are of one launch, and needs no norm over whole rows first)
+      const bool leave = ra.norm != 1 && (i == 2 || (i == 0 && j >= 2));
+      PF_DO(tga_rows_linear((int)b[PB_TQ + i], j - i, wt + i, y + i, n + i, xn, TGA_F32, R, dim, 0, nullptr, ws + w.part + used, (int64_t)PF_PART - used, nullptr, 0.f, nullptr, leave ? &ks : nullptr, stream));
+      for (int l = i; l < j; at += n[l++]) *src[l] = ks > 1 ? RopeSrc{(const float*)(ws + w.part + used) + at, (size_t)(R * run), (int)run, ks} : RopeSrc{(const float*)y[l], 0, (int)n[l], 1};
+      if (ks > 1) used += (ks * R * run * 4 + 255) & ~(int64_t)255;
       i = j;
     }
-    RopeArgs ra;
-    ra.q = q; ra.k = kk; ra.v = v; ra.qn = (const float*)b[PB_QN]; ra.kn = (const float*)b[PB_KN]; ra.rope = (const float*)m[PM_ROPE];
+    ra.qn = (const float*)b[PB_QN]; ra.kn = (const float*)b[PB_KN]; ra.rope = (const float*)m[PM_ROPE];
     ra.qh = (uint16_t*)(ws + w.qh); ra.ql = (uint16_t*)(ws + w.ql); ra.ck = (uint16_t*)b[PB_CK]; ra.cv = (uint16_t*)b[PB_CV];
     ra.zero = b[PB_MOE] ? (int*)(ws + w.counts) : nullptr; ra.n_zero = b[PB_MOE] ? (int)E : 0;
     ra.H = (int)H; ra.KV = (int)KV; ra.hd = (int)hd; ra.max_ctx = (int)m[PM_MAXCTX]; ra.P = (int)P; ra.pos0 = (int)pos0; ra.eps = eps;
-    ra.norm = !b[PB_QN] ? 0 : m[PM_QKNORM] == hd ? 2 : 1;
-    rows_rope_kernel<<<(unsigned)R, 256, 0, s>>>(ra);
+    rows_rope_kernel<<<(unsigned)R, 512, 0, s>>>(ra);
     TGA_LAUNCH_CHECK();
     // The last block's keys and values are in the cache, and the first logits come from the decode step behind the prompt: its rows go no further (8B-arch, 1024 tokens: 0.5 ms of 21).  A model of one
     // block takes the whole step: its workspace is where single blocks are compared with the reference
     if (bi > 0 && bi + 1 == m[PM_NBLOCKS]) break;
     RowsAttnArgs aa;
     aa.qh = ra.qh; aa.ql = ra.ql; aa.ck = ra.ck; aa.cv = ra.cv; aa.out = attn; aa.H = (int)H; aa.KV = (int)KV; aa.max_ctx = ra.max_ctx; aa.P = (int)P; aa.pos0 = (int)pos0; aa.nseq = (int)nseq;
-    aa.qtiles = (int)((P + 63) / 64); aa.scale = (float)(1.4426950408889634 / sqrt((double)hd));
+    aa.qtiles = (int)((P + 63) / 64); aa.cus = (int)(H * nseq < 256 ? 256 / (H * nseq) : 1); aa.scale = (float)(1.4426950408889634 / sqrt((double)hd));
     const unsigned ag = (unsigned)(aa.qtiles * H * nseq);
     if (hd == 64) rows_attn_kernel<64><<<ag, 256, 0, s>>>(aa); else rows_attn_kernel<128><<<ag, 256, 0, s>>>(aa);
     TGA_LAUNCH_CHECK();

@@ -200,9 +200,10 @@ static int rows_plan(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t p
   return ROWS_TALL;
 }
 
-// tga_qlinear_many; norm_w != nullptr (one matrix, epilogue 1 in place, fp32): also xn = fp16 RMSNorm of the result's rows
+// tga_qlinear_many; norm_w != nullptr (one matrix, epilogue 1 in place, fp32): also xn = fp16 RMSNorm of the result's rows; parts != nullptr (epilogue 0): the sums of a split K stay in the workspace,
+// [parts][M][outputs of all matrices], for the caller to complete in their order (parts 1: they are in y)
 int tga_rows_linear(int ggml_type, int nseg, const void* const* w, void* const* y, const int64_t* n, const void* x_f16, int y_dtype, int64_t M, int64_t K, int epilogue, const float* resid,
-                    void* workspace, int64_t workspace_bytes, const float* norm_w, float norm_eps, void* xn, void* stream) {
+                    void* workspace, int64_t workspace_bytes, const float* norm_w, float norm_eps, void* xn, int* parts, void* stream) {
   TGA_REQUIRE(w && y && n && x_f16 && nseg >= 1 && nseg <= 3, "tga_qlinear_many: null pointer or %d matrices", nseg);
   TGA_REQUIRE(epilogue >= 0 && epilogue <= 2 && (epilogue != 2 || nseg == 2) && (epilogue != 1 || (nseg == 1 && resid)), "tga_qlinear_many: epilogue %d with %d matrices", epilogue, nseg);
   TGA_REQUIRE(y_dtype == TGA_F32 || y_dtype == TGA_F16, "tga_qlinear_many: y_dtype must be TGA_F16 or TGA_F32");
@@ -229,6 +230,7 @@ int tga_rows_linear(int ggml_type, int nseg, const void* const* w, void* const* 
   if (const int rc = tga_rows_dispatch(fmt, a, tt, grid, (hipStream_t)stream)) return rc;
   const bool norm_here = norm_w && a.ntot <= ROWS_NORM_MAX && a.ntot % 4 == 0;
   if (norm_here) return rows_norm(a.part, a.ks, (float*)y[0], norm_w, (int)M, (int)a.ntot, norm_eps, xn, (hipStream_t)stream);
+  if (parts) { *parts = a.ks; return 0; }
   if (a.ks > 1) {
     a.epi = epilogue;
     const long long total = M * (a.ntot / 4), wg = (total + 255) / 256;
@@ -247,7 +249,7 @@ extern "C" {
 
 int tga_qlinear_many(int ggml_type, int nseg, const void* const* w, void* const* y, const int64_t* n, const void* x_f16, int y_dtype, int64_t M, int64_t K, int epilogue,
                      const float* resid, void* workspace, int64_t workspace_bytes, void* stream) {
-  return tga_rows_linear(ggml_type, nseg, w, y, n, x_f16, y_dtype, M, K, epilogue, resid, workspace, workspace_bytes, nullptr, 0.f, nullptr, stream);
+  return tga_rows_linear(ggml_type, nseg, w, y, n, x_f16, y_dtype, M, K, epilogue, resid, workspace, workspace_bytes, nullptr, 0.f, nullptr, nullptr, stream);
 }
 
 }  // extern "C"
