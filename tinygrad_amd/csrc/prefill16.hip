@@ -328,7 +328,7 @@ __global__ __launch_bounds__(HD) void x16_merge_kernel(const X16Attn a) {
 
 // ------------------------------------------------------------------------------------------------ ffn_norm and router logits
 // The arithmetic of moe_router_kernel, RT rows per workgroup: normalised once, the router's rows read once for all of them.  The normalised rows leave as the experts read them: the sixteen pairs
-// (value j, value j + 16) of a unit of 32 behind each other.
+// (value j, value j + 16) of a unit of 32 behind each other, those of j = g, g + 4, g + 8, g + 12 as a piece of sixteen bytes.
 struct X16Router { const float* x; const float* nw; const uint16_t* wr; uint16_t* xs; float* logits; int R, dim, E; float eps; };
 // Bound by the latency of the router's rows, which come from the L2s: sixteen waves share them, four of which form the norm (512 rows, 64 experts of 2048 values: 17.6 -> 9.1 us with sixteen waves instead of four).
 template <int RT>
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(1024) void x16_router_kernel(const X16Router a) {
   for (int t = 0; t < RT; t++)
     if (r0 + t < a.R)
       for (int d = tid; d < (a.dim >> 1); d += 1024) {
-        const int e = 32 * (d >> 4) + (d & 15);
+        const int e = 32 * (d >> 4) + 4 * (d & 3) + ((d >> 2) & 3);
         const uint32_t lo = xn[t][e], hi = xn[t][e + 16];
         ((uint32_t*)(a.xs + (size_t)(r0 + t) * a.dim))[d] = lo | (hi << 16);
       }
@@ -438,17 +438,35 @@ __global__ __launch_bounds__(64 * NS, 2) void x16_expert_kernel(const X16Expert 
   int t = s0 - it.tf * a.ngroups;
   it.grp = t / it.nt; t -= it.grp * it.nt;
   nx = item_behind(it);
-  uint32_t raw[34];
+  // this wave's eight units of the item's 64 columns: cw[u][t] holds, of column c of block t, the bytes g, g + 4, g + 8, g + 12 (g = blk) of unit u's sixteen - the weights of the four products that this
+  // lane's group of a matrix product takes -; sc the scale bytes of this lane's own column
+  uint32_t cw[8][4], sc[2];
   auto weights_of = [&](const Item& i) __attribute__((always_inline)) {
     const int col = SW ? i.grp * 32 + (blk & 1) * 16 + c : i.grp * 64 + lane;
     return (SW && blk >= 2 ? a.w[1] : a.w[0]) + i.e * a.estride + (long long)col * a.row_bytes + 136 * wave;      // (4-byte aligned: K is a multiple of 256)
   };
   auto load = [&](const Item& i) __attribute__((always_inline)) {
     const uint8_t* p = weights_of(i);
+    uint32_t raw[34];
 #pragma unroll
     for (int q = 0; q < 8; q++) { const u32x4 v = ld16(p + 16 * q); raw[4 * q] = v.x; raw[4 * q + 1] = v.y; raw[4 * q + 2] = v.z; raw[4 * q + 3] = v.w; }
     u32x2 v; __builtin_memcpy(&v, p + 128, 8); raw[32] = v.x; raw[33] = v.y;
     __builtin_amdgcn_s_waitcnt(0x0f70);                                    // (vmcnt 0: what is counted behind it are requests into LDS and stores)
+    // a lane's own column, bytes transposed within the unit, then across the four lanes that share c
+    sc[0] = sc[1] = 0;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int o = 17 * u;
+      sc[u >> 2] |= ((raw[o >> 2] >> (8 * (o & 3))) & 0xffu) << (8 * (u & 3));
+      uint32_t d[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) { const int at = o + 1 + 4 * q; d[q] = (at & 3) ? __builtin_amdgcn_alignbit(raw[(at >> 2) + 1], raw[at >> 2], 8 * (at & 3)) : raw[at >> 2]; }
+      const uint32_t e0 = __builtin_amdgcn_perm(d[1], d[0], 0x05010400u), e1 = __builtin_amdgcn_perm(d[1], d[0], 0x07030602u), e2 = __builtin_amdgcn_perm(d[3], d[2], 0x05010400u), e3 = __builtin_amdgcn_perm(d[3], d[2], 0x07030602u);
+      const uint32_t t0 = __builtin_amdgcn_perm(e2, e0, 0x05040100u), t1 = __builtin_amdgcn_perm(e2, e0, 0x07060302u), t2 = __builtin_amdgcn_perm(e3, e1, 0x05040100u), t3 = __builtin_amdgcn_perm(e3, e1, 0x07060302u);
+      const auto h02 = __builtin_amdgcn_permlane32_swap(t0, t2, false, false), h13 = __builtin_amdgcn_permlane32_swap(t1, t3, false, false);
+      const auto a01 = __builtin_amdgcn_permlane16_swap(h02[0], h13[0], false, false), a23 = __builtin_amdgcn_permlane16_swap(h02[1], h13[1], false, false);
+      cw[u][0] = a01[0]; cw[u][1] = a01[1]; cw[u][2] = a23[0]; cw[u][3] = a23[1];
+    }
   };
   load(it);
   uint8_t* rw = ring + wave * (3 * X16_RUN);
@@ -469,17 +487,18 @@ __global__ __launch_bounds__(64 * NS, 2) void x16_expert_kernel(const X16Expert 
   };
   point(it, t);
   request(0, 0); request(1, 1);
-  u32x4 x[2][4];
-  auto read_x = [&](u32x4 (&d)[4], int slot, int u) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) d[q] = *(const u32x4*)(ring + (((uint32_t)(wave * 3 + slot) * X16_RUN + c * 272) ^ (64 * u + 16 * q)));      // (c * 256 + 16 c: the low eight bits are the row's)
+  u32x4 x[2];
+  auto read_x = [&](u32x4& d, int slot, int u) __attribute__((always_inline)) {
+    d = *(const u32x4*)(ring + (((uint32_t)(wave * 3 + slot) * X16_RUN + c * 272) ^ (64 * u + 16 * blk)));      // (c * 256 + 16 c: the low eight bits are the row's)
   };
   asm volatile("s_waitcnt vmcnt(4)" ::: "memory");                        // run 0 has landed
   read_x(x[0], 0, 0);
-  // operands with their zero in place: pairs of even and of odd products
-  u32x2 we[2] = {u32x2{0u, 0u}, u32x2{0u, 0u}}, wo[2] = {u32x2{0u, 0u}, u32x2{0u, 0u}};
+  // weight operands with their zeros in place: pair i of a lane's four, for two blocks
+  u32x4 wz[2][4];
 #pragma unroll
-  for (int i = 0; i < 2; i++) asm volatile("" : "+v"(we[i]), "+v"(wo[i]));
+  for (int z = 0; z < 2; z++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) { wz[z][i] = u32x4{0u, 0u, 0u, 0u}; asm volatile("" : "+v"(wz[z][i])); }
   int slot = 0;
   bool fresh = true;                                                       // the first tile on these weights: the next item's are touched
   for (;;) {
@@ -502,27 +521,24 @@ __global__ __launch_bounds__(64 * NS, 2) void x16_expert_kernel(const X16Expert 
         if (fresh) asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
         read_x(x[(u + 1) & 1], nslot, 0);
       } else read_x(x[(u + 1) & 1], slot, (u & 3) + 1);
-      constexpr int o = 17 * u;
 #pragma unroll
-      for (int i = o / 4; i <= (o + 16) / 4; i++) asm volatile("" : "+v"(raw[i]));      // (decoded here and anew for every tile: decoded ahead, they do not fit the registers)
-      auto dword_at = [&](int b) __attribute__((always_inline)) { return (b & 3) ? __builtin_amdgcn_alignbit(raw[(b >> 2) + 1], raw[b >> 2], 8 * (b & 3)) : raw[b >> 2]; };
-      const uint32_t eb = (raw[o >> 2] >> (8 * (o & 3))) & 0xffu;
+      for (int i = 0; i < 4; i++) asm volatile("" : "+v"(cw[u][i]));       // (decoded here and anew for every tile: decoded ahead, they do not fit the registers)
+      asm volatile("" : "+v"(sc[u >> 2]));
+      const uint32_t eb = (sc[u >> 2] >> (8 * (u & 3))) & 0xffu;
       const uint32_t s02 = eb ? (eb << 23) : 0x00400000u;
-      v16f32 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      v4f32 acc[4];
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const uint32_t w = dword_at(o + 1 + 4 * q);
-        const u32x2 xl = {x[u & 1][q].x, x[u & 1][q].y}, xh = {x[u & 1][q].z, x[u & 1][q].w};
-        we[0].x = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0));
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xl), __builtin_bit_cast(v4f16, we[0]), acc, 0, 0, 0);
-        wo[0].y = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1));
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xl), __builtin_bit_cast(v4f16, wo[0]), acc, 0, 0, 0);
-        we[1].x = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2));
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xh), __builtin_bit_cast(v4f16, we[1]), acc, 0, 0, 0);
-        wo[1].y = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3));
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4f16, xh), __builtin_bit_cast(v4f16, wo[1]), acc, 0, 0, 0);
-        asm volatile("" : "+v"(we[0]), "+v"(wo[0]), "+v"(we[1]), "+v"(wo[1]));     // (their other halves are no constants to the compiler, which set them anew for every product)
-      }
+      for (int b = 0; b < 4; b++) acc[b] = v4f32{0.f, 0.f, 0.f, 0.f};
+      auto product = [&](auto i_) __attribute__((always_inline)) {         // four dot2 of every chain: those of pairs 4 i .. 4 i + 3
+        constexpr int i = decltype(i_)::value;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+          wz[b & 1][i][i] = as_u32(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(cw[u][b], 1.0f, i));
+          acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8f16, x[u & 1]), __builtin_bit_cast(v8f16, wz[b & 1][i]), acc[b], 0, 0, 0);
+          asm volatile("" : "+v"(wz[b & 1][i]));                           // (its other pairs are no constants to the compiler, which set them anew for every product)
+        }
+      };
+      x16_each(product, std::make_integer_sequence<int, 4>{});
       // the scales of the four blocks' column c
       const auto h = __builtin_amdgcn_permlane32_swap(s02, s02, false, false);
       const auto l0 = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false), l1 = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
@@ -530,7 +546,7 @@ __global__ __launch_bounds__(64 * NS, 2) void x16_expert_kernel(const X16Expert 
       const float sb[4] = {__builtin_bit_cast(float, su[0]), __builtin_bit_cast(float, su[1]), __builtin_bit_cast(float, su[2]), __builtin_bit_cast(float, su[3])};
 #pragma unroll
       for (int i = 0; i < 16; i++) {
-        float v = __builtin_fmaf(sb[i >> 2], acc[i], 0.f);
+        float v = __builtin_fmaf(sb[i >> 2], acc[i >> 2][i & 3], 0.f);
         if constexpr (u & 1) { v = st[0][i] + v; if constexpr (u & 2) { v = st[1][i] + v; if constexpr (u & 4) leaf[i] = st[2][i] + v; else st[2][i] = v; } else st[1][i] = v; }
         else st[0][i] = v;
       }
@@ -556,7 +572,7 @@ __global__ __launch_bounds__(64 * NS, 2) void x16_expert_kernel(const X16Expert 
       if constexpr (SW) {
         float v = silu_f(s[0]) * s[1];
         asm volatile("" : "+v"(v));                                       // (rounded to float32 first, as there)
-        ((uint16_t*)a.y)[(size_t)(it.first + row) * a.N + it.grp * 32 + 2 * cc + h] = (uint16_t)f2h_bits(v);
+        ((uint16_t*)a.y)[(size_t)(it.first + row) * a.N + it.grp * 32 + 8 * (cc & 3) + 2 * (cc >> 2) + h] = (uint16_t)f2h_bits(v);
       } else {
         float* y = (float*)a.y + (size_t)(it.first + row) * a.N + it.grp * 64 + cc;
         y[16 * h] = s[0]; y[16 * (h + 2)] = s[1];
