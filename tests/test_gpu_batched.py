@@ -177,3 +177,31 @@ def test_batched_glm4moe_like_decode(gpu, B, gate):
   model = BatchedTransformer(c, sd, B, max_new=32)
   assert [b["moe"] for b in model.blk] == [False, True, True]
   _per_sequence_check(gpu, model, cfg, host, prompts, 16, 128)
+
+@pytest.mark.parametrize("hd,kv,group,norm", [(64, 4, 1, 0), (64, 2, 8, 2), (128, 8, 4, 0), (128, 4, 2, 1), (128, 2, 5, 2), (64, 72, 1, 1)])
+def test_attention_of_few_splits_has_the_bits_of_two_launches(gpu, hd, kv, group, norm):
+  """Caches of one to four splits are one launch, of five the split launch and the merge: the same positions, the same bits of every output and cache row.  Positions at the splits' edges, groups that
+  are no multiple of four heads, every norm; (72 heads of five sequences are more workgroups than CUs: two launches either way)."""
+  rt, B = gpu, 5
+  rng = np.random.default_rng(hd + kv + group)
+  H, f32 = kv * group, np.float32
+  q, k, v = (rng.standard_normal((B, n * hd)).astype(f32) for n in (H, kv, kv))
+  qn, kn = (1 + 0.1 * rng.standard_normal((hd if norm == 2 else n * hd)).astype(f32) for n in (H, kv))
+  rope = rng.standard_normal((320, hd)).astype(f32)
+  ck, cv = (rng.standard_normal((B, kv, 320, hd)).astype(np.float16) for _ in range(2))
+  bufs = [rt.Buffer.from_numpy(a) for a in (q, k, v, qn, kn, rope)]
+  def run(ctx, pos):
+    kb, vb = (rt.Buffer.from_numpy(np.ascontiguousarray(c[:, :, :ctx])) for c in (ck, cv))
+    part = rt.Buffer((B * H * 5 * (hd + 2),), f32).zero_()
+    st = np.zeros(16, np.int32); st[0] = pos
+    state, o16, o32 = rt.Buffer.from_numpy(st), rt.Buffer((B, H * hd), np.float16), rt.Buffer((B, H * hd), f32)
+    rt.check(rt.lib().tga_attention_decode_batched(B, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, bufs[3].ptr if norm else None, bufs[4].ptr if norm else None, 1e-5, int(norm == 2), kb.ptr, vb.ptr, part.ptr,
+                                                   state.ptr, H, kv, hd, ctx, bufs[5].ptr, o16.ptr, o32.ptr, None))
+    return o16.numpy(), o32.numpy(), kb.numpy(), vb.numpy(), state.numpy()
+  for ctx in (64, 128, 192, 256):
+    for pos in sorted({0, 1, 63, 64, ctx - 65, ctx - 64, ctx - 1} & set(range(ctx))):
+      a, b = run(ctx, pos), run(320, pos)
+      assert a[0].tobytes() == b[0].tobytes() and a[1].tobytes() == b[1].tobytes(), (ctx, pos)
+      for x, y in zip(a[2:4], b[2:4]): assert x.tobytes() == np.ascontiguousarray(y[:, :, :ctx]).tobytes(), (ctx, pos)
+      assert not a[4][4]
+  assert run(128, 128)[4][4] == 2                                            # a position behind the cache is refused

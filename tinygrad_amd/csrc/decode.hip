@@ -205,19 +205,26 @@ __device__ __forceinline__ void block_sumsq2(const float* q, int nq, const float
 // scalar load in flight meanwhile, and only the rotation row waits for it.  NORM selects the q/k RMSNorm at compile time so that no
 // load sits behind a branch (a join makes the compiler wait for every outstanding load):
 //   0 none, 1 over the whole q and k vectors of at most 4096 values each (read in one batch), 2 per head, 3 over whole vectors of any length
-template <int HD8, int NORM>
-__global__ __launch_bounds__(256) void attn_decode_kernel(const AttnArgs args) {
+// FEW: a cache of at most ATTN_FEW splits (decode): four waves per split in one workgroup, which merges them in LDS with the arithmetic of attn_merge_kernel instead of leaving them to that launch (8B-arch
+// lockstep step of eight sequences, 128 positions of cache: 6.0 + 4.6 -> 7.6 us a block, the same bits).  Waves of splits behind the position take part and are left out of the merge.
+#define ATTN_FEW 4
+template <int HD8, int NORM, bool FEW>
+__global__ __launch_bounds__(FEW ? 256 * ATTN_FEW : 256) void attn_decode_kernel(const AttnArgs args) {
   const AttnArgs a = attn_args_of_sequence(args, blockIdx.z);   // field reads become kernel-argument loads in the entry block
   const int zrow = blockIdx.z * a.pos_step;
   constexpr int HD = HD8 * 8, RPI = 64 / HD8, NVI = 16 / RPI, NGRP = 4 * RPI, CSTR = HD + 4;
   constexpr int QPL = (HD / 2 + 63) / 64;               // query pairs per lane
-  const int kvh = blockIdx.x, split = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int NS = FEW ? ATTN_FEW : 1;
+  const int part = FEW ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  const int kvh = blockIdx.x, split = FEW ? part : blockIdx.y;
+  const int tid = FEW ? threadIdx.x & 255 : threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int half = HD >> 1, group = a.n_heads / a.n_kv;
-  __shared__ float qs[4][HD];                           // rotated queries of the 4 heads in flight
-  __shared__ float ks[HD], vs[HD];                      // rotated key / value of this token
-  __shared__ float comb[4 * NGRP * CSTR];               // [head in flight][run]: o[HD], m, l
-  __shared__ float red[8];
+  __shared__ float qs_[NS][4][HD];                      // rotated queries of the 4 heads in flight
+  __shared__ float ks_[NS][HD], vs_[NS][HD];            // rotated key / value of this token
+  __shared__ float comb_[NS][4 * NGRP * CSTR];          // [head in flight][run]: o[HD], m, l
+  __shared__ float red_[NS][8];
+  __shared__ float sums[FEW ? NS : 1][FEW ? 4 : 1][FEW ? HD + 2 : 1];      // FEW: the splits' partials of the 4 heads
+  float (&qs)[4][HD] = qs_[part]; float (&ks)[HD] = ks_[part]; float (&vs)[HD] = vs_[part]; float (&comb)[4 * NGRP * CSTR] = comb_[part]; float (&red)[8] = red_[part];
   const int vr = lane / HD8, vp = lane % HD8;
   const int p0 = split * 64 + wave * 16;                // first position of this wave
   // ---- loads that do not depend on the position
@@ -268,7 +275,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnArgs args) {
     if (kvh == 0 && split == 0 && tid == 0) atomicOr(&a.st->error, 2);
     return;
   }
-  if (split * 64 > pos) return;                         // nothing cached in this split yet
+  if (!FEW && split * 64 > pos) return;                 // nothing cached in this split yet
   const float kc = a.rope[(size_t)pos * HD + ki], ksn = a.rope[(size_t)pos * HD + half + ki];
   float qc[QPL], qsn[QPL];
 #pragma unroll
@@ -368,7 +375,9 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnArgs args) {
           float t = qq[0] * (float)k0.x; t += qq[1] * (float)k0.y; t += qq[2] * (float)k1.x; t += qq[3] * (float)k1.y;
           t += qq[4] * (float)k2.x; t += qq[5] * (float)k2.y; t += qq[6] * (float)k3.x; t += qq[7] * (float)k3.y;
           t = run_sum<HD8>(t);
-          sc[i] = (p0 + i * RPI + vr <= pos) ? t * a.scale : -INFINITY;
+          t *= a.scale;
+          if constexpr (FEW) asm volatile("" : "+v"(t));  // (a rounded score, as in the other variant: folded with the subtraction below it is not, and a lone position's weight is not 1)
+          sc[i] = (p0 + i * RPI + vr <= pos) ? t : -INFINITY;
           m = fmaxf(m, sc[i]);
         }
         // softmax partial of this lane run (rows i * RPI + vr of the wave): no cross-lane traffic, the fold below sums the runs
@@ -406,12 +415,36 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnArgs args) {
 #pragma unroll
         for (int j = 0; j < HD / 64; j++) od[j] += wg * cb[g * CSTR + lane + 64 * j];
       }
-      float* po = a.part + ((size_t)head * a.nsplit + split) * (HD + 2);
+      float* po = FEW ? sums[part][wave] : a.part + ((size_t)head * a.nsplit + split) * (HD + 2);
 #pragma unroll
       for (int j = 0; j < HD / 64; j++) po[lane + 64 * j] = od[j];
       if (lane == 0) { po[HD] = m; po[HD + 1] = l; }
     }
     __syncthreads();
+    if constexpr (FEW) {                                // (a rounded product and an addition where that kernel has them: o and l in its order)
+      const int ns = (pos >> 6) + 1;
+      for (int t = threadIdx.x; t < 4 * HD; t += blockDim.x) {
+        const int hh = t / HD, d = t % HD;
+        if (h0 + hh >= group) continue;
+        float m = sums[0][hh][HD], w[NS], l[NS], o = 0.f;
+#pragma unroll
+        for (int j = 1; j < NS; j++) if (j < ns) m = fmaxf(m, sums[j][hh][HD]);
+#pragma unroll
+        for (int j = 0; j < NS; j++) {
+          w[j] = j < ns ? __expf(sums[j][hh][HD] - m) : 0.f;
+          l[j] = j < ns ? sums[j][hh][HD + 1] * w[j] : 0.f;
+          float v = j < ns ? sums[j][hh][d] * w[j] : 0.f;
+          asm volatile("" : "+v"(l[j]), "+v"(v));
+          o += v;
+        }
+        static_assert(NS == 4 || !FEW, "the tree of a wave's sum");
+        o *= 1.0f / ((l[0] + l[1]) + (l[2] + l[3]));
+        const int e = (kvh * group + h0 + hh) * HD + d;
+        if (a.out16) a.out16[a.stage_fmt ? staged_pos(a.stage_fmt, e, a.stage_nu) : e] = (_Float16)o;
+        if (a.out32) a.out32[e] = o;
+      }
+      __syncthreads();
+    }
   }
 }
 
@@ -1050,8 +1083,12 @@ static int attention_launch(int chunk, int batch, const float* q, const float* k
   hipStream_t s = (hipStream_t)stream;
   const int norm = !q_norm_weight ? 0 : norm_per_head ? 2 : ((long long)n_heads * head_dim <= 4096 && (long long)n_kv_heads * head_dim <= 4096) ? 1 : 3;
 #define TGA_ATTN_LAUNCH(HD8) do { \
-    if (norm == 0) attn_decode_kernel<HD8, 0><<<grid, 256, 0, s>>>(a); else if (norm == 1) attn_decode_kernel<HD8, 1><<<grid, 256, 0, s>>>(a); \
-    else if (norm == 2) attn_decode_kernel<HD8, 2><<<grid, 256, 0, s>>>(a); else attn_decode_kernel<HD8, 3><<<grid, 256, 0, s>>>(a); } while (0)
+    if constexpr (HD8 <= 16) { if (few) { TGA_ATTN_NORM(HD8, true, 256 * a.nsplit); break; } } \
+    TGA_ATTN_NORM(HD8, false, 256); } while (0)
+#define TGA_ATTN_NORM(HD8, FEW, NT) do { \
+    if (norm == 0) attn_decode_kernel<HD8, 0, FEW><<<grid, NT, 0, s>>>(a); else if (norm == 1) attn_decode_kernel<HD8, 1, FEW><<<grid, NT, 0, s>>>(a); \
+    else if (norm == 2) attn_decode_kernel<HD8, 2, FEW><<<grid, NT, 0, s>>>(a); else attn_decode_kernel<HD8, 3, FEW><<<grid, NT, 0, s>>>(a); } while (0)
+  const bool few = !chunk && a.nsplit <= ATTN_FEW && head_dim <= 128 && n_kv_heads * batch <= 256;      // one launch merges its own splits (larger heads: four do not fit LDS; one workgroup fits a CU)
   static const bool chunk_mfma_off = getenv("TGA_ATTN_CHUNK") && !strcmp(getenv("TGA_ATTN_CHUNK"), "rows");
   const bool chunk_mfma = chunk && batch > 8 && norm == 0 && (head_dim == 64 || head_dim == 128) && n_heads / n_kv_heads <= 8 && !chunk_mfma_off;   // chunks of more than eight rows attend on the matrix cores
   for (int pass = chunk ? 1 : 0; pass <= (chunk ? 2 : 0); pass++) {   // chunked prefill: append every row, then attend from the cache
@@ -1073,13 +1110,15 @@ static int attention_launch(int chunk, int batch, const float* q, const float* k
       TGA_LAUNCH_CHECK();
       break;
     }
-    grid = dim3(n_kv_heads, pass == 1 ? 1 : a.nsplit, batch);
+    grid = dim3(n_kv_heads, pass == 1 || few ? 1 : a.nsplit, batch);
     if (head_dim == 64) TGA_ATTN_LAUNCH(8);
     else if (head_dim == 128) TGA_ATTN_LAUNCH(16);
     else TGA_ATTN_LAUNCH(32);
     TGA_LAUNCH_CHECK();
   }
 #undef TGA_ATTN_LAUNCH
+#undef TGA_ATTN_NORM
+  if (few) return 0;
   const dim3 mgrid(n_heads, batch);
   if (head_dim == 64) attn_merge_kernel<64><<<mgrid, 64, 0, s>>>(a);
   else if (head_dim == 128) attn_merge_kernel<128><<<mgrid, 128, 0, s>>>(a);
