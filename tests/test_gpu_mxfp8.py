@@ -344,3 +344,22 @@ def test_moe_feed_forward_has_the_bits_of_the_single_steps(gpu, case):
   got, ref = moe.moe_feed_forward(*args).numpy(), _single_steps(moe, *args)
   assert case != "tiny" or (ref & 0x7FFF).any()
   np.testing.assert_array_equal(got, ref)
+
+@pytest.mark.parametrize("T,E", [(70, 16), (900, 4)])
+def test_moe_feed_forward_of_values_that_are_not_finite(gpu, T, E):
+  """A row of infinities, one with a NaN and a NaN bias of one gate column (the largest magnitude of a block and its 32 results pass between lanes in registers): in low tiles and in full ones of
+  128 rows, NaN where the single steps give NaN and their bits elsewhere."""
+  from tinygrad_amd import moe
+  D, I, k = 512, 256, 2
+  rng = np.random.default_rng(T)
+  B = gpu.Buffer.from_numpy
+  x = rng.standard_normal((T, D)).astype(np.float32)
+  x[3] = np.inf; x[17, 5] = np.nan
+  wgu, wdn = (rng.standard_normal((E, 2 * I, D)) * D ** -0.5).astype(np.float32), (rng.standard_normal((E, D, I)) * I ** -0.5).astype(np.float32)
+  bgu, bdn = (rng.standard_normal((E, 2 * I)) * 0.1).astype(np.float32), (rng.standard_normal((E, D)) * 0.1).astype(np.float32)
+  bgu[1, 70] = np.nan
+  args = (B(moe.to_bf16_bits(x)), B(rng.standard_normal((T, E)).astype(np.float32)), k, tuple(map(B, omx.quantize_mxfp8(wgu))), B(bgu), tuple(map(B, omx.quantize_mxfp8(wdn))), B(bdn))
+  got, ref = moe.moe_feed_forward(*args).numpy(), _single_steps(moe, *args)
+  nan = lambda b: (b & 0x7FFF) > 0x7F80
+  np.testing.assert_array_equal(nan(got), nan(ref))
+  np.testing.assert_array_equal(np.where(nan(got), 0, got), np.where(nan(ref), 0, ref))

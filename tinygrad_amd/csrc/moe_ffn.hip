@@ -184,17 +184,27 @@ __device__ __forceinline__ float min_q(float a, float b) { float o; asm("v_min_f
 __device__ __forceinline__ float max_q(float a, float b) { float o; asm("v_max_f32 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b)); return o; }
 __device__ __forceinline__ float max3_abs(float m, float a, float b) { float o; asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(o) : "v"(m), "v"(a), "v"(b)); return o; }
 
-// The result of a tile: lane = row r16 of sub-tile WM i + wm, columns 4 kg .. 4 kg + 3 of n sub-tile j.  slab: 16 rows of 144 bytes of LDS that are this wave's; b: the bias of its 64 columns.
+__device__ __forceinline__ float lanes_max(float v) {                     // over lanes l, l ^ 16, l ^ 32, l ^ 48; no signalling NaN
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t m = __builtin_bit_cast(uint32_t, max_q(__builtin_bit_cast(float, (uint32_t)h[0]), __builtin_bit_cast(float, (uint32_t)h[1])));
+  const auto l = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+  return max_q(__builtin_bit_cast(float, (uint32_t)l[0]), __builtin_bit_cast(float, (uint32_t)l[1]));
+}
+
+// The result of a tile: lane = row r16 of sub-tile WM i + wm, columns 4 kg .. 4 kg + 3 of n sub-tile j. b: the bias of its 64 columns.
+// The four lanes of a row exchange their results in registers (a pass through LDS, with a barrier in front of it and a wait for the requests in flight that the compiler puts before its stores, and the
+// bias rounded by integer code: 84 + 45.5 us of the first size below, now 82.7 + 45.2).
 template <int RS, int WM, int BN, bool UP>
-__device__ __forceinline__ void ffn_epilogue(const FfnArgs& a, const FfnCur& c, const v4f32 (&acc)[RS][4], int nsub, int wm, int wn, uint8_t* slab, const float* b) {
+__device__ __forceinline__ void ffn_epilogue(const FfnArgs& a, const FfnCur& c, const v4f32 (&acc)[RS][4], int nsub, int wm, int wn, const float* b) {
   const int lane = threadIdx.x & 63, r16 = lane & 15, kg = lane >> 4, row0 = c.row0;
   const float limit = __builtin_canonicalizef(a.limit);
   f32x4 bias[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     bias[j] = *(const f32x4*)(b + 16 * j + 4 * kg);
-#pragma unroll
-    for (int i = 0; i < 4; i++) bias[j][i] = bf16_to_f(f_to_bf16(bias[j][i]));
+    const uint32_t b01 = pack_bf16x2(bias[j][0], bias[j][1]), b23 = pack_bf16x2(bias[j][2], bias[j][3]);
+    bias[j] = f32x4{bf16_lo(b01), bf16_hi(b01), bf16_lo(b23), bf16_hi(b23)};
   }
 #pragma unroll
   for (int i = 0; i < RS; i++) {
@@ -216,33 +226,33 @@ __device__ __forceinline__ void ffn_epilogue(const FfnArgs& a, const FfnCur& c, 
         y[2 * j] = bf16_lo(o); y[2 * j + 1] = bf16_hi(o);
         amax = max3_abs(amax, y[2 * j], y[2 * j + 1]);
       }
-      amax = fmaxf(amax, __shfl_xor(amax, 16)); amax = fmaxf(amax, __shfl_xor(amax, 32));     // the wave's 64 columns are one block of 32 results
+      amax = lanes_max(amax);     // the wave's 64 columns are one block of 32 results
       const int e = mx_e8(amax);
       const float sc = mx_scale(e);
-#pragma unroll
-      for (int j = 0; j < 4; j++) *(uint16_t*)(slab + r16 * 40 + 8 * j + 2 * kg) = (uint16_t)e4m3x2(y[2 * j] * sc, y[2 * j + 1] * sc);
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      const u32x2 o = *(const u32x2*)(slab + r16 * 40 + 8 * kg);
+      // two bytes of each of four n sub-tiles a lane -> the eight of n sub-tile kg: the rows' four lanes change places
+      const auto h = __builtin_amdgcn_permlane32_swap(e4m3x4(y[0] * sc, y[1] * sc, y[2] * sc, y[3] * sc), e4m3x4(y[4] * sc, y[5] * sc, y[6] * sc, y[7] * sc), false, false);
+      const auto l = __builtin_amdgcn_permlane16_swap(__builtin_amdgcn_perm(h[1], h[0], 0x05040100u), __builtin_amdgcn_perm(h[1], h[0], 0x07060302u), false, false);
+      const u32x2 o = {__builtin_amdgcn_perm(l[1], l[0], 0x05040100u), __builtin_amdgcn_perm(l[1], l[0], 0x07060302u)};
       if (r0 + r16 < c.valid) {
         const size_t row = (size_t)(row0 + r0 + r16);
         *(u32x2*)(a.yq + row * a.I + c.tn * (BN / 2) + wn * 32 + 8 * kg) = o;
         if (kg == 0) a.ye8[row * (a.I / 32) + c.tn * (BN / 64) + wn] = (uint8_t)e;
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     } else {
+      u32x2 o[4];
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const uint32_t h01 = pack_bf16x2(acc[i][j][0], acc[i][j][1]), h23 = pack_bf16x2(acc[i][j][2], acc[i][j][3]);
-        *(u32x2*)(slab + r16 * 144 + 32 * j + 8 * kg) = u32x2{pack_bf16x2(bf16_lo(h01) + bias[j][0], bf16_hi(h01) + bias[j][1]), pack_bf16x2(bf16_lo(h23) + bias[j][2], bf16_hi(h23) + bias[j][3])};
+        o[j] = u32x2{pack_bf16x2(bf16_lo(h01) + bias[j][0], bf16_hi(h01) + bias[j][1]), pack_bf16x2(bf16_lo(h23) + bias[j][2], bf16_hi(h23) + bias[j][3])};
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      const int rr = lane >> 3, rc = lane & 7;
+      uint16_t* to = (uint16_t*)a.z + (size_t)(row0 + r0 + r16) * a.D + c.tn * BN + wn * 64 + 16 * (kg & 1) + 4 * (kg & 2);
+      u32x4 q[2];
 #pragma unroll
-      for (int p = 0; p < 2; p++) {
-        const u32x4 o = *(const u32x4*)(slab + (rr + 8 * p) * 144 + 16 * rc);
-        if (r0 + rr + 8 * p < c.valid) *(u32x4*)(a.z + (size_t)(row0 + r0 + rr + 8 * p) * a.D + c.tn * BN + wn * 64 + 8 * rc) = o;
+      for (int p = 0; p < 2; p++) {                                      // an even lane group: eight columns of sub-tile 2 p, its own and the next group's; an odd one: of 2 p + 1
+        const auto x = __builtin_amdgcn_permlane16_swap(o[2 * p].x, o[2 * p + 1].x, false, false), y = __builtin_amdgcn_permlane16_swap(o[2 * p].y, o[2 * p + 1].y, false, false);
+        q[p] = u32x4{x[0], y[0], x[1], y[1]};
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (r0 + r16 < c.valid) { *(u32x4*)to = q[0]; *(u32x4*)(to + 32) = q[1]; }
     }
   }
 }
@@ -368,10 +378,8 @@ __device__ __forceinline__ void ffn_tall(const FfnArgs& a, uint8_t* smem, int* s
       store_s(st2);
       __syncthreads();
     }
-    // the stage the last step was read from is idle: wave-private slabs
-    ffn_epilogue<RS, WM, BN, UP>(a, cur, acc, nsub, wm, wn, smem + ((par + nsteps - 1) & 1) * STAGE + wave * 2304, a.bias[UP ? 0 : 1] + (size_t)cur.e * N + cur.tn * BN + wn * 64);
+    ffn_epilogue<RS, WM, BN, UP>(a, cur, acc, nsub, wm, wn, a.bias[UP ? 0 : 1] + (size_t)cur.e * N + cur.tn * BN + wn * 64);
     if (!more) break;
-    __syncthreads();                                                      // the slabs are free before any wave's next step writes that stage
     par = (par + nsteps) & 1; cur = nxt; t = tnext; which ^= 1;
   }
 }
@@ -383,9 +391,13 @@ __device__ __forceinline__ void ffn_tall(const FfnArgs& a, uint8_t* smem, int* s
 // A step's region: rows of 128 bytes, 16-byte chunk c of row R at chunk c ^ (R & 7) (a request covers eight whole rows, a read of sixteen rows meets each bank group once
 // per eight lanes).  Scales come four steps at a time, sixteen bytes a row: a dword a row and step was 64 cache lines a request, a fifth of the time.  Rows beyond the expert's repeat its last one.
 // UP: gate/up (rows gathered by token, epilogue bias + clamped interleaved SwiGLU + quantisation) or down (compact rows, epilogue bias).  ONCE: weights requested past the caches.
-// Measured (us, gate/up + down): 16000 rows of 64 experts skewed, D 2048, I 512, tiles of 128: 97.5 + 52.7 (tiles of 256 through registers) -> 79 + 42; 256 rows of 64 experts, I 768, tiles of 16:
-// 42.1 + 23.3 -> 35.8 + 20.2, past the caches 31.5 + 19.1: 5.2 TB/s of weights.  What bounds the first: a step is 1.4 us of which 0.45 are products (eight waves read 128 KB of LDS, then multiply, in one phase;
-// two groups of waves half a step apart with a barrier each half: 77 + 44, not kept), the epilogue's 400 vector instructions per sub-tile 6 us a tile, and 2.4 rounds of tiles on 256 CUs.
+// In full tiles of 128 rows the requests of a step go out between its products (in front of them 82.7 -> 80.0 + 44.8), and the scales' position in the row's sixteen bytes is a selector of the
+// byte permutation, not a branch per row (sixteen branches every four steps: -> 76.6 + 44.0).
+// Measured (us, gate/up + down): 16000 rows of 64 experts skewed, D 2048, I 512, tiles of 128: 97.5 + 52.7 (tiles of 256 through registers) -> 76.6 + 44.0; 256 rows of 64 experts, I 768, tiles of 16:
+// 42.1 + 23.3 -> 35.8 + 20.2, past the caches 31.5 + 19.1: 5.2 TB/s of weights.  What bounds the first: of 77 us, requests alone are 45 (14 TB/s out of L2), products and reads alone 44, the launch
+// itself 10, the epilogue 11 (down: 11 of 44, most of it the 64 MB it writes); what overlaps is what the two waves of a SIMD leave each other.  Not kept: two groups of waves half a step apart with a
+// barrier each half (77 + 44 where one was 79 + 42), the next step's weights read into registers while this one is multiplied (81 + 46.5), a last round of half tiles (78.4 + 44.6), tiles of 128 x 128
+// by four waves, two a CU (115).
 __device__ __forceinline__ const uint8_t* scalar_ptr(const uint8_t* p) {
   const uint64_t v = (uint64_t)(uintptr_t)p;
   uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
@@ -399,7 +411,8 @@ __global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a)
   constexpr int NW = WM * WN, BN = 64 * WN, RS = BM / 16 / WM;          // waves, weight rows of a tile, 16-row sub-tiles of a wave
   constexpr int IA = BM / 8 / NW, IB = BN / 8 / NW, SI = (BM + BN + 63) / 64, IS = (SI + NW - 1) / NW, NI = IA + IB;   // requests of a wave: eight rows of operands a step, 64 rows' scales of four steps
   constexpr int STAGE = (BM + BN) * 128;
-  static_assert(IA * 8 * NW == BM && IB * 8 * NW == BN && RS >= 1 && (NB == 2 || NB == 3) && STAGE >= NW * 2304, "tile shape");
+  constexpr bool SPREAD = RS == 4;                                       // a full tile's requests between its products
+  static_assert(IA * 8 * NW == BM && IB * 8 * NW == BN && RS >= 1 && (NB == 2 || NB == 3), "tile shape");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];        // NB steps, the scales of up to four steps, the experts' first rows and tiles
   __shared__ __attribute__((aligned(16))) float s_bias[2][BN];          // of the tile multiplied and the one requested
   __shared__ __attribute__((aligned(16))) int s_ids[UP ? NW : 1][UP ? 8 * IA + 64 * IS : 1];   // tokens of the rows this wave requests: operands, scales (its own: no barrier between their arrival and their use)
@@ -484,21 +497,27 @@ __global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a)
     }
   };
   // a step of the tile that is requested; q >= 0: the scales from that step on in front of it
-  auto request = [&](int q) __attribute__((always_inline)) {
+  auto request_front = [&](int q) __attribute__((always_inline)) {
     if (rs_ == 0) begin();
     if (q >= 0) request_scales(q);
     uint8_t* st = smem + rslot * STAGE;
 #pragma unroll
     for (int i = 0; i < IA; i++) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)pa[i], (__attribute__((address_space(3))) void*)(st + (wave * IA + i) * 1024), 16, 0, 0);
+  };
+  auto request_b = [&](int from, int to) __attribute__((always_inline)) {
+    uint8_t* st = smem + rslot * STAGE;
 #pragma unroll
-    for (int i = 0; i < IB; i++)                                         // (scalar base + the lane's offset: no vector address arithmetic)
+    for (int i = from; i < to; i++)                                      // (scalar base + the lane's offset: no vector address arithmetic)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(scalar_ptr(pb) + boff_lane[i]), (__attribute__((address_space(3))) void*)(st + BM * 128 + (wave * IB + i) * 1024), 16, 0, ONCE ? 2 : 0);
+  };
+  auto request_end = [&]() __attribute__((always_inline)) {
     pb += 128;
 #pragma unroll
     for (int i = 0; i < IA; i++) pa[i] += 128;
     rslot = rslot + 1 == NB ? 0 : rslot + 1;
     if (++rs_ == nsteps) { rs_ = 0; rt_ += step_wg; }
   };
+  auto request = [&](int q) __attribute__((always_inline)) { request_front(q); request_b(0, IB); request_end(); };
 
   FfnCur cur;
   find(t, cur);
@@ -529,20 +548,39 @@ __global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a)
       asm volatile("s_barrier" ::: "memory");
       // Into the position of the step before, which every wave has read; the scales of the next four steps once every wave has those of this group (read at its first step)
       const int p4 = s & ~3, len = min(4, nsteps - p4), q = p4 + len;
-      if (left >= NB - 1) request(s - p4 != max(1, len - (NB - 1)) ? -1 : q < nsteps ? q : t + step_wg < last ? 0 : -1);
+      const bool req = left >= NB - 1;
+      const int rq = s - p4 != max(1, len - (NB - 1)) ? -1 : q < nsteps ? q : t + step_wg < last ? 0 : -1;
+      const bool spread = SPREAD && nsub == RS;
+      if (req && !spread) request(rq);
       st = smem + slot * STAGE;
       slot = slot + 1 == NB ? 0 : slot + 1;
       if (s == p4) {
-        auto bytes = [&](int row) __attribute__((always_inline)) {       // byte i: the scale of step s + i of this lane's block
-          u32x4 d;
-          if (KB == 8) d = u32x4{((const uint32_t*)scales)[row], ((const uint32_t*)scales)[BM + BN + row], 0u, 0u}; else d = *(const u32x4*)(scales + row * 16);
-          const uint32_t lo = __builtin_amdgcn_perm(d.y, d.x, pick), hi = __builtin_amdgcn_perm(d.w, d.z, pick);
-          return KB != 8 && len == 2 ? hi : lo | (hi << 16);
-        };
+        // byte i: the scale of step s + i of this lane's block
+        if (KB == 8) {
+          const uint32_t* b8 = (const uint32_t*)scales + (BM + wn * 64 + r16); const uint32_t* a8 = (const uint32_t*)scales + (16 * wm + r16);
 #pragma unroll
-        for (int j = 0; j < 4; j++) scb[j] = bytes(BM + wn * 64 + 16 * j + r16);
+          for (int j = 0; j < 4; j++) scb[j] = __builtin_amdgcn_perm(b8[BM + BN + 16 * j], b8[16 * j], pick);
 #pragma unroll
-        for (int i = 0; i < RS; i++) sca[i] = bytes(16 * (WM * i + wm) + r16);
+          for (int i = 0; i < RS; i++) sca[i] = __builtin_amdgcn_perm(a8[BM + BN + 16 * WM * i], a8[16 * WM * i], pick);
+        } else {
+          const uint32_t halves = len == 2 ? 0x0C0C0504u : 0x05040100u;  // (the last two steps of a row lie behind the two before them)
+          auto bytes = [&](const u32x4& d) __attribute__((always_inline)) { return __builtin_amdgcn_perm(__builtin_amdgcn_perm(d.w, d.z, pick), __builtin_amdgcn_perm(d.y, d.x, pick), halves); };
+          // (by inline assembly, their wait with them: in front of plain reads the compiler would wait for all requests in flight)
+          const uint32_t at_b = (uint32_t)(uintptr_t)scales + (uint32_t)(BM + wn * 64 + r16) * 16u, at_a = (uint32_t)(uintptr_t)scales + (uint32_t)(16 * wm + r16) * 16u;
+          u32x4 d0, d1, d2, d3;
+          asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:256\n\tds_read_b128 %2, %4 offset:512\n\tds_read_b128 %3, %4 offset:768\n\ts_waitcnt lgkmcnt(0)" : "=&v"(d0), "=&v"(d1), "=&v"(d2), "=&v"(d3) : "v"(at_b) : "memory");
+          scb[0] = bytes(d0); scb[1] = bytes(d1); scb[2] = bytes(d2); scb[3] = bytes(d3);
+          if constexpr (RS == 1) {
+            asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(d0) : "v"(at_a) : "memory");
+            sca[0] = bytes(d0);
+          } else {
+#pragma unroll
+            for (int i = 0; i < RS; i += 2) {
+              asm volatile("ds_read_b128 %0, %2 offset:%3\n\tds_read_b128 %1, %2 offset:%4\n\ts_waitcnt lgkmcnt(0)" : "=&v"(d0), "=&v"(d1) : "v"(at_a), "n"(256 * WM * i), "n"(256 * WM * (i + 1)) : "memory");
+              sca[i] = bytes(d0); sca[(i + 1) % RS] = bytes(d1);
+            }
+          }
+        }
       }
       const uint8_t* As = st; const uint8_t* Bs = st + BM * 128 + wn * 4 * 2048;
       auto multiply = [&](auto full_tag) __attribute__((always_inline)) {
@@ -566,6 +604,9 @@ __global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a)
           if (FULL || i < nsub) {
 #pragma unroll
             for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[j], af[i & 1], acc[i][j], 0, 0, 0, (int)scb[j], 0, (int)sca[i]);
+            if constexpr (FULL && SPREAD) {
+              if (req) { if (i == 0) request_front(rq); else if (i == 1) request_b(0, IB / 2); else if (i == 2) { request_b(IB / 2, IB); request_end(); } }
+            }
           }
         }
       };
@@ -576,11 +617,8 @@ __global__ __launch_bounds__(64 * WM * WN) void ffn_gemm_kernel(const FfnArgs a)
       for (int i = 0; i < RS; i++) sca[i] >>= 8;
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // every read of this position is done: behind the next barrier it is requested into
     }
-    // ---- epilogue: the position the last step was read from is idle until the next barrier
-    asm volatile("s_barrier" ::: "memory");
-    ffn_epilogue<RS, WM, BN, UP>(a, cur, acc, nsub, wm, wn, st + wave * 2304, &s_bias[cn & 1][wn * 64]);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                    // the slab has been read
-    stores = nsub > 0 ? (UP ? 2 : 1) * nsub : 0;                         // (every sub-tile stores at least its first row)
+    ffn_epilogue<RS, WM, BN, UP>(a, cur, acc, nsub, wm, wn, &s_bias[cn & 1][wn * 64]);
+    stores = nsub > 0 ? 2 * nsub : 0;                                    // (every sub-tile stores at least its first row)
     t += step_wg; cn++;
     if (t >= last) break;
     find(t, cur);
