@@ -418,6 +418,9 @@ int tga_prefill_step(const int64_t* model, const int64_t* blocks, const int32_t*
  * says which models it takes).  _plan: *ok, and bytes of the caller's workspace for `rows` rows that end in front of position `end`. */
 int tga_prefill16_plan(const int64_t* model, const int64_t* blocks, int64_t rows, int64_t end, int* ok, int64_t* nbytes);
 int tga_prefill16_step(const int64_t* model, const int64_t* blocks, const int32_t* tokens, int64_t P, int64_t tail, int64_t pos0, void* workspace, void* state, void* stream);
+/* One to three positions of such a prompt together, with the bits of a decode step each (the last ones, which no step of four holds).  _plan: *ok, and bytes of the caller's workspace. */
+int tga_prefill16_tail_plan(const int64_t* model, const int64_t* blocks, int* ok, int64_t* nbytes);
+int tga_prefill16_tail(const int64_t* model, const int64_t* blocks, const int32_t* tokens, int64_t rows, int64_t pos0, void* workspace, void* state, void* stream);
 
 #ifdef __cplusplus
 }

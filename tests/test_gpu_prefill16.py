@@ -190,3 +190,21 @@ def test_values_that_are_not_finite_stay_with_later_positions(gpu, name, n, at):
     for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)):
       ca, cb = ca.numpy()[:, :at], cb.numpy()[:, :at]
       assert np.isfinite(cb).all(); np.testing.assert_array_equal(ca.view(np.uint16), cb.view(np.uint16))
+
+@pytest.mark.parametrize("name,n,ctx", [("2048x1024", 22, 576), ("2048x1024", 40, 1024), ("1536x768", 23, 128), ("1024x1536", 136, 256), ("1024x1536", 1399, 2048), ("512x256", 206, 768), ("512x256", 259, 1600), ("512x256", 132, 136)])
+def test_bits_of_the_last_positions(gpu, monkeypatch, name, n, ctx):
+  """The one to three positions behind a prompt's last step of four together (tga_prefill16_tail) against single steps: one, two and three tiles of attention per split, rows on either side of a split's
+  edge (the second prompt of 206: 127, 128, 129), a cache that ends soon behind the prompt, and prompts that keep a prefix and leave another number of them."""
+  from tinygrad_amd import llm
+  a, b = _models(CONFIGS[name], 3 + n, ctx)
+  prompt = np.random.default_rng(n).integers(0, BASE["vocab_size"], size=n).tolist()
+  for p in (prompt, prompt[:n // 2] + [9] * 28, prompt[:n - 1]):
+    if len(p) >= ctx: continue
+    for m, least in ((a, 1), (b, 1 << 30)):
+      monkeypatch.setattr(llm, "ROWS16_TAIL", least)
+      m.prefill(p, reuse_cache=p is not prompt[:n - 1])
+      m.check_state()
+    assert a._chunker._rows16_ws is not None and b._chunker._rows16_ws is not None
+    for i, (ba, bb) in enumerate(zip(a.blk, b.blk)):
+      for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): assert (ca.numpy().view(np.uint16) == cb.numpy().view(np.uint16)).all(), f"block {i}"
+    _same_bits(a, b, len(p))

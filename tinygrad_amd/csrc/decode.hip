@@ -143,6 +143,7 @@ struct AttnArgs {
   // chunk 1 = the launch that only rotates and appends every row's key / value, chunk 2 = the launch that attends from the cache alone
   // (the rows of the chunk were appended by the launch before; a row sees the positions up to its own).  0: decode.
   int chunk, pos_step;
+  int pos0;                                            // attn_split1_kernel, several rows: position of the first one
   int split_shift;                                     // log2 of the positions per split partial that the merge launch sums (6: splits of 64; the matrix-core chunk launch may cover several tiles per partial)
 };
 __device__ __forceinline__ AttnArgs attn_args_of_sequence(AttnArgs a, int z) {
@@ -624,11 +625,15 @@ __global__ __launch_bounds__(256) void attn_chunk_mfma_kernel(const AttnArgs a, 
 // (max, sum) pairs of the splits in 16 floats.
 // NORM: q and k pass through an RMSNorm before the rotation (nn.RMSNorm, tinygrad/nn/__init__.py:296-304): 1 = over the whole q / k rows with weights of that
 // length (model.py:169), 2 = per head with head_dim weights (model.py:180); the workgroup sums the squares for itself.
-template <int HD8, int IT, int NW, int NORM>
+// ROWS: rows blockIdx.y of one sequence at consecutive positions, operands *_bs apart.  Several: a launch that appends every row's key and value (chunk 1, a workgroup per kv head and row), then one
+// that attends (chunk 2); a single row does both (chunk 0).
+template <int HD8, int IT, int NW, int NORM, bool ROWS = false>
 __global__ __launch_bounds__(NW * 64) void attn_split1_kernel(const AttnArgs a) {
   constexpr int HD = HD8 * 8, RPI = 64 / HD8, NVI = 16 / RPI, NGRP = NW * RPI, CSTR = HD + 4, SP = 16 * NW * IT;
   const int group = a.n_heads / a.n_kv;
   const int kvh = blockIdx.x % a.n_kv, rest = blockIdx.x / a.n_kv, hh = rest % group, split = rest / group, head = kvh * group + hh;
+  const int z = ROWS ? blockIdx.y : 0;
+  const float* const aq = a.q + (ROWS ? z * a.q_bs : 0); const float* const ak = a.k + (ROWS ? z * a.kv_bs : 0); const float* const av = a.v + (ROWS ? z * a.kv_bs : 0);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = HD >> 1;
   __shared__ float qs[HD], ks[HD], vs[HD];
   __shared__ float comb[NGRP * CSTR];                   // [run]: o[HD], m, l
@@ -636,8 +641,8 @@ __global__ __launch_bounds__(NW * 64) void attn_split1_kernel(const AttnArgs a) 
   const int p0 = split * SP + wave * 16;                // first position of this wave's first tile; tile t starts 16 NW t further
   // ---- loads that do not depend on the position
   const int ki = tid < half ? tid : half - 1, vi = tid < HD ? tid : HD - 1;
-  const float kx1 = a.k[kvh * HD + ki], kx2 = a.k[kvh * HD + half + ki], vx = a.v[kvh * HD + vi];
-  const float qx1 = a.q[head * HD + ki], qx2 = a.q[head * HD + half + ki];
+  const float kx1 = ak[kvh * HD + ki], kx2 = ak[kvh * HD + half + ki], vx = av[kvh * HD + vi];
+  const float qx1 = aq[head * HD + ki], qx2 = aq[head * HD + half + ki];
   float kw1 = 1.f, kw2 = 1.f, qw1 = 1.f, qw2 = 1.f, ssq = 0.f, ssk = 0.f;   // norm weights of this thread's pairs; its share of the sums of squares
   if constexpr (NORM != 0) {
     const int kb = NORM == 2 ? 0 : kvh * HD, qb = NORM == 2 ? 0 : head * HD;
@@ -646,7 +651,7 @@ __global__ __launch_bounds__(NW * 64) void attn_split1_kernel(const AttnArgs a) 
     else {
       const int n4q = (a.n_heads * HD) >> 2, n4k = (a.n_kv * HD) >> 2, nmax = n4q > n4k ? n4q : n4k;
       for (int i = tid; i < nmax; i += NW * 64) {
-        const f32x4 x = ((const f32x4*)a.q)[i < n4q ? i : n4q - 1], y = ((const f32x4*)a.k)[i < n4k ? i : n4k - 1];
+        const f32x4 x = ((const f32x4*)aq)[i < n4q ? i : n4q - 1], y = ((const f32x4*)ak)[i < n4k ? i : n4k - 1];
         if (i < n4q) ssq += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
         if (i < n4k) ssk += y.x * y.x + y.y * y.y + y.z * y.z + y.w * y.w;
       }
@@ -666,12 +671,12 @@ __global__ __launch_bounds__(NW * 64) void attn_split1_kernel(const AttnArgs a) 
       }
     }
   }
-  const int pos = a.st->pos;
+  const int pos = ROWS ? a.pos0 + z : a.st->pos;
   if (pos >= a.max_ctx || pos < 0) {                    // no cache row and no rotation row for this position: nothing is written, the host sees the flag
     if (blockIdx.x == 0 && tid == 0) atomicOr(&a.st->error, 2);
     return;
   }
-  float* ph_ = a.part + (size_t)head * (a.nsplit * HD + 16);
+  float* ph_ = a.part + (ROWS ? z * a.part_bs : 0) + (size_t)head * (a.nsplit * HD + 16);
   float* po = ph_ + (size_t)split * HD;                    // this split's weighted V sums
   float* pml = ph_ + (size_t)a.nsplit * HD + 2 * split;    // and its (max, sum)
   if (split * SP > pos) {                               // nothing cached in this split yet
@@ -700,10 +705,11 @@ __global__ __launch_bounds__(NW * 64) void attn_split1_kernel(const AttnArgs a) 
   }
   if (tid < HD) vs[tid] = vx;
   __syncthreads();
-  if (hh == 0 && pos / SP == split && tid < HD) {       // one workgroup per kv head appends this token to the cache
+  if ((ROWS && a.chunk ? a.chunk == 1 : hh == 0 && pos / SP == split) && tid < HD) {       // one workgroup per kv head appends this token to the cache
     a.cache_k[((size_t)kvh * a.max_ctx + pos) * HD + tid] = (_Float16)ks[tid];
     a.cache_v[((size_t)kvh * a.max_ctx + pos) * HD + tid] = (_Float16)vs[tid];
   }
+  if (ROWS && a.chunk == 1) return;
   const u32x4 kcur = pack8_f16(ks + vp * 8), vcur = pack8_f16(vs + vp * 8);   // rounded to fp16 exactly like the cached copy
   float qq[8];
 #pragma unroll
@@ -1177,6 +1183,34 @@ static int attention_decode_split(const float* q, const float* k, const float* v
   TGA_LAUNCH_CHECK();
   return 0;
 }
+}  // extern "C"
+
+// (decode.h)
+int attn_split_rows_splits(int max_ctx) { int ns = 0; return max_ctx > 0 && attn_split1_waves() == 8 && attn_split1_tiles(max_ctx, &ns) ? ns : 0; }
+int attn_split_rows(const float* q, const float* k, const float* v, long long stride, const float* q_norm_weight, const float* k_norm_weight, float norm_eps, void* cache_k, void* cache_v, float* partials,
+                    int rows, int pos0, int n_heads, int n_kv_heads, int head_dim, int max_ctx, const float* rope_table, bool append_only, hipStream_t s) {
+  int ns = 0; const int it = attn_split1_tiles(max_ctx, &ns);
+  TGA_REQUIRE(it > 0 && attn_split1_waves() == 8 && (head_dim == 64 || head_dim == 128) && rows >= 1 && pos0 >= 0 && pos0 + rows <= max_ctx && n_heads % n_kv_heads == 0, "attn_split_rows: outside its range");
+  AttnArgs a = {};
+  a.q = q; a.k = k; a.v = v; a.cache_k = (_Float16*)cache_k; a.cache_v = (_Float16*)cache_v; a.part = partials;
+  a.n_heads = n_heads; a.n_kv = n_kv_heads; a.hd = head_dim; a.max_ctx = max_ctx; a.nsplit = ns; a.split_shift = 6; a.pos0 = pos0;
+  a.rope = rope_table; a.scale = 1.0f / sqrtf((float)head_dim);
+  a.q_norm = q_norm_weight; a.k_norm = k_norm_weight; a.norm_eps = norm_eps;
+  a.q_bs = a.kv_bs = stride; a.part_bs = (long long)n_heads * (ns * head_dim + 16);
+#define TGA_SPLIT1_R(HD8) do { if (it == 1) attn_split1_kernel<HD8, 1, 8, 1, true><<<grid, 512, 0, s>>>(a); else if (it == 2) attn_split1_kernel<HD8, 2, 8, 1, true><<<grid, 512, 0, s>>>(a); \
+    else if (it == 3) attn_split1_kernel<HD8, 3, 8, 1, true><<<grid, 512, 0, s>>>(a); else attn_split1_kernel<HD8, 4, 8, 1, true><<<grid, 512, 0, s>>>(a); } while (0)
+  for (a.chunk = rows > 1 || append_only ? 1 : 0; a.chunk <= 2; a.chunk += a.chunk ? 1 : 3) {
+    const dim3 grid(a.chunk == 1 ? n_kv_heads : n_heads * ns, rows);
+    if (head_dim == 64) TGA_SPLIT1_R(8); else TGA_SPLIT1_R(16);
+    TGA_LAUNCH_CHECK();
+    if (append_only) break;
+  }
+#undef TGA_SPLIT1_R
+  return 0;
+}
+
+extern "C" {
+
 int tga_attention_decode_split(const float* q, const float* k, const float* v, void* cache_k, void* cache_v, float* partials, const void* state,
                                int n_heads, int n_kv_heads, int head_dim, int max_ctx, const float* rope_table, void* stream) {
   return attention_decode_split(q, k, v, nullptr, nullptr, 0.f, 0, cache_k, cache_v, partials, state, n_heads, n_kv_heads, head_dim, max_ctx, rope_table, stream);

@@ -687,7 +687,78 @@ static int x16_experts(const X16Expert& e, int64_t K, int64_t N, hipStream_t s) 
   return 0;
 }
 
+// The last one to three positions of a prompt: rows with the bits of single steps, whose kernels these are, with a job per row - a weight matrix comes from HBM once for all of them - and without
+// the last block's feed-forward, which nothing reads.  A block of three rows of the OLMoE architecture: q / k / v 12.9 us (9.1 for one row), appending 4.6, attention 5.4 (5.7), attn_output 8.2 (5.1),
+// router 4, gate / up 19.1 (11.1), down 8.9 (5.2): 63 us against 119 in three steps.  A prompt and its first logits, 508 positions and 1 / 2 / 3 more, together / as single steps: 8000 / 8010, 8120 / 8650,
+// 8290 / 9380 us; six blocks of D 1024: 1355 / 1405, 1378 / 1585, 1395 / 1800.
+template <int T> int qgemv1_launch_format(QArgs a, hipStream_t s);       // qgemv1.h
+#define X16_TAIL 3
+struct X16TailWs { size_t x, x2, qkv, part, xn, logits, sel, probs, act, y, total; };
+static X16TailWs x16_tail_layout(const int64_t* m, int64_t nsplit) {
+  X16TailWs w = {}; size_t o = 0;
+  auto take = [&](size_t n) { const size_t at = o; o += (X16_TAIL * n + 255) & ~(size_t)255; return at; };
+  const int64_t dim = m[PM_DIM], H = m[PM_HEADS], KV = m[PM_KV], hd = m[PM_HD], k = m[PM_TOPK];
+  w.x = take(dim * 4); w.x2 = take(dim * 4); w.qkv = take((H + 2 * KV) * hd * 4); w.part = take(H * (nsplit * hd + 16) * 4); w.xn = take(dim * 2);
+  w.logits = take(m[PM_EXPERTS] * 4); w.sel = take(k * 4); w.probs = take(k * 4); w.act = take(k * m[PM_HIDDEN] * 2); w.y = take(k * dim * 4);
+  w.total = o;
+  return w;
+}
+// (a single step of such a model: the one-launch attention, its partials merged by attn_output, the weighted sum of at most eight experts completed by the next block's q / k / v)
+static bool prefill16_tail_ok(const int64_t* m, const int64_t* blocks) {
+  return prefill16_ok(m, blocks) && m[PM_TOPK] <= 8 && m[PM_HEADS] * m[PM_HD] >= 512 && attn_split_rows_splits((int)m[PM_MAXCTX]) > 0;
+}
+
 extern "C" {
+
+int tga_prefill16_tail_plan(const int64_t* m, const int64_t* blocks, int* ok, int64_t* nbytes) {
+  TGA_REQUIRE(m && blocks && ok && nbytes, "tga_prefill16_tail_plan: null pointer");
+  *ok = prefill16_tail_ok(m, blocks);
+  *nbytes = *ok ? (int64_t)x16_tail_layout(m, attn_split_rows_splits((int)m[PM_MAXCTX])).total : 0;
+  return 0;
+}
+
+int tga_prefill16_tail(const int64_t* m, const int64_t* blocks, const int32_t* tokens, int64_t rows, int64_t pos0, void* workspace, void* state, void* stream) {
+  TGA_REQUIRE(m && blocks && tokens && workspace && state && rows >= 1 && rows <= X16_TAIL && pos0 >= 0 && pos0 + rows <= m[PM_MAXCTX], "tga_prefill16_tail: null pointer, or rows beyond the cache or more than %d", X16_TAIL);
+  TGA_REQUIRE(prefill16_tail_ok(m, blocks), "tga_prefill16_tail: a model outside the range (tga_prefill16_tail_plan says which are inside)");
+  const int R = (int)rows, dim = (int)m[PM_DIM], H = (int)m[PM_HEADS], KV = (int)m[PM_KV], hd = (int)m[PM_HD], nq = H * hd, nk = KV * hd, E = (int)m[PM_EXPERTS], k = (int)m[PM_TOPK], hid = (int)m[PM_HIDDEN];
+  const int nsplit = attn_split_rows_splits((int)m[PM_MAXCTX]);
+  const X16TailWs w = x16_tail_layout(m, nsplit);
+  uint8_t* ws = (uint8_t*)workspace;
+  float* x = (float*)(ws + w.x); float* x_new = (float*)(ws + w.x2); float* qkv = (float*)(ws + w.qkv); float* part = (float*)(ws + w.part); float* logits = (float*)(ws + w.logits);
+  float* probs = (float*)(ws + w.probs); float* y = (float*)(ws + w.y); int* sel = (int*)(ws + w.sel);
+  void* xn = ws + w.xn; void* act = ws + w.act;
+  hipStream_t s = (hipStream_t)stream;
+  const float eps = bits_f(m[PM_EPS_BITS]);
+  int rc;
+#define PF_DO(call) do { if ((rc = (call))) return rc; } while (0)
+  PF_DO(tga_embed_rows((const void*)m[PM_EMB], (int)m[PM_EMB_TYPE], dim, tokens, R, state, x, stream));
+  QArgs j = {};                                                           // a job per row over one matrix: whatever sel holds, its experts lie 0 bytes apart
+  j.sel = sel; j.xdiv = 1; j.xdiv_jobs = R; j.x_f32 = j.y_f32 = 1;
+  for (int64_t bi = 0; bi < m[PM_NBLOCKS]; bi++) {
+    const int64_t* b = blocks + bi * PB_COUNT;
+    QArgs a = j;
+    a.nseg = 3; a.K = dim; a.x = x; a.norm_w = (const float*)b[PB_ATTN_NORM]; a.norm_eps = eps; a.ystride = nq + 2 * nk; a.ntot = nq + 2 * nk;
+    a.w[0] = (const uint8_t*)b[PB_WQ]; a.w[1] = (const uint8_t*)b[PB_WK]; a.w[2] = (const uint8_t*)b[PB_WV];
+    a.y[0] = qkv; a.y[1] = qkv + nq; a.y[2] = qkv + nq + nk; a.n[0] = nq; a.n[1] = a.n[2] = nk;
+    if (bi) { a.comb_y = y; a.comb_p = probs; a.comb_k = k; a.comb_x_out = x_new; }
+    PF_DO(qgemv1_launch_format<GGML_F16>(a, s));
+    if (bi) { float* t = x; x = x_new; x_new = t; }
+    const bool last = bi + 1 == m[PM_NBLOCKS];
+    PF_DO(attn_split_rows(qkv, qkv + nq, qkv + nq + nk, nq + 2 * nk, (const float*)b[PB_QN], (const float*)b[PB_KN], eps, (void*)b[PB_CK], (void*)b[PB_CV], part, R, (int)pos0, H, KV, hd, (int)m[PM_MAXCTX],
+                          (const float*)m[PM_ROPE], last, s));
+    if (last) break;
+    a = j;
+    a.nseg = 1; a.K = nq; a.x = part; a.epilogue = 1; a.attn_S = nsplit; a.attn_hd_log2 = hd == 64 ? 6 : 7; a.ystride = dim; a.ntot = dim;
+    a.w[0] = (const uint8_t*)b[PB_WO]; a.y[0] = x; a.resid[0] = x; a.n[0] = dim;
+    PF_DO(qgemv1_launch_format<GGML_F16>(a, s));
+    PF_DO(tga_moe_router_rows(x, (const float*)b[PB_FFN_NORM], eps, (const void*)b[PB_ROUTER], R, dim, E, xn, logits, stream));
+    PF_DO(tga_qlinear_experts_routed_rows(GGML_MXFP4, (const void*)b[PB_GATE], (const void*)b[PB_UP], E, logits, R, k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), sel, probs,
+                                          xn, act, TGA_F16, hid, dim, stream));
+    PF_DO(tga_qlinear_experts(GGML_MXFP4, (const void*)b[PB_DOWN], nullptr, E, sel, R * k, 1, act, TGA_F16, y, TGA_F32, dim, hid, stream));
+  }
+#undef PF_DO
+  return 0;
+}
 
 int tga_prefill16_plan(const int64_t* m, const int64_t* blocks, int64_t rows, int64_t end, int* ok, int64_t* nbytes) {
   TGA_REQUIRE(m && blocks && ok && nbytes && rows >= 1 && end >= rows, "tga_prefill16_plan: null pointer or no rows");

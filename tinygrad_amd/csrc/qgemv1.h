@@ -308,7 +308,8 @@ __device__ __forceinline__ void qgemv1_body(const QArgs& args, const unsigned bx
     for (int t = 0; t < F::XV; t++) xv[0][t] = xs[t * a.nu + uc];
     issue(b[0], lo);
     F::cfromx(xv[0], cv[0]);
-  } else if constexpr (PRO == 5) {
+  } else if constexpr (PRO == 5 || PRO == 9) {
+    const int jr = PRO == 9 ? job : 0;                           // (9: jobs, a row each with summands of its own; in 5 the addresses would cost a decode step of sixteen blocks 6 us)
     constexpr int CK = 8;                                        // rows of the weighted sum (fewer: the surplus ones reload row 0 with weight 0)
     const int i = (int)threadIdx.x < nq ? (int)threadIdx.x : nq - 1;
     f32x4 l = xr[2 * i], h = xr[2 * i + 1];
@@ -317,9 +318,9 @@ __device__ __forceinline__ void qgemv1_body(const QArgs& args, const unsigned bx
 #pragma unroll
     for (int j = 0; j < CK; j++) {
       const int jc = j < a.comb_k ? j : 0;
-      const f32x4* yr = (const f32x4*)(a.comb_y + (size_t)jc * a.K);
+      const f32x4* yr = (const f32x4*)(a.comb_y + (size_t)(jr * a.comb_k + jc) * a.K);
       yl[j] = yr[2 * i]; yh[j] = yr[2 * i + 1];
-      pj[j] = a.comb_p[jc];
+      pj[j] = a.comb_p[jr * a.comb_k + jc];
     }
 #pragma unroll
     for (int j = 0; j < CK; j++) {
@@ -327,7 +328,7 @@ __device__ __forceinline__ void qgemv1_body(const QArgs& args, const unsigned bx
       l.x += p * yl[j].x; l.y += p * yl[j].y; l.z += p * yl[j].z; l.w += p * yl[j].w;
       h.x += p * yh[j].x; h.y += p * yh[j].y; h.z += p * yh[j].z; h.w += p * yh[j].w;
     }
-    if (bx == 0 && blockIdx.y == 0 && (int)threadIdx.x < nq) { ((f32x4*)a.comb_x_out)[2 * i] = l; ((f32x4*)a.comb_x_out)[2 * i + 1] = h; }
+    if (bx == 0 && (PRO == 9 || blockIdx.y == 0) && (int)threadIdx.x < nq) { f32x4* xo = (f32x4*)(a.comb_x_out + (size_t)jr * a.K); xo[2 * i] = l; xo[2 * i + 1] = h; }
     float ss = (int)threadIdx.x < nq ? l.x * l.x + l.y * l.y + l.z * l.z + l.w * l.w + h.x * h.x + h.y * h.y + h.z * h.z + h.w * h.w : 0.f;
     ss = wave_sum(ss);
     if (lane == 0) nred[wave] = ss;
@@ -385,12 +386,12 @@ __device__ __forceinline__ void qgemv1_body(const QArgs& args, const unsigned bx
     __syncthreads();                                             // every wave holds its pieces: only now the first weights (as in prologue 1)
     issue(b[0], lo);
     lds_to_regs();
-  } else if constexpr (PRO == 7) {
+  } else if constexpr (PRO == 7 || PRO == 10) {                   // (10: jobs, a row's partials each)
     // the row is the merge of the attention's split partials (attn_split1_kernel): thread t merges elements 8t .. 8t + 7 of its head; a split
     // without cached positions carries max = -inf, sum = 0.  One instantiation per number of splits, so that exactly its loads go out, as one batch.
     const int i = (int)threadIdx.x < nq ? (int)threadIdx.x : nq - 1;
     const int hd = 1 << a.attn_hd_log2, head = (8 * i) >> a.attn_hd_log2, d0 = 8 * i - (head << a.attn_hd_log2);
-    const float* ph = (const float*)a.x + (size_t)head * (a.attn_S * hd + 16);
+    const float* ph = (const float*)a.x + (size_t)((PRO == 10 ? job * (a.K >> a.attn_hd_log2) : 0) + head) * (a.attn_S * hd + 16);
     f32x4 l, h;
     switch (a.attn_S) {
       case 1: attn_merge_piece<1>(ph, hd, d0, l, h); break; case 2: attn_merge_piece<2>(ph, hd, d0, l, h); break; case 3: attn_merge_piece<3>(ph, hd, d0, l, h); break;
@@ -567,7 +568,8 @@ static int launch_fast(QArgs a, hipStream_t s) {
   else {
   if constexpr (EPI == 1 && WK == 1 && !H) {
     if (a.attn_S > 0) {
-      if (a.K / 8 > NT || a.x_staged || !a.x_f32 || a.sel) return tga_set_error("tga_attn_merge_qlinear: needs one float32 partial row set of at most %d values", 8 * NT);
+      if (a.K / 8 > NT || a.x_staged || !a.x_f32 || (a.sel && T != GGML_F16)) return tga_set_error("tga_attn_merge_qlinear: needs one float32 partial row set of at most %d values", 8 * NT);
+      if constexpr (T == GGML_F16) { if (a.sel) return launch_fast_p<T, R, WK, WR, EPI, H, 10>(a, grid, lds, s); }
       return launch_fast_p<T, R, WK, WR, EPI, H, 7>(a, grid, lds, s);
     }
   }
@@ -575,7 +577,8 @@ static int launch_fast(QArgs a, hipStream_t s) {
   if constexpr (EPI == 1) { if (a.x_staged) return launch_fast_p<T, R, WK, WR, EPI, H, 2>(a, grid, lds, s); }
   if constexpr (WK == 1 && EPI == 0) {
     if (a.comb_y) {
-      if (a.x_staged || !a.norm_w || !a.x_f32 || a.K / 8 > NT || a.comb_k > 8) return tga_set_error("tga_moe_combine_rmsnorm_qlinear_multi: needs one float32 row of at most %d values and at most 8 summands", 8 * NT);
+      if (a.x_staged || !a.norm_w || !a.x_f32 || a.K / 8 > NT || a.comb_k > 8 || (a.sel && T != GGML_F16)) return tga_set_error("tga_moe_combine_rmsnorm_qlinear_multi: needs one float32 row of at most %d values and at most 8 summands", 8 * NT);
+      if constexpr (T == GGML_F16) { if (a.sel) return launch_fast_p<T, R, WK, WR, EPI, H, 9>(a, grid, lds, s); }
       return launch_fast_p<T, R, WK, WR, EPI, H, 5>(a, grid, lds, s);
     }
   }

@@ -62,6 +62,7 @@ MANY_ROWS_MIN = 17
 # step, six blocks, us: D 2048 k 2 x 1536 1144 / 871, 4 x 1024 1050 / 877, 8 x 1024 1248 / 1088, 8 x 1536 1222 / 1330; D 1024 694 / 600 (2 x 512), 925 / 818 (8 x 1024), 877 / 936 (8 x 1536); D 512 661 / 669
 # (4 x 1024), 745 / 876 (8 x 1536).  One more step of four: 21 tokens 1277 / 1611, 1194 / 1299 (D 2048, 8 x 1024 and 2 x 1536), 704 / 958 (D 1024, 2 x 512).
 ROWS16, ROWS16_MIN, ROWS16_BYTES = 1024, 20, 1 << 29
+ROWS16_TAIL = 1                    # ... and so many of the one to three positions behind its last step of four at least to be computed together (one: as fast as a single step or faster, figures in csrc/prefill16.hip)
 ROWS16_WIDE = 10240                # k times the experts' width from which on four positions fewer are enough
 
 def precompute_freqs_cis(dim: int, end: int, theta: float) -> np.ndarray:
@@ -696,6 +697,8 @@ class BatchedTransformer:
         self.rows64 = 2 if B <= 32 else 4 if B <= 64 else 8             # column groups of sixteen rows in the layout
     self._rows_tables, self._rows_ws, self._rows_tok = self._many_rows_tables(), None, None
     self._rows16_ws, self._rows16_tok = None, None                       # (prefill_rows16's)
+    # (a single step of the model takes the launches that tga_prefill16_tail takes for several rows)
+    self._tail_rows = chunk_of is not None and all(b.moe and b.can_fold_combine and b.fused_attn and b.route_in_experts for b in chunk_of.blk)
     self.many_rows = not c.num_experts                                  # lockstep prompts as steps of many rows (see Transformer.many_rows)
     self.x = None
     if not self.chunked: self._alloc_step()
@@ -788,7 +791,7 @@ class BatchedTransformer:
 
   def prefill_rows16(self, tokens: list[int], start: int, begin=None) -> int:
     """Chunked prefill for `chunk_of`, an MoE model: the rows of the steps of sixteen positions from start on, and of the one step each of eight and four behind them, all together and with the bits
-    of those steps (csrc/prefill16.hip).  Returns the number of positions done: none for models outside that kernel's range and where there is no memory for its buffers.
+    of those steps, then the one to three single steps behind those in launches of their own (csrc/prefill16.hip).  Returns the number of positions done: none for models outside that kernel's range and where there is no memory for its buffers.
     begin: as in prefill_rows."""
     c = self.config
     if not self.chunked or self._rows_tables is None or self.expert_path != "jobs": return 0
@@ -801,19 +804,27 @@ class BatchedTransformer:
     per = min(n, ROWS16)
     while plan(per) > ROWS16_BYTES and per > 64: per = per // 32 * 16
     if not ok.value: return 0
+    rest = total - n if total - n >= ROWS16_TAIL and self._tail_rows else 0      # positions of single steps that are computed together
+    if rest:
+      tail_ok, tail_need = ctypes.c_int(0), ctypes.c_int64(0)
+      rt.check(rt.lib().tga_prefill16_tail_plan(*self._rows_tables, ctypes.byref(tail_ok), ctypes.byref(tail_need)))
+      if tail_ok.value: need.value = max(need.value, tail_need.value)
+      else: rest = 0
     try:
       if self._rows16_ws is None or self._rows16_ws.nbytes < need.value: self._rows16_ws = Buffer((need.value,), np.uint8)
-      if self._rows16_tok is None or self._rows16_tok.nbytes < 4 * n: self._rows16_tok = Buffer((4 * n,), np.uint8)
+      if self._rows16_tok is None or self._rows16_tok.nbytes < 4 * (n + rest): self._rows16_tok = Buffer((4 * (n + rest),), np.uint8)
     except RuntimeError as e:
       if "HIP Error 2," not in str(e): raise
       return 0
     st = np.zeros(16, np.int32); st[0], st[3], st[5] = start, len(tokens), c.vocab_size
     self.state.copyin(st)
-    self._rows16_tok.view(0, (n,), np.int32).copyin(np.array(tokens[start:start + n], np.int32))
+    self._rows16_tok.view(0, (n + rest,), np.int32).copyin(np.array(tokens[start:start + n + rest], np.int32))
     self._owner_stream.synchronize()
     for i in range(0, n, per):
       m = min(per, n - i)
       rt.check(rt.lib().tga_prefill16_step(*self._rows_tables, self._rows16_tok.ptr + 4 * i, m, max(0, m - max(0, n - tail - i)), start + i, self._rows16_ws.ptr, self.state.ptr, self.stream.handle))
+    if rest: rt.check(rt.lib().tga_prefill16_tail(*self._rows_tables, self._rows16_tok.ptr + 4 * n, rest, start + n, self._rows16_ws.ptr, self.state.ptr, self.stream.handle))
+    n += rest
     if begin is not None and start + n == len(tokens) - 1: begin(self.stream)
     self.stream.synchronize()
     self.check_state()
