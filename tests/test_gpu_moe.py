@@ -261,3 +261,38 @@ def test_small_glm4moe_like_decode(gpu, gate):
     for pos, t in enumerate(hist): lg2 = o2.forward(t, pos)
     print(f"without {drop}: logits rel-err {ol.rel_err(lg2, lg_gpu):.3f}")
     assert ol.rel_err(lg2, lg_gpu) > 5e-3, drop                                    # five times the parity bar
+
+@pytest.mark.parametrize("E,k", [(1, 1), (2, 2), (7, 3), (16, 16), (33, 8), (63, 16), (64, 1), (64, 8), (64, 16)])
+@pytest.mark.parametrize("gating", [1, 2, 3, 4])
+def test_gating_in_lanes_has_the_bits_of_the_general_way(gpu, E, k, gating):
+  """At most 64 experts and 16 selected (an expert per lane) against the general way, which a selection bias of zeros takes: rows with ties, values that are not finite, both zeros, the type's lowest
+  and values far apart; the expert gate/up launch's own choice (its outputs carry the expert) on the same rows."""
+  from tinygrad_amd.nn import ExpertWeights, moe_gate
+  rng = np.random.default_rng(E * 17 + gating)
+  rows = [rng.standard_normal(E) * 2, np.zeros(E), np.where(rng.random(E) < .5, 0.0, -0.0), rng.integers(-2, 3, E), rng.standard_normal(E) * 200, np.full(E, -3.4028235e38), rng.standard_normal(E) * 1e-30]
+  for v in (np.nan, np.inf, -np.inf):
+    for at in (0, E // 2, E - 1): r = rng.standard_normal(E); r[at] = v; rows.append(r)
+  rows += [np.full(E, np.nan), np.full(E, -np.inf), np.full(E, np.inf), np.where(rng.random(E) < .5, -np.inf, 1.0)]
+  lg = np.array(rows, np.float32); T = len(lg)
+  if E == k: lg = lg[~np.isnan(lg).any(1)]; T = len(lg)                            # (several experts rank lowest there and share a slot)
+  if E == k and gating == 1: lg = lg[np.isfinite(lg).all(1)]; T = len(lg)
+  b = gpu.Buffer.from_numpy(np.ascontiguousarray(lg)); zero = gpu.Buffer((E,), np.float32).zero_()
+  def gate(g, norm, bias):
+    sel, p = gpu.Buffer((T * k,), np.int32), gpu.Buffer((T * k,), np.float32)
+    moe_gate(b, T, E, k, sel, p, g, norm, 1.5, bias=bias)
+    return sel, p
+  dim, n = 64, 16
+  w = [gpu.Buffer.from_numpy(np.repeat(np.arange(1, E + 1, dtype=np.float16) * 2.0 ** -6, n * dim).astype(np.float16).view(np.uint8)) for _ in range(2)]
+  ew, eu = (ExpertWeights(x, 1, E, n, dim) for x in w)
+  x = gpu.Buffer.from_numpy(np.full((T, dim), 1 / 16, np.float16))
+  for norm in (False, True):
+    sel, p = gate(gating, norm, None)
+    ref, rp = gate(3, False, zero) if gating == 1 and norm else gate(gating, norm, zero)      # (the softmax over all normed over the selected is the softmax over the selected)
+    np.testing.assert_array_equal(sel.numpy(), ref.numpy())
+    np.testing.assert_array_equal(p.numpy(), rp.numpy())
+    s1, p1, y0, y1 = gpu.Buffer((T * k,), np.int32), gpu.Buffer((T * k,), np.float32), gpu.Buffer((T * k, n), np.float32), gpu.Buffer((T * k, n), np.float32)
+    ew(sel, x, y0, jobs_per_x_row=k, up=eu)
+    ew(s1, x, y1, jobs_per_x_row=k, up=eu, route=(b, gating, norm, 1.5, p1))
+    np.testing.assert_array_equal(s1.numpy(), ref.numpy())
+    np.testing.assert_array_equal(p1.numpy(), rp.numpy())
+    np.testing.assert_array_equal(y1.numpy(), y0.numpy())

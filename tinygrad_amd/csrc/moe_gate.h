@@ -3,6 +3,51 @@
 #pragma once
 #include "common.h"
 
+// At most 64 experts of which at most 16 are taken (every model of the benchmarks): expert = lane, nothing in LDS.  The k largest scores are taken one after the other, the largest first - the wave's
+// maximum, of the lanes that hold it the lowest - which is the pairwise rank below as long as no score is NaN (those rank by themselves: the general way).  k steps of a reduction in registers, 
+// about 80 cycles each, against 64 reads of LDS with their comparisons and a maximum by way of LDS.
+#define GATE_LANES_E 64
+#define GATE_LANES_K 16
+__device__ __forceinline__ bool gate_in_lanes(int n_experts, int k) { return n_experts <= GATE_LANES_E && k <= GATE_LANES_K; }
+__device__ __forceinline__ int gate_kind(int gating, int norm_topk) { return gating == 1 && norm_topk ? 3 : gating; }      // model.py:116-117: softmax over the selected is all there is to it
+// the score of expert `lane` from its logit v (lanes behind the last expert: any v); false: a score is NaN
+__device__ __forceinline__ bool gate_score_lane(float v, int n_experts, int kind, int lane, float& s) {
+  const bool has = lane < n_experts;
+  if (kind == 3) s = v;
+  else if (kind == 1) {
+    const float mx = wave_max_dpp(has ? v : -INFINITY), e = has ? expf(v - mx) : 0.f, sum = wave_sum(e);
+    s = e * (1.0f / sum);
+  } else if (kind == 2) s = 1.0f / (1.0f + expf(-v));
+  else s = sqrtf(log1pf(expf(v)));
+  return __ballot(has && !(s == s)) == 0;
+}
+// the experts of the slots k - 1 down to `slot`: lane j holds slot j's expert and score, the result is slot's expert
+__device__ __forceinline__ int gate_pick_lanes(float s, int n_experts, int k, int slot, int lane, int& sel, float& p) {
+  unsigned long long left = n_experts >= 64 ? ~0ull : (1ull << n_experts) - 1;
+  float c = lane < n_experts ? s : -INFINITY;
+  int e = 0;
+  sel = 0; p = 0.f;
+  for (int j = k - 1; j >= slot; j--) {
+    e = __builtin_ctzll(__ballot(c == wave_max_dpp(c)) & left);
+    left &= ~(1ull << e);
+    const float se = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), e));
+    if (lane == e) c = -INFINITY;
+    if (lane == j) { sel = e; p = se; }
+  }
+  return e;
+}
+// the weight of slot `lane` (below k) from the slots' scores
+__device__ __forceinline__ float gate_weight_lanes(float p, int k, int gating, int norm_topk, float scale, int lane) {
+  auto sum = [&](float v) { float z = 0.f; for (int j = 0; j < k; j++) z += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), j)); return z; };
+  if (gate_kind(gating, norm_topk) == 3) {                // softmax over the selected logits
+    const float e = expf(p - wave_max_dpp(lane < k ? p : -INFINITY));
+    p = e * (1.0f / sum(e));
+    if (gating == 1) norm_topk = 0;
+  }
+  if (norm_topk) p = p / sum(p);
+  return p * scale;
+}
+
 // scores per ExpertGating (model.py:9-13, 116-121): 1 SOFTMAX, 2 SIGMOID, 3 SOFTMAX_WEIGHT (softmax over the selected logits),
 // 4 SQRT_SOFTPLUS.  Top-k by pairwise rank exactly as pairwise_topk (model.py:35-41): rank_i = #{j: s_i > s_j or (s_i == s_j and
 // i < j)}; the k highest ranks are emitted in ASCENDING rank order (the largest last), so among equal scores the lower index
@@ -14,6 +59,15 @@ __device__ __forceinline__ void gate_topk_wave(const float* lg, int n_experts, i
                                                int* __restrict__ sel, float* __restrict__ probs, float* sc, float* tmp, int lane,
                                                const float* bias = nullptr, float* scb = nullptr) {
   int* s_sel = (int*)tmp; float* s_p = tmp + 64; float* s_q = tmp + 128;
+  if (!bias && gate_in_lanes(n_experts, k)) {
+    float s, p; int e;
+    if (gate_score_lane(lg[lane < n_experts ? lane : n_experts - 1], n_experts, gate_kind(gating, norm_topk), lane, s)) {
+      gate_pick_lanes(s, n_experts, k, 0, lane, e, p);
+      p = gate_weight_lanes(p, k, gating, norm_topk, scale, lane);
+      if (lane < k) { s_sel[lane] = e; sel[lane] = e; probs[lane] = p; }
+      return;
+    }
+  }
   if (!bias) scb = sc;
   if (gating == 1 && norm_topk && !bias) { gating = 3; norm_topk = 0; }   // model.py:116-117 fast path (only without a selection bias)
   float mx = -INFINITY;

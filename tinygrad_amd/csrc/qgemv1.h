@@ -409,15 +409,31 @@ __device__ __forceinline__ void qgemv1_body(const QArgs& args, const unsigned bx
     for (int t = 0; t < 2; t++) v[t] = xh[(int)threadIdx.x + NT * t < nq ? (int)threadIdx.x + NT * t : nq - 1];
     // jobs xrow * k .. xrow * k + k - 1 belong to token xrow: every workgroup gates its own token
     const int slot = job - (int)xrow * a.route_k;
-    for (int i = threadIdx.x; i < a.route_E; i += NT) tk_lg[i] = a.route_logits[xrow * a.route_E + i];
-    __syncthreads();
-    if (wave == 0) gate_topk_wave(tk_lg, a.route_E, a.route_k, a.route_gating, a.route_norm_topk, a.route_scale, tk_sel, tk_p, tk_sc, tk_tmp, lane);
-    __syncthreads();
-    eoff = (long long)tk_sel[slot] * a.estride;
-    enter(0);                                                    // the weight bases of the selected expert
-    if (bx == 0 && slot == 0 && (int)threadIdx.x < a.route_k) {
-      a.sel[xrow * a.route_k + threadIdx.x] = tk_sel[threadIdx.x]; a.route_probs_out[xrow * a.route_k + threadIdx.x] = tk_p[threadIdx.x];
+    int expert = 0;
+    bool lanes = gate_in_lanes(a.route_E, a.route_k);
+    if (lanes) {                                                 // every wave for itself, as far as its slot, and no barrier in front of the weights
+      float sc; int es; float ps;
+      lanes = gate_score_lane(a.route_logits[xrow * a.route_E + (lane < a.route_E ? lane : a.route_E - 1)], a.route_E, gate_kind(a.route_gating, a.route_norm_topk), lane, sc);
+      if (lanes) {
+        expert = gate_pick_lanes(sc, a.route_E, a.route_k, slot, lane, es, ps);
+        if (bx == 0 && slot == 0 && wave == 0) {
+          ps = gate_weight_lanes(ps, a.route_k, a.route_gating, a.route_norm_topk, a.route_scale, lane);
+          if (lane < a.route_k) { a.sel[xrow * a.route_k + lane] = es; a.route_probs_out[xrow * a.route_k + lane] = ps; }
+        }
+      }
     }
+    if (!lanes) {
+      for (int i = threadIdx.x; i < a.route_E; i += NT) tk_lg[i] = a.route_logits[xrow * a.route_E + i];
+      __syncthreads();
+      if (wave == 0) gate_topk_wave(tk_lg, a.route_E, a.route_k, a.route_gating, a.route_norm_topk, a.route_scale, tk_sel, tk_p, tk_sc, tk_tmp, lane);
+      __syncthreads();
+      expert = __builtin_amdgcn_readfirstlane(tk_sel[slot]);
+      if (bx == 0 && slot == 0 && (int)threadIdx.x < a.route_k) {
+        a.sel[xrow * a.route_k + threadIdx.x] = tk_sel[threadIdx.x]; a.route_probs_out[xrow * a.route_k + threadIdx.x] = tk_p[threadIdx.x];
+      }
+    }
+    eoff = (long long)expert * a.estride;
+    enter(0);                                                    // the weight bases of the selected expert
     issue(b[0], lo);
 #pragma unroll
     for (int t = 0; t < 2; t++) { const int i = (int)threadIdx.x + NT * t; if (i < nq) put_piece(i, v[t]); }
