@@ -254,14 +254,24 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
 // ------------------------------------------------------------------------------------------------ grouping of the routed rows by expert
 #define PF_MAX_E 512
 // One wave per token: selection and weights (gate_topk_wave), and this assignment's place among the rows of its expert.  The order of places is that of arrival: a row's
-// values do not depend on its place, and the weighted sum of a token runs over its slots in order.
-__global__ __launch_bounds__(256) void rows_gate_kernel(const float* __restrict__ logits, int R, int E, int k, int gating, int norm_topk, float scale, int* __restrict__ sel,
+// values do not depend on its place, and the weighted sum of a token runs over its slots in order.  A workgroup counts its tokens' assignments in LDS and adds them up in one go (an addition per
+// assignment: the two lines that 64 counts are in were what all waves waited for; 508 rows of 64 experts, top 8: 11.6 -> 4.8 us).
+#define PF_GATE_T 16
+__global__ __launch_bounds__(64 * PF_GATE_T) void rows_gate_kernel(const float* __restrict__ logits, int R, int E, int k, int gating, int norm_topk, float scale, int* __restrict__ sel,
                                                         float* __restrict__ probs, int* __restrict__ counts, int* __restrict__ place) {
-  __shared__ float sc[4][PF_MAX_E]; __shared__ float tmp[4][192];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, t = blockIdx.x * 4 + wave;
-  if (t >= R) return;
-  gate_topk_wave(logits + (size_t)t * E, E, k, gating, norm_topk, scale, sel + (size_t)t * k, probs + (size_t)t * k, sc[wave], tmp[wave], lane);
-  if (lane < k) { const int e = ((const int*)tmp[wave])[lane]; place[(size_t)t * k + lane] = atomicAdd(&counts[e], 1); }
+  __shared__ float sc[PF_GATE_T][PF_MAX_E]; __shared__ float tmp[PF_GATE_T][192];
+  __shared__ int s_count[PF_MAX_E];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, t = blockIdx.x * PF_GATE_T + wave;
+  if (tid < E) s_count[tid] = 0;
+  if (t < R) gate_topk_wave(logits + (size_t)t * E, E, k, gating, norm_topk, scale, sel + (size_t)t * k, probs + (size_t)t * k, sc[wave], tmp[wave], lane);
+  __syncthreads();
+  const bool has = t < R && lane < k;
+  int e = 0, at = 0;
+  if (has) { e = ((const int*)tmp[wave])[lane]; at = atomicAdd(&s_count[e], 1); }
+  __syncthreads();
+  if (tid < E && s_count[tid]) s_count[tid] = atomicAdd(&counts[tid], s_count[tid]);
+  __syncthreads();
+  if (has) place[(size_t)t * k + lane] = s_count[e] + at;
 }
 // Offsets of the experts' rows, the list of tiles of tt rows, and every row's token and assignment; each workgroup scans the counts for itself, the first writes the lists
 __global__ __launch_bounds__(512) void rows_group_kernel(const int* __restrict__ counts, const int* __restrict__ sel, const int* __restrict__ place, int R, int E, int k, int tt,
@@ -293,7 +303,7 @@ __global__ __launch_bounds__(512) void rows_group_kernel(const int* __restrict__
 
 int pf_gate_group(const float* logits, int R, int E, int k, int gating, int norm_topk, float scale, int* sel, float* probs, int* counts, int* place, int tt, int* off, int2* tiles, int* n_tiles,
                   int* row_tok, int* row_dst, hipStream_t s) {
-  rows_gate_kernel<<<(unsigned)((R + 3) / 4), 256, 0, s>>>(logits, R, E, k, gating, norm_topk, scale, sel, probs, counts, place);
+  rows_gate_kernel<<<(unsigned)((R + PF_GATE_T - 1) / PF_GATE_T), 64 * PF_GATE_T, 0, s>>>(logits, R, E, k, gating, norm_topk, scale, sel, probs, counts, place);
   TGA_LAUNCH_CHECK();
   const int64_t gb = ((int64_t)R * k + 511) / 512;
   rows_group_kernel<<<(unsigned)(gb < 64 ? gb : 64), 512, 0, s>>>(counts, sel, place, R, E, k, tt, off, tiles, n_tiles, row_tok, row_dst);
