@@ -173,6 +173,8 @@ __global__ __launch_bounds__(256) void x16_rope_kernel(const X16Rope a) {
 // chunk: workgroup = (kv head, 64 positions, X16_ROWS rows); four (row, query head) pairs at a time.  Three workgroups fit a CU (153 registers; with
 // 128 they spill: 78 us): of 512 rows and 16 heads 1152 workgroups of 32 rows, 1.5 rounds of the chip, or 2304 of 16, three: 60.5 -> 56.7 us.  Values behind a row's position are dropped by selects:
 // 57.4 -> 62.5 us; a path of its own for tiles that hold a value that is not finite takes registers or hoisted conversions from the other one (61.5 .. 70.9 us).
+// Bound by vector instructions, 170 a pair and wave.  Pairs counted on instead of divided, 62.8 -> 61.2, and without a branch per pair 59.7 us; two pairs step by step, or a loop without masks for tiles
+// whose rows see all 64 positions (217 registers, or 168 with spills), were 62.8 and 62.8 .. 64.3.
 #define X16_ROWS 16
 struct X16Attn { const float* qr; const uint16_t* ck; const uint16_t* cv; float* part; uint16_t* out; int H, KV, max_ctx, P, pos0, nsplit; float scale; };
 
@@ -203,57 +205,60 @@ __global__ __launch_bounds__(256) void x16_attn_kernel(const X16Attn a) {
   }
   const int np = (row_end - row_first) * group;
   f32x4 qa[4], qb[4];
-  auto fetch = [&](int b) __attribute__((always_inline)) {
+  int fp = 0, fh = 0;                                                      // the next pair to fetch: number, head in its group
+  const float* fs = a.qr + ((size_t)row_first * a.H + kvh * group) * HD + vp * 8;
+  const int to_row = (a.H - group + 1) * HD;
+  auto fetch = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int hh = 0; hh < 4; hh++) {
-      const int p = min(b + hh, np - 1), row = row_first + p / group, head = kvh * group + p % group;
-      const float* s = a.qr + ((size_t)row * a.H + head) * HD + vp * 8;
-      qa[hh] = *(const f32x4*)s; qb[hh] = *(const f32x4*)(s + 4);
+      qa[hh] = *(const f32x4*)fs; qb[hh] = *(const f32x4*)(fs + 4);
+      if (++fp < np) { fh++; const bool turn = fh == group; fs += turn ? to_row : HD; fh = turn ? 0 : fh; }      // (past the end: the last pair again)
     }
   };
-  fetch(0);
+  fetch();
+  int pos = a.pos0 + row_first, ph = 0;                                    // the next pair's position, head in its group
+  int or_ = row_first + wave / group, oh = wave % group;                   // row, head in its group of the pair whose partials this wave folds; four pairs further: + (4 / group, 4 % group)
+  const int or4 = 4 / group, oh4 = 4 % group;
   for (int b = 0; b < np; b += 4) {
     f32x4 q0[4], q1[4];
 #pragma unroll
     for (int hh = 0; hh < 4; hh++) { q0[hh] = qa[hh]; q1[hh] = qb[hh]; }
-    fetch(b + 4);                                                          // (past the end: the last pair again)
+    fetch();
 #pragma unroll
-    for (int hh = 0; hh < 4; hh++) {
-      if (b + hh < np) {
-        const int pos = a.pos0 + row_first + (b + hh) / group;
-        const float qq[8] = {q0[hh].x, q0[hh].y, q0[hh].z, q0[hh].w, q1[hh].x, q1[hh].y, q1[hh].z, q1[hh].w};
-        float sc[NVI];
-        float m = -INFINITY;
+    for (int hh = 0; hh < 4; hh++) {                                       // (pairs past the end repeat the last one, nothing reads their sums: without a branch per pair the steps of one run beside those of the next)
+      const float qq[8] = {q0[hh].x, q0[hh].y, q0[hh].z, q0[hh].w, q1[hh].x, q1[hh].y, q1[hh].z, q1[hh].w};
+      float sc[NVI];
+      float m = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < NVI; i++) {
-          const u32x4 kk = kt[i];
-          const half2_t k0 = as_h2(kk.x), k1 = as_h2(kk.y), k2 = as_h2(kk.z), k3 = as_h2(kk.w);
-          float t = qq[0] * (float)k0.x; t += qq[1] * (float)k0.y; t += qq[2] * (float)k1.x; t += qq[3] * (float)k1.y;
-          t += qq[4] * (float)k2.x; t += qq[5] * (float)k2.y; t += qq[6] * (float)k3.x; t += qq[7] * (float)k3.y;
-          t = x16_run_sum<HD8>(t);
-          sc[i] = (p0 + i * RPI + vr <= pos) ? t * a.scale : -INFINITY;
-          m = fmaxf(m, sc[i]);
-        }
-        float l = 0.f;
-        f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < NVI; i++) {
-          const float pj = (p0 + i * RPI + vr <= pos) ? __expf(sc[i] - m) : 0.f;
-          l += pj;
-          u32x4 vv = vt[i];
-          if (p0 + i * RPI + vr > pos) vv = u32x4{0u, 0u, 0u, 0u};         // (a later position's: 0 times a value that is not finite would reach this row)
-          const half2_t v0 = as_h2(vv.x), v1 = as_h2(vv.y), v2 = as_h2(vv.z), v3 = as_h2(vv.w);
-          o0.x += pj * (float)v0.x; o0.y += pj * (float)v0.y; o0.z += pj * (float)v1.x; o0.w += pj * (float)v1.y;
-          o1.x += pj * (float)v2.x; o1.y += pj * (float)v2.y; o1.z += pj * (float)v3.x; o1.w += pj * (float)v3.y;
-        }
-        float* cw = comb + (size_t)(hh * NGRP + wave * RPI + vr) * CSTR;
-        *(f32x4*)(cw + vp * 8) = o0; *(f32x4*)(cw + vp * 8 + 4) = o1;
-        if (vp == 0) { cw[HD] = m; cw[HD + 1] = l; }
+      for (int i = 0; i < NVI; i++) {
+        const u32x4 kk = kt[i];
+        const half2_t k0 = as_h2(kk.x), k1 = as_h2(kk.y), k2 = as_h2(kk.z), k3 = as_h2(kk.w);
+        float t = qq[0] * (float)k0.x; t += qq[1] * (float)k0.y; t += qq[2] * (float)k1.x; t += qq[3] * (float)k1.y;
+        t += qq[4] * (float)k2.x; t += qq[5] * (float)k2.y; t += qq[6] * (float)k3.x; t += qq[7] * (float)k3.y;
+        t = x16_run_sum<HD8>(t);
+        sc[i] = (p0 + i * RPI + vr <= pos) ? t * a.scale : -INFINITY;
+        m = fmaxf(m, sc[i]);
       }
+      float l = 0.f;
+      f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < NVI; i++) {
+        const float pj = (p0 + i * RPI + vr <= pos) ? __expf(sc[i] - m) : 0.f;
+        l += pj;
+        u32x4 vv = vt[i];
+        if (p0 + i * RPI + vr > pos) vv = u32x4{0u, 0u, 0u, 0u};         // (a later position's: 0 times a value that is not finite would reach this row)
+        const half2_t v0 = as_h2(vv.x), v1 = as_h2(vv.y), v2 = as_h2(vv.z), v3 = as_h2(vv.w);
+        o0.x += pj * (float)v0.x; o0.y += pj * (float)v0.y; o0.z += pj * (float)v1.x; o0.w += pj * (float)v1.y;
+        o1.x += pj * (float)v2.x; o1.y += pj * (float)v2.y; o1.z += pj * (float)v3.x; o1.w += pj * (float)v3.y;
+      }
+      float* cw = comb + (size_t)(hh * NGRP + wave * RPI + vr) * CSTR;
+      *(f32x4*)(cw + vp * 8) = o0; *(f32x4*)(cw + vp * 8 + 4) = o1;
+      if (vp == 0) { cw[HD] = m; cw[HD + 1] = l; }
+      if (++ph == group) { ph = 0; pos++; }
     }
     __syncthreads();
     if (b + wave < np) {
-      const int row = row_first + (b + wave) / group, head = kvh * group + (b + wave) % group;
+      const int row = or_, head = kvh * group + oh;
       const float* cb = comb + (size_t)wave * NGRP * CSTR;
       float m = -INFINITY;
 #pragma unroll
@@ -274,6 +279,8 @@ __global__ __launch_bounds__(256) void x16_attn_kernel(const X16Attn a) {
       for (int j = 0; j < HD / 64; j++) po[lane + 64 * j] = od[j];
       if (lane == 0) { po[HD] = m; po[HD + 1] = l; }
     }
+    or_ += or4; oh += oh4;
+    if (oh >= group) { oh -= group; or_++; }
     __syncthreads();
   }
 }
