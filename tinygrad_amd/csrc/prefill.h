@@ -8,7 +8,5 @@ enum { PB_ATTN_NORM, PB_FFN_NORM, PB_QN, PB_KN, PB_CK, PB_CV, PB_MOE, PB_WQ, PB_
 
 static inline float bits_f(int64_t b) { uint32_t u = (uint32_t)b; float f; memcpy(&f, &u, 4); return f; }
 
-// Gating of R rows of router logits and the grouping of their assignments by expert (prefill.hip): selection and weights per row, offsets of the experts' rows, tiles of tt rows,
-// and every grouped row's token and assignment.  counts: E zeros
-int pf_gate_group(const float* logits, int R, int E, int k, int gating, int norm_topk, float scale, int* sel, float* probs, int* counts, int* place, int tt, int* off, int2* tiles, int* n_tiles,
-                  int* row_tok, int* row_dst, hipStream_t s);
+// Gating of R rows of router logits (prefill.hip): selection and weights per row, the experts' counts (E zeros before) and each assignment's place among its expert's rows
+int pf_gate(const float* logits, int R, int E, int k, int gating, int norm_topk, float scale, int* sel, float* probs, int* counts, int* place, hipStream_t s);

@@ -301,10 +301,12 @@ __global__ __launch_bounds__(512) void rows_group_kernel(const int* __restrict__
   }
 }
 
-int pf_gate_group(const float* logits, int R, int E, int k, int gating, int norm_topk, float scale, int* sel, float* probs, int* counts, int* place, int tt, int* off, int2* tiles, int* n_tiles,
-                  int* row_tok, int* row_dst, hipStream_t s) {
+int pf_gate(const float* logits, int R, int E, int k, int gating, int norm_topk, float scale, int* sel, float* probs, int* counts, int* place, hipStream_t s) {
   rows_gate_kernel<<<(unsigned)((R + PF_GATE_T - 1) / PF_GATE_T), 64 * PF_GATE_T, 0, s>>>(logits, R, E, k, gating, norm_topk, scale, sel, probs, counts, place);
   TGA_LAUNCH_CHECK();
+  return 0;
+}
+static int pf_group(const int* counts, const int* sel, const int* place, int R, int E, int k, int tt, int* off, int2* tiles, int* n_tiles, int* row_tok, int* row_dst, hipStream_t s) {
   const int64_t gb = ((int64_t)R * k + 511) / 512;
   rows_group_kernel<<<(unsigned)(gb < 64 ? gb : 64), 512, 0, s>>>(counts, sel, place, R, E, k, tt, off, tiles, n_tiles, row_tok, row_dst);
   TGA_LAUNCH_CHECK();
@@ -441,7 +443,8 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
     const int tt = avg <= 32 ? 32 : avg <= 96 ? 64 : 128;
     const int64_t max_tiles = R * k / tt + (R * k < E ? R * k : E);
     int2* tiles = (int2*)(ws + w.tiles); int* nt = (int*)(ws + w.ntiles); int* off = (int*)(ws + w.off); int* row_tok = (int*)(ws + w.row_tok); int* row_dst = (int*)(ws + w.row_dst);
-    PF_DO(pf_gate_group(logits, (int)R, (int)E, (int)k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), sel, (float*)(ws + w.probs), counts, place, tt, off, tiles, nt, row_tok, row_dst, s));
+    PF_DO(pf_gate(logits, (int)R, (int)E, (int)k, (int)m[PM_GATING], (int)m[PM_NORM_TOPK], bits_f(m[PM_SCALE_BITS]), sel, (float*)(ws + w.probs), counts, place, s));
+    PF_DO(pf_group(counts, sel, place, (int)R, (int)E, (int)k, tt, off, tiles, nt, row_tok, row_dst, s));
     const int64_t hid = m[PM_HIDDEN];
     PF_DO(pf_experts((int)b[PB_TGATE], (const void*)b[PB_GATE], (const void*)b[PB_UP], hid, dim, xn, ws + w.act_e, 0, tt, max_tiles, tiles, nt, off, row_tok, nullptr, s));
     PF_DO(pf_experts((int)b[PB_TDOWN], (const void*)b[PB_DOWN], nullptr, dim, hid, (const uint16_t*)(ws + w.act_e), ws + w.y_e, 1, tt, max_tiles, tiles, nt, off, nullptr, row_dst, s));
