@@ -188,6 +188,26 @@ def test_rows_beyond_the_prompt_do_not_count(gpu, n):
   for ba, bb in zip(a.blk, b.blk):
     for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): np.testing.assert_array_equal(ca.numpy()[:, :n - 1], cb.numpy()[:, :n - 1])
 
+@pytest.mark.parametrize("cfg", [DENSE, DENSE128], ids=["hd64", "hd128"])
+@pytest.mark.parametrize("n", [194, 257, 471])
+def test_attention_of_rows_in_two_parts(gpu, cfg, n):
+  """Chains of four tiles of keys and more, which two groups of waves share: rows that see no key of the second group's first tile beside rows that do (prefixes of 5 and 122 positions), an odd and an even number
+  of tiles, caches that hold NaN behind the prompt; within 2e-3 of the model prefilled token by token, as above."""
+  a, b = _model(cfg, 23, ctx=640), _model(cfg, 23, ctx=640)
+  for blk in a.blk:
+    for cache in (blk.cache_k, blk.cache_v): cache.copyin(np.full(cache.shape, np.nan, np.float16))
+  b.prefill_chunk = 1
+  rng = np.random.default_rng(n)
+  prompt = rng.integers(0, cfg["vocab_size"], size=n).tolist()
+  for keep in (0, 5, 122):
+    p = prompt[:keep] + rng.integers(0, cfg["vocab_size"], size=n + keep % 7).tolist()
+    for m in (a, b): m.prefill(p)
+    for ba, bb in zip(a.blk, b.blk):
+      for ca, cb in ((ba.cache_k, bb.cache_k), (ba.cache_v, bb.cache_v)): assert ol.rel_err(ca.numpy()[:, :len(p) - 1].astype(np.float32), cb.numpy()[:, :len(p) - 1].astype(np.float32)) <= 2e-3
+    for m in (a, b): m.decode_step(); m.check_state()
+    assert ol.rel_err(a.logits(), b.logits()) <= 2e-3
+    prompt = p
+
 def _regions(model, cfg, n):
   """q, k, v and the attention's result of the last block in a step's workspace (x, xn, q, k, v, two halves of the query, result: pf_layout)."""
   nq, nk, at, out = cfg["n_heads"] * cfg["head_dim"], cfg["n_kv_heads"] * cfg["head_dim"], 0, {}

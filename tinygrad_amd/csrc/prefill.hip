@@ -114,18 +114,23 @@ __global__ __launch_bounds__(512) void rows_rope_kernel(const RopeArgs a) {
 // per dword, pieces XORed with the dimension.  The next tile is fetched while this one is multiplied.  flattened workgroup = (kv head, sequence) innermost: with eight
 // kv heads all readers of a head's rows run on one XCD and share its L2; the longest row tiles come first, in runs of as many tiles as give every CU a workgroup (cus), every second run
 // the other way round: the workgroups that share a CU have long and short tiles (1023 rows, 32 heads, two workgroups a CU: 41.4 -> 39.5 us).
+// NG = 2: eight waves, of which four take the even tiles of keys and four the odd ones; their sums meet in LDS.  A workgroup is a chain of tiles, 2.4 us each where it has a CU to itself and little less
+// where two share one, and registers leave room for eight waves a CU: for as many workgroups as CUs from four tiles on (heads of 128, 192 / 256 workgroups of up to 6 / 8 tiles 16.4 -> 15.5 / 20.4 ->
+// 18.1 us; of 64, 128 / 256 of up to 16 / 32 28.8 -> 20.5 / 55 -> 37), and for twice as many where chains are long (384 of up to 12 tiles 31.5 -> 27, 512 of up to 16 41.0 -> 38.9; not
+// taken: 192 of 3 tiles 10.9 / 11.7, 384 of 3 12.9 / 17.2, 512 of 4 / 8 16.9 / 21.0, 24 / 26, 768 of up to 24 71 / 82, 1024 of up to 32 114 / 129).
 // Two fp16 values hold 22 bits and more of a query or probability, and sums are formed in few additions at their full size (remainders first, two chains per score, a tile's products from
 // zero).  Share of fp16 results that are not the rounded float64 attention, 64 and 1024 positions, heads of 64 and 128, scores of standard deviation 0.03 .. 5: 1.8e-4 .. 2.2e-3; the float32
 // kernel of eight rows and fewer: 2.4e-4 .. 2.4e-3.  (Queries beyond 65504 have no such pair, as keys beyond have no cache row.)
 #define PSCALE 32768.0f             // of probabilities on their way to two fp16 values (the remainder of 0.2 is a subnormal number already: the absolute step 2^-24)
 struct RowsAttnArgs { const uint16_t* qh; const uint16_t* ql; const uint16_t* ck; const uint16_t* cv; uint16_t* out; int H, KV, max_ctx, P, pos0, nseq, qtiles, cus; float scale; };
 
-template <int HD>
-__global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
+template <int HD, int NG>
+__global__ __launch_bounds__(256 * NG) void rows_attn_kernel(const RowsAttnArgs a) {
   constexpr int NJ = HD / 32, NH = HD / 16, PC = HD / 8, IK = HD / 32, IV = HD / 64;     // 16-byte pieces per row; loads per thread and tile
-  __shared__ __attribute__((aligned(16))) uint8_t kl[64 * HD * 2];
-  __shared__ __attribute__((aligned(16))) uint8_t vl[HD * 128];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, c = lane & 15;
+  __shared__ __attribute__((aligned(16))) uint8_t kl_[NG][64 * HD * 2];
+  __shared__ __attribute__((aligned(16))) uint8_t vl_[NG][HD * 128];
+  const int part_ = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = NG > 1 ? threadIdx.x & 255 : threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, c = lane & 15;
+  uint8_t* const kl = kl_[part_]; uint8_t* const vl = vl_[part_];
   const int group = a.H / a.KV, kz = a.KV * a.nseq;
   int b = blockIdx.x;
   const int kvz = b % kz; b /= kz;
@@ -172,10 +177,10 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
 #pragma unroll
   for (int h = 0; h < NH; h++) O[h] = v4f32{0.f, 0.f, 0.f, 0.f};
   float M = -INFINITY, L = 0.f;
-  fetch(0);
-  for (int t = 0; t < ntiles; t++) {
+  fetch(part_);
+  for (int t = part_; t - part_ < ntiles; t += NG) {                       // (every part as often: a tile behind the last one is skipped below)
     put();
-    if (t + 1 < ntiles) fetch(t + 1);
+    if (t - part_ + NG < ntiles) fetch(t + NG);
     __syncthreads();
     if (64 * t <= last_wave) {
       v4f32 sc[4];
@@ -208,7 +213,8 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
           sc[k][i] = s; m = fmaxf(m, s);
         }
       m = fmaxf(m, __shfl_xor(m, 16)); m = fmaxf(m, __shfl_xor(m, 32));
-      const float mn = fmaxf(M, m * a.scale);                              // (finite: key 0 is visible to every row; log2(e) folded into the scale)
+      const float mt = fmaxf(M, m * a.scale);                              // (log2(e) folded into the scale)
+      const float mn = NG > 1 && mt == -INFINITY ? 0.f : mt;              // (key 0 is visible to every row, but none of the other part's may be)
       const float alpha = __builtin_amdgcn_exp2f(M - mn);
       float l = 0.f;
       u32x4 ph[2], pl[2];
@@ -225,7 +231,7 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
           pl[u][w] = f2h_bits(q0 - (float)h0) | (f2h_bits(q1 - (float)h1) << 16);
         }
       l += __shfl_xor(l, 16); l += __shfl_xor(l, 32);
-      L = L * alpha + l; M = mn;
+      L = L * alpha + l; M = mt;
 #pragma unroll
       for (int h = 0; h < NH; h++) {
         // (the tile's products sum from zero, remainders first: one addition at the size of the whole sum)
@@ -242,6 +248,24 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const RowsAttnArgs a) {
       }
     }
     __syncthreads();
+  }
+  if constexpr (NG > 1) {                                                 // the other part's sums, by way of LDS
+    f32x4* const so = (f32x4*)kl_ + wave * NH * 64 + lane; float* const sm = (float*)vl_ + tid * 2;
+    if (part_) {
+#pragma unroll
+      for (int h = 0; h < NH; h++) so[h * 64] = f32x4{O[h][0], O[h][1], O[h][2], O[h][3]};
+      sm[0] = M; sm[1] = L;
+    }
+    __syncthreads();
+    if (part_) return;
+    const float mt = fmaxf(M, sm[0]), f0 = __builtin_amdgcn_exp2f(M - mt), f1 = __builtin_amdgcn_exp2f(sm[0] - mt);
+    L = L * f0 + sm[1] * f1;
+#pragma unroll
+    for (int h = 0; h < NH; h++) {
+      const f32x4 o = so[h * 64];
+#pragma unroll
+      for (int i = 0; i < 4; i++) O[h][i] = __builtin_fmaf(O[h][i], f0, o[i] * f1);
+    }
   }
   if (wrow + c < a.P) {
     const float inv = (1.0f / PSCALE) / L;
@@ -423,7 +447,10 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
     aa.qh = ra.qh; aa.ql = ra.ql; aa.ck = ra.ck; aa.cv = ra.cv; aa.out = attn; aa.H = (int)H; aa.KV = (int)KV; aa.max_ctx = ra.max_ctx; aa.P = (int)P; aa.pos0 = (int)pos0; aa.nseq = (int)nseq;
     aa.qtiles = (int)((P + 63) / 64); aa.cus = (int)(H * nseq < 256 ? 256 / (H * nseq) : 1); aa.scale = (float)(1.4426950408889634 / sqrt((double)hd));
     const unsigned ag = (unsigned)(aa.qtiles * H * nseq);
-    if (hd == 64) rows_attn_kernel<64><<<ag, 256, 0, s>>>(aa); else rows_attn_kernel<128><<<ag, 256, 0, s>>>(aa);
+    if (ag <= 256 ? (pos0 + P + 63) / 64 >= 4 : ag <= 512 && (pos0 + P + 63) / 64 >= 12) {
+      aa.cus = aa.qtiles;                                                 // (one workgroup per CU: the longest first)
+      if (hd == 64) rows_attn_kernel<64, 2><<<ag, 512, 0, s>>>(aa); else rows_attn_kernel<128, 2><<<ag, 512, 0, s>>>(aa);
+    } else if (hd == 64) rows_attn_kernel<64, 1><<<ag, 256, 0, s>>>(aa); else rows_attn_kernel<128, 1><<<ag, 256, 0, s>>>(aa);
     TGA_LAUNCH_CHECK();
     PF_DO(linear_norm((int)b[PB_TO], b[PB_WO], attn, nq, (const float*)b[PB_FFN_NORM]));
     if (!b[PB_MOE]) {
