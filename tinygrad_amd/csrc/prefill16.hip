@@ -114,38 +114,40 @@ __global__ __launch_bounds__(1024) void x16_fold_norm_kernel(const float* __rest
 }
 
 // ------------------------------------------------------------------------------------------------ q / k norm over whole rows, rotation, append
-// One workgroup per row; the sums of squares as attn_decode_kernel forms them (four 16-byte pieces per thread, waves in order).  q leaves rotated in float32.
+// One workgroup per row; the sums of squares as attn_decode_kernel forms them (four 16-byte pieces per thread of four waves, waves in order); eight waves rotate (four: 508 rows 9.0 us, eight 7.3).  q leaves rotated in float32.
 __device__ __forceinline__ float x16_rope_lo(float x1, float x2, float c, float s) { return __builtin_fmaf(x1, c, -(x2 * s)); }
 __device__ __forceinline__ float x16_rope_hi(float x1, float x2, float c, float s) { return __builtin_fmaf(x2, c, x1 * s); }
 struct X16Rope { const float* q; const float* k; const float* v; const float* qn; const float* kn; const float* rope; float* qr; uint16_t* ck; uint16_t* cv; int* zero; int H, KV, hd, max_ctx, pos0, n_zero; float eps; };
-__global__ __launch_bounds__(256) void x16_rope_kernel(const X16Rope a) {
+__global__ __launch_bounds__(512) void x16_rope_kernel(const X16Rope a) {
   __shared__ float red[8];
   const int row = blockIdx.x, pos = a.pos0 + row, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = a.hd >> 1;
   const int nq = a.H * a.hd, nk = a.KV * a.hd;
-  if (row == 0) for (int i = tid; i < a.n_zero; i += 256) a.zero[i] = 0;
+  if (row == 0) for (int i = tid; i < a.n_zero; i += 512) a.zero[i] = 0;
   const float* q = a.q + (size_t)row * nq; const float* k = a.k + (size_t)row * nk; const float* v = a.v + (size_t)row * nk;
   const int n4q = nq >> 2, n4k = nk >> 2;
-  f32x4 nq4[4], nk4[4];
+  if (wave < 4) {
+    f32x4 nq4[4], nk4[4];
 #pragma unroll
-  for (int t = 0; t < 4; t++) {
-    const int i = tid + 256 * t;
-    nq4[t] = ((const f32x4*)q)[i < n4q ? i : n4q - 1]; nk4[t] = ((const f32x4*)k)[i < n4k ? i : n4k - 1];
-  }
-  float s0 = 0.f, s1 = 0.f;
+    for (int t = 0; t < 4; t++) {
+      const int i = tid + 256 * t;
+      nq4[t] = ((const f32x4*)q)[i < n4q ? i : n4q - 1]; nk4[t] = ((const f32x4*)k)[i < n4k ? i : n4k - 1];
+    }
+    float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-  for (int t = 0; t < 4; t++) {
-    const int i = tid + 256 * t;
-    const f32x4 x = nq4[t], y = nk4[t];
-    s0 += i < n4q ? x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w : 0.f;
-    s1 += i < n4k ? y.x * y.x + y.y * y.y + y.z * y.z + y.w * y.w : 0.f;
+    for (int t = 0; t < 4; t++) {
+      const int i = tid + 256 * t;
+      const f32x4 x = nq4[t], y = nk4[t];
+      s0 += i < n4q ? x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w : 0.f;
+      s1 += i < n4k ? y.x * y.x + y.y * y.y + y.z * y.z + y.w * y.w : 0.f;
+    }
+    s0 = wave_sum(s0); s1 = wave_sum(s1);
+    if (lane == 0) { red[wave] = s0; red[4 + wave] = s1; }
   }
-  s0 = wave_sum(s0); s1 = wave_sum(s1);
-  if (lane == 0) { red[wave] = s0; red[4 + wave] = s1; }
   __syncthreads();
   const float qscale = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)(a.H * a.hd) + a.eps);
   const float kscale = 1.0f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)(a.KV * a.hd) + a.eps);
   const size_t cstep = (size_t)a.max_ctx * a.hd, crow = (size_t)pos * a.hd;
-  for (int e = 4 * tid; e < nk; e += 1024) {
+  for (int e = 4 * tid; e < nk; e += 2048) {
     const int hh = e / a.hd;
     const f32x4 x = *(const f32x4*)(v + e);
     *(u32x2*)(a.cv + crow + hh * cstep + (e - hh * a.hd)) = u32x2{f2h_bits(x.x) | (f2h_bits(x.y) << 16), f2h_bits(x.z) | (f2h_bits(x.w) << 16)};
@@ -154,7 +156,7 @@ __global__ __launch_bounds__(256) void x16_rope_kernel(const X16Rope a) {
   const int i = live ? lane : half - 1;
   const float c = a.rope[(size_t)pos * a.hd + i], s = a.rope[(size_t)pos * a.hd + half + i];
 #pragma unroll 4
-  for (int h = wave; h < a.H + a.KV; h += 4) {
+  for (int h = wave; h < a.H + a.KV; h += 8) {
     const bool isq = h < a.H;
     const int o = (isq ? h : h - a.H) * a.hd;
     const float* src = isq ? q + o : k + o; const float* wn = isq ? a.qn + o : a.kn + o;
@@ -825,7 +827,7 @@ int tga_prefill16_step(const int64_t* m, const int64_t* blocks, const int32_t* t
     X16Rope ra;
     ra.q = q; ra.k = kk; ra.v = v; ra.qn = (const float*)b[PB_QN]; ra.kn = (const float*)b[PB_KN]; ra.rope = (const float*)m[PM_ROPE]; ra.qr = (float*)(ws + w.qr); ra.ck = (uint16_t*)b[PB_CK]; ra.cv = (uint16_t*)b[PB_CV];
     ra.zero = (int*)(ws + w.counts); ra.n_zero = (int)E; ra.H = (int)H; ra.KV = (int)KV; ra.hd = (int)hd; ra.max_ctx = (int)m[PM_MAXCTX]; ra.pos0 = (int)pos0; ra.eps = eps;
-    x16_rope_kernel<<<(unsigned)R, 256, 0, s>>>(ra);
+    x16_rope_kernel<<<(unsigned)R, 512, 0, s>>>(ra);
     TGA_LAUNCH_CHECK();
     if (bi + 1 == m[PM_NBLOCKS]) break;                                   // the last block's keys and values are in the cache; what follows them there is read by nobody
     X16Attn aa;
