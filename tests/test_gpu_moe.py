@@ -262,10 +262,10 @@ def test_small_glm4moe_like_decode(gpu, gate):
     print(f"without {drop}: logits rel-err {ol.rel_err(lg2, lg_gpu):.3f}")
     assert ol.rel_err(lg2, lg_gpu) > 5e-3, drop                                    # five times the parity bar
 
-@pytest.mark.parametrize("E,k", [(1, 1), (2, 2), (7, 3), (16, 16), (33, 8), (63, 16), (64, 1), (64, 8), (64, 16)])
+@pytest.mark.parametrize("E,k", [(1, 1), (2, 2), (7, 3), (8, 8), (17, 9), (32, 16), (33, 8), (63, 16), (64, 1), (64, 8), (64, 16), (64, 17)])
 @pytest.mark.parametrize("gating", [1, 2, 3, 4])
 def test_gating_in_lanes_has_the_bits_of_the_general_way(gpu, E, k, gating):
-  """At most 64 experts and 16 selected (an expert per lane) against the general way, which a selection bias of zeros takes: rows with ties, values that are not finite, both zeros, the type's lowest
+  """At most 64 experts and 8, or 16 and half of them, selected (an expert per lane) against the general way, which a selection bias of zeros takes: rows with ties, values that are not finite, both zeros, the type's lowest
   and values far apart; the expert gate/up launch's own choice (its outputs carry the expert) on the same rows."""
   from tinygrad_amd.nn import ExpertWeights, moe_gate
   rng = np.random.default_rng(E * 17 + gating)
