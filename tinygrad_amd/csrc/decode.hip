@@ -171,12 +171,12 @@ __device__ __forceinline__ float run_sum(float v) {
   if constexpr (HD8 == 32) v += __shfl_xor(v, 16, 64);
   return v;
 }
-// sums of squares of two float vectors (lengths % 4 == 0, 16-byte aligned) over the whole workgroup of 256 threads; red: 8 floats
-// of LDS.  The loads of four loop iterations of both vectors go out as one batch.
-__device__ __forceinline__ void block_sumsq2(const float* q, int nq, const float* k, int nk, float* red, float& sq, float& sk) {
+// sums of squares of two float vectors (lengths % 4 == 0, 16-byte aligned) over 256 threads, of which the caller is number tid (a workgroup may hold several such groups, each with the same vectors and
+// 8 floats of LDS of its own: red).  The loads of four loop iterations of both vectors go out as one batch.
+__device__ __forceinline__ void block_sumsq2(int tid, const float* q, int nq, const float* k, int nk, float* red, float& sq, float& sk) {
   float s0 = 0.f, s1 = 0.f;
   const int n4q = nq >> 2, n4k = nk >> 2, nmax = n4q > n4k ? n4q : n4k;
-  for (int b = threadIdx.x; b < nmax; b += 1024) {
+  for (int b = tid; b < nmax; b += 1024) {
     f32x4 vq[4], vk[4];
 #pragma unroll
     for (int t = 0; t < 4; t++) { const int i = b + 256 * t; vq[t] = ((const f32x4*)q)[i < n4q ? i : n4q - 1]; vk[t] = ((const f32x4*)k)[i < n4k ? i : n4k - 1]; }
@@ -188,7 +188,7 @@ __device__ __forceinline__ void block_sumsq2(const float* q, int nq, const float
     }
   }
   s0 = wave_sum(s0); s1 = wave_sum(s1);
-  if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6] = s0; red[4 + (threadIdx.x >> 6)] = s1; }
+  if ((tid & 63) == 0) { red[tid >> 6] = s0; red[4 + (tid >> 6)] = s1; }
   __syncthreads();
   sq = red[0] + red[1] + red[2] + red[3]; sk = red[4] + red[5] + red[6] + red[7];
 }
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(FEW ? 256 * ATTN_FEW : 256) void attn_decode_kernel
     kscale = 1.0f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)(a.n_kv * HD) + a.norm_eps);
   } else if constexpr (NORM == 3) {
     float sq, sk;
-    block_sumsq2(a.q, a.n_heads * HD, a.k, a.n_kv * HD, red, sq, sk);
+    block_sumsq2(tid, a.q, a.n_heads * HD, a.k, a.n_kv * HD, red, sq, sk);
     qscale = 1.0f / sqrtf(sq / (float)(a.n_heads * HD) + a.norm_eps);
     kscale = 1.0f / sqrtf(sk / (float)(a.n_kv * HD) + a.norm_eps);
   } else if constexpr (NORM == 2) {                     // the key of this kv head over the workgroup, the wave's query inside the wave
