@@ -182,7 +182,8 @@ def test_wide_tiles_keep_their_requests_in_flight():
   assert _wide_findings(good[:9] + [("scratch_load_dword v1, off, off", False)] + good[9:])
 
 def test_tall_tiles_wait_only_by_hand():
-  """qgemm_tall_kernel (csrc/qgemm_tall.hip): its loop over K holds no spill and no wait for vector memory but the four in front of its barriers, which leave the younger requests under way."""
+  """qgemm_tall_kernel (csrc/qgemm_tall.hip): its loop over K holds no spill and no wait for vector memory but the four in front of its barriers, which leave the younger requests under way; a request
+  into LDS never follows the write of m0, where it goes, directly (one wait state lies between them, which the compiler sees to in its own code and not in inline assembly)."""
   try: hipcc = tb._hipcc()
   except RuntimeError: pytest.skip("hipcc not found")
   with tempfile.TemporaryDirectory() as d:
@@ -200,3 +201,6 @@ def test_tall_tiles_wait_only_by_hand():
     assert len(loops) == 1, name
     assert [t for t in loops[0] if "vmcnt" in t] == ["s_waitcnt vmcnt(%d)" % n for n in (14, 15, 3, 2)], name
     assert not any(t.startswith("scratch_") for t in loops[0]) and sum(t == "s_barrier" for t in loops[0]) == 4 and sum(" lds" in t for t in loops[0]) == 21, name
+    code = [l for l in lines if l and not l.startswith((".", "s_waitcnt"))]
+    after = [t for m0, t in zip(code, code[1:]) if re.search(r"\bm0\b", m0)]
+    assert len(after) == sum(t.endswith(" lds") for t in code) >= 21 and not any(t.endswith(" lds") for t in after), name      # (and m0 has no other use)

@@ -74,13 +74,14 @@ template <> struct TallFmt<GGML_Q4_K> {                 // low nibbles of 32 byt
   }
 };
 
-// A request of the wave: lane l's sixteen bytes at descriptor + off + at land at LDS byte dst + 16 l
+// A request of the wave: lane l's sixteen bytes at descriptor + off + at land at LDS byte dst + 16 l (m0; one wait state between its write and the request, which the compiler does not add inside an asm statement; m0
+// is no clobber, as the compiler calls that undefined: it uses none of its own in this kernel)
 __device__ __forceinline__ void tall_request(u32x4 r, uint32_t dst, uint32_t off, int at) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(dst), "v"(off), "s"(r), "s"(at) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(dst), "v"(off), "s"(r), "s"(at) : "memory");
 }
 // ... four bytes a lane: what brings a line nearer
 __device__ __forceinline__ void tall_touch(u32x4 r, uint32_t dst, uint32_t off) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" :: "s"(dst), "v"(off), "s"(r) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" :: "s"(dst), "v"(off), "s"(r) : "memory");
 }
 __device__ __forceinline__ u32x4 tall_desc(const void* p) {                             // (as wide_desc: nothing relies on its range check)
   const uint64_t v = (uint64_t)(uintptr_t)p;
