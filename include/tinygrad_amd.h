@@ -409,6 +409,8 @@ int tga_synth_weights(int ggml_type, void* out, int64_t n_elements, uint32_t see
 int tga_qlinear_many(int ggml_type, int nseg, const void* const* w, void* const* y, const int64_t* n, const void* x_f16, int y_dtype, int64_t M, int64_t K, int epilogue,
                      const float* resid, void* workspace, int64_t workspace_bytes, void* stream);
 int tga_rows_format_ok(int ggml_type, int64_t K, int* ok);
+/* What such a linear with that much workspace (sixteen-byte aligned weights) is cut into: weight rows and activation rows of a tile, parts of K. */
+int tga_qlinear_many_tile(int ggml_type, int nseg, const int64_t* n, int64_t M, int64_t K, int epilogue, int64_t workspace_bytes, int* weight_rows, int* x_rows, int* parts);
 /* A prefill step of any number of rows (prefill.hip; model.py:464, 476-481): positions pos0 .. pos0 + P - 1 of nseq sequences through all blocks, keys and values appended to
  * the caches.  model / blocks: tables of int64 (pointers as integers) in the order of the PM_ / PB_ enumerations of csrc/prefill.h; tokens: (nseq, P) ids on the device.
  * _plan: bytes of the caller's workspace for that many rows (nseq * P). */

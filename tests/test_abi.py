@@ -119,3 +119,17 @@ def test_a_capture_gets_no_block(gpu):
       gpu.Buffer((n,), np.uint8)
   gpu.check(gpu.lib().tga_copy_kernel(dst.ptr, src.ptr, 4096, stream.handle)); stream.synchronize()
   assert gpu.Buffer((n,), np.uint8).ptr in kept                                    # the capture is over: kept blocks are handed out again
+
+def many_tile(t, n, m, k, epi=0, ws=64 << 20):
+  """(weight rows, activation rows) of a tile of tga_qlinear_many and the parts of K; host only."""
+  from tinygrad_amd import runtime as rt
+  out = [ctypes.c_int(0) for _ in range(3)]
+  lib = rt.load_library()
+  assert lib.tga_qlinear_many_tile(t, len(n), (ctypes.c_int64 * len(n))(*n), m, k, epi, ws, *map(ctypes.byref, out)) == 0
+  return (out[0].value, out[1].value), out[2].value
+
+@pytest.mark.parametrize("t", [2, 12], ids=["Q4_0", "Q4_K"])
+def test_tall_tiles_have_rows_of_1024_values_or_more(t):
+  """Shorter rows are outside what the rule was measured on, and rows of 256 values shorter than what the kernel's touches bring (their address lay in front of the row)."""
+  for k in (256, 512, 768): assert many_tile(t, (28672,), 1023, k)[0] != (512, 128) and many_tile(t, (14336, 14336), 2047, k, 2)[0] != (512, 128)
+  assert many_tile(t, (28672,), 1023, 1024) == ((512, 128), 1)

@@ -35,6 +35,7 @@ int64_t tga_rows_row_bytes(int fmt, int64_t K) {
 }
 int tga_rows_tall(int fmt, const RowsArgs& a, unsigned grid, hipStream_t s);             // qgemm_tall.hip
 #define ROWS_TALL 512             // the tile height that asks for it
+#define TALL_K_MIN 1024
 int tga_rows_dispatch(int fmt, const RowsArgs& a, int tt, unsigned grid, hipStream_t s) {
   if (tt == ROWS_TALL) return tga_rows_tall(fmt, a, grid, s);
   switch (fmt) {
@@ -170,8 +171,8 @@ static double rows_us(const RowsArgs& a, int tt) {
 }
 static int rows_plan(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t part_bytes) {
   const int tt = rows_plan_small(a, fmt, swiglu, may_split, part_bytes);
-  // (whole sub-tiles of sixteen rows, requests of sixteen bytes)
-  if ((fmt != F_Q4_0P && fmt != GGML_Q4_K) || tt == 32 || a.K % 256 || a.K > (1 << 20) || a.ntot >= (1ll << 30)) return tt;
+  // (whole sub-tiles of sixteen rows, requests of sixteen bytes; below TALL_K_MIN nothing is measured, and the kernel's touches take two steps)
+  if ((fmt != F_Q4_0P && fmt != GGML_Q4_K) || tt == 32 || a.K % 256 || a.K < TALL_K_MIN || a.K > (1 << 20) || a.ntot >= (1ll << 30)) return tt;
   for (int i = 0; i < (swiglu ? 2 : a.nseg); i++) if (a.n[i] % 16 || ((uintptr_t)a.w[i] & 15)) return tt;
   RowsArgs t = a, best = a;
   double us = rows_us(a, tt);
@@ -250,6 +251,23 @@ extern "C" {
 int tga_qlinear_many(int ggml_type, int nseg, const void* const* w, void* const* y, const int64_t* n, const void* x_f16, int y_dtype, int64_t M, int64_t K, int epilogue,
                      const float* resid, void* workspace, int64_t workspace_bytes, void* stream) {
   return tga_rows_linear(ggml_type, nseg, w, y, n, x_f16, y_dtype, M, K, epilogue, resid, workspace, workspace_bytes, nullptr, 0.f, nullptr, nullptr, stream);
+}
+
+int tga_qlinear_many_tile(int ggml_type, int nseg, const int64_t* n, int64_t M, int64_t K, int epilogue, int64_t workspace_bytes, int* weight_rows, int* x_rows, int* parts) {
+  const int fmt = tga_rows_fmt(ggml_type, K);
+  TGA_REQUIRE(n && weight_rows && x_rows && parts && nseg >= 1 && nseg <= 3 && (epilogue != 2 || nseg == 2) && fmt >= 0 && M >= 1 && M * K < (1ll << 32) && M < (1 << 24) && workspace_bytes >= 0,
+              "tga_qlinear_many_tile: null pointer, or a linear outside the range");
+  RowsArgs a = {};
+  a.nseg = epilogue == 2 ? 1 : nseg; a.M = (int)M; a.K = (int)K;
+  bool split = epilogue != 2 && workspace_bytes > 0;
+  for (int i = 0; i < nseg; i++) {
+    TGA_REQUIRE(n[i] > 0, "tga_qlinear_many_tile: matrix %d has no rows", i);
+    a.n[i] = n[i];
+    if (i < a.nseg) { a.ntot += n[i]; split = split && n[i] % 4 == 0; }
+  }
+  const int tt = rows_plan(a, fmt, epilogue == 2, split, (size_t)workspace_bytes);
+  *weight_rows = tt == ROWS_TALL ? 512 : tt == ROWS_WIDE ? WIDE_WT : ROWS_WT; *x_rows = tt == ROWS_TALL ? 128 : tt == ROWS_WIDE ? WIDE_TT : tt; *parts = a.ks;
+  return 0;
 }
 
 }  // extern "C"

@@ -83,7 +83,7 @@ __device__ __forceinline__ void tall_request(u32x4 r, uint32_t dst, uint32_t off
 __device__ __forceinline__ void tall_touch(u32x4 r, uint32_t dst, uint32_t off) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" :: "s"(dst), "v"(off), "s"(r) : "memory");
 }
-__device__ __forceinline__ u32x4 tall_desc(const void* p) {                             // (as wide_desc: nothing relies on its range check)
+__device__ __forceinline__ u32x4 tall_desc(const void* p) {                             // (as wide_desc: no request relies on its range check; a touch near the end of a matrix does, with a range of its own)
   const uint64_t v = (uint64_t)(uintptr_t)p;
   return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v), (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) & 0xFFFFu, 0xFFFFFFFFu, 0x00027000u};
 }
@@ -207,6 +207,7 @@ __global__ __launch_bounds__(512, 1) void qgemm_tall_kernel(const RowsArgs a) {
 }
 
 int tga_rows_tall(int fmt, const RowsArgs& a, unsigned grid, hipStream_t s) {
+  TGA_REQUIRE(a.K >= 512 && a.K % 256 == 0, "tga_rows_tall: rows of %d values", a.K);    // (a touch brings two steps of a row)
   const dim3 g(grid, a.ks);
   const bool sw = a.epi == ROWS_SWIGLU;
   if (fmt == F_Q4_0P) { if (sw) qgemm_tall_kernel<F_Q4_0P, true><<<g, 512, 0, s>>>(a); else qgemm_tall_kernel<F_Q4_0P, false><<<g, 512, 0, s>>>(a); }

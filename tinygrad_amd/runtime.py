@@ -45,6 +45,7 @@ def _declare(lib):
     "tga_qlinear_experts_routed": [i, vp, vp, i64, vp, i, i, i, ctypes.c_float, vp, vp, vp, vp, i, i64, i64, vp],
     "tga_qlinear_experts_routed_rows": [i, vp, vp, i64, vp, i, i, i, i, ctypes.c_float, vp, vp, vp, vp, i, i64, i64, vp],
     "tga_qlinear_many": [i, i, c_void_pp, c_void_pp, ctypes.POINTER(i64), vp, i, i64, i64, i, vp, vp, i64, vp],
+    "tga_qlinear_many_tile": [i, i, ctypes.POINTER(i64), i64, i64, i, i64, ctypes.POINTER(i), ctypes.POINTER(i), ctypes.POINTER(i)],
     "tga_rows_format_ok": [i, i64, ctypes.POINTER(i)], "tga_prefill_plan": [ctypes.POINTER(i64), i64, ctypes.POINTER(i64)],
     "tga_prefill16_plan": [ctypes.POINTER(i64), ctypes.POINTER(i64), i64, i64, ctypes.POINTER(i), ctypes.POINTER(i64)],
     "tga_prefill16_tail_plan": [ctypes.POINTER(i64), ctypes.POINTER(i64), ctypes.POINTER(i), ctypes.POINTER(i64)],
