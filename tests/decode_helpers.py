@@ -1,4 +1,5 @@
 """Shared by the GPU decode tests: step-by-step greedy decoding on the GPU against the oracle fed the same token history."""
+import ctypes
 import numpy as np
 
 def greedy_vs_reference_numerics(model, oracle, prompt, n_new):
@@ -23,3 +24,10 @@ def greedy_vs_reference_numerics(model, oracle, prompt, n_new):
   model.check_state()
   return got, ref, worst, margin, rms
 
+def many_tile(t, n, m, k, epi=0, ws=64 << 20):
+  """(weight rows, activation rows) of a tile of tga_qlinear_many and the parts of K; host only."""
+  from tinygrad_amd import runtime as rt
+  out = [ctypes.c_int(0) for _ in range(3)]
+  lib = rt.load_library()
+  assert lib.tga_qlinear_many_tile(t, len(n), (ctypes.c_int64 * len(n))(*n), m, k, epi, ws, *map(ctypes.byref, out)) == 0
+  return (out[0].value, out[1].value), out[2].value

@@ -1,6 +1,7 @@
 """The C-ABI library loads and exports every symbol include/tinygrad_amd.h declares (no GPU call is made)."""
 import ctypes, pathlib, re
 import pytest
+from decode_helpers import many_tile
 
 ROOT = pathlib.Path(__file__).resolve().parent.parent
 
@@ -119,14 +120,6 @@ def test_a_capture_gets_no_block(gpu):
       gpu.Buffer((n,), np.uint8)
   gpu.check(gpu.lib().tga_copy_kernel(dst.ptr, src.ptr, 4096, stream.handle)); stream.synchronize()
   assert gpu.Buffer((n,), np.uint8).ptr in kept                                    # the capture is over: kept blocks are handed out again
-
-def many_tile(t, n, m, k, epi=0, ws=64 << 20):
-  """(weight rows, activation rows) of a tile of tga_qlinear_many and the parts of K; host only."""
-  from tinygrad_amd import runtime as rt
-  out = [ctypes.c_int(0) for _ in range(3)]
-  lib = rt.load_library()
-  assert lib.tga_qlinear_many_tile(t, len(n), (ctypes.c_int64 * len(n))(*n), m, k, epi, ws, *map(ctypes.byref, out)) == 0
-  return (out[0].value, out[1].value), out[2].value
 
 @pytest.mark.parametrize("t", [2, 12], ids=["Q4_0", "Q4_K"])
 def test_tall_tiles_have_rows_of_1024_values_or_more(t):

@@ -180,7 +180,7 @@ def test_batched_glm4moe_like_decode(gpu, B, gate):
 
 @pytest.mark.parametrize("hd,kv,group,norm", [(64, 4, 1, 0), (64, 2, 8, 2), (128, 8, 4, 0), (128, 4, 2, 1), (128, 2, 5, 2), (128, 40, 1, 1), (128, 8, 5, 1), (64, 48, 2, 1), (64, 72, 1, 1)])
 def test_attention_of_few_splits_has_the_bits_of_two_launches(gpu, hd, kv, group, norm):
-  """Caches of one to four splits are one launch, of five the split launch and the merge: the same positions, the same bits of every output and cache row.  Positions at the splits' edges, groups that
+  """Caches of one or two splits are one launch, of three and more the split launch and the merge: the same positions, the same bits of every output and cache row.  Positions at the splits' edges, groups that
   are no multiple of four heads, every norm - over whole rows of up to 4096 values and of more, whose squares each split's waves sum for themselves -; (72 heads of five sequences are more workgroups than
   CUs: two launches either way)."""
   rt, B = gpu, 5

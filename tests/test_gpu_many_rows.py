@@ -2,6 +2,7 @@
 sequence and several, dense and MoE, one step and a prompt cut into several - against the same models prefilled position by position."""
 import ctypes, dataclasses
 import numpy as np, pytest
+from decode_helpers import many_tile
 from oracle import ggml as og, linear as ol, llm as ollm
 from tinygrad_amd import synth
 
@@ -76,13 +77,15 @@ def test_wide_tiles_of_q4_0(gpu, m, n, k, epi):
   if epi == 2: refs = [refs[0] / (1 + np.exp(-refs[0])) * refs[1]]
   for o, ref in zip(outs, refs): assert ol.rel_err(o.numpy(), ref + r if epi == 1 else ref) <= (2e-4 if epi == 2 else 5e-5)
 
-@pytest.mark.parametrize("t", [2, 12], ids=["Q4_0", "Q4_K"])
-@pytest.mark.parametrize("m,n,k,epi", [(385, (16400,), 1280, 0), (513, (12304,), 1536, 0), (1023, (4112,), 2816, 1), (1025, (4096, 1040, 2064), 1280, 0), (641, (7184,), 1280, 2), (300, (4096,), 14336, 1), (2047, (6160,), 3072, 0)],
-                         ids=["one-row", "ragged", "split", "three", "swiglu", "split-eight", "rounds"])
-def test_tall_tiles(gpu, t, m, n, k, epi):
-  """The 512 x 128 tiles: last tiles of 1, 44 and 127 rows and of 16 and 32 outputs, five to fourteen steps a workgroup, odd and even, matrices that meet inside a tile, K split into unequal parts, float32 and fp16 results.
+TALL = [("one-row", 385, (16400,), 1280, 0, 1, 1), ("ragged", 513, (14352,), 1536, 0, 1, 1), ("split", 1023, (4112,), 4096, 1, 3, 3), ("split-even", 1023, (4112,), 2816, 1, 2, None), ("three", 1025, (4096, 1040, 2064), 1280, 0, 1, 1),
+        ("swiglu", 641, (7184,), 1280, 2, 1, 1), ("split-four", 1023, (4096,), 14336, 1, 4, 4), ("split-ten", 300, (4096,), 14336, 1, 10, None), ("rounds", 2047, (6160,), 3072, 0, 1, 1), ("four-steps", 1023, (14352, 14352), 1024, 0, 1, 1)]
+@pytest.mark.parametrize("t,m,n,k,epi,parts", [pytest.param(t, *c[1:5], c[5 + i], id=f"{c[0]}-{name}") for i, (t, name) in enumerate([(2, "Q4_0"), (12, "Q4_K")]) for c in TALL if c[5 + i]])
+def test_tall_tiles(gpu, t, m, n, k, epi, parts):
+  """The 512 x 128 tiles, which the rule takes for each of these: last tiles of 1, 44 and 127 rows and of 16 outputs, four to fourteen steps a workgroup, odd and even, matrices that meet inside a tile, K split into two to ten
+  parts, equal and not, for either type, float32 and fp16 results.
   Weights that begin four bytes behind a sixteen-byte line take the other tiles: the same fp16 weights in another order of sums, float32 sums of K products differ by about sqrt(K) 2^-24 of their absolute sum, 5e-5
   of the largest result at most.  So do those of the reference for Q4_0; for Q4_K, whose weights round differently now and then, the bar is that of test_many_rows_linear_at_tile_edges."""
+  assert many_tile(t, n * 2 if epi == 2 else n, m, k, epi) == ((512, 128), parts)
   from tinygrad_amd import runtime as rt
   rng = np.random.default_rng(m + t)
   ws = rt.Buffer((64 << 20,), np.uint8)

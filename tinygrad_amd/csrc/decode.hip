@@ -207,8 +207,8 @@ __device__ __forceinline__ void block_sumsq2(int tid, const float* q, int nq, co
 // load sits behind a branch (a join makes the compiler wait for every outstanding load):
 //   0 none, 1 over the whole q and k vectors of at most 4096 values each (read in one batch), 2 per head, 3 over whole vectors of any length
 // FEW: a cache of at most ATTN_FEW splits (decode): four waves per split in one workgroup, which merges them in LDS with the arithmetic of attn_merge_kernel instead of leaving them to that launch (8B-arch
-// lockstep step of eight sequences, 128 positions of cache: 6.0 + 4.6 -> 7.6 us a block, the same bits).  Waves of splits behind the position take part and are left out of the merge.
-#define ATTN_FEW 4
+// lockstep step of eight sequences, 128 positions of cache: 6.0 + 4.6 -> 7.6 us a block, the same bits; by size: attention_few).  Waves of splits behind the position take part and are left out of the merge.
+#define ATTN_FEW 2
 template <int HD8, int NORM, bool FEW>
 __global__ __launch_bounds__(FEW ? 256 * ATTN_FEW : 256) void attn_decode_kernel(const AttnArgs args) {
   const AttnArgs a = attn_args_of_sequence(args, blockIdx.z);   // field reads become kernel-argument loads in the entry block
@@ -438,8 +438,8 @@ __global__ __launch_bounds__(FEW ? 256 * ATTN_FEW : 256) void attn_decode_kernel
           asm volatile("" : "+v"(l[j]), "+v"(v));
           o += v;
         }
-        static_assert(NS == 4 || !FEW, "the tree of a wave's sum");
-        o *= 1.0f / ((l[0] + l[1]) + (l[2] + l[3]));
+        static_assert(NS == 2 || !FEW, "the tree of a wave's sum");
+        o *= 1.0f / (l[0] + l[NS - 1]);
         const int e = (kvh * group + h0 + hh) * HD + d;
         if (a.out16) a.out16[a.stage_fmt ? staged_pos(a.stage_fmt, e, a.stage_nu) : e] = (_Float16)o;
         if (a.out32) a.out32[e] = o;
@@ -1058,6 +1058,14 @@ int tga_rmsnorm(const float* x, const float* weight, int dim, float eps, void* o
   return tga_rmsnorm_rows(x, weight, 1, dim, eps, out_f16, out_f32, stage_type, stream);
 }
 
+// Caches of one or two splits are one launch that merges its own.  What it saves is a launch, what it costs: waves that each serve all query heads of the group, in passes of four with a merge each, on as many CUs as
+// there are (kv head, sequence) pairs instead of splits times as many, whatever the position.  us, one launch / two, replayed in a graph:
+//   one split, groups of 1 / 4 / 8, head_dim 128, 8 pairs 4.2 / 6.7, 5.4 / 7.7, 8.3 / 9.9, 64 pairs 4.7 / 7.7, 5.9 / 8.6, 8.9 / 11.1, 256 pairs (4, 8) 6.9 / 10.0, 9.8 / 12.9; of 64, groups of 4, 8 / 256 pairs 4.8 / 7.0, 5.9 / 8.9
+//   two, position in the second, groups of 1 / 4 / 8, 8 pairs 4.9 / 6.7, 6.2 / 7.6, 9.5 / 9.9, 64 pairs 5.5 / 8.0, 6.9 / 9.0, 10.2 / 11.5, 256 pairs (4, 8) 8.5 / 12.1, 11.8 / 15.6; in the first 64 pairs (4) 6.8 / 8.6, 32 (6) 10.5 / 10.5
+//   not taken: two splits, groups of 12 / 16, 16 / 32 pairs 12.8 / 12.3, 16.5 / 15.6; three and four (with this split of the work), groups of 4, 8 / 64 pairs 7.9 / 7.7, 8.7 / 9.3 and 9.4 / 7.7, 10.4 / 9.7,
+//   256 pairs 11.9 / 14.6 and 14.5 / 16.4, but 14.1 / 12.7 with the position in the first of four; groups of 8, 8 / 64 pairs 12.2 / 10.0, 13.0 / 11.8 and 15.1 / 10.0, 16.0 / 12.3.
+// (More pairs than CUs, which was not measured when the line was drawn: two splits, groups of 4, 384 / 512 pairs 12.1 / 15.3, 12.9 / 16.9; in the first 11.8 / 12.5.)
+static bool attention_few(int nsplit, int group, int head_dim, int pairs) { return nsplit <= ATTN_FEW && group <= 8 && head_dim <= 128 && pairs <= 256; }
 static int attention_launch(int chunk, int batch, const float* q, const float* k, const float* v, const float* q_norm_weight, const float* k_norm_weight, float norm_eps,
                             int norm_per_head, void* cache_k, void* cache_v, float* partials, const void* state,
                             int n_heads, int n_kv_heads, int head_dim, int max_ctx, const float* rope_table, void* out_f16, float* out_f32, int stage_type, void* stream) {
@@ -1094,7 +1102,7 @@ static int attention_launch(int chunk, int batch, const float* q, const float* k
 #define TGA_ATTN_NORM(HD8, FEW, NT) do { \
     if (norm == 0) attn_decode_kernel<HD8, 0, FEW><<<grid, NT, 0, s>>>(a); else if (norm == 1) attn_decode_kernel<HD8, 1, FEW><<<grid, NT, 0, s>>>(a); \
     else if (norm == 2) attn_decode_kernel<HD8, 2, FEW><<<grid, NT, 0, s>>>(a); else attn_decode_kernel<HD8, 3, FEW><<<grid, NT, 0, s>>>(a); } while (0)
-  const bool few = !chunk && a.nsplit <= ATTN_FEW && head_dim <= 128 && n_kv_heads * batch <= 256;      // one launch merges its own splits (larger heads: four do not fit LDS; one workgroup fits a CU)
+  const bool few = !chunk && attention_few(a.nsplit, n_heads / n_kv_heads, head_dim, n_kv_heads * batch);
   static const bool chunk_mfma_off = getenv("TGA_ATTN_CHUNK") && !strcmp(getenv("TGA_ATTN_CHUNK"), "rows");
   const bool chunk_mfma = chunk && batch > 8 && norm == 0 && (head_dim == 64 || head_dim == 128) && n_heads / n_kv_heads <= 8 && !chunk_mfma_off;   // chunks of more than eight rows attend on the matrix cores
   for (int pass = chunk ? 1 : 0; pass <= (chunk ? 2 : 0); pass++) {   // chunked prefill: append every row, then attend from the cache
