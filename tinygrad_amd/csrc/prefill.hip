@@ -8,6 +8,7 @@
 #include "decode.h"
 #include "moe_gate.h"
 #include "prefill.h"
+#include <type_traits>
 
 int tga_rows_fmt(int ggml_type, int64_t K);                                              // qgemm_rows.hip
 int64_t tga_rows_row_bytes(int fmt, int64_t K);
@@ -20,14 +21,29 @@ int tga_rows_norm(float* x, const float* w, int M, int n, float eps, void* xn, v
 // One workgroup per row.  q is rotated (after its norm) and leaves as TWO fp16 values per element, the rounded value and what the rounding left over, for matrix-core
 // scores of the float32 query (rows_attn_kernel); k is rotated into the cache, v copied.  The rotation is apply_rope's (model.py:29-33) written as one rounded product and one fused multiply-add,
 // like every kernel that rotates, so a cache row has the same bits whichever path appended it.  norm: 0 none, 1 RMSNorm over the whole q / k rows (model.py:169), 2 per head (:180).
-// Rows come as the linears leave them: whole (ks 1), or as the sums of a split K, plane values apart, which are completed here in their order (a launch of its own that writes and reads them again before:
-// 1023 rows of 4096 + 2 x 1024 values, two sums each, 12.6 + 10.3 -> 14.4 us a block; 508 rows, three and eight sums, 17 -> 8.9).
+// Rows come as the linears leave them: whole (ks 1), or as the sums of a split K, plane values apart, which are completed here in their order.  A launch that completes them and a rotation of whole rows / here, us:
+// 4096 + 2 x 1024 values, 1023 and 508 rows of two parts 12.0 + 13.7 / 15.4, 7.0 + 8.0 / 8.8, 256 and 129 of five 7.2 + 5.2 / 7.7, 5.0 + 5.0 / 5.9, 26 of eight 4.4 + 4.3 / 5.9; 2048 + 2 x 512, 699 rows of three
+// 7.3 + 8.3 / 9.6, 97 and 22 of four 4.2 + 3.9 / 4.2, 3.3 + 3.9 / 4.2.  Few rows are a chain of trips to memory: with a trip per part the last of these was 10.9.
 struct RopeSrc { const float* p; size_t plane; int stride, ks; };
 struct RopeArgs {
   RopeSrc q, k, v; const float* qn; const float* kn; const float* rope;
   uint16_t* qh; uint16_t* ql; uint16_t* ck; uint16_t* cv; int* zero;      // zero: n_zero counters cleared for the launches behind this one
   int H, KV, hd, max_ctx, P, pos0, norm, n_zero; float eps;
 };
+// f(N, p) for the parts p .. p + N - 1 of ks, whose values f requests together: up to four at once (a loop over the parts is a trip to memory for each)
+template <class F> __device__ __forceinline__ void rope_parts(int ks, F f) {
+  if (ks == 1) f(std::integral_constant<int, 1>{}, 0);
+  else if (ks == 2) f(std::integral_constant<int, 2>{}, 0);
+  else if (ks == 3) f(std::integral_constant<int, 3>{}, 0);
+  else {
+    f(std::integral_constant<int, 4>{}, 0);
+    int p = 4;
+    for (; p + 4 <= ks; p += 4) f(std::integral_constant<int, 4>{}, p);
+    if (ks - p == 3) f(std::integral_constant<int, 3>{}, p);
+    else if (ks - p == 2) f(std::integral_constant<int, 2>{}, p);
+    else if (ks - p == 1) f(std::integral_constant<int, 1>{}, p);
+  }
+}
 __global__ __launch_bounds__(512) void rows_rope_kernel(const RopeArgs a) {
   __shared__ float red[8];
   const int r = blockIdx.x, z = r / a.P, pos = a.pos0 + r % a.P, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = a.hd >> 1;
@@ -35,12 +51,18 @@ __global__ __launch_bounds__(512) void rows_rope_kernel(const RopeArgs a) {
   if (r == 0) for (int i = tid; i < a.n_zero; i += 512) a.zero[i] = 0;
   const float* q = a.q.p + (size_t)r * a.q.stride; const float* k = a.k.p + (size_t)r * a.k.stride; const float* v = a.v.p + (size_t)r * a.v.stride;
   const size_t crow = ((size_t)z * a.KV * a.max_ctx + pos) * a.hd, cstep = (size_t)a.max_ctx * a.hd;
-#pragma unroll 2
-  for (int e = 4 * tid; e < nk; e += 2048) {
+  for (int e = 4 * (511 - tid); e < nk; e += 2048) {                      // (the last waves first: they have the fewest heads)
     const int hh = e / a.hd;
-    f32x4 x = *(const f32x4*)(v + e);
-#pragma unroll 4
-    for (int p = 1; p < a.v.ks; p++) { const f32x4 y = *(const f32x4*)(v + p * a.v.plane + e); x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w; }
+    f32x4 x;
+    rope_parts(a.v.ks, [&](auto n, int p) {
+      constexpr int N = decltype(n)::value;
+      f32x4 y[N];
+#pragma unroll
+      for (int j = 0; j < N; j++) y[j] = *(const f32x4*)(v + (p + j) * a.v.plane + e);
+      if (p == 0) x = y[0];
+#pragma unroll
+      for (int j = 0; j < N; j++) if (p + j > 0) { x.x += y[j].x; x.y += y[j].y; x.z += y[j].z; x.w += y[j].w; }
+    });
     *(u32x2*)(a.cv + crow + hh * cstep + (e - hh * a.hd)) = u32x2{f2h_bits(x.x) | (f2h_bits(x.y) << 16), f2h_bits(x.z) | (f2h_bits(x.w) << 16)};
   }
   float qs = 1.f, ks = 1.f;
@@ -63,20 +85,22 @@ __global__ __launch_bounds__(512) void rows_rope_kernel(const RopeArgs a) {
   const int nh = a.H + a.KV;
   for (int h0 = wave; h0 < nh; h0 += 8 * RU) {
     float xa[RU], xb[RU];
+    rope_parts(a.q.ks, [&](auto n, int p) {                               // (q and k are of one launch where they are split)
+      constexpr int N = decltype(n)::value;
+      float ya[N][RU], yb[N][RU];
 #pragma unroll
-    for (int u = 0; u < RU; u++) {
-      const int h = min(h0 + 8 * u, nh - 1);
-      const float* src = h < a.H ? q + h * a.hd : k + (h - a.H) * a.hd;
-      xa[u] = src[i]; xb[u] = src[half + i];
-    }
-#pragma unroll 3
-    for (int p = 1; p < a.q.ks; p++)                                      // (q and k are of one launch where they are split)
+      for (int j = 0; j < N; j++)
 #pragma unroll
-      for (int u = 0; u < RU; u++) {
-        const int h = min(h0 + 8 * u, nh - 1);
-        const float* src = (h < a.H ? q + h * a.hd : k + (h - a.H) * a.hd) + p * a.q.plane;
-        xa[u] += src[i]; xb[u] += src[half + i];
-      }
+        for (int u = 0; u < RU; u++) {
+          const int h = min(h0 + 8 * u, nh - 1);
+          const float* src = (h < a.H ? q + h * a.hd : k + (h - a.H) * a.hd) + (p + j) * a.q.plane;
+          ya[j][u] = src[i]; yb[j][u] = src[half + i];
+        }
+#pragma unroll
+      for (int j = 0; j < N; j++)
+#pragma unroll
+        for (int u = 0; u < RU; u++) { xa[u] = p + j ? xa[u] + ya[j][u] : ya[j][u]; xb[u] = p + j ? xb[u] + yb[j][u] : yb[j][u]; }
+    });
 #pragma unroll
     for (int u = 0; u < RU; u++) {
       const int h = h0 + 8 * u;
