@@ -8,7 +8,6 @@
 #include "decode.h"
 #include "moe_gate.h"
 #include "prefill.h"
-#include <type_traits>
 
 int tga_rows_fmt(int ggml_type, int64_t K);                                              // qgemm_rows.hip
 int64_t tga_rows_row_bytes(int fmt, int64_t K);
@@ -22,28 +21,17 @@ int tga_rows_norm(float* x, const float* w, int M, int n, float eps, void* xn, v
 // scores of the float32 query (rows_attn_kernel); k is rotated into the cache, v copied.  The rotation is apply_rope's (model.py:29-33) written as one rounded product and one fused multiply-add,
 // like every kernel that rotates, so a cache row has the same bits whichever path appended it.  norm: 0 none, 1 RMSNorm over the whole q / k rows (model.py:169), 2 per head (:180).
 // Rows come as the linears leave them: whole (ks 1), or as the sums of a split K, plane values apart, which are completed here in their order.  A launch that completes them and a rotation of whole rows / here, us:
-// 4096 + 2 x 1024 values, 1023 and 508 rows of two parts 12.0 + 13.7 / 15.4, 7.0 + 8.0 / 8.8, 256 and 129 of five 7.2 + 5.2 / 7.7, 5.0 + 5.0 / 5.9, 26 of eight 4.4 + 4.3 / 5.9; 2048 + 2 x 512, 699 rows of three
-// 7.3 + 8.3 / 9.6, 97 and 22 of four 4.2 + 3.9 / 4.2, 3.3 + 3.9 / 4.2.  Few rows are a chain of trips to memory: with a trip per part the last of these was 10.9.
+// 4096 + 2 x 1024 values, 1023 and 508 rows of two parts 12.0 + 8.9 / 12.0, 7.0 + 5.8 / 7.2, 256 and 129 of five 7.2 + 5.1 / 8.0, 5.0 + 4.8 / 6.2, 26 of eight 4.6 + 4.4 / 6.2; 2048 + 2 x 512, 699 rows of three
+// 7.1 + 5.2 / 6.8, 97 and 22 of four 4.1 + 3.7 / 4.1, 2.8 + 3.7 / 4.0; 1024 + 2 x 256, 1099 of two 5.2 + 5.2 / 5.5.  Few rows are a chain of trips to memory: with a trip per part the 22 rows took 10.9.
 struct RopeSrc { const float* p; size_t plane; int stride, ks; };
 struct RopeArgs {
   RopeSrc q, k, v; const float* qn; const float* kn; const float* rope;
   uint16_t* qh; uint16_t* ql; uint16_t* ck; uint16_t* cv; int* zero;      // zero: n_zero counters cleared for the launches behind this one
   int H, KV, hd, max_ctx, P, pos0, norm, n_zero; float eps;
 };
-// f(N, p) for the parts p .. p + N - 1 of ks, whose values f requests together: up to four at once (a loop over the parts is a trip to memory for each)
-template <class F> __device__ __forceinline__ void rope_parts(int ks, F f) {
-  if (ks == 1) f(std::integral_constant<int, 1>{}, 0);
-  else if (ks == 2) f(std::integral_constant<int, 2>{}, 0);
-  else if (ks == 3) f(std::integral_constant<int, 3>{}, 0);
-  else {
-    f(std::integral_constant<int, 4>{}, 0);
-    int p = 4;
-    for (; p + 4 <= ks; p += 4) f(std::integral_constant<int, 4>{}, p);
-    if (ks - p == 3) f(std::integral_constant<int, 3>{}, p);
-    else if (ks - p == 2) f(std::integral_constant<int, 2>{}, p);
-    else if (ks - p == 1) f(std::integral_constant<int, 1>{}, p);
-  }
-}
+// RU: heads of a wave whose values are requested together, and with them up to four parts of each: a head or a part at a time, each is a trip to memory.  PARTS: ks of q and k, 5: more than four (kernels of
+// their own: one that holds them all takes 224 registers, whole rows 50, and half as many workgroups share a CU)
+template <int RU, int PARTS>
 __global__ __launch_bounds__(512) void rows_rope_kernel(const RopeArgs a) {
   __shared__ float red[8];
   const int r = blockIdx.x, z = r / a.P, pos = a.pos0 + r % a.P, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = a.hd >> 1;
@@ -53,16 +41,14 @@ __global__ __launch_bounds__(512) void rows_rope_kernel(const RopeArgs a) {
   const size_t crow = ((size_t)z * a.KV * a.max_ctx + pos) * a.hd, cstep = (size_t)a.max_ctx * a.hd;
   for (int e = 4 * (511 - tid); e < nk; e += 2048) {                      // (the last waves first: they have the fewest heads)
     const int hh = e / a.hd;
-    f32x4 x;
-    rope_parts(a.v.ks, [&](auto n, int p) {
-      constexpr int N = decltype(n)::value;
-      f32x4 y[N];
+    f32x4 x = *(const f32x4*)(v + e);
+    for (int p = 1; p < a.v.ks; p += 3) {                                 // (the last part again behind it, and not added)
+      f32x4 y[3];
 #pragma unroll
-      for (int j = 0; j < N; j++) y[j] = *(const f32x4*)(v + (p + j) * a.v.plane + e);
-      if (p == 0) x = y[0];
+      for (int j = 0; j < 3; j++) y[j] = *(const f32x4*)(v + min(p + j, a.v.ks - 1) * a.v.plane + e);
 #pragma unroll
-      for (int j = 0; j < N; j++) if (p + j > 0) { x.x += y[j].x; x.y += y[j].y; x.z += y[j].z; x.w += y[j].w; }
-    });
+      for (int j = 0; j < 3; j++) if (p + j < a.v.ks) { x.x += y[j].x; x.y += y[j].y; x.z += y[j].z; x.w += y[j].w; }
+    }
     *(u32x2*)(a.cv + crow + hh * cstep + (e - hh * a.hd)) = u32x2{f2h_bits(x.x) | (f2h_bits(x.y) << 16), f2h_bits(x.z) | (f2h_bits(x.w) << 16)};
   }
   float qs = 1.f, ks = 1.f;
@@ -80,27 +66,38 @@ __global__ __launch_bounds__(512) void rows_rope_kernel(const RopeArgs a) {
   const bool live = lane < half;                                          // (half is 32 or 64)
   const int i = live ? lane : half - 1;
   const float c = rr[i], s = rr[half + i];
-  // (a wave's heads in groups of RU, whose values are requested together: a head at a time, each is a trip to memory)
-  constexpr int RU = 5;
   const int nh = a.H + a.KV;
   for (int h0 = wave; h0 < nh; h0 += 8 * RU) {
-    float xa[RU], xb[RU];
-    rope_parts(a.q.ks, [&](auto n, int p) {                               // (q and k are of one launch where they are split)
-      constexpr int N = decltype(n)::value;
-      float ya[N][RU], yb[N][RU];
+    constexpr int N = PARTS < 5 ? PARTS : 4;
+    float xa[RU], xb[RU], ya[N][RU], yb[N][RU];
+    auto request = [&](int p) __attribute__((always_inline)) {              // parts p .. p + N - 1 (q and k are of one launch where they are split); behind the last one that one again
 #pragma unroll
       for (int j = 0; j < N; j++)
 #pragma unroll
         for (int u = 0; u < RU; u++) {
           const int h = min(h0 + 8 * u, nh - 1);
-          const float* src = (h < a.H ? q + h * a.hd : k + (h - a.H) * a.hd) + (p + j) * a.q.plane;
+          const float* src = (h < a.H ? q + h * a.hd : k + (h - a.H) * a.hd) + (PARTS < 5 ? j : min(p + j, a.q.ks - 1)) * a.q.plane;
           ya[j][u] = src[i]; yb[j][u] = src[half + i];
         }
+    };
+    request(0);
 #pragma unroll
-      for (int j = 0; j < N; j++)
+    for (int u = 0; u < RU; u++) {
+      xa[u] = ya[0][u]; xb[u] = yb[0][u];
 #pragma unroll
-        for (int u = 0; u < RU; u++) { xa[u] = p + j ? xa[u] + ya[j][u] : ya[j][u]; xb[u] = p + j ? xb[u] + yb[j][u] : yb[j][u]; }
-    });
+      for (int j = 1; j < N; j++) { xa[u] += ya[j][u]; xb[u] += yb[j][u]; }
+    }
+    if constexpr (PARTS == 5) {
+#pragma clang loop unroll(disable)
+      for (int p = 4; p < a.q.ks; p += 4) {
+        request(p);
+#pragma unroll
+        for (int j = 0; j < N; j++)
+          if (p + j < a.q.ks)
+#pragma unroll
+            for (int u = 0; u < RU; u++) { xa[u] += ya[j][u]; xb[u] += yb[j][u]; }
+      }
+    }
 #pragma unroll
     for (int u = 0; u < RU; u++) {
       const int h = h0 + 8 * u;
@@ -129,6 +126,16 @@ __global__ __launch_bounds__(512) void rows_rope_kernel(const RopeArgs a) {
       }
     }
   }
+}
+
+// (heads of a wave dealt evenly to as few groups of five as hold them)
+static void rows_rope_launch(const RopeArgs& a, unsigned rows, hipStream_t s) {
+  const int n = (a.H + a.KV + 7) / 8, groups = (n + 4) / 5, ru = (n + groups - 1) / groups, parts = a.q.ks < 5 ? a.q.ks : 5;
+#define ROPE_P(RU, PARTS) if (parts == PARTS) rows_rope_kernel<RU, PARTS><<<rows, 512, 0, s>>>(a)
+#define ROPE(RU) do { ROPE_P(RU, 1); ROPE_P(RU, 2); ROPE_P(RU, 3); ROPE_P(RU, 4); ROPE_P(RU, 5); } while (0)
+  if (ru <= 2) ROPE(2); else if (ru == 3) ROPE(3); else ROPE(5);
+#undef ROPE
+#undef ROPE_P
 }
 
 // ------------------------------------------------------------------------------------------------ attention
@@ -463,7 +470,7 @@ int tga_prefill_step(const int64_t* m, const int64_t* blocks, const int32_t* tok
     ra.qh = (uint16_t*)(ws + w.qh); ra.ql = (uint16_t*)(ws + w.ql); ra.ck = (uint16_t*)b[PB_CK]; ra.cv = (uint16_t*)b[PB_CV];
     ra.zero = b[PB_MOE] ? (int*)(ws + w.counts) : nullptr; ra.n_zero = b[PB_MOE] ? (int)E : 0;
     ra.H = (int)H; ra.KV = (int)KV; ra.hd = (int)hd; ra.max_ctx = (int)m[PM_MAXCTX]; ra.P = (int)P; ra.pos0 = (int)pos0; ra.eps = eps;
-    rows_rope_kernel<<<(unsigned)R, 512, 0, s>>>(ra);
+    rows_rope_launch(ra, (unsigned)R, s);
     TGA_LAUNCH_CHECK();
     // The last block's keys and values are in the cache, and the first logits come from the decode step behind the prompt: its rows go no further (8B-arch, 1024 tokens: 0.5 ms of 21).  A model of one
     // block takes the whole step: its workspace is where single blocks are compared with the reference
