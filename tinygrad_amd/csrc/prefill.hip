@@ -147,8 +147,8 @@ static void rows_rope_launch(const RopeArgs& a, unsigned rows, hipStream_t s) {
 // the other way round: the workgroups that share a CU have long and short tiles (1023 rows, 32 heads, two workgroups a CU: 41.4 -> 39.5 us).
 // NG = 2: eight waves, of which four take the even tiles of keys and four the odd ones; their sums meet in LDS.  A workgroup is a chain of tiles, 2.4 us each where it has a CU to itself and little less
 // where two share one, and registers leave room for eight waves a CU: for as many workgroups as CUs from four tiles on (heads of 128, 192 / 256 workgroups of up to 6 / 8 tiles 16.4 -> 15.5 / 20.4 ->
-// 18.1 us; of 64, 128 / 256 of up to 16 / 32 28.8 -> 20.5 / 55 -> 37), and for twice as many where chains are long (384 of up to 12 tiles 31.5 -> 27, 512 of up to 16 41.0 -> 38.9 beside
-// fp16 linears, 41 either way in the Q4_0 8B model; not
+// 18.1 us; of 64, 128 / 256 of up to 16 / 32 28.8 -> 20.5 / 55 -> 37), and for twice as many where chains are long (heads of 128, 288 of up to 12 tiles 28.0 -> 23.5, 384 of up to 16
+// 36.7 -> 30.7, 448 / 512 of up to 16 36.8 -> 36.0 / 39.2 -> 38.1 in the Q4_0 8B model, 512 of up to 32 67 -> 62; of 64, 512 of up to 16 / 32 29.2 -> 24.3, 54.4 -> 41.6; not
 // taken: 192 of 3 tiles 10.9 / 11.7, 384 of 3 12.9 / 17.2, 512 of 4 / 8 16.9 / 21.0, 24 / 26, 768 of up to 24 71 / 82, 1024 of up to 32 114 / 129).
 // Two fp16 values hold 22 bits and more of a query or probability, and sums are formed in few additions at their full size (remainders first, two chains per score, a tile's products from
 // zero).  Share of fp16 results that are not the rounded float64 attention, 64 and 1024 positions, heads of 64 and 128, scores of standard deviation 0.03 .. 5: 1.8e-4 .. 2.2e-3; the float32
