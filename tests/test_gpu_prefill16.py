@@ -51,11 +51,14 @@ WIDE = {f"{h}x{hd}": dict(num_blocks=2, dim=512, hidden_dim=256, n_heads=h, n_kv
         for h, kv, hd in ((18, 6, 128), (40, 8, 64), (24, 24, 128), (32, 8, 128))}
 LONG = {f"long-{h}x{hd}": dict(num_blocks=2, dim=512, hidden_dim=256, n_heads=h, n_kv_heads=h // 2, head_dim=hd, qk_norm=h * hd, num_experts=16, num_experts_per_tok=2, **BASE) for h, hd in ((8, 64), (4, 128))}
 
-@pytest.mark.parametrize("name,n", [(name, 95) for name in WIDE] + [(name, 1667) for name in LONG])
+# gating by way of LDS: few experts of which many are taken, and more experts than a workgroup has lanes
+MANY = {f"{e}-experts": dict(num_blocks=2, dim=512, hidden_dim=256, n_heads=8, n_kv_heads=8, head_dim=64, qk_norm=512, num_experts=e, num_experts_per_tok=k, **BASE) for e, k in ((24, 18), (80, 8), (300, 3))}
+
+@pytest.mark.parametrize("name,n", [(name, 95) for name in {**WIDE, **MANY}] + [(name, 1667) for name in LONG])
 def test_bits_over_the_rest_of_the_range(gpu, monkeypatch, name, n):
-  """94 positions of wide attention rows; 1666 positions (27 splits of 64, two steps: 1024 rows and 642 with the tail of eight)."""
+  """94 positions of wide attention rows, and of experts that are gated four or eight tokens a workgroup; 1666 positions (27 splits of 64, two steps: 1024 rows and 642 with the tail of eight)."""
   from tinygrad_amd import llm
-  a, b = _models({**WIDE, **LONG}[name], 5 + n, 128 if n < 128 else 2048)
+  a, b = _models({**WIDE, **MANY, **LONG}[name], 5 + n, 128 if n < 128 else 2048)
   prompt = np.random.default_rng(n).integers(0, BASE["vocab_size"], size=n).tolist()
   a.prefill(prompt)
   assert a._chunker._rows16_ws is not None and a._chunker.x is None

@@ -7,7 +7,7 @@
 // maximum, of the lanes that hold it the lowest - which is the pairwise rank below as long as no score is NaN (those rank by themselves: the general way).  k steps of a reduction in registers,
 // about 80 cycles each, against as many reads of LDS as there are experts, with their comparisons, and a maximum by way of LDS.  A launch of moe_gate_kernel, us, in lanes / the general way: 64 experts, one token,
 // k 1 / 8 / 16: 2.9 / 2.9 / 3.4 against 5.6; 4096 tokens 3.0 / 3.8 / 5.0 against 7.5; 16 experts, 4096 tokens, k 4 / 8 3.3 / 3.8 against 4.5, k 16 5.0 against 4.5 (not taken).
-__device__ __forceinline__ bool gate_in_lanes(int n_experts, int k) { return n_experts <= 64 && (k <= 8 || (k <= 16 && 2 * k <= n_experts)); }
+__host__ __device__ __forceinline__ bool gate_in_lanes(int n_experts, int k) { return n_experts <= 64 && (k <= 8 || (k <= 16 && 2 * k <= n_experts)); }
 __device__ __forceinline__ int gate_kind(int gating, int norm_topk) { return gating == 1 && norm_topk ? 3 : gating; }      // model.py:116-117: softmax over the selected is all there is to it
 // the score of expert `lane` from its logit v (lanes behind the last expert: any v); false: a score is NaN
 __device__ __forceinline__ bool gate_score_lane(float v, int n_experts, int kind, int lane, float& s) {

@@ -311,21 +311,24 @@ __global__ __launch_bounds__(256 * NG) void rows_attn_kernel(const RowsAttnArgs 
 #define PF_MAX_E 512
 // One wave per token: selection and weights (gate_topk_wave), and this assignment's place among the rows of its expert.  The order of places is that of arrival: a row's
 // values do not depend on its place, and the weighted sum of a token runs over its slots in order.  A workgroup counts its tokens' assignments in LDS and adds them up in one go (an addition per
-// assignment: the two lines that 64 counts are in were what all waves waited for; 508 rows of 64 experts, top 8: 11.6 -> 4.8 us).
-#define PF_GATE_T 16
-__global__ __launch_bounds__(64 * PF_GATE_T) void rows_gate_kernel(const float* __restrict__ logits, int R, int E, int k, int gating, int norm_topk, float scale, int* __restrict__ sel,
+// assignment: the two lines that 64 counts are in were what all waves waited for; 508 rows of 64 experts, top 8: 11.6 -> 4.8 us).  T tokens a workgroup: sixteen where a wave gates in registers; by way of LDS its
+// reads are what bounds it - all waves of a CU share them - and fewer tokens a workgroup spread them.  us with 4 / 8 / 16 tokens a workgroup, 100 and 1024 rows: 64 experts, 24 taken 5.8 / 5.9 / 7.1, 9.9 / 7.6 / 7.4;
+// 96, 8 taken 8.7 / 9.6 / 12.1, 13.1 / 11.0 / 12.3; 128, 8 taken 10.8 / 11.1 / 14.4, 14.5 / 12.7 / 14.6; 160, 6 taken 16.8 / 17.6 / 22.8, 20.0 / 19.0 / 23.1; 256, 8 taken 30.4 / 32.0 / 42.5, 33.3 / 33.2 / 42.9;
+// 512, 10 taken 106.5 / 114.0 / 153.5, 107.3 / 114.4 / 153.2.
+template <int T>
+__global__ __launch_bounds__(64 * T) void rows_gate_kernel(const float* __restrict__ logits, int R, int E, int k, int gating, int norm_topk, float scale, int* __restrict__ sel,
                                                         float* __restrict__ probs, int* __restrict__ counts, int* __restrict__ place) {
-  __shared__ float sc[PF_GATE_T][PF_MAX_E]; __shared__ float tmp[PF_GATE_T][192];
+  __shared__ float sc[T][PF_MAX_E]; __shared__ float tmp[T][192];
   __shared__ int s_count[PF_MAX_E];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, t = blockIdx.x * PF_GATE_T + wave;
-  if (tid < E) s_count[tid] = 0;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, t = blockIdx.x * T + wave;
+  for (int i = tid; i < E; i += 64 * T) s_count[i] = 0;
   if (t < R) gate_topk_wave(logits + (size_t)t * E, E, k, gating, norm_topk, scale, sel + (size_t)t * k, probs + (size_t)t * k, sc[wave], tmp[wave], lane);
   __syncthreads();
   const bool has = t < R && lane < k;
   int e = 0, at = 0;
   if (has) { e = ((const int*)tmp[wave])[lane]; at = atomicAdd(&s_count[e], 1); }
   __syncthreads();
-  if (tid < E && s_count[tid]) s_count[tid] = atomicAdd(&counts[tid], s_count[tid]);
+  for (int i = tid; i < E; i += 64 * T) if (s_count[i]) s_count[i] = atomicAdd(&counts[i], s_count[i]);
   __syncthreads();
   if (has) place[(size_t)t * k + lane] = s_count[e] + at;
 }
@@ -358,7 +361,9 @@ __global__ __launch_bounds__(512) void rows_group_kernel(const int* __restrict__
 }
 
 int pf_gate(const float* logits, int R, int E, int k, int gating, int norm_topk, float scale, int* sel, float* probs, int* counts, int* place, hipStream_t s) {
-  rows_gate_kernel<<<(unsigned)((R + PF_GATE_T - 1) / PF_GATE_T), 64 * PF_GATE_T, 0, s>>>(logits, R, E, k, gating, norm_topk, scale, sel, probs, counts, place);
+#define PF_GATE(T) rows_gate_kernel<T><<<(unsigned)((R + T - 1) / T), 64 * T, 0, s>>>(logits, R, E, k, gating, norm_topk, scale, sel, probs, counts, place)
+  if (gate_in_lanes(E, k)) PF_GATE(16); else if (E <= 64) PF_GATE(8); else PF_GATE(4);
+#undef PF_GATE
   TGA_LAUNCH_CHECK();
   return 0;
 }
