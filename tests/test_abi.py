@@ -126,3 +126,9 @@ def test_tall_tiles_have_rows_of_1024_values_or_more(t):
   """Shorter rows are outside what the rule was measured on, and rows of 256 values shorter than what the kernel's touches bring (their address lay in front of the row)."""
   for k in (256, 512, 768): assert many_tile(t, (28672,), 1023, k)[0] != (512, 128) and many_tile(t, (14336, 14336), 2047, k, 2)[0] != (512, 128)
   assert many_tile(t, (28672,), 1023, 1024) == ((512, 128), 1)
+
+@pytest.mark.parametrize("t,m,n,k,epi,tall", [(2, 1261, 9296, 1280, 2, False), (2, 1023, 17312, 1280, 2, False), (2, 1024, 12464, 1024, 2, True), (2, 2047, 8784, 1536, 2, True), (2, 1024, 22768, 1024, 0, False),
+                                              (12, 1024, 18896, 1024, 2, False), (12, 768, 24288, 1536, 2, False), (12, 1024, 18672, 2048, 2, True)])
+def test_tall_tiles_of_several_rounds_and_few_steps(t, m, n, k, epi, tall):
+  """Two and more rounds of tall tiles of few steps, the last one less than 75 or 78 % full, were 2 - 7 % slower than the other tiles: taken from there on."""
+  assert (many_tile(t, (n, n) if epi == 2 else (n,), m, k, epi)[0] == (512, 128)) == tall

@@ -161,6 +161,9 @@ static int rows_plan_small(RowsArgs& a, int fmt, bool swiglu, bool may_split, si
 // 135 / 106, 148 / 120, 215 / 230 (not taken), 291 / 237, 606 / 511; Q4_0 14336 -> 4096, 300, 508, 1023, 2047 rows 69 / 61, 86 / 77, 142 / 124, 257 / 217; 4096 -> 6144 of 768, 1023, 2047 rows 77 / 60, 76 / 70,
 // 134 / 100; 4096 -> 4096 of 1023 rows 57 / 59 (not taken); 2048 -> 2 x 5632 of 1023 rows 65 / 53, of 640 43 / 52 (not taken); 3072 -> 2 x 8448 of 1280 rows,
 // two rounds two thirds full, 146 / 156 (not taken); 14336 -> 4096 of 150 rows 45 / 47 (not taken).
+// Several rounds of few steps pay each round's ramp (5 us above the estimate) and need a fuller last one: Q4_0, fewer than six steps, 71 % full 1280 -> 2 x 17312 of 1023 rows 119 / 125 (not taken), 77 % 1024 -> 2 x 12464 of
+// 1024 rows 77 / 73; from six on 73 % 1536 -> 2 x 8784 of 2047 rows 146 / 143; Q4_K, fewer than eight, 77 % 1024 -> 2 x 18896 of 1024 rows 114 / 123, 74 % 1536 -> 2 x 24288 of 768 rows 152 / 161 (not taken), 81 %
+// 1536 of 2 rounds 117 / 108; from eight on 76 % 2048 -> 2 x 18672 of 1024 rows 213 / 206.
 static double rows_split_us(const RowsArgs& a) { return a.ks == 1 ? 0. : 2. + (double)a.ks * a.M * a.ntot * 8e-6 / 6.5; }
 static double rows_us(const RowsArgs& a, int tt) {
   const long long wg = (long long)a.row_tiles * a.tok_tiles * a.ks;
@@ -191,8 +194,9 @@ static int rows_plan(RowsArgs& a, int fmt, bool swiglu, bool may_split, size_t p
     }
     const long long rounds = (per * t.ks + 31) / 32;
     const double full = (double)(tiles * t.ks) / (double)(256 * rounds);
-    if (full < (rounds == 1 ? 0.5 : 0.7)) continue;
-    const double step = (5.1 + (full > 0.6 ? 3. * (full - 0.6) : 0.)) * (fmt == GGML_Q4_K ? 1.16 : 1.);
+    const bool q4_k = fmt == GGML_Q4_K;
+    if (full < (rounds == 1 ? 0.5 : steps / t.ks >= (q4_k ? 8 : 6) ? 0.7 : q4_k ? 0.78 : 0.75)) continue;
+    const double step = (5.1 + (full > 0.6 ? 3. * (full - 0.6) : 0.)) * (q4_k ? 1.16 : 1.);
     const double e = (double)rounds * (9. + step * steps / t.ks) + rows_split_us(t);
     if (e < us) { us = e; best = t; taken = true; }
   }
