@@ -1064,6 +1064,7 @@ int tga_rmsnorm(const float* x, const float* weight, int dim, float eps, void* o
 //   two, position in the second, groups of 1 / 4 / 8, 8 pairs 4.9 / 6.7, 6.2 / 7.6, 9.5 / 9.9, 64 pairs 5.5 / 8.0, 6.9 / 9.0, 10.2 / 11.5, 256 pairs (4, 8) 8.5 / 12.1, 11.8 / 15.6; in the first 64 pairs (4) 6.8 / 8.6, 32 (6) 10.5 / 10.5
 //   not taken: two splits, groups of 12 / 16, 16 / 32 pairs 12.8 / 12.3, 16.5 / 15.6; three and four (with this split of the work), groups of 4, 8 / 64 pairs 7.9 / 7.7, 8.7 / 9.3 and 9.4 / 7.7, 10.4 / 9.7,
 //   256 pairs 11.9 / 14.6 and 14.5 / 16.4, but 14.1 / 12.7 with the position in the first of four; groups of 8, 8 / 64 pairs 12.2 / 10.0, 13.0 / 11.8 and 15.1 / 10.0, 16.0 / 12.3.
+//   with q / k norms (whole rows of 2048 .. 5120 values, per head), groups of 1, 2, 4, 5 and 8, 5 .. 240 pairs, one and two splits: 1.00 (groups of 8, two splits, whole rows) .. 1.67 times as fast as the two launches;
 //   more pairs than CUs keep the two launches, though one would gain there too: two splits, groups of 4, 384 / 512 pairs 12.1 / 15.3, 12.9 / 16.9, position in the first 11.8 / 12.5 (other groups and norms are not measured).
 static bool attention_few(int nsplit, int group, int head_dim, int pairs) { return nsplit <= ATTN_FEW && group <= 8 && head_dim <= 128 && pairs <= 256; }
 static int attention_launch(int chunk, int batch, const float* q, const float* k, const float* v, const float* q_norm_weight, const float* k_norm_weight, float norm_eps,
